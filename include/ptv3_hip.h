@@ -508,9 +508,16 @@ int ptv3_linear_gemm_fwd(const void *x, const void *w, const void *bias, const v
  * enable_flash=False, model.py:458-474; half-precision layers whose widths the kernels above do not take):
  * out = resid + act(x w^T + bias), act = exact GELU when gelu != 0, resid (n, nout) or NULL (it may be `out`
  * itself: every element is read before it is written, by the same thread). fp32 / fp16 / bf16, any k and nout;
- * fp32 FMA arithmetic, one rounding. Not tuned: the MFMA kernels above take the shapes of the released models. */
+ * fp32 arithmetic, one rounding. fp32 runs on the matrix cores (ptv3_linear_f32_fwd); half precision is not tuned
+ * here: the MFMA kernels above take the shapes of the released models. */
 int ptv3_linear_any_fwd(const void *x, const void *w, const void *bias, const void *resid, int dtype, int64_t n,
                         int k, int nout, int gelu, void *out, void *stream);
+/* The fp32 layer, any k and nout, on the fp32 MFMA. x (n, k) is PTV3_F32, or PTV3_F16 rows that are converted on the
+ * way in; out (n, nout) is PTV3_F32, or PTV3_F16 (one rounding): the projections on either side of an attention that
+ * reads and writes halves in a float model. Half rows on either side: k a multiple of 4, x and w 16-byte aligned, not
+ * both x and out (PTV3_ESHAPE). w, bias, resid are fp32. */
+int ptv3_linear_f32_fwd(const void *x, int x_dtype, const float *w, const float *bias, const float *resid, int64_t n,
+                        int k, int nout, int gelu, void *out, int out_dtype, void *stream);
 /* The same followed by an inference-mode nn.BatchNorm1d and optionally the GELU, the projections of
  * model.py:726-735 (Linear -> BatchNorm1d -> GELU) in one kernel; statistics and affine parameters as
  * for ptv3_bn_act. The Linear's result is rounded to dtype before the normalisation, as when stored. */

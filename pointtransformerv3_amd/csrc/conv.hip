@@ -1142,6 +1142,11 @@ extern "C" int ptv3_subm_conv_fwd(const void* feat, int dtype, int64_t n, int ci
     PTV3_RETURN_LAUNCH();
 }
 
+int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
+                             const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot,
+                             const float* weight, const float* bias, int cout, float* y, float* out,
+                             hipStream_t stream);   // gemmf32.hip
+
 extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, int cin, int taps,
                                         int64_t n_pairs, const int32_t* tap_ptr,
                                         const int32_t* row_ptr, const int32_t* pair_in,
@@ -1149,12 +1154,15 @@ extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, 
                                         const void* bias, int cout, void* y, void* out,
                                         void* stream_) {
     if (n < 0 || cin < 1 || cout < 1 || taps < 1 || n_pairs < 0 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
-    if (dtype != PTV3_F16 && dtype != PTV3_BF16) return PTV3_ESHAPE;   // fp32 goes through ptv3_subm_conv_fwd
-    if (cin % 16 != 0 || cout % 8 != 0) return PTV3_ESHAPE;
+    if (dtype < PTV3_F32 || dtype > PTV3_BF16) return PTV3_ESHAPE;
+    if (dtype != PTV3_F32 && (cin % 16 != 0 || cout % 8 != 0)) return PTV3_ESHAPE;
     if (n == 0) return PTV3_OK;
     if (!feat || !tap_ptr || !row_ptr || !weight || !out) return PTV3_EINVAL;
     if (n_pairs > 0 && (!pair_in || !pair_slot || !y)) return PTV3_EINVAL;
     hipStream_t stream = (hipStream_t)stream_;
+    if (dtype == PTV3_F32)
+        return ptv3_subm_conv_pairs_f32((const float*)feat, n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot,
+                                        (const float*)weight, (const float*)bias, cout, (float*)y, (float*)out, stream);
     const dim3 sgrid((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), sblock(256);
     int rc = PTV3_OK;
     if (dtype == PTV3_F16) {

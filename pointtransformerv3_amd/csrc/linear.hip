@@ -302,10 +302,9 @@ int dispatch_linear(const void* x, const void* w, const void* bias, const LinBn*
     return PTV3_ESHAPE;
 }
 
-// The general shape: any number of inputs and outputs, fp32 as well as fp16 / bf16, plain FMA arithmetic in
-// fp32 on 64 x 64 output tiles with 16-input slices of x and w in LDS. It serves the fp32 model (the
-// reference's parity path, model.py:458-474 with enable_flash=False) and half-precision layers whose widths the
-// MFMA kernels above do not take; not tuned.
+// The general half-precision shape: any number of inputs and outputs, plain FMA arithmetic in fp32 on 64 x 64 output
+// tiles with 16-input slices of x and w in LDS, for the layers whose widths the MFMA kernels above do not take; not
+// tuned. (fp32 layers of any shape: gemmf32.hip.)
 constexpr int ANY_TILE = 64, ANY_KC = 16;
 
 template <typename T> __device__ __forceinline__ float any_f(T v) { return (float)v; }
@@ -427,7 +426,9 @@ extern "C" int ptv3_linear_any_fwd(const void* x, const void* w, const void* bia
     if (!x || !w || !out) return PTV3_EINVAL;
     hipStream_t stream = (hipStream_t)stream_;
     switch (dtype) {
-        case PTV3_F32: return launch_linear_any<float>(x, w, bias, resid, n, k, nout, gelu, out, stream);
+        case PTV3_F32:
+            return ptv3_linear_f32_fwd(x, PTV3_F32, (const float*)w, (const float*)bias, (const float*)resid, n, k, nout, gelu,
+                                       out, PTV3_F32, stream_);
         case PTV3_F16: return launch_linear_any<_Float16>(x, w, bias, resid, n, k, nout, gelu, out, stream);
         case PTV3_BF16: return launch_linear_any<__bf16>(x, w, bias, resid, n, k, nout, gelu, out, stream);
         default: return PTV3_EINVAL;

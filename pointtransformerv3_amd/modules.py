@@ -335,9 +335,26 @@ class SerializedAttention(PointModule):
         return ops.patch_attention(qkv, self.num_heads, slot_src, slot_dst, cu_seqlens,
                                    max_seqlen, self.scale)
 
+    def _halves_between(self, x):
+        """A float layer outside autograd whose attention works in half (model.py:477, :483): qkv is rounded in the
+        epilogue of its projection and the output projection reads halves, without conversion passes."""
+        return (x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and self.enable_flash and self.channels % 8 == 0
+                and all(type(m) is nn.Linear and m.weight.dtype == torch.float32 for m in (self.qkv, self.proj))
+                and not ops.wants_grad(x, *self.parameters()) and not (self.training and self.attn_drop > 0.0))
+
+    def qkv_rows(self, x):
+        return ops.linear_f32(x, self.qkv.weight, self.qkv.bias, torch.float16) if self._halves_between(x) else ops.linear(x, self.qkv)
+
+    def proj_rows(self, x, dtype):
+        """The output projection of attention rows in the dtype of the block's rows."""
+        if x.dtype == torch.float16 and dtype == torch.float32:   # the halves of qkv_rows
+            return ops.linear_f32(x, self.proj.weight, self.proj.bias)
+        return ops.linear(x, self.proj)
+
     def forward(self, point):
-        feat = self.attend(point, ops.linear(point.feat, self.qkv))
-        feat = ops.linear(feat, self.proj)
+        dtype = point.feat.dtype
+        feat = self.attend(point, self.qkv_rows(point.feat))
+        feat = self.proj_rows(feat, dtype)
         feat = self.proj_drop(feat)
         point.feat = feat
         return point
@@ -440,20 +457,20 @@ class Block(PointModule):
         shift = mlp.fc2.bias if (plain_mlp and not fused_mlp) else None
         if qkv is None:
             point.feat = normed
-            qkv = ops.linear(normed, self.attn.qkv)
+            qkv = self.attn.qkv_rows(normed)
         attn_out = self.attn.attend(point, qkv)
-        if (fused_mlp and self.channels in ops.BLOCK_TAIL_WIDE_CHANNELS and type(self.attn.proj) is nn.Linear
+        if (fused_mlp and attn_out.dtype == feat.dtype and self.channels in ops.BLOCK_TAIL_WIDE_CHANNELS and type(self.attn.proj) is nn.Linear
                 and self.attn.proj.bias is not None and not (self.training and self.attn.proj_drop.p > 0)):
             # proj, the residual, the MLP's pre-norm and the MLP with its residual in one kernel
             feat = ops.block_tail_wide(attn_out, feat, self.attn.proj, ln2, mlp)
             point.feat = feat
             point.sparse_conv_feat = point.sparse_conv_feat.replace_feature(feat)
             return point
-        if ops.linear_ln_ok(attn_out, self.attn.proj) and not (self.training and self.attn.proj_drop.p > 0):
+        if attn_out.dtype == feat.dtype and ops.linear_ln_ok(attn_out, self.attn.proj) and not (self.training and self.attn.proj_drop.p > 0):
             # proj, the residual and the MLP's pre-norm in one kernel
             feat, normed = ops.linear_ln(attn_out, self.attn.proj, feat, ln2, 2, shift=shift)
         else:
-            branch = self.attn.proj_drop(ops.linear(attn_out, self.attn.proj))
+            branch = self.attn.proj_drop(self.attn.proj_rows(attn_out, feat.dtype))
             feat, normed = ops.layer_norm(branch, ln2.weight, ln2.bias, ln2.eps, residual=feat, mode=2, shift=shift)
         if fused_mlp:
             # fc1 + GELU + fc2 + residual in one kernel, the 4C-wide hidden tensor never leaves the CU

@@ -810,7 +810,7 @@ def conv_plan_direct(indices, ks):
 
 
 def subm_conv_pairs(feat, plan, weight, bias=None):
-    """Submanifold convolution over the plan's active pairs only (fp16 / bf16)."""
+    """Submanifold convolution over the plan's active pairs only."""
     _dev(feat, weight, bias)
     lib = _lib.load()
     feat = feat.contiguous()
@@ -1359,6 +1359,20 @@ def linear_any(x, weight, bias=None, gelu=False, resid=None):
     _lib.check(_lib.load().ptv3_linear_any_fwd(_ptr(x2), _ptr(w), _ptr(b), _ptr(resid), _dtype_code(x2), n, k, w.shape[0],
                                                int(bool(gelu)), _ptr(out), _stream()), "ptv3_linear_any_fwd")
     return out if resid is not None else out.reshape(*lead, w.shape[0])
+
+
+def linear_f32(x, weight, bias=None, out_dtype=torch.float32):
+    """x W^T + b with a float weight: x in float or half (converted on the way in), the result in float or half (one
+    rounding; not both half). The qkv and output projections of a float model whose attention works in half."""
+    _dev(x, weight, bias)
+    x = x.contiguous()
+    n, k = x.shape
+    w = weight.contiguous()
+    b = None if bias is None else bias.contiguous()
+    out = torch.empty((n, w.shape[0]), dtype=out_dtype, device=x.device)
+    _lib.check(_lib.load().ptv3_linear_f32_fwd(_ptr(x), _dtype_code(x), _ptr(w), _ptr(b), None, n, k, w.shape[0], 0, _ptr(out),
+                                               _DTYPE_CODE[out_dtype], _stream()), "ptv3_linear_f32_fwd")
+    return out
 
 
 def linear_gemm_ok(x, weight):

@@ -143,12 +143,11 @@ class SubMConv3d(nn.Module):
 
     def convolve(self, x, feat, weight, bias, packed=None):
         """The convolution of feat (N, Cin) over x's neighbourhoods with weight (Cout, V, Cin), on whichever
-        form fits: dense output-stationary (fp32, or many active taps), pair lists, tiles, or sparse tiles.
+        form fits: pair lists (always in fp32), dense output-stationary (many active taps), tiles, or sparse tiles.
         packed() hands out the weight in the tile kernels' order when the caller has it cached."""
         cout, _, cin = weight.shape
-        if feat.dtype == torch.float32:
-            nbr = x.neighbour_map(self.kernel_size, self.indice_key)
-            return ops.subm_conv(feat, nbr, weight, bias, tap_major=True)
+        if feat.dtype == torch.float32:   # fp32 MFMA over the active pairs
+            return ops.subm_conv_pairs(feat, x.conv_plan(self.kernel_size, self.indice_key), weight, bias)
         if cin % 16 != 0:
             # the MFMA kernels consume input channels 16 at a time: zero-pad the thin stem input
             pad = 16 - cin % 16
