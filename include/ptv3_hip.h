@@ -620,6 +620,74 @@ int ptv3_block_tail_fused(const void *attn, const void *shortcut, const void *w_
                           const void *b1, const void *w2, const void *b2, int dtype, int64_t n,
                           int channels, int hidden, void *out, void *stream);
 
+/* ---- The index of a whole forward: what follows from the coordinates alone, every encoder level at once ------------
+ * (model.py:81-136 serialization, :138-174 sparsify, :382-453 padding and slot tables, :652-703 pooled tables, and the
+ * pair and tile lists of the convolutions). Four stages, each queued on `stream`; between them the caller waits
+ * (ptv3_index_wait) for words that the last kernel of a stage stores in `host_slot`, pinned host memory of
+ * ptv3_index_slot_words(levels, scenes) int64: [0..2] the sequence number of the stage that has come through (the
+ * caller passes a number the words do not hold yet), then data:
+ *   begin  scene ids, sparse indices, level 0's voxel hash and pair counts. Data: grid extent (3 words), scene ends.
+ *   sort   codes, order, inverse of level 0, cells of every pooled level. Data: their number, pooled scene ends.
+ *   pool   pooled tables, padding and slot tables, pair counts of the pooled levels. Data: pair counts.
+ *   lists  pair lists and tile lists (want[l]: PTV3_LISTS_*).
+ * The caller allocates: `state` (PTV3_INDEX_STATE_BYTES host bytes, kept until after `lists`), and the device buffers
+ * whose sizes the *_bytes calls return; begin's and pool's scratch must stay until `lists` has run on the stream,
+ * the rest as long as the tables are used. ptv3_index_levels describes the result. Nothing is allocated or kept
+ * inside. At most PTV3_MAX_LEVELS levels and PTV3_MAX_ORDERS orders; n < 2^24 where tile lists are wanted. */
+#define PTV3_MAX_LEVELS 8
+#define PTV3_MAX_ORDERS 8
+#define PTV3_INDEX_STATE_BYTES 16384
+#define PTV3_SLOT_DATA 3                    /* extent (3), unused (1), cells per pooled level (8), pair counts (2 per level) */
+#define PTV3_SLOT_ENDS (PTV3_SLOT_DATA + 4 + PTV3_MAX_LEVELS + 2 * PTV3_MAX_LEVELS)   /* scene ends, level by level */
+#define PTV3_LISTS_PAIRS 1                  /* 3x3x3: row_ptr, pair_in, pair_slot */
+#define PTV3_LISTS_TILES 2                  /* 3x3x3: tile_tap, tile_pair, vox_taps */
+#define PTV3_LISTS_PAIRS5 4                 /* level 0, 5x5x5 */
+
+typedef struct ptv3_index_cfg {
+    int64_t n;                              /* points of level 0 */
+    int32_t n_levels, n_orders, n_scenes;
+    int32_t stem5;                          /* level 0 has 5x5x5 lists as well */
+    int32_t pads_all;                       /* pad / unpad on every level (else on level 0 only) */
+    int32_t reserved;
+    int32_t pool_depth[PTV3_MAX_LEVELS];    /* [j]: coordinate bits dropped between level j - 1 and j */
+    int32_t patch[PTV3_MAX_LEVELS];
+    int32_t only128[PTV3_MAX_LEVELS];       /* the level's tile form is the 128-channel one: tiles may hold 96 outputs */
+    uint32_t slot_orders[PTV3_MAX_LEVELS];  /* bit r: attention reads the level along row r of its tables */
+} ptv3_index_cfg;
+
+typedef struct ptv3_level {
+    int64_t n, n_pad, n_seq, n_pairs, n_pairs5;
+    int64_t *code, *order, *inverse;        /* (orders, n) */
+    int32_t *grid;                          /* (n, 3) */
+    int64_t *batch, *offset;                /* (n,), (scenes,) */
+    int32_t *indices;                       /* (n, 4) */
+    int64_t *cluster, *idx_ptr;             /* cell of every point of the level above; its members (n + 1) */
+    int64_t *pad, *unpad;
+    int32_t *cu;                            /* (n_seq + 1,) */
+    int32_t *slot_src[PTV3_MAX_ORDERS], *slot_dst[PTV3_MAX_ORDERS];
+    int32_t *tap_ptr, *row_ptr, *pair_in, *pair_slot, *tile_tap, *tile_pair, *vox_taps;
+    int32_t *tap_ptr5, *row_ptr5, *pair_in5, *pair_slot5;
+    int32_t tile_voxels, depth;
+} ptv3_level;
+
+int64_t ptv3_index_slot_words(int n_levels, int n_scenes);
+size_t ptv3_index_begin_bytes(const ptv3_index_cfg *cfg);
+/* batch_in: scene ids the caller has, or NULL (then they are written to batch_out from the scene ends) */
+int ptv3_index_begin(void *state, const ptv3_index_cfg *cfg, const int32_t *grid_coord, const int64_t *batch_in,
+                     const int64_t *offset, int64_t *batch_out, void *workspace, size_t workspace_bytes,
+                     int64_t *host_slot, int64_t seq, void *stream);
+int ptv3_index_wait(const int64_t *host_slot, int which, int64_t seq, void *stream);
+size_t ptv3_index_sort_bytes(const void *state);
+int ptv3_index_sort(void *state, int depth, int key_bits, const int32_t *order_ids, int64_t *code, int64_t *order,
+                    int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);
+int ptv3_index_pool_bytes(void *state, size_t *tables, size_t *scratch);
+/* perms: (levels - 1, orders) host array, row r of a pooled level's tables comes from row perms[r] of the level above */
+int ptv3_index_pool(void *state, const int32_t *perms, void *tables, size_t tables_bytes, void *scratch,
+                    size_t scratch_bytes, void *stream);
+int ptv3_index_lists_bytes(void *state, const int32_t *want, size_t *bytes);
+int ptv3_index_lists(void *state, const int32_t *want, void *lists, size_t lists_bytes, void *stream);
+const ptv3_level *ptv3_index_levels(const void *state);
+
 #ifdef __cplusplus
 }
 #endif

@@ -111,6 +111,17 @@ SIGNATURES = {
                                      _vp, _vp, _vp]),
     "ptv3_block_tail_fused": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                      _vp, _vp]),
+    "ptv3_index_slot_words": (_i64, [_i32, _i32]),
+    "ptv3_index_begin_bytes": (_sz, [_vp]),
+    "ptv3_index_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _i64, _vp]),
+    "ptv3_index_wait": (_i32, [_vp, _i32, _i64, _vp]),
+    "ptv3_index_sort_bytes": (_sz, [_vp]),
+    "ptv3_index_sort": (_i32, [_vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "ptv3_index_pool_bytes": (_i32, [_vp, _vp, _vp]),
+    "ptv3_index_pool": (_i32, [_vp, _vp, _vp, _sz, _vp, _sz, _vp]),
+    "ptv3_index_lists_bytes": (_i32, [_vp, _vp, _vp]),
+    "ptv3_index_lists": (_i32, [_vp, _vp, _vp, _sz, _vp]),
+    "ptv3_index_levels": (_vp, [_vp]),
     "ptv3_layer_norm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _f32, _i32, _vp, _vp, _vp]),
 }
 

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(SORT_THREADS) void scatter_kernel(
     const KI* __restrict__ keys_in, const int32_t* __restrict__ idx_in, int64_t n, int shift, int pass,
     const uint32_t* __restrict__ totals, uint64_t* look, int tiles, uint32_t* __restrict__ gave_up,
     KO* __restrict__ keys_out, int32_t* __restrict__ idx_out, int64_t* __restrict__ order,
-    int64_t* __restrict__ inverse) {
+    int64_t* __restrict__ inverse, KO* __restrict__ sorted) {
     __shared__ uint32_t whist[SORT_WAVES][RADIX];   // per wave and digit: count, then start inside the sorted tile
     __shared__ uint32_t gdelta[RADIX];              // global start of the digit's run minus its start inside the tile
     __shared__ uint32_t wsum[SORT_WAVES];
@@ -208,6 +208,7 @@ __global__ __launch_bounds__(SORT_THREADS) void scatter_kernel(
             if (LAST) {
                 order[rbase + pos] = iv;
                 inverse[rbase + iv] = pos;
+                if (sorted) sorted[rbase + pos] = kv;
             } else {
                 keys_out[rbase + pos] = kv;
                 idx_out[rbase + pos] = iv;
@@ -249,8 +250,8 @@ SortWs carve(void* base, int64_t n, int k) {
 }
 
 template <typename KO>
-int run_passes(const int64_t* code, int64_t n, int k, int passes, int64_t* order, int64_t* inverse, const SortWs& w,
-                hipStream_t stream) {
+int run_passes(const int64_t* code, int64_t n, int k, int passes, int64_t* order, int64_t* inverse, void* sorted,
+               const SortWs& w, hipStream_t stream) {
     const int tiles = (int)ptv3_ceil_div(n, SORT_TILE);
     const size_t lds = (sizeof(KO) + sizeof(int32_t)) * SORT_TILE;
     const dim3 grid((unsigned)tiles, (unsigned)k), block(SORT_THREADS);
@@ -272,7 +273,7 @@ int run_passes(const int64_t* code, int64_t n, int k, int passes, int64_t* order
         static LdsGrant grant; /* per instantiation and device: the tile needs more than the default 64 KB */ \
         if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant)) return rc_;                      \
         hipLaunchKernelGGL(kern, grid, block, lds, stream, IN, iin, n, shift, p, totals, w.look, tiles, gave_up, kout, \
-                           iout, order, inverse);                                                           \
+                           iout, order, inverse, (KO*)sorted);                                              \
     } while (0)
         if (first && last) PTV3_SCATTER(int64_t, code, true, true);
         else if (first) PTV3_SCATTER(int64_t, code, true, false);
@@ -292,20 +293,26 @@ extern "C" size_t ptv3_argsort_workspace_bytes(int64_t n, int k) {
     return carve(nullptr, n, k).bytes;
 }
 
-extern "C" int ptv3_argsort(const int64_t* code, int64_t n, int k, int key_bits, int64_t* order,
-                            int64_t* inverse, void* workspace, size_t workspace_bytes,
-                            void* stream_) {
+// sorted_keys: where the sorted keys of every row go (uint32_t when key_bits <= 32, else uint64_t), or null
+int ptv3_argsort_keys(const int64_t* code, int64_t n, int k, int key_bits, int64_t* order, int64_t* inverse,
+                      void* sorted_keys, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if (n < 0 || k < 1 || k > 65535 || n >= (1ll << 31)) return PTV3_EINVAL;
     if (key_bits < 1 || key_bits > 63) return PTV3_EDEPTH;
     if (n == 0) return PTV3_OK;
     if (!code || !order || !inverse || !workspace) return PTV3_EINVAL;
     SortWs w = carve(workspace, n, k);
     if (workspace_bytes < w.bytes) return PTV3_EWORKSPACE;
-    hipStream_t stream = (hipStream_t)stream_;
     const int passes = (key_bits + 7) / 8;
     // the bits above key_bits are equal across a row (the contract), so cutting the keys to 32 bits keeps the order
-    const int rc = key_bits <= 32 ? run_passes<uint32_t>(code, n, k, passes, order, inverse, w, stream)
-                                  : run_passes<uint64_t>(code, n, k, passes, order, inverse, w, stream);
+    const int rc = key_bits <= 32 ? run_passes<uint32_t>(code, n, k, passes, order, inverse, sorted_keys, w, stream)
+                                  : run_passes<uint64_t>(code, n, k, passes, order, inverse, sorted_keys, w, stream);
     if (rc != PTV3_OK) return rc;
     PTV3_RETURN_LAUNCH();
+}
+
+extern "C" int ptv3_argsort(const int64_t* code, int64_t n, int k, int key_bits, int64_t* order,
+                            int64_t* inverse, void* workspace, size_t workspace_bytes,
+                            void* stream_) {
+    return ptv3_argsort_keys(code, n, k, key_bits, order, inverse, nullptr, workspace, workspace_bytes,
+                             (hipStream_t)stream_);
 }

@@ -129,10 +129,8 @@ __global__ __launch_bounds__(256) void vh_fill_kernel(VoxelHash h, int64_t cap) 
     }
 }
 
-__global__ __launch_bounds__(256) void vh_insert_kernel(const int32_t* __restrict__ indices, int64_t n, VoxelHash h) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int4 v = ((const int4*)indices)[i];
+__device__ __forceinline__ void vh_insert(const int4* __restrict__ indices, int64_t i, const VoxelHash& h) {
+    const int4 v = indices[i];
     const int xs = v.y + VH_SHIFT, ys = v.z + VH_SHIFT, zs = v.w + VH_SHIFT;
     const uint64_t key = vh_block_key(v.x, xs >> 2, ys >> 2, zs >> 2);
     const int bit = (xs & 3) << 4 | (ys & 3) << 2 | (zs & 3);
@@ -147,6 +145,11 @@ __global__ __launch_bounds__(256) void vh_insert_kernel(const int32_t* __restric
         }
         slot = (slot + 1) & h.mask;
     }
+}
+
+__global__ __launch_bounds__(256) void vh_insert_kernel(const int32_t* __restrict__ indices, int64_t n, VoxelHash h) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) vh_insert((const int4*)indices, i, h);
 }
 
 // headers for the worst case of one voxel per block at load <= 2/3
