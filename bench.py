@@ -6,7 +6,7 @@ A step is one full PointTransformerV3 forward (default architecture, fp16, eval)
 of 4 synthetic room scenes of ~100k voxelised points each, inputs resident in HBM. Prints one
 JSON line: throughput in points/s, the roofline of the dominant kernel (patch attention,
 MFMA-bound nominally, VALU-bound in fact: both fractions are given) and of the sparse convolutions,
-measured with HIP events around every launch inside the timed region, the CPU oracle timed on
+measured with HIP events around every launch in further loops of the same forwards, the CPU oracle timed on
 this machine's host cores (one of the four scenes, and baseline config 1 in full), and short
 runs of the other baseline configurations (5, 2, 3) after the timed region.
 """
@@ -714,8 +714,9 @@ def main():
             return model(dict(data))
 
     def timed_loop(events):
-        """`steps` forwards back to back between two synchronisations, with HIP events around the launches named."""
-        t = LaunchTimer(events)
+        """`steps` forwards back to back between two synchronisations, with HIP events around the launches named (a
+        launch timer has the forward queued module by module, which is what announces the launches)."""
+        t = LaunchTimer(events) if events != () else None
         ops.set_launch_timer(t)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -729,8 +730,7 @@ def main():
     model.overlap_index_prologue = not args.no_overlap
     for _ in range(args.warmup):
         step()
-    # the timed region: events around the launches of the dominant kernel only
-    timer, wall, out = timed_loop({"patch_attn"})
+    _, wall, out = timed_loop(())   # the timed region
     assert torch.isfinite(out.feat.float()).all()
     plain_ms = None
     if model.overlap_index_prologue:
@@ -738,12 +738,13 @@ def main():
         model.overlap_index_prologue = False
         for _ in range(2):
             step()
-        plain_ms = timed_loop({"patch_attn"})[1] / args.steps * 1e3
-    # and once more (plain schedule) with events around every launch the operators announce: the convolutions and the
-    # index kernels against their rooflines, measured inside the forward but outside the timed region
+        plain_ms = timed_loop(())[1] / args.steps * 1e3
+    # and twice more (plain schedule) with events around the attention's launches, then around every launch the operators
+    # announce: the kernels against their rooflines, measured inside the forward but outside the timed region
     model.overlap_index_prologue = False
     for _ in range(2):
         step()
+    timer = timed_loop({"patch_attn"})[0]
     every, every_wall, _ = timed_loop(None)
     model.overlap_index_prologue = not args.no_overlap
 

@@ -688,6 +688,60 @@ int ptv3_index_lists_bytes(void *state, const int32_t *want, size_t *bytes);
 int ptv3_index_lists(void *state, const int32_t *want, void *lists, size_t lists_bytes, void *stream);
 const ptv3_level *ptv3_index_levels(const void *state);
 
+/* ---- The feature side of a forward in one call (model.py:972-982 over an index of ptv3_index_*) -------------------
+ * Weights are pointers to device memory in `dtype` (the rows' dtype; BatchNorm statistics in float when stats_f32).
+ * Covers the default architecture: blocks of 32 / 64 / 128 / 256 / 512 channels with hidden = 4 x channels, affine
+ * LayerNorms of one eps, biases everywhere, BatchNorm + exact GELU behind stem, poolings and unpoolings. In half
+ * precision stem_w has its input channels padded to a multiple of 16 (ptv3_pad_rows over the weight's rows), and the
+ * packed copies are those of ptv3_subm_conv_pack_weight (conv_packed, 32 / 64 / 128 channels), ptv3_mlp_pack_weights_batch
+ * (mlp_packed from 128 channels on, proj_packed at 128 and 256, head_packed = xCPE Linear + qkv at 128).
+ * Level l needs the lists ptv3_conv_form names for its blocks' channels (float: pairs), level 0 also the 5x5x5 lists.
+ * stage_out: NULL, or per stage a buffer for the encoder stage's rows (or NULL in it); out: the decoder's (n, channels)
+ * rows. Queues only; allocates and keeps nothing. */
+typedef struct ptv3_linear_w { const void *w, *b; int32_t in, out; } ptv3_linear_w;
+typedef struct ptv3_norm_w { const void *g, *b; float eps; int32_t reserved; } ptv3_norm_w;
+typedef struct ptv3_bn_w { const void *mean, *var, *g, *b; float eps; int32_t stats_f32; } ptv3_bn_w;
+typedef struct ptv3_block_w {
+    int32_t channels, heads, row, reserved;   /* row: which order row the attention reads along */
+    float scale, reserved2;
+    const void *conv_w, *conv_b, *conv_packed;
+    ptv3_linear_w cpe, qkv, proj, fc1, fc2;
+    ptv3_norm_w ln_cpe, ln1, ln2;
+    const void *mlp_packed, *proj_packed, *head_packed;
+} ptv3_block_w;
+typedef struct ptv3_stage_w {
+    int32_t channels, dec_channels, n_enc, n_dec, pool_reduce, reserved;
+    const ptv3_block_w *enc, *dec;
+    ptv3_linear_w pool, up, up_skip;          /* pool: in front of this stage; up: from the stage below to this one */
+    ptv3_bn_w pool_bn, up_bn, up_skip_bn;
+} ptv3_stage_w;
+typedef struct ptv3_net {
+    int32_t dtype, n_stages, decoder, stem_in;
+    int32_t patch[PTV3_MAX_LEVELS];
+    const void *stem_w;
+    ptv3_bn_w stem_bn;
+    ptv3_stage_w stage[PTV3_MAX_LEVELS];
+} ptv3_net;
+/* jobs that bring the copies of a net's weights up to date: casts first, then the padded stem and the packed copies */
+typedef struct ptv3_refresh {
+    int32_t dtype, n_cast, n_conv, n_mlp;
+    int64_t cast_blocks, conv_blocks, mlp_blocks;
+    const ptv3_cast_job *cast;
+    const ptv3_pack_job *conv;
+    const ptv3_mlp_pack_job *mlp;
+    const void *stem_src;                     /* NULL: no stem copy */
+    void *stem_dst;
+    int64_t stem_rows;
+    int32_t stem_in, stem_padded;
+} ptv3_refresh;
+
+int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels);
+int ptv3_pad_rows(const void *x, int x_dtype, int64_t n, int c, int padded, void *out, int out_dtype, void *stream);
+size_t ptv3_features_bytes(const ptv3_net *net, const ptv3_level *levels, void *const *stage_out);
+int ptv3_features_fwd(const ptv3_net *net, const ptv3_level *levels, const void *feat, int feat_dtype,
+                      void *const *stage_out, void *out, void *workspace, size_t workspace_bytes, void *stream);
+int ptv3_net_refresh(const ptv3_refresh *jobs, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -122,6 +122,11 @@ SIGNATURES = {
     "ptv3_index_lists_bytes": (_i32, [_vp, _vp, _vp]),
     "ptv3_index_lists": (_i32, [_vp, _vp, _vp, _sz, _vp]),
     "ptv3_index_levels": (_vp, [_vp]),
+    "ptv3_conv_form": (_i32, [_i64, _i64, _i32]),
+    "ptv3_pad_rows": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _i32, _vp]),
+    "ptv3_features_bytes": (_sz, [_vp, _vp, _vp]),
+    "ptv3_features_fwd": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp]),
+    "ptv3_net_refresh": (_i32, [_vp, _vp]),
     "ptv3_layer_norm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _f32, _i32, _vp, _vp, _vp]),
 }
 

@@ -101,11 +101,12 @@ class Index:
         return buf[at:at + size].view(dtype).view(shape)
 
 
-def build(layout, grid_coord, offset, batch, orders, shuffle, want):
+def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None):
     """Queues the whole index on the current stream and waits for what the host has to know. grid_coord (n, 3) int32 and
     offset (scenes,) int64 contiguous, batch (n,) int64 or None; orders: names of the curves, shuffled with torch's CPU
     generator when `shuffle` (and per pooling module as layout.shuffles says, in the order the modules would draw);
-    want(level number, Level) -> PTV3_LISTS_* flags of the level once its pair count is known."""
+    want(level number, Level) -> PTV3_LISTS_* flags of the level once its pair count is known;
+    between() is called behind the first stage's launches, while the host would wait for them."""
     lib = _lib.load()
     stream = ops._stream()
     dev = grid_coord.device
@@ -124,6 +125,8 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want):
     check(lib.ptv3_index_begin(state, ctypes.byref(cfg), grid_coord.data_ptr(), None if batch is None else batch.data_ptr(),
                                offset.data_ptr(), out.batch.data_ptr(), first.data_ptr(), nbytes, slot.ptr, seq, stream),
           "ptv3_index_begin")
+    if between is not None:
+        between()
     check(lib.ptv3_index_wait(slot.ptr, 0, seq, stream), "ptv3_index_wait")
     out.grid_max = words[_SLOT_DATA:_SLOT_DATA + 3]
     out.offset_host = words[_SLOT_ENDS:_SLOT_ENDS + nb]

@@ -1,0 +1,479 @@
+"""The inference forward of a PointTransformerV3 from native code: the index by ptv3_index_* (levels.py), the features by one
+ptv3_features_fwd call over a description of the model's weights (ptv3_net). Module by module the same launches cost the
+host about 5 ms per forward; described once and queued natively they cost about a tenth of that.
+
+An Engine describes one model in one compute dtype. It takes the default architecture (see Engine._describe); any other
+model, a model with hooks or submodules in training mode, and inputs that carry tables of their own go through the
+modules (model.py), which stay the definition of the result."""
+import ctypes
+import weakref
+
+import numpy as np
+import torch
+import torch.nn as nn
+
+from . import _lib, levels, ops
+from .modules import (MLP, Block, DropPath, Embedding, LayerNorm, PointSequential, SerializedAttention, SerializedPooling,
+                      SerializedUnpooling)
+from .point import AttrDict, Point, batch2offset
+from .sparse import SparseConvTensor, SubMConv3d
+
+_i32, _i64, _f32, _ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
+
+
+class _Linear(ctypes.Structure):
+    _fields_ = [("w", _ptr), ("b", _ptr), ("cin", _i32), ("cout", _i32)]
+
+
+class _Norm(ctypes.Structure):
+    _fields_ = [("g", _ptr), ("b", _ptr), ("eps", _f32), ("reserved", _i32)]
+
+
+class _Bn(ctypes.Structure):
+    _fields_ = [("mean", _ptr), ("var", _ptr), ("g", _ptr), ("b", _ptr), ("eps", _f32), ("stats_f32", _i32)]
+
+
+class _Block(ctypes.Structure):
+    _fields_ = [("channels", _i32), ("heads", _i32), ("row", _i32), ("reserved", _i32), ("scale", _f32), ("reserved2", _f32),
+                ("conv_w", _ptr), ("conv_b", _ptr), ("conv_packed", _ptr),
+                ("cpe", _Linear), ("qkv", _Linear), ("proj", _Linear), ("fc1", _Linear), ("fc2", _Linear),
+                ("ln_cpe", _Norm), ("ln1", _Norm), ("ln2", _Norm),
+                ("mlp_packed", _ptr), ("proj_packed", _ptr), ("head_packed", _ptr)]
+
+
+class _Stage(ctypes.Structure):
+    _fields_ = [("channels", _i32), ("dec_channels", _i32), ("n_enc", _i32), ("n_dec", _i32), ("pool_reduce", _i32),
+                ("reserved", _i32), ("enc", _ptr), ("dec", _ptr), ("pool", _Linear), ("up", _Linear), ("up_skip", _Linear),
+                ("pool_bn", _Bn), ("up_bn", _Bn), ("up_skip_bn", _Bn)]
+
+
+class _Net(ctypes.Structure):
+    _fields_ = [("dtype", _i32), ("n_stages", _i32), ("decoder", _i32), ("stem_in", _i32), ("patch", _i32 * levels.MAX_LEVELS),
+                ("stem_w", _ptr), ("stem_bn", _Bn), ("stage", _Stage * levels.MAX_LEVELS)]
+
+
+class _Refresh(ctypes.Structure):
+    _fields_ = [("dtype", _i32), ("n_cast", _i32), ("n_conv", _i32), ("n_mlp", _i32), ("cast_blocks", _i64),
+                ("conv_blocks", _i64), ("mlp_blocks", _i64), ("cast", _ptr), ("conv", _ptr), ("mlp", _ptr),
+                ("stem_src", _ptr), ("stem_dst", _ptr), ("stem_rows", _i64), ("stem_in", _i32), ("stem_padded", _i32)]
+
+
+class Unsupported(Exception):
+    """The model is not one the native forward covers."""
+
+
+def _need(ok, why):
+    if not ok:
+        raise Unsupported(why)
+
+
+CHANNELS = (32, 64, 128, 256, 512)
+CONV_PACKED = (32, 64, 128)     # widths whose convolutions may take a tile form
+
+# keys a caller may have put on the input that stand for work this path would do itself
+_OWN_KEYS = ("serialized_code", "serialized_order", "serialized_inverse", "serialized_depth", "sparse_shape",
+             "sparse_conv_feat", "pad", "unpad", "cu_seqlens_key", "pooling_inverse", "pooling_parent")
+
+
+class Structure:
+    """What of a model's modules the native paths rely on, and whether it still holds."""
+
+    def __init__(self, model):
+        self.modules = list(model.modules())
+        _need(all("forward" not in m.__dict__ for m in self.modules), "a module's forward was replaced")
+        self.children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
+        self.slots, self.tensors = [], []
+        for m in self.modules:
+            for name, p in m._parameters.items():
+                if p is not None:
+                    self.slots.append((m._parameters, name))
+                    self.tensors.append(p)
+            if isinstance(m, nn.BatchNorm1d) and m.running_mean is not None:
+                for name in ("running_mean", "running_var"):
+                    self.slots.append((m._buffers, name))
+                    self.tensors.append(m._buffers[name])
+        self.pointers = [d[k].data_ptr() for d, k in self.slots]
+        # modules whose training flag changes what an evaluation computes
+        self.flagged = [m for m in self.modules if isinstance(m, nn.BatchNorm1d)
+                        or (isinstance(m, nn.Dropout) and m.p > 0) or (isinstance(m, DropPath) and m.drop_prob > 0)
+                        or (isinstance(m, SerializedAttention) and m.attn_drop > 0)]
+
+    def hooked(self):
+        hooks = torch.nn.modules.module
+        return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks
+                    or any(m._forward_hooks or m._forward_pre_hooks for m in self.modules))
+
+    def same(self):
+        """The module tree and the places of all weights are those this was made from."""
+        return (all(d[k] is c for d, k, c in self.children)
+                and [d[k].data_ptr() for d, k in self.slots] == self.pointers)
+
+
+class Engine:
+    def __init__(self, model, dtype):
+        self.structure = Structure(model)
+        self.dtype = dtype
+        self.device = self.structure.tensors[0].device
+        params = [t for t in self.structure.tensors if isinstance(t, nn.Parameter)]
+        kinds = {p.dtype for p in params}
+        _need(kinds == {dtype} or (kinds == {torch.float32} and dtype != torch.float32), "weights of several dtypes")
+        _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() for p in self.structure.tensors), "placement")
+        self._keep = []
+        self._casts, self._cast_out, self._cast_at = {}, None, 0
+        self._jobs_conv, self._jobs_mlp = [], []
+        self._cast = kinds != {dtype}
+        if self._cast:
+            total = sum(-(-p.numel() // 128) * 128 for p in params)
+            self._cast_out = torch.empty(total, dtype=dtype, device=self.device)
+        self._describe(model)
+        self._finish_jobs()
+
+    # ---- pointers -------------------------------------------------------------------------------------------------
+    def _p(self, t):
+        """Address of a parameter in the compute dtype: its own, or that of its copy (casts)."""
+        if t is None:
+            return None
+        if not self._cast:
+            return t.data_ptr()
+        held = self._casts.get(t)
+        if held is None:
+            held = self._casts[t] = self._cast_out.data_ptr() + self._cast_at * self._cast_out.element_size()
+            self._cast_at += -(-t.numel() // 128) * 128
+        return held
+
+    def _linear(self, m, cin=None, cout=None, bias=True):
+        _need(type(m) is nn.Linear and (m.bias is not None or not bias), "Linear")
+        _need((cin is None or m.in_features == cin) and (cout is None or m.out_features == cout), "Linear shape")
+        return _Linear(self._p(m.weight), self._p(m.bias), m.in_features, m.out_features)
+
+    def _norm(self, m, c):
+        _need(type(m) is LayerNorm and m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
+        return _Norm(self._p(m.weight), self._p(m.bias), m.eps, 0)
+
+    def _bn(self, m, c):
+        _need(type(m) is nn.BatchNorm1d and m.track_running_stats and m.running_mean is not None and m.num_features == c
+              and m.weight is not None and m.bias is not None, "BatchNorm1d")
+        stats = m.running_mean.dtype
+        _need(m.running_var.dtype == stats and stats in (torch.float32, self.dtype), "BatchNorm1d statistics")
+        return _Bn(m.running_mean.data_ptr(), m.running_var.data_ptr(), self._p(m.weight), self._p(m.bias), m.eps,
+                   int(stats == torch.float32))
+
+    @staticmethod
+    def _gelu(m):
+        _need(type(m) is nn.GELU and m.approximate == "none", "activation")
+
+    def _packed(self, elements):
+        t = torch.empty(elements, dtype=self.dtype, device=self.device)
+        self._keep.append(t)
+        return t.data_ptr()
+
+    def _block(self, b, c):
+        _need(type(b) is Block and b.pre_norm and b.channels == c and c in CHANNELS, "Block")
+        for seq, kind, count in ((b.cpe, PointSequential, 3), (b.norm1, PointSequential, 1), (b.norm2, PointSequential, 1),
+                                 (b.mlp, PointSequential, 1)):
+            _need(type(seq) is kind and len(seq) == count, "Block parts")
+        conv, lin, attn, mlp = b.cpe[0], b.cpe[1], b.attn, b.mlp[0]
+        _need(type(conv) is SubMConv3d and conv.kernel_size == 3 and conv.in_channels == conv.out_channels == c
+              and conv.bias is not None, "xCPE convolution")
+        _need(type(attn) is SerializedAttention and attn.enable_flash and attn.rpe is None and attn.channels == c
+              and c % attn.num_heads == 0, "attention")
+        _need(type(mlp) is MLP, "MLP")
+        self._gelu(mlp.act)
+        d = _Block(channels=c, heads=attn.num_heads, row=attn.order_index, scale=attn.scale)
+        d.conv_w, d.conv_b = self._p(conv.weight), self._p(conv.bias)
+        d.cpe, d.qkv, d.proj = self._linear(lin, c, c), self._linear(attn.qkv, c, 3 * c), self._linear(attn.proj, c, c)
+        d.fc1, d.fc2 = self._linear(mlp.fc1, c, 4 * c), self._linear(mlp.fc2, 4 * c, c)
+        d.ln_cpe, d.ln1, d.ln2 = self._norm(b.cpe[2], c), self._norm(b.norm1[0], c), self._norm(b.norm2[0], c)
+        _need(b.cpe[2].eps == b.norm1[0].eps, "LayerNorm eps")
+        if self.dtype != torch.float32:
+            if c in CONV_PACKED:
+                d.conv_packed = self._packed(27 * c * c)
+                self._jobs_conv.append((d.conv_w, d.conv_packed, c, 27))
+            if c >= 128:
+                d.mlp_packed = self._packed(8 * c * c)
+                self._jobs_mlp.append((d.fc1.w, d.fc2.w, d.mlp_packed, c, 0))
+            if c in (128, 256):
+                d.proj_packed = self._packed(c * c)
+                self._jobs_mlp.append((d.proj.w, 0, d.proj_packed, c, 1))
+            if c == 128:
+                d.head_packed = self._packed(4 * c * c)
+                self._jobs_mlp.append((d.cpe.w, 0, d.head_packed, c, 1))
+                self._jobs_mlp.append((d.qkv.w, 0, d.head_packed + c * c * 2, c, 3))
+        return d
+
+    def _describe(self, model):
+        """ptv3_net of the model; Unsupported where it is not the default architecture."""
+        S = model.num_stages
+        orders = list(model.order)
+        _need(2 <= S <= levels.MAX_LEVELS and 1 <= len(orders) <= levels.MAX_ORDERS, "stages")
+        _need(type(model.embedding) is Embedding and type(model.enc) is PointSequential, "stem")
+        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=S, decoder=int(not model.cls_mode))
+        stem = model.embedding.stem
+        _need(type(stem) is PointSequential and list(stem._modules) == ["conv", "norm", "act"], "stem")
+        conv = stem[0]
+        _need(type(conv) is SubMConv3d and conv.kernel_size == 5 and conv.bias is None, "stem convolution")
+        self._gelu(stem[2])
+        net.stem_in = conv.in_channels
+        net.stem_w = self._p(conv.weight)
+        net.stem_bn = self._bn(stem[1], conv.out_channels)
+        self._refresh = r = _Refresh(dtype=net.dtype)
+        if self.dtype != torch.float32:
+            padded = -(-conv.in_channels // 16) * 16
+            r.stem_rows, r.stem_in, r.stem_padded = conv.out_channels * 125, conv.in_channels, padded
+            r.stem_src = net.stem_w
+            r.stem_dst = net.stem_w = self._packed(r.stem_rows * padded)
+        _need(list(model.enc._modules) == [f"enc{s}" for s in range(S)], "encoder")
+        slot_rows, convs, patches, shuffles = [], [], [], []
+        c_below = conv.out_channels
+        for s in range(S):
+            stage = model.enc[s]
+            _need(type(stage) is PointSequential, "encoder stage")
+            parts = list(stage._modules.items())
+            d = net.stage[s]
+            if s:
+                _need(parts and parts[0][0] == "down" and type(parts[0][1]) is SerializedPooling, "pooling")
+                down = parts.pop(0)[1]
+                _need(down.norm is not None and len(down.norm) == 1 and down.act is not None and len(down.act) == 1, "pooling norm")
+                _need(down.plan_kernel_sizes == (3,) and down.stride == model.stride[s - 1], "pooling")
+                self._gelu(down.act[0])
+                d.pool = self._linear(down.proj, c_below, down.out_channels)
+                d.pool_bn, d.pool_reduce = self._bn(down.norm[0], down.out_channels), ops.REDUCE_OPS[down.reduce]
+                _need(down.out_channels in CHANNELS and (not model.cls_mode or down.traceable), "pooling width")
+                shuffles.append(down.shuffle_orders)
+                c_below = down.out_channels
+            enc = [b for _, b in parts]
+            dec = []
+            d.channels, d.n_enc = c_below, len(enc)
+            if not model.cls_mode and s < S - 1:
+                dstage = model.dec._modules.get(f"dec{s}")
+                _need(type(dstage) is PointSequential and list(dstage._modules)[:1] == ["up"], "decoder stage")
+                up, dec = dstage[0], list(dstage._modules.values())[1:]
+                _need(type(up) is SerializedUnpooling and not up.traceable, "unpooling")
+                for seq in (up.proj, up.proj_skip):
+                    _need(type(seq) is PointSequential and len(seq) == 3, "unpooling")
+                    self._gelu(seq[2])
+                d.dec_channels = up.proj_skip[0].out_features
+                d.up, d.up_skip = self._linear(up.proj[0], None, d.dec_channels), self._linear(up.proj_skip[0], c_below, d.dec_channels)
+                d.up_bn, d.up_skip_bn = self._bn(up.proj[1], d.dec_channels), self._bn(up.proj_skip[1], d.dec_channels)
+                _need(d.dec_channels in CHANNELS, "decoder width")
+                d.n_dec = len(dec)
+            for attr, bs, c in (("enc", enc, c_below), ("dec", dec, d.dec_channels)):
+                if bs:
+                    arr = (_Block * len(bs))(*[self._block(b, c) for b in bs])
+                    self._keep.append(arr)
+                    setattr(d, attr, ctypes.addressof(arr))
+            _need(c_below in CHANNELS, "width")
+            both = enc + dec
+            sizes = [b.attn.patch_size for b in both]
+            # the tables of a level are made for the patch size of the first attention that reaches it
+            patch = sizes[0] if sizes else 1024
+            _need(all(v >= patch for v in sizes), "patch sizes that shrink from the encoder to the decoder")
+            net.patch[s] = patch
+            patches.append(patch)
+            slot_rows.append([b.attn.order_index for b in both])
+            convs.append([(b.channels, b.channels) for b in both])
+        if not model.cls_mode:
+            below = net.stage[S - 1].channels
+            for s in reversed(range(S - 1)):
+                _need(net.stage[s].up.cin == below, "decoder widths")
+                below = net.stage[s].dec_channels
+            self.out_channels = below
+            _need(list(model.dec._modules) == [f"dec{s}" for s in reversed(range(S - 1))], "decoder")
+        self.layout = levels.Layout(len(orders), model.stride, patches, slot_rows, convs, True, shuffles,
+                                    only_pads0=not model.cls_mode)
+        half = self.dtype != torch.float32
+        form = _lib.load().ptv3_conv_form
+        widths = [sorted({c for c, _ in cs}) for cs in convs]
+
+        def want(level, v):
+            flags = levels.PAIRS5 if level == 0 else 0
+            for c in widths[level]:
+                flags |= levels.TILES if half and form(v.n, v.n_pairs, c) else levels.PAIRS
+            return flags
+
+        self.want = want
+
+    def _finish_jobs(self):
+        lib, r = _lib.load(), self._refresh
+
+        def table(rows, dtype):
+            if not rows:
+                return None
+            t = torch.frombuffer(bytearray(np.array(rows, dtype=dtype).tobytes()), dtype=torch.uint8).to(self.device)
+            self._keep.append(t)
+            return t.data_ptr()
+
+        rows, at = [], 0
+        for t, dst in self._casts.items():
+            rows.append((t.data_ptr(), dst, 1, 1, t.numel(), 0, at))
+            at += lib.ptv3_cast_params_blocks(1, 1, t.numel(), 0)
+        r.cast, r.n_cast, r.cast_blocks = table(rows, ops._CAST_JOB), len(rows), at
+        rows, at = [], 0
+        for src, dst, c, taps in self._jobs_conv:
+            rows.append((src, dst, c, taps, at))
+            at += lib.ptv3_subm_conv_pack_weight_blocks(c, taps)
+        r.conv, r.n_conv, r.conv_blocks = table(rows, ops._PACK_JOB), len(rows), at
+        rows, at = [], 0
+        for w1, w2, dst, c, k in self._jobs_mlp:
+            rows.append((w1, w2, dst, c, k, at))
+            at += k * lib.ptv3_linear_pack_weights_blocks(c) if k else lib.ptv3_mlp_pack_weights_blocks(c)
+        r.mlp, r.n_mlp, r.mlp_blocks = table(rows, ops._MLP_PACK_JOB), len(rows), at
+
+    # ---- one forward ----------------------------------------------------------------------------------------------
+    def forward(self, model, data):
+        """The Point that PointTransformerV3.forward returns for these inputs (see Inputs in `accepts`)."""
+        lib = _lib.load()
+        feat = data["feat"].contiguous()
+        point = Point.__new__(Point)
+        dict.update(point, data)
+        point._ensure_grid_coord()
+        grid = point["grid_coord"].to(torch.int32).contiguous()
+        batch = point.get("batch")
+        if "offset" not in point:
+            point["offset"] = batch2offset(batch)
+        offset = point["offset"].to(torch.int64).contiguous()
+        if batch is not None:
+            batch = batch.to(torch.int64).contiguous()
+
+        def refresh():
+            # whoever writes the parameters behind autograd's back leaves no trace on them: every derived copy is
+            # redone once per forward
+            _lib.check(lib.ptv3_net_refresh(ctypes.byref(self._refresh), ops._stream()), "ptv3_net_refresh")
+
+        args = (self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want)
+        if model.overlap_index_prologue:
+            if model._prologue_state is None or model._prologue_state.device != feat.device:
+                model._prologue_state = ops.PrologueOverlap(feat.device)
+            refresh()
+            with model._prologue_state.scope():
+                index = levels.build(*args)
+        else:
+            model._prologue_state = None
+            index = levels.build(*args, between=refresh)
+        lv = index.levels
+        n = feat.shape[0]
+        stage_out, rows = None, None
+        if model.cls_mode:
+            rows = [torch.empty((lv[s].n, self.net.stage[s].channels), dtype=self.dtype, device=feat.device)
+                    for s in range(self.net.n_stages)]
+            stage_out = (_ptr * len(rows))(*[t.data_ptr() for t in rows])
+            out = rows[-1]
+        else:
+            out = torch.empty((n, self.out_channels), dtype=self.dtype, device=feat.device)
+        nbytes = lib.ptv3_features_bytes(ctypes.byref(self.net), lv, stage_out)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=feat.device)
+        _lib.check(lib.ptv3_features_fwd(ctypes.byref(self.net), lv, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype], stage_out,
+                                         None if model.cls_mode else out.data_ptr(), ws.data_ptr(), nbytes, ops._stream()),
+                   "ptv3_features_fwd")
+        point["batch"] = index.batch
+        self._fill(point, index, 0, rows[0] if model.cls_mode else out)
+        if model.cls_mode:
+            for s in range(1, len(rows)):
+                point = self._pooled(point, index, s, rows[s])
+        if model._prologue_state is not None:
+            model._prologue_state.forward_queued(point)
+        return point
+
+    def _fill(self, point, index, s, feat):
+        """The keys of a level that serialization, sparsify and the attention put on its Point."""
+        v, k = index.levels[s], index.n_orders
+        i64, i32 = torch.int64, torch.int32
+        point["feat"] = feat
+        if s == 0:
+            point["serialized_code"], point["serialized_order"], point["serialized_inverse"] = index.code, index.order, index.inverse
+            point["_grid_max_host"] = index.grid_max
+        point["serialized_depth"] = v.depth
+        point["_offset_host"] = index.level_offsets[s]
+        point["_sparse_indices"] = indices = index.tensor(v.indices, (v.n, 4), i32, "tables" if s else "first")
+        point["sparse_shape"] = shape = [g + 96 for g in point["_grid_max_host"]]
+        point["sparse_conv_feat"] = SparseConvTensor(feat, indices, shape, len(index.level_offsets[s]))
+        if v.pad:
+            point["pad"], point["unpad"] = index.tensor(v.pad, (v.n_pad,), i64), index.tensor(v.unpad, (v.n,), i64)
+        point["cu_seqlens_key"] = index.tensor(v.cu, (v.n_seq + 1,), i32)
+        point["_pad_patch"] = self.net.patch[s]
+
+    def _pooled(self, parent, index, s, feat):
+        v, k = index.levels[s], index.n_orders
+        i64 = torch.int64
+        idx_ptr = index.tensor(v.idx_ptr, (v.n + 1,), i64)
+        members = parent["serialized_order"][0]
+        shift = parent["serialized_depth"] - v.depth
+        point = Point.__new__(Point)
+        if "coord" in parent:
+            point["coord"] = ops.segment_reduce(parent["coord"].float(), members, idx_ptr, "mean")
+        dict.update(
+            point, grid_coord=index.tensor(v.grid, (v.n, 3), torch.int32), serialized_code=index.tensor(v.code, (k, v.n), i64),
+            serialized_order=index.tensor(v.order, (k, v.n), i64), serialized_inverse=index.tensor(v.inverse, (k, v.n), i64),
+            batch=index.tensor(v.batch, (v.n,), i64),
+            offset=index.tensor(v.offset, (len(index.level_offsets[s]),), i64, "first"), _pool_members=(members, idx_ptr),
+            _grid_max_host=[g >> shift for g in parent["_grid_max_host"]],
+            pooling_inverse=index.tensor(v.cluster, (index.levels[s - 1].n,), i64), pooling_parent=parent)
+        for key in ("condition", "context"):
+            if key in parent:
+                point[key] = parent[key]
+        self._fill(point, index, s, feat)
+        return point
+
+
+_ENGINES = weakref.WeakKeyDictionary()   # model -> {compute dtype: Engine, or None where the model is not covered}
+
+
+def _compute_dtype(feat, weight):
+    """The dtype the model's rows would have, or None where the modules mix dtypes."""
+    if torch.is_autocast_enabled():
+        dt = torch.get_autocast_dtype("cuda")
+        return dt if weight.dtype in (torch.float32, dt) and dt != torch.float32 else None
+    return feat.dtype if feat.dtype == weight.dtype else None
+
+
+def engine_for(model, data):
+    """The Engine that computes model(data), or None: the modules do."""
+    if (model.training or torch.is_grad_enabled() or ops._LAUNCH_TIMER is not None or ops.Readback.blocking
+            or type(data) not in (dict, AttrDict, Point)):
+        return None
+    feat = data.get("feat")
+    if not isinstance(feat, torch.Tensor) or not feat.is_cuda or feat.dim() != 2 or feat.shape[0] < 1 or feat.dtype not in ops.DTYPE_CODES:
+        return None
+    if any(k in data for k in _OWN_KEYS) or any(k.startswith("_") for k in data) or not ("offset" in data or "batch" in data):
+        return None
+    where = data.get("grid_coord", data.get("coord"))
+    ends = data.get("offset", data.get("batch"))
+    if not (isinstance(where, torch.Tensor) and where.is_cuda and where.shape[0] == feat.shape[0] and ends.is_cuda and ends.numel()):
+        return None
+    weight = model.embedding.stem._modules["conv"].weight
+    dtype = _compute_dtype(feat, weight)
+    if dtype not in ops.DTYPE_CODES or feat.shape[1] != weight.shape[-1]:
+        return None
+    held = _ENGINES.setdefault(model, {})
+    key = (dtype, model.cls_mode)
+    engine = held.get(key)
+    if engine is not None and not engine.structure.same():
+        engine = None
+        held.pop(key)
+    if engine is None and key not in held:
+        try:
+            engine = Engine(model, dtype)
+            _need(engine.structure.same(), "structure")
+            held[key] = engine
+        except Unsupported as e:
+            held[key] = _Refused(model, str(e))
+            return None
+    if isinstance(engine, _Refused):
+        return None
+    if engine.structure.hooked() or any(m.training for m in engine.structure.flagged):
+        return None
+    return engine
+
+
+class _Refused:
+    """A model the native forward does not cover, remembered until its structure or weights move."""
+
+    def __init__(self, model, why):
+        self.why = why
+        try:
+            self.structure = Structure(model)
+        except Unsupported:
+            self.structure = self
+
+    def same(self):
+        return True

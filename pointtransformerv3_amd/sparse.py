@@ -7,7 +7,7 @@ import weakref
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import _lib, ops
 
 
 class SparseConvTensor:
@@ -79,12 +79,6 @@ class SubMConv3d(nn.Module):
     # (no pair-matrix round trip, but MFMA work for every tap); a 2 cm surface scan goes from 0.05
     # at full resolution to 0.5 at the coarsest level, where the two forms measure about equal
     PAIR_MODE_MAX_DENSITY = 0.6
-    # from this many pairs per voxel on, the tile form (sums kept on chip, no pair matrix through memory)
-    # measured faster than the pair form at 64 and 128 channels; sparser levels stay on the pair form
-    TILE_MODE_MIN_PAIRS_PER_VOXEL = 4.0
-    # 32 and 64 channels: the sparse tile form (work in proportion to the pairs) up to this many pairs per voxel;
-    # measured faster than both other forms from 2.5 to 10 pairs per voxel, a full grid (27) is the tile form's case
-    SPARSE_MODE_MAX_PAIRS_PER_VOXEL = 14.0
 
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, padding=0, dilation=1,
                  groups=1, bias=True, indice_key=None):
@@ -119,13 +113,9 @@ class SubMConv3d(nn.Module):
     def _tile_form(self, plan, cin, cout):
         """Which of the two forms that walk the plan's tile lists takes this convolution in half precision:
         "sparse", "tile" or None (pair or dense form)."""
-        if self.kernel_size != 3 or cin != cout or plan.n >= (1 << 24):
+        if self.kernel_size != 3 or cin != cout:
             return None
-        if cin in ops.CONV_SPARSE_CHANNELS and plan.n_pairs <= self.SPARSE_MODE_MAX_PAIRS_PER_VOXEL * plan.n:
-            return "sparse"
-        if cin in ops.CONV_TILE_CHANNELS and plan.n_pairs >= self.TILE_MODE_MIN_PAIRS_PER_VOXEL * plan.n:
-            return "tile"
-        return None
+        return (None, "sparse", "tile")[_lib.load().ptv3_conv_form(plan.n, plan.n_pairs, cin)]
 
     def lists_ahead(self, x):
         """Makes (and caches on x, under this module's indice_key) the index lists the half-precision forward of this

@@ -1,0 +1,93 @@
+"""The natively queued inference forward against the same model's modules."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV, rel_err
+
+pytestmark = pytest.mark.gpu
+
+KW = dict(enc_depths=(1, 1, 2, 1, 1), dec_depths=(1, 2, 1, 1), enc_patch_size=(256,) * 5, dec_patch_size=(256,) * 4)
+
+
+def _inputs(seed, sizes, dtype, grid=0.04):
+    from pointtransformerv3_amd import synthetic
+    d = synthetic.collate([synthetic.room_scene(n, seed + i, grid) for i, n in enumerate(sizes)])
+    feat = torch.from_numpy(synthetic.room_features(d["coord"], seed)).to(DEV).to(dtype)
+    return dict(feat=feat, coord=torch.from_numpy(d["coord"]).to(DEV), grid_coord=torch.from_numpy(d["grid_coord"]).to(DEV),
+                offset=torch.from_numpy(d["offset"]).to(DEV))
+
+
+def _both(model, data, monkeypatch, amp=None):
+    from pointtransformerv3_amd import native
+    taken, real = [], native.engine_for
+    outs = []
+    for use in (True, False):
+        monkeypatch.setattr(native, "engine_for",
+                            (lambda m, d: taken.append(real(m, d)) or taken[-1]) if use else (lambda m, d: None))
+        torch.manual_seed(9)
+        with torch.inference_mode(), torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            outs.append(model(dict(data)))
+    monkeypatch.setattr(native, "engine_for", real)
+    assert taken[0] is not None, "the native path was not taken"
+    return outs
+
+
+@pytest.mark.parametrize("sizes", [(5000,), (9000, 61, 4000), (40,)])
+@pytest.mark.parametrize("dtype,amp", [(torch.float16, None), (torch.bfloat16, None), (torch.float32, None),
+                                       (torch.float32, torch.float16)])
+def test_native_forward_equals_the_modules(dtype, amp, sizes, monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().to(dtype).to(DEV)
+    got, want = _both(model, _inputs(4, sizes, dtype), monkeypatch, amp)
+    assert got.feat.dtype == want.feat.dtype
+    assert torch.equal(got.feat, want.feat)
+    for key in ("batch", "offset", "serialized_code", "serialized_order", "serialized_inverse", "pad", "unpad", "cu_seqlens_key"):
+        assert torch.equal(got[key], want[key]), key
+    assert got.serialized_depth == want.serialized_depth and got.sparse_shape == want.sparse_shape
+    assert torch.equal(got.sparse_conv_feat.indices, want.sparse_conv_feat.indices)
+    assert torch.equal(got.sparse_conv_feat.features, want.feat)
+
+
+def test_native_encoder_only_fills_every_level(monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(cls_mode=True, **KW).eval().half().to(DEV)
+    got, want = _both(model, _inputs(4, (3000, 7000), torch.float16), monkeypatch)
+    depth = 0
+    while True:
+        keys = {k for k in want if isinstance(want[k], torch.Tensor) and not k.startswith("_")}
+        assert keys <= set(got) and got.serialized_depth == want.serialized_depth
+        for key in keys:
+            assert torch.equal(got[key], want[key]), (depth, key)
+        if "pooling_parent" not in want:
+            break
+        got, want, depth = got.pooling_parent, want.pooling_parent, depth + 1
+    assert depth == 4
+
+
+def test_native_forward_follows_changed_weights_and_leaves_changed_models_alone(monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3, native
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().half().to(DEV)
+    data = _inputs(7, (4000,), torch.float16)
+    first = _both(model, data, monkeypatch)[0].feat
+    model.enc.enc2.block0.mlp[0].fc1.weight.data.mul_(1.5)                     # in place, behind autograd's back
+    got, want = _both(model, data, monkeypatch)
+    assert torch.equal(got.feat, want.feat) and not torch.equal(got.feat, first)
+    model.dec.dec1.block0.attn.qkv.weight = torch.nn.Parameter(model.dec.dec1.block0.attn.qkv.weight.data * 0.5)   # another tensor
+    got, want = _both(model, data, monkeypatch)
+    assert torch.equal(got.feat, want.feat)
+    with torch.inference_mode():
+        handle = model.enc.enc1.register_forward_hook(lambda m, a, r: None)    # hooks want the modules to run
+        assert native.engine_for(model, data) is None
+        handle.remove()
+        assert native.engine_for(model, data) is not None
+        assert native.engine_for(model, dict(data, sparse_shape=[1, 2, 3])) is None
+        model.enc.enc1.down.norm[0].train()
+        assert native.engine_for(model, data) is None
+        model.eval()
+        model.dec.dec0.block0.mlp[0].fc1 = torch.nn.Sequential(model.dec.dec0.block0.mlp[0].fc1)   # not the default architecture
+        assert native.engine_for(model, data) is None
+    assert native.engine_for(model, data) is None                              # grad mode: the modules
