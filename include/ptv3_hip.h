@@ -487,8 +487,8 @@ int ptv3_bn_act(const void *x, const void *running_mean, const void *running_var
 
 /* nn.Linear of the wide blocks (model.py:541-545 cpe.1, :450 qkv, :487 proj, :510-512 fc1 + GELU):
  * out = act(x w^T + bias), x (n, k), w (nout, k), bias (nout,) or NULL, out (n, nout), act = exact
- * (erf) GELU when gelu != 0. fp16/bf16, k in {32, 64, 128, 256, 512}, nout a multiple of 32 (PTV3_ESHAPE
- * otherwise: ptv3_linear_any_fwd takes every shape). Tall-and-skinny form: rows held in MFMA operand registers, no loop
+ * (erf) GELU when gelu != 0. fp16/bf16, k in {32, 64, 128, 256, 512} (without the GELU also 96, 192, 384:
+ * the input gradients of the qkv layers), nout a multiple of 32 (PTV3_ESHAPE otherwise: ptv3_linear_any_fwd takes every shape). Tall-and-skinny form: rows held in MFMA operand registers, no loop
  * over memory along k. */
 int ptv3_linear_fwd(const void *x, const void *w, const void *bias, int dtype, int64_t n, int k, int nout,
                     int gelu, void *out, void *stream);
@@ -642,6 +642,9 @@ int ptv3_block_tail_fused(const void *attn, const void *shortcut, const void *w_
 #define PTV3_LISTS_PAIRS 1                  /* 3x3x3: row_ptr, pair_in, pair_slot */
 #define PTV3_LISTS_TILES 2                  /* 3x3x3: tile_tap, tile_pair, vox_taps */
 #define PTV3_LISTS_PAIRS5 4                 /* level 0, 5x5x5 */
+#define PTV3_LISTS_PAIR_OUT 8               /* with PAIRS: the output voxel of every pair (weight gradients) */
+#define PTV3_LISTS_NBR 16                   /* 3x3x3 neighbour map, tap-major (27, n), -1 where there is none */
+#define PTV3_LISTS_PAIR_OUT5 32             /* with PAIRS5 */
 
 typedef struct ptv3_index_cfg {
     int64_t n;                              /* points of level 0 */
@@ -667,6 +670,7 @@ typedef struct ptv3_level {
     int32_t *slot_src[PTV3_MAX_ORDERS], *slot_dst[PTV3_MAX_ORDERS];
     int32_t *tap_ptr, *row_ptr, *pair_in, *pair_slot, *tile_tap, *tile_pair, *vox_taps;
     int32_t *tap_ptr5, *row_ptr5, *pair_in5, *pair_slot5;
+    int32_t *pair_out, *pair_out5, *nbr;
     int32_t tile_voxels, depth;
 } ptv3_level;
 
@@ -741,6 +745,67 @@ size_t ptv3_features_bytes(const ptv3_net *net, const ptv3_level *levels, void *
 int ptv3_features_fwd(const ptv3_net *net, const ptv3_level *levels, const void *feat, int feat_dtype,
                       void *const *stage_out, void *out, void *workspace, size_t workspace_bytes, void *stream);
 int ptv3_net_refresh(const ptv3_refresh *jobs, void *stream);
+
+/* ---- A training step under half-precision autocast: forward and backward of the feature side, one call each -------
+ * (model.py:972-982 in training mode, with what autograd does behind it). Float masters; `dtype` (PTV3_F16 / PTV3_BF16)
+ * copies of the weights are pointers: w as it is, wt transposed (in x out swapped), the convolutions' tap-mirrored weight
+ * and both packed for the tile forms (32 / 64 / 128 channels), the stem's with its inputs padded. Norm parameters in
+ * float, BatchNorm's also in dtype. The residual stream is float, rows between layers are in dtype. Gradients are
+ * written, not accumulated, to `grads` + the g* offsets (floats; a BatchNorm's bias gradient follows its weight's);
+ * `zero` lists the ranges that are summed with atomics (the LayerNorms').
+ * Levels need: tile lists or pair lists as ptv3_conv_form says, below 128 channels pair lists with PAIR_OUT, from 128 on
+ * the neighbour map, level 0 PAIRS5 with PAIR_OUT5. masks: per block, encoder stages then decoder stages from the
+ * bottom, the row factors (n,) in dtype of the attention's and the MLP's stochastic depth, or NULL.
+ * Same forward as ptv3_train_fwd's buffers: acts is kept by the caller until after the backward, which only reads it. */
+typedef struct ptv3_train_linear { const void *w, *wt, *b; int32_t in, out; int64_t gw, gb; } ptv3_train_linear;
+typedef struct ptv3_train_norm { const float *g, *b; float eps; int32_t reserved; int64_t gg, gb; } ptv3_train_norm;
+typedef struct ptv3_train_bn {
+    const float *g, *b;
+    const void *g16, *b16;
+    float *running_mean, *running_var;        /* updated by the forward, or NULL */
+    float eps, momentum;
+    int64_t gg;
+} ptv3_train_bn;
+typedef struct ptv3_train_block {
+    int32_t channels, heads, row, reserved;
+    float scale, reserved2;
+    const void *conv_w, *conv_b, *conv_mirror, *conv_packed, *conv_mirror_packed;
+    int64_t g_conv_w, g_conv_b;
+    ptv3_train_linear cpe, qkv, proj, fc1, fc2;
+    ptv3_train_norm ln_cpe, ln1, ln2;
+} ptv3_train_block;
+typedef struct ptv3_train_stage {
+    int32_t channels, dec_channels, n_enc, n_dec, pool_reduce, reserved;
+    const ptv3_train_block *enc, *dec;
+    ptv3_train_linear pool, up, up_skip;
+    ptv3_train_bn pool_bn, up_bn, up_skip_bn;
+} ptv3_train_stage;
+typedef struct ptv3_train_stem {
+    const void *w;                            /* (out, 125, cin_padded) in dtype */
+    int32_t cin, cin_padded;
+    int64_t gw;
+    ptv3_train_bn bn;
+} ptv3_train_stem;
+typedef struct ptv3_zero_range { int64_t at, count, first_block; } ptv3_zero_range;   /* blocks of 256 floats */
+typedef struct ptv3_train_net {
+    int32_t dtype, n_stages;
+    int32_t patch[PTV3_MAX_LEVELS];
+    ptv3_train_stem stem;
+    const ptv3_zero_range *zero;              /* device array */
+    int32_t n_zero, reserved;
+    int64_t zero_blocks;
+    ptv3_train_stage stage[PTV3_MAX_LEVELS];
+} ptv3_train_net;
+
+int ptv3_zero_ranges(float *base, const ptv3_zero_range *ranges, int count, int64_t blocks, void *stream);
+int ptv3_cut_rows(const float *x, int64_t rows, int from, int to, float *out, void *stream);   /* first `to` of `from` columns */
+int ptv3_train_bytes(const ptv3_train_net *net, const ptv3_level *levels, size_t *acts, size_t *fwd_scratch,
+                     size_t *bwd_scratch);
+int ptv3_train_fwd(const ptv3_train_net *net, const ptv3_level *levels, const void *feat, int feat_dtype,
+                   const void *const *masks, void *acts, void *scratch, size_t scratch_size, float *out, void *stream);
+int ptv3_train_bwd(const ptv3_train_net *net, const ptv3_level *levels, const void *dout, int dout_dtype,
+                   const void *const *masks, const void *acts, void *scratch, size_t scratch_size, float *grads,
+                   void *stream);
 
 #ifdef __cplusplus
 }

@@ -127,6 +127,11 @@ SIGNATURES = {
     "ptv3_features_bytes": (_sz, [_vp, _vp, _vp]),
     "ptv3_features_fwd": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_net_refresh": (_i32, [_vp, _vp]),
+    "ptv3_zero_ranges": (_i32, [_vp, _vp, _i32, _i64, _vp]),
+    "ptv3_cut_rows": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp]),
+    "ptv3_train_bytes": (_i32, [_vp, _vp, _vp, _vp, _vp]),
+    "ptv3_train_fwd": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp, _vp]),
+    "ptv3_train_bwd": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp, _vp]),
     "ptv3_layer_norm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _f32, _i32, _vp, _vp, _vp]),
 }
 

@@ -31,6 +31,7 @@
 #include <hip/hip_fp16.h>
 
 #include "common.h"
+#include "outer.h"
 
 namespace {
 
@@ -483,20 +484,30 @@ __global__ __launch_bounds__(256) void outer_rows_wide_kernel(const T* __restric
 
 // out[i] = sum over the splits' slabs (of `stride` floats, the first `total` of them summed): a work-group takes 32 neighbouring values, its 8 thread rows share
 // out the splits (four loads in flight each) and meet in LDS
+// The sums of several results share a launch (ptv3_slab_sums): alone, a small layer's is mostly the launch.
 // With tap_ptr (pair-list ranges) the value i = (m * taps + tap) * k_total + k of the first result only has the
 // ranges its tap's list reaches: ceil(pairs of the tap / rows_per_split) of them; the others were never written.
-__global__ __launch_bounds__(256) void slab_sum_kernel(const float* __restrict__ slabs, int64_t stride, int64_t total,
-                                                       int splits, float* __restrict__ out, int64_t first,
-                                                       float* __restrict__ out2, const int32_t* __restrict__ tap_ptr,
-                                                       int taps, int k_total, int64_t rows_per_split) {
+struct SlabJobs {
+    int count;
+    int first_block[SLAB_JOBS + 1];
+    SlabJob job[SLAB_JOBS];
+};
+
+__global__ __launch_bounds__(256) void slab_sum_kernel(SlabJobs jobs) {
     __shared__ float part[8][32];
+    int which = 0;
+    while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.first_block[which + 1]) ++which;
+    const SlabJob& job = jobs.job[which];
     const int e = threadIdx.x % 32, lane_s = threadIdx.x / 32;
-    const int64_t i = (int64_t)blockIdx.x * 32 + e;
+    const int64_t i = (int64_t)((int)blockIdx.x - jobs.first_block[which]) * 32 + e;
+    const float* slabs = job.slabs;
+    const int64_t stride = job.stride;
+    int splits = job.splits;
     float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
-    if (i < total) {
-        if (tap_ptr && i < first) {
-            const int t = (int)(((uint32_t)i / (uint32_t)k_total) % (uint32_t)taps);   // first < 2^31: checked at launch
-            const int64_t have = ((int64_t)tap_ptr[t + 1] - tap_ptr[t] + rows_per_split - 1) / rows_per_split;
+    if (i < job.total) {
+        if (job.tap_ptr && i < job.first) {
+            const int t = (int)(((uint32_t)i / (uint32_t)job.k_total) % (uint32_t)job.taps);   // first < 2^31: checked at launch
+            const int64_t have = ((int64_t)job.tap_ptr[t + 1] - job.tap_ptr[t] + job.rows_per_split - 1) / job.rows_per_split;
             if (have < splits) splits = (int)have;
         }
         int s = lane_s;
@@ -510,11 +521,11 @@ __global__ __launch_bounds__(256) void slab_sum_kernel(const float* __restrict__
     }
     part[lane_s][e] = (v0 + v1) + (v2 + v3);
     __syncthreads();
-    if (lane_s == 0 && i < total) {
+    if (lane_s == 0 && i < job.total) {
         float v = 0.f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) v += part[k][e];
-        if (i < first) out[i] = v; else out2[i - first] = v;   // a slab's tail goes to the second result
+        if (i < job.first) job.out[i] = v; else job.out2[i - job.first] = v;   // a slab's tail goes to the second result
     }
 }
 
@@ -914,6 +925,38 @@ __global__ __launch_bounds__(256) void scaled_add_kernel(AnyRows skip, AnyRows b
     }
 }
 
+// a + b * scale_in in float and, times scale_out, in half precision from one pass: a block's residual sum and the half
+// copy the next convolution reads; going back, a block's output gradient and its branch's (times the stochastic-depth
+// factor).
+__global__ __launch_bounds__(256) void two_sums_kernel(AnyRows a, AnyRows b, AnyRows scale_in, AnyRows scale_out, int64_t n, int c,
+                                                       float* __restrict__ out32, AnyRowsOut out16) {
+    const int64_t groups = n * (c / 8);
+    for (int64_t gi = (int64_t)blockIdx.x * 256 + threadIdx.x; gi < groups; gi += (int64_t)gridDim.x * 256) {
+        const int64_t off = gi * 8;
+        const Raw8 rb = raw8_load(b.p, b.dtype, off);
+        Raw8 ra = rb;
+        if (a.p) ra = raw8_load(a.p, a.dtype, off);
+        const float mi = scale_in.p ? load1_any(scale_in.p, scale_in.dtype, off / c) : 1.f;
+        const float mo = scale_out.p ? load1_any(scale_out.p, scale_out.dtype, off / c) : 1.f;
+        float v[8];
+        raw8_floats(rb, b.dtype, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] *= mi;
+        if (a.p) {
+            float av[8];
+            raw8_floats(ra, a.dtype, av);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] += av[i];
+        }
+        if (out32) Row8<float>::store(out32 + off, v);
+        if (out16.p) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] *= mo;
+            store8_any(out16.p, out16.dtype, off, v);
+        }
+    }
+}
+
 // ---- BatchNorm1d in training mode (+ exact GELU)
 __device__ __forceinline__ float gelu_grad(float z) {
     const float cdf = 0.5f * (1.f + erff(z * 0.70710678118654752f));
@@ -1180,7 +1223,7 @@ size_t outer_workspace(int64_t n, int m_total, int k_total, int taps) {
 template <typename T, bool GATHER>
 int launch_outer(const void* a, const void* b, int64_t n, int m_total, int k_total, const int32_t* nbr, int taps,
                  float* d, float* colsum, void* workspace, size_t workspace_bytes, hipStream_t stream,
-                 const int32_t* tap_ptr = nullptr, const int32_t* pair_in = nullptr) {
+                 const int32_t* tap_ptr = nullptr, const int32_t* pair_in = nullptr, SlabJob* defer = nullptr) {
     const int side = outer_side(m_total, k_total);
     const int64_t bm = ptv3_ceil_div(m_total, side), bk = ptv3_ceil_div(k_total, side);
     int64_t splits, rows;
@@ -1200,12 +1243,11 @@ int launch_outer(const void* a, const void* b, int64_t n, int m_total, int k_tot
     else
         hipLaunchKernelGGL((outer_rows_kernel<T, GATHER>), grid, dim3(256), 0, stream, (const T*)a, (const T*)b, n,
                            m_total, k_total, nbr, tap_ptr, pair_in, taps, (int)splits, rows, stride, slabs, cols);
-    if (splits > 1) {
-        if (tap_ptr && count >= (1ll << 31)) return PTV3_EINVAL;
-        const int64_t total = colsum ? stride : count;
-        hipLaunchKernelGGL(slab_sum_kernel, dim3((unsigned)ptv3_ceil_div(total, 32)), dim3(256), 0, stream,
-                           (const float*)slabs, stride, total, (int)splits, d, count, colsum, tap_ptr, taps, k_total, rows);
-    }
+    if (tap_ptr && count >= (1ll << 31)) return PTV3_EINVAL;
+    SlabJob job = {(const float*)slabs, stride, colsum ? stride : count, splits > 1 ? (int)splits : 0, d, count, colsum,
+                   tap_ptr, taps, k_total, rows};
+    if (defer) *defer = job;
+    else if (job.splits) return ptv3_slab_sums(&job, 1, stream);
     PTV3_RETURN_LAUNCH();
 }
 
@@ -1237,6 +1279,52 @@ int launch_segment_bwd(const void* src, const void* out, const void* dout, int c
 }
 
 }  // namespace
+
+int ptv3_slab_sums(const SlabJob* jobs, int count, hipStream_t stream) {
+    for (int at = 0; at < count;) {
+        SlabJobs t = {};
+        int blocks = 0;
+        for (; at < count && t.count < SLAB_JOBS; ++at) {
+            if (!jobs[at].splits) continue;
+            const int64_t b = ptv3_ceil_div(jobs[at].total, 32);
+            if (b + blocks >= (1ll << 31)) return PTV3_EINVAL;
+            t.first_block[t.count] = blocks;
+            t.job[t.count++] = jobs[at];
+            blocks += (int)b;
+        }
+        t.first_block[t.count] = blocks;
+        if (t.count) hipLaunchKernelGGL(slab_sum_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, t);
+    }
+    PTV3_RETURN_LAUNCH();
+}
+
+int ptv3_linear_wgrad_slabs(const void* x, const void* dout, int dtype, int64_t n, int k, int nout, float* dweight, float* dbias,
+                            void* workspace, size_t workspace_bytes, SlabJob* job, hipStream_t stream) {
+    if (dtype == PTV3_F16)
+        return launch_outer<_Float16, false>(dout, x, n, nout, k, nullptr, 1, dweight, dbias, workspace, workspace_bytes, stream,
+                                             nullptr, nullptr, job);
+    return launch_outer<__bf16, false>(dout, x, n, nout, k, nullptr, 1, dweight, dbias, workspace, workspace_bytes, stream,
+                                       nullptr, nullptr, job);
+}
+
+int ptv3_subm_conv_wgrad_slabs(const void* feat, const void* dout, int dtype, int64_t n, int cin, int cout, const int32_t* nbr,
+                               const int32_t* tap_ptr, const int32_t* pair_in, int taps, float* dweight, float* dbias,
+                               void* workspace, size_t workspace_bytes, SlabJob* job, hipStream_t stream) {
+    if (dtype == PTV3_F16)
+        return launch_outer<_Float16, true>(dout, feat, n, cout, cin, nbr, taps, dweight, dbias, workspace, workspace_bytes, stream,
+                                            tap_ptr, pair_in, job);
+    return launch_outer<__bf16, true>(dout, feat, n, cout, cin, nbr, taps, dweight, dbias, workspace, workspace_bytes, stream,
+                                      tap_ptr, pair_in, job);
+}
+
+int ptv3_two_sums(const void* a, int a_dtype, const void* b, int b_dtype, const void* scale_in, const void* scale_out,
+                  int scale_dtype, int64_t n, int c, void* out32, void* out16, int out16_dtype, hipStream_t stream) {
+    const int64_t blocks = ptv3_ceil_div(n * (c / 8), 256);
+    hipLaunchKernelGGL(two_sums_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, stream, AnyRows{a, a_dtype},
+                       AnyRows{b, b_dtype}, AnyRows{scale_in, scale_dtype}, AnyRows{scale_out, scale_dtype}, n, c, (float*)out32,
+                       AnyRowsOut{out16, out16_dtype});
+    PTV3_RETURN_LAUNCH();
+}
 
 static bool wgrad_on_mfma(int dtype, int cin, int cout) {
     return dtype != PTV3_F32 && cin % 8 == 0 && cout % 8 == 0;

@@ -415,6 +415,7 @@ struct ListLevel {
     int32_t *tap_ptr, *row_ptr, *pair_in, *pair_slot, *tile_tap;
     uint32_t *tile_pair, *vox_taps;
     int32_t *tap_ptr5, *row_ptr5, *pair_in5, *pair_slot5;
+    int32_t *pair_out, *pair_out5, *nbr;
 };
 
 struct ListArgs {
@@ -577,6 +578,7 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
     __shared__ uint32_t hslot[8][GT];
     __shared__ uint32_t stage_q[STAGE];
     __shared__ int32_t stage_in[STAGE], stage_slot[STAGE];
+    __shared__ uint8_t stage_vox[STAGE];
     const int l = list_level(a);
     const ListLevel& v = a.lv[l];
     const int g = (int)blockIdx.x - a.first_block[l], tid = threadIdx.x, lane = tid % PTV3_WAVE, wave = tid / PTV3_WAVE;
@@ -604,7 +606,8 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
     };
 
     auto make = [&](uint64_t flo, uint64_t fhi, int taps, int edge, const int32_t* tap_ptr, const uint32_t* tap_off,
-                    const uint32_t* row_off, int32_t* row_ptr, int32_t* pair_in, int32_t* pair_slot, bool pairs, bool tiles) {
+                    const uint32_t* row_off, int32_t* row_ptr, int32_t* pair_in, int32_t* pair_slot, int32_t* pair_out, int32_t* nbr,
+                    bool pairs, bool tiles) {
         for (int e = tid; e < 256; e += GT) (&mask[0][0])[e] = 0;
         for (int t = tid; t < taps; t += GT) tap_base[t] = pairs ? (uint32_t)tap_ptr[t] + tap_off[(int64_t)g * taps + t] : 0u;
         const uint32_t cnt = (uint32_t)(__popcll(flo) + __popcll(fhi));
@@ -648,6 +651,9 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
             if (tiles && v.vox_taps) v.vox_taps[i] = (uint32_t)flo;
         }
         const bool staged = total <= (uint32_t)STAGE;
+        if (nbr && live)
+            for (int t = 0; t < taps; ++t)
+                if (!((flo >> t) & 1ull)) nbr[(int64_t)t * v.n + i] = -1;
         uint32_t slot = slot0;
         uint64_t f0 = flo, f1 = fhi;
         while (f0 | f1) {
@@ -657,12 +663,18 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
             const int32_t src = source(t / (edge * edge) - edge / 2, (t / edge) % edge - edge / 2, t % edge - edge / 2);
             const uint32_t rank = (uint32_t)__popcll(mask[wave][t] & below) + (wave ? (uint32_t)__popcll(mask[0][t]) : 0u);
             const uint32_t q = tap_base[t] + rank, e = tap_start[t] + rank;
+            if (nbr) nbr[(int64_t)t * v.n + i] = src;
             if (staged) {
-                stage_q[e] = pairs ? q : (uint32_t)tid;
+                stage_q[e] = q;
                 stage_in[e] = src;
                 stage_slot[e] = (int32_t)slot;
+                stage_vox[e] = (uint8_t)tid;
             } else {
-                if (pairs) { pair_in[q] = src; pair_slot[q] = (int32_t)slot; }
+                if (pairs) {
+                    pair_in[q] = src;
+                    pair_slot[q] = (int32_t)slot;
+                    if (pair_out) pair_out[q] = (int32_t)i;
+                }
                 if (tiles) v.tile_pair[base + e] = (uint32_t)tid << 24 | (uint32_t)src;
             }
             ++slot;
@@ -670,35 +682,26 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
         if (staged) {
             __syncthreads();
             for (uint32_t e = tid; e < total; e += GT) {
+                const int32_t src = stage_in[e];
+                const uint32_t vox = stage_vox[e];
                 if (pairs) {
                     const uint32_t q = stage_q[e];
-                    pair_in[q] = stage_in[e];
+                    pair_in[q] = src;
                     pair_slot[q] = stage_slot[e];
-                } else if (tiles) {
-                    v.tile_pair[base + e] = stage_q[e] << 24 | (uint32_t)stage_in[e];
+                    if (pair_out) pair_out[q] = (int32_t)((int64_t)g * v.group + vox);
                 }
-            }
-            if (pairs && tiles) {   // second list of the same pairs: the voxel inside the tile follows from the slot's owner
-                __syncthreads();
-                uint64_t h0 = flo;
-                while (h0) {
-                    const int t = __builtin_ctzll(h0);
-                    h0 &= h0 - 1;
-                    const uint32_t rank = (uint32_t)__popcll(mask[wave][t] & below) + (wave ? (uint32_t)__popcll(mask[0][t]) : 0u);
-                    stage_q[tap_start[t] + rank] = (uint32_t)tid;
-                }
-                __syncthreads();
-                for (uint32_t e = tid; e < total; e += GT) v.tile_pair[base + e] = stage_q[e] << 24 | (uint32_t)stage_in[e];
+                if (tiles) v.tile_pair[base + e] = vox << 24 | (uint32_t)src;
             }
         }
         __syncthreads();
     };
     if (KS == 5 && (v.want & PTV3_LISTS_PAIRS5))
-        make(lo, hi, TAPS5, 5, v.tap_ptr5, v.tap5, v.row5, v.row_ptr5, v.pair_in5, v.pair_slot5, true, false);
+        make(lo, hi, TAPS5, 5, v.tap_ptr5, v.tap5, v.row5, v.row_ptr5, v.pair_in5, v.pair_slot5,
+             v.pair_out5, nullptr, true, false);
     const bool pairs = v.want & PTV3_LISTS_PAIRS, tiles = v.want & PTV3_LISTS_TILES;
-    if (pairs || tiles)
+    if (pairs || tiles || v.nbr)
         make(KS == 5 ? (uint64_t)inner_taps(lo, hi) : lo, 0, TAPS3, 3, v.tap_ptr, v.tap, v.row, pairs ? v.row_ptr : nullptr,
-             v.pair_in, v.pair_slot, pairs, tiles);
+             v.pair_in, v.pair_slot, pairs ? v.pair_out : nullptr, v.nbr, pairs, tiles);
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------------
@@ -1025,12 +1028,14 @@ size_t carve_lists(State& s, const int32_t* want, void* base) {
         v.want = want[l];
         v.row_ptr = v.pair_in = v.pair_slot = v.tile_tap = nullptr;
         v.tile_pair = v.vox_taps = nullptr;
-        v.row_ptr5 = v.pair_in5 = v.pair_slot5 = nullptr;
+        v.row_ptr5 = v.pair_in5 = v.pair_slot5 = v.pair_out = v.pair_out5 = v.nbr = nullptr;
         if (want[l] & PTV3_LISTS_PAIRS) {
             v.row_ptr = c.take<int32_t>(v.n + 1);
             v.pair_in = c.take<int32_t>(out.n_pairs);
             v.pair_slot = c.take<int32_t>(out.n_pairs);
+            if (want[l] & PTV3_LISTS_PAIR_OUT) v.pair_out = c.take<int32_t>(out.n_pairs);
         }
+        if (want[l] & PTV3_LISTS_NBR) v.nbr = c.take<int32_t>(TAPS3 * v.n);
         if (want[l] & PTV3_LISTS_TILES) {
             v.tile_tap = c.take<int32_t>((size_t)v.groups * TILE_WORDS);
             v.tile_pair = c.take<uint32_t>(out.n_pairs);
@@ -1040,6 +1045,7 @@ size_t carve_lists(State& s, const int32_t* want, void* base) {
             v.row_ptr5 = c.take<int32_t>(v.n + 1);
             v.pair_in5 = c.take<int32_t>(out.n_pairs5);
             v.pair_slot5 = c.take<int32_t>(out.n_pairs5);
+            if (want[l] & PTV3_LISTS_PAIR_OUT5) v.pair_out5 = c.take<int32_t>(out.n_pairs5);
         }
     }
     return c.off;
@@ -1179,6 +1185,9 @@ extern "C" int ptv3_index_lists(void* state, const int32_t* want, void* lists, s
         o.row_ptr5 = v.row_ptr5;
         o.pair_in5 = v.pair_in5;
         o.pair_slot5 = v.pair_slot5;
+        o.pair_out = v.pair_out;
+        o.pair_out5 = v.pair_out5;
+        o.nbr = v.nbr;
         o.tile_voxels = v.group;
     }
     PTV3_RETURN_LAUNCH();

@@ -274,6 +274,8 @@ int launch_linear(const void* x, const void* w, const void* bias, LinBn bn, int6
     // without GELU, and at 512 inputs where the x fragments alone need 128 registers, the 8-wave shape is faster
     if constexpr (K == 256 && ACT != ACT_NONE)
         return launch_linear_shape<T, K, ACT, BN, 16, 32>(x, w, bias, bn, n, nout, out, aux, stream);
+    if constexpr (K % 64 != 0 && K > 64)   // 96 inputs: rows staged 32 channels at a time
+        return launch_linear_shape<T, K, ACT, BN, 8, 32>(x, w, bias, bn, n, nout, out, aux, stream);
     return launch_linear_shape<T, K, ACT, BN, 8, 64>(x, w, bias, bn, n, nout, out, aux, stream);
 }
 
@@ -293,6 +295,15 @@ int dispatch_linear(const void* x, const void* w, const void* bias, const LinBn*
             default: return launch_linear<T, K, ACT_GELU_GRAD, false>(x, w, bias, none, n, nout, out, aux, stream);   \
         }                                                                                                             \
     }
+    // the input gradients of the qkv layers at 32, 64 and 128 channels read 3 C inputs: plain layers only
+#define PTV3_LIN3(T, K) \
+    if (k == K && !bn && act == ACT_NONE) return launch_linear<T, K, ACT_NONE, false>(x, w, bias, none, n, nout, out, aux, stream);
+    if (dtype == PTV3_F16) {
+        PTV3_LIN3(_Float16, 96) PTV3_LIN3(_Float16, 192) PTV3_LIN3(_Float16, 384)
+    } else {
+        PTV3_LIN3(__bf16, 96) PTV3_LIN3(__bf16, 192) PTV3_LIN3(__bf16, 384)
+    }
+#undef PTV3_LIN3
     if (dtype == PTV3_F16) {
         PTV3_LIN(_Float16, 32) PTV3_LIN(_Float16, 64) PTV3_LIN(_Float16, 128) PTV3_LIN(_Float16, 256) PTV3_LIN(_Float16, 512)
     } else {
@@ -379,7 +390,8 @@ int check_linear(int dtype, int64_t n, int k, int nout) {
 
 extern "C" int ptv3_linear_fwd(const void* x, const void* w, const void* bias, int dtype, int64_t n, int k, int nout,
                                int gelu, void* out, void* stream_) {
-    const int rc = check_linear(dtype, n, k, nout);
+    const bool plain3 = !gelu && (k == 96 || k == 192 || k == 384);
+    const int rc = check_linear(dtype, n, plain3 ? 128 : k, nout);
     if (rc != PTV3_OK) return rc;
     if (n == 0) return PTV3_OK;
     if (!x || !w || !out) return PTV3_EINVAL;

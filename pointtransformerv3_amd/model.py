@@ -7,7 +7,7 @@ import torch.nn as nn
 
 from .modules import (MLP, Block, DropPath, Embedding, LayerNorm, PDNorm, PointModule, PointSequential,  # noqa: F401
                       SerializedAttention, SerializedPooling, SerializedUnpooling)
-from . import native, ops
+from . import native, native_train, ops
 from .point import Point, batch2offset, offset2batch, offset2bincount  # noqa: F401
 from .sparse import SparseConvTensor, SubMConv3d  # noqa: F401
 
@@ -149,7 +149,8 @@ class PointTransformerV3(PointModule):
         # under no_grad) leaves no trace on them: the derived copies (half-precision casts of float masters,
         # the tile convolutions' packed weights) are redone once per forward, in evaluation as well
         ops.invalidate_casts()
-        engine = native.engine_for(self, data_dict)   # inference of the default architecture: queued from native code
+        # the default architecture, in inference or training under autocast, is queued from native code
+        engine = native.engine_for(self, data_dict) or native_train.engine_for(self, data_dict)
         if engine is not None:
             return engine.forward(self, data_dict)
         point = self._index_prologue(data_dict)

@@ -81,6 +81,8 @@ class Structure:
     def __init__(self, model):
         self.modules = list(model.modules())
         _need(all("forward" not in m.__dict__ for m in self.modules), "a module's forward was replaced")
+        self.hooks = [d for m in self.modules for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
+                                                        m._backward_pre_hooks)]
         self.children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
         self.slots, self.tensors = [], []
         for m in self.modules:
@@ -100,13 +102,138 @@ class Structure:
 
     def hooked(self):
         hooks = torch.nn.modules.module
-        return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks
-                    or any(m._forward_hooks or m._forward_pre_hooks for m in self.modules))
+        return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks or hooks._global_backward_hooks
+                    or hooks._global_backward_pre_hooks or any(self.hooks))
 
     def same(self):
         """The module tree and the places of all weights are those this was made from."""
         return (all(d[k] is c for d, k, c in self.children)
                 and [d[k].data_ptr() for d, k in self.slots] == self.pointers)
+
+
+def _check_gelu(m):
+    _need(type(m) is nn.GELU and m.approximate == "none", "activation")
+
+
+def _check_block(b, c):
+    _need(type(b) is Block and b.pre_norm and b.channels == c and c in CHANNELS, "Block")
+    for seq, count in ((b.cpe, 3), (b.norm1, 1), (b.norm2, 1), (b.mlp, 1), (b.drop_path, 1)):
+        _need(type(seq) is PointSequential and len(seq) == count, "Block parts")
+    conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
+    _need(type(conv) is SubMConv3d and conv.kernel_size == 3 and conv.in_channels == conv.out_channels == c
+          and conv.bias is not None, "xCPE convolution")
+    _need(type(attn) is SerializedAttention and attn.enable_flash and attn.rpe is None and attn.channels == c
+          and c % attn.num_heads == 0, "attention")
+    _need(type(mlp) is MLP and type(b.drop_path[0]) in (DropPath, nn.Identity), "MLP")
+    _check_gelu(mlp.act)
+    _need(all(type(m) is LayerNorm for m in (b.cpe[2], b.norm1[0], b.norm2[0])) and b.cpe[2].eps == b.norm1[0].eps, "LayerNorm")
+
+
+class Parts:
+    """The modules of a model of the default architecture, stage by stage; Unsupported for any other."""
+
+    class Stage:
+        down = up = None
+        enc = dec = ()
+        channels = dec_channels = patch = 0
+
+    def __init__(self, model):
+        S = model.num_stages
+        self.n_orders = len(list(model.order))
+        _need(2 <= S <= levels.MAX_LEVELS and 1 <= self.n_orders <= levels.MAX_ORDERS, "stages")
+        _need(type(model.embedding) is Embedding and type(model.enc) is PointSequential, "stem")
+        stem = model.embedding.stem
+        _need(type(stem) is PointSequential and list(stem._modules) == ["conv", "norm", "act"], "stem")
+        self.stem_conv, self.stem_bn = stem[0], stem[1]
+        _need(type(stem[0]) is SubMConv3d and stem[0].kernel_size == 5 and stem[0].bias is None, "stem convolution")
+        _check_gelu(stem[2])
+        _need(list(model.enc._modules) == [f"enc{s}" for s in range(S)], "encoder")
+        self.stages, below = [], stem[0].out_channels
+        for s in range(S):
+            stage, st = model.enc[s], Parts.Stage()
+            _need(type(stage) is PointSequential, "encoder stage")
+            parts = list(stage._modules.items())
+            if s:
+                _need(parts and parts[0][0] == "down" and type(parts[0][1]) is SerializedPooling, "pooling")
+                st.down = parts.pop(0)[1]
+                _need(st.down.norm is not None and len(st.down.norm) == 1 and st.down.act is not None and len(st.down.act) == 1
+                      and st.down.plan_kernel_sizes == (3,) and st.down.stride == model.stride[s - 1]
+                      and (not model.cls_mode or st.down.traceable) and st.down.proj.in_features == below, "pooling")
+                _check_gelu(st.down.act[0])
+                below = st.down.out_channels
+            st.channels, st.enc = below, [b for _, b in parts]
+            if not model.cls_mode and s < S - 1:
+                dstage = model.dec._modules.get(f"dec{s}")
+                _need(type(dstage) is PointSequential and list(dstage._modules)[:1] == ["up"], "decoder stage")
+                st.up, st.dec = dstage[0], list(dstage._modules.values())[1:]
+                _need(type(st.up) is SerializedUnpooling and not st.up.traceable, "unpooling")
+                for seq in (st.up.proj, st.up.proj_skip):
+                    _need(type(seq) is PointSequential and len(seq) == 3 and type(seq[0]) is nn.Linear, "unpooling")
+                    _check_gelu(seq[2])
+                st.dec_channels = st.up.proj_skip[0].out_features
+                _need(st.dec_channels in CHANNELS and st.up.proj[0].out_features == st.dec_channels, "decoder width")
+            _need(below in CHANNELS, "width")
+            for bs, c in ((st.enc, st.channels), (st.dec, st.dec_channels)):
+                for b in bs:
+                    _check_block(b, c)
+            sizes = [b.attn.patch_size for b in (*st.enc, *st.dec)]
+            # the tables of a level are made for the patch size of the first attention that reaches it
+            st.patch = sizes[0] if sizes else 1024
+            _need(all(v >= st.patch for v in sizes), "patch sizes that shrink from the encoder to the decoder")
+            self.stages.append(st)
+        if not model.cls_mode:
+            _need(list(model.dec._modules) == [f"dec{s}" for s in reversed(range(S - 1))], "decoder")
+            width = self.stages[S - 1].channels
+            for s in reversed(range(S - 1)):
+                _need(self.stages[s].up.proj[0].in_features == width, "decoder widths")
+                width = self.stages[s].dec_channels
+
+    def layout(self, model):
+        both = [[*st.enc, *st.dec] for st in self.stages]
+        return levels.Layout(self.n_orders, model.stride, [st.patch for st in self.stages],
+                             [[b.attn.order_index for b in bs] for bs in both],
+                             [[(b.channels, b.channels) for b in bs] for bs in both], True,
+                             [st.down.shuffle_orders for st in self.stages[1:]], only_pads0=not model.cls_mode)
+
+    def widths(self):
+        """Per level, the channel counts of its 3x3x3 convolutions."""
+        return [sorted({b.channels for b in (*st.enc, *st.dec)}) for st in self.stages]
+
+
+def job_table(rows, dtype, device):
+    """A job table of the batch kernels in device memory, or None when it is empty."""
+    if not rows:
+        return None
+    return torch.frombuffer(bytearray(np.array(rows, dtype=dtype).tobytes()), dtype=torch.uint8).to(device)
+
+
+def coordinates(point):
+    """(grid_coord int32, offset int64, batch int64 or None), contiguous, from a Point fresh from the caller."""
+    point._ensure_grid_coord()
+    batch = point.get("batch")
+    if "offset" not in point:
+        point["offset"] = batch2offset(batch)
+    return (point["grid_coord"].to(torch.int32).contiguous(), point["offset"].to(torch.int64).contiguous(),
+            None if batch is None else batch.to(torch.int64).contiguous())
+
+
+def fill_point(point, index, s, feat, patch):
+    """The keys of a level that serialization, sparsify and the attention put on its Point."""
+    v = index.levels[s]
+    i64, i32 = torch.int64, torch.int32
+    point["feat"] = feat
+    if s == 0:
+        point["serialized_code"], point["serialized_order"], point["serialized_inverse"] = index.code, index.order, index.inverse
+        point["_grid_max_host"] = index.grid_max
+    point["serialized_depth"] = v.depth
+    point["_offset_host"] = index.level_offsets[s]
+    point["_sparse_indices"] = indices = index.tensor(v.indices, (v.n, 4), i32, "tables" if s else "first")
+    point["sparse_shape"] = shape = [g + 96 for g in point["_grid_max_host"]]
+    point["sparse_conv_feat"] = SparseConvTensor(feat, indices, shape, len(index.level_offsets[s]))
+    if v.pad:
+        point["pad"], point["unpad"] = index.tensor(v.pad, (v.n_pad,), i64), index.tensor(v.unpad, (v.n,), i64)
+    point["cu_seqlens_key"] = index.tensor(v.cu, (v.n_seq + 1,), i32)
+    point["_pad_patch"] = patch
 
 
 class Engine:
@@ -158,33 +285,18 @@ class Engine:
         return _Bn(m.running_mean.data_ptr(), m.running_var.data_ptr(), self._p(m.weight), self._p(m.bias), m.eps,
                    int(stats == torch.float32))
 
-    @staticmethod
-    def _gelu(m):
-        _need(type(m) is nn.GELU and m.approximate == "none", "activation")
-
     def _packed(self, elements):
         t = torch.empty(elements, dtype=self.dtype, device=self.device)
         self._keep.append(t)
         return t.data_ptr()
 
     def _block(self, b, c):
-        _need(type(b) is Block and b.pre_norm and b.channels == c and c in CHANNELS, "Block")
-        for seq, kind, count in ((b.cpe, PointSequential, 3), (b.norm1, PointSequential, 1), (b.norm2, PointSequential, 1),
-                                 (b.mlp, PointSequential, 1)):
-            _need(type(seq) is kind and len(seq) == count, "Block parts")
         conv, lin, attn, mlp = b.cpe[0], b.cpe[1], b.attn, b.mlp[0]
-        _need(type(conv) is SubMConv3d and conv.kernel_size == 3 and conv.in_channels == conv.out_channels == c
-              and conv.bias is not None, "xCPE convolution")
-        _need(type(attn) is SerializedAttention and attn.enable_flash and attn.rpe is None and attn.channels == c
-              and c % attn.num_heads == 0, "attention")
-        _need(type(mlp) is MLP, "MLP")
-        self._gelu(mlp.act)
         d = _Block(channels=c, heads=attn.num_heads, row=attn.order_index, scale=attn.scale)
         d.conv_w, d.conv_b = self._p(conv.weight), self._p(conv.bias)
         d.cpe, d.qkv, d.proj = self._linear(lin, c, c), self._linear(attn.qkv, c, 3 * c), self._linear(attn.proj, c, c)
         d.fc1, d.fc2 = self._linear(mlp.fc1, c, 4 * c), self._linear(mlp.fc2, 4 * c, c)
         d.ln_cpe, d.ln1, d.ln2 = self._norm(b.cpe[2], c), self._norm(b.norm1[0], c), self._norm(b.norm2[0], c)
-        _need(b.cpe[2].eps == b.norm1[0].eps, "LayerNorm eps")
         if self.dtype != torch.float32:
             if c in CONV_PACKED:
                 d.conv_packed = self._packed(27 * c * c)
@@ -203,87 +315,37 @@ class Engine:
 
     def _describe(self, model):
         """ptv3_net of the model; Unsupported where it is not the default architecture."""
-        S = model.num_stages
-        orders = list(model.order)
-        _need(2 <= S <= levels.MAX_LEVELS and 1 <= len(orders) <= levels.MAX_ORDERS, "stages")
-        _need(type(model.embedding) is Embedding and type(model.enc) is PointSequential, "stem")
-        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=S, decoder=int(not model.cls_mode))
-        stem = model.embedding.stem
-        _need(type(stem) is PointSequential and list(stem._modules) == ["conv", "norm", "act"], "stem")
-        conv = stem[0]
-        _need(type(conv) is SubMConv3d and conv.kernel_size == 5 and conv.bias is None, "stem convolution")
-        self._gelu(stem[2])
-        net.stem_in = conv.in_channels
-        net.stem_w = self._p(conv.weight)
-        net.stem_bn = self._bn(stem[1], conv.out_channels)
+        p = Parts(model)
+        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages), decoder=int(not model.cls_mode))
+        net.stem_in = p.stem_conv.in_channels
+        net.stem_w = self._p(p.stem_conv.weight)
+        net.stem_bn = self._bn(p.stem_bn, p.stem_conv.out_channels)
         self._refresh = r = _Refresh(dtype=net.dtype)
         if self.dtype != torch.float32:
-            padded = -(-conv.in_channels // 16) * 16
-            r.stem_rows, r.stem_in, r.stem_padded = conv.out_channels * 125, conv.in_channels, padded
+            padded = -(-p.stem_conv.in_channels // 16) * 16
+            r.stem_rows, r.stem_in, r.stem_padded = p.stem_conv.out_channels * 125, p.stem_conv.in_channels, padded
             r.stem_src = net.stem_w
             r.stem_dst = net.stem_w = self._packed(r.stem_rows * padded)
-        _need(list(model.enc._modules) == [f"enc{s}" for s in range(S)], "encoder")
-        slot_rows, convs, patches, shuffles = [], [], [], []
-        c_below = conv.out_channels
-        for s in range(S):
-            stage = model.enc[s]
-            _need(type(stage) is PointSequential, "encoder stage")
-            parts = list(stage._modules.items())
+        for s, st in enumerate(p.stages):
             d = net.stage[s]
-            if s:
-                _need(parts and parts[0][0] == "down" and type(parts[0][1]) is SerializedPooling, "pooling")
-                down = parts.pop(0)[1]
-                _need(down.norm is not None and len(down.norm) == 1 and down.act is not None and len(down.act) == 1, "pooling norm")
-                _need(down.plan_kernel_sizes == (3,) and down.stride == model.stride[s - 1], "pooling")
-                self._gelu(down.act[0])
-                d.pool = self._linear(down.proj, c_below, down.out_channels)
-                d.pool_bn, d.pool_reduce = self._bn(down.norm[0], down.out_channels), ops.REDUCE_OPS[down.reduce]
-                _need(down.out_channels in CHANNELS and (not model.cls_mode or down.traceable), "pooling width")
-                shuffles.append(down.shuffle_orders)
-                c_below = down.out_channels
-            enc = [b for _, b in parts]
-            dec = []
-            d.channels, d.n_enc = c_below, len(enc)
-            if not model.cls_mode and s < S - 1:
-                dstage = model.dec._modules.get(f"dec{s}")
-                _need(type(dstage) is PointSequential and list(dstage._modules)[:1] == ["up"], "decoder stage")
-                up, dec = dstage[0], list(dstage._modules.values())[1:]
-                _need(type(up) is SerializedUnpooling and not up.traceable, "unpooling")
-                for seq in (up.proj, up.proj_skip):
-                    _need(type(seq) is PointSequential and len(seq) == 3, "unpooling")
-                    self._gelu(seq[2])
-                d.dec_channels = up.proj_skip[0].out_features
-                d.up, d.up_skip = self._linear(up.proj[0], None, d.dec_channels), self._linear(up.proj_skip[0], c_below, d.dec_channels)
-                d.up_bn, d.up_skip_bn = self._bn(up.proj[1], d.dec_channels), self._bn(up.proj_skip[1], d.dec_channels)
-                _need(d.dec_channels in CHANNELS, "decoder width")
-                d.n_dec = len(dec)
-            for attr, bs, c in (("enc", enc, c_below), ("dec", dec, d.dec_channels)):
+            d.channels, d.n_enc, d.dec_channels, d.n_dec = st.channels, len(st.enc), st.dec_channels, len(st.dec)
+            if st.down is not None:
+                d.pool = self._linear(st.down.proj, None, st.channels)
+                d.pool_bn, d.pool_reduce = self._bn(st.down.norm[0], st.channels), ops.REDUCE_OPS[st.down.reduce]
+            if st.up is not None:
+                d.up, d.up_skip = self._linear(st.up.proj[0]), self._linear(st.up.proj_skip[0], st.channels)
+                d.up_bn, d.up_skip_bn = self._bn(st.up.proj[1], st.dec_channels), self._bn(st.up.proj_skip[1], st.dec_channels)
+            for attr, bs, c in (("enc", st.enc, st.channels), ("dec", st.dec, st.dec_channels)):
                 if bs:
                     arr = (_Block * len(bs))(*[self._block(b, c) for b in bs])
                     self._keep.append(arr)
                     setattr(d, attr, ctypes.addressof(arr))
-            _need(c_below in CHANNELS, "width")
-            both = enc + dec
-            sizes = [b.attn.patch_size for b in both]
-            # the tables of a level are made for the patch size of the first attention that reaches it
-            patch = sizes[0] if sizes else 1024
-            _need(all(v >= patch for v in sizes), "patch sizes that shrink from the encoder to the decoder")
-            net.patch[s] = patch
-            patches.append(patch)
-            slot_rows.append([b.attn.order_index for b in both])
-            convs.append([(b.channels, b.channels) for b in both])
-        if not model.cls_mode:
-            below = net.stage[S - 1].channels
-            for s in reversed(range(S - 1)):
-                _need(net.stage[s].up.cin == below, "decoder widths")
-                below = net.stage[s].dec_channels
-            self.out_channels = below
-            _need(list(model.dec._modules) == [f"dec{s}" for s in reversed(range(S - 1))], "decoder")
-        self.layout = levels.Layout(len(orders), model.stride, patches, slot_rows, convs, True, shuffles,
-                                    only_pads0=not model.cls_mode)
+            net.patch[s] = st.patch
+        self.out_channels = p.stages[0].dec_channels or None
+        self.layout = p.layout(model)
         half = self.dtype != torch.float32
         form = _lib.load().ptv3_conv_form
-        widths = [sorted({c for c, _ in cs}) for cs in convs]
+        widths = p.widths()
 
         def want(level, v):
             flags = levels.PAIRS5 if level == 0 else 0
@@ -297,11 +359,9 @@ class Engine:
         lib, r = _lib.load(), self._refresh
 
         def table(rows, dtype):
-            if not rows:
-                return None
-            t = torch.frombuffer(bytearray(np.array(rows, dtype=dtype).tobytes()), dtype=torch.uint8).to(self.device)
+            t = job_table(rows, dtype, self.device)
             self._keep.append(t)
-            return t.data_ptr()
+            return t.data_ptr() if t is not None else None
 
         rows, at = [], 0
         for t, dst in self._casts.items():
@@ -326,14 +386,7 @@ class Engine:
         feat = data["feat"].contiguous()
         point = Point.__new__(Point)
         dict.update(point, data)
-        point._ensure_grid_coord()
-        grid = point["grid_coord"].to(torch.int32).contiguous()
-        batch = point.get("batch")
-        if "offset" not in point:
-            point["offset"] = batch2offset(batch)
-        offset = point["offset"].to(torch.int64).contiguous()
-        if batch is not None:
-            batch = batch.to(torch.int64).contiguous()
+        grid, offset, batch = coordinates(point)
 
         def refresh():
             # whoever writes the parameters behind autograd's back leaves no trace on them: every derived copy is
@@ -366,31 +419,13 @@ class Engine:
                                          None if model.cls_mode else out.data_ptr(), ws.data_ptr(), nbytes, ops._stream()),
                    "ptv3_features_fwd")
         point["batch"] = index.batch
-        self._fill(point, index, 0, rows[0] if model.cls_mode else out)
+        fill_point(point, index, 0, rows[0] if model.cls_mode else out, self.net.patch[0])
         if model.cls_mode:
             for s in range(1, len(rows)):
                 point = self._pooled(point, index, s, rows[s])
         if model._prologue_state is not None:
             model._prologue_state.forward_queued(point)
         return point
-
-    def _fill(self, point, index, s, feat):
-        """The keys of a level that serialization, sparsify and the attention put on its Point."""
-        v, k = index.levels[s], index.n_orders
-        i64, i32 = torch.int64, torch.int32
-        point["feat"] = feat
-        if s == 0:
-            point["serialized_code"], point["serialized_order"], point["serialized_inverse"] = index.code, index.order, index.inverse
-            point["_grid_max_host"] = index.grid_max
-        point["serialized_depth"] = v.depth
-        point["_offset_host"] = index.level_offsets[s]
-        point["_sparse_indices"] = indices = index.tensor(v.indices, (v.n, 4), i32, "tables" if s else "first")
-        point["sparse_shape"] = shape = [g + 96 for g in point["_grid_max_host"]]
-        point["sparse_conv_feat"] = SparseConvTensor(feat, indices, shape, len(index.level_offsets[s]))
-        if v.pad:
-            point["pad"], point["unpad"] = index.tensor(v.pad, (v.n_pad,), i64), index.tensor(v.unpad, (v.n,), i64)
-        point["cu_seqlens_key"] = index.tensor(v.cu, (v.n_seq + 1,), i32)
-        point["_pad_patch"] = self.net.patch[s]
 
     def _pooled(self, parent, index, s, feat):
         v, k = index.levels[s], index.n_orders
@@ -411,7 +446,7 @@ class Engine:
         for key in ("condition", "context"):
             if key in parent:
                 point[key] = parent[key]
-        self._fill(point, index, s, feat)
+        fill_point(point, index, s, feat, self.net.patch[s])
         return point
 
 
@@ -426,20 +461,26 @@ def _compute_dtype(feat, weight):
     return feat.dtype if feat.dtype == weight.dtype else None
 
 
-def engine_for(model, data):
-    """The Engine that computes model(data), or None: the modules do."""
-    if (model.training or torch.is_grad_enabled() or ops._LAUNCH_TIMER is not None or ops.Readback.blocking
-            or type(data) not in (dict, AttrDict, Point)):
-        return None
+def plain_inputs(data):
+    """Whether `data` is what a caller hands to a forward and nothing a forward would have made itself: features and
+    coordinates on the GPU, scene ends or ids, no tables."""
+    if type(data) not in (dict, AttrDict, Point) or ops._LAUNCH_TIMER is not None or ops.Readback.blocking:
+        return False
     feat = data.get("feat")
     if not isinstance(feat, torch.Tensor) or not feat.is_cuda or feat.dim() != 2 or feat.shape[0] < 1 or feat.dtype not in ops.DTYPE_CODES:
-        return None
+        return False
     if any(k in data for k in _OWN_KEYS) or any(k.startswith("_") for k in data) or not ("offset" in data or "batch" in data):
-        return None
+        return False
     where = data.get("grid_coord", data.get("coord"))
     ends = data.get("offset", data.get("batch"))
-    if not (isinstance(where, torch.Tensor) and where.is_cuda and where.shape[0] == feat.shape[0] and ends.is_cuda and ends.numel()):
+    return isinstance(where, torch.Tensor) and where.is_cuda and where.shape[0] == feat.shape[0] and ends.is_cuda and ends.numel() > 0
+
+
+def engine_for(model, data):
+    """The Engine that computes model(data), or None: the modules do."""
+    if model.training or torch.is_grad_enabled() or not plain_inputs(data):
         return None
+    feat = data["feat"]
     weight = model.embedding.stem._modules["conv"].weight
     dtype = _compute_dtype(feat, weight)
     if dtype not in ops.DTYPE_CODES or feat.shape[1] != weight.shape[-1]:
@@ -447,26 +488,19 @@ def engine_for(model, data):
     held = _ENGINES.setdefault(model, {})
     key = (dtype, model.cls_mode)
     engine = held.get(key)
-    if engine is not None and not engine.structure.same():
-        engine = None
-        held.pop(key)
-    if engine is None and key not in held:
+    if engine is None or not engine.structure.same():
         try:
             engine = Engine(model, dtype)
-            _need(engine.structure.same(), "structure")
-            held[key] = engine
         except Unsupported as e:
-            held[key] = _Refused(model, str(e))
-            return None
-    if isinstance(engine, _Refused):
-        return None
-    if engine.structure.hooked() or any(m.training for m in engine.structure.flagged):
+            engine = Refused(model, str(e))
+        held[key] = engine
+    if isinstance(engine, Refused) or engine.structure.hooked() or any(m.training for m in engine.structure.flagged):
         return None
     return engine
 
 
-class _Refused:
-    """A model the native forward does not cover, remembered until its structure or weights move."""
+class Refused:
+    """A model the native paths do not cover, remembered until its structure or weights move."""
 
     def __init__(self, model, why):
         self.why = why

@@ -1,0 +1,285 @@
+"""A training step's forward and backward from native code (ptv3_train_fwd / ptv3_train_bwd): under half-precision
+autocast the whole feature side of a PointTransformerV3 is one autograd node whose parameter gradients come as views of
+one flat buffer. Module by module the same step is some 250 Python autograd functions each way and about 20 ms of host
+time whatever the batch. Takes the default architecture in training mode (see native.Parts, TrainEngine); anything else
+goes through the modules (model.py), which stay the definition of the result."""
+import ctypes
+import weakref
+
+import torch
+import torch.nn as nn
+
+from . import _lib, levels, native, ops
+from .modules import DropPath
+from .native import Parts, Structure, Unsupported, _need
+from .point import AttrDict, Point, batch2offset
+
+_i32, _i64, _f32, _ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
+
+
+class _Linear(ctypes.Structure):
+    _fields_ = [("w", _ptr), ("wt", _ptr), ("b", _ptr), ("cin", _i32), ("cout", _i32), ("gw", _i64), ("gb", _i64)]
+
+
+class _Norm(ctypes.Structure):
+    _fields_ = [("g", _ptr), ("b", _ptr), ("eps", _f32), ("reserved", _i32), ("gg", _i64), ("gb", _i64)]
+
+
+class _Bn(ctypes.Structure):
+    _fields_ = [("g", _ptr), ("b", _ptr), ("g16", _ptr), ("b16", _ptr), ("running_mean", _ptr), ("running_var", _ptr),
+                ("eps", _f32), ("momentum", _f32), ("gg", _i64)]
+
+
+class _Block(ctypes.Structure):
+    _fields_ = [("channels", _i32), ("heads", _i32), ("row", _i32), ("reserved", _i32), ("scale", _f32), ("reserved2", _f32),
+                ("conv_w", _ptr), ("conv_b", _ptr), ("conv_mirror", _ptr), ("conv_packed", _ptr), ("conv_mirror_packed", _ptr),
+                ("g_conv_w", _i64), ("g_conv_b", _i64),
+                ("cpe", _Linear), ("qkv", _Linear), ("proj", _Linear), ("fc1", _Linear), ("fc2", _Linear),
+                ("ln_cpe", _Norm), ("ln1", _Norm), ("ln2", _Norm)]
+
+
+class _Stage(ctypes.Structure):
+    _fields_ = [("channels", _i32), ("dec_channels", _i32), ("n_enc", _i32), ("n_dec", _i32), ("pool_reduce", _i32),
+                ("reserved", _i32), ("enc", _ptr), ("dec", _ptr), ("pool", _Linear), ("up", _Linear), ("up_skip", _Linear),
+                ("pool_bn", _Bn), ("up_bn", _Bn), ("up_skip_bn", _Bn)]
+
+
+class _Stem(ctypes.Structure):
+    _fields_ = [("w", _ptr), ("cin", _i32), ("cin_padded", _i32), ("gw", _i64), ("bn", _Bn)]
+
+
+class _Net(ctypes.Structure):
+    _fields_ = [("dtype", _i32), ("n_stages", _i32), ("patch", _i32 * levels.MAX_LEVELS), ("stem", _Stem), ("zero", _ptr),
+                ("n_zero", _i32), ("reserved", _i32), ("zero_blocks", _i64), ("stage", _Stage * levels.MAX_LEVELS)]
+
+
+class TrainEngine:
+    """Describes one model (float masters) for training under autocast to `dtype`."""
+
+    def __init__(self, model, dtype):
+        self.structure = Structure(model)
+        self.dtype = dtype
+        self.params = [p for p in model.parameters()]
+        self.device = self.params[0].device
+        _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() and p.dtype == torch.float32
+                  for p in self.structure.tensors), "float weights on one GPU")
+        _need(not model.cls_mode, "the encoder-only model hands out intermediate features")
+        self._keep, self._casts, self._packs, self._zero = [], [], [], []
+        self._at, offset = {}, 0        # parameter -> place of its gradient
+        for p in self.params:
+            self._at[p] = offset
+            offset += p.numel()
+        self.total = offset
+        self._describe(model)
+        self._finish()
+        self.batches = [m.num_batches_tracked for m in self.structure.modules
+                        if isinstance(m, nn.BatchNorm1d) and m.num_batches_tracked is not None]
+
+    def _buffer(self, elements):
+        t = torch.empty(elements, dtype=self.dtype, device=self.device)
+        self._keep.append(t)
+        return t.data_ptr()
+
+    def _copy(self, t, layout="plain"):
+        """Address of the parameter's copy in the compute dtype (ops.cast_cached's layouts)."""
+        shape, _ = ops._cast_shape(t, layout)
+        dst = self._buffer(t.numel())
+        self._casts.append((t, dst, shape, int(layout != "plain")))
+        return dst
+
+    def _linear(self, m, cin, cout):
+        _need(type(m) is nn.Linear and m.bias is not None and m.in_features == cin and m.out_features == cout, "Linear")
+        return _Linear(self._copy(m.weight), self._copy(m.weight, "transpose"), self._copy(m.bias), cin, cout,
+                       self._at[m.weight], self._at[m.bias])
+
+    def _norm(self, m, c):
+        _need(m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
+        self._zero += [(self._at[m.weight], c), (self._at[m.bias], c)]
+        return _Norm(m.weight.data_ptr(), m.bias.data_ptr(), m.eps, 0, self._at[m.weight], self._at[m.bias])
+
+    def _bn(self, m, c):
+        _need(type(m) is nn.BatchNorm1d and m.num_features == c and m.weight is not None and m.bias is not None
+              and m.track_running_stats and m.running_mean is not None and m.momentum is not None, "BatchNorm1d")
+        _need(self._at[m.bias] == self._at[m.weight] + c, "order of a BatchNorm's parameters")
+        return _Bn(m.weight.data_ptr(), m.bias.data_ptr(), self._copy(m.weight), self._copy(m.bias), m.running_mean.data_ptr(),
+                   m.running_var.data_ptr(), m.eps, m.momentum, self._at[m.weight])
+
+    def _block(self, b, c):
+        conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
+        _need(attn.attn_drop == 0 and attn.proj_drop.p == 0 and mlp.drop.p == 0 and c // attn.num_heads == 16, "dropout or head size")
+        d = _Block(channels=c, heads=attn.num_heads, row=attn.order_index, scale=attn.scale)
+        d.conv_w, d.conv_b, d.conv_mirror = self._copy(conv.weight), self._copy(conv.bias), self._copy(conv.weight, "mirror")
+        if c in native.CONV_PACKED:
+            d.conv_packed, d.conv_mirror_packed = self._buffer(27 * c * c), self._buffer(27 * c * c)
+            self._packs += [(d.conv_w, d.conv_packed, c, 27), (d.conv_mirror, d.conv_mirror_packed, c, 27)]
+        d.g_conv_w, d.g_conv_b = self._at[conv.weight], self._at[conv.bias]
+        d.cpe, d.qkv, d.proj = self._linear(b.cpe[1], c, c), self._linear(attn.qkv, c, 3 * c), self._linear(attn.proj, c, c)
+        d.fc1, d.fc2 = self._linear(mlp.fc1, c, 4 * c), self._linear(mlp.fc2, 4 * c, c)
+        d.ln_cpe, d.ln1, d.ln2 = self._norm(b.cpe[2], c), self._norm(b.norm1[0], c), self._norm(b.norm2[0], c)
+        return d
+
+    def _describe(self, model):
+        p = Parts(model)
+        _need(all(st.enc for st in p.stages) and all(st.dec for st in p.stages[:-1]), "a stage without blocks")
+        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages))
+        conv = p.stem_conv
+        padded = -(-conv.in_channels // 16) * 16
+        net.stem.w = self._buffer(conv.out_channels * 125 * padded)
+        net.stem.cin, net.stem.cin_padded, net.stem.gw = conv.in_channels, padded, self._at[conv.weight]
+        net.stem.bn = self._bn(p.stem_bn, conv.out_channels)
+        self._refresh = native._Refresh(dtype=net.dtype, stem_src=self._copy(conv.weight), stem_dst=net.stem.w,
+                                        stem_rows=conv.out_channels * 125, stem_in=conv.in_channels, stem_padded=padded)
+        self.drops, below = [], conv.out_channels
+        for s, st in enumerate(p.stages):
+            d = net.stage[s]
+            d.channels, d.n_enc, d.dec_channels, d.n_dec = st.channels, len(st.enc), st.dec_channels, len(st.dec)
+            if st.down is not None:
+                d.pool, d.pool_bn = self._linear(st.down.proj, below, st.channels), self._bn(st.down.norm[0], st.channels)
+                d.pool_reduce = ops.REDUCE_OPS[st.down.reduce]
+            if st.up is not None:
+                d.up = self._linear(st.up.proj[0], st.up.proj[0].in_features, st.dec_channels)
+                d.up_skip = self._linear(st.up.proj_skip[0], st.channels, st.dec_channels)
+                d.up_bn, d.up_skip_bn = self._bn(st.up.proj[1], st.dec_channels), self._bn(st.up.proj_skip[1], st.dec_channels)
+            for attr, bs, c in (("enc", st.enc, st.channels), ("dec", st.dec, st.dec_channels)):
+                if bs:
+                    arr = (_Block * len(bs))(*[self._block(b, c) for b in bs])
+                    self._keep.append(arr)
+                    setattr(d, attr, ctypes.addressof(arr))
+            net.patch[s] = st.patch
+            below = st.channels
+        order = [(s, b) for s, st in enumerate(p.stages) for b in st.enc]
+        order += [(s, b) for s in reversed(range(len(p.stages) - 1)) for b in p.stages[s].dec]
+        self.drops = [(s, b.drop_path[0]) for s, b in order]
+        self.out_channels = p.stages[0].dec_channels
+        self.layout = p.layout(model)
+        form, widths = _lib.load().ptv3_conv_form, p.widths()
+
+        def want(level, v):
+            flags = levels.PAIRS5 | levels.PAIR_OUT5 if level == 0 else 0
+            for c in widths[level]:
+                flags |= levels.TILES if form(v.n, v.n_pairs, c) else levels.PAIRS
+                flags |= levels.PAIRS | levels.PAIR_OUT if c < ops.OUTER_WIDE_CHANNELS else levels.NBR
+            return flags
+
+        self.want = want
+
+    def _finish(self):
+        lib, r = _lib.load(), self._refresh
+        rows, at = [], 0
+        for t, dst, (a, b, c), mirror in self._casts:
+            rows.append((t.data_ptr(), dst, a, b, c, mirror, at))
+            at += lib.ptv3_cast_params_blocks(a, b, c, mirror)
+        r.cast, r.n_cast, r.cast_blocks = self._table(rows, ops._CAST_JOB), len(rows), at
+        rows, at = [], 0
+        for src, dst, c, taps in self._packs:
+            rows.append((src, dst, c, taps, at))
+            at += lib.ptv3_subm_conv_pack_weight_blocks(c, taps)
+        r.conv, r.n_conv, r.conv_blocks = self._table(rows, ops._PACK_JOB), len(rows), at
+        rows, at = [], 0
+        for start, count in self._zero:
+            rows.append((start, count, at))
+            at += -(-count // 256)
+        net = self.net
+        net.zero, net.n_zero, net.zero_blocks = self._table(rows, [("at", "<i8"), ("count", "<i8"), ("block", "<i8")]), len(rows), at
+
+    def _table(self, rows, dtype):
+        t = native.job_table(rows, dtype, self.device)
+        self._keep.append(t)
+        return t.data_ptr() if t is not None else None
+
+    def masks(self, index):
+        """The stochastic-depth row factors in the order the blocks would draw them (DropPath.mask; model.py:602-604)."""
+        out, keeps, drawn = [], [], []
+        for s, drop in self.drops:
+            rate = drop.drop_prob if isinstance(drop, DropPath) else 0.0
+            for _ in range(2):
+                if rate == 0.0:
+                    out.append(None)
+                    continue
+                m = torch.empty((index.levels[s].n, 1), dtype=self.dtype, device=self.device).bernoulli_(1.0 - rate)
+                if drop.scale_by_keep and rate < 1.0:
+                    drawn.append(m)
+                    keeps.append(1.0 - rate)
+                out.append(m)
+        if drawn:
+            torch._foreach_div_(drawn, keeps)
+        return out
+
+    def forward(self, model, data):
+        feat = data["feat"].detach().contiguous()
+        point = Point.__new__(Point)
+        dict.update(point, data)
+        grid, offset, batch = native.coordinates(point)
+
+        def refresh():   # float masters are cast, transposed and packed once per step
+            _lib.check(_lib.load().ptv3_net_refresh(ctypes.byref(self._refresh), ops._stream()), "ptv3_net_refresh")
+
+        model._prologue_state = None
+        index = levels.build(self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want, between=refresh)
+        if any(v.n < 2 for v in index.levels):
+            raise ValueError("Expected more than 1 value per channel when training")   # as BatchNorm1d does
+        if self.batches:
+            torch._foreach_add_(self.batches, 1)
+        out = _Step.apply(self, feat, index, self.masks(index), *self.params)
+        point["batch"] = index.batch
+        native.fill_point(point, index, 0, out, self.net.patch[0])
+        return point
+
+
+class _Step(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, engine, feat, index, masks, *params):
+        lib = _lib.load()
+        u8 = dict(dtype=torch.uint8, device=feat.device)
+        sizes = (ctypes.c_size_t * 3)()
+        at = ctypes.addressof(sizes)
+        _lib.check(lib.ptv3_train_bytes(ctypes.byref(engine.net), index.levels, at, at + 8, at + 16), "ptv3_train_bytes")
+        acts, scratch = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
+        out = torch.empty((feat.shape[0], engine.out_channels), dtype=torch.float32, device=feat.device)
+        mask_ptrs = (_ptr * len(masks))(*[None if m is None else m.data_ptr() for m in masks])
+        _lib.check(lib.ptv3_train_fwd(ctypes.byref(engine.net), index.levels, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype], mask_ptrs,
+                                      acts.data_ptr(), scratch.data_ptr(), sizes[1], out.data_ptr(), ops._stream()), "ptv3_train_fwd")
+        ctx.engine, ctx.index, ctx.mask_ptrs, ctx.scratch_bytes = engine, index, mask_ptrs, sizes[2]
+        # freed by autograd after the backward, as the activations of separate nodes would be
+        ctx.save_for_backward(acts, *[m for m in masks if m is not None])
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout):
+        engine, index = ctx.engine, ctx.index
+        acts = ctx.saved_tensors[0]
+        dout = dout.contiguous()
+        scratch = torch.empty(ctx.scratch_bytes, dtype=torch.uint8, device=dout.device)
+        grads = torch.empty(engine.total, dtype=torch.float32, device=dout.device)
+        _lib.check(_lib.load().ptv3_train_bwd(ctypes.byref(engine.net), index.levels, dout.data_ptr(), ops.DTYPE_CODES[dout.dtype],
+                                              ctx.mask_ptrs, acts.data_ptr(), scratch.data_ptr(), ctx.scratch_bytes,
+                                              grads.data_ptr(), ops._stream()), "ptv3_train_bwd")
+        views = torch._utils._unflatten_dense_tensors(grads, engine.params)
+        needed = ctx.needs_input_grad[4:]
+        return (None,) * 4 + tuple(g if need else None for g, need in zip(views, needed))
+
+
+_ENGINES = weakref.WeakKeyDictionary()   # model -> {dtype: TrainEngine or native.Refused}
+
+
+def engine_for(model, data):
+    """The TrainEngine that computes model(data), or None: the modules do."""
+    if not (model.training and torch.is_grad_enabled() and torch.is_autocast_enabled()) or model.cls_mode:
+        return None
+    dtype = torch.get_autocast_dtype("cuda")
+    if dtype not in (torch.float16, torch.bfloat16) or not native.plain_inputs(data) or data["feat"].requires_grad:
+        return None
+    held = _ENGINES.setdefault(model, {})
+    engine = held.get(dtype)
+    if engine is None or not engine.structure.same():
+        try:
+            engine = TrainEngine(model, dtype)
+        except Unsupported as e:
+            engine = native.Refused(model, str(e))
+        held[dtype] = engine
+    if isinstance(engine, native.Refused) or data["feat"].shape[1] != engine.net.stem.cin or data["feat"].shape[0] < 2:
+        return None
+    if engine.structure.hooked() or not all(m.training for m in engine.structure.flagged):
+        return None
+    return engine if any(p.requires_grad for p in engine.params) else None

@@ -1,0 +1,98 @@
+"""The natively queued training step against the same model's modules: rows, running statistics, every gradient."""
+import copy
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV
+from test_gpu_native import KW, _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(model, data, dtype, use, monkeypatch, seed=11):
+    from pointtransformerv3_amd import native_train
+    taken, real = [], native_train.engine_for
+    monkeypatch.setattr(native_train, "engine_for",
+                        (lambda m, d: taken.append(real(m, d)) or taken[-1]) if use else (lambda m, d: None))
+    model.zero_grad(set_to_none=True)
+    torch.manual_seed(seed)
+    with torch.autocast("cuda", dtype=dtype):
+        point = model(dict(data))
+    g = torch.Generator(device=DEV).manual_seed(1)
+    # a coherent gradient (few classes, by place): a sum of independent signs would amplify every rounding
+    label = (data["grid_coord"].sum(1) % 5).long()
+    w = torch.randn(5, point.feat.shape[1], generator=g, device=DEV)
+    point.feat.backward((w[label] * 0.05).to(point.feat.dtype))
+    monkeypatch.setattr(native_train, "engine_for", real)
+    assert not use or taken[0] is not None, "the native path was not taken"
+    return point
+
+
+def _compare(model, data, dtype, monkeypatch, tol):
+    other = copy.deepcopy(model)
+    a, b = _step(model, data, dtype, True, monkeypatch), _step(other, data, dtype, False, monkeypatch)
+    assert a.feat.dtype == b.feat.dtype == torch.float32
+    rel = lambda x, y: float((x.double() - y.double()).norm() / y.double().norm().clamp_min(1e-30))
+    errs = {"feat": rel(a.feat.detach(), b.feat.detach())}
+    for (name, p), q in zip(model.named_parameters(), other.parameters()):
+        assert p.grad.shape == q.grad.shape and torch.isfinite(p.grad).all(), name
+        errs[name] = rel(p.grad, q.grad)
+    bufs = [(n, x, y) for (n, x), y in zip(model.named_buffers(), other.buffers())]
+    for n, x, y in bufs:
+        assert torch.equal(x, y) if not x.is_floating_point() else rel(x, y) < tol, (n, rel(x, y))
+    for key in ("batch", "serialized_order", "pad", "unpad", "cu_seqlens_key"):
+        assert torch.equal(a[key], b[key])
+    flat = lambda m: torch.cat([p.grad.reshape(-1) for p in m.parameters()])
+    assert rel(flat(model), flat(other)) < tol, sorted(errs.items(), key=lambda kv: -kv[1])[:5]
+    ranked = sorted(errs.values())
+    assert ranked[len(ranked) // 2] < tol, ranked[len(ranked) // 2]
+    return errs
+
+
+@pytest.mark.parametrize("sizes", [(6000,), (9000, 150, 4000)])
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 2e-2), (torch.bfloat16, 6e-2)])
+def test_native_training_step_matches_the_modules(dtype, tol, sizes, monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(**dict(KW, enc_depths=(1, 2, 2, 1, 1))).to(DEV).train()
+    _compare(model, _inputs(4, sizes, torch.float32), dtype, monkeypatch, tol)
+
+
+def test_native_training_step_without_stochastic_depth_and_with_frozen_parameters(monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0, **KW).to(DEV).train()
+    data = _inputs(4, (7000,), torch.float32)
+    _compare(model, data, torch.float16, monkeypatch, 2e-2)
+    model.enc.enc2.requires_grad_(False)
+    _step(model, data, torch.float16, True, monkeypatch)
+    assert all((p.grad is None) == n.startswith("enc.enc2.") for n, p in model.named_parameters())
+
+
+def test_native_training_follows_the_optimizer_and_leaves_other_modes_alone(monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3, native_train
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0, **KW).to(DEV).train()
+    data = _inputs(4, (5000,), torch.float32)
+    opt = torch.optim.AdamW(model.parameters(), lr=1e-3, fused=True)
+    for _ in range(2):
+        _step(model, data, torch.bfloat16, True, monkeypatch)
+        opt.step()
+    _compare(model, data, torch.bfloat16, monkeypatch, 6e-2)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert native_train.engine_for(model, data) is not None
+        model.enc.enc1.down.norm[0].eval()                       # a frozen BatchNorm: the modules
+        assert native_train.engine_for(model, data) is None
+        model.train()
+        assert native_train.engine_for(model, dict(data, feat=data["feat"].clone().requires_grad_())) is None
+        with torch.no_grad():
+            assert native_train.engine_for(model, data) is None
+    assert native_train.engine_for(model, data) is None          # no autocast: the modules
+    # a second backward over a step whose graph was freed fails as any other does
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = model(dict(data)).feat
+    out.sum().backward()
+    with pytest.raises(RuntimeError):
+        out.sum().backward()
