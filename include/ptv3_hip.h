@@ -86,6 +86,12 @@ size_t ptv3_argsort_workspace_bytes(int64_t n, int k);
 int ptv3_argsort(const int64_t *code, int64_t n, int k, int key_bits, int64_t *order,
                  int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);
 
+/* ptv3_encode and ptv3_argsort of the codes in one call (the codes are counted where they are made); workspace as
+ * ptv3_argsort's. key_bits covers the curve bits and the scene bits above them. */
+int ptv3_serialize(const int32_t *grid_coord, const int64_t *batch, int64_t n, int depth,
+                   const int32_t *order_ids_host, int k, int key_bits, int64_t *code, int64_t *order,
+                   int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);
+
 /* model.py:392-437. ptv3_pad_sizes is host-only arithmetic on a HOST copy of `offset`
  * (nb cumulative scene ends): total padded length and number of sequences.
  * ptv3_pad_index fills pad (n_pad,), unpad (n,), cu_seqlens (n_seq+1,) int32 from the
@@ -681,6 +687,12 @@ int ptv3_index_begin(void *state, const ptv3_index_cfg *cfg, const int32_t *grid
                      const int64_t *offset, int64_t *batch_out, void *workspace, size_t workspace_bytes,
                      int64_t *host_slot, int64_t seq, void *stream);
 int ptv3_index_wait(const int64_t *host_slot, int which, int64_t seq, void *stream);
+
+/* Grid extent and scene ends alone, reported like the first stage (model.py:98-101): the maximum of every axis at
+ * host_slot[PTV3_SLOT_DATA..], the ends at host_slot[PTV3_SLOT_ENDS..], `seq` in word 0. */
+size_t ptv3_scene_facts_bytes(int64_t n);
+int ptv3_scene_facts(const int32_t *grid_coord, int64_t n, const int64_t *offset, int n_scenes, void *workspace,
+                     size_t workspace_bytes, int64_t *host_slot, int64_t seq, void *stream);
 size_t ptv3_index_sort_bytes(const void *state);
 int ptv3_index_sort(void *state, int depth, int key_bits, const int32_t *order_ids, int64_t *code, int64_t *order,
                     int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);

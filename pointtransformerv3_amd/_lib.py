@@ -23,6 +23,7 @@ SIGNATURES = {
     "ptv3_offset2batch": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "ptv3_argsort_workspace_bytes": (_sz, [_i64, _i32]),
     "ptv3_argsort": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
+    "ptv3_serialize": (_i32, [_vp, _vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_pad_sizes": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "ptv3_pad_index_workspace_bytes": (_sz, [_i32]),
     "ptv3_pad_index": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
@@ -115,6 +116,8 @@ SIGNATURES = {
     "ptv3_index_begin_bytes": (_sz, [_vp]),
     "ptv3_index_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _i64, _vp]),
     "ptv3_index_wait": (_i32, [_vp, _i32, _i64, _vp]),
+    "ptv3_scene_facts_bytes": (_sz, [_i64]),
+    "ptv3_scene_facts": (_i32, [_vp, _i64, _vp, _i32, _vp, _sz, _vp, _i64, _vp]),
     "ptv3_index_sort_bytes": (_sz, [_vp]),
     "ptv3_index_sort": (_i32, [_vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_index_pool_bytes": (_i32, [_vp, _vp, _vp]),

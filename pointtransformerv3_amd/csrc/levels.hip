@@ -19,8 +19,9 @@
 
 #include "voxelhash.h"
 
-int ptv3_argsort_keys(const int64_t* code, int64_t n, int k, int key_bits, int64_t* order, int64_t* inverse,
-                      void* sorted_keys, void* workspace, size_t workspace_bytes, hipStream_t stream);   // sort.hip
+int ptv3_serialize_keys(const int32_t* grid_coord, const int64_t* batch, int64_t n, int depth, const int32_t* order_ids_host, int k,
+                        int key_bits, int64_t* code, int64_t* order, int64_t* inverse, void* sorted_keys, void* workspace,
+                        size_t workspace_bytes, hipStream_t stream);   // sort.hip
 
 namespace {
 
@@ -29,6 +30,7 @@ constexpr int LB = 256;             // positions per block of the cell passes
 constexpr int GT = 128;             // threads of a pair-list work-group: a tile of 128 or 96 voxels
 constexpr int TAPS5 = 125, TAPS3 = 27;
 constexpr int TILE_WORDS = 32;
+constexpr int MAX_FACT_BLOCKS = 1024;
 
 // ---- stage 1: scene ids, sparse indices, grid extent ---------------------------------------------------------------
 
@@ -39,10 +41,10 @@ __global__ __launch_bounds__(256) void facts_kernel(const int32_t* __restrict__ 
     __shared__ int32_t red[4][3];
     int32_t m[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        int64_t b;
+        int64_t b = 0;
         if (batch_in) {
             b = batch_in[i];
-        } else {
+        } else if (batch) {
             int lo = 0, hi = nb;   // first scene whose end is > i
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
@@ -52,7 +54,7 @@ __global__ __launch_bounds__(256) void facts_kernel(const int32_t* __restrict__ 
             batch[i] = b;
         }
         const int32_t x = grid[3 * i], y = grid[3 * i + 1], z = grid[3 * i + 2];
-        indices[i] = make_int4((int32_t)b, x, y, z);
+        if (indices) indices[i] = make_int4((int32_t)b, x, y, z);
         m[0] = max(m[0], x);
         m[1] = max(m[1], y);
         m[2] = max(m[2], z);
@@ -813,7 +815,7 @@ size_t carve_begin(State& s, void* base) {
     Carver c(base);
     const int64_t n = g.n;
     s.lv[0].indices = c.take<int32_t>(4 * n);
-    s.part = c.take<int32_t>(3 * 1024);
+    s.part = c.take<int32_t>(3 * MAX_FACT_BLOCKS);
     const int pooled = g.n_levels - 1;
     for (int l = 0; l < g.n_levels; ++l) {
         if (l > 0) s.lv[l].offset = c.take<int64_t>(g.n_scenes);
@@ -857,6 +859,11 @@ extern "C" int64_t ptv3_index_slot_words(int n_levels, int n_scenes) {
     return n_levels < 1 || n_scenes < 1 ? 0 : PTV3_SLOT_ENDS + (int64_t)n_levels * n_scenes;
 }
 
+static int fact_blocks(int64_t n) {
+    const int64_t want = ptv3_ceil_div(n, 256);
+    return (int)(want < MAX_FACT_BLOCKS ? want : MAX_FACT_BLOCKS);
+}
+
 extern "C" int ptv3_index_begin(void* state, const ptv3_index_cfg* cfg, const int32_t* grid_coord, const int64_t* batch_in,
                                 const int64_t* offset, int64_t* batch_out, void* workspace, size_t workspace_bytes,
                                 int64_t* host_slot, int64_t seq, void* stream_) {
@@ -877,14 +884,30 @@ extern "C" int ptv3_index_begin(void* state, const ptv3_index_cfg* cfg, const in
     s.lv[0].batch = (int64_t*)s.batch;
     s.lv[0].offset = (int64_t*)offset;
     s.lv[0].grid = (int32_t*)grid_coord;
-    const int64_t want = ptv3_ceil_div(cfg->n, 256);
-    const int blocks = (int)(want < 1024 ? want : 1024);
+    const int blocks = fact_blocks(cfg->n);
     hipLaunchKernelGGL(facts_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, grid_coord, batch_in, offset, cfg->n_scenes,
                        cfg->n, batch_out, (int4*)s.lv[0].indices, s.part);
     hipLaunchKernelGGL(publish_facts_kernel, dim3(1), dim3(256), 0, stream, (const int32_t*)s.part, blocks, offset,
                        cfg->n_scenes, host_slot, seq);
     // level 0's neighbour search needs the coordinates only: it runs while the host reads the extent
     return launch_hash_count(s, 0, 1, stream);
+}
+
+extern "C" size_t ptv3_scene_facts_bytes(int64_t n) {
+    return 3 * (size_t)fact_blocks(n) * sizeof(int32_t);
+}
+
+extern "C" int ptv3_scene_facts(const int32_t* grid_coord, int64_t n, const int64_t* offset, int n_scenes, void* workspace,
+                                size_t workspace_bytes, int64_t* host_slot, int64_t seq, void* stream_) {
+    if (n < 1 || n_scenes < 1 || !grid_coord || !offset || !workspace || !host_slot) return PTV3_EINVAL;
+    if (workspace_bytes < ptv3_scene_facts_bytes(n)) return PTV3_EWORKSPACE;
+    const int blocks = fact_blocks(n);
+    hipStream_t stream = (hipStream_t)stream_;
+    hipLaunchKernelGGL(facts_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, grid_coord, nullptr, offset, n_scenes, n, nullptr,
+                       nullptr, (int32_t*)workspace);
+    hipLaunchKernelGGL(publish_facts_kernel, dim3(1), dim3(256), 0, stream, (const int32_t*)workspace, blocks, offset, n_scenes,
+                       host_slot, seq);
+    PTV3_RETURN_LAUNCH();
 }
 
 extern "C" int ptv3_index_wait(const int64_t* host_slot, int which, int64_t seq, void* stream_) {
@@ -916,9 +939,8 @@ extern "C" int ptv3_index_sort(void* state, int depth, int key_bits, const int32
     State& s = *(State*)state;
     const ptv3_index_cfg& g = s.cfg;
     hipStream_t stream = (hipStream_t)stream_;
-    int rc = ptv3_encode(s.grid, s.batch, g.n, depth, order_ids, g.n_orders, code, stream_);
-    if (rc != PTV3_OK) return rc;
-    rc = ptv3_argsort_keys(code, g.n, g.n_orders, key_bits, order, inverse, s.keys, workspace, workspace_bytes, stream);
+    int rc = ptv3_serialize_keys(s.grid, s.batch, g.n, depth, order_ids, g.n_orders, key_bits, code, order, inverse, s.keys, workspace,
+                                 workspace_bytes, stream);
     if (rc != PTV3_OK) return rc;
     s.depth = depth;
     s.key_bits = key_bits;

@@ -66,6 +66,28 @@ def _take_slot(words):
     return slot
 
 
+class SceneFacts:
+    """Grid extent and scene ends of (n, 3) int32 coordinates, on their way to the host behind the work queued so far."""
+
+    def __init__(self, grid_coord, offset):
+        lib = _lib.load()
+        self.nb = offset.shape[0]
+        self.slot, self.seq, self.stream = _take_slot(_SLOT_ENDS + self.nb), next(_SEQ), ops._stream()
+        nbytes = lib.ptv3_scene_facts_bytes(grid_coord.shape[0])
+        self.scratch = torch.empty(nbytes, dtype=torch.uint8, device=grid_coord.device)
+        _lib.check(lib.ptv3_scene_facts(grid_coord.data_ptr(), grid_coord.shape[0], offset.data_ptr(), self.nb,
+                                        self.scratch.data_ptr(), nbytes, self.slot.ptr, self.seq, self.stream), "ptv3_scene_facts")
+
+    def get(self):
+        """(per-axis maxima, scene ends) as lists."""
+        if self.slot.words[0] != self.seq:
+            ops.refresh_derived_copies()   # as Readback.get: work for the wait
+        _lib.check(_lib.load().ptv3_index_wait(self.slot.ptr, 0, self.seq, self.stream), "ptv3_index_wait")
+        out = self.slot.words[_SLOT_DATA:_SLOT_DATA + 3], self.slot.words[_SLOT_ENDS:_SLOT_ENDS + self.nb]
+        _SLOTS.append(self.slot)
+        return out
+
+
 class Layout:
     """What the index of a model needs to know of its modules, worked out once: per level the pooling in front of it, the
     patch size, the attention rows in use and the convolutions that share the level's lists."""

@@ -317,6 +317,23 @@ def argsort_rows(code, key_bits):
     return order, inverse
 
 
+def serialize(grid_coord, batch, depth, orders, key_bits):
+    """encode_orders and argsort_rows of the codes: (code, order, inverse), each (k, N) int64."""
+    _dev(grid_coord, batch)
+    lib = _lib.load()
+    g = grid_coord.to(torch.int32).contiguous()
+    b = batch.to(torch.int64).contiguous()
+    n, k = g.shape[0], len(orders)
+    ids = (ctypes.c_int32 * k)(*[ORDER_IDS[o] for o in orders])
+    code, order, inverse = (torch.empty((k, n), dtype=torch.int64, device=g.device) for _ in range(3))
+    nbytes = lib.ptv3_argsort_workspace_bytes(n, k)
+    ws = _ws(nbytes, g.device)
+    _timed("serialize", (n, k, int(key_bits)), lambda: _lib.check(
+        lib.ptv3_serialize(_ptr(g), _ptr(b), n, int(depth), ids, k, int(key_bits), _ptr(code), _ptr(order), _ptr(inverse), _ptr(ws),
+                           nbytes, _stream()), "ptv3_serialize"))
+    return code, order, inverse
+
+
 def pad_sizes(offset_host, patch):
     """(n_pad, n_seq) from a host list of cumulative scene ends."""
     lib = _lib.load()

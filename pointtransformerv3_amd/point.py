@@ -12,7 +12,7 @@ import math
 
 import torch
 
-from . import ops
+from . import levels, ops
 
 
 @torch.inference_mode()
@@ -76,6 +76,16 @@ class Point(AttrDict):
     def _fetch_host(self):
         want_offset = "_offset_host" not in self
         want_grid = "_grid_max_host" not in self and ("grid_coord" in self or {"grid_size", "coord"} <= self.keys())
+        if want_offset and want_grid:
+            self._ensure_grid_coord()
+            grid, offset = self["grid_coord"], self["offset"]
+            if (grid.is_cuda and offset.is_cuda and grid.shape[0] > 0 and offset.shape[0] > 0 and not ops.Readback.blocking
+                    and grid.dtype == torch.int32 and grid.is_contiguous() and offset.dtype == torch.int64 and offset.is_contiguous()):
+                facts = levels.SceneFacts(grid, offset)
+                for ks in self.pop("_plan_ahead", ()):
+                    self.start_plan(ks)
+                self["_grid_max_host"], self["_offset_host"] = facts.get()
+                return
         parts = []
         if want_offset:
             parts.append(self["offset"].long())
@@ -136,9 +146,8 @@ class Point(AttrDict):
             # on nothing but its order, so encoding the orders in permuted sequence gives the same tables
             perm = torch.randperm(len(orders)).tolist()       # CPU generator, as model.py:129
             orders = [orders[i] for i in perm]
-        code = ops.encode_orders(self["grid_coord"], self["batch"], depth, orders)
         key_bits = 3 * depth + max(1, (n_scenes - 1).bit_length())
-        sort_order, inverse = ops.argsort_rows(code, key_bits)
+        code, sort_order, inverse = ops.serialize(self["grid_coord"], self["batch"], depth, orders, key_bits)
 
         self["serialized_code"] = code
         self["serialized_order"] = sort_order
