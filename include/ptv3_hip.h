@@ -65,7 +65,8 @@ int ptv3_grid_max(const int32_t *grid_coord, int64_t n, int32_t *out3, void *str
  * int64 cumulative scene ends, all on the device. Outputs, sized for n by the caller: grid_coord
  * (m,3) int32 and index (m,) int64 of the kept points in input order, inverse (n,) int64 = position
  * of every input point's voxel among the kept ones (or NULL), offset_out (n_scenes,) int64 = scene
- * ends of the kept points, counts (2,) int64 on the device = {m, status}; status 1 means a grid
+ * ends of the kept points. m and a status go to host_slot[PTV3_SLOT_DATA] and the word behind it, then `seq` to word 0
+ * (pinned host memory, see ptv3_index_wait; the last kernels run while the host reads them); status 1 means a grid
  * coordinate needs more than 16 bits (the serialization's limit, model.py:108) and the rest is
  * meaningless. n < 2^30. pick_seed 0 keeps the first point in input order (GridSample's test mode); any other
  * value keeps a member of every voxel drawn uniformly, a different draw per seed (its train mode; the
@@ -73,7 +74,16 @@ int ptv3_grid_max(const int32_t *grid_coord, int64_t n, int32_t *out3, void *str
 size_t ptv3_voxelize_workspace_bytes(int64_t n, int n_scenes);
 int ptv3_voxelize(const float *coord, int64_t n, const int64_t *offset, int n_scenes, float grid_size,
                   int32_t *grid_coord, int64_t *index, int64_t *inverse, int64_t *offset_out,
-                  int64_t *counts, uint32_t pick_seed, void *workspace, size_t workspace_bytes, void *stream);
+                  int64_t *host_slot, int64_t seq, uint32_t pick_seed, void *workspace, size_t workspace_bytes,
+                  void *stream);
+
+/* Rows index[0 .. m) of up to PTV3_GATHER_MAX arrays in one launch (what coord[index], feat[index], ... do one by one in
+ * front of model.py:966-973): dst[a] (m, row_bytes[a]) from src[a], rows of at most PTV3_GATHER_MAX_ROW bytes. src, dst
+ * and row_bytes are host arrays; index int64 on the device, every entry a row of every source. m < 2^31. */
+#define PTV3_GATHER_MAX 8
+#define PTV3_GATHER_MAX_ROW 4095
+int ptv3_gather_rows(const void *const *src, void *const *dst, const int64_t *row_bytes, int count, const int64_t *index,
+                     int64_t m, void *stream);
 
 /* model.py:35-40 (offset2batch): scene id of each of the n points from the cumulative scene ends
  * offset (n_scenes,) int64 on the device, n = offset[n_scenes - 1] known to the caller. */

@@ -19,7 +19,8 @@ SIGNATURES = {
     "ptv3_decode": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp]),
     "ptv3_grid_max": (_i32, [_vp, _i64, _vp, _vp]),
     "ptv3_voxelize_workspace_bytes": (_sz, [_i64, _i32]),
-    "ptv3_voxelize": (_i32, [_vp, _i64, _vp, _i32, _f32, _vp, _vp, _vp, _vp, _vp, ctypes.c_uint32, _vp, _sz, _vp]),
+    "ptv3_voxelize": (_i32, [_vp, _i64, _vp, _i32, _f32, _vp, _vp, _vp, _vp, _vp, _i64, ctypes.c_uint32, _vp, _sz, _vp]),
+    "ptv3_gather_rows": (_i32, [_vp, _vp, _vp, _i32, _vp, _i64, _vp]),
     "ptv3_offset2batch": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "ptv3_argsort_workspace_bytes": (_sz, [_i64, _i32]),
     "ptv3_argsort": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),

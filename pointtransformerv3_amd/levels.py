@@ -1,17 +1,15 @@
 """The index of a whole forward from one batched pass (ptv3_index_*): every table that follows from the coordinates
 alone, for every encoder level, in about 24 launches and three waits (model.py:81-174, :382-453, :652-703)."""
-import collections
 import ctypes
-import itertools
 import math
 
 import torch
 
-from . import _lib, ops
+from . import _lib, hostslot, ops
 
 MAX_LEVELS = MAX_ORDERS = 8
 _STATE_BYTES = 16384
-_SLOT_DATA = 3
+_SLOT_DATA = hostslot.DATA
 _SLOT_ENDS = _SLOT_DATA + 4 + MAX_LEVELS + 2 * MAX_LEVELS
 PAIRS, TILES, PAIRS5, PAIR_OUT, NBR, PAIR_OUT5 = 1, 2, 4, 8, 16, 32
 
@@ -36,43 +34,13 @@ class Level(ctypes.Structure):
                 + [("tile_voxels", _i32), ("depth", _i32)])
 
 
-class _Slot:
-    """Pinned words that the stages report to."""
-
-    def __init__(self, words):
-        self.tensor = torch.zeros(words, dtype=torch.int64, pin_memory=True)
-        self.ptr = self.tensor.data_ptr()
-        self.words = (ctypes.c_int64 * words).from_address(self.ptr)
-
-
-_SLOTS = collections.deque(maxlen=16)   # free slots; append and pop are atomic
-_SEQ = itertools.count(1)
-
-
-def _take_slot(words):
-    kept = []
-    slot = None
-    while slot is None:
-        try:
-            s = _SLOTS.pop()
-        except IndexError:
-            slot = _Slot(max(words, 256))
-            break
-        if len(s.words) >= words:
-            slot = s
-        else:
-            kept.append(s)
-    _SLOTS.extend(kept)
-    return slot
-
-
 class SceneFacts:
     """Grid extent and scene ends of (n, 3) int32 coordinates, on their way to the host behind the work queued so far."""
 
     def __init__(self, grid_coord, offset):
         lib = _lib.load()
         self.nb = offset.shape[0]
-        self.slot, self.seq, self.stream = _take_slot(_SLOT_ENDS + self.nb), next(_SEQ), ops._stream()
+        self.slot, self.seq, self.stream = hostslot.take(_SLOT_ENDS + self.nb), hostslot.next_seq(), ops._stream()
         nbytes = lib.ptv3_scene_facts_bytes(grid_coord.shape[0])
         self.scratch = torch.empty(nbytes, dtype=torch.uint8, device=grid_coord.device)
         _lib.check(lib.ptv3_scene_facts(grid_coord.data_ptr(), grid_coord.shape[0], offset.data_ptr(), self.nb,
@@ -84,7 +52,7 @@ class SceneFacts:
             ops.refresh_derived_copies()   # as Readback.get: work for the wait
         _lib.check(_lib.load().ptv3_index_wait(self.slot.ptr, 0, self.seq, self.stream), "ptv3_index_wait")
         out = self.slot.words[_SLOT_DATA:_SLOT_DATA + 3], self.slot.words[_SLOT_ENDS:_SLOT_ENDS + self.nb]
-        _SLOTS.append(self.slot)
+        hostslot.give(self.slot)
         return out
 
 
@@ -139,8 +107,8 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     out = Index()
     u8 = dict(dtype=torch.uint8, device=dev)
     state = ctypes.create_string_buffer(_STATE_BYTES)
-    slot = _take_slot(lib.ptv3_index_slot_words(cfg.n_levels, nb))
-    words, seq = slot.words, next(_SEQ)
+    slot = hostslot.take(lib.ptv3_index_slot_words(cfg.n_levels, nb))
+    words, seq = slot.words, hostslot.next_seq()
     nbytes = lib.ptv3_index_begin_bytes(ctypes.byref(cfg))
     first = torch.empty(nbytes, **u8)
     out.batch = batch if batch is not None else torch.empty(n, dtype=torch.int64, device=dev)
@@ -185,7 +153,7 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     check(lib.ptv3_index_lists_bytes(state, wanted, sizes), "ptv3_index_lists_bytes")
     lists = torch.empty(sizes[0], **u8)
     check(lib.ptv3_index_lists(state, wanted, lists.data_ptr(), sizes[0], stream), "ptv3_index_lists")
-    _SLOTS.append(slot)
+    hostslot.give(slot)
     out.state = state                # `levels` lies in it
     out.offset, out.grid_coord, out.depth, out.n_orders = offset, grid_coord, depth, k
     # `first` holds level 0's sparse indices, the pooled scene ends and level 0's tap_ptr; `scratch` the pooled tap_ptr

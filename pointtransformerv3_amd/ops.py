@@ -5,13 +5,14 @@ the HIP kernels. All tensors must live on the GPU; CPU tensors are rejected.
 """
 import contextlib
 import ctypes
+import math
 import weakref
 
 import numpy as np
 import torch
 from torch.optim.optimizer import register_optimizer_step_post_hook as _register_step_hook
 
-from . import _lib
+from . import _lib, hostslot
 
 ORDER_IDS = {"z": 0, "z-trans": 1, "hilbert": 2, "hilbert-trans": 3}
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
@@ -276,18 +277,42 @@ def voxelize(coord, offset, grid_size, with_inverse=True, seed=0):
     index = torch.empty(n, dtype=torch.int64, device=dev)
     inverse = torch.empty(n, dtype=torch.int64, device=dev) if with_inverse else None
     off_out = torch.empty(nb, dtype=torch.int64, device=dev)
-    counts = torch.empty(2, dtype=torch.int64, device=dev)
     nbytes = lib.ptv3_voxelize_workspace_bytes(n, nb)
     ws = _ws(nbytes, dev)
+    slot, seq, stream = hostslot.take(hostslot.DATA + 2), hostslot.next_seq(), _stream()
     _lib.check(lib.ptv3_voxelize(_ptr(coord), n, _ptr(off), nb, float(grid_size), _ptr(grid), _ptr(index), _ptr(inverse),
-                                 _ptr(off_out), _ptr(counts), int(seed) & 0xFFFFFFFF, _ptr(ws), nbytes, _stream()),
+                                 _ptr(off_out), slot.ptr, seq, int(seed) & 0xFFFFFFFF, _ptr(ws), nbytes, stream),
                "ptv3_voxelize")
-    m, status = Readback(counts).get()
+    hostslot.wait(slot, 0, seq, stream)
+    m, status = slot.words[hostslot.DATA:hostslot.DATA + 2]
+    hostslot.give(slot)
     if status:
         raise RuntimeError("voxelize: a grid coordinate does not fit 16 bits (grid_size too small for the scene extent)")
     out = dict(grid_coord=grid[:m], index=index[:m], offset=off_out)
     if with_inverse:
         out["inverse"] = inverse
+    return out
+
+
+def gather_rows(tensors, index):
+    """[t[index] for t in tensors]: rows of several tensors in one launch. index (M,) int64, as voxelize returns it.
+    Tensors that are not contiguous or have rows of more than 4095 bytes are indexed by torch."""
+    out, jobs = [], []
+    m = index.shape[0]
+    for t in tensors:
+        row = t.element_size() * math.prod(t.shape[1:])
+        if not t.is_cuda or t.device != index.device or not t.is_contiguous() or not 0 < row <= 4095 or m == 0:
+            out.append(t[index])
+            continue
+        dst = torch.empty((m, *t.shape[1:]), dtype=t.dtype, device=t.device)
+        out.append(dst)
+        jobs.append((t.data_ptr(), dst.data_ptr(), row))
+    lib = _lib.load()
+    for at in range(0, len(jobs), 8):
+        src, dst, row = zip(*jobs[at:at + 8])
+        k = len(src)
+        _lib.check(lib.ptv3_gather_rows((ctypes.c_void_p * k)(*src), (ctypes.c_void_p * k)(*dst), (ctypes.c_int64 * k)(*row), k,
+                                        _ptr(index), m, _stream()), "ptv3_gather_rows")
     return out
 
 

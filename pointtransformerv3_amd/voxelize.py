@@ -29,10 +29,9 @@ def grid_sample(coord, offset, grid_size, feat=None, keys=(), mode="test", seed=
         pick = int(torch.randint(1, 2 ** 32, (1,)).item()) if seed is None else (int(seed) % (2 ** 32 - 1)) + 1
     vox = ops.voxelize(coord, offset, grid_size, seed=pick)
     index = vox["index"]
-    out = dict(coord=coord[index], grid_coord=vox["grid_coord"], offset=vox["offset"], grid_size=grid_size,
+    names = ["coord"] + (["feat"] if feat is not None else []) + [name for name, _ in keys]
+    rows = ops.gather_rows([coord] + ([feat] if feat is not None else []) + [tensor for _, tensor in keys], index)
+    out = dict(coord=None, grid_coord=vox["grid_coord"], offset=vox["offset"], grid_size=grid_size,
                index=index, inverse=vox["inverse"])
-    if feat is not None:
-        out["feat"] = feat[index]
-    for name, tensor in keys:
-        out[name] = tensor[index]
+    out.update(zip(names, rows))
     return out
