@@ -636,6 +636,16 @@ int ptv3_block_tail_fused(const void *attn, const void *shortcut, const void *w_
                           const void *b1, const void *w2, const void *b2, int dtype, int64_t n,
                           int channels, int hidden, void *out, void *stream);
 
+/* The same second half of a block layer by layer (model.py:485-487, :594-595, :599-602), for few rows: 64, 256 and 512
+ * channels where ptv3_block_tail_few_pays says so. Weights as nn.Linear stores them (w1 (4 channels, channels), w2 the
+ * other way), biases may be NULL; workspace of ptv3_block_tail_few_bytes. fp16/bf16, channels in 64s. */
+int ptv3_block_tail_few_pays(int64_t n, int channels);
+size_t ptv3_block_tail_few_bytes(int64_t n, int channels);
+int ptv3_block_tail_few(const void *attn, const void *shortcut, const void *w_proj, const void *b_proj,
+                        const void *ln2_gamma, const void *ln2_beta, float ln2_eps, const void *w1, const void *b1,
+                        const void *w2, const void *b2, int dtype, int64_t n, int channels, void *workspace,
+                        size_t workspace_bytes, void *out, void *stream);
+
 /* ---- The index of a whole forward: what follows from the coordinates alone, every encoder level at once ------------
  * (model.py:81-136 serialization, :138-174 sparsify, :382-453 padding and slot tables, :652-703 pooled tables, and the
  * pair and tile lists of the convolutions). Four stages, each queued on `stream`; between them the caller waits

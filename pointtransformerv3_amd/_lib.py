@@ -80,6 +80,9 @@ SIGNATURES = {
     "ptv3_bn_act": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _i32, _i64, _i32, _f32, _i32, _vp, _vp]),
     "ptv3_linear_fwd": (_i32, [_vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _vp]),
     "ptv3_linear_wide_fwd": (_i32, [_vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _vp]),
+    "ptv3_block_tail_few_pays": (_i32, [_i64, _i32]),
+    "ptv3_block_tail_few_bytes": (_sz, [_i64, _i32]),
+    "ptv3_block_tail_few": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _vp, _sz, _vp, _vp]),
     "ptv3_linear_gemm_fwd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _vp, _vp]),
     "ptv3_linear_any_fwd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _vp]),
     "ptv3_linear_f32_fwd": (_i32, [_vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _vp]),

@@ -103,6 +103,9 @@ int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, co
     const int c = b.channels;
     const size_t mark = r.mem.at;
     void *conv = r.rows(n, c), *feat = r.rows(n, c), *qkv = r.rows(n, 3 * c), *attn = r.rows(n, c), *normed = r.rows(n, c);
+    const bool few = ptv3_block_tail_few_pays(n, c);
+    const size_t few_bytes = few ? ptv3_block_tail_few_bytes(n, c) : 0;
+    void* few_ws = few ? r.mem.take(few_bytes) : nullptr;
     TRY(conv3(r, b, v, xs, conv));
     if (!r.dry) {
         if (c <= 64) {
@@ -112,7 +115,7 @@ int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, co
             TRY(ptv3_block_head_wide(conv, x, b.head_packed, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b,
                                      b.ln1.eps, b.qkv.b, r.dt, n, c, feat, qkv, r.stream));
         } else {
-            if (c == 256) {
+            if (c == 256 && !few) {
                 TRY(ptv3_linear_ln_fwd(conv, b.cpe.w, b.cpe.b, x, b.ln_cpe.g, b.ln_cpe.b, b.ln1.g, b.ln1.b, nullptr, r.dt, n, c, 3,
                                        b.ln_cpe.eps, feat, normed, r.stream));
             } else {
@@ -123,7 +126,10 @@ int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, co
             TRY(linear(r, normed, b.qkv, n, qkv));
         }
         TRY(attention(r, b, v, patch, qkv, r.dt, attn));
-        if (c <= 64) {
+        if (few) {
+            TRY(ptv3_block_tail_few(attn, feat, b.proj.w, b.proj.b, b.ln2.g, b.ln2.b, b.ln2.eps, b.fc1.w, b.fc1.b, b.fc2.w, b.fc2.b,
+                                    r.dt, n, c, few_ws, few_bytes, out, r.stream));
+        } else if (c <= 64) {
             TRY(ptv3_block_tail_fused(attn, feat, b.proj.w, b.proj.b, b.ln2.g, b.ln2.b, b.ln2.eps, b.fc1.w, b.fc1.b, b.fc2.w,
                                       b.fc2.b, r.dt, n, c, 4 * c, out, r.stream));
         } else if (c <= 256) {

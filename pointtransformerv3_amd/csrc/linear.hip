@@ -12,6 +12,7 @@
 // written once; rows move between global memory and registers as contiguous 16-byte pieces
 // through a wave-private LDS buffer. The bias, and for fc1 the exact GELU, are applied on the
 // accumulators; results are rounded to the storage type once, as the separate layers round.
+#include "lintile.h"
 #include "rowtile.h"
 
 namespace {
@@ -33,7 +34,6 @@ struct LinBn {
 // what follows the bias (and the BatchNorm): nothing, the exact GELU, the GELU with the value in front of it
 // kept in aux as well (training: its backward needs it), or a multiplication by gelu'(aux) -- the input
 // gradient of a Linear whose input came out of a GELU (model.py:505-507, fc2 back through act)
-enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_KEEP = 2, ACT_GELU_GRAD = 3 };
 
 // NW waves per work-group, rows staged SW channels at a time (64, or 32 where the weights leave LDS for
 // narrow tile buffers only and the work-group has 16 waves instead of 8)
@@ -282,11 +282,19 @@ int launch_linear(const void* x, const void* w, const void* bias, LinBn bn, int6
 // act: one of ACT_*; the BatchNorm epilogue comes with ACT_NONE and ACT_GELU only
 int dispatch_linear(const void* x, const void* w, const void* bias, const LinBn* bn, int dtype, int64_t n, int k,
                     int nout, int act, void* out, void* aux, hipStream_t stream) {
+    const int kind = bn ? (act ? ACT_BN_GELU : ACT_BN) : act;
+    if (lin_tiled_pays(n, k, nout, kind)) {
+        LinArgs a = {};
+        a.x = x, a.w = w, a.bias = bias, a.n = n, a.k = k, a.nout = nout, a.act = kind, a.out = out, a.aux = aux;
+        if (bn) a.mean = bn->mean, a.var = bn->var, a.gamma = bn->gamma, a.beta = bn->beta, a.bn_eps = bn->eps, a.stats_f32 = bn->stats_f32;
+        return lin_tiled(a, dtype, stream);
+    }
     const LinBn none = {nullptr, nullptr, nullptr, nullptr, 0.f, 0};
 #define PTV3_LIN(T, K)                                                                                                \
     if (k == K) {                                                                                                     \
-        if (bn) return act ? launch_linear<T, K, ACT_GELU, true>(x, w, bias, *bn, n, nout, out, aux, stream)          \
-                           : launch_linear<T, K, ACT_NONE, true>(x, w, bias, *bn, n, nout, out, aux, stream);         \
+        if constexpr (K < 256)                                                                                        \
+            if (bn) return act ? launch_linear<T, K, ACT_GELU, true>(x, w, bias, *bn, n, nout, out, aux, stream)      \
+                               : launch_linear<T, K, ACT_NONE, true>(x, w, bias, *bn, n, nout, out, aux, stream);     \
         switch (act) {                                                                                                \
             case ACT_NONE: return launch_linear<T, K, ACT_NONE, false>(x, w, bias, none, n, nout, out, aux, stream);  \
             case ACT_GELU: return launch_linear<T, K, ACT_GELU, false>(x, w, bias, none, n, nout, out, aux, stream);  \
@@ -305,9 +313,9 @@ int dispatch_linear(const void* x, const void* w, const void* bias, const LinBn*
     }
 #undef PTV3_LIN3
     if (dtype == PTV3_F16) {
-        PTV3_LIN(_Float16, 32) PTV3_LIN(_Float16, 64) PTV3_LIN(_Float16, 128) PTV3_LIN(_Float16, 256) PTV3_LIN(_Float16, 512)
+        PTV3_LIN(_Float16, 32) PTV3_LIN(_Float16, 64) PTV3_LIN(_Float16, 128) PTV3_LIN(_Float16, 256)
     } else {
-        PTV3_LIN(__bf16, 32) PTV3_LIN(__bf16, 64) PTV3_LIN(__bf16, 128) PTV3_LIN(__bf16, 256) PTV3_LIN(__bf16, 512)
+        PTV3_LIN(__bf16, 32) PTV3_LIN(__bf16, 64) PTV3_LIN(__bf16, 128) PTV3_LIN(__bf16, 256)
     }
 #undef PTV3_LIN
     return PTV3_ESHAPE;

@@ -15,6 +15,7 @@
 // next four steps (a whole tile) are in flight in a ring of registers that runs on across tile boundaries.
 // Bias and the exact GELU are applied on the accumulators; results are rounded to the storage type once and leave
 // as whole row segments (8 rows x 128 B per store) through the wave's own LDS rows.
+#include "lintile.h"
 #include "rowtile.h"
 
 namespace {
@@ -480,191 +481,6 @@ int launch_linear_wide(const void* x, const void* w, const void* bias, int64_t n
     return e == hipSuccess ? PTV3_OK : (int)e;
 }
 
-
-// ---- Linear layers with long contractions (fc2 of the 256- and 512-channel blocks: 1024 -> 256, 2048 -> 512;
-// the 512 -> 1536 qkv): out = resid + x W^T + b, an LDS-tiled GEMM. A work-group of 4 waves owns a
-// (MT * 64) x 128 tile of the result; a wave multiplies MT * 32 rows by 64 output channels (MT x 2 accumulator
-// tiles: with MT = 4 six operand fragments feed eight MFMAs, 0.75 KB of LDS traffic per MFMA). Both operands
-// come through LDS in 64-channel steps, double-buffered, one barrier per step; the pieces of the next two steps
-// are in flight in registers. The residual (the stored sum fc2 accumulates onto, model.py:602) is added in fp32
-// before the single rounding.
-// A 128 x 128 tile moves (128 + 128) x K x 2 bytes out of L2 for 2 x 128 x 128 x K flops, 64 flop per byte: at the
-// ~6.5 TB/s the L2s deliver to 256 CUs that is ~410 TFLOP/s, which is what this kernel measures on all three
-// shapes (43-48 us; a 256 x 160 tile would move 98 flop per byte). In the default model it takes the two
-// 512 -> 1536 qkv layers; fc2 of the wide blocks runs inside the fused MLP kernel.
-constexpr int GT_THREADS = 256;
-constexpr int GT_N = 128, GT_KC = 64;
-constexpr int GT_STRIDE = GT_KC + 8;         // halfs per staged row
-constexpr int GT_OSTRIDE = 64 + 8;           // halfs per row of a wave's result staging
-constexpr int GT_DEPTH = 2;
-
-template <typename T, int MT>
-__global__ __launch_bounds__(GT_THREADS, 2) void linear_gemm_kernel(
-    const T* __restrict__ x, const T* __restrict__ weight, const T* __restrict__ bias, const T* resid,
-    int64_t n, int k, int nout, T* out) {   // resid may be out itself (fc2 accumulating onto the stored sum)
-    typedef typename H16<T>::v8 v8;
-    constexpr int GT_M = MT * 64;
-    constexpr int XBUF = GT_M * GT_STRIDE, WBUF = GT_N * GT_STRIDE;
-    constexpr int PPR = GT_KC / 8;                                           // 16-byte pieces per staged row
-    constexpr int RPS = GT_THREADS / PPR;                                    // rows staged per pass of the work-group
-    constexpr int XP = GT_M / RPS, WP = GT_N / RPS;                          // pieces per thread and step
-    extern __shared__ __align__(16) unsigned char gt_smem[];
-    T* lds = (T*)gt_smem;                                // [2 buffers][x tile | w tile]
-    static_assert(4 * 32 * GT_OSTRIDE <= 2 * (XBUF + WBUF), "the waves' staging rows fit where the operands were");
-    static_assert(GT_M % RPS == 0 && GT_N % RPS == 0, "whole passes");
-    const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
-    const int col = lane & 31, hf = lane >> 5;
-    const int64_t m0 = (int64_t)blockIdx.x * GT_M;
-    const int n0 = blockIdx.y * GT_N;
-    const int wr = (wave >> 1) * (MT * 32), wc = (wave & 1) * 64;   // the wave's rows and output channels inside the tile
-    // staging: thread -> row tid / PPR (+ RPS i), 16-byte piece tid % PPR; rows past the end repeat the last row
-    const int srow = tid / PPR, spc = tid % PPR;
-    const T* xp[XP];
-    const T* wp[WP];
-#pragma unroll
-    for (int i = 0; i < XP; ++i) {
-        const int64_t r = m0 + srow + RPS * i;
-        xp[i] = x + (r < n ? r : n - 1) * k + spc * 8;
-    }
-#pragma unroll
-    for (int i = 0; i < WP; ++i) wp[i] = weight + (int64_t)(n0 + srow + RPS * i) * k + spc * 8;
-    const int steps = k / GT_KC;
-    u32x4 xr[GT_DEPTH][XP], wr4[GT_DEPTH][WP];
-#pragma unroll
-    for (int d = 0; d < GT_DEPTH; ++d) {
-        const int sd = d < steps ? d : steps - 1;
-#pragma unroll
-        for (int i = 0; i < XP; ++i) xr[d][i] = *(const u32x4*)(xp[i] + sd * GT_KC);
-#pragma unroll
-        for (int i = 0; i < WP; ++i) wr4[d][i] = *(const u32x4*)(wp[i] + sd * GT_KC);
-    }
-    f32x16 acc[MT][2];
-#pragma unroll
-    for (int a = 0; a < MT; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-    // nothing in flight when the loop is entered: the wait-count bookkeeping of a loop is the union of its entry
-    // and its back edge, and with loads pending at entry it settled for draining everything once per trip
-#pragma unroll
-    for (int d = 0; d < GT_DEPTH; ++d) {
-#pragma unroll
-        for (int i = 0; i < XP; ++i) asm volatile("" ::"v"(xr[d][i]));
-#pragma unroll
-        for (int i = 0; i < WP; ++i) asm volatile("" ::"v"(wr4[d][i]));
-    }
-    // two steps per trip so that the ring position and the buffer are compile-time constants (steps is even)
-    for (int s0 = 0; s0 < steps; s0 += 2) {
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const int s = s0 + d;
-            T* xb = lds + d * (XBUF + WBUF);
-            T* wb = xb + XBUF;
-#pragma unroll
-            for (int i = 0; i < XP; ++i) *(u32x4*)(xb + (srow + RPS * i) * GT_STRIDE + spc * 8) = xr[d][i];
-#pragma unroll
-            for (int i = 0; i < WP; ++i) *(u32x4*)(wb + (srow + RPS * i) * GT_STRIDE + spc * 8) = wr4[d][i];
-            const int sn = s + GT_DEPTH < steps ? s + GT_DEPTH : steps - 1;   // past the end: a valid address, never used
-#pragma unroll
-            for (int i = 0; i < XP; ++i) xr[d][i] = *(const u32x4*)(xp[i] + sn * GT_KC);
-#pragma unroll
-            for (int i = 0; i < WP; ++i) wr4[d][i] = *(const u32x4*)(wp[i] + sn * GT_KC);
-            __syncthreads();
-#pragma unroll
-            for (int ks = 0; ks < GT_KC / 16; ++ks) {
-                u32x4 xf[MT], wf[2];
-#pragma unroll
-                for (int a = 0; a < MT; ++a) xf[a] = *(const u32x4*)(xb + (wr + a * 32 + col) * GT_STRIDE + ks * 16 + hf * 8);
-#pragma unroll
-                for (int b = 0; b < 2; ++b) wf[b] = *(const u32x4*)(wb + (wc + b * 32 + col) * GT_STRIDE + ks * 16 + hf * 8);
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int a = 0; a < MT; ++a)
-                        acc[a][b] = H16<T>::mfma(__builtin_bit_cast(v8, wf[b]), __builtin_bit_cast(v8, xf[a]), acc[a][b]);
-            }
-        }
-    }
-    __syncthreads();   // every wave is through with the operand tiles: their room takes the results
-    // acc[a][b][v]: output channel n0 + wc + b*32 + 8*(v/4) + 4*hf + v%4 of row m0 + wr + a*32 + col
-    T* stage = lds + wave * (32 * GT_OSTRIDE);
-    // bias of the lane's output channels: 4 consecutive ones per (b, q)
-    float bb[2][4][4];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int c = n0 + wc + b * 32 + 8 * q + 4 * hf;
-            u32x2 raw = {0u, 0u};
-            if (bias) raw = *(const u32x2*)(bias + c);
-            bb[b][q][0] = H16<T>::lo(raw[0]); bb[b][q][1] = H16<T>::hi(raw[0]);
-            bb[b][q][2] = H16<T>::lo(raw[1]); bb[b][q][3] = H16<T>::hi(raw[1]);
-        }
-#pragma unroll
-    for (int a = 0; a < MT; ++a) {
-        // the residual rows come in as whole row segments (8 rows x 128 B per load) and pass through the wave's
-        // LDS rows into the accumulators' layout: one 8-byte piece per lane read straight from memory would touch
-        // 32 cache lines per instruction
-        if (resid) {
-#pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int orow = it * 8 + (lane >> 3), opc = lane & 7;
-                const int64_t row = m0 + wr + a * 32 + orow;
-                u32x4 old = {0u, 0u, 0u, 0u};
-                if (row < n) old = *(const u32x4*)(resid + row * nout + n0 + wc + opc * 8);
-                *(u32x4*)(stage + orow * GT_OSTRIDE + opc * 8) = old;
-            }
-            asm volatile("" ::: "memory");
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                T* at = stage + col * GT_OSTRIDE + b * 32 + 8 * q + 4 * hf;
-                float r[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) r[i] = acc[a][b][4 * q + i] + bb[b][q][i];
-                if (resid) {
-                    const u32x2 old = *(const u32x2*)at;
-                    r[0] += H16<T>::lo(old[0]); r[1] += H16<T>::hi(old[0]);
-                    r[2] += H16<T>::lo(old[1]); r[3] += H16<T>::hi(old[1]);
-                }
-                *(u32x2*)at = (u32x2){H16<T>::pack2(r[0], r[1]), H16<T>::pack2(r[2], r[3])};
-            }
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int orow = it * 8 + (lane >> 3), opc = lane & 7;
-            const u32x4 val = *(const u32x4*)(stage + orow * GT_OSTRIDE + opc * 8);
-            const int64_t row = m0 + wr + a * 32 + orow;
-            if (row < n) *(u32x4*)(out + row * nout + n0 + wc + opc * 8) = val;
-        }
-        asm volatile("" ::: "memory");
-    }
-}
-
-template <typename T, int MT>
-int launch_linear_gemm_mt(const void* x, const void* w, const void* bias, const void* resid, int64_t n, int k, int nout,
-                          void* out, hipStream_t stream) {
-    const size_t lds = 2 * (size_t)(MT * 64 + GT_N) * GT_STRIDE * sizeof(T);
-    auto kern = linear_gemm_kernel<T, MT>;
-    static LdsGrant grant_allowed;   // per instantiation and device
-    if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_allowed)) return rc_;
-    hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n, MT * 64), (unsigned)(nout / GT_N)), dim3(GT_THREADS), lds,
-                       stream, (const T*)x, (const T*)w, (const T*)bias, (const T*)resid, n, k, nout, (T*)out);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? PTV3_OK : (int)e;
-}
-
-template <typename T>
-int launch_linear_gemm(const void* x, const void* w, const void* bias, const void* resid, int64_t n, int k, int nout,
-                       void* out, hipStream_t stream) {
-    // 128 x 128 tiles: 256-row tiles would halve the weight traffic per row but need more registers than two
-    // work-groups per CU leave, and on these shapes give fewer work-groups than there are CUs
-    return launch_linear_gemm_mt<T, 2>(x, w, bias, resid, n, k, nout, out, stream);
-}
-
 }  // namespace
 
 // called by ptv3_linear_ln_fwd for 256 channels (modes 2 and 3)
@@ -692,21 +508,14 @@ extern "C" int ptv3_linear_wide_fwd(const void* x, const void* w, const void* bi
     if (n == 0) return PTV3_OK;
     if (!x || !w || !out) return PTV3_EINVAL;
     hipStream_t stream = (hipStream_t)stream_;
+    if (lin_tiled_pays(n, k, nout, gelu ? ACT_GELU : ACT_NONE)) {
+        LinArgs a = {};
+        a.x = x, a.w = w, a.bias = bias, a.n = n, a.k = k, a.nout = nout, a.act = gelu ? ACT_GELU : ACT_NONE, a.out = out;
+        return lin_tiled(a, dtype, stream);
+    }
     if (dtype == PTV3_F16)
         return gelu ? launch_linear_wide<_Float16, true>(x, w, bias, n, nout, out, stream)
                     : launch_linear_wide<_Float16, false>(x, w, bias, n, nout, out, stream);
     return gelu ? launch_linear_wide<__bf16, true>(x, w, bias, n, nout, out, stream)
                 : launch_linear_wide<__bf16, false>(x, w, bias, n, nout, out, stream);
-}
-
-extern "C" int ptv3_linear_gemm_fwd(const void* x, const void* w, const void* bias, const void* resid, int dtype,
-                                    int64_t n, int k, int nout, void* out, void* stream_) {
-    if (n < 0 || k < 1 || nout < 1) return PTV3_EINVAL;
-    if (dtype != PTV3_F16 && dtype != PTV3_BF16) return PTV3_ESHAPE;
-    if (k % (2 * GT_KC) != 0 || nout % GT_N != 0) return PTV3_ESHAPE;
-    if (n == 0) return PTV3_OK;
-    if (!x || !w || !out) return PTV3_EINVAL;
-    hipStream_t stream = (hipStream_t)stream_;
-    if (dtype == PTV3_F16) return launch_linear_gemm<_Float16>(x, w, bias, resid, n, k, nout, out, stream);
-    return launch_linear_gemm<__bf16>(x, w, bias, resid, n, k, nout, out, stream);
 }

@@ -1,0 +1,23 @@
+// Linear layers as tiles of the output (lintile.hip), for the layers' own files to hand small and long shapes to.
+#pragma once
+#include "common.h"
+
+enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_KEEP = 2, ACT_GELU_GRAD = 3, ACT_BN = 4, ACT_BN_GELU = 5 };
+
+struct LinArgs {
+    const void *x, *w, *bias;                   // (n, k), (nout, k), (nout,) or NULL
+    int64_t n;
+    int k, nout, act;
+    int row_tiles, col_tiles, order;            // filled in by the launch
+    const void* resid;                          // ACT_NONE: added in fp32; may be out
+    void* aux;                                  // ACT_GELU_KEEP: the value in front of the GELU, out; ACT_GELU_GRAD: in
+    const void *mean, *var, *gamma, *beta;      // ACT_BN, ACT_BN_GELU
+    float bn_eps;
+    int stats_f32;
+    void* out;
+};
+
+// whether the tiled form takes the layer and is the faster one
+bool lin_tiled_pays(int64_t n, int k, int nout, int act);
+bool lin_tiled_takes(int k, int nout);
+int lin_tiled(LinArgs& a, int dtype, hipStream_t stream);

@@ -432,7 +432,8 @@ class Block(PointModule):
             # HBM and back, so the block runs as conv, head kernel, attention, tail kernel
             feat, qkv = ops.block_head_fused(conv, point.feat, self.cpe[1], ln_cpe, ln1, self.attn.qkv)
             attn = self.attn.attend(point, qkv)
-            feat = ops.block_tail_fused(attn, feat, self.attn.proj, ln2, mlp.fc1, mlp.fc2)
+            tail = ops.block_tail_few if ops.block_tail_few_pays(feat.shape[0], self.channels) else ops.block_tail_fused
+            feat = tail(attn, feat, self.attn.proj, ln2, mlp.fc1, mlp.fc2)
             point.feat = feat
             point.sparse_conv_feat = point.sparse_conv_feat.replace_feature(feat)
             return point
@@ -443,7 +444,7 @@ class Block(PointModule):
                 and self.attn.enable_flash):
             # cpe Linear, its LayerNorm, the residual, the attention's pre-norm and qkv in one kernel
             feat, qkv = ops.block_head_wide(conv, point.feat, self.cpe[1], ln_cpe, ln1, self.attn.qkv)
-        elif ops.linear_ln_ok(conv, self.cpe[1]) and same_eps:
+        elif ops.linear_ln_ok(conv, self.cpe[1]) and same_eps and not ops.block_tail_few_pays(conv.shape[0], self.channels):
             # cpe Linear, its LayerNorm, the residual and the attention's pre-norm in one kernel
             feat, normed = ops.linear_ln(conv, self.cpe[1], point.feat, ln_cpe, 3, ln2=ln1)
         else:
@@ -459,10 +460,12 @@ class Block(PointModule):
             point.feat = normed
             qkv = self.attn.qkv_rows(normed)
         attn_out = self.attn.attend(point, qkv)
-        if (fused_mlp and attn_out.dtype == feat.dtype and self.channels in ops.BLOCK_TAIL_WIDE_CHANNELS and type(self.attn.proj) is nn.Linear
+        few = fused_mlp and ops.block_tail_few_pays(feat.shape[0], self.channels)
+        if (fused_mlp and attn_out.dtype == feat.dtype and (few or self.channels in ops.BLOCK_TAIL_WIDE_CHANNELS) and type(self.attn.proj) is nn.Linear
                 and self.attn.proj.bias is not None and not (self.training and self.attn.proj_drop.p > 0)):
-            # proj, the residual, the MLP's pre-norm and the MLP with its residual in one kernel
-            feat = ops.block_tail_wide(attn_out, feat, self.attn.proj, ln2, mlp)
+            # proj, the residual, the MLP's pre-norm and the MLP with its residual: one kernel, or a few short ones
+            feat = (ops.block_tail_few(attn_out, feat, self.attn.proj, ln2, mlp.fc1, mlp.fc2) if few
+                    else ops.block_tail_wide(attn_out, feat, self.attn.proj, ln2, mlp))
             point.feat = feat
             point.sparse_conv_feat = point.sparse_conv_feat.replace_feature(feat)
             return point

@@ -1672,6 +1672,29 @@ def block_tail_wide(attn, shortcut, proj, ln2, mlp):
     return out
 
 
+def block_tail_few_pays(n, channels):
+    """Whether the second half of a block of n rows is faster layer by layer (ptv3_block_tail_few_pays)."""
+    return bool(_lib.load().ptv3_block_tail_few_pays(n, channels))
+
+
+def block_tail_few(attn, shortcut, proj, ln2, fc1, fc2):
+    """block_tail_wide / block_tail_fused layer by layer, for few rows: the modules' own weights, no packed copies."""
+    _dev(attn, shortcut, proj.weight, fc1.weight, fc2.weight)
+    lib = _lib.load()
+    attn = attn.contiguous()
+    dt = attn.dtype
+    shortcut = shortcut.to(dt).contiguous()
+    n, c = attn.shape
+    keep = [None if t is None else cast_cached(t, dt).detach().contiguous()
+            for t in (proj.weight, proj.bias, ln2.weight, ln2.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias)]
+    wp, bp, g, be, w1, b1, w2, b2 = [_ptr(t) for t in keep]
+    nbytes = lib.ptv3_block_tail_few_bytes(n, c)
+    ws, out = _ws(nbytes, attn.device), torch.empty_like(attn)
+    _lib.check(lib.ptv3_block_tail_few(_ptr(attn), _ptr(shortcut), wp, bp, g, be, float(ln2.eps), w1, b1, w2, b2, _dtype_code(attn),
+                                       n, c, _ptr(ws), nbytes, _ptr(out), _stream()), "ptv3_block_tail_few")
+    return out
+
+
 def mlp_fused_module(x, resid, mlp):
     """resid + mlp(x) from the fused kernel for a module with fc1 and fc2. At MLP_PACKED_CHANNELS the weights go
     through a packed copy that the module keeps per dtype and that is redone, in place, when a parameter may have
