@@ -321,9 +321,13 @@ bool net_ok(const ptv3_net* net, const ptv3_level* lv) {
 
 // The form the 3x3x3 convolution of a half-precision level takes: 0 pair lists, 1 sparse tiles, 2 tiles. The rule on pairs
 // per voxel: 32 and 64 channels take the sparse tile form up to 14 (work in proportion to the pairs; faster than both other
-// forms from 2.5 to 10), 64 and 128 the tile form from 4 on (sums kept on chip, no pair matrix through memory).
+// forms from 2.5 to 10), 64 and 128 the tile form from 4 on (sums kept on chip, no pair matrix through memory). A tile
+// walks its taps one after the other, 14 - 23 us (64 channels) or 42 - 54 us (128) however few tiles there are, while the
+// pair form is two short launches that spread over the part: 64 channels 11 against 14 us at 20k pairs, 16 against 17 at
+// 71k, 25 against 21 at 139k; 128 channels 13 against 42 us at 7k pairs, 33 against 43 at 201k, 60 against 54 at 420k.
 extern "C" int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels) {
     if (n < 1 || n >= (1ll << 24)) return 0;
+    if ((channels == 64 && n_pairs <= 70000) || (channels == 128 && n_pairs <= 300000)) return 0;
     if ((channels == 32 || channels == 64) && n_pairs <= 14 * n) return 1;
     if ((channels == 64 || channels == 128) && n_pairs >= 4 * n) return 2;
     return 0;
