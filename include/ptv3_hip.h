@@ -669,7 +669,6 @@ int ptv3_block_tail_few(const void *attn, const void *shortcut, const void *w_pr
 #define PTV3_LISTS_TILES 2                  /* 3x3x3: tile_tap, tile_pair, vox_taps */
 #define PTV3_LISTS_PAIRS5 4                 /* level 0, 5x5x5 */
 #define PTV3_LISTS_PAIR_OUT 8               /* with PAIRS: the output voxel of every pair (weight gradients) */
-#define PTV3_LISTS_NBR 16                   /* 3x3x3 neighbour map, tap-major (27, n), -1 where there is none */
 #define PTV3_LISTS_PAIR_OUT5 32             /* with PAIRS5 */
 
 typedef struct ptv3_index_cfg {
@@ -696,7 +695,7 @@ typedef struct ptv3_level {
     int32_t *slot_src[PTV3_MAX_ORDERS], *slot_dst[PTV3_MAX_ORDERS];
     int32_t *tap_ptr, *row_ptr, *pair_in, *pair_slot, *tile_tap, *tile_pair, *vox_taps;
     int32_t *tap_ptr5, *row_ptr5, *pair_in5, *pair_slot5;
-    int32_t *pair_out, *pair_out5, *nbr;
+    int32_t *pair_out, *pair_out5;
     int32_t tile_voxels, depth;
 } ptv3_level;
 

@@ -76,10 +76,8 @@ class SubMConv(torch.autograd.Function):
             if x.dtype != torch.float32 and cin % 8:
                 x = torch.nn.functional.pad(x, (0, -cin % 8))   # the matrix-core kernel reads channels 8 at a time
             want_bias = ctx.has_bias and ctx.needs_input_grad[2]
-            if x.dtype != torch.float32 and cout % 8 == 0 and min(x.shape[1], cout) < ops.OUTER_WIDE_CHANNELS:
+            if x.dtype != torch.float32 and cout % 8 == 0:
                 # the forward's pair lists: no neighbour map to build, no compaction, ranges of equal length
-                # (half the time on the 64 x 64 block kernel; the 128 x 128 one measured 10 % slower that way:
-                # it wants more and shorter work-groups than full ranges give it)
                 dw, db = ops.subm_conv_wgrad_pairs(x, dout, sparse.conv_plan(module.kernel_size, module.indice_key),
                                                    with_bias=True)
             else:

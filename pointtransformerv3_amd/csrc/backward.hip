@@ -36,6 +36,7 @@
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int WG_T = 64;     // weight block: WG_T output x WG_T input channels
@@ -129,7 +130,9 @@ __device__ __forceinline__ bool outer_item(int taps, int splits, int m_total, in
     if (x >= (int64_t)taps * splits) return false;
     const int blk = slot % (bm * bk);
     *tap = (int)(x / splits);
-    *split = (int)(x % splits);
+    // (turned by the tap: only a tap with many pairs reaches the last ranges, and with splits a multiple of 8 those would
+    // all be one XCD's)
+    *split = (int)((x + *tap) % splits);
     *m0 = (blk % bm) * SIDE;
     *k0 = (blk / bm) * SIDE;
     return true;
@@ -493,13 +496,49 @@ struct SlabJobs {
     SlabJob job[SLAB_JOBS];
 };
 
+// A result of SLAB_LARGE values or more fills the part with four neighbouring values a thread, eight slabs in flight. In the
+// form above such a result is a work-group per 32 values, most of it idle with the few slabs it has (7 - 20): the weight
+// gradient of 9.6k x 512 with its sum 295 -> 208 us, of a Linear 600 x 512 -> 2048 32 -> 20 us.
+constexpr int64_t SLAB_LARGE = 1 << 18;
+__device__ __forceinline__ void slab_sum_large(const SlabJob& job, int block) {
+    const int64_t i = ((int64_t)block * 256 + threadIdx.x) * 4;
+    if (i >= job.total) return;
+    const float* slabs = job.slabs + i;
+    const int64_t stride = job.stride;
+    int splits = job.splits;
+    if (job.tap_ptr && i < job.first) {   // k_total is a multiple of 4: the four values share their tap
+        const int t = (int)(((uint32_t)i / (uint32_t)job.k_total) % (uint32_t)job.taps);
+        const int64_t have = ((int64_t)job.tap_ptr[t + 1] - job.tap_ptr[t] + job.rows_per_split - 1) / job.rows_per_split;
+        if (have < splits) splits = (int)have;
+    }
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < splits; s += 8) {
+        f32x4 p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = *(const f32x4*)(slabs + (int64_t)min(s + u, splits - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + u < splits) v += p[u];
+    }
+    float* out = i < job.first ? job.out + i : job.out2 + (i - job.first);   // a slab's tail goes to the second result
+    if (((uintptr_t)out & 15) == 0) {
+        *(f32x4*)out = v;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) out[u] = v[u];
+    }
+}
+int64_t slab_blocks(const SlabJob& job) { return ptv3_ceil_div(job.total, job.total >= SLAB_LARGE ? 1024 : 32); }
+
 __global__ __launch_bounds__(256) void slab_sum_kernel(SlabJobs jobs) {
     __shared__ float part[8][32];
     int which = 0;
     while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.first_block[which + 1]) ++which;
     const SlabJob& job = jobs.job[which];
+    const int block = (int)blockIdx.x - jobs.first_block[which];
+    if (job.total >= SLAB_LARGE) return slab_sum_large(job, block);
     const int e = threadIdx.x % 32, lane_s = threadIdx.x / 32;
-    const int64_t i = (int64_t)((int)blockIdx.x - jobs.first_block[which]) * 32 + e;
+    const int64_t i = (int64_t)block * 32 + e;
     const float* slabs = job.slabs;
     const int64_t stride = job.stride;
     int splits = job.splits;
@@ -1208,14 +1247,35 @@ void outer_split(int64_t n, int64_t blocks, int taps, int64_t cap, int64_t* spli
     *splits = ptv3_ceil_div(n, r);
 }
 
+// Rows per range of the gathering 128 x 128 form. Over all taps there are about ten pairs per voxel at the levels that have
+// these widths: about 1200 work-groups, between the slabs that shorter ranges write (384 rows: 246 against 168 us at 156k
+// x 128) and the uneven end of longer ones (4096: 284 against 200 us at 43k x 256). A result whose blocks and taps alone
+// fill the part is left without slabs while its rows are few (570 x 512: 22 us against 49 in two ranges).
+int64_t outer_gather_rows(int64_t n, int64_t blocks, int taps) {
+    if (n <= 1024 && blocks * taps >= 256) return ptv3_ceil_div(n, 128) * 128;
+    const int64_t r = ptv3_ceil_div(n * blocks, 120 * 128) * 128;
+    return r < 384 ? 384 : r > 1408 ? 1408 : r;
+}
+
 // block side: 128 when both sides of the result have that many channels, else 64
 int outer_side(int m_total, int k_total) { return (m_total >= OW_C && k_total >= OW_C) ? OW_C : OR_C; }
 
 template <bool GATHER>
-size_t outer_workspace(int64_t n, int m_total, int k_total, int taps) {
+void outer_ranges(int64_t n, int m_total, int k_total, int taps, int64_t* splits, int64_t* rows) {
     const int side = outer_side(m_total, k_total);
+    const int64_t blocks = ptv3_ceil_div(m_total, side) * ptv3_ceil_div(k_total, side);
+    if (GATHER && side == OW_C) {
+        *rows = outer_gather_rows(n, blocks, taps);
+        *splits = ptv3_ceil_div(n, *rows);
+    } else {
+        outer_split(n, blocks, taps, GATHER ? OR_LIST : 0, splits, rows);
+    }
+}
+
+template <bool GATHER>
+size_t outer_workspace(int64_t n, int m_total, int k_total, int taps) {
     int64_t splits, rows;
-    outer_split(n, ptv3_ceil_div(m_total, side) * ptv3_ceil_div(k_total, side), taps, GATHER ? OR_LIST : 0, &splits, &rows);
+    outer_ranges<GATHER>(n, m_total, k_total, taps, &splits, &rows);
     return splits > 1 ? ptv3_align256((size_t)splits * ((size_t)m_total * taps * k_total + m_total) * sizeof(float)) : 0;
 }
 
@@ -1227,7 +1287,7 @@ int launch_outer(const void* a, const void* b, int64_t n, int m_total, int k_tot
     const int side = outer_side(m_total, k_total);
     const int64_t bm = ptv3_ceil_div(m_total, side), bk = ptv3_ceil_div(k_total, side);
     int64_t splits, rows;
-    outer_split(n, bm * bk, taps, GATHER ? OR_LIST : 0, &splits, &rows);
+    outer_ranges<GATHER>(n, m_total, k_total, taps, &splits, &rows);
     if ((int64_t)taps * splits >= (1ll << 31)) return PTV3_EINVAL;
     const int64_t count = (int64_t)m_total * taps * k_total;
     const int64_t stride = count + m_total;
@@ -1286,7 +1346,7 @@ int ptv3_slab_sums(const SlabJob* jobs, int count, hipStream_t stream) {
         int blocks = 0;
         for (; at < count && t.count < SLAB_JOBS; ++at) {
             if (!jobs[at].splits) continue;
-            const int64_t b = ptv3_ceil_div(jobs[at].total, 32);
+            const int64_t b = slab_blocks(jobs[at]);
             if (b + blocks >= (1ll << 31)) return PTV3_EINVAL;
             t.first_block[t.count] = blocks;
             t.job[t.count++] = jobs[at];

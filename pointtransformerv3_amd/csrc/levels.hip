@@ -417,7 +417,7 @@ struct ListLevel {
     int32_t *tap_ptr, *row_ptr, *pair_in, *pair_slot, *tile_tap;
     uint32_t *tile_pair, *vox_taps;
     int32_t *tap_ptr5, *row_ptr5, *pair_in5, *pair_slot5;
-    int32_t *pair_out, *pair_out5, *nbr;
+    int32_t *pair_out, *pair_out5;
 };
 
 struct ListArgs {
@@ -608,8 +608,7 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
     };
 
     auto make = [&](uint64_t flo, uint64_t fhi, int taps, int edge, const int32_t* tap_ptr, const uint32_t* tap_off,
-                    const uint32_t* row_off, int32_t* row_ptr, int32_t* pair_in, int32_t* pair_slot, int32_t* pair_out, int32_t* nbr,
-                    bool pairs, bool tiles) {
+                    const uint32_t* row_off, int32_t* row_ptr, int32_t* pair_in, int32_t* pair_slot, int32_t* pair_out, bool pairs, bool tiles) {
         for (int e = tid; e < 256; e += GT) (&mask[0][0])[e] = 0;
         for (int t = tid; t < taps; t += GT) tap_base[t] = pairs ? (uint32_t)tap_ptr[t] + tap_off[(int64_t)g * taps + t] : 0u;
         const uint32_t cnt = (uint32_t)(__popcll(flo) + __popcll(fhi));
@@ -653,9 +652,6 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
             if (tiles && v.vox_taps) v.vox_taps[i] = (uint32_t)flo;
         }
         const bool staged = total <= (uint32_t)STAGE;
-        if (nbr && live)
-            for (int t = 0; t < taps; ++t)
-                if (!((flo >> t) & 1ull)) nbr[(int64_t)t * v.n + i] = -1;
         uint32_t slot = slot0;
         uint64_t f0 = flo, f1 = fhi;
         while (f0 | f1) {
@@ -665,7 +661,6 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
             const int32_t src = source(t / (edge * edge) - edge / 2, (t / edge) % edge - edge / 2, t % edge - edge / 2);
             const uint32_t rank = (uint32_t)__popcll(mask[wave][t] & below) + (wave ? (uint32_t)__popcll(mask[0][t]) : 0u);
             const uint32_t q = tap_base[t] + rank, e = tap_start[t] + rank;
-            if (nbr) nbr[(int64_t)t * v.n + i] = src;
             if (staged) {
                 stage_q[e] = q;
                 stage_in[e] = src;
@@ -699,11 +694,11 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
     };
     if (KS == 5 && (v.want & PTV3_LISTS_PAIRS5))
         make(lo, hi, TAPS5, 5, v.tap_ptr5, v.tap5, v.row5, v.row_ptr5, v.pair_in5, v.pair_slot5,
-             v.pair_out5, nullptr, true, false);
+             v.pair_out5, true, false);
     const bool pairs = v.want & PTV3_LISTS_PAIRS, tiles = v.want & PTV3_LISTS_TILES;
-    if (pairs || tiles || v.nbr)
+    if (pairs || tiles)
         make(KS == 5 ? (uint64_t)inner_taps(lo, hi) : lo, 0, TAPS3, 3, v.tap_ptr, v.tap, v.row, pairs ? v.row_ptr : nullptr,
-             v.pair_in, v.pair_slot, pairs ? v.pair_out : nullptr, v.nbr, pairs, tiles);
+             v.pair_in, v.pair_slot, pairs ? v.pair_out : nullptr, pairs, tiles);
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------------
@@ -1050,14 +1045,13 @@ size_t carve_lists(State& s, const int32_t* want, void* base) {
         v.want = want[l];
         v.row_ptr = v.pair_in = v.pair_slot = v.tile_tap = nullptr;
         v.tile_pair = v.vox_taps = nullptr;
-        v.row_ptr5 = v.pair_in5 = v.pair_slot5 = v.pair_out = v.pair_out5 = v.nbr = nullptr;
+        v.row_ptr5 = v.pair_in5 = v.pair_slot5 = v.pair_out = v.pair_out5 = nullptr;
         if (want[l] & PTV3_LISTS_PAIRS) {
             v.row_ptr = c.take<int32_t>(v.n + 1);
             v.pair_in = c.take<int32_t>(out.n_pairs);
             v.pair_slot = c.take<int32_t>(out.n_pairs);
             if (want[l] & PTV3_LISTS_PAIR_OUT) v.pair_out = c.take<int32_t>(out.n_pairs);
         }
-        if (want[l] & PTV3_LISTS_NBR) v.nbr = c.take<int32_t>(TAPS3 * v.n);
         if (want[l] & PTV3_LISTS_TILES) {
             v.tile_tap = c.take<int32_t>((size_t)v.groups * TILE_WORDS);
             v.tile_pair = c.take<uint32_t>(out.n_pairs);
@@ -1209,7 +1203,6 @@ extern "C" int ptv3_index_lists(void* state, const int32_t* want, void* lists, s
         o.pair_slot5 = v.pair_slot5;
         o.pair_out = v.pair_out;
         o.pair_out5 = v.pair_out5;
-        o.nbr = v.nbr;
         o.tile_voxels = v.group;
     }
     PTV3_RETURN_LAUNCH();

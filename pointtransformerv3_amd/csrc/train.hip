@@ -271,10 +271,8 @@ struct Run {
         const int c = b.channels;
         const size_t bytes = ptv3_subm_conv_wgrad_workspace_bytes(dt, v.n, c, c, 27);
         void* ws = bytes ? scratch.take(bytes) : nullptr;
-        const bool pairs = c < 128;   // the 128 x 128 block kernel measured 10 % slower over pair lists than over the map
-        DO(ptv3_subm_conv_wgrad_slabs(x, dy, dt, v.n, c, c, pairs ? v.pair_out : v.nbr, pairs ? v.tap_ptr : nullptr,
-                                       pairs ? v.pair_in : nullptr, 27, grads + b.g_conv_w, grads + b.g_conv_b, ws, bytes,
-                                       &jobs[n_jobs], hs));
+        DO(ptv3_subm_conv_wgrad_slabs(x, dy, dt, v.n, c, c, v.pair_out, v.tap_ptr, v.pair_in, 27, grads + b.g_conv_w,
+                                       grads + b.g_conv_b, ws, bytes, &jobs[n_jobs], hs));
         return ++n_jobs == SLAB_JOBS ? flush() : PTV3_OK;
     }
     int bn_bwd(const ptv3_train_bn& b, const BnActs& a, int64_t n, int c, const void* dy, void* dx) {

@@ -11,7 +11,7 @@ MAX_LEVELS = MAX_ORDERS = 8
 _STATE_BYTES = 16384
 _SLOT_DATA = hostslot.DATA
 _SLOT_ENDS = _SLOT_DATA + 4 + MAX_LEVELS + 2 * MAX_LEVELS
-PAIRS, TILES, PAIRS5, PAIR_OUT, NBR, PAIR_OUT5 = 1, 2, 4, 8, 16, 32
+PAIRS, TILES, PAIRS5, PAIR_OUT, PAIR_OUT5 = 1, 2, 4, 8, 32
 
 _i32, _i64, _ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p
 
@@ -30,7 +30,7 @@ class Level(ctypes.Structure):
                                        "pad", "unpad", "cu")]
                 + [("slot_src", _ptr * MAX_ORDERS), ("slot_dst", _ptr * MAX_ORDERS)]
                 + [(f, _ptr) for f in ("tap_ptr", "row_ptr", "pair_in", "pair_slot", "tile_tap", "tile_pair", "vox_taps",
-                                       "tap_ptr5", "row_ptr5", "pair_in5", "pair_slot5", "pair_out", "pair_out5", "nbr")]
+                                       "tap_ptr5", "row_ptr5", "pair_in5", "pair_slot5", "pair_out", "pair_out5")]
                 + [("tile_voxels", _i32), ("depth", _i32)])
 
 

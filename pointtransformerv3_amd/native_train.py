@@ -158,7 +158,7 @@ class TrainEngine:
             flags = levels.PAIRS5 | levels.PAIR_OUT5 if level == 0 else 0
             for c in widths[level]:
                 flags |= levels.TILES if form(v.n, v.n_pairs, c) else levels.PAIRS
-                flags |= levels.PAIRS | levels.PAIR_OUT if c < ops.OUTER_WIDE_CHANNELS else levels.NBR
+                flags |= levels.PAIRS | levels.PAIR_OUT
             return flags
 
         self.want = want

@@ -572,9 +572,6 @@ def subm_conv_wgrad(feat, dout, nbr, with_bias=False):
     return (dw, db) if with_bias else dw
 
 
-OUTER_WIDE_CHANNELS = 128   # from here on both sides, the weight-gradient kernels work on 128 x 128 blocks
-
-
 def subm_conv_wgrad_pairs(feat, dout, plan, with_bias=False):
     """The same weight gradient (and bias gradient) from a ConvPlan's pair lists instead of the neighbour map
     (ptv3_subm_conv_wgrad_pairs): half precision, channels in 8s."""

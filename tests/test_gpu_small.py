@@ -30,7 +30,7 @@ def test_long_segments(lengths, c, reduce, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("c,n,extent", [(64, 2000, 14), (64, 9000, 40), (128, 700, 10), (128, 9000, 24)])
+@pytest.mark.parametrize("c,n,extent", [(64, 2000, 14), (64, 6000, 40), (128, 700, 10), (128, 7000, 24)])
 def test_convolution_of_few_pairs(c, n, extent, dtype):
     import numpy as np
 
@@ -44,5 +44,5 @@ def test_convolution_of_few_pairs(c, n, extent, dtype):
     plan = ops.conv_plan_direct(to_dev(idx), 3)
     assert _lib.load().ptv3_conv_form(len(grid), plan.n_pairs, c) == 0
     got = conv(SparseConvTensor(x.to(DEV), to_dev(idx), [extent + 96] * 3, 2)).features
-    want = OF.subm_conv(x.float(), conv.weight.float().cpu(), OI.subm_kmap(idx), conv.bias.float().cpu())
+    want = OF.subm_conv(x.float(), OI.subm_kmap(idx), conv.weight.float().cpu(), conv.bias.float().cpu())
     assert rel_err(got, want) < {torch.float16: 2e-2, torch.bfloat16: 2e-2}[dtype]
