@@ -116,17 +116,40 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(const T* __restrict__ x
 // then read back as MFMA operands.
 constexpr int XCDS = 8;   // work-groups of a launch go to the XCDs round-robin; each XCD has an L2 of its own
 
+// One reduction of a launch: a (rows, m_total), b (rows, k_total) -> d; several without a gather share one (the weight
+// gradients of a block's Linear layers: alone, each fills a part of its rounds and pays its own start and end).
+struct OuterJob {
+    const void *a, *b;
+    int64_t n;
+    int m_total, k_total;
+    const int32_t *nbr, *tap_ptr, *pair_in;
+    int taps, splits;
+    int64_t rows_per_split, slab_stride;
+    float *d, *colsum;
+};
+constexpr int OUTER_BATCH = 8;
+struct OuterBatch {
+    int count;
+    int first[OUTER_BATCH + 1];   // first work-group of every job, multiples of 8
+    OuterJob job[OUTER_BATCH];
+};
+__device__ __forceinline__ int outer_which(const OuterBatch& batch) {
+    int which = 0;
+    while (which + 1 < batch.count && (int)blockIdx.x >= batch.first[which + 1]) ++which;
+    return which;
+}
+
 // Which (tap, range of rows, block of the result) this work-group takes. All blocks of one (tap, range) read the
 // same rows, so they should meet in one L2: they are dealt to the same XCD, next to each other, while the (tap,
 // range) pairs themselves stay interleaved over the XCDs in launch order (with one block per range this is the
 // plain order; handing each XCD a contiguous eighth of the pairs measured 25 % slower on the gathering form).
 // The grid is ceil(taps * splits / 8) * 8 * blocks work-groups; the ones past the last pair leave.
 template <int SIDE>
-__device__ __forceinline__ bool outer_item(int taps, int splits, int m_total, int k_total, int* tap, int* split, int* m0,
+__device__ __forceinline__ bool outer_item(int id, int taps, int splits, int m_total, int k_total, int* tap, int* split, int* m0,
                                            int* k0) {
     const int bm = (m_total + SIDE - 1) / SIDE, bk = (k_total + SIDE - 1) / SIDE;
-    const int slot = blockIdx.x / XCDS;
-    const int64_t x = (int64_t)(slot / (bm * bk)) * XCDS + blockIdx.x % XCDS;
+    const int slot = id / XCDS;
+    const int64_t x = (int64_t)(slot / (bm * bk)) * XCDS + id % XCDS;
     if (x >= (int64_t)taps * splits) return false;
     const int blk = slot % (bm * bk);
     *tap = (int)(x / splits);
@@ -168,20 +191,22 @@ __device__ __forceinline__ void put_transposed4(uint16_t* tile, int g, int q, co
 }
 
 template <typename T, bool GATHER>
-__global__ __launch_bounds__(256) void outer_rows_kernel(const T* __restrict__ a, const T* __restrict__ b, int64_t n,
-                                                         int m_total, int k_total, const int32_t* __restrict__ nbr,
-                                                         const int32_t* __restrict__ tap_ptr,
-                                                         const int32_t* __restrict__ pair_in,
-                                                         int taps, int splits, int64_t rows_per_split,
-                                                         int64_t slab_stride, float* __restrict__ d,
-                                                         float* __restrict__ colsum) {
+__global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
+    const int which = outer_which(batch);
+    const OuterJob& job = batch.job[which];
+    const T* __restrict__ a = (const T*)job.a;
+    const T* __restrict__ b = (const T*)job.b;
+    const int64_t n = job.n, rows_per_split = job.rows_per_split, slab_stride = job.slab_stride;
+    const int m_total = job.m_total, k_total = job.k_total, taps = job.taps, splits = job.splits;
+    const int32_t *__restrict__ nbr = job.nbr, *__restrict__ tap_ptr = job.tap_ptr, *__restrict__ pair_in = job.pair_in;
+    float *__restrict__ d = job.d, *__restrict__ colsum = job.colsum;
     typedef typename Mfma16<T>::v8 v8;
     __shared__ float wave_cols[4][OR_C];
     __shared__ __align__(16) uint16_t tiles[4][2][OR_C * OR_S];
     __shared__ int32_t list_a[GATHER ? OR_LIST : 1], list_b[GATHER ? OR_LIST : 1];
     __shared__ int list_n;
     int tap, split, m0, k0;
-    if (!outer_item<OR_C>(taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
+    if (!outer_item<OR_C>((int)blockIdx.x - batch.first[which], taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
     const int tm = min(2, (m_total - m0 + 31) / 32), tk = min(2, (k_total - k0 + 31) / 32);
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
     int64_t r0 = (int64_t)split * rows_per_split;
@@ -339,20 +364,22 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(const T* __restrict__ a
 constexpr int OW_C = 128;
 
 template <typename T, bool GATHER>
-__global__ __launch_bounds__(256) void outer_rows_wide_kernel(const T* __restrict__ a, const T* __restrict__ b, int64_t n,
-                                                              int m_total, int k_total, const int32_t* __restrict__ nbr,
-                                                              const int32_t* __restrict__ tap_ptr,
-                                                              const int32_t* __restrict__ pair_in,
-                                                              int taps, int splits, int64_t rows_per_split,
-                                                              int64_t slab_stride, float* __restrict__ d,
-                                                              float* __restrict__ colsum) {
+__global__ __launch_bounds__(256) void outer_rows_wide_kernel(OuterBatch batch) {
+    const int which = outer_which(batch);
+    const OuterJob& job = batch.job[which];
+    const T* __restrict__ a = (const T*)job.a;
+    const T* __restrict__ b = (const T*)job.b;
+    const int64_t n = job.n, rows_per_split = job.rows_per_split, slab_stride = job.slab_stride;
+    const int m_total = job.m_total, k_total = job.k_total, taps = job.taps, splits = job.splits;
+    const int32_t *__restrict__ nbr = job.nbr, *__restrict__ tap_ptr = job.tap_ptr, *__restrict__ pair_in = job.pair_in;
+    float *__restrict__ d = job.d, *__restrict__ colsum = job.colsum;
     typedef typename Mfma16<T>::v8 v8;
     __shared__ __align__(16) uint16_t tiles[2][2][OW_C * OR_S];
     __shared__ int32_t list_a[GATHER ? OR_LIST : 1], list_b[GATHER ? OR_LIST : 1];
     __shared__ int list_n;
     __shared__ float wave_cols[2][OW_C];
     int tap, split, m0, k0;
-    if (!outer_item<OW_C>(taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
+    if (!outer_item<OW_C>((int)blockIdx.x - batch.first[which], taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
     int64_t r0 = (int64_t)split * rows_per_split;
     const int64_t r1 = min(n, r0 + rows_per_split);
@@ -1279,36 +1306,62 @@ size_t outer_workspace(int64_t n, int m_total, int k_total, int taps) {
     return splits > 1 ? ptv3_align256((size_t)splits * ((size_t)m_total * taps * k_total + m_total) * sizeof(float)) : 0;
 }
 
-// d (m_total, taps, k_total) fp32 is written in full; so is colsum (m_total,) when given: the column sums of a
-template <typename T, bool GATHER>
-int launch_outer(const void* a, const void* b, int64_t n, int m_total, int k_total, const int32_t* nbr, int taps,
-                 float* d, float* colsum, void* workspace, size_t workspace_bytes, hipStream_t stream,
-                 const int32_t* tap_ptr = nullptr, const int32_t* pair_in = nullptr, SlabJob* defer = nullptr) {
+// One reduction made ready: its job, the sum over its slabs, its work-groups. d (m_total, taps, k_total) fp32 is written in
+// full; so is colsum (m_total,) when given: the column sums of a
+int outer_prepare(const void* a, const void* b, int64_t n, int m_total, int k_total, const int32_t* nbr, int taps, float* d,
+                  float* colsum, void* workspace, size_t workspace_bytes, const int32_t* tap_ptr, const int32_t* pair_in,
+                  int64_t splits, int64_t rows, OuterJob* job, SlabJob* slab, int* groups) {
     const int side = outer_side(m_total, k_total);
-    const int64_t bm = ptv3_ceil_div(m_total, side), bk = ptv3_ceil_div(k_total, side);
-    int64_t splits, rows;
-    outer_ranges<GATHER>(n, m_total, k_total, taps, &splits, &rows);
     if ((int64_t)taps * splits >= (1ll << 31)) return PTV3_EINVAL;
     const int64_t count = (int64_t)m_total * taps * k_total;
     const int64_t stride = count + m_total;
     if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * stride * sizeof(float))) return PTV3_EWORKSPACE;
     float* slabs = splits > 1 ? (float*)workspace : d;
     float* cols = !colsum ? nullptr : (splits > 1 ? slabs + count : colsum);
-    const int64_t items = ptv3_ceil_div((int64_t)taps * splits, XCDS) * XCDS * bm * bk;   // see outer_item
-    if (items >= (1ll << 31)) return PTV3_EINVAL;
-    const dim3 grid((unsigned)items);
-    if (side == OW_C)
-        hipLaunchKernelGGL((outer_rows_wide_kernel<T, GATHER>), grid, dim3(256), 0, stream, (const T*)a, (const T*)b, n,
-                           m_total, k_total, nbr, tap_ptr, pair_in, taps, (int)splits, rows, stride, slabs, cols);
-    else
-        hipLaunchKernelGGL((outer_rows_kernel<T, GATHER>), grid, dim3(256), 0, stream, (const T*)a, (const T*)b, n,
-                           m_total, k_total, nbr, tap_ptr, pair_in, taps, (int)splits, rows, stride, slabs, cols);
-    if (tap_ptr && count >= (1ll << 31)) return PTV3_EINVAL;
-    SlabJob job = {(const float*)slabs, stride, colsum ? stride : count, splits > 1 ? (int)splits : 0, d, count, colsum,
-                   tap_ptr, taps, k_total, rows};
-    if (defer) *defer = job;
-    else if (job.splits) return ptv3_slab_sums(&job, 1, stream);
+    const int64_t items = ptv3_ceil_div((int64_t)taps * splits, XCDS) * XCDS * ptv3_ceil_div(m_total, side) * ptv3_ceil_div(k_total, side);   // see outer_item
+    if (items >= (1ll << 30) || (tap_ptr && count >= (1ll << 31))) return PTV3_EINVAL;
+    *job = OuterJob{a, b, n, m_total, k_total, nbr, tap_ptr, pair_in, taps, (int)splits, rows, stride, slabs, cols};
+    *slab = SlabJob{(const float*)slabs, stride, colsum ? stride : count, splits > 1 ? (int)splits : 0, d, count, colsum,
+                    tap_ptr, taps, k_total, rows};
+    *groups = (int)items;
+    return PTV3_OK;
+}
+
+template <typename T, bool GATHER>
+void outer_launch(const OuterBatch& batch, int side, hipStream_t stream) {
+    const dim3 grid((unsigned)batch.first[batch.count]);
+    if (side == OW_C) hipLaunchKernelGGL((outer_rows_wide_kernel<T, GATHER>), grid, dim3(256), 0, stream, batch);
+    else hipLaunchKernelGGL((outer_rows_kernel<T, GATHER>), grid, dim3(256), 0, stream, batch);
+}
+
+template <typename T, bool GATHER>
+int launch_outer(const void* a, const void* b, int64_t n, int m_total, int k_total, const int32_t* nbr, int taps,
+                 float* d, float* colsum, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                 const int32_t* tap_ptr = nullptr, const int32_t* pair_in = nullptr, SlabJob* defer = nullptr) {
+    int64_t splits, rows;
+    outer_ranges<GATHER>(n, m_total, k_total, taps, &splits, &rows);
+    OuterBatch batch = {};
+    SlabJob slab;
+    batch.count = 1;
+    const int rc = outer_prepare(a, b, n, m_total, k_total, nbr, taps, d, colsum, workspace, workspace_bytes, tap_ptr, pair_in, splits,
+                                 rows, &batch.job[0], &slab, &batch.first[1]);
+    if (rc != PTV3_OK) return rc;
+    outer_launch<T, GATHER>(batch, outer_side(m_total, k_total), stream);
+    if (defer) *defer = slab;
+    else if (slab.splits) return ptv3_slab_sums(&slab, 1, stream);
     PTV3_RETURN_LAUNCH();
+}
+
+// Ranges of rows for the Linear layers `jobs` that share a launch: as outer_split for all their blocks together
+void outer_batch_ranges(const LinearGrad* jobs, int count, int side, int64_t* splits, int64_t* rows) {
+    int64_t blocks = 0, n = 0;
+    for (int i = 0; i < count; ++i) {
+        if (outer_side(jobs[i].nout, jobs[i].k) != side) continue;
+        blocks += ptv3_ceil_div(jobs[i].nout, side) * ptv3_ceil_div(jobs[i].k, side);
+        n = jobs[i].n;
+    }
+    *splits = *rows = 0;
+    if (blocks) outer_split(n, blocks, 1, 0, splits, rows);
 }
 
 template <typename T>
@@ -1358,13 +1411,44 @@ int ptv3_slab_sums(const SlabJob* jobs, int count, hipStream_t stream) {
     PTV3_RETURN_LAUNCH();
 }
 
-int ptv3_linear_wgrad_slabs(const void* x, const void* dout, int dtype, int64_t n, int k, int nout, float* dweight, float* dbias,
-                            void* workspace, size_t workspace_bytes, SlabJob* job, hipStream_t stream) {
-    if (dtype == PTV3_F16)
-        return launch_outer<_Float16, false>(dout, x, n, nout, k, nullptr, 1, dweight, dbias, workspace, workspace_bytes, stream,
-                                             nullptr, nullptr, job);
-    return launch_outer<__bf16, false>(dout, x, n, nout, k, nullptr, 1, dweight, dbias, workspace, workspace_bytes, stream,
-                                       nullptr, nullptr, job);
+size_t ptv3_linear_wgrads_bytes(const LinearGrad* jobs, int count) {
+    size_t bytes = 0;
+    for (int side : {OR_C, OW_C}) {
+        int64_t splits, rows;
+        outer_batch_ranges(jobs, count, side, &splits, &rows);
+        for (int i = 0; i < count; ++i)
+            if (splits > 1 && outer_side(jobs[i].nout, jobs[i].k) == side)
+                bytes += ptv3_align256((size_t)splits * ((size_t)jobs[i].nout * jobs[i].k + jobs[i].nout) * sizeof(float));
+    }
+    return bytes;
+}
+
+int ptv3_linear_wgrads_slabs(const LinearGrad* jobs, int count, int dtype, void* workspace, size_t workspace_bytes, SlabJob* slabs,
+                             hipStream_t stream) {
+    if (count > OUTER_BATCH) return PTV3_EINVAL;
+    char* at = (char*)workspace;
+    for (int side : {OR_C, OW_C}) {
+        int64_t splits, rows;
+        outer_batch_ranges(jobs, count, side, &splits, &rows);
+        if (!splits) continue;
+        OuterBatch batch = {};
+        for (int i = 0; i < count; ++i) {
+            const LinearGrad& g = jobs[i];
+            if (outer_side(g.nout, g.k) != side) continue;
+            const size_t bytes = splits > 1 ? ptv3_align256((size_t)splits * ((size_t)g.nout * g.k + g.nout) * sizeof(float)) : 0;
+            int groups;
+            const int rc = outer_prepare(g.dy, g.x, g.n, g.nout, g.k, nullptr, 1, g.dweight, g.dbias, at,
+                                         workspace_bytes - (size_t)(at - (char*)workspace), nullptr, nullptr, splits, rows,
+                                         &batch.job[batch.count], &slabs[i], &groups);
+            if (rc != PTV3_OK) return rc;
+            batch.first[batch.count + 1] = batch.first[batch.count] + groups;
+            ++batch.count;
+            at += bytes;
+        }
+        if (dtype == PTV3_F16) outer_launch<_Float16, false>(batch, side, stream);
+        else outer_launch<__bf16, false>(batch, side, stream);
+    }
+    PTV3_RETURN_LAUNCH();
 }
 
 int ptv3_subm_conv_wgrad_slabs(const void* feat, const void* dout, int dtype, int64_t n, int cin, int cout, const int32_t* nbr,

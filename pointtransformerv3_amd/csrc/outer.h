@@ -17,9 +17,17 @@ struct SlabJob {
 constexpr int SLAB_JOBS = 16;
 
 // as ptv3_linear_wgrad / ptv3_subm_conv_wgrad / ptv3_subm_conv_wgrad_pairs (half precision, channels in 8s), the sum over
-// the slabs left to ptv3_slab_sums; `workspace` must stay until then
-int ptv3_linear_wgrad_slabs(const void* x, const void* dout, int dtype, int64_t n, int k, int nout, float* dweight, float* dbias,
-                            void* workspace, size_t workspace_bytes, SlabJob* job, hipStream_t stream);
+// the slabs left to ptv3_slab_sums; `workspace` must stay until then. The Linear layers of up to 8 jobs, all of as many
+// rows, share a launch (two where some have a side below 128 channels); slabs[i] is job i's sum.
+struct LinearGrad {
+    const void *x, *dy;         // (n, k), (n, nout)
+    int64_t n;
+    int k, nout;
+    float *dweight, *dbias;
+};
+size_t ptv3_linear_wgrads_bytes(const LinearGrad* jobs, int count);
+int ptv3_linear_wgrads_slabs(const LinearGrad* jobs, int count, int dtype, void* workspace, size_t workspace_bytes, SlabJob* slabs,
+                             hipStream_t stream);
 int ptv3_subm_conv_wgrad_slabs(const void* feat, const void* dout, int dtype, int64_t n, int cin, int cout, const int32_t* nbr,
                                const int32_t* tap_ptr, const int32_t* pair_in, int taps, float* dweight, float* dbias,
                                void* workspace, size_t workspace_bytes, SlabJob* job, hipStream_t stream);

@@ -254,18 +254,32 @@ struct Run {
     float* grads = nullptr;
     SlabJob jobs[SLAB_JOBS];
     int n_jobs = 0;
+    LinearGrad linears[8];
+    int n_linears = 0;
 
-    int flush() {
+    // the weight gradients of the Linear layers put off so far (of one number of rows), then all slab sums
+    int flush(Space& scratch) {
+        TRY(linear_wgrads(scratch));
         const int n = n_jobs;
         n_jobs = 0;
         return n && !dry ? ptv3_slab_sums(jobs, n, hs) : PTV3_OK;
     }
-    // a job's slabs stay in `scratch` until flush
-    int wgrad(const ptv3_train_linear& l, int in, int out, const void* x, const void* dy, int64_t n, Space& scratch) {
-        const size_t bytes = ptv3_linear_wgrad_workspace_bytes(n, in, out);
+    int linear_wgrads(Space& scratch) {
+        const int n = n_linears;
+        n_linears = 0;
+        if (!n) return PTV3_OK;
+        const size_t bytes = ptv3_linear_wgrads_bytes(linears, n);
         void* ws = bytes ? scratch.take(bytes) : nullptr;
-        DO(ptv3_linear_wgrad_slabs(x, dy, dt, n, in, out, grads + l.gw, grads + l.gb, ws, bytes, &jobs[n_jobs], hs));
-        return ++n_jobs == SLAB_JOBS ? flush() : PTV3_OK;
+        DO(ptv3_linear_wgrads_slabs(linears, n, dt, ws, bytes, jobs + n_jobs, hs));
+        n_jobs += n;
+        return PTV3_OK;
+    }
+    // x and dy stay until flush, and so do a job's slabs in `scratch`
+    int wgrad(const ptv3_train_linear& l, int in, int out, const void* x, const void* dy, int64_t n, Space& scratch) {
+        if (n_linears && (n_linears == 8 || linears[0].n != n)) TRY(linear_wgrads(scratch));
+        if (n_jobs + n_linears >= SLAB_JOBS) TRY(flush(scratch));
+        linears[n_linears++] = LinearGrad{x, dy, n, in, out, grads + l.gw, grads + l.gb};
+        return PTV3_OK;
     }
     int conv_wgrad(const ptv3_train_block& b, const ptv3_level& v, const void* x, const void* dy, Space& scratch) {
         const int c = b.channels;
@@ -273,7 +287,7 @@ struct Run {
         void* ws = bytes ? scratch.take(bytes) : nullptr;
         DO(ptv3_subm_conv_wgrad_slabs(x, dy, dt, v.n, c, c, v.pair_out, v.tap_ptr, v.pair_in, 27, grads + b.g_conv_w,
                                        grads + b.g_conv_b, ws, bytes, &jobs[n_jobs], hs));
-        return ++n_jobs == SLAB_JOBS ? flush() : PTV3_OK;
+        return ++n_jobs + n_linears >= SLAB_JOBS ? flush(scratch) : PTV3_OK;
     }
     int bn_bwd(const ptv3_train_bn& b, const BnActs& a, int64_t n, int c, const void* dy, void* dx) {
         if (dry) return PTV3_OK;
@@ -319,7 +333,7 @@ struct Run {
         TRY(linear(dcpe, b.cpe.wt, nullptr, c, c, n, h1));
         TRY(conv_wgrad(b, v, a.xs, h1, scratch));
         TRY(conv(b, v, true, h1, scratch, dxs));
-        TRY(flush());
+        TRY(flush(scratch));
         scratch.at = mark;
         return PTV3_OK;
     }
@@ -384,7 +398,7 @@ struct Run {
             TRY(wgrad(g.up, g.up.in, c, child_rows, dlin2, below.n, scratch));
             void* dnext = s + 1 < S - 1 ? from_up[s + 1] : from_skip[S - 1];
             TRY(linear(dlin2, g.up.wt, nullptr, c, g.up.in, below.n, dnext));
-            TRY(flush());
+            TRY(flush(scratch));
             scratch.at = mark;
             d = dnext;
             d_dt = dt;
@@ -407,7 +421,7 @@ struct Run {
                                             dproj, stream));
                 TRY(wgrad(g.pool, g.pool.in, c, st[s - 1].enc[net.stage[s - 1].n_enc - 1].out16, dproj, up.n, scratch));
                 TRY(linear(dproj, g.pool.wt, nullptr, c, g.pool.in, up.n, from_pool[s - 1]));
-                TRY(flush());
+                TRY(flush(scratch));
             } else {
                 TRY(bn_bwd(net.stem.bn, stem_bn, v.n, c, dx, dseg));
                 const int cp = net.stem.cin_padded;
@@ -416,7 +430,7 @@ struct Run {
                 float* dw = (float*)scratch.take((size_t)c * 125 * cp * 4);
                 DO(ptv3_subm_conv_wgrad_slabs(stem_in, dseg, dt, v.n, cp, c, v.pair_out5, v.tap_ptr5, v.pair_in5, 125, dw, nullptr,
                                                ws, bytes, &jobs[n_jobs++], hs));
-                TRY(flush());
+                TRY(flush(scratch));
                 DO(ptv3_cut_rows(dw, (int64_t)c * 125, cp, net.stem.cin, grads + net.stem.gw, stream));
             }
             scratch.at = mark;
