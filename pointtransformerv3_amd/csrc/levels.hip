@@ -476,19 +476,14 @@ __global__ __launch_bounds__(GT) void list_count_kernel(ListArgs a) {
     uint64_t lo = 0, hi = 0;
     if (tid < v.group && i < v.n) {
         const int4 c = v.idx[i];
-        const VoxelWindow w = vh_window<R>(v.h, c.x, c.y, c.z, c.w);
+        uint32_t slot[8];
+        vh_taps<R>(v.h, c.x, c.y, c.z, c.w, slot, lo, hi);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            uint64_t m = w.hits[k];
-            while (m) {
-                const int bit = __builtin_ctzll(m);
-                m &= m - 1;
-                const int t = vh_tap_of<R>(w, k, bit, c.y, c.z, c.w);
-                if (t < 64) lo |= 1ull << t; else hi |= 1ull << (t - 64);
-                atomicOr(&mask[wave][t], 1ull << lane);
-            }
-            v.slot[(int64_t)k * v.n + i] = w.slot[k];
-        }
+        for (int k = 0; k < 8; ++k) v.slot[(int64_t)k * v.n + i] = slot[k];
+        uint64_t f = lo;
+        while (f) { const int t = __builtin_ctzll(f); f &= f - 1; atomicOr(&mask[wave][t], 1ull << lane); }
+        f = hi;
+        while (f) { const int t = 64 + __builtin_ctzll(f); f &= f - 1; atomicOr(&mask[wave][t], 1ull << lane); }
         v.found[i] = lo;
         if (KS == 5) v.found[v.n + i] = hi;
     }
@@ -578,9 +573,10 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
     __shared__ unsigned long long mask[2][128];
     __shared__ uint32_t tap_base[128], tap_start[128], wrows[2];
     __shared__ uint32_t hslot[8][GT];
+    __shared__ uint8_t first_cell[GT];   // 2 bits per axis: where a voxel's window starts in its first block
     __shared__ uint32_t stage_q[STAGE];
-    __shared__ int32_t stage_in[STAGE], stage_slot[STAGE];
-    __shared__ uint8_t stage_vox[STAGE];
+    __shared__ int32_t stage_slot[STAGE];
+    __shared__ uint16_t stage_vt[STAGE];   // voxel << 7 | tap
     const int l = list_level(a);
     const ListLevel& v = a.lv[l];
     const int g = (int)blockIdx.x - a.first_block[l], tid = threadIdx.x, lane = tid % PTV3_WAVE, wave = tid / PTV3_WAVE;
@@ -596,15 +592,14 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) hslot[k][tid] = v.slot[(int64_t)k * v.n + i];
     }
-    const int xs = c.y + VH_SHIFT, ys = c.z + VH_SHIFT, zs = c.w + VH_SHIFT;
-    const int bx0 = (xs - R) >> 2, by0 = (ys - R) >> 2, bz0 = (zs - R) >> 2;
-    // row of the voxel at (dx, dy, dz) from mine
-    auto source = [&](int dx, int dy, int dz) -> int32_t {
-        if ((dx | dy | dz) == 0) return (int32_t)i;
-        const int cx = xs + dx, cy = ys + dy, cz = zs + dz;
-        const int k = ((cx >> 2) - bx0) << 2 | ((cy >> 2) - by0) << 1 | ((cz >> 2) - bz0);
-        const int bit = (cx & 3) << 4 | (cy & 3) << 2 | (cz & 3);
-        return v.h.rows[(int64_t)hslot[k][tid] * 64 + bit];
+    first_cell[tid] = (uint8_t)(((c.y + VH_SHIFT - R) & 3) << 4 | ((c.z + VH_SHIFT - R) & 3) << 2 | ((c.w + VH_SHIFT - R) & 3));
+    // row of the voxel at tap t (of edge^3) of the tile's voxel `vox`
+    auto source = [&](int vox, int t, int edge) -> int32_t {
+        if (t == edge * edge * edge / 2) return (int32_t)((int64_t)g * v.group + vox);
+        const int at = first_cell[vox], in = R - edge / 2;
+        const int cx = (at >> 4) + t / (edge * edge) + in, cy = (at >> 2 & 3) + t / edge % edge + in, cz = (at & 3) + t % edge + in;
+        const int k = cx >> 2 << 2 | cy >> 2 << 1 | cz >> 2, bit = (cx & 3) << 4 | (cy & 3) << 2 | (cz & 3);
+        return v.h.rows[(int64_t)hslot[k][vox] * 64 + bit];
     };
 
     auto make = [&](uint64_t flo, uint64_t fhi, int taps, int edge, const int32_t* tap_ptr, const uint32_t* tap_off,
@@ -658,15 +653,14 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
             int t;
             if (f0) { t = __builtin_ctzll(f0); f0 &= f0 - 1; }
             else { t = 64 + __builtin_ctzll(f1); f1 &= f1 - 1; }
-            const int32_t src = source(t / (edge * edge) - edge / 2, (t / edge) % edge - edge / 2, t % edge - edge / 2);
             const uint32_t rank = (uint32_t)__popcll(mask[wave][t] & below) + (wave ? (uint32_t)__popcll(mask[0][t]) : 0u);
             const uint32_t q = tap_base[t] + rank, e = tap_start[t] + rank;
             if (staged) {
                 stage_q[e] = q;
-                stage_in[e] = src;
                 stage_slot[e] = (int32_t)slot;
-                stage_vox[e] = (uint8_t)tid;
+                stage_vt[e] = (uint16_t)(tid << 7 | t);
             } else {
+                const int32_t src = source(tid, t, edge);
                 if (pairs) {
                     pair_in[q] = src;
                     pair_slot[q] = (int32_t)slot;
@@ -678,16 +672,28 @@ __global__ __launch_bounds__(GT) void list_fill_kernel(ListArgs a) {
         }
         if (staged) {
             __syncthreads();
-            for (uint32_t e = tid; e < total; e += GT) {
-                const int32_t src = stage_in[e];
-                const uint32_t vox = stage_vox[e];
-                if (pairs) {
-                    const uint32_t q = stage_q[e];
-                    pair_in[q] = src;
-                    pair_slot[q] = stage_slot[e];
-                    if (pair_out) pair_out[q] = (int32_t)((int64_t)g * v.group + vox);
+            // the rows are looked up here, four pairs of a thread at a time, not in the loop above, where every lane
+            // waited for the fullest one's lookups one after the other
+            for (uint32_t e0 = tid; e0 < total; e0 += 4 * GT) {
+                int32_t src[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint32_t e = min(e0 + u * GT, total - 1), vt = stage_vt[e];
+                    src[u] = source((int)(vt >> 7), (int)(vt & 127), edge);
                 }
-                if (tiles) v.tile_pair[base + e] = vox << 24 | (uint32_t)src;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint32_t e = e0 + u * GT;
+                    if (e >= total) break;
+                    const uint32_t vox = (uint32_t)stage_vt[e] >> 7;
+                    if (pairs) {
+                        const uint32_t q = stage_q[e];
+                        pair_in[q] = src[u];
+                        pair_slot[q] = stage_slot[e];
+                        if (pair_out) pair_out[q] = (int32_t)((int64_t)g * v.group + vox);
+                    }
+                    if (tiles) v.tile_pair[base + e] = vox << 24 | (uint32_t)src[u];
+                }
             }
         }
         __syncthreads();

@@ -111,6 +111,74 @@ __device__ __forceinline__ VoxelWindow vh_window(const VoxelHash& h, int b, int 
     return w;
 }
 
+// four nibbles of the low half -> the low nibbles of four bytes
+__device__ __forceinline__ uint32_t vh_spread4(uint32_t v) {
+    v = (v | v << 8) & 0x00ff00ffu;
+    return (v | v << 4) & 0x0f0f0f0fu;
+}
+
+// The taps that exist around the voxel at (x, y, z) of scene b, bit t = (kx * KS + ky) * KS + kz of hi:lo, and the header
+// slots of the up-to-8 blocks around it. The window is cut out of the 8 x 8 x 8 cells of those blocks by shifts, the same
+// 160 (KS 5) or 70 instructions for every lane: a loop over the occupied cells of each block ran as long as the fullest
+// lane's, block by block, some 20 us of one wave's dependent instructions.
+template <int R>
+__device__ __forceinline__ void vh_taps(const VoxelHash& h, int b, int x, int y, int z, uint32_t (&slot)[8], uint64_t& lo, uint64_t& hi) {
+    constexpr int KS = 2 * R + 1;
+    const int x0 = x + VH_SHIFT - R, y0 = y + VH_SHIFT - R, z0 = z + VH_SHIFT - R;   // first cell of the window
+    const int nx = ((x0 & 3) + KS - 1) >> 2, ny = ((y0 & 3) + KS - 1) >> 2, nz = ((z0 & 3) + KS - 1) >> 2;   // 0 or 1
+    uint64_t key[8], m[8];
+    VoxelBlock cur[8];
+    bool live[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int bx = k >> 2, by = (k >> 1) & 1, bz = k & 1;
+        live[k] = bx <= nx && by <= ny && bz <= nz;
+        key[k] = vh_block_key(b, (x0 >> 2) + bx, (y0 >> 2) + by, (z0 >> 2) + bz);
+        slot[k] = (uint32_t)vh_mix(key[k]) & h.mask;
+        cur[k].key = VH_EMPTY;
+        cur[k].mask = 0;
+        if (live[k]) cur[k] = vh_load(h, slot[k]);   // all first probes in flight together
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (live[k])
+            for (uint32_t probe = 0; probe < h.mask && cur[k].key != key[k] && cur[k].key != VH_EMPTY; ++probe) {
+                slot[k] = (slot[k] + 1) & h.mask;
+                cur[k] = vh_load(h, slot[k]);
+            }
+        m[k] = cur[k].key == key[k] ? cur[k].mask : 0;
+    }
+    // along x: slices 0 .. 3 of the window as the 16-bit quarters of `a`, slice 4 in `e`, for each (by, bz)
+    const int sx = 16 * (x0 & 3), sy = 4 * (y0 & 3), sz = z0 & 3;
+    uint64_t a[4];
+    uint32_t e[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        a[q] = m[q] >> sx | m[q + 4] << 1 << (63 - sx);
+        e[q] = (uint32_t)(m[q + 4] >> sx) & 0xffffu;
+    }
+    lo = hi = 0;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        // along y: KS nibbles of each bz; along z: a nibble of either, side by side in a byte, shifted
+        uint32_t s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = i == 4 ? e[q] : (uint32_t)(a[q] >> (16 * i)) & 0xffffu;
+        const uint32_t r0 = (s[0] | s[2] << 16) >> sy, r1 = (s[1] | s[3] << 16) >> sy;
+        constexpr uint32_t RUN = (1u << KS) - 1u;
+        const uint32_t four = (vh_spread4(r0 & 0xffffu) | vh_spread4(r1 & 0xffffu) << 4) >> sz;
+        // (a byte's shifted-in upper bits lie above its run: sz + KS <= 8)
+        uint64_t w = four & RUN;
+#pragma unroll
+        for (int j = 1; j < (KS < 4 ? KS : 4); ++j) w |= (uint64_t)(four >> (8 * j) & RUN) << (KS * j);
+        if (KS == 5) w |= (uint64_t)(((r0 >> 16 & 15u) | (r1 >> 16 & 15u) << 4) >> sz & RUN) << 20;
+        const int at = KS * KS * i;
+        if (at < 64) lo |= w << at;
+        if (at < 64 && at + KS * KS > 64) hi |= w >> (64 - at);
+        if (at >= 64) hi |= w << (at - 64);
+    }
+}
+
 // tap index (kx * ks + ky) * ks + kz of cell `bit` of block k of the window of a voxel at (x, y, z)
 template <int R>
 __device__ __forceinline__ int vh_tap_of(const VoxelWindow& w, int k, int bit, int x, int y, int z) {

@@ -91,12 +91,13 @@ class Index:
         return buf[at:at + size].view(dtype).view(shape)
 
 
-def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None):
+def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None, sized=None):
     """Queues the whole index on the current stream and waits for what the host has to know. grid_coord (n, 3) int32 and
     offset (scenes,) int64 contiguous, batch (n,) int64 or None; orders: names of the curves, shuffled with torch's CPU
     generator when `shuffle` (and per pooling module as layout.shuffles says, in the order the modules would draw);
     want(level number, Level) -> PTV3_LISTS_* flags of the level once its pair count is known;
-    between() is called behind the first stage's launches, while the host would wait for them."""
+    between() is called behind the first stage's launches, while the host would wait for them, sized(levels) behind the
+    third's, when every level's number of points is known."""
     lib = _lib.load()
     stream = ops._stream()
     dev = grid_coord.device
@@ -142,9 +143,11 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     tables, scratch = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
     check(lib.ptv3_index_pool(state, perms, tables.data_ptr(), sizes[0], scratch.data_ptr(), sizes[1], stream),
           "ptv3_index_pool")
+    out.levels = levels = (Level * cfg.n_levels).from_address(lib.ptv3_index_levels(state))
+    if sized is not None:
+        sized(levels)
     check(lib.ptv3_index_wait(slot.ptr, 2, seq, stream), "ptv3_index_wait")
     out.level_offsets = [words[_SLOT_ENDS + level * nb:_SLOT_ENDS + (level + 1) * nb] for level in range(cfg.n_levels)]
-    out.levels = levels = (Level * cfg.n_levels).from_address(lib.ptv3_index_levels(state))
     wanted = (ctypes.c_int32 * cfg.n_levels)()
     # the pair counts enter `levels` with the size query; the flags decide what is sized, so the query runs twice
     check(lib.ptv3_index_lists_bytes(state, wanted, sizes), "ptv3_index_lists_bytes")

@@ -187,7 +187,7 @@ class TrainEngine:
         self._keep.append(t)
         return t.data_ptr() if t is not None else None
 
-    def masks(self, index):
+    def masks(self, sizes):
         """The stochastic-depth row factors in the order the blocks would draw them (DropPath.mask; model.py:602-604)."""
         out, keeps, drawn = [], [], []
         for s, drop in self.drops:
@@ -196,7 +196,7 @@ class TrainEngine:
                 if rate == 0.0:
                     out.append(None)
                     continue
-                m = torch.empty((index.levels[s].n, 1), dtype=self.dtype, device=self.device).bernoulli_(1.0 - rate)
+                m = torch.empty((sizes[s].n, 1), dtype=self.dtype, device=self.device).bernoulli_(1.0 - rate)
                 if drop.scale_by_keep and rate < 1.0:
                     drawn.append(m)
                     keeps.append(1.0 - rate)
@@ -214,13 +214,20 @@ class TrainEngine:
         def refresh():   # float masters are cast, transposed and packed once per step
             _lib.check(_lib.load().ptv3_net_refresh(ctypes.byref(self._refresh), ops._stream()), "ptv3_net_refresh")
 
+        masks = []
+
+        def sized(sizes):   # some 45 small launches while the host would wait for the pair counts
+            if any(v.n < 2 for v in sizes):
+                return
+            if self.batches:
+                torch._foreach_add_(self.batches, 1)
+            masks.extend(self.masks(sizes))
+
         model._prologue_state = None
-        index = levels.build(self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want, between=refresh)
+        index = levels.build(self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want, between=refresh, sized=sized)
         if any(v.n < 2 for v in index.levels):
             raise ValueError("Expected more than 1 value per channel when training")   # as BatchNorm1d does
-        if self.batches:
-            torch._foreach_add_(self.batches, 1)
-        out = _Step.apply(self, feat, index, self.masks(index), *self.params)
+        out = _Step.apply(self, feat, index, masks, *self.params)
         point["batch"] = index.batch
         native.fill_point(point, index, 0, out, self.net.patch[0])
         return point
