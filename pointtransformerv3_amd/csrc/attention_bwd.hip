@@ -15,6 +15,7 @@
 //      enter through the MFMAs' C operands), dS and dQ^T += K^T dS^T. lse and D go to a workspace.
 //   2. keys: Q, dO (rows), Q^T, dO^T (transposed), -lse and -D in LDS; per 32-key tile
 //      dV^T += dO^T P and dK^T += Q^T dS over all queries.
+// Where the forward kept the log-sum-exps and the sequences are long, one kernel does both (attn_bwd_both_kernel).
 // fp32: one thread per query / per key, operands staged through LDS in chunks.
 #include "attn_half.h"
 
@@ -24,6 +25,8 @@ constexpr int BWD_THREADS = 512;    // keys kernel: 8 waves, two key tiles each 
 constexpr int BWD_WAVES = BWD_THREADS / PTV3_WAVE;
 constexpr int BWQ_THREADS = 1024;   // queries kernel: 16 waves, four per SIMD
 constexpr int BWQ_WAVES = BWQ_THREADS / PTV3_WAVE;
+constexpr int BOTH_KEYS = 1024;     // both-sides kernel: the keys that its waves hold in registers
+constexpr int BOTH_WAVES = 8;
 constexpr float LN2 = 0.6931471805599453f;
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -87,13 +90,15 @@ __device__ __forceinline__ f32x16 splat16(float x) {
 // Work-group id -> (item, part of parts): the first full_items work-groups take one (sequence, head) item each;
 // the items of the last, partly filled round of resident work-groups are cut into `split` ranges of tiles, one
 // work-group each, so that the round is short (every range stages the sequence again).
-__device__ __forceinline__ void item_of_block(int full_items, int split, int* item, int* part, int* parts) {
-    if ((int)blockIdx.x < full_items) {
-        *item = xcd_chunked_id(blockIdx.x, full_items);   // heads that share cache lines meet in one L2
+// The first `first` work-groups are not in the grid: the both-sides kernel below took their items.
+__device__ __forceinline__ void item_of_block(int first, int full_items, int split, int* item, int* part, int* parts) {
+    const int block = first + blockIdx.x;
+    if (block < full_items) {
+        *item = xcd_chunked_id(block, full_items);   // heads that share cache lines meet in one L2
         *part = 0;
         *parts = 1;
     } else {
-        const int r = blockIdx.x - full_items;
+        const int r = block - full_items;
         *item = full_items + r / split;
         *part = r % split;
         *parts = split;
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(BWQ_THREADS) void attn_bwd_q_kernel(
     const T* __restrict__ qkv, const T* __restrict__ out, const T* __restrict__ dout, int channels, int heads,
     const int32_t* __restrict__ slot_src, const int32_t* __restrict__ slot_dst,
     const int32_t* __restrict__ cu_seqlens, int lds_keys, float scale, int64_t n_pad, T* __restrict__ dqkv,
-    float* lse_ws, float* __restrict__ d_ws, int full_items, int split, Dropout drop) {
+    float* lse_ws, float* __restrict__ d_ws, int first, int full_items, int split, Dropout drop) {
     typedef typename Half<T>::v8 v8;
     extern __shared__ __align__(16) unsigned char smem[];
     // K rows, V rows, K^T, 96 B of zeros
@@ -117,7 +122,7 @@ __global__ __launch_bounds__(BWQ_THREADS) void attn_bwd_q_kernel(
     unsigned char* zero_lds = kt_lds + (size_t)HD * kt_stride;
 
     int item, part, parts;
-    item_of_block(full_items, split, &item, &part, &parts);
+    item_of_block(first, full_items, split, &item, &part, &parts);
     const int seq = item / heads, head = item % heads;
     const int s0 = cu_seqlens[seq];
     const int len = cu_seqlens[seq + 1] - s0;
@@ -272,9 +277,8 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
     const int32_t* __restrict__ slot_src, const int32_t* __restrict__ slot_dst,
     const int32_t* __restrict__ cu_seqlens, int lds_keys, float scale, int64_t n_pad,
     const float* __restrict__ lse_ws, const float* __restrict__ d_ws, T* __restrict__ dqkv, T* __restrict__ fill,
-    int full_items, int split, Dropout drop) {
+    int first, int full_items, int split, Dropout drop) {
     typedef typename Half<T>::v8 v8;
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
     extern __shared__ __align__(16) unsigned char smem[];
     const int t_stride = lds_keys * 2 + VT_PAD_BYTES;
     unsigned char* q_lds = smem;                                      // Q * scale * log2(e), rows
@@ -286,7 +290,7 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
     unsigned char* zero_lds = (unsigned char*)(nd_lds + lds_keys);
 
     int item, part, parts;
-    item_of_block(full_items, split, &item, &part, &parts);
+    item_of_block(first, full_items, split, &item, &part, &parts);
     const int seq = item / heads, head = item % heads;
     const int s0 = cu_seqlens[seq];
     const int len = cu_seqlens[seq + 1] - s0;
@@ -451,6 +455,257 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
             *(u32x2*)(base + channels) = lo;
             *(u32x2*)(base + channels + 8) = hi;
         }
+    }
+}
+
+// ---- both sides in one kernel: one work-group per (sequence, head), scores computed once
+//
+// A wave owns KG groups of 16 keys; their K and V, and the sums of their dK and dV, stay in its registers while the
+// work-group walks over the queries in LDS. In a step a wave takes one block of 32 queries:
+//   S and dP as 16 x 16 tiles with a lane per key (registers: queries), P = 2^(S - lse), dS = P (dP - D);
+//   dV^T += dO^T P and dK^T += Q^T dS straight from those registers (the transposed Q and dO lie in LDS with the queries
+//   in the order in which the tiles hold them);
+//   dS^T, which dQ^T += K^T dS^T needs with a lane per query, by a product with the identity: exact, and it costs the
+//   matrix pipe 16 cycles a tile where the vector pipe would repeat the exponentials.
+// dQ sums over the keys of all waves: in step s wave w takes block (w + s) mod WAVES, so a block's fp32 sums in LDS
+// belong to one wave at a time, in a fixed order, and a barrier a step is all that this needs.
+//
+// Bound by the two pipes of a SIMD together: for 32 x 32 scores 56 vector instructions (16 of them exponentials, which take
+// two issue slots), 18 matrix instructions and 288 cycles of the matrix pipe, about 400 cycles if all overlapped, 585
+// measured with two waves a SIMD; the two kernels above take 890 together, the exponentials twice. Eight waves of 128 keys
+// and not 16 of 64: the query side of a step and the dQ sums pass LDS half as often, and the registers for a group ahead
+// are there (16 waves spill). bf16, 1024 slots: 1400 items 630 -> 489 us, 788 items 374 -> 298 us, 384 items 188 -> 154 us.
+template <typename T, int WAVES, bool DROP>
+__global__ __launch_bounds__(WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
+    const T* __restrict__ qkv, const T* __restrict__ out, const T* __restrict__ dout, int channels, int heads,
+    const int32_t* __restrict__ slot_src, const int32_t* __restrict__ slot_dst, const int32_t* __restrict__ cu_seqlens,
+    float scale, int64_t n_pad, const float* __restrict__ lse, T* __restrict__ dqkv, T* __restrict__ fill, Dropout drop) {
+    constexpr int KG = BOTH_KEYS / 16 / WAVES;     // 16-key groups per wave
+    constexpr int T_STRIDE = BOTH_KEYS * 2 + VT_PAD_BYTES;
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char* q_lds = smem;                                  // Q * scale * log2(e), rows
+    unsigned char* do_lds = q_lds + BOTH_KEYS * 32;               // dO rows
+    unsigned char* qt_lds = do_lds + BOTH_KEYS * 32;              // the same two, transposed
+    unsigned char* dot_lds = qt_lds + HD * T_STRIDE;
+    float* nlse_lds = (float*)(dot_lds + HD * T_STRIDE);          // -lse (log2 units), -D per query slot
+    float* nd_lds = nlse_lds + BOTH_KEYS;
+    int32_t* dst_lds = (int32_t*)(nd_lds + BOTH_KEYS);            // the row that a query slot writes
+    float* dq_lds = (float*)(dst_lds + BOTH_KEYS);                // WAVES blocks of two 16-query tiles in lane order
+
+    const int item = xcd_chunked_id(blockIdx.x, gridDim.x);
+    const int seq = item / heads, head = item % heads;
+    const int s0 = cu_seqlens[seq];
+    const int len = min(cu_seqlens[seq + 1] - s0, BOTH_KEYS);
+    if (len <= 0) return;
+    const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
+    const int col = lane & 15, grp = lane >> 4;
+    const int64_t row_stride = 3 * (int64_t)channels;
+    const float scale_log2e = scale * LOG2E;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+    // identity operand: row (or column) col of the 16 x 16 unit matrix, entries 4 grp .. 4 grp + 3
+    u32x2 unit;
+    {
+        const float one = (col >> 2) == grp ? 1.f : 0.f;
+        unit[0] = Half<T>::pack2((col & 3) == 0 ? one : 0.f, (col & 3) == 1 ? one : 0.f);
+        unit[1] = Half<T>::pack2((col & 3) == 2 ? one : 0.f, (col & 3) == 3 ? one : 0.f);
+    }
+
+    // Everything that the work-group reads, in two rounds of loads. A thread stages eight channels of four queries; a
+    // query that does not exist, or a filler slot, gets lse = +inf: its probabilities come out as zero. A wave's keys:
+    // lane = key, four channels; a key that does not exist repeats the last one, so that its scores stay in range.
+    constexpr int THREADS = WAVES * PTV3_WAVE, QP = BOTH_KEYS * 2 / THREADS;
+    const int half8 = tid & 1;
+    const int key0 = wave * KG * 16;
+    const bool mine = key0 < len;                        // the same for the whole wave
+    u32x2 kf[KG], vf[KG];
+    u32x4 kt[KG / 2];
+    f32x4 acc_k[KG], acc_v[KG];
+    {
+        int dst[QP], src[KG];
+        u32x4 q[QP], g[QP], o[QP];
+        float l[QP];
+#pragma unroll
+        for (int j = 0; j < QP; ++j) {
+            const int slot = (tid + j * THREADS) >> 1;
+            dst[j] = slot < len ? slot_dst[s0 + slot] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < KG; ++k) src[k] = slot_src[s0 + min(key0 + k * 16 + col, len - 1)];
+#pragma unroll
+        for (int j = 0; j < QP; ++j) {
+            q[j] = g[j] = o[j] = (u32x4){0, 0, 0, 0};
+            l[j] = INFINITY;
+            if (dst[j] >= 0) {
+                q[j] = *(const u32x4*)(qkv + (int64_t)dst[j] * row_stride + head * HD + half8 * 8);
+                g[j] = *(const u32x4*)(dout + (int64_t)dst[j] * channels + head * HD + half8 * 8);
+                o[j] = *(const u32x4*)(out + (int64_t)dst[j] * channels + head * HD + half8 * 8);
+                l[j] = lse[(int64_t)head * n_pad + s0 + ((tid + j * THREADS) >> 1)];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            const T* r = qkv + (int64_t)src[k] * row_stride + channels + head * HD + grp * 4;
+            kf[k] = *(const u32x2*)r;
+            vf[k] = *(const u32x2*)(r + channels);
+            acc_k[k] = zero;
+            acc_v[k] = zero;
+        }
+#pragma unroll
+        for (int j = 0; j < QP; ++j) {
+            const int e = tid + j * THREADS, slot = e >> 1;
+            float d = dot8<T>(g[j], o[j]);
+            d += __shfl_xor(d, 1, PTV3_WAVE);
+            *(u32x4*)(q_lds + e * 16) = scale8<T>(q[j], scale_log2e);
+            *(u32x4*)(do_lds + e * 16) = g[j];
+            if (half8 == 0) {
+                nlse_lds[slot] = -l[j];
+                nd_lds[slot] = -d;
+                dst_lds[slot] = dst[j];
+            }
+        }
+    }
+    // The transposed rows, again by the identity: a wave has just written 32 whole queries per piece and turns those. The
+    // queries of a channel lie in the order in which the score tiles hold them: lane group grp's four of the first tile, then
+    // of the second
+    auto turned = [&](u32x2 a, u32x2 b) {
+        const f32x4 x = Half<T>::mfma16(a, unit, zero), y = Half<T>::mfma16(b, unit, zero);
+        return (u32x4){Half<T>::pack2(x[0], x[1]), Half<T>::pack2(x[2], x[3]), Half<T>::pack2(y[0], y[1]), Half<T>::pack2(y[2], y[3])};
+    };
+#pragma unroll
+    for (int j = 0; j < QP; ++j) {
+        const int at = (wave * PTV3_WAVE + j * THREADS) >> 1;
+        const int row = (at + col) * 32 + grp * 8, t = col * T_STRIDE + at * 2 + grp * 16;
+        *(u32x4*)(qt_lds + t) = turned(*(const u32x2*)(q_lds + row), *(const u32x2*)(q_lds + row + 16 * 32));
+        *(u32x4*)(dot_lds + t) = turned(*(const u32x2*)(do_lds + row), *(const u32x2*)(do_lds + row + 16 * 32));
+    }
+#pragma unroll
+    for (int p = 0; p < KG / 2; ++p) {   // K^T, a lane per channel: here a key that does not exist is zero
+        const u32x2 none = {0, 0};
+        kt[p] = turned(key0 + 32 * p + col < len ? kf[2 * p] : none, key0 + 32 * p + 16 + col < len ? kf[2 * p + 1] : none);
+    }
+    const int blocks = (len + 31) / 32;
+    __syncthreads();
+
+    u32x2 qa[2], ga[2];
+    f32x4 cl[2], cd[2];
+    u32x4 qt, gt;
+    auto fetch = [&](int block) {   // the query side of a step
+        const int at = block * 32;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            qa[t] = *(const u32x2*)(q_lds + (at + t * 16 + col) * 32 + grp * 8);
+            ga[t] = *(const u32x2*)(do_lds + (at + t * 16 + col) * 32 + grp * 8);
+            cl[t] = *(const f32x4*)(nlse_lds + at + t * 16 + grp * 4);
+            cd[t] = *(const f32x4*)(nd_lds + at + t * 16 + grp * 4);
+        }
+        qt = *(const u32x4*)(qt_lds + col * T_STRIDE + at * 2 + grp * 16);
+        gt = *(const u32x4*)(dot_lds + col * T_STRIDE + at * 2 + grp * 16);
+    };
+    fetch(wave);
+    for (int b0 = 0; b0 < blocks; b0 += WAVES) {
+        for (int s = 0; s < WAVES; ++s) {
+            const int blk = (wave + s) & (WAVES - 1);
+            const bool there = b0 + blk < blocks;
+            f32x4 dq[2] = {zero, zero};
+            if (there && mine) {
+                const int at = (b0 + blk) * 32;
+                // group k + 1's scores are on the matrix pipe while group k's exponentials are taken, group k - 1's
+                // transposed dS come back
+                f32x4 sc[2][2], dp[2][2], tr[2][2];
+                u32x4 dst_t[2];   // dS^T of 32 keys for the queries of tile 0 and 1
+                auto scores = [&](int k) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        sc[k & 1][t] = Half<T>::mfma16(qa[t], kf[k], cl[t]);                 // S - lse
+                        dp[k & 1][t] = Half<T>::mfma16(ga[t], vf[k], DROP ? zero : cd[t]);   // dP - D
+                    }
+                };
+                auto collect = [&](int k) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        dst_t[t][2 * (k & 1)] = Half<T>::pack2(tr[k & 1][t][0], tr[k & 1][t][1]);
+                        dst_t[t][2 * (k & 1) + 1] = Half<T>::pack2(tr[k & 1][t][2], tr[k & 1][t][3]);
+                    }
+                    if (k & 1)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) dq[t] = Half<T>::mfma32(kt[k >> 1], dst_t[t], dq[t]);
+                };
+                scores(0);
+#pragma unroll
+                for (int k = 0; k < KG; ++k) {
+                    if (k + 1 < KG) scores(k + 1);
+                    u32x4 pp, dd;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        float e[4], ds[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            e[r] = __builtin_amdgcn_exp2f(sc[k & 1][t][r]);
+                            if (DROP) {
+                                // dV sees the kept, rescaled probabilities, dS = P o (mask o dP / (1 - p) - D)
+                                const uint32_t qs = (uint32_t)(s0 + at + t * 16 + grp * 4 + r);
+                                const bool keep = drop_keep(drop_hq(drop.seed, (uint32_t)head, qs),
+                                                            (uint32_t)(s0 + key0 + k * 16 + col), drop.threshold);
+                                ds[r] = e[r] * ((keep ? dp[k & 1][t][r] * drop.inv_keep : 0.f) + cd[t][r]);
+                                e[r] = keep ? e[r] * drop.inv_keep : 0.f;
+                            } else {
+                                ds[r] = e[r] * dp[k & 1][t][r];
+                            }
+                        }
+                        pp[2 * t] = Half<T>::pack2(e[0], e[1]);
+                        pp[2 * t + 1] = Half<T>::pack2(e[2], e[3]);
+                        dd[2 * t] = Half<T>::pack2(ds[0], ds[1]);
+                        dd[2 * t + 1] = Half<T>::pack2(ds[2], ds[3]);
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) tr[k & 1][t] = Half<T>::mfma16((u32x2){dd[2 * t], dd[2 * t + 1]}, unit, zero);
+                    acc_k[k] = Half<T>::mfma32(qt, dd, acc_k[k]);
+                    acc_v[k] = Half<T>::mfma32(gt, pp, acc_v[k]);
+                    if (k > 0) collect(k - 1);
+                }
+                collect(KG - 1);
+                // as many vector instructions between two matrix instructions as there are per one (224 : 72)
+#pragma unroll
+                for (int i = 0; i < 9 * KG; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x402, 3, 0);   // VALU, transcendental
+                }
+            }
+            if (s + 1 < WAVES) fetch(b0 + ((blk + 1) & (WAVES - 1)));
+            else fetch(min(b0 + WAVES + wave, BOTH_KEYS / 32 - 1));
+            __syncthreads();   // the sums that step s - 1 left are complete, and nobody touches them any more
+            if (there) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    f32x4* sum = (f32x4*)(dq_lds + (blk * 2 + t) * 256 + lane * 4);
+                    if (s > 0) dq[t] += *sum;
+                    if (s < WAVES - 1) {
+                        *sum = dq[t];
+                    } else {
+                        const int dst = dst_lds[(b0 + blk) * 32 + t * 16 + col];
+                        if (dst >= 0)
+                            *(u32x2*)(dqkv + (int64_t)dst * row_stride + head * HD + 4 * grp) =
+                                (u32x2){Half<T>::pack2(dq[t][0] * scale, dq[t][1] * scale),
+                                        Half<T>::pack2(dq[t][2] * scale, dq[t][3] * scale)};
+                    }
+                }
+            }
+        }
+    }
+
+#pragma unroll
+    for (int k = 0; k < KG; ++k) {
+        const int key = key0 + k * 16 + col;
+        if (key >= len) continue;
+        // a real slot owns its row of dqkv; a filler's share is parked per slot and added afterwards.
+        // Q^T was staged times scale * log2(e): dK = scale * dS^T Q = (dS^T Q_staged) * ln 2
+        const int dst = dst_lds[key];
+        T* base = dst >= 0 ? dqkv + (int64_t)dst * row_stride + channels + head * HD + 4 * grp
+                           : fill + (int64_t)(s0 + key) * 2 * channels + head * HD + 4 * grp;
+        *(u32x2*)base = (u32x2){Half<T>::pack2(acc_k[k][0] * LN2, acc_k[k][1] * LN2),
+                                Half<T>::pack2(acc_k[k][2] * LN2, acc_k[k][3] * LN2)};
+        *(u32x2*)(base + channels) = (u32x2){Half<T>::pack2(acc_v[k][0], acc_v[k][1]), Half<T>::pack2(acc_v[k][2], acc_v[k][3])};
     }
 }
 
@@ -766,21 +1021,39 @@ int launch_half_bwd(const void* qkv, const void* out, const void* dout, int chan
     const int64_t total = n_seq * heads;
     const int64_t rem = total % slots;
     int64_t full = total - rem, split = 1;
-    if (rem != 0) {
-        double best = 1.0;
+    double best = 1.0;
+    if (rem != 0)
         for (int64_t sp = 2; sp <= 4; ++sp) {
             const double cost = (double)((rem * sp + slots - 1) / slots) * (1.0 / (double)sp + 0.15);
             if (cost < best - 1e-9) { best = cost; split = sp; }
         }
+    // The both-sides kernel holds BOTH_KEYS keys and needs the forward's log-sum-exps. It does an item in 0.78 of the time
+    // of the two kernels (84 against 107 us for 240 items of 1024 slots), so a last round that their ranges bring below 0.7
+    // is left to them, as are sequences that would leave half of its waves without keys (1600 items of 200 slots: 109
+    // against 104 us; 800 of 700 slots: 199 against 214 us).
+    int64_t first = 0;
+    if (lse && max_seqlen <= BOTH_KEYS && max_seqlen > BOTH_KEYS / 2) first = rem == 0 || best > 0.7 ? total : full;
+    if (split == 1 || first == total) full = total;
+    if (first > 0) {
+        constexpr size_t lds_both = 2 * BOTH_KEYS * 32 + 2 * HD * (BOTH_KEYS * 2 + VT_PAD_BYTES) + 3 * BOTH_KEYS * sizeof(float) +
+                                    BOTH_WAVES * 32 * HD * sizeof(float);
+        static_assert(lds_both <= 160 * 1024, "one work-group fills a CU's LDS");
+        auto kb = dropping ? attn_bwd_both_kernel<T, BOTH_WAVES, true> : attn_bwd_both_kernel<T, BOTH_WAVES, false>;
+        static LdsGrant grant_both[2];
+        if (const int rc_ = ptv3_allow_lds((const void*)kb, lds_both, grant_both[dropping])) return rc_;
+        hipLaunchKernelGGL(kb, dim3((unsigned)first), dim3(BOTH_WAVES * PTV3_WAVE), lds_both, stream, (const T*)qkv, (const T*)out,
+                           (const T*)dout, channels, heads, slot_src, slot_dst, cu_seqlens, scale, n_pad, lse, (T*)dqkv,
+                           (T*)ws.fill, drop);
     }
-    if (split == 1) full = total;
-    const unsigned grid = (unsigned)(full + (total - full) * split);
-    hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, stream, (const T*)qkv, (const T*)out, (const T*)dout,
-                       channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, (T*)dqkv, lse_buf, ws.d,
-                       (int)full, (int)split, drop);
-    hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, stream, (const T*)qkv, (const T*)dout, channels,
-                       heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, lse_buf, ws.d, (T*)dqkv,
-                       (T*)ws.fill, (int)full, (int)split, drop);
+    if (first < total) {
+        const unsigned grid = (unsigned)(full - first + (total - full) * split);
+        hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, stream, (const T*)qkv, (const T*)out, (const T*)dout,
+                           channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, (T*)dqkv, lse_buf, ws.d,
+                           (int)first, (int)full, (int)split, drop);
+        hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, stream, (const T*)qkv, (const T*)dout, channels,
+                           heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, lse_buf, ws.d, (T*)dqkv,
+                           (T*)ws.fill, (int)first, (int)full, (int)split, drop);
+    }
     const int64_t items = n_pad * (2 * channels / 8);
     hipLaunchKernelGGL(attn_bwd_fill_kernel<T>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
                        (const T*)ws.fill, channels, slot_src, slot_dst, n_pad, (T*)dqkv);

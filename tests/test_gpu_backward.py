@@ -155,6 +155,42 @@ def test_attention_backward_recomputes_lse_when_not_kept(dtype):
     assert rel_err(redone, kept.float().cpu()) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,heads,drop_p", [([1024] * 130, 2, 0.0), ([1024] * 86, 3, 0.2), ([513, 1024, 1000, 1, 33] * 20, 3, 0.0),
+                                               ([545] * 65, 4, 0.1), ([1023] * 150, 3, 0.0)])
+def test_attention_backward_both_sides(dtype, lens, heads, drop_p):
+    """Enough long sequences for the kernel that takes queries and keys at once, some with a last round for the other two:
+    every third row of the first sequence is repeated by filler slots of the second. Against the two kernels (a call
+    without the log-sum-exps) and, three sequences, fp32 autograd."""
+    o = ops()
+    g = torch.Generator().manual_seed(len(lens) + heads)
+    n_slots, C = sum(lens), heads * 16
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32)
+    fillers = torch.arange(lens[0], lens[0] + lens[1], 3)[:lens[0] // 3]   # slots of the second sequence
+    real = torch.ones(n_slots, dtype=torch.bool)
+    real[fillers] = False
+    n = int(real.sum())
+    src = torch.empty(n_slots, dtype=torch.int32)
+    src[real] = torch.randperm(n, generator=g).int()
+    src[fillers] = src[torch.arange(0, 3 * len(fillers), 3)]
+    dst = torch.where(real, src, torch.full_like(src, -1))
+    qkv = torch.randn(n, 3 * C, generator=g).to(dtype)
+    dout = torch.randn(n, C, generator=g).to(dtype)
+    args = (heads, to_dev(src), to_dev(dst), to_dev(cu), max(lens), 0.25)
+    x, d = qkv.to(DEV), dout.to(DEV)
+    out, lse = o.patch_attention_lse(x, *args, dropout_p=drop_p, seed=5)
+    got = o.patch_attention_bwd(x, out, d, *args, lse=lse, dropout_p=drop_p, seed=5)
+    assert torch.equal(got, o.patch_attention_bwd(x, out, d, *args, lse=lse, dropout_p=drop_p, seed=5))
+    assert rel_err(got, o.patch_attention_bwd(x, out, d, *args, dropout_p=drop_p, seed=5).float().cpu()) < TOL[dtype]
+    if drop_p == 0.0:
+        for s in (2, len(lens) // 2, len(lens) - 1):
+            rows = src[cu[s]:cu[s + 1]].long()
+            p = qkv[rows].float().reshape(-1, 3, heads, 16).permute(1, 2, 0, 3).contiguous().requires_grad_(True)
+            y = torch.softmax(p[0] @ p[1].transpose(1, 2).contiguous() * 0.25, -1) @ p[2]
+            y.backward(dout[rows].float().reshape(-1, heads, 16).permute(1, 0, 2).contiguous())
+            assert rel_err(got.cpu()[rows], p.grad.permute(2, 0, 1, 3).reshape(-1, 3 * C)) < TOL[dtype]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("cin,cout,ks,n", [(6, 32, 5, 1500), (32, 32, 3, 2000), (64, 64, 3, 3000), (128, 128, 3, 1200),
                                            (48, 80, 3, 700)])
