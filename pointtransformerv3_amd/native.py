@@ -386,23 +386,25 @@ class Engine:
         feat = data["feat"].contiguous()
         point = Point.__new__(Point)
         dict.update(point, data)
-        grid, offset, batch = coordinates(point)
 
         def refresh():
             # whoever writes the parameters behind autograd's back leaves no trace on them: every derived copy is
             # redone once per forward
             _lib.check(lib.ptv3_net_refresh(ctypes.byref(self._refresh), ops._stream()), "ptv3_net_refresh")
 
-        args = (self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want)
+        def index_of(between=None):
+            return levels.build(self.layout, *coordinates(point), model.order, model.shuffle_orders, self.want, between=between)
+
         if model.overlap_index_prologue:
             if model._prologue_state is None or model._prologue_state.device != feat.device:
                 model._prologue_state = ops.PrologueOverlap(feat.device)
             refresh()
             with model._prologue_state.scope():
-                index = levels.build(*args)
+                # the conversions of the inputs too: that stream waits for nothing, so what it reads is made on it
+                index = index_of()
         else:
             model._prologue_state = None
-            index = levels.build(*args, between=refresh)
+            index = index_of(between=refresh)
         lv = index.levels
         n = feat.shape[0]
         stage_out, rows = None, None

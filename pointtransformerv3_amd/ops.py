@@ -713,7 +713,8 @@ class PrologueOverlap:
     whatever the caller queued on its results before calling again. The few tensors of a result that a caller may
     still read after that (PUBLIC_KEYS) are marked for the current stream by forward_queued()."""
 
-    PUBLIC_KEYS = ("batch", "serialized_code", "serialized_order", "serialized_inverse", "pad", "unpad", "cu_seqlens_key")
+    PUBLIC_KEYS = ("batch", "offset", "grid_coord", "serialized_code", "serialized_order", "serialized_inverse", "pad", "unpad",
+                   "cu_seqlens_key", "_sparse_indices", "pooling_inverse")
 
     def __init__(self, device):
         self.device = device
@@ -750,10 +751,12 @@ class PrologueOverlap:
         may read on the current stream at any later time are marked for that stream (the allocator then holds their
         memory back until those reads are over); everything else of the index belongs to the forward."""
         main = torch.cuda.current_stream(self.device)
-        for key in self.PUBLIC_KEYS:
-            t = point.get(key)
-            if isinstance(t, torch.Tensor) and t.is_cuda:
-                t.record_stream(main)
+        while point is not None:   # an encoder-only result hands out the levels above as well
+            for key in self.PUBLIC_KEYS:
+                t = point.get(key)
+                if isinstance(t, torch.Tensor) and t.is_cuda:
+                    t.record_stream(main)
+            point = point.get("pooling_parent")
 
 
 def conv_plan_direct_start(indices, ks):

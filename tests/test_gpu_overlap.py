@@ -51,6 +51,54 @@ def test_overlapped_prologue_changes_no_bit_over_a_sequence_of_different_inputs(
     assert all(torch.equal(a[0], b[0]) for a, b in zip(want, again))
 
 
+def _converted(data, form):
+    """The same scenes in a form whose tensors the model has to convert before its kernels can read them."""
+    if form == "int64 coordinates":
+        return dict(data, grid_coord=data["grid_coord"].long())
+    if form == "strided coordinates":
+        return dict(data, grid_coord=data["grid_coord"].t().contiguous().t())
+    if form == "int32 offset":
+        return dict(data, offset=data["offset"].int())
+    rest = {k: v for k, v in data.items() if k != ("offset" if "batch" in form else "grid_coord")}
+    if form in ("batch", "int32 batch"):
+        ends = torch.nn.functional.pad(data["offset"], (1, 0))
+        batch = torch.arange(len(data["offset"]), device=DEV).repeat_interleave(ends[1:] - ends[:-1])
+        return dict(rest, batch=batch.int() if "int32" in form else batch)
+    # a scene's coordinates at a quarter of the grid: the division truncates to the same cells
+    return dict(rest, coord=(data["grid_coord"].float() + 0.25) * 0.5, grid_size=0.5)
+
+
+@pytest.mark.parametrize("form", ["int64 coordinates", "strided coordinates", "int32 offset", "batch", "int32 batch",
+                                  "coord and grid size"])
+@pytest.mark.parametrize("use_native", [True, False])
+def test_overlapped_prologue_converts_its_inputs_behind_nothing_else(form, use_native, monkeypatch):
+    """Inputs that are complete before the call but need a conversion: made on the stream that reads them."""
+    from pointtransformerv3_amd import PointTransformerV3, native
+    if not use_native:
+        monkeypatch.setattr(native, "engine_for", lambda m, d: None)
+    torch.manual_seed(3)
+    kw = dict(enc_depths=(1, 1, 2, 1, 1), dec_depths=(1, 1, 1, 1), enc_patch_size=(256,) * 5, dec_patch_size=(256,) * 4)
+    model = PointTransformerV3(**kw).eval().half().to(DEV)
+    datas = [_converted(_inputs(s, n, p), form) for s, n, p in ((11, 2, 9000), (23, 3, 4000), (37, 1, 15000))]
+    seq = [0, 1, 2, 2, 0, 1, 0, 0, 2, 1]
+    torch.cuda.synchronize()
+
+    def run(flag):
+        model.overlap_index_prologue = flag
+        outs = []
+        with torch.inference_mode():
+            for k, i in enumerate(seq):
+                torch.manual_seed(100 + k)
+                out = model(dict(datas[i]))
+                outs.append([out[key].clone() for key in ("feat", "serialized_order", "grid_coord", "offset")])
+                del out
+        torch.cuda.synchronize()
+        return outs
+
+    for want, got in zip(run(False), run(True)):
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
 def test_overlap_is_left_alone_in_training_mode_and_under_autograd():
     from pointtransformerv3_amd import PointTransformerV3
     torch.manual_seed(5)
