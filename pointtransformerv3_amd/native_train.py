@@ -233,6 +233,10 @@ class TrainEngine:
         return point
 
 
+def _addresses(tensors):
+    return (_ptr * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
+
+
 class _Step(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, feat, index, masks, *params):
@@ -243,10 +247,10 @@ class _Step(torch.autograd.Function):
         _lib.check(lib.ptv3_train_bytes(ctypes.byref(engine.net), index.levels, at, at + 8, at + 16), "ptv3_train_bytes")
         acts, scratch = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
         out = torch.empty((feat.shape[0], engine.out_channels), dtype=torch.float32, device=feat.device)
-        mask_ptrs = (_ptr * len(masks))(*[None if m is None else m.data_ptr() for m in masks])
-        _lib.check(lib.ptv3_train_fwd(ctypes.byref(engine.net), index.levels, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype], mask_ptrs,
-                                      acts.data_ptr(), scratch.data_ptr(), sizes[1], out.data_ptr(), ops._stream()), "ptv3_train_fwd")
-        ctx.engine, ctx.index, ctx.mask_ptrs, ctx.scratch_bytes = engine, index, mask_ptrs, sizes[2]
+        _lib.check(lib.ptv3_train_fwd(ctypes.byref(engine.net), index.levels, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype],
+                                      _addresses(masks), acts.data_ptr(), scratch.data_ptr(), sizes[1], out.data_ptr(), ops._stream()), "ptv3_train_fwd")
+        ctx.engine, ctx.index, ctx.scratch_bytes = engine, index, sizes[2]
+        ctx.masked = [m is not None for m in masks]
         # freed by autograd after the backward, as the activations of separate nodes would be
         ctx.save_for_backward(acts, *[m for m in masks if m is not None])
         return out
@@ -255,12 +259,17 @@ class _Step(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dout):
         engine, index = ctx.engine, ctx.index
-        acts = ctx.saved_tensors[0]
+        # under saved-tensor hooks (checkpointing, offloading) these are not the tensors of the forward but what the hooks
+        # made of them: every address is taken here, and the views the kernels assume are made sure of
+        acts, *kept = [t if t.is_contiguous() and t.data_ptr() % 256 == 0 else t.clone(memory_format=torch.contiguous_format)
+                       for t in ctx.saved_tensors]
+        kept = iter(kept)
+        masks = [next(kept) if masked else None for masked in ctx.masked]
         dout = dout.contiguous()
         scratch = torch.empty(ctx.scratch_bytes, dtype=torch.uint8, device=dout.device)
         grads = torch.empty(engine.total, dtype=torch.float32, device=dout.device)
         _lib.check(_lib.load().ptv3_train_bwd(ctypes.byref(engine.net), index.levels, dout.data_ptr(), ops.DTYPE_CODES[dout.dtype],
-                                              ctx.mask_ptrs, acts.data_ptr(), scratch.data_ptr(), ctx.scratch_bytes,
+                                              _addresses(masks), acts.data_ptr(), scratch.data_ptr(), ctx.scratch_bytes,
                                               grads.data_ptr(), ops._stream()), "ptv3_train_bwd")
         views = torch._utils._unflatten_dense_tensors(grads, engine.params)
         needed = ctx.needs_input_grad[4:]

@@ -96,3 +96,44 @@ def test_native_training_follows_the_optimizer_and_leaves_other_modes_alone(monk
     out.sum().backward()
     with pytest.raises(RuntimeError):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("how", ["checkpoint", "offload"])
+def test_native_training_step_under_saved_tensor_hooks(how):
+    """What autograd keeps for the backward may be recomputed or moved: stochastic-depth factors and activations are read
+    from where they are when the backward runs. The same step twice: the batch statistics are summed by atomics, so single
+    roundings to half differ as they do between this path and the modules, whose tolerance is taken; another set of rows
+    kept by stochastic depth, or activations overwritten, would be wrong by the size of a branch."""
+    from torch.utils.checkpoint import checkpoint
+    from pointtransformerv3_amd import PointTransformerV3, native_train
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).to(DEV).train()
+    data = _inputs(4, (6000,), torch.float32)
+    taken, real = [], native_train.engine_for
+
+    def step(hooked):
+        model.zero_grad(set_to_none=True)
+        torch.manual_seed(5)
+        with torch.autocast("cuda", dtype=torch.float16):
+            if hooked and how == "checkpoint":
+                feat = checkpoint(lambda d: model(dict(d)).feat, data, use_reentrant=False)
+            elif hooked:
+                with torch.autograd.graph.save_on_cpu():
+                    feat = model(dict(data)).feat
+            else:
+                feat = model(dict(data)).feat
+        # other work takes the memory that was let go
+        fill = [torch.full((1 << k,), float("nan"), device=DEV) for k in range(6, 22)]
+        del fill
+        feat.backward(torch.full_like(feat, 0.01))
+        return feat.detach().clone(), [p.grad.clone() for p in model.parameters()]
+
+    native_train.engine_for = lambda m, d: taken.append(real(m, d)) or taken[-1]
+    try:
+        want, got = step(False), step(True)
+    finally:
+        native_train.engine_for = real
+    assert len(taken) >= 2 and all(e is not None for e in taken)
+    rel = lambda x, y: float((x.double() - y.double()).norm() / y.double().norm())
+    assert rel(got[0], want[0]) < 2e-2
+    assert rel(*(torch.cat([g.reshape(-1) for g in gs]) for gs in (got[1], want[1]))) < 2e-2

@@ -1,11 +1,12 @@
 """Host-side rules of the natively queued paths that need no GPU."""
 import contextlib
+import ctypes
 import types
 
 import pytest
 import torch
 
-from pointtransformerv3_amd import native
+from pointtransformerv3_amd import native, native_train
 
 
 class _Stop(Exception):
@@ -40,3 +41,65 @@ def test_inputs_are_converted_where_the_index_reads_them(overlap, monkeypatch):
     with pytest.raises(_Stop):
         engine.forward(model, dict(feat=torch.zeros(4, 6), grid_coord=torch.zeros(4, 3, dtype=torch.int64), offset=torch.tensor([4])))
     assert seen == [overlap]
+
+
+class _TrainLib:
+    """Stands in for the library: the two calls of a training step, their stochastic-depth factors read as kernels would."""
+
+    def __init__(self, rows):
+        self.rows, self.read = rows, []
+
+    def ptv3_train_bytes(self, net, levels, acts, fwd, bwd):
+        for at in (acts, fwd, bwd):
+            ctypes.c_size_t.from_address(at).value = 512
+        return 0
+
+    def _masks(self, masks):
+        self.read.append([None if not at else list((ctypes.c_float * self.rows).from_address(at)) for at in masks])
+        return 0
+
+    def ptv3_train_fwd(self, net, levels, feat, dt, masks, *rest):
+        return self._masks(masks)
+
+    def ptv3_train_bwd(self, net, levels, dout, dt, masks, *rest):
+        ctypes.memset(rest[3], 0, 4)   # the one gradient
+        return self._masks(masks)
+
+
+@pytest.fixture
+def train_step(monkeypatch):
+    """step(masks) -> rows of a step whose engine holds one parameter, over stand-ins for the library's two calls."""
+    lib = _TrainLib(6)
+    monkeypatch.setattr(native_train._lib, "load", lambda: lib)
+    monkeypatch.setattr(native_train.ops, "_stream", lambda: None)
+    weight = torch.nn.Parameter(torch.ones(1))
+    engine = types.SimpleNamespace(net=native_train._Net(), out_channels=4, total=1, params=[weight])
+    index = types.SimpleNamespace(levels=None)
+
+    def step(masks):
+        return native_train._Step.apply(engine, torch.zeros(6, 6), index, masks, weight)
+
+    return types.SimpleNamespace(step=step, lib=lib, weight=weight, engine=engine)
+
+
+@pytest.mark.parametrize("hooks", ["none", "copies", "misaligned copies"])
+def test_backward_of_a_step_reads_the_masks_that_autograd_kept(hooks, train_step):
+    """Saved-tensor hooks (checkpointing, offloading to the host) keep copies and let the originals go."""
+    masks = [None, torch.arange(6.0).view(6, 1), None, torch.arange(6.0).neg().view(6, 1)]
+    want = [None if m is None else m.flatten().tolist() for m in masks]
+
+    def unpack(t):
+        if hooks != "misaligned copies" or t.dtype == torch.uint8:
+            return t
+        return torch.cat([t.new_zeros(1, 1), t])[1:]
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), unpack) if hooks != "none" else contextlib.nullcontext():
+        out = train_step.step(masks)
+    if hooks != "none":
+        for m in masks:     # what their memory holds once it has been handed out again
+            if m is not None:
+                m.fill_(7.0)
+    del masks
+    out.sum().backward()
+    assert train_step.lib.read == [want, want]
+    assert float(train_step.weight.grad) == 0.0
