@@ -64,7 +64,9 @@ class TrainEngine:
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() and p.dtype == torch.float32
                   for p in self.structure.tensors), "float weights on one GPU")
         _need(not model.cls_mode, "the encoder-only model hands out intermediate features")
+        _need(not any(p.is_inference() for p in self.params), "inference tensors")
         self._keep, self._casts, self._packs, self._zero = [], [], [], []
+        self.read_back = []             # parameters whose values the backward reads, itself or as a copy made by the forward
         self._at, offset = {}, 0        # parameter -> place of its gradient
         for p in self.params:
             self._at[p] = offset
@@ -87,20 +89,26 @@ class TrainEngine:
         self._casts.append((t, dst, shape, int(layout != "plain")))
         return dst
 
+    def versions(self):
+        return [p._version for p in self.read_back]
+
     def _linear(self, m, cin, cout):
         _need(type(m) is nn.Linear and m.bias is not None and m.in_features == cin and m.out_features == cout, "Linear")
+        self.read_back.append(m.weight)
         return _Linear(self._copy(m.weight), self._copy(m.weight, "transpose"), self._copy(m.bias), cin, cout,
                        self._at[m.weight], self._at[m.bias])
 
     def _norm(self, m, c):
         _need(m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
         self._zero += [(self._at[m.weight], c), (self._at[m.bias], c)]
+        self.read_back.append(m.weight)
         return _Norm(m.weight.data_ptr(), m.bias.data_ptr(), m.eps, 0, self._at[m.weight], self._at[m.bias])
 
     def _bn(self, m, c):
         _need(type(m) is nn.BatchNorm1d and m.num_features == c and m.weight is not None and m.bias is not None
               and m.track_running_stats and m.running_mean is not None and m.momentum is not None, "BatchNorm1d")
         _need(self._at[m.bias] == self._at[m.weight] + c, "order of a BatchNorm's parameters")
+        self.read_back += [m.weight, m.bias]
         return _Bn(m.weight.data_ptr(), m.bias.data_ptr(), self._copy(m.weight), self._copy(m.bias), m.running_mean.data_ptr(),
                    m.running_var.data_ptr(), m.eps, m.momentum, self._at[m.weight])
 
@@ -108,6 +116,7 @@ class TrainEngine:
         conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
         _need(attn.attn_drop == 0 and attn.proj_drop.p == 0 and mlp.drop.p == 0 and c // attn.num_heads == 16, "dropout or head size")
         d = _Block(channels=c, heads=attn.num_heads, row=attn.order_index, scale=attn.scale)
+        self.read_back.append(conv.weight)
         d.conv_w, d.conv_b, d.conv_mirror = self._copy(conv.weight), self._copy(conv.bias), self._copy(conv.weight, "mirror")
         if c in native.CONV_PACKED:
             d.conv_packed, d.conv_mirror_packed = self._buffer(27 * c * c), self._buffer(27 * c * c)
@@ -251,8 +260,9 @@ class _Step(torch.autograd.Function):
                                       _addresses(masks), acts.data_ptr(), scratch.data_ptr(), sizes[1], out.data_ptr(), ops._stream()), "ptv3_train_fwd")
         ctx.engine, ctx.index, ctx.scratch_bytes = engine, index, sizes[2]
         ctx.masked = [m is not None for m in masks]
-        # freed by autograd after the backward, as the activations of separate nodes would be
-        ctx.save_for_backward(acts, *[m for m in masks if m is not None])
+        # freed by autograd after the backward, as the activations of separate nodes would be; the versions go with them, so
+        # that activations which a checkpoint computes again are held against the weights they were computed with
+        ctx.save_for_backward(acts, torch.tensor(engine.versions()), *[m for m in masks if m is not None])
         return out
 
     @staticmethod
@@ -261,8 +271,14 @@ class _Step(torch.autograd.Function):
         engine, index = ctx.engine, ctx.index
         # under saved-tensor hooks (checkpointing, offloading) these are not the tensors of the forward but what the hooks
         # made of them: every address is taken here, and the views the kernels assume are made sure of
+        acts, versions, *kept = ctx.saved_tensors
+        # the weights' copies are the engine's and follow the weights at every forward, so a weight that was written since
+        # this step's forward is an error, as it is where every node saves its own
+        if versions.tolist() != engine.versions():
+            raise RuntimeError("one of the variables needed for gradient computation has been modified by an inplace operation: "
+                               "a parameter of PointTransformerV3 was written between a training step's forward and its backward")
         acts, *kept = [t if t.is_contiguous() and t.data_ptr() % 256 == 0 else t.clone(memory_format=torch.contiguous_format)
-                       for t in ctx.saved_tensors]
+                       for t in (acts, *kept)]
         kept = iter(kept)
         masks = [next(kept) if masked else None for masked in ctx.masked]
         dout = dout.contiguous()

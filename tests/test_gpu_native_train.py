@@ -137,3 +137,21 @@ def test_native_training_step_under_saved_tensor_hooks(how):
     rel = lambda x, y: float((x.double() - y.double()).norm() / y.double().norm())
     assert rel(got[0], want[0]) < 2e-2
     assert rel(*(torch.cat([g.reshape(-1) for g in gs]) for gs in (got[1], want[1]))) < 2e-2
+
+
+def test_native_training_step_notices_weights_written_before_its_backward():
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0, **KW).to(DEV).train()
+    data = _inputs(4, (3000,), torch.float32)
+    step = lambda: model(dict(data)).feat
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        first = step()
+        with torch.no_grad():
+            model.enc.enc2.block0.attn.proj.weight.mul_(1.5)
+            model.enc.enc2.block0.attn.proj.bias.mul_(1.5)
+        second = step()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        first.sum().backward()
+    second.sum().backward()
+    assert all(torch.isfinite(p.grad).all() for p in model.parameters())

@@ -73,7 +73,9 @@ def train_step(monkeypatch):
     monkeypatch.setattr(native_train._lib, "load", lambda: lib)
     monkeypatch.setattr(native_train.ops, "_stream", lambda: None)
     weight = torch.nn.Parameter(torch.ones(1))
-    engine = types.SimpleNamespace(net=native_train._Net(), out_channels=4, total=1, params=[weight])
+    engine = types.SimpleNamespace(net=native_train._Net(), out_channels=4,
+                                   total=1, params=[weight], read_back=[weight])
+    engine.versions = types.MethodType(native_train.TrainEngine.versions, engine)
     index = types.SimpleNamespace(levels=None)
 
     def step(masks):
@@ -89,7 +91,7 @@ def test_backward_of_a_step_reads_the_masks_that_autograd_kept(hooks, train_step
     want = [None if m is None else m.flatten().tolist() for m in masks]
 
     def unpack(t):
-        if hooks != "misaligned copies" or t.dtype == torch.uint8:
+        if hooks != "misaligned copies" or t.dim() < 2:
             return t
         return torch.cat([t.new_zeros(1, 1), t])[1:]
 
@@ -103,3 +105,23 @@ def test_backward_of_a_step_reads_the_masks_that_autograd_kept(hooks, train_step
     out.sum().backward()
     assert train_step.lib.read == [want, want]
     assert float(train_step.weight.grad) == 0.0
+
+
+def test_backward_of_a_step_refuses_weights_written_since_its_forward(train_step):
+    """The engine's copies of the weights follow the weights: the gradients would be those of another function."""
+    out = train_step.step([None])
+    with torch.no_grad():
+        train_step.weight.mul_(2.0)
+    again = train_step.step([None])
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+    again.sum().backward()           # a step whose weights stand is not held up
+
+
+def test_checkpointed_step_is_held_against_the_weights_it_was_computed_again_with(train_step):
+    from torch.utils.checkpoint import checkpoint
+    out = checkpoint(lambda: train_step.step([None]), use_reentrant=False)
+    with torch.no_grad():
+        train_step.weight.mul_(2.0)
+    out.sum().backward()             # the forward ran again, with the weights as they are now
+    assert len(train_step.lib.read) == 3
