@@ -59,19 +59,17 @@ class TrainEngine:
     def __init__(self, model, dtype):
         self.structure = Structure(model)
         self.dtype = dtype
-        self.params = [p for p in model.parameters()]
-        self.device = self.params[0].device
+        self.device = self.structure.tensors[0].device
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() and p.dtype == torch.float32
                   for p in self.structure.tensors), "float weights on one GPU")
         _need(not model.cls_mode, "the encoder-only model hands out intermediate features")
-        _need(not any(p.is_inference() for p in self.params), "inference tensors")
+        _need(not any(p.is_inference() for p in self.structure.tensors), "inference tensors")
         self._keep, self._casts, self._packs, self._zero = [], [], [], []
         self.read_back = []             # parameters whose values the backward reads, itself or as a copy made by the forward
-        self._at, offset = {}, 0        # parameter -> place of its gradient
-        for p in self.params:
-            self._at[p] = offset
-            offset += p.numel()
-        self.total = offset
+        # the parameters of the step's node, in the order their gradients lie in the flat buffer: those that the
+        # description places, each of which the backward writes once and in whole. A subclass may hold more (a head, a
+        # mask token): they are no part of this node
+        self.params, self._placed, self.total = [], set(), 0
         self._describe(model)
         self._finish()
         self.batches = [m.num_batches_tracked for m in self.structure.modules
@@ -89,6 +87,15 @@ class TrainEngine:
         self._casts.append((t, dst, shape, int(layout != "plain")))
         return dst
 
+    def _at(self, p):
+        """Place of the parameter's gradient. Gradients are written, not added up: a parameter has one place."""
+        _need(p not in self._placed, "a parameter that is used twice")
+        self._placed.add(p)
+        self.params.append(p)
+        at = self.total
+        self.total += p.numel()
+        return at
+
     def versions(self):
         return [p._version for p in self.read_back]
 
@@ -96,21 +103,23 @@ class TrainEngine:
         _need(type(m) is nn.Linear and m.bias is not None and m.in_features == cin and m.out_features == cout, "Linear")
         self.read_back.append(m.weight)
         return _Linear(self._copy(m.weight), self._copy(m.weight, "transpose"), self._copy(m.bias), cin, cout,
-                       self._at[m.weight], self._at[m.bias])
+                       self._at(m.weight), self._at(m.bias))
 
     def _norm(self, m, c):
         _need(m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
-        self._zero += [(self._at[m.weight], c), (self._at[m.bias], c)]
+        gg, gb = self._at(m.weight), self._at(m.bias)
+        self._zero += [(gg, c), (gb, c)]
         self.read_back.append(m.weight)
-        return _Norm(m.weight.data_ptr(), m.bias.data_ptr(), m.eps, 0, self._at[m.weight], self._at[m.bias])
+        return _Norm(m.weight.data_ptr(), m.bias.data_ptr(), m.eps, 0, gg, gb)
 
     def _bn(self, m, c):
         _need(type(m) is nn.BatchNorm1d and m.num_features == c and m.weight is not None and m.bias is not None
               and m.track_running_stats and m.running_mean is not None and m.momentum is not None, "BatchNorm1d")
-        _need(self._at[m.bias] == self._at[m.weight] + c, "order of a BatchNorm's parameters")
+        gg, gb = self._at(m.weight), self._at(m.bias)   # the kernel writes both, one behind the other
+        assert gb == gg + c
         self.read_back += [m.weight, m.bias]
         return _Bn(m.weight.data_ptr(), m.bias.data_ptr(), self._copy(m.weight), self._copy(m.bias), m.running_mean.data_ptr(),
-                   m.running_var.data_ptr(), m.eps, m.momentum, self._at[m.weight])
+                   m.running_var.data_ptr(), m.eps, m.momentum, gg)
 
     def _block(self, b, c):
         conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
@@ -121,7 +130,7 @@ class TrainEngine:
         if c in native.CONV_PACKED:
             d.conv_packed, d.conv_mirror_packed = self._buffer(27 * c * c), self._buffer(27 * c * c)
             self._packs += [(d.conv_w, d.conv_packed, c, 27), (d.conv_mirror, d.conv_mirror_packed, c, 27)]
-        d.g_conv_w, d.g_conv_b = self._at[conv.weight], self._at[conv.bias]
+        d.g_conv_w, d.g_conv_b = self._at(conv.weight), self._at(conv.bias)
         d.cpe, d.qkv, d.proj = self._linear(b.cpe[1], c, c), self._linear(attn.qkv, c, 3 * c), self._linear(attn.proj, c, c)
         d.fc1, d.fc2 = self._linear(mlp.fc1, c, 4 * c), self._linear(mlp.fc2, 4 * c, c)
         d.ln_cpe, d.ln1, d.ln2 = self._norm(b.cpe[2], c), self._norm(b.norm1[0], c), self._norm(b.norm2[0], c)
@@ -134,7 +143,7 @@ class TrainEngine:
         conv = p.stem_conv
         padded = -(-conv.in_channels // 16) * 16
         net.stem.w = self._buffer(conv.out_channels * 125 * padded)
-        net.stem.cin, net.stem.cin_padded, net.stem.gw = conv.in_channels, padded, self._at[conv.weight]
+        net.stem.cin, net.stem.cin_padded, net.stem.gw = conv.in_channels, padded, self._at(conv.weight)
         net.stem.bn = self._bn(p.stem_bn, conv.out_channels)
         self._refresh = native._Refresh(dtype=net.dtype, stem_src=self._copy(conv.weight), stem_dst=net.stem.w,
                                         stem_rows=conv.out_channels * 125, stem_in=conv.in_channels, stem_padded=padded)

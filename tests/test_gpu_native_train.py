@@ -155,3 +155,55 @@ def test_native_training_step_notices_weights_written_before_its_backward():
         first.sum().backward()
     second.sum().backward()
     assert all(torch.isfinite(p.grad).all() for p in model.parameters())
+
+
+@pytest.mark.parametrize("extra", ["head", "mask token", "shared block", "shared norm"])
+def test_gradients_of_models_that_hold_more_or_less_than_the_backbone(extra, monkeypatch):
+    """A parameter outside the backbone gets its own gradient and nothing else; one used twice gets the sum of both."""
+    from pointtransformerv3_amd import PointTransformerV3, native_train
+
+    class Segmentor(PointTransformerV3):
+        def __init__(self, **kw):
+            super().__init__(**kw)
+            if extra == "head":
+                self.head = torch.nn.Linear(64, 13)
+            elif extra == "mask token":
+                self.token = torch.nn.Parameter(torch.ones(64))
+
+        def forward(self, data):
+            point = super().forward(data)
+            if extra == "head":
+                point.feat = self.head(point.feat)
+            elif extra == "mask token":
+                point.feat = point.feat * self.token
+            return point
+
+    torch.manual_seed(3)
+    model = Segmentor(drop_path=0.0, **dict(KW, enc_depths=(1, 2, 2, 1, 1))).to(DEV).train()
+    if extra == "shared block":
+        model.enc.enc1.block1 = model.enc.enc1.block0
+    elif extra == "shared norm":
+        model.enc.enc2.block1.norm2 = model.enc.enc2.block0.norm1
+    data = _inputs(4, (5000,), torch.float32)
+    other = copy.deepcopy(model)
+    label = (data["grid_coord"].sum(1) % 5).long()
+    taken, real = [], native_train.engine_for
+
+    def grads(m, use):
+        monkeypatch.setattr(native_train, "engine_for", (lambda a, b: taken.append(real(a, b)) or taken[-1]) if use else lambda a, b: None)
+        torch.full((1 << 24,), float("nan"), device=DEV)     # what freed memory holds
+        torch.manual_seed(5)
+        with torch.autocast("cuda", dtype=torch.float16):
+            feat = m(dict(data)).feat
+        w = torch.randn(5, feat.shape[1], generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+        feat.backward((w[label] * 0.05).to(feat.dtype))
+        return {n: p.grad for n, p in m.named_parameters()}
+
+    got, want = grads(model, True), grads(other, False)
+    assert (taken[0] is None) == extra.startswith("shared")
+    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30))
+    assert set(got) == set(want) and all(torch.isfinite(g).all() for g in got.values())
+    errs = {n: rel(got[n], want[n]) for n in want}
+    assert rel(torch.cat([got[n].flatten() for n in want]), torch.cat([want[n].flatten() for n in want])) < 2e-2, errs
+    for n in ("head.weight", "head.bias", "token"):
+        assert errs.get(n, 0.0) < 2e-2, errs

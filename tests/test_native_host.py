@@ -125,3 +125,50 @@ def test_checkpointed_step_is_held_against_the_weights_it_was_computed_again_wit
         train_step.weight.mul_(2.0)
     out.sum().backward()             # the forward ran again, with the weights as they are now
     assert len(train_step.lib.read) == 3
+
+
+def _described(model):
+    """A TrainEngine's description of a model on the CPU (nothing is launched; placement is not looked at)."""
+    engine = native_train.TrainEngine.__new__(native_train.TrainEngine)
+    engine.dtype, engine.device = torch.float16, torch.device("cpu")
+    engine._keep, engine._casts, engine._packs, engine._zero, engine.read_back = [], [], [], [], []
+    engine.params, engine._placed, engine.total = [], set(), 0
+    engine._describe(model)
+    return engine
+
+
+SMALL = dict(enc_depths=(1, 2, 1), enc_channels=(32, 64, 128), enc_num_head=(2, 4, 8), enc_patch_size=(64,) * 3, stride=(2, 2),
+             dec_depths=(1, 1), dec_channels=(64, 64), dec_num_head=(4, 4), dec_patch_size=(64,) * 2)
+
+
+def test_step_node_holds_the_parameters_it_writes_gradients_for_and_no_others():
+    """A segmentation head or a mask token of a subclass is no part of the backbone's node: its gradient is not this node's
+    to give."""
+    from pointtransformerv3_amd import PointTransformerV3
+
+    class Segmentor(PointTransformerV3):
+        def __init__(self, **kw):
+            super().__init__(**kw)
+            self.mask_token = torch.nn.Parameter(torch.zeros(1, 6))
+            self.head = torch.nn.Linear(64, 13)
+
+    model = Segmentor(**SMALL)
+    engine = _described(model)
+    backbone = [p for part in (model.embedding, model.enc, model.dec) for p in part.parameters()]
+    assert {id(p) for p in engine.params} == {id(p) for p in backbone} and len(engine.params) == len(backbone)
+    assert engine.total == sum(p.numel() for p in backbone)
+
+
+@pytest.mark.parametrize("share", ["block", "norm", "weight"])
+def test_parameters_used_twice_are_left_to_the_modules(share):
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(**SMALL)
+    a, b = model.enc.enc1.block0, model.enc.enc1.block1
+    if share == "block":
+        model.enc.enc1.block1 = a
+    elif share == "norm":
+        b.norm2 = a.norm1
+    else:
+        b.mlp[0].fc1.weight = a.mlp[0].fc1.weight
+    with pytest.raises(native.Unsupported):
+        _described(model)
