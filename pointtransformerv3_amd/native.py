@@ -6,6 +6,7 @@ An Engine describes one model in one compute dtype. It takes the default archite
 model, a model with hooks or submodules in training mode, and inputs that carry tables of their own go through the
 modules (model.py), which stay the definition of the result."""
 import ctypes
+import operator
 import weakref
 
 import numpy as np
@@ -75,30 +76,80 @@ _OWN_KEYS = ("serialized_code", "serialized_order", "serialized_inverse", "seria
              "sparse_conv_feat", "pad", "unpad", "cu_seqlens_key", "pooling_inverse", "pooling_parent")
 
 
+# what the native paths read of a module besides its children, parameters and buffers, once, when the model is described
+# (a BatchNorm's momentum, a DropPath's rate and the orders are read at every forward)
+_READ = {
+    nn.Linear: ("in_features", "out_features"), nn.GELU: ("approximate",), nn.Dropout: ("p",),
+    nn.BatchNorm1d: ("eps", "num_features", "track_running_stats"), LayerNorm: ("eps", "normalized_shape"),
+    SubMConv3d: ("kernel_size", "in_channels", "out_channels"), Block: ("channels", "pre_norm"),
+    SerializedAttention: ("channels", "num_heads", "scale", "order_index", "patch_size", "enable_flash", "enable_rpe", "attn_drop"),
+    SerializedPooling: ("stride", "reduce", "shuffle_orders", "traceable"), SerializedUnpooling: ("traceable",),
+}
+_PLAIN = (bool, int, float, str, tuple)
+_GEOMETRY = operator.attrgetter("shape"), torch.Tensor.stride
+
+
+def _names(m):
+    """What _READ names of a module."""
+    names = _READ.get(type(m), ())
+    if type(m) is SerializedAttention and not m.__dict__.get("enable_flash"):
+        names = tuple(n for n in names if n != "patch_size")   # such a layer sets it at every forward
+    return names
+
+
 class Structure:
-    """What of a model's modules the native paths rely on, and whether it still holds."""
+    """What of a model's modules the native paths rely on, and whether it still holds: which modules there are and of what
+    type, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
+    makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, about 0.15 ms), so it
+    is lists compared by mapped C functions."""
 
     def __init__(self, model):
+        self.why = None     # why no model of this structure is covered, as far as it shows here
         self.modules = list(model.modules())
-        _need(all("forward" not in m.__dict__ for m in self.modules), "a module's forward was replaced")
+        # an instance attribute in the place of a method: the model does something else than its classes say
+        if any(callable(getattr(type(m), name, None)) for m in self.modules for name in m.__dict__):
+            self.why = "a method was replaced"
         self.hooks = [d for m in self.modules for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
                                                         m._backward_pre_hooks)]
-        self.children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
-        self.slots, self.tensors = [], []
-        for m in self.modules:
-            for name, p in m._parameters.items():
-                if p is not None:
-                    self.slots.append((m._parameters, name))
-                    self.tensors.append(p)
-            if isinstance(m, nn.BatchNorm1d) and m.running_mean is not None:
-                for name in ("running_mean", "running_var"):
-                    self.slots.append((m._buffers, name))
-                    self.tensors.append(m._buffers[name])
-        self.pointers = [d[k].data_ptr() for d, k in self.slots]
-        # modules whose training flag changes what an evaluation computes
-        self.flagged = [m for m in self.modules if isinstance(m, nn.BatchNorm1d)
-                        or (isinstance(m, nn.Dropout) and m.p > 0) or (isinstance(m, DropPath) and m.drop_prob > 0)
-                        or (isinstance(m, SerializedAttention) and m.attn_drop > 0)]
+        self._model, self._n_orders = model, len(model.order)
+        self._types = list(map(type, self.modules))
+        self._forwards = [(t, t.forward) for t in set(self._types)]
+        children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
+        self._child_at, self._children = ([d for d, _, _ in children], [k for _, k, _ in children]), [c for _, _, c in children]
+        # a child or an instance attribute (a replaced forward) that came or went
+        self._sized = [m.__dict__ for m in self.modules] + [m._modules for m in self.modules if m._modules]
+        self._sizes = list(map(len, self._sized))
+        self._reads, self._values = [], []
+        reads = [(m.__dict__, _names(m)) for m in self.modules] + [(model.__dict__, ("num_stages", "stride", "cls_mode"))]
+        for attributes, names in reads:
+            if not names:
+                continue
+            getter = operator.itemgetter(*names)
+            try:
+                values = getter(attributes)
+            except KeyError as e:
+                self.why = f"no attribute {e}"
+                continue
+            if not all(isinstance(v, _PLAIN) for v in (values if type(values) is tuple else (values,))):
+                self.why = "an attribute that is no plain value"
+                continue
+            self._reads.append((getter, attributes))
+            self._values.append(values)
+        slots = [(m._parameters, name) for m in self.modules for name in m._parameters]
+        norms = [m for m in self.modules if isinstance(m, nn.BatchNorm1d)]
+        slots += [(m._buffers, name) for m in norms for name in ("running_mean", "running_var")]
+        self.tensors = [d[k] for d, k in slots if d[k] is not None]
+        slots += [(m._buffers, "num_batches_tracked") for m in norms]
+        self._slots = [d for d, _ in slots], [k for _, k in slots]
+        self._held = list(map(operator.getitem, *self._slots))
+        self._matrices = [t for t in self.tensors if t.dim() > 1]
+        self._places = self._places_now()
+        # modules whose training flag changes what they compute
+        self.flagged = [m for m in self.modules if isinstance(m, (nn.BatchNorm1d, nn.Dropout, DropPath, SerializedAttention))]
+
+    def _places_now(self):
+        # the same address with another shape or stride is another weight too; rows of one dimension are what they are
+        return [list(map(torch.Tensor.data_ptr, self.tensors)), *[list(map(g, self._matrices)) for g in _GEOMETRY]]
 
     def hooked(self):
         hooks = torch.nn.modules.module
@@ -106,9 +157,16 @@ class Structure:
                     or hooks._global_backward_pre_hooks or any(self.hooks))
 
     def same(self):
-        """The module tree and the places of all weights are those this was made from."""
-        return (all(d[k] is c for d, k, c in self.children)
-                and [d[k].data_ptr() for d, k in self.slots] == self.pointers)
+        """Whether everything this was made from still is what it was."""
+        try:
+            return (list(map(len, self._sized)) == self._sizes and list(map(type, self.modules)) == self._types
+                    and all(t.forward is f for t, f in self._forwards) and len(self._model.order) == self._n_orders
+                    and all(map(operator.is_, map(operator.getitem, *self._child_at), self._children))
+                    and [f(d) for f, d in self._reads] == self._values
+                    and all(map(operator.is_, map(operator.getitem, *self._slots), self._held))
+                    and self._places_now() == self._places)
+        except KeyError:   # something went that was there
+            return False
 
 
 def _check_gelu(m):
@@ -243,6 +301,7 @@ class Engine:
         self.device = self.structure.tensors[0].device
         params = [t for t in self.structure.tensors if isinstance(t, nn.Parameter)]
         kinds = {p.dtype for p in params}
+        _need(self.structure.why is None, self.structure.why)
         _need(kinds == {dtype} or (kinds == {torch.float32} and dtype != torch.float32), "weights of several dtypes")
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() for p in self.structure.tensors), "placement")
         self._keep = []
@@ -393,7 +452,7 @@ class Engine:
             _lib.check(lib.ptv3_net_refresh(ctypes.byref(self._refresh), ops._stream()), "ptv3_net_refresh")
 
         def index_of(between=None):
-            return levels.build(self.layout, *coordinates(point), model.order, model.shuffle_orders, self.want, between=between)
+            return levels.build(self.layout, *coordinates(point), list(model.order), model.shuffle_orders, self.want, between=between)
 
         if model.overlap_index_prologue:
             if model._prologue_state is None or model._prologue_state.device != feat.device:
@@ -505,11 +564,4 @@ class Refused:
     """A model the native paths do not cover, remembered until its structure or weights move."""
 
     def __init__(self, model, why):
-        self.why = why
-        try:
-            self.structure = Structure(model)
-        except Unsupported:
-            self.structure = self
-
-    def same(self):
-        return True
+        self.why, self.structure = why, Structure(model)

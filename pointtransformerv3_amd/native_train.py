@@ -58,6 +58,7 @@ class TrainEngine:
 
     def __init__(self, model, dtype):
         self.structure = Structure(model)
+        _need(self.structure.why is None, self.structure.why)
         self.dtype = dtype
         self.device = self.structure.tensors[0].device
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() and p.dtype == torch.float32
@@ -70,6 +71,7 @@ class TrainEngine:
         # description places, each of which the backward writes once and in whole. A subclass may hold more (a head, a
         # mask token): they are no part of this node
         self.params, self._placed, self.total = [], set(), 0
+        self._norms = []                # (its ptv3 description, module): the momentum may follow a schedule
         self._describe(model)
         self._finish()
         self.batches = [m.num_batches_tracked for m in self.structure.modules
@@ -114,12 +116,12 @@ class TrainEngine:
 
     def _bn(self, m, c):
         _need(type(m) is nn.BatchNorm1d and m.num_features == c and m.weight is not None and m.bias is not None
-              and m.track_running_stats and m.running_mean is not None and m.momentum is not None, "BatchNorm1d")
+              and m.track_running_stats and m.running_mean is not None, "BatchNorm1d")
         gg, gb = self._at(m.weight), self._at(m.bias)   # the kernel writes both, one behind the other
         assert gb == gg + c
         self.read_back += [m.weight, m.bias]
         return _Bn(m.weight.data_ptr(), m.bias.data_ptr(), self._copy(m.weight), self._copy(m.bias), m.running_mean.data_ptr(),
-                   m.running_var.data_ptr(), m.eps, m.momentum, gg)
+                   m.running_var.data_ptr(), m.eps, 0.0, gg)
 
     def _block(self, b, c):
         conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
@@ -145,6 +147,7 @@ class TrainEngine:
         net.stem.w = self._buffer(conv.out_channels * 125 * padded)
         net.stem.cin, net.stem.cin_padded, net.stem.gw = conv.in_channels, padded, self._at(conv.weight)
         net.stem.bn = self._bn(p.stem_bn, conv.out_channels)
+        self._norms.append((net.stem.bn, p.stem_bn))
         self._refresh = native._Refresh(dtype=net.dtype, stem_src=self._copy(conv.weight), stem_dst=net.stem.w,
                                         stem_rows=conv.out_channels * 125, stem_in=conv.in_channels, stem_padded=padded)
         self.drops, below = [], conv.out_channels
@@ -154,10 +157,12 @@ class TrainEngine:
             if st.down is not None:
                 d.pool, d.pool_bn = self._linear(st.down.proj, below, st.channels), self._bn(st.down.norm[0], st.channels)
                 d.pool_reduce = ops.REDUCE_OPS[st.down.reduce]
+                self._norms.append((d.pool_bn, st.down.norm[0]))
             if st.up is not None:
                 d.up = self._linear(st.up.proj[0], st.up.proj[0].in_features, st.dec_channels)
                 d.up_skip = self._linear(st.up.proj_skip[0], st.channels, st.dec_channels)
                 d.up_bn, d.up_skip_bn = self._bn(st.up.proj[1], st.dec_channels), self._bn(st.up.proj_skip[1], st.dec_channels)
+                self._norms += [(d.up_bn, st.up.proj[1]), (d.up_skip_bn, st.up.proj_skip[1])]
             for attr, bs, c in (("enc", st.enc, st.channels), ("dec", st.dec, st.dec_channels)):
                 if bs:
                     arr = (_Block * len(bs))(*[self._block(b, c) for b in bs])
@@ -205,6 +210,14 @@ class TrainEngine:
         self._keep.append(t)
         return t.data_ptr() if t is not None else None
 
+    def averaging(self):
+        """Whether the running statistics follow an exponential average (momentum None: a cumulative one)."""
+        return all(m.momentum is not None for _, m in self._norms)
+
+    def follow_momentum(self):
+        for d, m in self._norms:
+            d.momentum = m.momentum
+
     def masks(self, sizes):
         """The stochastic-depth row factors in the order the blocks would draw them (DropPath.mask; model.py:602-604)."""
         out, keeps, drawn = [], [], []
@@ -241,8 +254,9 @@ class TrainEngine:
                 torch._foreach_add_(self.batches, 1)
             masks.extend(self.masks(sizes))
 
+        self.follow_momentum()
         model._prologue_state = None
-        index = levels.build(self.layout, grid, offset, batch, model.order, model.shuffle_orders, self.want, between=refresh, sized=sized)
+        index = levels.build(self.layout, grid, offset, batch, list(model.order), model.shuffle_orders, self.want, between=refresh, sized=sized)
         if any(v.n < 2 for v in index.levels):
             raise ValueError("Expected more than 1 value per channel when training")   # as BatchNorm1d does
         out = _Step.apply(self, feat, index, masks, *self.params)
@@ -323,4 +337,4 @@ def engine_for(model, data):
         return None
     if engine.structure.hooked() or not all(m.training for m in engine.structure.flagged):
         return None
-    return engine if any(p.requires_grad for p in engine.params) else None
+    return engine if engine.averaging() and any(p.requires_grad for p in engine.params) else None

@@ -91,3 +91,45 @@ def test_native_forward_follows_changed_weights_and_leaves_changed_models_alone(
         model.dec.dec0.block0.mlp[0].fc1 = torch.nn.Sequential(model.dec.dec0.block0.mlp[0].fc1)   # not the default architecture
         assert native.engine_for(model, data) is None
     assert native.engine_for(model, data) is None                              # grad mode: the modules
+
+
+def _each(model, kind, name, value):
+    for m in model.modules():
+        if type(m).__name__ == kind:
+            setattr(m, name, value)
+
+
+@pytest.mark.parametrize("change,native_again", [
+    (lambda m: _each(m, "LayerNorm", "eps", 1e-2), True), (lambda m: _each(m, "BatchNorm1d", "eps", 0.5), True),
+    (lambda m: _each(m, "SerializedAttention", "scale", 0.6), True), (lambda m: _each(m, "SerializedAttention", "patch_size", 64), True),
+    (lambda m: _each(m, "SerializedAttention", "order_index", 1), True),
+    (lambda m: _each(m, "SerializedPooling", "reduce", "mean"), True),
+    (lambda m: _each(m, "SerializedPooling", "shuffle_orders", False), True),
+    (lambda m: _each(m, "GELU", "approximate", "tanh"), False),
+    (lambda m: m.enc.enc1.add(torch.nn.LayerNorm(64).half().to(DEV), name="extra"), False),
+    (lambda m: setattr(m.enc.enc2.block0.mlp[0], "forward", lambda x: x), False),
+    (lambda m: m.dec.dec0._modules.pop("block0"), True), (lambda m: setattr(m.enc.enc2.block0.mlp[0].fc1, "bias", None), False)],
+    ids=["layer_norm_eps", "batch_norm_eps", "scale", "patch_size", "order_index", "reduce", "shuffle_orders", "gelu", "child_added",
+         "forward", "child_removed", "no_bias"])
+def test_a_model_changed_after_its_first_forward_is_described_again_or_left_to_the_modules(change, native_again, monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3, native
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().half().to(DEV)
+    data = _inputs(7, (4000, 900), torch.float16)
+    _both(model, data, monkeypatch)
+    change(model)
+    real = native.engine_for
+    outs = []
+    for use in (True, False):
+        taken = []
+        monkeypatch.setattr(native, "engine_for", (lambda m, d: taken.append(real(m, d)) or taken[-1]) if use else (lambda m, d: None))
+        torch.manual_seed(9)
+        with torch.inference_mode():
+            try:
+                outs.append(model(dict(data)).feat)
+            except Exception as e:      # what the modules refuse is refused the same way
+                outs.append(type(e))
+        if use:
+            assert (taken[0] is not None) == native_again
+    got, want = outs
+    assert type(got) is type(want) and (torch.equal(got, want) if isinstance(want, torch.Tensor) else got is want)

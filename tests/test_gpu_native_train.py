@@ -207,3 +207,23 @@ def test_gradients_of_models_that_hold_more_or_less_than_the_backbone(extra, mon
     assert rel(torch.cat([got[n].flatten() for n in want]), torch.cat([want[n].flatten() for n in want])) < 2e-2, errs
     for n in ("head.weight", "head.bias", "token"):
         assert errs.get(n, 0.0) < 2e-2, errs
+
+
+def test_native_training_step_follows_a_momentum_schedule(monkeypatch):
+    """Running statistics after steps whose BatchNorm momentum changes in between (and is None in the last)."""
+    from pointtransformerv3_amd import PointTransformerV3, native_train
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0, **KW).to(DEV).train()
+    other = copy.deepcopy(model)
+    data = _inputs(4, (3000,), torch.float32)
+    for i, momentum in enumerate((0.01, 0.5, 0.2)):
+        for m, use in ((model, True), (other, False)):
+            for bn in m.modules():
+                if isinstance(bn, torch.nn.BatchNorm1d):
+                    bn.momentum = momentum
+            _step(m, data, torch.float16, use, monkeypatch)
+        for (n, x), y in zip(model.named_buffers(), other.buffers()):
+            assert torch.allclose(x.float(), y.float(), rtol=2e-2, atol=2e-2 * float(y.float().abs().max())), (i, n)
+    model.enc.enc1.down.norm[0].momentum = None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert native_train.engine_for(model, data) is None

@@ -132,7 +132,7 @@ def _described(model):
     engine = native_train.TrainEngine.__new__(native_train.TrainEngine)
     engine.dtype, engine.device = torch.float16, torch.device("cpu")
     engine._keep, engine._casts, engine._packs, engine._zero, engine.read_back = [], [], [], [], []
-    engine.params, engine._placed, engine.total = [], set(), 0
+    engine.params, engine._placed, engine.total, engine._norms = [], set(), 0, []
     engine._describe(model)
     return engine
 
@@ -172,3 +172,96 @@ def test_parameters_used_twice_are_left_to_the_modules(share):
         b.mlp[0].fc1.weight = a.mlp[0].fc1.weight
     with pytest.raises(native.Unsupported):
         _described(model)
+
+
+def _set(path, value):
+    """A change of one attribute: path is its owner within enc.enc1 and its name."""
+    def change(stage):
+        *owner, name = path.split(".")
+        at = stage
+        for key in owner:
+            at = at[int(key)] if key.isdigit() else getattr(at, key)
+        setattr(at, name, value(getattr(at, name)) if callable(value) and not isinstance(value, torch.nn.Module) else value)
+    return change
+
+
+def _replace_forward(stage):
+    stage.block0.mlp[0].forward = lambda x: x
+
+
+def _transposed(stage):
+    w = stage.block0.attn.proj.weight
+    w.data = w.data.t()                   # the same address, another matrix
+
+
+def _narrowed(stage):
+    w = stage.block0.mlp[0].fc1.weight
+    w.data = w.data[:16]
+
+
+def _same_data(stage):
+    lin = stage.block0.mlp[0].fc2
+    lin.weight = torch.nn.Parameter(lin.weight.data)
+
+
+CHANGES = dict(
+    norm_eps=_set("block0.norm1.0.eps", 1e-3), batch_norm_eps=_set("down.norm.0.eps", 0.1), scale=_set("block0.attn.scale", 0.5),
+    patch_size=_set("block0.attn.patch_size", 32), order_index=_set("block1.attn.order_index", 2), heads=_set("block0.attn.num_heads", 8),
+    flash=_set("block0.attn.enable_flash", False), attn_drop=_set("block0.attn.attn_drop", 0.1),
+    proj_drop=_set("block0.attn.proj_drop.p", 0.1), mlp_drop=_set("block1.mlp.0.drop.p", 0.1),
+    gelu=_set("block0.mlp.0.act.approximate", "tanh"), pre_norm=_set("block0.pre_norm", False),
+    shuffle_orders=_set("down.shuffle_orders", False), reduce=_set("down.reduce", "mean"), traceable=_set("down.traceable", False),
+    plan_kernel_sizes=_set("down.plan_kernel_sizes", (5,)), track=_set("down.norm.0.track_running_stats", False),
+    forward=_replace_forward, child_added=lambda st: st.add(torch.nn.ReLU(), name="extra"),
+    child_removed=lambda st: st._modules.pop("block1"), child_replaced=lambda st: st.block0.drop_path._modules.update({"0": torch.nn.Dropout(0.5)}),
+    bias_gone=_set("block0.mlp.0.fc1.bias", None), norm_without_weight=_set("block0.norm2.0.weight", None),
+    statistics_gone=_set("down.norm.0.running_var", None), counter_replaced=_set("down.norm.0.num_batches_tracked", lambda t: t.clone()),
+    statistics_replaced=_set("down.norm.0.running_mean", lambda t: t.clone()), parameter_replaced=_same_data,
+    data_replaced=lambda st: setattr(st.block0.attn.qkv.weight, "data", st.block0.attn.qkv.weight.data.clone()),
+    data_transposed=_transposed, data_narrowed=_narrowed,
+    attribute_gone=lambda st: delattr(st.block0.attn, "scale"), scale_no_number=_set("block0.attn.scale", torch.tensor(0.5)),
+)
+
+
+@pytest.mark.parametrize("name", sorted(CHANGES))
+def test_structure_notices_what_the_modules_would_act_on(name):
+    """What was read when the model was described is compared at every forward; nothing of it raises."""
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(**SMALL)
+    structure = native.Structure(model)
+    assert structure.why is None and structure.same() and structure.same()
+    CHANGES[name](model.enc.enc1)
+    assert structure.same() is False
+    again = native.Structure(model)
+    assert again.same()
+    if name in ("forward", "attribute_gone", "scale_no_number"):
+        assert again.why is not None      # left to the modules whatever they make of it
+
+
+def test_number_of_orders_belongs_to_the_structure_but_their_names_do_not():
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(order=["z", "hilbert"], **SMALL)
+    structure = native.Structure(model)
+    model.order = ["hilbert", "z-trans"]
+    assert structure.same()
+    model.order.append("z")
+    assert not structure.same()
+
+
+def test_step_follows_a_momentum_schedule():
+    """A BatchNorm's momentum is read at every step; a cumulative average (None) is left to the modules."""
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(**SMALL)
+    engine = _described(model)
+    norms = [m for m in model.modules() if isinstance(m, torch.nn.BatchNorm1d)]
+    assert sorted(map(id, norms)) == sorted(id(m) for _, m in engine._norms)
+    places = [engine.net.stem.bn] + [engine.net.stage[s].pool_bn for s in (1, 2)]
+    places += [b for s in (0, 1) for b in (engine.net.stage[s].up_bn, engine.net.stage[s].up_skip_bn)]
+    for i, m in enumerate(norms):
+        m.momentum = 0.1 + 0.05 * i
+    assert engine.averaging()
+    engine.follow_momentum()
+    got = sorted(round(d.momentum, 4) for d in places)
+    assert got == [round(0.1 + 0.05 * i, 4) for i in range(len(norms))]
+    norms[1].momentum = None
+    assert not engine.averaging()
