@@ -100,21 +100,28 @@ def _names(m):
 class Structure:
     """What of a model's modules the native paths rely on, and whether it still holds: which modules there are and of what
     type, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
-    makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, about 0.15 ms), so it
-    is lists compared by mapped C functions."""
+    makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, about 0.17 ms), so it
+    is lists compared by mapped C functions.
+
+    It looks at the backbone (embedding, enc, dec) only; what else a subclass holds runs outside this forward. It holds the
+    backbone's modules but not the model, whose table of engines (_ENGINES) would otherwise keep it alive for good."""
+
+    PARTS = ("embedding", "enc", "dec")
 
     def __init__(self, model):
         self.why = None     # why no model of this structure is covered, as far as it shows here
-        self.modules = list(model.modules())
+        roots = [model._modules.get(name) for name in self.PARTS]
+        self.modules = [m for root in roots if root is not None for m in root.modules()]
         # an instance attribute in the place of a method: the model does something else than its classes say
         if any(callable(getattr(type(m), name, None)) for m in self.modules for name in m.__dict__):
             self.why = "a method was replaced"
-        self.hooks = [d for m in self.modules for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
-                                                        m._backward_pre_hooks)]
-        self._model, self._n_orders = model, len(model.order)
+        self.hooks = [d for m in (model, *self.modules) for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
+                                                                  m._backward_pre_hooks)]
+        self._attributes, self._n_orders = model.__dict__, len(model.order)
         self._types = list(map(type, self.modules))
         self._forwards = [(t, t.forward) for t in set(self._types)]
         children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
+        children += [(model._modules, name, root) for name, root in zip(self.PARTS, roots) if root is not None]
         self._child_at, self._children = ([d for d, _, _ in children], [k for _, k, _ in children]), [c for _, _, c in children]
         # a child or an instance attribute (a replaced forward) that came or went
         self._sized = [m.__dict__ for m in self.modules] + [m._modules for m in self.modules if m._modules]
@@ -160,7 +167,7 @@ class Structure:
         """Whether everything this was made from still is what it was."""
         try:
             return (list(map(len, self._sized)) == self._sizes and list(map(type, self.modules)) == self._types
-                    and all(t.forward is f for t, f in self._forwards) and len(self._model.order) == self._n_orders
+                    and all(t.forward is f for t, f in self._forwards) and len(self._attributes["order"]) == self._n_orders
                     and all(map(operator.is_, map(operator.getitem, *self._child_at), self._children))
                     and [f(d) for f, d in self._reads] == self._values
                     and all(map(operator.is_, map(operator.getitem, *self._slots), self._held))
@@ -294,8 +301,26 @@ def fill_point(point, index, s, feat, patch):
     point["_pad_patch"] = patch
 
 
-class Engine:
+class Copies:
+    """The weight copies of an engine in device memory. They go when the model does, or when it has to be described again:
+    a stream other than the one they were made on has to be known to the allocator by then."""
+
+    def __init__(self):
+        self._keep, self._streams = [], set()
+
+    def used_here(self):
+        """The kernels about to be queued on the current stream read the copies."""
+        handle = ops._stream()
+        if handle not in self._streams:
+            for t in self._keep:
+                if isinstance(t, torch.Tensor):
+                    t.record_stream(torch.cuda.current_stream(self.device))   # nothing where it is the one they were made on
+            self._streams.add(handle)
+
+
+class Engine(Copies):
     def __init__(self, model, dtype):
+        super().__init__()
         self.structure = Structure(model)
         self.dtype = dtype
         self.device = self.structure.tensors[0].device
@@ -304,13 +329,13 @@ class Engine:
         _need(self.structure.why is None, self.structure.why)
         _need(kinds == {dtype} or (kinds == {torch.float32} and dtype != torch.float32), "weights of several dtypes")
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() for p in self.structure.tensors), "placement")
-        self._keep = []
         self._casts, self._cast_out, self._cast_at = {}, None, 0
         self._jobs_conv, self._jobs_mlp = [], []
         self._cast = kinds != {dtype}
         if self._cast:
             total = sum(-(-p.numel() // 128) * 128 for p in params)
             self._cast_out = torch.empty(total, dtype=dtype, device=self.device)
+            self._keep.append(self._cast_out)
         self._describe(model)
         self._finish_jobs()
 
@@ -445,6 +470,7 @@ class Engine:
         feat = data["feat"].contiguous()
         point = Point.__new__(Point)
         dict.update(point, data)
+        self.used_here()
 
         def refresh():
             # whoever writes the parameters behind autograd's back leaves no trace on them: every derived copy is
@@ -511,7 +537,8 @@ class Engine:
         return point
 
 
-_ENGINES = weakref.WeakKeyDictionary()   # model -> {compute dtype: Engine, or None where the model is not covered}
+# model -> {(compute dtype, encoder only): Engine or Refused}; neither holds the model, so it goes when its user lets it go
+_ENGINES = weakref.WeakKeyDictionary()
 
 
 def _compute_dtype(feat, weight):

@@ -53,10 +53,11 @@ class _Net(ctypes.Structure):
                 ("n_zero", _i32), ("reserved", _i32), ("zero_blocks", _i64), ("stage", _Stage * levels.MAX_LEVELS)]
 
 
-class TrainEngine:
+class TrainEngine(native.Copies):
     """Describes one model (float masters) for training under autocast to `dtype`."""
 
     def __init__(self, model, dtype):
+        super().__init__()
         self.structure = Structure(model)
         _need(self.structure.why is None, self.structure.why)
         self.dtype = dtype
@@ -65,7 +66,7 @@ class TrainEngine:
                   for p in self.structure.tensors), "float weights on one GPU")
         _need(not model.cls_mode, "the encoder-only model hands out intermediate features")
         _need(not any(p.is_inference() for p in self.structure.tensors), "inference tensors")
-        self._keep, self._casts, self._packs, self._zero = [], [], [], []
+        self._casts, self._packs, self._zero = [], [], []
         self.read_back = []             # parameters whose values the backward reads, itself or as a copy made by the forward
         # the parameters of the step's node, in the order their gradients lie in the flat buffer: those that the
         # description places, each of which the backward writes once and in whole. A subclass may hold more (a head, a
@@ -255,6 +256,7 @@ class TrainEngine:
             masks.extend(self.masks(sizes))
 
         self.follow_momentum()
+        self.used_here()
         model._prologue_state = None
         index = levels.build(self.layout, grid, offset, batch, list(model.order), model.shuffle_orders, self.want, between=refresh, sized=sized)
         if any(v.n < 2 for v in index.levels):
@@ -315,7 +317,7 @@ class _Step(torch.autograd.Function):
         return (None,) * 4 + tuple(g if need else None for g, need in zip(views, needed))
 
 
-_ENGINES = weakref.WeakKeyDictionary()   # model -> {dtype: TrainEngine or native.Refused}
+_ENGINES = weakref.WeakKeyDictionary()   # model -> {dtype: TrainEngine or native.Refused}, as native._ENGINES
 
 
 def engine_for(model, data):

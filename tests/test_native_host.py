@@ -1,7 +1,9 @@
 """Host-side rules of the natively queued paths that need no GPU."""
 import contextlib
 import ctypes
+import gc
 import types
+import weakref
 
 import pytest
 import torch
@@ -36,6 +38,7 @@ def test_inputs_are_converted_where_the_index_reads_them(overlap, monkeypatch):
     monkeypatch.setattr(native.levels, "build", build)
     engine = native.Engine.__new__(native.Engine)
     engine.layout = engine.want = None
+    engine.used_here = lambda: None
     engine._refresh = native._Refresh()   # nothing to refresh: launches nothing
     model = types.SimpleNamespace(overlap_index_prologue=overlap, _prologue_state=Overlap(), order=("z",), shuffle_orders=False)
     with pytest.raises(_Stop):
@@ -265,3 +268,23 @@ def test_step_follows_a_momentum_schedule():
     assert got == [round(0.1 + 0.05 * i, 4) for i in range(len(norms))]
     norms[1].momentum = None
     assert not engine.averaging()
+
+
+def test_a_described_or_refused_model_is_let_go():
+    """The tables of engines are keyed by the model: what they hold must not hold it."""
+    from pointtransformerv3_amd import PointTransformerV3
+    for table, make in ((native._ENGINES, lambda m: native.Refused(m, "for the test")),
+                        (native_train._ENGINES, lambda m: native.Refused(m, "for the test")), (native_train._ENGINES, _engine_of)):
+        model = PointTransformerV3(**SMALL)
+        table.setdefault(model, {})["held"] = make(model)
+        seen, weight = weakref.ref(model), weakref.ref(model.enc.enc1.block0.attn.qkv.weight)
+        before = len(table)
+        del model
+        gc.collect()
+        assert seen() is None and weight() is None and len(table) == before - 1
+
+
+def _engine_of(model):
+    engine = _described(model)
+    engine.structure = native.Structure(model)
+    return engine
