@@ -176,22 +176,49 @@ class Structure:
             return False
 
 
+def _child(m, name, kind, why):
+    """The child module of that name, which has to be of exactly that type."""
+    child = m._modules.get(name)
+    _need(type(child) is kind, why)
+    return child
+
+
+def _sequence(m, name, kinds, why):
+    """The children of the PointSequential of that name; kinds says of which types they are to be."""
+    parts = list(_child(m, name, PointSequential, why)._modules.values())
+    _need(len(parts) == len(kinds) and all(type(c) in (k if type(k) is tuple else (k,)) for c, k in zip(parts, kinds)), why)
+    return parts
+
+
 def _check_gelu(m):
-    _need(type(m) is nn.GELU and m.approximate == "none", "activation")
+    _need(m.approximate == "none", "activation")
 
 
-def _check_block(b, c):
+def _check_conv(m, kernel_size, biased):
+    _need(m.kernel_size == kernel_size and (m.bias is not None) == biased
+          and tuple(m.weight.shape) == (m.out_channels, *[kernel_size] * 3, m.in_channels)
+          and (m.bias is None or m.bias.shape == (m.out_channels,)), "convolution")
+
+
+def _check_block(b, c, n_orders):
     _need(type(b) is Block and b.pre_norm and b.channels == c and c in CHANNELS, "Block")
-    for seq, count in ((b.cpe, 3), (b.norm1, 1), (b.norm2, 1), (b.mlp, 1), (b.drop_path, 1)):
-        _need(type(seq) is PointSequential and len(seq) == count, "Block parts")
-    conv, attn, mlp = b.cpe[0], b.attn, b.mlp[0]
-    _need(type(conv) is SubMConv3d and conv.kernel_size == 3 and conv.in_channels == conv.out_channels == c
-          and conv.bias is not None, "xCPE convolution")
-    _need(type(attn) is SerializedAttention and attn.enable_flash and attn.rpe is None and attn.channels == c
-          and c % attn.num_heads == 0, "attention")
-    _need(type(mlp) is MLP and type(b.drop_path[0]) in (DropPath, nn.Identity), "MLP")
-    _check_gelu(mlp.act)
-    _need(all(type(m) is LayerNorm for m in (b.cpe[2], b.norm1[0], b.norm2[0])) and b.cpe[2].eps == b.norm1[0].eps, "LayerNorm")
+    conv, _, ln = _sequence(b, "cpe", (SubMConv3d, nn.Linear, LayerNorm), "xCPE")
+    norms = [*_sequence(b, "norm1", (LayerNorm,), "norm"), *_sequence(b, "norm2", (LayerNorm,), "norm")]
+    _need(ln.eps == norms[0].eps, "norm")
+    _check_conv(conv, 3, True)
+    _need(conv.in_channels == conv.out_channels == c, "xCPE")
+    attn = _child(b, "attn", SerializedAttention, "attention")
+    _need(attn.enable_flash and not attn.enable_rpe and "rpe" not in attn._modules and attn.channels == c
+          and 1 <= attn.num_heads <= c and c % attn.num_heads == 0 and 0 <= attn.order_index < n_orders and attn.patch_size >= 1, "attention")
+    for name in ("qkv", "proj"):
+        _child(attn, name, nn.Linear, "attention")
+    _child(attn, "proj_drop", nn.Dropout, "attention")
+    mlp, = _sequence(b, "mlp", (MLP,), "MLP")
+    for name in ("fc1", "fc2"):
+        _child(mlp, name, nn.Linear, "MLP")
+    _child(mlp, "drop", nn.Dropout, "MLP")
+    _check_gelu(_child(mlp, "act", nn.GELU, "MLP"))
+    _sequence(b, "drop_path", ((DropPath, nn.Identity),), "stochastic depth")
 
 
 class Parts:
@@ -200,54 +227,57 @@ class Parts:
     class Stage:
         down = up = None
         enc = dec = ()
+        bn = None            # of the pooling
         channels = dec_channels = patch = 0
 
     def __init__(self, model):
         S = model.num_stages
-        self.n_orders = len(list(model.order))
-        _need(2 <= S <= levels.MAX_LEVELS and 1 <= self.n_orders <= levels.MAX_ORDERS, "stages")
-        _need(type(model.embedding) is Embedding and type(model.enc) is PointSequential, "stem")
-        stem = model.embedding.stem
-        _need(type(stem) is PointSequential and list(stem._modules) == ["conv", "norm", "act"], "stem")
-        self.stem_conv, self.stem_bn = stem[0], stem[1]
-        _need(type(stem[0]) is SubMConv3d and stem[0].kernel_size == 5 and stem[0].bias is None, "stem convolution")
-        _check_gelu(stem[2])
-        _need(list(model.enc._modules) == [f"enc{s}" for s in range(S)], "encoder")
-        self.stages, below = [], stem[0].out_channels
+        self.n_orders = len(model.order)
+        _need(2 <= S <= levels.MAX_LEVELS and 1 <= self.n_orders <= levels.MAX_ORDERS and len(model.stride) == S - 1, "stages")
+        embedding, enc = _child(model, "embedding", Embedding, "stem"), _child(model, "enc", PointSequential, "encoder")
+        self.stem_conv, self.stem_bn, act = _sequence(embedding, "stem", (SubMConv3d, nn.BatchNorm1d, nn.GELU), "stem")
+        _check_conv(self.stem_conv, 5, False)
+        _check_gelu(act)
+        _need(list(enc._modules) == [f"enc{s}" for s in range(S)], "encoder")
+        dec = None if model.cls_mode else _child(model, "dec", PointSequential, "decoder")
+        _need(dec is None or list(dec._modules) == [f"dec{s}" for s in reversed(range(S - 1))], "decoder")
+        self.stages, below = [], self.stem_conv.out_channels
         for s in range(S):
-            stage, st = model.enc[s], Parts.Stage()
-            _need(type(stage) is PointSequential, "encoder stage")
-            parts = list(stage._modules.items())
+            stage, st = _child(enc, f"enc{s}", PointSequential, "encoder stage"), Parts.Stage()
+            st.enc = list(stage._modules.values())
             if s:
-                _need(parts and parts[0][0] == "down" and type(parts[0][1]) is SerializedPooling, "pooling")
-                st.down = parts.pop(0)[1]
-                _need(st.down.norm is not None and len(st.down.norm) == 1 and st.down.act is not None and len(st.down.act) == 1
-                      and st.down.plan_kernel_sizes == (3,) and st.down.stride == model.stride[s - 1]
-                      and (not model.cls_mode or st.down.traceable) and st.down.proj.in_features == below, "pooling")
-                _check_gelu(st.down.act[0])
-                below = st.down.out_channels
-            st.channels, st.enc = below, [b for _, b in parts]
-            if not model.cls_mode and s < S - 1:
-                dstage = model.dec._modules.get(f"dec{s}")
-                _need(type(dstage) is PointSequential and list(dstage._modules)[:1] == ["up"], "decoder stage")
-                st.up, st.dec = dstage[0], list(dstage._modules.values())[1:]
-                _need(type(st.up) is SerializedUnpooling and not st.up.traceable, "unpooling")
-                for seq in (st.up.proj, st.up.proj_skip):
-                    _need(type(seq) is PointSequential and len(seq) == 3 and type(seq[0]) is nn.Linear, "unpooling")
-                    _check_gelu(seq[2])
-                st.dec_channels = st.up.proj_skip[0].out_features
-                _need(st.dec_channels in CHANNELS and st.up.proj[0].out_features == st.dec_channels, "decoder width")
+                _need(list(stage._modules)[:1] == ["down"] and type(st.enc[0]) is SerializedPooling, "pooling")
+                st.down = st.enc.pop(0)
+                st.bn, = _sequence(st.down, "norm", (nn.BatchNorm1d,), "pooling")
+                act, = _sequence(st.down, "act", (nn.GELU,), "pooling")
+                _check_gelu(act)
+                _need(st.down.plan_kernel_sizes == (3,) and st.down.stride == model.stride[s - 1] and st.down.reduce in ops.REDUCE_OPS
+                      and (not model.cls_mode or st.down.traceable)
+                      and _child(st.down, "proj", nn.Linear, "pooling").in_features == below, "pooling")
+                below = st.down.proj.out_features
+            st.channels = below
+            if dec is not None and s < S - 1:
+                dstage = _child(dec, f"dec{s}", PointSequential, "decoder stage")
+                st.dec = list(dstage._modules.values())
+                _need(list(dstage._modules)[:1] == ["up"] and type(st.dec[0]) is SerializedUnpooling, "unpooling")
+                st.up = st.dec.pop(0)
+                _need(not st.up.traceable, "unpooling")
+                kinds = nn.Linear, nn.BatchNorm1d, nn.GELU
+                up, skip = _sequence(st.up, "proj", kinds, "unpooling"), _sequence(st.up, "proj_skip", kinds, "unpooling")
+                _check_gelu(up[2])
+                _check_gelu(skip[2])
+                st.dec_channels = skip[0].out_features
+                _need(st.dec_channels in CHANNELS and up[0].out_features == st.dec_channels, "decoder width")
             _need(below in CHANNELS, "width")
             for bs, c in ((st.enc, st.channels), (st.dec, st.dec_channels)):
                 for b in bs:
-                    _check_block(b, c)
+                    _check_block(b, c, self.n_orders)
             sizes = [b.attn.patch_size for b in (*st.enc, *st.dec)]
             # the tables of a level are made for the patch size of the first attention that reaches it
             st.patch = sizes[0] if sizes else 1024
             _need(all(v >= st.patch for v in sizes), "patch sizes that shrink from the encoder to the decoder")
             self.stages.append(st)
-        if not model.cls_mode:
-            _need(list(model.dec._modules) == [f"dec{s}" for s in reversed(range(S - 1))], "decoder")
+        if dec is not None:
             width = self.stages[S - 1].channels
             for s in reversed(range(S - 1)):
                 _need(self.stages[s].up.proj[0].in_features == width, "decoder widths")
@@ -263,6 +293,23 @@ class Parts:
     def widths(self):
         """Per level, the channel counts of its 3x3x3 convolutions."""
         return [sorted({b.channels for b in (*st.enc, *st.dec)}) for st in self.stages]
+
+
+def check_linear(m, cin=None, cout=None, bias=True):
+    """That a Linear is what its attributes say, of the widths asked for."""
+    _need(type(m) is nn.Linear and (m.bias is not None or not bias) and tuple(m.weight.shape) == (m.out_features, m.in_features)
+          and (m.bias is None or tuple(m.bias.shape) == (m.out_features,)), "Linear")
+    _need((cin is None or m.in_features == cin) and (cout is None or m.out_features == cout), "Linear shape")
+
+
+def check_layer_norm(m, c):
+    _need(type(m) is LayerNorm and tuple(m.normalized_shape) == (c,)
+          and all(p is not None and tuple(p.shape) == (c,) for p in (m.weight, m.bias)), "LayerNorm")
+
+
+def check_batch_norm(m, c):
+    _need(type(m) is nn.BatchNorm1d and m.track_running_stats and m.num_features == c
+          and all(p is not None and tuple(p.shape) == (c,) for p in (m.weight, m.bias, m.running_mean, m.running_var)), "BatchNorm1d")
 
 
 def job_table(rows, dtype, device):
@@ -322,6 +369,7 @@ class Engine(Copies):
     def __init__(self, model, dtype):
         super().__init__()
         self.structure = Structure(model)
+        parts = Parts(model)
         self.dtype = dtype
         self.device = self.structure.tensors[0].device
         params = [t for t in self.structure.tensors if isinstance(t, nn.Parameter)]
@@ -336,7 +384,7 @@ class Engine(Copies):
             total = sum(-(-p.numel() // 128) * 128 for p in params)
             self._cast_out = torch.empty(total, dtype=dtype, device=self.device)
             self._keep.append(self._cast_out)
-        self._describe(model)
+        self._describe(model, parts)
         self._finish_jobs()
 
     # ---- pointers -------------------------------------------------------------------------------------------------
@@ -353,17 +401,15 @@ class Engine(Copies):
         return held
 
     def _linear(self, m, cin=None, cout=None, bias=True):
-        _need(type(m) is nn.Linear and (m.bias is not None or not bias), "Linear")
-        _need((cin is None or m.in_features == cin) and (cout is None or m.out_features == cout), "Linear shape")
+        check_linear(m, cin, cout, bias)
         return _Linear(self._p(m.weight), self._p(m.bias), m.in_features, m.out_features)
 
     def _norm(self, m, c):
-        _need(type(m) is LayerNorm and m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
+        check_layer_norm(m, c)
         return _Norm(self._p(m.weight), self._p(m.bias), m.eps, 0)
 
     def _bn(self, m, c):
-        _need(type(m) is nn.BatchNorm1d and m.track_running_stats and m.running_mean is not None and m.num_features == c
-              and m.weight is not None and m.bias is not None, "BatchNorm1d")
+        check_batch_norm(m, c)
         stats = m.running_mean.dtype
         _need(m.running_var.dtype == stats and stats in (torch.float32, self.dtype), "BatchNorm1d statistics")
         return _Bn(m.running_mean.data_ptr(), m.running_var.data_ptr(), self._p(m.weight), self._p(m.bias), m.eps,
@@ -397,9 +443,8 @@ class Engine(Copies):
                 self._jobs_mlp.append((d.qkv.w, 0, d.head_packed + c * c * 2, c, 3))
         return d
 
-    def _describe(self, model):
-        """ptv3_net of the model; Unsupported where it is not the default architecture."""
-        p = Parts(model)
+    def _describe(self, model, p):
+        """ptv3_net of the model, p its Parts; Unsupported where it is not the default architecture."""
         net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages), decoder=int(not model.cls_mode))
         net.stem_in = p.stem_conv.in_channels
         net.stem_w = self._p(p.stem_conv.weight)
@@ -415,7 +460,7 @@ class Engine(Copies):
             d.channels, d.n_enc, d.dec_channels, d.n_dec = st.channels, len(st.enc), st.dec_channels, len(st.dec)
             if st.down is not None:
                 d.pool = self._linear(st.down.proj, None, st.channels)
-                d.pool_bn, d.pool_reduce = self._bn(st.down.norm[0], st.channels), ops.REDUCE_OPS[st.down.reduce]
+                d.pool_bn, d.pool_reduce = self._bn(st.bn, st.channels), ops.REDUCE_OPS[st.down.reduce]
             if st.up is not None:
                 d.up, d.up_skip = self._linear(st.up.proj[0]), self._linear(st.up.proj_skip[0], st.channels)
                 d.up_bn, d.up_skip_bn = self._bn(st.up.proj[1], st.dec_channels), self._bn(st.up.proj_skip[1], st.dec_channels)
@@ -564,13 +609,21 @@ def plain_inputs(data):
     return isinstance(where, torch.Tensor) and where.is_cuda and where.shape[0] == feat.shape[0] and ends.is_cuda and ends.numel() > 0
 
 
+def _stem_weight(model):
+    """The weight of the stem's convolution, or None where the model has another embedding."""
+    conv = model._modules.get("embedding")
+    for name in ("stem", "conv"):
+        conv = None if conv is None else conv._modules.get(name)
+    return conv.weight if type(conv) is SubMConv3d else None
+
+
 def engine_for(model, data):
     """The Engine that computes model(data), or None: the modules do."""
     if model.training or torch.is_grad_enabled() or not plain_inputs(data):
         return None
     feat = data["feat"]
-    weight = model.embedding.stem._modules["conv"].weight
-    dtype = _compute_dtype(feat, weight)
+    weight = _stem_weight(model)
+    dtype = None if weight is None else _compute_dtype(feat, weight)
     if dtype not in ops.DTYPE_CODES or feat.shape[1] != weight.shape[-1]:
         return None
     held = _ENGINES.setdefault(model, {})

@@ -60,6 +60,7 @@ class TrainEngine(native.Copies):
         super().__init__()
         self.structure = Structure(model)
         _need(self.structure.why is None, self.structure.why)
+        parts = Parts(model)
         self.dtype = dtype
         self.device = self.structure.tensors[0].device
         _need(all(p.is_cuda and p.device == self.device and p.is_contiguous() and p.dtype == torch.float32
@@ -73,7 +74,7 @@ class TrainEngine(native.Copies):
         # mask token): they are no part of this node
         self.params, self._placed, self.total = [], set(), 0
         self._norms = []                # (its ptv3 description, module): the momentum may follow a schedule
-        self._describe(model)
+        self._describe(model, parts)
         self._finish()
         self.batches = [m.num_batches_tracked for m in self.structure.modules
                         if isinstance(m, nn.BatchNorm1d) and m.num_batches_tracked is not None]
@@ -103,21 +104,20 @@ class TrainEngine(native.Copies):
         return [p._version for p in self.read_back]
 
     def _linear(self, m, cin, cout):
-        _need(type(m) is nn.Linear and m.bias is not None and m.in_features == cin and m.out_features == cout, "Linear")
+        native.check_linear(m, cin, cout)
         self.read_back.append(m.weight)
         return _Linear(self._copy(m.weight), self._copy(m.weight, "transpose"), self._copy(m.bias), cin, cout,
                        self._at(m.weight), self._at(m.bias))
 
     def _norm(self, m, c):
-        _need(m.weight is not None and m.bias is not None and tuple(m.normalized_shape) == (c,), "LayerNorm")
+        native.check_layer_norm(m, c)
         gg, gb = self._at(m.weight), self._at(m.bias)
         self._zero += [(gg, c), (gb, c)]
         self.read_back.append(m.weight)
         return _Norm(m.weight.data_ptr(), m.bias.data_ptr(), m.eps, 0, gg, gb)
 
     def _bn(self, m, c):
-        _need(type(m) is nn.BatchNorm1d and m.num_features == c and m.weight is not None and m.bias is not None
-              and m.track_running_stats and m.running_mean is not None, "BatchNorm1d")
+        native.check_batch_norm(m, c)
         gg, gb = self._at(m.weight), self._at(m.bias)   # the kernel writes both, one behind the other
         assert gb == gg + c
         self.read_back += [m.weight, m.bias]
@@ -139,8 +139,7 @@ class TrainEngine(native.Copies):
         d.ln_cpe, d.ln1, d.ln2 = self._norm(b.cpe[2], c), self._norm(b.norm1[0], c), self._norm(b.norm2[0], c)
         return d
 
-    def _describe(self, model):
-        p = Parts(model)
+    def _describe(self, model, p):
         _need(all(st.enc for st in p.stages) and all(st.dec for st in p.stages[:-1]), "a stage without blocks")
         net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages))
         conv = p.stem_conv
@@ -156,9 +155,9 @@ class TrainEngine(native.Copies):
             d = net.stage[s]
             d.channels, d.n_enc, d.dec_channels, d.n_dec = st.channels, len(st.enc), st.dec_channels, len(st.dec)
             if st.down is not None:
-                d.pool, d.pool_bn = self._linear(st.down.proj, below, st.channels), self._bn(st.down.norm[0], st.channels)
+                d.pool, d.pool_bn = self._linear(st.down.proj, below, st.channels), self._bn(st.bn, st.channels)
                 d.pool_reduce = ops.REDUCE_OPS[st.down.reduce]
-                self._norms.append((d.pool_bn, st.down.norm[0]))
+                self._norms.append((d.pool_bn, st.bn))
             if st.up is not None:
                 d.up = self._linear(st.up.proj[0], st.up.proj[0].in_features, st.dec_channels)
                 d.up_skip = self._linear(st.up.proj_skip[0], st.channels, st.dec_channels)

@@ -136,7 +136,7 @@ def _described(model):
     engine.dtype, engine.device = torch.float16, torch.device("cpu")
     engine._keep, engine._casts, engine._packs, engine._zero, engine.read_back = [], [], [], [], []
     engine.params, engine._placed, engine.total, engine._norms = [], set(), 0, []
-    engine._describe(model)
+    engine._describe(model, native.Parts(model))
     return engine
 
 
@@ -288,3 +288,48 @@ def _engine_of(model):
     engine = _described(model)
     engine.structure = native.Structure(model)
     return engine
+
+
+class _OwnStem(torch.nn.Module):
+    def forward(self, point):
+        return point
+
+
+def _without(*names):
+    def change(model):
+        for name in names:
+            at, key = (model.get_submodule(name.rpartition(".")[0]), name.rpartition(".")[2])
+            delattr(at, key)
+    return change
+
+
+FOREIGN = dict(
+    own_embedding=lambda m: setattr(m, "embedding", _OwnStem()), no_embedding=_without("embedding"), no_encoder=_without("enc"),
+    no_decoder=_without("dec"), no_stem_norm=_without("embedding.stem.norm"), no_mlp=_without("enc.enc1.block0.mlp"),
+    no_attention=_without("dec.dec0.block0.attn"), no_projection=_without("enc.enc1.block0.attn.proj"),
+    own_norm=lambda m: setattr(m.enc.enc1.down, "norm", torch.nn.LayerNorm(64)), no_norm=lambda m: setattr(m.enc.enc1.down, "norm", None),
+    no_pool_projection=_without("enc.enc1.down.proj"), identity=lambda m: setattr(m.dec.dec0.up, "proj", torch.nn.Identity()),
+    nothing=lambda m: [_without(n)(m) for n in ("embedding", "enc", "dec")], row=_set("enc.enc1.block0.attn.order_index", 7),
+    reduce=_set("enc.enc1.down.reduce", "median"), strides=_set("stride", (2,)),
+    pruned=lambda m: setattr(m.enc.enc1.block0.mlp[0].fc1.weight, "data", m.enc.enc1.block0.mlp[0].fc1.weight.data[:64]),
+    pruned_norm=lambda m: setattr(m.enc.enc1.block0.norm1[0].weight, "data", torch.ones(32)),
+    heads=_set("enc.enc1.block0.attn.num_heads", 0),
+)
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("name", sorted(FOREIGN))
+def test_models_of_another_architecture_are_left_to_the_modules(name, train, monkeypatch):
+    """What the native paths do not cover is the modules' to run or to refuse: looking at it raises nothing."""
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(**SMALL).train(train)
+    FOREIGN[name](model)
+    with pytest.raises(native.Unsupported):
+        native.Parts(model)
+        _described(model)
+    monkeypatch.setattr(native, "plain_inputs", lambda data: True)
+    data = dict(feat=torch.zeros(4, 6), grid_coord=torch.zeros(4, 3, dtype=torch.int32), offset=torch.tensor([4]))
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *a: train)
+    with torch.set_grad_enabled(train):
+        for _ in range(2):
+            assert (native_train if train else native).engine_for(model, data) is None
