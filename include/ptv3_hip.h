@@ -700,11 +700,11 @@ typedef struct ptv3_level {
 } ptv3_level;
 
 int64_t ptv3_index_slot_words(int n_levels, int n_scenes);
-size_t ptv3_index_begin_bytes(const ptv3_index_cfg *cfg);
+int ptv3_index_begin_bytes(const ptv3_index_cfg *cfg, size_t *tables, size_t *scratch);
 /* batch_in: scene ids the caller has, or NULL (then they are written to batch_out from the scene ends) */
 int ptv3_index_begin(void *state, const ptv3_index_cfg *cfg, const int32_t *grid_coord, const int64_t *batch_in,
-                     const int64_t *offset, int64_t *batch_out, void *workspace, size_t workspace_bytes,
-                     int64_t *host_slot, int64_t seq, void *stream);
+                     const int64_t *offset, int64_t *batch_out, void *tables, size_t tables_bytes, void *scratch,
+                     size_t scratch_bytes, int64_t *host_slot, int64_t seq, void *stream);
 int ptv3_index_wait(const int64_t *host_slot, int which, int64_t seq, void *stream);
 
 /* Grid extent and scene ends alone, reported like the first stage (model.py:98-101): the maximum of every axis at

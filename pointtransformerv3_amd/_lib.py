@@ -117,8 +117,8 @@ SIGNATURES = {
     "ptv3_block_tail_fused": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                      _vp, _vp]),
     "ptv3_index_slot_words": (_i64, [_i32, _i32]),
-    "ptv3_index_begin_bytes": (_sz, [_vp]),
-    "ptv3_index_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _i64, _vp]),
+    "ptv3_index_begin_bytes": (_i32, [_vp, _vp, _vp]),
+    "ptv3_index_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp, _i64, _vp]),
     "ptv3_index_wait": (_i32, [_vp, _i32, _i64, _vp]),
     "ptv3_scene_facts_bytes": (_sz, [_i64]),
     "ptv3_scene_facts": (_i32, [_vp, _i64, _vp, _i32, _vp, _sz, _vp, _i64, _vp]),

@@ -752,7 +752,8 @@ int list_blocks(ListArgs& a, int first, int levels, int kind) {   // kind 0: hea
     return at;
 }
 
-void carve_list_scratch(Carver& c, ListLevel& v, bool five) {
+// c: what only the index stages read; kept: what the convolutions read as well
+void carve_list_scratch(Carver& c, Carver& kept, ListLevel& v, bool five) {
     v.cap = vh_capacity(v.n);
     v.groups = (int)ptv3_ceil_div(v.n, v.group);
     v.h.blocks = c.take<VoxelBlock>(v.cap);
@@ -764,7 +765,7 @@ void carve_list_scratch(Carver& c, ListLevel& v, bool five) {
     v.row = c.take<uint32_t>(v.groups);
     v.tap_total = c.take<uint32_t>(TAPS3 + 1);
     v.row_total = c.take<uint32_t>(1);
-    v.tap_ptr = c.take<int32_t>(TAPS3 + 1);
+    v.tap_ptr = kept.take<int32_t>(TAPS3 + 1);
     v.tap5 = v.row5 = v.tap_total5 = v.row_total5 = nullptr;
     v.tap_ptr5 = nullptr;
     if (five) {
@@ -772,7 +773,7 @@ void carve_list_scratch(Carver& c, ListLevel& v, bool five) {
         v.row5 = c.take<uint32_t>(v.groups);
         v.tap_total5 = c.take<uint32_t>(TAPS5 + 1);
         v.row_total5 = c.take<uint32_t>(1);
-        v.tap_ptr5 = c.take<int32_t>(TAPS5 + 1);
+        v.tap_ptr5 = kept.take<int32_t>(TAPS5 + 1);
     }
 }
 
@@ -811,15 +812,22 @@ template <typename KT> int launch_cells_tables(State& s, hipStream_t stream) {
     PTV3_RETURN_LAUNCH();
 }
 
-size_t carve_begin(State& s, void* base) {
+// The tables are small (16 bytes a point) and what a caller keeps; the scratch is 650 - 800 bytes a point, most of it the
+// voxel hash, and is free again once the lists are made. In one buffer the 6 MB of sparse indices in a returned Point
+// held 0.3 GB of a 400k-point batch.
+struct Bytes {
+    size_t tables, scratch;
+};
+
+Bytes carve_begin(State& s, void* tables, void* scratch) {
     const ptv3_index_cfg& g = s.cfg;
-    Carver c(base);
+    Carver kept(tables), c(scratch);
     const int64_t n = g.n;
-    s.lv[0].indices = c.take<int32_t>(4 * n);
+    s.lv[0].indices = kept.take<int32_t>(4 * n);
     s.part = c.take<int32_t>(3 * MAX_FACT_BLOCKS);
     const int pooled = g.n_levels - 1;
     for (int l = 0; l < g.n_levels; ++l) {
-        if (l > 0) s.lv[l].offset = c.take<int64_t>(g.n_scenes);
+        if (l > 0) s.lv[l].offset = kept.take<int64_t>(g.n_scenes);
         s.pads.pad_start[l] = c.take<int64_t>(g.n_scenes + 1);
         s.pads.seq_start[l] = c.take<int64_t>(g.n_scenes + 1);
     }
@@ -831,9 +839,9 @@ size_t carve_begin(State& s, void* base) {
     ListLevel& v = s.lists.lv[0];
     v.n = n;
     v.group = group_of(n, g.only128[0]);
-    carve_list_scratch(c, v, g.stem5);
+    carve_list_scratch(c, kept, v, g.stem5);
     v.idx = (const int4*)s.lv[0].indices;
-    return c.off;
+    return {kept.off, c.off};
 }
 
 bool cfg_ok(const ptv3_index_cfg* g) {
@@ -847,13 +855,14 @@ bool cfg_ok(const ptv3_index_cfg* g) {
 
 }  // namespace
 
-extern "C" size_t ptv3_index_begin_bytes(const ptv3_index_cfg* cfg) {
-    if (!cfg_ok(cfg)) return 0;
-    State* s = new State();
-    s->cfg = *cfg;
-    const size_t bytes = carve_begin(*s, nullptr);
-    delete s;
-    return bytes;
+extern "C" int ptv3_index_begin_bytes(const ptv3_index_cfg* cfg, size_t* tables, size_t* scratch) {
+    if (!cfg_ok(cfg) || !tables || !scratch) return PTV3_EINVAL;
+    State s = {};
+    s.cfg = *cfg;
+    const Bytes need = carve_begin(s, nullptr, nullptr);
+    *tables = need.tables;
+    *scratch = need.scratch;
+    return PTV3_OK;
 }
 
 extern "C" int64_t ptv3_index_slot_words(int n_levels, int n_scenes) {
@@ -866,15 +875,16 @@ static int fact_blocks(int64_t n) {
 }
 
 extern "C" int ptv3_index_begin(void* state, const ptv3_index_cfg* cfg, const int32_t* grid_coord, const int64_t* batch_in,
-                                const int64_t* offset, int64_t* batch_out, void* workspace, size_t workspace_bytes,
-                                int64_t* host_slot, int64_t seq, void* stream_) {
-    if (!state || !cfg_ok(cfg) || !grid_coord || !offset || (!batch_in && !batch_out) || !workspace || !host_slot)
+                                const int64_t* offset, int64_t* batch_out, void* tables, size_t tables_bytes, void* scratch,
+                                size_t scratch_bytes, int64_t* host_slot, int64_t seq, void* stream_) {
+    if (!state || !cfg_ok(cfg) || !grid_coord || !offset || (!batch_in && !batch_out) || !tables || !scratch || !host_slot)
         return PTV3_EINVAL;
     State& s = *(State*)state;
     memset(&s, 0, sizeof(State));
     s.cfg = *cfg;
-    if (workspace_bytes < carve_begin(s, nullptr)) return PTV3_EWORKSPACE;
-    carve_begin(s, workspace);
+    const Bytes need = carve_begin(s, nullptr, nullptr);
+    if (tables_bytes < need.tables || scratch_bytes < need.scratch) return PTV3_EWORKSPACE;
+    carve_begin(s, tables, scratch);
     hipStream_t stream = (hipStream_t)stream_;
     s.slot = host_slot;
     s.seq = seq;
@@ -996,9 +1006,9 @@ void read_sizes(State& s) {
     }
 }
 
-size_t carve_tables(State& s, void* base) {
+Bytes carve_pool(State& s, void* tables, void* scratch) {
     const ptv3_index_cfg& g = s.cfg;
-    Carver c(base);
+    Carver c(tables), free(scratch);
     const int k = g.n_orders;
     for (int l = 0; l < g.n_levels; ++l) {
         ptv3_level& v = s.lv[l];
@@ -1026,21 +1036,15 @@ size_t carve_tables(State& s, void* base) {
             }
         }
     }
-    return c.off;
-}
-
-size_t carve_scratch(State& s, void* base) {
-    const ptv3_index_cfg& g = s.cfg;
-    Carver c(base);
-    c.take<char>(1);   // never empty, also where there is no pooled level
+    free.take<char>(1);   // never empty, also where there is no pooled level
     for (int l = 1; l < g.n_levels; ++l) {
-        s.cells.cid[l] = c.take<int32_t>(g.n);
+        s.cells.cid[l] = free.take<int32_t>(g.n);
         ListLevel& v = s.lists.lv[l];
         v.n = s.lv[l].n;
         v.group = group_of(v.n, g.only128[l]);
-        carve_list_scratch(c, v, false);
+        carve_list_scratch(free, c, v, false);
     }
-    return c.off;
+    return {c.off, free.off};
 }
 
 size_t carve_lists(State& s, const int32_t* want, void* base) {
@@ -1081,8 +1085,9 @@ extern "C" int ptv3_index_pool_bytes(void* state, size_t* tables, size_t* scratc
     read_sizes(s);
     for (int l = 0; l < s.cfg.n_levels; ++l)
         if (s.lv[l].n < 1 || s.lv[l].n > s.cfg.n || s.lv[l].n_pad >= (1ll << 31)) return PTV3_EINVAL;
-    *tables = carve_tables(s, nullptr);
-    *scratch = carve_scratch(s, nullptr);
+    const Bytes need = carve_pool(s, nullptr, nullptr);
+    *tables = need.tables;
+    *scratch = need.scratch;
     return PTV3_OK;
 }
 
@@ -1092,9 +1097,9 @@ extern "C" int ptv3_index_pool(void* state, const int32_t* perms, void* tables, 
     State& s = *(State*)state;
     const ptv3_index_cfg& g = s.cfg;
     hipStream_t stream = (hipStream_t)stream_;
-    if (tables_bytes < carve_tables(s, nullptr) || scratch_bytes < carve_scratch(s, nullptr)) return PTV3_EWORKSPACE;
-    carve_tables(s, tables);
-    carve_scratch(s, scratch);
+    const Bytes need = carve_pool(s, nullptr, nullptr);
+    if (tables_bytes < need.tables || scratch_bytes < need.scratch) return PTV3_EWORKSPACE;
+    carve_pool(s, tables, scratch);
     CellArgs& a = s.cells;
     const int k = g.n_orders;
     // rows of the tables are permuted at every pooling: row r of level j is row perms[j][r] of the level above

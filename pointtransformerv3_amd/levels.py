@@ -110,12 +110,14 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     state = ctypes.create_string_buffer(_STATE_BYTES)
     slot = hostslot.take(lib.ptv3_index_slot_words(cfg.n_levels, nb))
     words, seq = slot.words, hostslot.next_seq()
-    nbytes = lib.ptv3_index_begin_bytes(ctypes.byref(cfg))
-    first = torch.empty(nbytes, **u8)
+    sizes = (ctypes.c_size_t * 2)()
+    check(lib.ptv3_index_begin_bytes(ctypes.byref(cfg), ctypes.byref(sizes, 0), ctypes.byref(sizes, 8)), "ptv3_index_begin_bytes")
+    # the scratch of this stage and of the pooling goes when this function returns: later work on the stream may have it
+    first, scratch0 = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
     out.batch = batch if batch is not None else torch.empty(n, dtype=torch.int64, device=dev)
     check(lib.ptv3_index_begin(state, ctypes.byref(cfg), grid_coord.data_ptr(), None if batch is None else batch.data_ptr(),
-                               offset.data_ptr(), out.batch.data_ptr(), first.data_ptr(), nbytes, slot.ptr, seq, stream),
-          "ptv3_index_begin")
+                               offset.data_ptr(), out.batch.data_ptr(), first.data_ptr(), sizes[0], scratch0.data_ptr(), sizes[1],
+                               slot.ptr, seq, stream), "ptv3_index_begin")
     if between is not None:
         between()
     check(lib.ptv3_index_wait(slot.ptr, 0, seq, stream), "ptv3_index_wait")
@@ -138,7 +140,6 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     check(lib.ptv3_index_sort(state, depth, key_bits, ids, out.code.data_ptr(), out.order.data_ptr(), out.inverse.data_ptr(),
                               ws.data_ptr(), nbytes, stream), "ptv3_index_sort")
     check(lib.ptv3_index_wait(slot.ptr, 1, seq, stream), "ptv3_index_wait")
-    sizes = (ctypes.c_size_t * 2)()
     check(lib.ptv3_index_pool_bytes(state, ctypes.byref(sizes, 0), ctypes.byref(sizes, 8)), "ptv3_index_pool_bytes")
     tables, scratch = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
     check(lib.ptv3_index_pool(state, perms, tables.data_ptr(), sizes[0], scratch.data_ptr(), sizes[1], stream),
@@ -159,7 +160,8 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     hostslot.give(slot)
     out.state = state                # `levels` lies in it
     out.offset, out.grid_coord, out.depth, out.n_orders = offset, grid_coord, depth, k
-    # `first` holds level 0's sparse indices, the pooled scene ends and level 0's tap_ptr; `scratch` the pooled tap_ptr
-    out.buffers = dict(first=first, tables=tables, scratch=scratch, lists=lists)
+    # `first` holds level 0's sparse indices, the pooled scene ends and level 0's tap_ptr
+    out.buffers = dict(first=first, tables=tables, lists=lists)
+    out.buffers["scratch"] = tables   # where the pooled tap_ptr lie, under the name of the buffer that used to hold them
     out.lists = list(wanted)
     return out

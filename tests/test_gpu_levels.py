@@ -120,3 +120,39 @@ def test_index_pass_single_list_kinds(want):
             shape = ((p,), (m + 1,), (m,))[kind]
             assert torch.equal(both.tensor(getattr(both.levels[lv], f), shape, torch.int32, "lists"),
                                one.tensor(getattr(one.levels[lv], f), shape, torch.int32, "lists"))
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_nothing_of_the_index_scratch_outlives_the_index(train):
+    """Bytes that stay allocated for a forward's result: its own tensors and the tables its keys are views of (about 100
+    bytes a point of codes, orders and inverses, up to 300 of pooled tables), no voxel hash."""
+    from pointtransformerv3_amd import PointTransformerV3, synthetic
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0).to(DEV)
+    model = model.train() if train else model.eval().half()
+    d = synthetic.collate([synthetic.room_scene(60_000, 5 + i, 0.02) for i in range(2)])
+    data = dict(feat=torch.from_numpy(synthetic.room_features(d["coord"], 1)).to(DEV).to(torch.float32 if train else torch.float16),
+                grid_coord=torch.from_numpy(d["grid_coord"]).to(DEV), offset=torch.from_numpy(d["offset"]).to(DEV))
+    n = data["feat"].shape[0]
+
+    def forward():
+        if train:
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                return model(dict(data))
+        with torch.inference_mode():
+            return model(dict(data))
+
+    forward()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    point = forward()
+    if train:
+        point.feat.sum().backward()
+        grads = sum(p.numel() * 4 for p in model.parameters())
+        point.feat = point.feat.detach()
+        point.sparse_conv_feat.features = point.feat
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_allocated() - before - (grads if train else 0)
+    indices = point.sparse_conv_feat.indices
+    assert indices.untyped_storage().nbytes() <= 16 * n + 4096
+    assert held <= n * (16 + 96 + 8 + 64 * point.feat.element_size() + 330) + (1 << 20), held / n

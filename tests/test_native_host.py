@@ -333,3 +333,15 @@ def test_models_of_another_architecture_are_left_to_the_modules(name, train, mon
     with torch.set_grad_enabled(train):
         for _ in range(2):
             assert (native_train if train else native).engine_for(model, data) is None
+
+
+@pytest.mark.parametrize("n", [1, 2000, 400_000])
+def test_index_tables_are_apart_from_the_scratch(n):
+    """The buffer that a returned Point's sparse indices lie in holds little else; voxel hash, keys and counts are another."""
+    from pointtransformerv3_amd import _lib, levels
+    cfg = levels.Cfg(n=n, n_levels=5, n_orders=4, n_scenes=4, stem5=1, patch=(ctypes.c_int32 * 8)(*[1024] * 8))
+    tables, scratch = ctypes.c_size_t(), ctypes.c_size_t()
+    lib = _lib.load()
+    assert lib.ptv3_index_begin_bytes(ctypes.byref(cfg), ctypes.byref(tables), ctypes.byref(scratch)) == 0
+    assert 16 * n <= tables.value <= 16 * n + 4096 and scratch.value >= 100 * n
+    assert lib.ptv3_index_begin_bytes(ctypes.byref(cfg), None, ctypes.byref(scratch)) != 0
