@@ -270,6 +270,13 @@ int ptv3_subm_conv_pairs_fwd(const void *feat, int dtype, int64_t n, int cin, in
                              int64_t n_pairs, const int32_t *tap_ptr, const int32_t *row_ptr,
                              const int32_t *pair_in, const int32_t *pair_slot, const void *weight,
                              const void *bias, int cout, void *y, void *out, void *stream);
+/* The same with channels in and out equal, 64 or 128, fp16/bf16, and the product rows kept in float (y: n_pairs x channels
+ * floats): the sum of a voxel's taps is rounded once, as in the tile forms that these widths take where there are more
+ * pairs (ptv3_conv_few_pairs). */
+int ptv3_subm_conv_pairs_wide_fwd(const void *feat, int dtype, int64_t n, int channels, int taps, int64_t n_pairs,
+                                  const int32_t *tap_ptr, const int32_t *row_ptr, const int32_t *pair_in,
+                                  const int32_t *pair_slot, const void *weight, const void *bias, float *y, void *out,
+                                  void *stream);
 
 /* Tile form of the 3x3x3 convolution with cin == cout == channels in {64, 128} (the xCPE of
  * every block, model.py:546-552; ptv3_subm_conv_pack_weight itself takes any multiple of 32), fp16/bf16: a work-group keeps the fp32 sums of a tile of 128
@@ -771,6 +778,7 @@ typedef struct ptv3_refresh {
 } ptv3_refresh;
 
 int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels);
+int ptv3_conv_few_pairs(int64_t n_pairs, int channels);   /* form 0 with product rows in float (ptv3_subm_conv_pairs_wide_fwd) */
 int ptv3_pad_rows(const void *x, int x_dtype, int64_t n, int c, int padded, void *out, int out_dtype, void *stream);
 size_t ptv3_features_bytes(const ptv3_net *net, const ptv3_level *levels, void *const *stage_out);
 int ptv3_features_fwd(const ptv3_net *net, const ptv3_level *levels, const void *feat, int feat_dtype,

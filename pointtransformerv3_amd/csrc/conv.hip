@@ -338,6 +338,43 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_dense_kernel(
     }
 }
 
+// A 32-row group's products from accumulators (lane: 4 consecutive channels of row `col`) to row segments in memory.
+// They go through the wave's LDS rows so that a store instruction writes 8 rows x 128 B. Product rows in half take two
+// 32-channel accumulators per segment, float rows one; the LDS rows are XS_STRIDE halfs = 144 B either way. slot_of(it):
+// the row of y that row it * 8 + lane / 8 goes to, negative for none.
+template <typename T, typename Y, int NT, typename SlotOf>
+__device__ __forceinline__ void store_products(const f32x16 (&acc)[NT], T* xs, int lane, int cout0, int cout, Y* __restrict__ y,
+                                               SlotOf slot_of) {
+    constexpr int TILES = sizeof(Y) == 4 ? 1 : 2, PIECE = 16 / sizeof(Y);
+    const int col = lane & 31, hf = lane >> 5, opc = lane & 7;
+#pragma unroll
+    for (int b0 = 0; b0 < NT; b0 += TILES) {
+#pragma unroll
+        for (int b = b0; b < b0 + TILES && b < NT; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (sizeof(Y) == 4) {
+                    typedef float f32x4 __attribute__((ext_vector_type(4)));
+                    const f32x4 pk = {acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2], acc[b][4 * q + 3]};
+                    *(f32x4*)((float*)(xs + col * XS_STRIDE) + 8 * q + 4 * hf) = pk;
+                } else {
+                    const u32x2 pk = {HalfOps<T>::pack2(acc[b][4 * q], acc[b][4 * q + 1]),
+                                      HalfOps<T>::pack2(acc[b][4 * q + 2], acc[b][4 * q + 3])};
+                    *(u32x2*)(xs + col * XS_STRIDE + (b - b0) * 32 + 8 * q + 4 * hf) = pk;
+                }
+            }
+        lds_fence();
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const int co = cout0 + b0 * 32 + opc * PIECE;
+            const u32x4 val = *(const u32x4*)(xs + (it * 8 + (lane >> 3)) * XS_STRIDE + opc * 8);
+            const int32_t slot = slot_of(it);
+            if (slot >= 0 && co < cout && (NT - b0 >= TILES || opc * PIECE < (NT - b0) * 32)) *(u32x4*)(y + (int64_t)slot * cout + co) = val;
+        }
+        lds_fence();
+    }
+}
+
 // Pair mode for wide inputs (cin a multiple of 32 * DEPTH), persistent work-groups.
 // A tile is ROWS consecutive entries of ONE tap of the tap-major pair list times COUT_TILE output
 // channels; the contraction runs in 32-channel steps. Both a step's MFMA work (a few hundred
@@ -350,10 +387,10 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_dense_kernel(
 //   * addresses are per-lane pointers set up once per tile (a step adds a constant), and the
 //     loop body has no branches: rows past the end of a tile and output channels past cout read
 //     a valid address and their products are never stored.
-template <typename T, int MT, int NT, int DEPTH>
+template <typename T, int MT, int NT, int DEPTH, typename Y>
 __global__ __launch_bounds__(CONV_THREADS, 2) void pair_gemm_kernel(
     const T* __restrict__ feat, int cin, int taps, const T* __restrict__ weight, int cout,
-    T* __restrict__ y, const int32_t* __restrict__ pair_in, const int32_t* __restrict__ pair_slot,
+    Y* __restrict__ y, const int32_t* __restrict__ pair_in, const int32_t* __restrict__ pair_slot,
     const int32_t* __restrict__ tap_ptr) {
     typedef typename HalfOps<T>::v8 v8;
     constexpr int KC = 32;
@@ -514,32 +551,9 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void pair_gemm_kernel(
         run_steps(nxt, 0);
 
         // acc[a][b][v]: output channel cout0 + b*32 + 8*(v/4) + 4*hf + v%4 of pair row0 + a*32 + col.
-        // Back to row-segment shape 64 channels at a time, 16 bytes per lane to y[slot].
 #pragma unroll
-        for (int a = 0; a < MT; ++a) {
-#pragma unroll
-            for (int b0 = 0; b0 < NT; b0 += 2) {
-#pragma unroll
-                for (int bb = 0; bb < 2 && b0 + bb < NT; ++bb)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int b = b0 + bb;
-                        u32x2 pk = {HalfOps<T>::pack2(acc[a][b][4 * q], acc[a][b][4 * q + 1]),
-                                    HalfOps<T>::pack2(acc[a][b][4 * q + 2], acc[a][b][4 * q + 3])};
-                        *(u32x2*)(xs + col * XS_STRIDE + bb * 32 + 8 * q + 4 * hf) = pk;
-                    }
-                lds_fence();
-#pragma unroll
-                for (int it = 0; it < 4; ++it) {
-                    const int orow = it * 8 + (lane >> 3), opc = lane & 7;
-                    const int co = cur.cout0 + b0 * 32 + opc * 8;
-                    const u32x4 val = *(const u32x4*)(xs + orow * XS_STRIDE + opc * 8);
-                    if (cur.slot[a][it] >= 0 && co < cout && (NT - b0 >= 2 || opc < 4))
-                        *(u32x4*)(y + (int64_t)cur.slot[a][it] * cout + co) = val;
-                }
-                lds_fence();
-            }
-        }
+        for (int a = 0; a < MT; ++a)
+            store_products<T, Y, NT>(acc[a], xs, lane, cur.cout0, cout, y, [&](int it) { return cur.slot[a][it]; });
         cur = nxt;
     }
 }
@@ -742,10 +756,10 @@ __global__ __launch_bounds__(WS_THREADS, 2) void pair_wstat_kernel(
 // lines per instruction instead of 32 is what keeps the address path from bounding the kernel.
 // PKC: input channels per step (64, or 32 where the 128-register accumulator leaves no room for
 // a 64-channel prefetch). A staged row segment is PKC*2 bytes = LPR lanes x 16 B.
-template <typename T, int MT, int NT, int PKC>
+template <typename T, int MT, int NT, int PKC, typename Y>
 __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_pairs_kernel(
     const T* __restrict__ feat, int cin, int taps, const T* __restrict__ weight, int cout,
-    T* __restrict__ y, const int32_t* __restrict__ pair_in, const int32_t* __restrict__ pair_slot,
+    Y* __restrict__ y, const int32_t* __restrict__ pair_in, const int32_t* __restrict__ pair_slot,
     const int32_t* __restrict__ tap_ptr, int range_rows) {
     typedef typename HalfOps<T>::v8 v8;
     constexpr int ROWS = CONV_WAVES * MT * 32;
@@ -895,37 +909,13 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_pairs_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // acc[a][b][v]: output channel cout0 + b*32 + 8*(v/4) + 4*hf + v%4 of the lane's row.
-        // Back to staging shape, 64 channels (two 32-channel tiles) at a time, then 16-byte stores.
+        // acc[a][b][v]: output channel cout0 + b*32 + 8*(v/4) + 4*hf + v%4 of the lane's row. The slot of row `r` sits in the
+        // lane that staged it: group (it*8)/RPI, lane (row within the group) * LPR
 #pragma unroll
-        for (int a = 0; a < MT; ++a) {
-#pragma unroll
-            for (int b0 = 0; b0 < NT; b0 += 2) {
-#pragma unroll
-                for (int bb = 0; bb < 2 && b0 + bb < NT; ++bb)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const int b = b0 + bb;
-                        u32x2 pk = {HalfOps<T>::pack2(acc[a][b][4 * g], acc[a][b][4 * g + 1]),
-                                    HalfOps<T>::pack2(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3])};
-                        *(u32x2*)(xs + col * XS_STRIDE + bb * 32 + 8 * g + 4 * hf) = pk;
-                    }
-                lds_fence();
-                // 64 output channels of 32 rows = 8 lanes x 16 B per row, 8 rows per store
-#pragma unroll
-                for (int it = 0; it < 4; ++it) {
-                    const int orow = it * 8 + (lane >> 3), opc = lane & 7;
-                    const int co = cout0 + b0 * 32 + opc * 8;
-                    const u32x4 v = *(const u32x4*)(xs + orow * XS_STRIDE + opc * 8);
-                    // the slot of row `orow` sits in the lane that staged it: group (it*8)/RPI, lane
-                    // (row within the group) * LPR
-                    const int32_t slot = __shfl(slot_c[a][(it * 8) / RPI], (((it * 8) % RPI) + (lane >> 3)) * LPR, PTV3_WAVE);
-                    if (slot >= 0 && co < cout && (NT - b0 >= 2 || opc < 4))
-                        *(u32x4*)(y + (int64_t)slot * cout + co) = v;
-                }
-                lds_fence();
-            }
-        }
+        for (int a = 0; a < MT; ++a)
+            store_products<T, Y, NT>(acc[a], xs, lane, cout0, cout, y, [&](int it) {
+                return __shfl(slot_c[a][(it * 8) / RPI], (((it * 8) % RPI) + (lane >> 3)) * LPR, PTV3_WAVE);
+            });
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
@@ -937,13 +927,13 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_pairs_kernel(
 }
 
 // y (n_pairs, cout) in output-major slot order -> out[i] = bias + sum of voxel i's slots
-template <typename T>
-__global__ __launch_bounds__(256) void pair_segment_sum_kernel(const T* __restrict__ y,
+template <typename T, typename Y>
+__global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restrict__ y,
                                                                const int32_t* __restrict__ row_ptr,
                                                                int64_t n, int cout,
                                                                const T* __restrict__ bias,
                                                                T* __restrict__ out) {
-    typedef typename HalfOps<T>::v8 v8;
+    typedef Y v8 __attribute__((ext_vector_type(8)));
     const int groups = cout / 8;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n * groups) return;
@@ -954,20 +944,19 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const T* __restri
     for (int k = 0; k < 8; ++k) acc[k] = bias ? HalfOps<T>::to_float(bias[c + k]) : 0.f;
     const int s0 = row_ptr[i], s1 = row_ptr[i + 1];
     // four rows in flight per thread; the additions keep the order s0, s0+1, ...
-    const T* src = y + (int64_t)s0 * cout + c;
+    const Y* src = y + (int64_t)s0 * cout + c;
     for (int s = s0; s < s1; s += 4, src += 4 * (int64_t)cout) {
-        u32x4 raw[4];
+        v8 raw[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            raw[j] = (u32x4){0, 0, 0, 0};
-            if (s + j < s1) raw[j] = *(const u32x4*)(src + (int64_t)j * cout);
+            raw[j] = (v8){0, 0, 0, 0, 0, 0, 0, 0};
+            if (s + j < s1) raw[j] = *(const v8*)(src + (int64_t)j * cout);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (s + j < s1) {
-                const v8 v = __builtin_bit_cast(v8, raw[j]);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) acc[k] += (float)v[k];
+                for (int k = 0; k < 8; ++k) acc[k] += (float)raw[j][k];
             }
         }
     }
@@ -1023,14 +1012,14 @@ void dispatch_dense(const void* feat, int64_t n, int cin, const int32_t* nbr, in
 #undef PTV3_DENSE
 }
 
-template <typename T, int MT, int NT>
+template <typename T, int MT, int NT, typename Y>
 int launch_pairs(const void* feat, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
                  const int32_t* pair_in, const int32_t* pair_slot, const void* weight, int cout, void* y,
                  hipStream_t stream) {
     constexpr int ROWS = CONV_WAVES * MT * 32, COUT_TILE = NT * 32;
     const size_t lds = ((size_t)COUT_TILE * (cin + W_PAD) + (size_t)CONV_WAVES * 32 * XS_STRIDE) * sizeof(T);
     if (lds > 160 * 1024) return PTV3_ESHAPE;
-    auto kern = subm_conv_pairs_kernel<T, MT, NT, (NT >= 4 ? 32 : 64)>;
+    auto kern = subm_conv_pairs_kernel<T, MT, NT, (NT >= 4 ? 32 : 64), Y>;
     static LdsGrant grant_lds_allowed;   // per instantiation and device; raised monotonically
     if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_lds_allowed)) return rc_;
     // Rows per work-group: long enough to amortise staging the weights, short enough to give
@@ -1040,7 +1029,7 @@ int launch_pairs(const void* feat, int cin, int taps, int64_t n_pairs, const int
     while (range_rows > ROWS && (n_pairs / range_rows + taps) * col_tiles < 1024) range_rows /= 2;
     dim3 grid((unsigned)(n_pairs / range_rows + taps), (unsigned)col_tiles);   // every tap may end with a partial range
     hipLaunchKernelGGL(kern, grid, dim3(CONV_THREADS), lds, stream, (const T*)feat, cin, taps, (const T*)weight, cout,
-                       (T*)y, pair_in, pair_slot, tap_ptr, (int)range_rows);
+                       (Y*)y, pair_in, pair_slot, tap_ptr, (int)range_rows);
     return PTV3_OK;
 }
 
@@ -1056,7 +1045,7 @@ int launch_pairs_chunked_v(const void* feat, int cin, int taps, int64_t n_pairs,
                        (const T*)nullptr, cout, (T*)y, pair_in, pair_slot, tap_ptr);
     return PTV3_OK;
 }
-template <typename T, int MT, int NT, int DEPTH>
+template <typename T, int MT, int NT, int DEPTH, typename Y>
 int launch_pair_gemm(const void* feat, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
                      const int32_t* pair_in, const int32_t* pair_slot, const void* weight, int cout, void* y,
                      hipStream_t stream) {
@@ -1065,8 +1054,8 @@ int launch_pair_gemm(const void* feat, int cin, int taps, int64_t n_pairs, const
     const int64_t tiles_max = (n_pairs / ROWS + taps) * ptv3_ceil_div(cout, COUT_TILE);
     const int64_t resident = 256 * 2;
     dim3 grid((unsigned)(tiles_max < resident ? tiles_max : resident));
-    hipLaunchKernelGGL((pair_gemm_kernel<T, MT, NT, DEPTH>), grid, dim3(CONV_THREADS), 0, stream, (const T*)feat, cin,
-                       taps, (const T*)weight, cout, (T*)y, pair_in, pair_slot, tap_ptr);
+    hipLaunchKernelGGL((pair_gemm_kernel<T, MT, NT, DEPTH, Y>), grid, dim3(CONV_THREADS), 0, stream, (const T*)feat, cin,
+                       taps, (const T*)weight, cout, (Y*)y, pair_in, pair_slot, tap_ptr);
     return PTV3_OK;
 }
 template <typename T>
@@ -1097,7 +1086,7 @@ int launch_pairs_chunked(const void* feat, int cin, int taps, int64_t n_pairs, c
         return launch_pair_wstat<T>(feat, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
     // the ring of the persistent kernel is four 32-channel steps deep
     if (cin % 128 == 0 && taps <= 128)
-        return launch_pair_gemm<T, 1, 4, 4>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
+        return launch_pair_gemm<T, 1, 4, 4, T>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
     return launch_pairs_chunked_v<T, 2, 4, 32>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
 }
 
@@ -1109,11 +1098,25 @@ int dispatch_pairs(const void* feat, int cin, int taps, int64_t n_pairs, const i
     // tile kernel, which keeps more waves in flight than one tap's weights in LDS allow
     if (cin >= 128 && cout > 64)
         return launch_pairs_chunked<T>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
-#define PTV3_PAIRS(MT, NT) return launch_pairs<T, MT, NT>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream)
+#define PTV3_PAIRS(MT, NT) return launch_pairs<T, MT, NT, T>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream)
     if (cout <= 32) PTV3_PAIRS(2, 1);
     if (cout <= 64) PTV3_PAIRS(2, 2);
     PTV3_PAIRS(2, 4);
 #undef PTV3_PAIRS
+}
+
+// product rows in float: the widths whose other forms keep their sums on chip in float
+template <typename T>
+int dispatch_pairs_wide(const void* feat, int c, int taps, int64_t n_pairs, const int32_t* tap_ptr, const int32_t* pair_in,
+                        const int32_t* pair_slot, const void* weight, void* y, hipStream_t stream) {
+    if (c == 64) return launch_pairs<T, 2, 2, float>(feat, c, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, c, y, stream);
+    return launch_pair_gemm<T, 1, 4, 4, float>(feat, c, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, c, y, stream);
+}
+
+template <typename T, typename Y>
+void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int cout, const void* bias, void* out, hipStream_t stream) {
+    hipLaunchKernelGGL((pair_segment_sum_kernel<T, Y>), dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream,
+                       (const Y*)y, row_ptr, n, cout, (const T*)bias, (T*)out);
 }
 
 }  // namespace
@@ -1163,20 +1166,38 @@ extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, 
     if (dtype == PTV3_F32)
         return ptv3_subm_conv_pairs_f32((const float*)feat, n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot,
                                         (const float*)weight, (const float*)bias, cout, (float*)y, (float*)out, stream);
-    const dim3 sgrid((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), sblock(256);
     int rc = PTV3_OK;
     if (dtype == PTV3_F16) {
         if (n_pairs > 0)
             rc = dispatch_pairs<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        hipLaunchKernelGGL(pair_segment_sum_kernel<_Float16>, sgrid, sblock, 0, stream, (const _Float16*)y,
-                           row_ptr, n, cout, (const _Float16*)bias, (_Float16*)out);
+        launch_segment_sum<_Float16, _Float16>(y, row_ptr, n, cout, bias, out, stream);
     } else {
         if (n_pairs > 0)
             rc = dispatch_pairs<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        hipLaunchKernelGGL(pair_segment_sum_kernel<__bf16>, sgrid, sblock, 0, stream, (const __bf16*)y, row_ptr,
-                           n, cout, (const __bf16*)bias, (__bf16*)out);
+        launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, cout, bias, out, stream);
     }
+    PTV3_RETURN_LAUNCH();
+}
+
+extern "C" int ptv3_subm_conv_pairs_wide_fwd(const void* feat, int dtype, int64_t n, int channels, int taps, int64_t n_pairs,
+                                             const int32_t* tap_ptr, const int32_t* row_ptr, const int32_t* pair_in,
+                                             const int32_t* pair_slot, const void* weight, const void* bias, float* y, void* out,
+                                             void* stream_) {
+    if (n < 0 || taps < 1 || taps > 128 || n_pairs < 0 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
+    if ((dtype != PTV3_F16 && dtype != PTV3_BF16) || (channels != 64 && channels != 128)) return PTV3_ESHAPE;
+    if (n == 0) return PTV3_OK;
+    if (!feat || !tap_ptr || !row_ptr || !weight || !out) return PTV3_EINVAL;
+    if (n_pairs > 0 && (!pair_in || !pair_slot || !y)) return PTV3_EINVAL;
+    hipStream_t stream = (hipStream_t)stream_;
+    if (n_pairs > 0) {
+        const int rc = dtype == PTV3_F16
+                           ? dispatch_pairs_wide<_Float16>(feat, channels, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, y, stream)
+                           : dispatch_pairs_wide<__bf16>(feat, channels, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, y, stream);
+        if (rc != PTV3_OK) return rc;
+    }
+    if (dtype == PTV3_F16) launch_segment_sum<_Float16, float>(y, row_ptr, n, channels, bias, out, stream);
+    else launch_segment_sum<__bf16, float>(y, row_ptr, n, channels, bias, out, stream);
     PTV3_RETURN_LAUNCH();
 }

@@ -77,8 +77,12 @@ int conv3(Run& r, const ptv3_block_w& b, const ptv3_level& v, const void* x, voi
     const int form = r.dt == PTV3_F32 ? 0 : ptv3_conv_form(v.n, v.n_pairs, c);
     if (form == 0) {
         const size_t mark = r.mem.at;
-        void* y = r.rows(v.n_pairs, c);
-        if (!r.dry)
+        const bool wide = r.dt != PTV3_F32 && ptv3_conv_few_pairs(v.n_pairs, c);
+        void* y = r.mem.take((size_t)v.n_pairs * c * (wide ? 4 : r.es));
+        if (!r.dry && wide)
+            TRY(ptv3_subm_conv_pairs_wide_fwd(x, r.dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, b.conv_w,
+                                              b.conv_b, (float*)y, out, r.stream));
+        else if (!r.dry)
             TRY(ptv3_subm_conv_pairs_fwd(x, r.dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, b.conv_w,
                                          b.conv_b, c, y, out, r.stream));
         r.mem.at = mark;
@@ -319,15 +323,23 @@ bool net_ok(const ptv3_net* net, const ptv3_level* lv) {
 
 }  // namespace
 
-// The form the 3x3x3 convolution of a half-precision level takes: 0 pair lists, 1 sparse tiles, 2 tiles. The rule on pairs
-// per voxel: 32 and 64 channels take the sparse tile form up to 14 (work in proportion to the pairs; faster than both other
-// forms from 2.5 to 10), 64 and 128 the tile form from 4 on (sums kept on chip, no pair matrix through memory). A tile
-// walks its taps one after the other, 14 - 23 us (64 channels) or 42 - 54 us (128) however few tiles there are, while the
-// pair form is two short launches that spread over the part: 64 channels 11 against 14 us at 20k pairs, 16 against 17 at
-// 71k, 25 against 21 at 139k; 128 channels 13 against 42 us at 7k pairs, 33 against 43 at 201k, 60 against 54 at 420k.
+// 64 and 128 channels with few pairs: the pair form, its product rows in float. A tile form walks its taps one after the
+// other, 22 - 24 us (64 channels, sparse tiles) or 42 - 44 us (128) however few tiles there are, while the pair form is two
+// short launches that spread over the part. Float rows make its sums what the tile forms keep on chip, rounded once: the
+// error against 64 bits is theirs (2.08e-4 in fp16; half rows 2.31e-4 at 2 us less). Measured in fp16, pair form with float
+// rows against the tile form, us: 64 channels 13.0 / 22.4 at 10k pairs, 20.3 / 23.9 at 67k, 23.7 / 22.3 at 119k; 128 channels
+// 13.5 / 42.0 at 8k, 26.4 / 43.0 at 92k, 41.8 / 43.4 at 167k, 55.5 / 43.7 at 238k.
+extern "C" int ptv3_conv_few_pairs(int64_t n_pairs, int channels) {
+    return (channels == 64 && n_pairs <= 70000) || (channels == 128 && n_pairs <= 185000);
+}
+
+// The form the 3x3x3 convolution of a half-precision level takes: 0 pair lists, 1 sparse tiles, 2 tiles. Above the few pairs
+// of ptv3_conv_few_pairs the rule is on pairs per voxel: 32 and 64 channels take the sparse tile form up to 14 (work in
+// proportion to the pairs; faster than both other forms from 2.5 to 10), 64 and 128 the tile form from 4 on (sums kept on
+// chip, no pair matrix through memory).
 extern "C" int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels) {
     if (n < 1 || n >= (1ll << 24)) return 0;
-    if ((channels == 64 && n_pairs <= 70000) || (channels == 128 && n_pairs <= 300000)) return 0;
+    if (ptv3_conv_few_pairs(n_pairs, channels)) return 0;
     if ((channels == 32 || channels == 64) && n_pairs <= 14 * n) return 1;
     if ((channels == 64 || channels == 128) && n_pairs >= 4 * n) return 2;
     return 0;

@@ -148,9 +148,14 @@ struct Run {
             return ptv3_subm_conv_tiles_fwd_sized(x, dt, v.n, c, 27, v.tile_voxels, packed, bias, v.tile_tap, v.tile_pair,
                                                   v.vox_taps, out, stream);
         const size_t mark = scratch.at;
-        void* y = scratch.take((size_t)v.n_pairs * c * 2);
-        DO(ptv3_subm_conv_pairs_fwd(x, dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, w, bias, c, y, out,
-                                     stream));
+        const bool wide = ptv3_conv_few_pairs(v.n_pairs, c);
+        void* y = scratch.take((size_t)v.n_pairs * c * (wide ? 4 : 2));
+        if (wide)
+            DO(ptv3_subm_conv_pairs_wide_fwd(x, dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, w, bias,
+                                             (float*)y, out, stream));
+        else
+            DO(ptv3_subm_conv_pairs_fwd(x, dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, w, bias, c, y,
+                                        out, stream));
         scratch.at = mark;
         return PTV3_OK;
     }

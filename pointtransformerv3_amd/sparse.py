@@ -150,7 +150,8 @@ class SubMConv3d(nn.Module):
             return (ops.subm_conv_sparse if form == "sparse" else ops.subm_conv_tiles)(feat, plan, tiles, bias)
         weight = weight.to(feat.dtype)
         if plan.density() <= self.PAIR_MODE_MAX_DENSITY and cout % 8 == 0:
-            return ops.subm_conv_pairs(feat, plan, weight, bias)
+            wide = self.kernel_size == 3 and cin == cout and _lib.load().ptv3_conv_few_pairs(plan.n_pairs, cin)
+            return ops.subm_conv_pairs(feat, plan, weight, bias, wide=bool(wide))
         return ops.subm_conv(feat, x.neighbour_map(self.kernel_size, self.indice_key), weight, bias, tap_major=True)
 
     def forward(self, x):

@@ -46,3 +46,52 @@ def test_convolution_of_few_pairs(c, n, extent, dtype):
     got = conv(SparseConvTensor(x.to(DEV), to_dev(idx), [extent + 96] * 3, 2)).features
     want = OF.subm_conv(x.float(), OI.subm_kmap(idx), conv.weight.float().cpu(), conv.bias.float().cpu())
     assert rel_err(got, want) < {torch.float16: 2e-2, torch.bfloat16: 2e-2}[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c,n,extent", [(64, 1, 2), (64, 33, 4), (64, 2000, 14), (64, 6000, 40), (128, 1, 2), (128, 129, 8), (128, 700, 10), (128, 7000, 24)])
+def test_convolution_of_few_pairs_rounds_once(c, n, extent, dtype):
+    """The pair form with product rows in float against 64 bits: products exact in float, sums of at most 27 taps in float,
+    one rounding to half, as in the tile form whose place it takes -- its error is the tile form's, not 1.1 times it."""
+    import numpy as np
+
+    from pointtransformerv3_amd import _lib, ops
+    grid, batch, _ = unique_voxels(np.random.default_rng(n), n, extent, nb=2)
+    idx = to_dev(np.concatenate([batch[:, None], grid], 1).astype(np.int32))
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(len(grid), c, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(c, 27, c, generator=g, device=DEV) / (27 * c) ** 0.5).to(dtype)
+    bias = torch.randn(c, generator=g, device=DEV).to(dtype)
+    plan = ops.conv_plan_direct(idx, 3)
+    assert _lib.load().ptv3_conv_few_pairs(plan.n_pairs, c) and not _lib.load().ptv3_conv_few_pairs(plan.n_pairs, 32)
+    want = bias.double().expand(len(grid), c).clone()
+    nbr = ops.kmap_build(idx, 3).long()
+    for t in range(27):
+        on = nbr[:, t] >= 0
+        want[on] += x.double()[nbr[on, t]] @ w[:, t].double().t()
+    err = lambda y: float((y.double() - want).norm() / want.norm())
+    wide = err(ops.subm_conv_pairs(x, plan, w, bias, wide=True))
+    tile = err(ops.subm_conv_tiles(x, plan, ops.conv_pack_weight(w, 27, dtype), bias))
+    eps = torch.finfo(dtype).eps
+    assert wide <= 1.02 * tile + 0.02 * eps and wide < 0.5 * eps
+    assert torch.equal(ops.subm_conv_pairs(x, plan, w, None, wide=True), ops.subm_conv_pairs(x, plan, w, torch.zeros_like(bias), wide=True))
+
+
+@pytest.mark.parametrize("n", [2000, 6000])
+def test_few_pairs_in_model_and_training_take_float_rows(n, monkeypatch):
+    """SubMConv3d in inference and both directions of its training ask for them where the rule says so."""
+    import numpy as np
+
+    from pointtransformerv3_amd import ops
+    from pointtransformerv3_amd.sparse import SparseConvTensor, SubMConv3d
+    grid, batch, _ = unique_voxels(np.random.default_rng(n), n, 30, nb=1)
+    idx = to_dev(np.concatenate([batch[:, None], grid], 1).astype(np.int32))
+    seen, real = [], ops.subm_conv_pairs
+    monkeypatch.setattr(ops, "subm_conv_pairs", lambda *a, wide=False: seen.append(wide) or real(*a, wide=wide))
+    conv = SubMConv3d(128, 128, 3, bias=True, indice_key="k").half().to(DEV)
+    x = torch.randn(n, 128, device=DEV, dtype=torch.half, requires_grad=True)
+    sparse = lambda: SparseConvTensor(x, idx, [128] * 3, 1)
+    with torch.no_grad():
+        conv(sparse())
+    conv(sparse()).features.sum().backward()
+    assert seen == [True] * 3
