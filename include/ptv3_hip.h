@@ -270,13 +270,19 @@ int ptv3_subm_conv_pairs_fwd(const void *feat, int dtype, int64_t n, int cin, in
                              int64_t n_pairs, const int32_t *tap_ptr, const int32_t *row_ptr,
                              const int32_t *pair_in, const int32_t *pair_slot, const void *weight,
                              const void *bias, int cout, void *y, void *out, void *stream);
-/* The same with channels in and out equal, 64 or 128, fp16/bf16, and the product rows kept in float (y: n_pairs x channels
- * floats): the sum of a voxel's taps is rounded once, as in the tile forms that these widths take where there are more
- * pairs (ptv3_conv_few_pairs). */
-int ptv3_subm_conv_pairs_wide_fwd(const void *feat, int dtype, int64_t n, int channels, int taps, int64_t n_pairs,
+/* The same in fp16/bf16 with the product rows kept in float (y: n_pairs x cout floats): a voxel's sum is rounded once, as in
+ * the forms that keep it on chip. cin in 16s and cout in 8s; above 64 outputs cin in 128s, else up to 512. */
+int ptv3_subm_conv_pairs_wide_fwd(const void *feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs,
                                   const int32_t *tap_ptr, const int32_t *row_ptr, const int32_t *pair_in,
-                                  const int32_t *pair_slot, const void *weight, const void *bias, float *y, void *out,
-                                  void *stream);
+                                  const int32_t *pair_slot, const void *weight, const void *bias, int cout, float *y,
+                                  void *out, void *stream);
+/* Which of these three a layer that no tile form takes (ptv3_conv_form 0, or not 3x3x3) runs on: the pair form, the pair
+ * form with float rows, or the dense form over the neighbour map (ptv3_subm_conv_fwd). max_density: pairs over voxels x
+ * taps above which product rows are avoided. */
+#define PTV3_CONV_PAIRS 0
+#define PTV3_CONV_PAIRS_WIDE 1
+#define PTV3_CONV_DENSE 2
+int ptv3_conv_pair_form(int dtype, int64_t n, int64_t n_pairs, int taps, int cin, int cout, float max_density);
 
 /* Tile form of the 3x3x3 convolution with cin == cout == channels in {64, 128} (the xCPE of
  * every block, model.py:546-552; ptv3_subm_conv_pack_weight itself takes any multiple of 32), fp16/bf16: a work-group keeps the fp32 sums of a tile of 128
@@ -760,6 +766,7 @@ typedef struct ptv3_stage_w {
 typedef struct ptv3_net {
     int32_t dtype, n_stages, decoder, stem_in;
     int32_t patch[PTV3_MAX_LEVELS];
+    float max_pair_density, reserved;         /* ptv3_conv_pair_form */
     const void *stem_w;
     ptv3_bn_w stem_bn;
     ptv3_stage_w stage[PTV3_MAX_LEVELS];
@@ -778,7 +785,7 @@ typedef struct ptv3_refresh {
 } ptv3_refresh;
 
 int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels);
-int ptv3_conv_few_pairs(int64_t n_pairs, int channels);   /* form 0 with product rows in float (ptv3_subm_conv_pairs_wide_fwd) */
+int ptv3_conv_few_pairs(int64_t n_pairs, int channels);
 int ptv3_pad_rows(const void *x, int x_dtype, int64_t n, int c, int padded, void *out, int out_dtype, void *stream);
 size_t ptv3_features_bytes(const ptv3_net *net, const ptv3_level *levels, void *const *stage_out);
 int ptv3_features_fwd(const ptv3_net *net, const ptv3_level *levels, const void *feat, int feat_dtype,
@@ -829,6 +836,7 @@ typedef struct ptv3_zero_range { int64_t at, count, first_block; } ptv3_zero_ran
 typedef struct ptv3_train_net {
     int32_t dtype, n_stages;
     int32_t patch[PTV3_MAX_LEVELS];
+    float max_pair_density, reserved2;        /* ptv3_conv_pair_form */
     ptv3_train_stem stem;
     const ptv3_zero_range *zero;              /* device array */
     int32_t n_zero, reserved;

@@ -131,7 +131,8 @@ SIGNATURES = {
     "ptv3_index_levels": (_vp, [_vp]),
     "ptv3_conv_form": (_i32, [_i64, _i64, _i32]),
     "ptv3_conv_few_pairs": (_i32, [_i64, _i32]),
-    "ptv3_subm_conv_pairs_wide_fwd": (_i32, [_vp, _i32, _i64, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "ptv3_subm_conv_pairs_wide_fwd": (_i32, [_vp, _i32, _i64, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp]),
+    "ptv3_conv_pair_form": (_i32, [_i32, _i64, _i64, _i32, _i32, _i32, _f32]),
     "ptv3_pad_rows": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _i32, _vp]),
     "ptv3_features_bytes": (_sz, [_vp, _vp, _vp]),
     "ptv3_features_fwd": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz, _vp]),

@@ -1105,12 +1105,15 @@ int dispatch_pairs(const void* feat, int cin, int taps, int64_t n_pairs, const i
 #undef PTV3_PAIRS
 }
 
-// product rows in float: the widths whose other forms keep their sums on chip in float
+// product rows in float, for shapes whose other forms keep a voxel's sum on chip in float (ptv3_conv_pair_form)
+bool wide_ok(int cin, int cout) { return cin % 16 == 0 && cout % 8 == 0 && (cout <= 64 ? cin <= 512 : cin % 128 == 0); }
+
 template <typename T>
-int dispatch_pairs_wide(const void* feat, int c, int taps, int64_t n_pairs, const int32_t* tap_ptr, const int32_t* pair_in,
-                        const int32_t* pair_slot, const void* weight, void* y, hipStream_t stream) {
-    if (c == 64) return launch_pairs<T, 2, 2, float>(feat, c, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, c, y, stream);
-    return launch_pair_gemm<T, 1, 4, 4, float>(feat, c, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, c, y, stream);
+int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr, const int32_t* pair_in,
+                        const int32_t* pair_slot, const void* weight, int cout, void* y, hipStream_t stream) {
+    if (cout <= 32) return launch_pairs<T, 2, 1, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
+    if (cout <= 64) return launch_pairs<T, 2, 2, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
+    return launch_pair_gemm<T, 1, 4, 4, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
 }
 
 template <typename T, typename Y>
@@ -1181,23 +1184,40 @@ extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, 
     PTV3_RETURN_LAUNCH();
 }
 
-extern "C" int ptv3_subm_conv_pairs_wide_fwd(const void* feat, int dtype, int64_t n, int channels, int taps, int64_t n_pairs,
+extern "C" int ptv3_subm_conv_pairs_wide_fwd(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs,
                                              const int32_t* tap_ptr, const int32_t* row_ptr, const int32_t* pair_in,
-                                             const int32_t* pair_slot, const void* weight, const void* bias, float* y, void* out,
-                                             void* stream_) {
-    if (n < 0 || taps < 1 || taps > 128 || n_pairs < 0 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
-    if ((dtype != PTV3_F16 && dtype != PTV3_BF16) || (channels != 64 && channels != 128)) return PTV3_ESHAPE;
+                                             const int32_t* pair_slot, const void* weight, const void* bias, int cout, float* y,
+                                             void* out, void* stream_) {
+    if (n < 0 || cin < 1 || cout < 1 || taps < 1 || taps > 128 || n_pairs < 0 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
+    if ((dtype != PTV3_F16 && dtype != PTV3_BF16) || !wide_ok(cin, cout)) return PTV3_ESHAPE;
     if (n == 0) return PTV3_OK;
     if (!feat || !tap_ptr || !row_ptr || !weight || !out) return PTV3_EINVAL;
     if (n_pairs > 0 && (!pair_in || !pair_slot || !y)) return PTV3_EINVAL;
     hipStream_t stream = (hipStream_t)stream_;
     if (n_pairs > 0) {
         const int rc = dtype == PTV3_F16
-                           ? dispatch_pairs_wide<_Float16>(feat, channels, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, y, stream)
-                           : dispatch_pairs_wide<__bf16>(feat, channels, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, y, stream);
+                           ? dispatch_pairs_wide<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream)
+                           : dispatch_pairs_wide<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
     }
-    if (dtype == PTV3_F16) launch_segment_sum<_Float16, float>(y, row_ptr, n, channels, bias, out, stream);
-    else launch_segment_sum<__bf16, float>(y, row_ptr, n, channels, bias, out, stream);
+    if (dtype == PTV3_F16) launch_segment_sum<_Float16, float>(y, row_ptr, n, cout, bias, out, stream);
+    else launch_segment_sum<__bf16, float>(y, row_ptr, n, cout, bias, out, stream);
     PTV3_RETURN_LAUNCH();
+}
+
+// See ptv3_conv_few_pairs for the first rule. The second is on dense volumes, where most taps of most voxels are there: the
+// dense form writes no product rows (27 a voxel, in memory and time) and rounds a sum once, but walks all taps in every
+// work-group, 38 us (32 channels) to 340 us (512) at 27 taps and 155 us at 125 however few voxels there are. Up to 8500
+// pairs a tap the pair form with float rows gives the same sums in less: float rows against dense form, fp16, us: 13 / 38 at
+// 22k pairs of 32 channels, 27 / 37 at 231k, 37 / 38 at 439k; 512 channels 35 / 348, 316 / 377, 583 / 477; 5x5x5 16 -> 32
+// channels 60 / 155 at 992k, 110 / 155 at 1.9M.
+// In float the pair form runs on the matrix cores and the dense form does not (84 us against 5.1 ms at 439k pairs of 64
+// channels), so the dense form is only what is left where the product rows would take more than 32 GiB.
+extern "C" int ptv3_conv_pair_form(int dtype, int64_t n, int64_t n_pairs, int taps, int cin, int cout, float max_density) {
+    const bool dense = (double)n_pairs > (double)max_density * (double)n * taps;
+    if (dtype == PTV3_F32) return dense && n_pairs * cout > (8ll << 30) ? PTV3_CONV_DENSE : PTV3_CONV_PAIRS;
+    if (taps == 27 && cin == cout && ptv3_conv_few_pairs(n_pairs, cin)) return PTV3_CONV_PAIRS_WIDE;
+    if (cout % 8 != 0) return PTV3_CONV_DENSE;
+    if (!dense) return PTV3_CONV_PAIRS;
+    return n_pairs <= 8500ll * taps && wide_ok(cin, cout) ? PTV3_CONV_PAIRS_WIDE : PTV3_CONV_DENSE;
 }

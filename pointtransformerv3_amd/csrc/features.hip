@@ -35,6 +35,7 @@ struct Run {
     bool dry;
     int dt;          // dtype of the rows
     size_t es;
+    int32_t *map3[PTV3_MAX_LEVELS] = {}, *map5 = nullptr;   // neighbour maps, where a convolution takes the dense form
     Run(const ptv3_net* n, const ptv3_level* l, void* s, void* ws)
         : net(n), lv(l), stream(s), mem(ws), dry(ws == nullptr), dt(n->dtype), es(n->dtype == PTV3_F32 ? 4 : 2) {}
     void* rows(int64_t n, int64_t c) { return mem.take((size_t)n * c * es); }
@@ -72,22 +73,65 @@ int linear_bn_gelu(Run& r, const void* x, const ptv3_linear_w& w, const ptv3_bn_
                  : ptv3_bn_act(y, bn.mean, bn.var, bn.stats_f32, bn.g, bn.b, r.dt, n, w.out, bn.eps, 1, out, r.stream);
 }
 
-int conv3(Run& r, const ptv3_block_w& b, const ptv3_level& v, const void* x, void* out) {
-    const int c = b.channels;
-    const int form = r.dt == PTV3_F32 ? 0 : ptv3_conv_form(v.n, v.n_pairs, c);
-    if (form == 0) {
-        const size_t mark = r.mem.at;
-        const bool wide = r.dt != PTV3_F32 && ptv3_conv_few_pairs(v.n_pairs, c);
-        void* y = r.mem.take((size_t)v.n_pairs * c * (wide ? 4 : r.es));
-        if (!r.dry && wide)
-            TRY(ptv3_subm_conv_pairs_wide_fwd(x, r.dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, b.conv_w,
-                                              b.conv_b, (float*)y, out, r.stream));
-        else if (!r.dry)
-            TRY(ptv3_subm_conv_pairs_fwd(x, r.dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, b.conv_w,
-                                         b.conv_b, c, y, out, r.stream));
-        r.mem.at = mark;
-        return PTV3_OK;
+// A convolution that no tile form takes: product rows, or the neighbour map where ptv3_conv_pair_form says so (then made
+// in front of the forward, make_map).
+int pair_form(const Run& r, int s, int taps, int cin, int cout) {
+    const ptv3_level& v = r.lv[s];
+    return ptv3_conv_pair_form(r.dt, v.n, taps == 27 ? v.n_pairs : v.n_pairs5, taps, cin, cout, r.net->max_pair_density);
+}
+int conv_rows(Run& r, int s, int taps, const void* x, int cin, const void* w, const void* bias, int cout, void* out) {
+    const ptv3_level& v = r.lv[s];
+    const bool inner = taps == 27;
+    const int64_t n_pairs = inner ? v.n_pairs : v.n_pairs5;
+    const int32_t *tap_ptr = inner ? v.tap_ptr : v.tap_ptr5, *row_ptr = inner ? v.row_ptr : v.row_ptr5;
+    const int32_t *pair_in = inner ? v.pair_in : v.pair_in5, *pair_slot = inner ? v.pair_slot : v.pair_slot5;
+    const int form = pair_form(r, s, taps, cin, cout);
+    if (form == PTV3_CONV_DENSE)
+        return r.dry ? PTV3_OK
+                     : ptv3_subm_conv_fwd(x, r.dt, v.n, cin, inner ? r.map3[s] : r.map5, taps, 1, w, bias, cout, out, r.stream);
+    const bool wide = form == PTV3_CONV_PAIRS_WIDE;
+    const size_t mark = r.mem.at;
+    void* y = r.mem.take((size_t)n_pairs * cout * (wide ? 4 : r.es));
+    r.mem.at = mark;
+    if (r.dry) return PTV3_OK;
+    if (wide)
+        return ptv3_subm_conv_pairs_wide_fwd(x, r.dt, v.n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot, w, bias, cout,
+                                             (float*)y, out, r.stream);
+    return ptv3_subm_conv_pairs_fwd(x, r.dt, v.n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot, w, bias, cout, y, out,
+                                    r.stream);
+}
+// the tap-major neighbour map of level s, for the whole forward
+int make_map(Run& r, int s, int ks, int32_t** map) {
+    const ptv3_level& v = r.lv[s];
+    *map = (int32_t*)r.mem.take((size_t)v.n * ks * ks * ks * sizeof(int32_t));
+    const size_t mark = r.mem.at, bytes = ptv3_kmap_workspace_bytes(v.n);
+    void* ws = r.mem.take(bytes);
+    r.mem.at = mark;
+    return r.dry ? PTV3_OK : ptv3_kmap_build(v.indices, v.n, ks, 1, *map, ws, bytes, r.stream);
+}
+int stem_inputs(const ptv3_net& net) { return net.dtype == PTV3_F32 ? net.stem_in : (net.stem_in + 15) / 16 * 16; }
+int make_maps(Run& r) {
+    const ptv3_net& net = *r.net;
+    if (pair_form(r, 0, 125, stem_inputs(net), net.stage[0].channels) == PTV3_CONV_DENSE) TRY(make_map(r, 0, 5, &r.map5));
+    for (int s = 0; s < net.n_stages; ++s) {
+        const ptv3_stage_w& st = net.stage[s];
+        bool need = false;
+        for (int side = 0; side < 2; ++side) {
+            const int c = side ? st.dec_channels : st.channels;
+            if (!(side ? net.decoder && st.n_dec : st.n_enc)) continue;
+            if (r.dt != PTV3_F32 && ptv3_conv_form(r.lv[s].n, r.lv[s].n_pairs, c) != 0) continue;
+            need |= pair_form(r, s, 27, c, c) == PTV3_CONV_DENSE;
+        }
+        if (need) TRY(make_map(r, s, 3, &r.map3[s]));
     }
+    return PTV3_OK;
+}
+
+int conv3(Run& r, const ptv3_block_w& b, int s, const void* x, void* out) {
+    const int c = b.channels;
+    const ptv3_level& v = r.lv[s];
+    const int form = r.dt == PTV3_F32 ? 0 : ptv3_conv_form(v.n, v.n_pairs, c);
+    if (form == 0) return conv_rows(r, s, 27, x, c, b.conv_w, b.conv_b, c, out);
     if (r.dry) return PTV3_OK;
     if (form == 1)
         return ptv3_subm_conv_sparse_fwd(x, r.dt, v.n, c, 27, b.conv_packed, b.conv_b, v.tile_tap, v.tile_pair, out, r.stream);
@@ -102,7 +146,9 @@ int attention(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, con
 }
 
 // A block (model.py:586-606): x its rows, xs what its convolution reads, out the new rows.
-int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, const void* xs, const void* x, void* out) {
+int block_half(Run& r, const ptv3_block_w& b, int s, const void* xs, const void* x, void* out) {
+    const ptv3_level& v = r.lv[s];
+    const int patch = r.net->patch[s];
     const int64_t n = v.n;
     const int c = b.channels;
     const size_t mark = r.mem.at;
@@ -110,7 +156,7 @@ int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, co
     const bool few = ptv3_block_tail_few_pays(n, c);
     const size_t few_bytes = few ? ptv3_block_tail_few_bytes(n, c) : 0;
     void* few_ws = few ? r.mem.take(few_bytes) : nullptr;
-    TRY(conv3(r, b, v, xs, conv));
+    TRY(conv3(r, b, s, xs, conv));
     if (!r.dry) {
         if (c <= 64) {
             TRY(ptv3_block_head_fused(conv, x, b.cpe.w, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b, b.ln1.eps,
@@ -151,14 +197,16 @@ int block_half(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, co
 }
 
 // the same in a float model: the attention works in half (model.py:477, :483), everything else in float
-int block_float(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, const void* xs, const void* x, void* out) {
+int block_float(Run& r, const ptv3_block_w& b, int s, const void* xs, const void* x, void* out) {
+    const ptv3_level& v = r.lv[s];
+    const int patch = r.net->patch[s];
     const int64_t n = v.n;
     const int c = b.channels;
     const size_t mark = r.mem.at;
     void *conv = r.rows(n, c), *feat = r.rows(n, c), *normed = r.rows(n, c), *hidden = r.rows(n, 4 * c);
     void* qkv = r.mem.take((size_t)n * 3 * c * 2);
     void* attn = r.mem.take((size_t)n * c * 2);
-    TRY(conv3(r, b, v, xs, conv));
+    TRY(conv3(r, b, s, xs, conv));
     if (!r.dry) {
         TRY(linear(r, conv, b.cpe, n, hidden));
         TRY(ptv3_layer_norm(hidden, x, b.ln_cpe.g, b.ln_cpe.b, b.ln1.g, b.ln1.b, nullptr, r.dt, n, c, b.ln_cpe.eps, 3, feat, normed,
@@ -180,19 +228,19 @@ int block_float(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, c
     return PTV3_OK;
 }
 
-int block(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, const void* xs, const void* x, void* out) {
-    return r.dt == PTV3_F32 ? block_float(r, b, v, patch, xs, x, out) : block_half(r, b, v, patch, xs, x, out);
+int block(Run& r, const ptv3_block_w& b, int s, const void* xs, const void* x, void* out) {
+    return r.dt == PTV3_F32 ? block_float(r, b, s, xs, x, out) : block_half(r, b, s, xs, x, out);
 }
 
 // blocks of a stage from (xs, x); the last one writes `out` (n, channels)
-int blocks(Run& r, const ptv3_block_w* bs, int count, const ptv3_level& v, int patch, const void* xs, const void* x, void* out) {
+int blocks(Run& r, const ptv3_block_w* bs, int count, int s, const void* xs, const void* x, void* out) {
     if (count == 0) return PTV3_OK;
     const size_t mark = r.mem.at;
     void* tmp[2] = {nullptr, nullptr};
-    for (int i = 0; i < 2 && i < count - 1; ++i) tmp[i] = r.rows(v.n, bs[0].channels);
+    for (int i = 0; i < 2 && i < count - 1; ++i) tmp[i] = r.rows(r.lv[s].n, bs[0].channels);
     for (int i = 0; i < count; ++i) {
         void* to = i == count - 1 ? out : tmp[i & 1];
-        TRY(block(r, bs[i], v, patch, xs, x, to));
+        TRY(block(r, bs[i], s, xs, x, to));
         xs = x = to;
     }
     r.mem.at = mark;
@@ -202,6 +250,7 @@ int blocks(Run& r, const ptv3_block_w* bs, int count, const ptv3_level& v, int p
 int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, void* out) {
     const ptv3_net& net = *r.net;
     const int S = net.n_stages;
+    TRY(make_maps(r));
     // ---- stem: 5x5x5 convolution, BatchNorm, GELU (model.py:753-783)
     void* level_rows[PTV3_MAX_LEVELS] = {};
     for (int s = 0; s < S; ++s) {
@@ -215,22 +264,17 @@ int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, vo
     {
         const size_t m2 = r.mem.at;
         const void* in = feat;
-        int cin = net.stem_in;
+        const int cin = stem_inputs(net);
         if (r.dt != PTV3_F32) {   // the matrix cores take input channels 16 at a time
-            const int padded = (cin + 15) / 16 * 16;
-            void* p = r.rows(n0, padded);
-            if (!r.dry) TRY(ptv3_pad_rows(feat, feat_dtype, n0, cin, padded, p, r.dt, r.stream));
+            void* p = r.rows(n0, cin);
+            if (!r.dry) TRY(ptv3_pad_rows(feat, feat_dtype, n0, net.stem_in, cin, p, r.dt, r.stream));
             in = p;
-            cin = padded;
         }
-        void* y = r.rows(r.lv[0].n_pairs5, c0);
         void* z = r.rows(n0, c0);
-        if (!r.dry) {
-            TRY(ptv3_subm_conv_pairs_fwd(in, r.dt, n0, cin, 125, r.lv[0].n_pairs5, r.lv[0].tap_ptr5, r.lv[0].row_ptr5,
-                                         r.lv[0].pair_in5, r.lv[0].pair_slot5, net.stem_w, nullptr, c0, y, z, r.stream));
+        TRY(conv_rows(r, 0, 125, in, cin, net.stem_w, nullptr, c0, z));
+        if (!r.dry)
             TRY(ptv3_bn_act(z, net.stem_bn.mean, net.stem_bn.var, net.stem_bn.stats_f32, net.stem_bn.g, net.stem_bn.b, r.dt, n0, c0,
                             net.stem_bn.eps, 1, x, r.stream));
-        }
         r.mem.at = m2;
     }
     // ---- encoder
@@ -251,7 +295,7 @@ int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, vo
             }
             r.mem.at = m2;
         }
-        TRY(blocks(r, st.enc, st.n_enc, v, net.patch[s], x, x, level_rows[s]));
+        TRY(blocks(r, st.enc, st.n_enc, s, x, x, level_rows[s]));
     }
     r.mem.at = mark;
     if (!net.decoder) return PTV3_OK;
@@ -278,7 +322,7 @@ int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, vo
         } else {
             if (!r.dry) TRY(ptv3_unpool_add(skip, p, r.dt, v.n, c, below.cluster, below.n, sum, r.stream));
             // the first block's convolution reads the skip projection alone (model.py:746)
-            TRY(blocks(r, st.dec, st.n_dec, v, net.patch[s], skip, sum, to));
+            TRY(blocks(r, st.dec, st.n_dec, s, skip, sum, to));
         }
         child = to;
         r.mem.at = m2;
@@ -308,7 +352,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const TI* __restrict__ x,
 
 bool net_ok(const ptv3_net* net, const ptv3_level* lv) {
     if (!net || !lv || net->n_stages < 1 || net->n_stages > PTV3_MAX_LEVELS || net->stem_in < 1) return false;
-    if (net->dtype < PTV3_F32 || net->dtype > PTV3_BF16) return false;
+    if (net->dtype < PTV3_F32 || net->dtype > PTV3_BF16 || !(net->max_pair_density >= 0.f)) return false;
     for (int s = 0; s < net->n_stages; ++s) {
         const ptv3_stage_w& st = net->stage[s];
         if (lv[s].n < 1 || st.n_enc < 0 || st.n_dec < 0 || (st.n_enc && !st.enc) || (st.n_dec && !st.dec)) return false;

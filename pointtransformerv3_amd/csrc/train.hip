@@ -69,6 +69,8 @@ struct Run {
     BlockActs pool[MAX_BLOCKS];
     BnActs stem_bn;
     void *stem_in, *stem_x;     // padded input rows, the stem's rows
+    int32_t *map3[PTV3_MAX_LEVELS] = {}, *map5 = nullptr;   // neighbour maps of levels whose convolutions take the dense form
+    bool has_map3[PTV3_MAX_LEVELS] = {};
     Run(const ptv3_train_net& n, const ptv3_level* l, void* s) : net(n), lv(l), stream(s), hs((hipStream_t)s), dt(n.dtype) {}
 
     void place_bn(Space& m, BnActs& b, int64_t n, int c) {
@@ -115,6 +117,7 @@ struct Run {
             st[s].dec = next;
             for (int i = 0; i < g.n_dec; ++i) place_block(m, *next++, g.dec[i], lv[s]);
         }
+        place_maps(m);
     }
 
     // what each block's convolution reads
@@ -147,16 +150,64 @@ struct Run {
         if (form == 2)
             return ptv3_subm_conv_tiles_fwd_sized(x, dt, v.n, c, 27, v.tile_voxels, packed, bias, v.tile_tap, v.tile_pair,
                                                   v.vox_taps, out, stream);
+        return conv_rows((int)(&v - lv), 27, x, c, w, bias, c, out, scratch);
+    }
+    // one that no tile form takes, as in features.hip; the neighbour maps of the dense form lie beside the activations
+    int pair_form(int s, int taps, int cin, int cout) const {
+        const ptv3_level& v = lv[s];
+        return ptv3_conv_pair_form(dt, v.n, taps == 27 ? v.n_pairs : v.n_pairs5, taps, cin, cout, net.max_pair_density);
+    }
+    int conv_rows(int s, int taps, const void* x, int cin, const void* w, const void* bias, int cout, void* out, Space& scratch) {
+        const ptv3_level& v = lv[s];
+        const bool inner = taps == 27;
+        const int64_t n_pairs = inner ? v.n_pairs : v.n_pairs5;
+        const int32_t *tap_ptr = inner ? v.tap_ptr : v.tap_ptr5, *row_ptr = inner ? v.row_ptr : v.row_ptr5;
+        const int32_t *pair_in = inner ? v.pair_in : v.pair_in5, *pair_slot = inner ? v.pair_slot : v.pair_slot5;
+        const int form = pair_form(s, taps, cin, cout);
+        if (form == PTV3_CONV_DENSE) {
+            DO(ptv3_subm_conv_fwd(x, dt, v.n, cin, inner ? map3[s] : map5, taps, 1, w, bias, cout, out, stream));
+            return PTV3_OK;
+        }
+        const bool wide = form == PTV3_CONV_PAIRS_WIDE;
         const size_t mark = scratch.at;
-        const bool wide = ptv3_conv_few_pairs(v.n_pairs, c);
-        void* y = scratch.take((size_t)v.n_pairs * c * (wide ? 4 : 2));
-        if (wide)
-            DO(ptv3_subm_conv_pairs_wide_fwd(x, dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, w, bias,
-                                             (float*)y, out, stream));
-        else
-            DO(ptv3_subm_conv_pairs_fwd(x, dt, v.n, c, 27, v.n_pairs, v.tap_ptr, v.row_ptr, v.pair_in, v.pair_slot, w, bias, c, y,
-                                        out, stream));
+        void* y = scratch.take((size_t)n_pairs * cout * (wide ? 4 : 2));
         scratch.at = mark;
+        if (dry) return PTV3_OK;
+        if (wide)
+            return ptv3_subm_conv_pairs_wide_fwd(x, dt, v.n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot, w, bias, cout,
+                                                 (float*)y, out, stream);
+        return ptv3_subm_conv_pairs_fwd(x, dt, v.n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot, w, bias, cout, y, out,
+                                        stream);
+    }
+    bool dense3(int s) const {
+        const ptv3_train_stage& g = net.stage[s];
+        for (int side = 0; side < 2; ++side) {
+            const int c = side ? g.dec_channels : g.channels;
+            if ((side ? g.n_dec : g.n_enc) && ptv3_conv_form(lv[s].n, lv[s].n_pairs, c) == 0 &&
+                pair_form(s, 27, c, c) == PTV3_CONV_DENSE)
+                return true;
+        }
+        return false;
+    }
+    void place_maps(Space& m) {
+        if (pair_form(0, 125, net.stem.cin_padded, net.stage[0].channels) == PTV3_CONV_DENSE)
+            map5 = (int32_t*)m.take((size_t)lv[0].n * 125 * 4);
+        for (int s = 0; s < net.n_stages; ++s) {
+            has_map3[s] = dense3(s);
+            if (has_map3[s]) map3[s] = (int32_t*)m.take((size_t)lv[s].n * 27 * 4);
+        }
+    }
+    int make_map(int s, int ks, int32_t* map, Space& scratch) {
+        const size_t mark = scratch.at, bytes = ptv3_kmap_workspace_bytes(lv[s].n);
+        void* ws = scratch.take(bytes);
+        scratch.at = mark;
+        DO(ptv3_kmap_build(lv[s].indices, lv[s].n, ks, 1, map, ws, bytes, stream));
+        return PTV3_OK;
+    }
+    int make_maps(Space& scratch) {   // by the forward; the backward finds them where they were placed
+        if (pair_form(0, 125, net.stem.cin_padded, net.stage[0].channels) == PTV3_CONV_DENSE) TRY(make_map(0, 5, map5, scratch));
+        for (int s = 0; s < net.n_stages; ++s)
+            if (has_map3[s]) TRY(make_map(s, 3, map3[s], scratch));
         return PTV3_OK;
     }
 
@@ -218,11 +269,8 @@ struct Run {
         const ptv3_level& v0 = lv[0];
         const int c0 = net.stage[0].channels;
         DO(ptv3_pad_rows(feat, feat_dt, v0.n, net.stem.cin, net.stem.cin_padded, stem_in, dt, stream));
-        const size_t mark = scratch.at;
-        void* y = scratch.take((size_t)v0.n_pairs5 * c0 * 2);
-        DO(ptv3_subm_conv_pairs_fwd(stem_in, dt, v0.n, net.stem.cin_padded, 125, v0.n_pairs5, v0.tap_ptr5, v0.row_ptr5, v0.pair_in5,
-                                     v0.pair_slot5, net.stem.w, nullptr, c0, y, stem_bn.x, stream));
-        scratch.at = mark;
+        TRY(make_maps(scratch));
+        TRY(conv_rows(0, 125, stem_in, net.stem.cin_padded, net.stem.w, nullptr, c0, stem_bn.x, scratch));
         TRY(bn_gelu(net.stem.bn, stem_bn, v0.n, c0, scratch));
         const void* x = stem_bn.y;
         for (int s = 0; s < S; ++s) {
@@ -463,7 +511,7 @@ __global__ __launch_bounds__(256) void cut_rows_kernel(const float* __restrict__
 
 bool net_ok(const ptv3_train_net* net, const ptv3_level* lv) {
     if (!net || !lv || net->n_stages < 2 || net->n_stages > PTV3_MAX_LEVELS) return false;
-    if (net->dtype != PTV3_F16 && net->dtype != PTV3_BF16) return false;
+    if ((net->dtype != PTV3_F16 && net->dtype != PTV3_BF16) || !(net->max_pair_density >= 0.f)) return false;
     int blocks = 0;
     for (int s = 0; s < net->n_stages; ++s) {
         const ptv3_train_stage& g = net->stage[s];

@@ -50,7 +50,7 @@ class _Stage(ctypes.Structure):
 
 class _Net(ctypes.Structure):
     _fields_ = [("dtype", _i32), ("n_stages", _i32), ("decoder", _i32), ("stem_in", _i32), ("patch", _i32 * levels.MAX_LEVELS),
-                ("stem_w", _ptr), ("stem_bn", _Bn), ("stage", _Stage * levels.MAX_LEVELS)]
+                ("max_pair_density", _f32), ("reserved", _f32), ("stem_w", _ptr), ("stem_bn", _Bn), ("stage", _Stage * levels.MAX_LEVELS)]
 
 
 class _Refresh(ctypes.Structure):
@@ -117,6 +117,7 @@ class Structure:
             self.why = "a method was replaced"
         self.hooks = [d for m in (model, *self.modules) for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
                                                                   m._backward_pre_hooks)]
+        self.density = SubMConv3d.PAIR_MODE_MAX_DENSITY
         self._attributes, self._n_orders = model.__dict__, len(model.order)
         self._types = list(map(type, self.modules))
         self._forwards = [(t, t.forward) for t in set(self._types)]
@@ -168,6 +169,7 @@ class Structure:
         try:
             return (list(map(len, self._sized)) == self._sizes and list(map(type, self.modules)) == self._types
                     and all(t.forward is f for t, f in self._forwards) and len(self._attributes["order"]) == self._n_orders
+                    and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
                     and all(map(operator.is_, map(operator.getitem, *self._child_at), self._children))
                     and [f(d) for f, d in self._reads] == self._values
                     and all(map(operator.is_, map(operator.getitem, *self._slots), self._held))
@@ -195,7 +197,7 @@ def _check_gelu(m):
 
 
 def _check_conv(m, kernel_size, biased):
-    _need(m.kernel_size == kernel_size and (m.bias is not None) == biased
+    _need(m.kernel_size == kernel_size and m.PAIR_MODE_MAX_DENSITY == SubMConv3d.PAIR_MODE_MAX_DENSITY and (m.bias is not None) == biased
           and tuple(m.weight.shape) == (m.out_channels, *[kernel_size] * 3, m.in_channels)
           and (m.bias is None or m.bias.shape == (m.out_channels,)), "convolution")
 
@@ -446,7 +448,7 @@ class Engine(Copies):
     def _describe(self, model, p):
         """ptv3_net of the model, p its Parts; Unsupported where it is not the default architecture."""
         net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages), decoder=int(not model.cls_mode))
-        net.stem_in = p.stem_conv.in_channels
+        net.stem_in, net.max_pair_density = p.stem_conv.in_channels, self.structure.density
         net.stem_w = self._p(p.stem_conv.weight)
         net.stem_bn = self._bn(p.stem_bn, p.stem_conv.out_channels)
         self._refresh = r = _Refresh(dtype=net.dtype)

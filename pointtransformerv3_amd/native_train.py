@@ -49,7 +49,8 @@ class _Stem(ctypes.Structure):
 
 
 class _Net(ctypes.Structure):
-    _fields_ = [("dtype", _i32), ("n_stages", _i32), ("patch", _i32 * levels.MAX_LEVELS), ("stem", _Stem), ("zero", _ptr),
+    _fields_ = [("dtype", _i32), ("n_stages", _i32), ("patch", _i32 * levels.MAX_LEVELS),
+                ("max_pair_density", _f32), ("reserved2", _f32), ("stem", _Stem), ("zero", _ptr),
                 ("n_zero", _i32), ("reserved", _i32), ("zero_blocks", _i64), ("stage", _Stage * levels.MAX_LEVELS)]
 
 
@@ -141,7 +142,7 @@ class TrainEngine(native.Copies):
 
     def _describe(self, model, p):
         _need(all(st.enc for st in p.stages) and all(st.dec for st in p.stages[:-1]), "a stage without blocks")
-        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages))
+        net = self.net = _Net(dtype=ops.DTYPE_CODES[self.dtype], n_stages=len(p.stages), max_pair_density=self.structure.density)
         conv = p.stem_conv
         padded = -(-conv.in_channels // 16) * 16
         net.stem.w = self._buffer(conv.out_channels * 125 * padded)

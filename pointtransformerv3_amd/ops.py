@@ -852,8 +852,7 @@ def conv_plan_direct(indices, ks):
 
 
 def subm_conv_pairs(feat, plan, weight, bias=None, wide=False):
-    """Submanifold convolution over the plan's active pairs only. wide: product rows in float also for half-precision rows
-    (64 or 128 channels)."""
+    """Submanifold convolution over the plan's active pairs only. wide: product rows in float also for half-precision rows."""
     _dev(feat, weight, bias)
     lib = _lib.load()
     feat = feat.contiguous()
@@ -863,13 +862,12 @@ def subm_conv_pairs(feat, plan, weight, bias=None, wide=False):
     b = None if bias is None else bias.to(feat.dtype).contiguous()
     y = torch.empty((max(plan.n_pairs, 1), cout), dtype=torch.float32 if wide else feat.dtype, device=feat.device)
     out = torch.empty((n, cout), dtype=feat.dtype, device=feat.device)
-    assert not wide or cin == cout
 
     def call():
         if wide:
             _lib.check(lib.ptv3_subm_conv_pairs_wide_fwd(_ptr(feat), _dtype_code(feat), n, cin, plan.taps, plan.n_pairs,
                                                          _ptr(plan.tap_ptr), _ptr(plan.row_ptr), _ptr(plan.pair_in),
-                                                         _ptr(plan.pair_slot), _ptr(w), _ptr(b), _ptr(y), _ptr(out),
+                                                         _ptr(plan.pair_slot), _ptr(w), _ptr(b), cout, _ptr(y), _ptr(out),
                                                          _stream()), "ptv3_subm_conv_pairs_wide_fwd")
             return
         _lib.check(lib.ptv3_subm_conv_pairs_fwd(_ptr(feat), _dtype_code(feat), n, cin, plan.taps, plan.n_pairs,
@@ -884,6 +882,7 @@ def subm_conv_pairs(feat, plan, weight, bias=None, wide=False):
     return out
 
 
+CONV_PAIRS, CONV_PAIRS_WIDE, CONV_DENSE = range(3)   # ptv3_conv_pair_form
 CONV_TILE_CHANNELS = (64, 128)   # cin == cout widths of the tile form of the 3x3x3 convolution
 
 

@@ -75,9 +75,8 @@ class SubMConv3d(nn.Module):
     (out, k, k, k, in) layout so checkpoints keep loading; `padding` is accepted and unused,
     as submanifold convolutions are centred by construction."""
 
-    # above this fraction of active (voxel, tap) pairs the dense output-stationary kernel is used
-    # (no pair-matrix round trip, but MFMA work for every tap); a 2 cm surface scan goes from 0.05
-    # at full resolution to 0.5 at the coarsest level, where the two forms measure about equal
+    # above this fraction of active (voxel, tap) pairs product rows are avoided (ptv3_conv_pair_form): a 2 cm surface scan
+    # goes from 0.05 at full resolution to 0.5 at the coarsest level, where pair and dense form measure about equal
     PAIR_MODE_MAX_DENSITY = 0.6
 
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, padding=0, dilation=1,
@@ -133,25 +132,26 @@ class SubMConv3d(nn.Module):
 
     def convolve(self, x, feat, weight, bias, packed=None):
         """The convolution of feat (N, Cin) over x's neighbourhoods with weight (Cout, V, Cin), on whichever
-        form fits: pair lists (always in fp32), dense output-stationary (many active taps), tiles, or sparse tiles.
+        form fits: pair lists, dense output-stationary (many active taps), tiles, or sparse tiles.
         packed() hands out the weight in the tile kernels' order when the caller has it cached."""
         cout, _, cin = weight.shape
-        if feat.dtype == torch.float32:   # fp32 MFMA over the active pairs
-            return ops.subm_conv_pairs(feat, x.conv_plan(self.kernel_size, self.indice_key), weight, bias)
-        if cin % 16 != 0:
+        half = feat.dtype != torch.float32
+        plan = x.conv_plan(self.kernel_size, self.indice_key)
+        form = self._tile_form(plan, cin, cout) if half else None
+        if form is not None:
+            tiles = packed() if packed is not None else ops.conv_pack_weight(weight, 27, feat.dtype)
+            return (ops.subm_conv_sparse if form == "sparse" else ops.subm_conv_tiles)(feat, plan, tiles, bias)
+        if half and cin % 16 != 0:
             # the MFMA kernels consume input channels 16 at a time: zero-pad the thin stem input
             pad = 16 - cin % 16
             feat = nn.functional.pad(feat, (0, pad))
             weight = nn.functional.pad(weight, (0, pad))
-        plan = x.conv_plan(self.kernel_size, self.indice_key)
-        form = self._tile_form(plan, cin, cout)
-        if form is not None:
-            tiles = packed() if packed is not None else ops.conv_pack_weight(weight, 27, feat.dtype)
-            return (ops.subm_conv_sparse if form == "sparse" else ops.subm_conv_tiles)(feat, plan, tiles, bias)
+            cin += pad
         weight = weight.to(feat.dtype)
-        if plan.density() <= self.PAIR_MODE_MAX_DENSITY and cout % 8 == 0:
-            wide = self.kernel_size == 3 and cin == cout and _lib.load().ptv3_conv_few_pairs(plan.n_pairs, cin)
-            return ops.subm_conv_pairs(feat, plan, weight, bias, wide=bool(wide))
+        rows = _lib.load().ptv3_conv_pair_form(ops.DTYPE_CODES[feat.dtype], plan.n, plan.n_pairs, plan.taps, cin, cout,
+                                               self.PAIR_MODE_MAX_DENSITY)
+        if rows != ops.CONV_DENSE:
+            return ops.subm_conv_pairs(feat, plan, weight, bias, wide=rows == ops.CONV_PAIRS_WIDE)
         return ops.subm_conv(feat, x.neighbour_map(self.kernel_size, self.indice_key), weight, bias, tap_major=True)
 
     def forward(self, x):

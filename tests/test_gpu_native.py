@@ -193,3 +193,36 @@ def test_copies_outlive_their_engine_where_another_stream_reads_them(train):
     torch.cuda.synchronize()
     wanted = [(t.data_ptr(), side.cuda_stream) for t in copies]
     assert [m for m in marked if m in wanted] == wanted      # each of them, once
+
+
+def _volume(extent, dtype, fill=1.0):
+    """A solid block of voxels: most taps of most voxels are there."""
+    g = np.stack(np.meshgrid(*[np.arange(extent)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    g = g[np.random.default_rng(extent).random(len(g)) < fill].astype(np.int32)
+    gen = torch.Generator(device=DEV).manual_seed(extent)
+    return dict(feat=torch.randn(len(g), 6, generator=gen, device=DEV).to(dtype), grid_coord=torch.from_numpy(g).to(DEV),
+                offset=torch.tensor([len(g)], device=DEV))
+
+
+@pytest.mark.parametrize("extent,fill", [(12, 1.0), (32, 1.0), (32, 0.8)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_native_forward_takes_the_modules_forms_in_dense_volumes(dtype, extent, fill, monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3, ops
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().to(dtype).to(DEV)
+    dense, real = [], ops.subm_conv
+    monkeypatch.setattr(ops, "subm_conv", lambda x, *a, **k: dense.append(x.shape) or real(x, *a, **k))
+    got, want = _both(model, _volume(extent, dtype, fill), monkeypatch)
+    assert torch.equal(got.feat, want.feat)
+    assert bool(dense) == (dtype == torch.float16 and extent == 32)
+
+
+def test_dense_volumes_follow_the_module_class_setting(monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3, SubMConv3d
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().half().to(DEV)
+    data = _volume(32, torch.float16)
+    first = _both(model, data, monkeypatch)[0].feat
+    monkeypatch.setattr(SubMConv3d, "PAIR_MODE_MAX_DENSITY", 1.0)
+    got, want = _both(model, data, monkeypatch)
+    assert torch.equal(got.feat, want.feat) and not torch.equal(got.feat, first)

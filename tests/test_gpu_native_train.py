@@ -227,3 +227,13 @@ def test_native_training_step_follows_a_momentum_schedule(monkeypatch):
     model.enc.enc1.down.norm[0].momentum = None
     with torch.autocast("cuda", dtype=torch.float16):
         assert native_train.engine_for(model, data) is None
+
+
+@pytest.mark.parametrize("extent", [18, 32])
+def test_native_training_step_in_dense_volumes(extent, monkeypatch):
+    """Float rows in the small volume, the neighbour map in the large one: forward and input gradients as the modules'."""
+    from pointtransformerv3_amd import PointTransformerV3
+    from test_gpu_native import _volume
+    torch.manual_seed(3)
+    model = PointTransformerV3(drop_path=0.0, **KW).to(DEV).train()
+    _compare(model, _volume(extent, torch.float32), torch.float16, monkeypatch, 2e-2)

@@ -77,6 +77,38 @@ def test_convolution_of_few_pairs_rounds_once(c, n, extent, dtype):
     assert torch.equal(ops.subm_conv_pairs(x, plan, w, None, wide=True), ops.subm_conv_pairs(x, plan, w, torch.zeros_like(bias), wide=True))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("ks,cin,cout,n,extent", [(3, 32, 32, 1700, 12), (3, 256, 256, 900, 10), (3, 512, 512, 500, 8), (5, 16, 32, 1000, 10),
+                                                  (3, 16, 8, 65, 5), (3, 48, 40, 300, 8), (3, 128, 200, 300, 8), (3, 512, 64, 200, 7)])
+def test_pair_form_with_float_rows_rounds_once(ks, cin, cout, n, extent, dtype):
+    """The shapes that take it in small dense volumes, and the edges of what it takes, against 64 bits: below one rounding."""
+    import numpy as np
+
+    from pointtransformerv3_amd import ops
+    grid, batch, _ = unique_voxels(np.random.default_rng(n), n, extent)
+    idx = to_dev(np.concatenate([batch[:, None], grid], 1).astype(np.int32))
+    g = torch.Generator(device=DEV).manual_seed(n)
+    taps = ks ** 3
+    x = torch.randn(n, cin, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(cout, taps, cin, generator=g, device=DEV) / (taps * cin) ** 0.5).to(dtype)
+    bias = torch.randn(cout, generator=g, device=DEV).to(dtype)
+    want = bias.double().expand(n, cout).clone()
+    nbr = ops.kmap_build(idx, ks).long()
+    for t in range(taps):
+        on = nbr[:, t] >= 0
+        want[on] += x.double()[nbr[on, t]] @ w[:, t].double().t()
+    got = ops.subm_conv_pairs(x, ops.conv_plan_direct(idx, ks), w, bias, wide=True)
+    assert float((got.double() - want).norm() / want.norm()) < 0.5 * torch.finfo(dtype).eps
+
+
+def test_pair_form_with_float_rows_refuses_other_shapes():
+    from pointtransformerv3_amd import _lib
+    lib, x = _lib.load(), torch.zeros(64, device=DEV)
+    call = lambda dt, cin, cout, taps=27: lib.ptv3_subm_conv_pairs_wide_fwd(x.data_ptr(), dt, 1, cin, taps, 0, x.data_ptr(), x.data_ptr(),
+                                                                           0, 0, x.data_ptr(), 0, cout, 0, x.data_ptr(), None)
+    assert all(call(*a) != 0 for a in ((0, 64, 64), (1, 24, 64), (1, 64, 12), (1, 96, 96), (1, 528, 64), (1, 64, 64, 129), (1, 0, 64)))
+
+
 @pytest.mark.parametrize("n", [2000, 6000])
 def test_few_pairs_in_model_and_training_take_float_rows(n, monkeypatch):
     """SubMConv3d in inference and both directions of its training ask for them where the rule says so."""

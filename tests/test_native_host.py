@@ -133,7 +133,7 @@ def test_checkpointed_step_is_held_against_the_weights_it_was_computed_again_wit
 def _described(model):
     """A TrainEngine's description of a model on the CPU (nothing is launched; placement is not looked at)."""
     engine = native_train.TrainEngine.__new__(native_train.TrainEngine)
-    engine.dtype, engine.device = torch.float16, torch.device("cpu")
+    engine.dtype, engine.device, engine.structure = torch.float16, torch.device("cpu"), native.Structure(model)
     engine._keep, engine._casts, engine._packs, engine._zero, engine.read_back = [], [], [], [], []
     engine.params, engine._placed, engine.total, engine._norms = [], set(), 0, []
     engine._describe(model, native.Parts(model))
@@ -285,9 +285,7 @@ def test_a_described_or_refused_model_is_let_go():
 
 
 def _engine_of(model):
-    engine = _described(model)
-    engine.structure = native.Structure(model)
-    return engine
+    return _described(model)
 
 
 class _OwnStem(torch.nn.Module):
@@ -345,3 +343,29 @@ def test_index_tables_are_apart_from_the_scratch(n):
     assert lib.ptv3_index_begin_bytes(ctypes.byref(cfg), ctypes.byref(tables), ctypes.byref(scratch)) == 0
     assert 16 * n <= tables.value <= 16 * n + 4096 and scratch.value >= 100 * n
     assert lib.ptv3_index_begin_bytes(ctypes.byref(cfg), None, ctypes.byref(scratch)) != 0
+
+
+def test_rule_of_convolutions_that_no_tile_form_takes():
+    """Few pairs and small dense volumes: float rows; larger dense volumes: the neighbour map; else half rows. Float: pair
+    rows unless a dense volume's would take more than 32 GiB."""
+    from pointtransformerv3_amd import _lib, ops
+    form = _lib.load().ptv3_conv_pair_form
+    f32, f16 = ops.DTYPE_CODES[torch.float32], ops.DTYPE_CODES[torch.float16]
+    few = _lib.load().ptv3_conv_few_pairs
+    for c in (64, 128):
+        line = max(p for p in range(1000, 400_000, 1000) if few(p, c))
+        assert form(f16, 10_000_000, line, 27, c, c, 0.6) == form(f16, line // 27, line, 27, c, c, 0.6) == ops.CONV_PAIRS_WIDE
+        assert form(f16, 10_000_000, line + 1000, 27, c, c, 0.6) == ops.CONV_PAIRS
+    for c in (32, 256, 512):
+        assert form(f16, 1000, 16_000, 27, c, c, 0.6) == ops.CONV_PAIRS
+        assert form(f16, 1000, 16_300, 27, c, c, 0.6) == form(f16, 9000, 229_500, 27, c, c, 0.6) == ops.CONV_PAIRS_WIDE
+        assert form(f16, 9000, 229_501, 27, c, c, 0.6) == ops.CONV_DENSE
+        assert form(f16, 9000, 229_501, 27, c, c, 1.0) == ops.CONV_PAIRS
+    assert form(f16, 9000, 1_000_000, 125, 16, 32, 0.6) == ops.CONV_PAIRS_WIDE
+    assert form(f16, 12_000, 1_100_000, 125, 16, 32, 0.6) == ops.CONV_DENSE
+    assert form(f16, 1000, 20_000, 27, 48, 96, 0.6) == ops.CONV_DENSE      # no float rows of this shape
+    assert form(f16, 1000, 2_000, 27, 32, 12, 0.6) == ops.CONV_DENSE       # outputs not in 8s
+    assert form(f32, 10_000_000, 27 * 10_000_000, 27, 31, 31, 0.6) == ops.CONV_PAIRS
+    assert form(f32, 10_000_000, 27 * 10_000_000, 27, 32, 32, 0.6) == ops.CONV_DENSE
+    assert form(f32, 100_000_000, 27 * 10_000_000, 27, 512, 512, 0.6) == ops.CONV_PAIRS
+    assert form(f16, 0, 0, 27, 32, 32, 0.6) == ops.CONV_PAIRS
