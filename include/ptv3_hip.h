@@ -96,6 +96,10 @@ size_t ptv3_argsort_workspace_bytes(int64_t n, int k);
 int ptv3_argsort(const int64_t *code, int64_t n, int k, int key_bits, int64_t *order,
                  int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);
 
+/* ptv3_argsort whose tiles wait at most spin_limit polls for the counts of the tiles in front of them before they count
+ * those keys themselves (negative: they never wait). Same result, slower; what ptv3_argsort does after seconds. */
+int ptv3_argsort_impatient(const int64_t *code, int64_t n, int k, int key_bits, int spin_limit, int64_t *order,
+                           int64_t *inverse, void *workspace, size_t workspace_bytes, void *stream);
 /* ptv3_encode and ptv3_argsort of the codes in one call (the codes are counted where they are made); workspace as
  * ptv3_argsort's. key_bits covers the curve bits and the scene bits above them. */
 int ptv3_serialize(const int32_t *grid_coord, const int64_t *batch, int64_t n, int depth,

@@ -23,6 +23,7 @@ SIGNATURES = {
     "ptv3_gather_rows": (_i32, [_vp, _vp, _vp, _i32, _vp, _i64, _vp]),
     "ptv3_offset2batch": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "ptv3_argsort_workspace_bytes": (_sz, [_i64, _i32]),
+    "ptv3_argsort_impatient": (_i32, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_argsort": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_serialize": (_i32, [_vp, _vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ptv3_pad_sizes": (_i32, [_vp, _i32, _i64, _vp, _vp]),

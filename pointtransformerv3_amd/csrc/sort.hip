@@ -19,7 +19,7 @@
 //                  status in the upper half, the count in the lower, and is written and read with device-scope atomics, so
 //                  that the pair is seen whole and seen across the XCDs' L2s. Work-groups are dispatched in launch
 //                  order, so everything a tile waits for is already running or done; the wait is bounded all the
-//                  same (a flag in the workspace is raised and the sort goes on, wrong, rather than hang).
+//                  same: a tile that has waited for seconds counts the keys in front of it itself.
 //                  The tile is put in digit order in LDS first, so that the global writes of one digit are
 //                  contiguous runs. Between passes a point travels as (key, 32-bit index); the key is cut to 32
 //                  bits where what later passes look at fits (the first pass drops its own digit).
@@ -38,7 +38,7 @@ constexpr int SORT_WAVES = SORT_THREADS / PTV3_WAVE;
 constexpr int MAX_RADIX = 512;
 constexpr int MAX_PASSES = 8;
 constexpr int GROUP = 8;              // tiles per group, and words read at a time
-constexpr int SPIN_LIMIT = 1 << 20;   // look-back polls before a tile gives up waiting (seconds; never reached)
+constexpr int SPIN_LIMIT = 1 << 20;   // look-back polls before a tile stops waiting (seconds; never reached)
 constexpr int SMALL_THREADS = 1024;
 // rows of one work-group: at 4,096 keys 15 us against 20 by the general path, at 8,192 (eight keys a thread) 28 against 23
 constexpr int SMALL_KEYS = 4096;
@@ -157,9 +157,10 @@ __device__ __forceinline__ uint32_t wave_inclusive(uint32_t x, int lane) {
 }
 
 // Sum of the counts of one digit in `count` (at most GROUP) words `step` apart, all read in one round trip, from
-// `p` downwards; stops at the first inclusive one when `stop` is given.
-template <typename W>
-__device__ __forceinline__ uint32_t look_sum(const W* p, int64_t step, int count, uint32_t s_counts, bool* stop, bool* timed_out) {
+// `p` downwards; stops at the first inclusive one when `stop` is given. recount(j): the count that word j stands for, from
+// the keys, where `limit` polls have not brought it (every word where limit is negative).
+template <typename W, typename Recount>
+__device__ __forceinline__ uint32_t look_sum(const W* p, int64_t step, int count, uint32_t s_counts, int limit, bool* stop, Recount recount) {
     constexpr W MASK = ((W)1 << HALF<W>) - 1;
     W w[GROUP];
 #pragma unroll
@@ -169,8 +170,11 @@ __device__ __forceinline__ uint32_t look_sum(const W* p, int64_t step, int count
 #pragma unroll
     for (int j = 0; j < GROUP; ++j) {
         if (closed || j >= count) continue;
-        for (int spin = 0; (uint32_t)(w[j] >> HALF<W>) < s_counts; ++spin) {
-            if (spin >= SPIN_LIMIT) { *timed_out = true; break; }
+        for (int spin = 0; limit < 0 || (uint32_t)(w[j] >> HALF<W>) < s_counts; ++spin) {
+            if (spin >= limit) {
+                w[j] = (W)s_counts << HALF<W> | recount(j);
+                break;
+            }
             __builtin_amdgcn_s_sleep(1);
             w[j] = look_load(p - j * step);
         }
@@ -187,7 +191,7 @@ template <typename K> struct __align__(2 * sizeof(K)) Keyed { K key; int32_t idx
 template <typename KL, typename KO, bool FIRST, bool LAST, int BITS, int ITEMS, bool ALL>
 __device__ __forceinline__ void scatter_tile(
     const void* __restrict__ in, int count, int tbase, int shift, int drop, int pass, uint32_t row_total, TileWord* my_word,
-    GroupWord* my_group, int tile, uint32_t* __restrict__ gave_up, Keyed<KO>* __restrict__ out, int64_t* __restrict__ order,
+    GroupWord* my_group, int tile, int spin_limit, Keyed<KO>* __restrict__ out, int64_t* __restrict__ order,
     int64_t* __restrict__ inverse, KO* __restrict__ sorted, uint32_t (*whist)[1 << BITS], uint32_t* gdelta, uint32_t* wsum,
     uint32_t* rsum, Keyed<KL>* stage) {
     constexpr int R = 1 << BITS;
@@ -221,16 +225,27 @@ __device__ __forceinline__ void scatter_tile(
     }
     __syncthreads();
     if (tid < R) {
-        bool timed_out = false;
         const int group = tile / GROUP, place = tile % GROUP;
+        // keys of this digit in `tiles` tiles from `from` on, all of them in front of this one and therefore full; the
+        // pass reads one buffer and writes another, so they stand whatever the other tiles are doing
+        auto keys_in = [&](int from, int tiles) {
+            constexpr int TILE = SORT_THREADS * ITEMS;
+            uint32_t found = 0;
+            for (int64_t i = (int64_t)from * TILE - tbase; i < (int64_t)(from + tiles) * TILE - tbase; ++i) {
+                const KL key = FIRST ? (KL)((const int64_t*)in)[i] : ((const Keyed<KL>*)in)[i].key;
+                found += ((uint32_t)(key >> shift) & (R - 1)) == (uint32_t)tid;
+            }
+            return found;
+        };
         uint32_t own = 0, before = 0;
-        if (place > 0) own = look_sum(my_word - R, R, place, s_counts, nullptr, &timed_out);
+        if (place > 0)
+            own = look_sum(my_word - R, R, place, s_counts, spin_limit, nullptr, [&](int j) { return keys_in(tile - 1 - j, 1); });
         if (place == GROUP - 1) look_store(my_group, group == 0 ? s_sums : s_counts, own + total);
         bool closed = false;
-        for (int g = group - 1; g >= 0 && !closed && !timed_out; g -= GROUP)
-            before += look_sum(my_group - (int64_t)(group - g) * R, R, g + 1 < GROUP ? g + 1 : GROUP, s_counts, &closed, &timed_out);
+        for (int g = group - 1; g >= 0 && !closed; g -= GROUP)
+            before += look_sum(my_group - (int64_t)(group - g) * R, R, g + 1 < GROUP ? g + 1 : GROUP, s_counts, spin_limit, &closed,
+                               [&](int j) { return keys_in((g - j) * GROUP, GROUP); });
         if (place == GROUP - 1 && group > 0) look_store(my_group, s_sums, before + own + total);
-        if (timed_out) atomicOr(gave_up, 1u);
         uint32_t start = x - total, rstart = rx - row_total;
         for (int w = 0; w < wave; ++w) { start += wsum[w]; rstart += rsum[w]; }
         gdelta[tid] = rstart + before + own - start;
@@ -265,7 +280,7 @@ __device__ __forceinline__ void scatter_tile(
 template <typename KL, typename KO, bool FIRST, bool LAST, int BITS, int ITEMS>
 __global__ __launch_bounds__(SORT_THREADS) void scatter_kernel(
     const void* __restrict__ in, int64_t n, int shift, int drop, int pass, const uint32_t* __restrict__ totals, TileWord* look,
-    GroupWord* glook, int tiles, int groups, uint32_t* __restrict__ gave_up, Keyed<KO>* __restrict__ out, int64_t* __restrict__ order,
+    GroupWord* glook, int tiles, int groups, int spin_limit, Keyed<KO>* __restrict__ out, int64_t* __restrict__ order,
     int64_t* __restrict__ inverse, KO* __restrict__ sorted) {
     constexpr int R = 1 << BITS, TILE = SORT_THREADS * ITEMS;
     __shared__ uint32_t whist[SORT_WAVES][R];   // per wave and digit: count, then start inside the sorted tile
@@ -287,11 +302,11 @@ __global__ __launch_bounds__(SORT_THREADS) void scatter_kernel(
     Keyed<KL>* stage = (Keyed<KL>*)sort_smem;
     if (n - tbase >= TILE)
         scatter_tile<KL, KO, FIRST, LAST, BITS, ITEMS, true>(src, TILE, (int)tbase, shift, drop, pass, row_total, my_word, my_group, tile,
-                                                             gave_up, out, order, inverse, sorted, whist, gdelta, wsum, rsum, stage);
+                                                             spin_limit, out, order, inverse, sorted, whist, gdelta, wsum, rsum, stage);
     else
         scatter_tile<KL, KO, FIRST, LAST, BITS, ITEMS, false>(src, (int)(n - tbase), (int)tbase, shift, drop, pass, row_total, my_word,
-                                                              my_group, tile, gave_up, out, order, inverse, sorted, whist, gdelta, wsum,
-                                                              rsum, stage);
+                                                              my_group, tile, spin_limit, out, order, inverse, sorted, whist, gdelta,
+                                                              wsum, rsum, stage);
 }
 
 constexpr int INV_ITEMS = 8;
@@ -390,7 +405,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void small_sort_kernel(Points pts, i
 
 struct SortWs {
     void* items[2];     // (k, n) of Keyed<uint64_t> (or Keyed<uint32_t>: the same room is reserved either way)
-    uint32_t* totals;   // [MAX_PASSES][k][R], then one word: a look-back gave up waiting
+    uint32_t* totals;   // [MAX_PASSES][k][R]
     TileWord* look;     // [k][tiles][R]
     GroupWord* glook;   // [k][groups][R]
     size_t zero_words;  // 32-bit words from `totals` on that are cleared before a sort
@@ -408,7 +423,7 @@ SortWs carve(void* base, int64_t n, int k, int tile, int radix) {
     }
     const size_t zero_from = off;
     w.totals = (uint32_t*)(p + off);
-    off += ptv3_align256(((size_t)MAX_PASSES * k * radix + 1) * sizeof(uint32_t));
+    off += ptv3_align256((size_t)MAX_PASSES * k * radix * sizeof(uint32_t));
     w.look = (TileWord*)(p + off);
     off += ptv3_align256((size_t)k * tiles * radix * sizeof(TileWord));
     w.glook = (GroupWord*)(p + off);
@@ -427,6 +442,7 @@ struct Job {
     void* sorted;
     void* workspace;
     hipStream_t stream;
+    int spin_limit = SPIN_LIMIT;
 };
 
 template <typename K, int BITS, int ITEMS>
@@ -451,7 +467,7 @@ int run_pass(const Job& j, const SortWs& w, int p, int drop, int64_t* inverse) {
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)j.k), dim3(SORT_THREADS), lds, j.stream,
                        FIRST ? (const void*)j.code : w.items[(p & 1) ^ 1], j.n, BITS * p - (FIRST ? 0 : drop), FIRST ? drop : 0, p,
                        w.totals + ((size_t)p * j.k << BITS), w.look, w.glook, tiles, groups,
-                       w.totals + ((size_t)MAX_PASSES * j.k << BITS), (Keyed<KO>*)w.items[p & 1], j.order, inverse, (KO*)j.sorted);
+                       j.spin_limit, (Keyed<KO>*)w.items[p & 1], j.order, inverse, (KO*)j.sorted);
     return PTV3_OK;
 }
 
@@ -539,6 +555,16 @@ extern "C" int ptv3_argsort(const int64_t* code, int64_t n, int k, int key_bits,
                             void* stream_) {
     return ptv3_argsort_keys(code, n, k, key_bits, order, inverse, nullptr, workspace, workspace_bytes,
                              (hipStream_t)stream_);
+}
+
+extern "C" int ptv3_argsort_impatient(const int64_t* code, int64_t n, int k, int key_bits, int spin_limit, int64_t* order,
+                                      int64_t* inverse, void* workspace, size_t workspace_bytes, void* stream_) {
+    if (n < 0 || k < 1 || k > 65535 || n >= (1ll << 31) || spin_limit > SPIN_LIMIT) return PTV3_EINVAL;
+    if (key_bits < 1 || key_bits > 63) return PTV3_EDEPTH;
+    if (n == 0) return PTV3_OK;
+    if (!code || !order || !inverse || !workspace) return PTV3_EINVAL;
+    Job j = {Points{}, const_cast<int64_t*>(code), n, k, key_bits, 0, order, inverse, nullptr, workspace, (hipStream_t)stream_, spin_limit};
+    return run(j, workspace_bytes);
 }
 
 // The curve codes of every order and their argsort; sorted_keys as in ptv3_argsort_keys.

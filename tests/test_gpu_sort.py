@@ -25,6 +25,24 @@ def test_argsort_forms(n, k, bits):
     assert torch.equal(inverse.gather(1, order), torch.arange(n, device=DEV).expand(k, n))
 
 
+@pytest.mark.parametrize("limit", [-1, 0, 3])
+@pytest.mark.parametrize("n,k,bits", [(4097, 2, 24), (2048 * 9 + 1, 4, 32), (2048 * 66 + 5, 2, 33), (4096 * 20 - 1, 3, 41), (6144 * 20 + 5, 4, 25)])
+def test_tiles_that_do_not_wait_count_the_keys_in_front_of_them(n, k, bits, limit):
+    """The way out of a wait that lasts too long, forced from the host: the same order, whoever does the counting."""
+    from pointtransformerv3_amd import _lib
+    lib = _lib.load()
+    code = np.random.default_rng(n).integers(0, 1 << bits, size=(k, n), dtype=np.int64)
+    code[0] >>= bits // 2
+    dev = to_dev(code)
+    order, inverse = torch.full((2, k, n), -1, dtype=torch.int64, device=DEV)
+    nbytes = lib.ptv3_argsort_workspace_bytes(n, k)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    assert lib.ptv3_argsort_impatient(dev.data_ptr(), n, k, bits, limit, order.data_ptr(), inverse.data_ptr(), ws.data_ptr(), nbytes,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+    assert np.array_equal(order.cpu().numpy(), np.argsort(code, axis=1, kind="stable"))
+    assert torch.equal(inverse.gather(1, order), torch.arange(n, device=DEV).expand(k, n))
+
+
 def test_argsort_of_a_row_with_its_own_inverse_pass():
     from pointtransformerv3_amd import ops
     n = (1 << 20) + 77
