@@ -6,6 +6,7 @@ An Engine describes one model in one compute dtype. It takes the default archite
 model, a model with hooks or submodules in training mode, and inputs that carry tables of their own go through the
 modules (model.py), which stay the definition of the result."""
 import ctypes
+import itertools
 import operator
 import weakref
 
@@ -79,14 +80,14 @@ _OWN_KEYS = ("serialized_code", "serialized_order", "serialized_inverse", "seria
 # what the native paths read of a module besides its children, parameters and buffers, once, when the model is described
 # (a BatchNorm's momentum, a DropPath's rate and the orders are read at every forward)
 _READ = {
-    nn.Linear: ("in_features", "out_features"), nn.GELU: ("approximate",), nn.Dropout: ("p",),
+    nn.GELU: ("approximate",), nn.Dropout: ("p",),
     nn.BatchNorm1d: ("eps", "num_features", "track_running_stats"), LayerNorm: ("eps", "normalized_shape"),
     SubMConv3d: ("kernel_size", "in_channels", "out_channels"), Block: ("channels", "pre_norm"),
     SerializedAttention: ("channels", "num_heads", "scale", "order_index", "patch_size", "enable_flash", "enable_rpe", "attn_drop"),
     SerializedPooling: ("stride", "reduce", "shuffle_orders", "traceable"), SerializedUnpooling: ("traceable",),
 }
 _PLAIN = (bool, int, float, str, tuple)
-_GEOMETRY = operator.attrgetter("shape"), torch.Tensor.stride
+_shape = operator.attrgetter("shape")
 
 
 def _names(m):
@@ -97,10 +98,18 @@ def _names(m):
     return names
 
 
+def _values(dicts):
+    return itertools.chain.from_iterable(map(dict.values, dicts))
+
+
+def _same_objects(a, b):
+    return len(a) == len(b) and all(map(operator.is_, a, b))
+
+
 class Structure:
-    """What of a model's modules the native paths rely on, and whether it still holds: which modules there are and of what
-    type, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
-    makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, about 0.17 ms), so it
+    """What of a model's modules the native paths rely on, and whether it still holds: which modules there are, their types'
+    forward, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
+    makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, 0.08 - 0.13 ms), so it
     is lists compared by mapped C functions.
 
     It looks at the backbone (embedding, enc, dec) only; what else a subclass holds runs outside this forward. It holds the
@@ -119,14 +128,13 @@ class Structure:
                                                                   m._backward_pre_hooks)]
         self.density = SubMConv3d.PAIR_MODE_MAX_DENSITY
         self._attributes, self._n_orders = model.__dict__, len(model.order)
-        self._types = list(map(type, self.modules))
-        self._forwards = [(t, t.forward) for t in set(self._types)]
-        children = [(m._modules, name, child) for m in self.modules for name, child in m._modules.items()]
-        children += [(model._modules, name, root) for name, root in zip(self.PARTS, roots) if root is not None]
-        self._child_at, self._children = ([d for d, _, _ in children], [k for _, k, _ in children]), [c for _, _, c in children]
-        # a child or an instance attribute (a replaced forward) that came or went
-        self._sized = [m.__dict__ for m in self.modules] + [m._modules for m in self.modules if m._modules]
-        self._sizes = list(map(len, self._sized))
+        self._forwards = [(t, t.forward) for t in set(map(type, self.modules))]
+        self._roots = [(model._modules, name, root) for name, root in zip(self.PARTS, roots) if root is not None]
+        self._holders = [m._modules for m in self.modules if m._modules]
+        self._children = list(_values(self._holders))
+        # an instance attribute (a replaced forward) that came or went
+        self._dicts = [m.__dict__ for m in self.modules]
+        self._sizes = list(map(len, self._dicts))
         self._reads, self._values = [], []
         reads = [(m.__dict__, _names(m)) for m in self.modules] + [(model.__dict__, ("num_stages", "stride", "cls_mode"))]
         for attributes, names in reads:
@@ -143,21 +151,20 @@ class Structure:
                 continue
             self._reads.append((getter, attributes))
             self._values.append(values)
-        slots = [(m._parameters, name) for m in self.modules for name in m._parameters]
         norms = [m for m in self.modules if isinstance(m, nn.BatchNorm1d)]
-        slots += [(m._buffers, name) for m in norms for name in ("running_mean", "running_var")]
-        self.tensors = [d[k] for d, k in slots if d[k] is not None]
-        slots += [(m._buffers, "num_batches_tracked") for m in norms]
-        self._slots = [d for d, _ in slots], [k for _, k in slots]
-        self._held = list(map(operator.getitem, *self._slots))
+        self._tables = [m._parameters for m in self.modules if m._parameters] + [m._buffers for m in norms]
+        self._held = list(_values(self._tables))
+        counters = {id(m._buffers.get("num_batches_tracked")) for m in norms}
+        self.tensors = [t for t in self._held if t is not None and id(t) not in counters]
         self._matrices = [t for t in self.tensors if t.dim() > 1]
+        self._square = [t for t in self._matrices if t.dim() == 2 and t.shape[0] == t.shape[1]]
         self._places = self._places_now()
         # modules whose training flag changes what they compute
         self.flagged = [m for m in self.modules if isinstance(m, (nn.BatchNorm1d, nn.Dropout, DropPath, SerializedAttention))]
 
     def _places_now(self):
-        # the same address with another shape or stride is another weight too; rows of one dimension are what they are
-        return [list(map(torch.Tensor.data_ptr, self.tensors)), *[list(map(g, self._matrices)) for g in _GEOMETRY]]
+        # the same address with another shape is another weight too, and a square matrix may lie there transposed
+        return [list(map(torch.Tensor.data_ptr, self.tensors)), list(map(_shape, self._matrices)), list(map(torch.Tensor.stride, self._square))]
 
     def hooked(self):
         hooks = torch.nn.modules.module
@@ -167,13 +174,11 @@ class Structure:
     def same(self):
         """Whether everything this was made from still is what it was."""
         try:
-            return (list(map(len, self._sized)) == self._sizes and list(map(type, self.modules)) == self._types
-                    and all(t.forward is f for t, f in self._forwards) and len(self._attributes["order"]) == self._n_orders
-                    and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
-                    and all(map(operator.is_, map(operator.getitem, *self._child_at), self._children))
-                    and [f(d) for f, d in self._reads] == self._values
-                    and all(map(operator.is_, map(operator.getitem, *self._slots), self._held))
-                    and self._places_now() == self._places)
+            return (list(map(len, self._dicts)) == self._sizes and all(t.forward is f for t, f in self._forwards)
+                    and len(self._attributes["order"]) == self._n_orders and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
+                    and all(d.get(name) is root for d, name, root in self._roots)
+                    and list(_values(self._holders)) == self._children and [f(d) for f, d in self._reads] == self._values
+                    and _same_objects(list(_values(self._tables)), self._held) and self._places_now() == self._places)
         except KeyError:   # something went that was there
             return False
 
