@@ -133,41 +133,43 @@ def _grouped(rows, groups, per):
     return out
 
 
+INDEX = ["hash_", "list_", "cell_", "slots_kernel", "facts_kernel", "publish_", "plan_", "direct_", "vh_", "kmap", "inner_",
+         "pool_gather", "pool_offsets", "cluster_", "attn_slots", "pad_index", "pad_prefix", "offset2batch"]
+SERIALIZATION = ["scatter_kernel", "digit_totals", "zero_words", "order_", "encode", "grid_max", "small_sort", "inverse_kernel"]
+CONV = ["pair_gemm", "pair_wstat", "pair_segment", "subm_conv", "conv_tile", "conv_sparse"]
+LINEAR = ["linear_rows", "linear_ln", "linear_wide", "linear_tile", "few_kernel", "linear_any", "gemm_f32"]
+
 FORWARD_GROUPS = collections.OrderedDict([
     ("patch attention", ["patch_attn"]),
-    ("sparse conv (sparse tile and tile forms, pair kernels, segment sum)",
-     ["pair_gemm", "pair_wstat", "pair_segment", "subm_conv", "conv_tile", "conv_sparse"]),
-    ("Linear kernels (linear_rows with GELU / BatchNorm epilogues, linear_wide, linear_ln, linear_any)",
-     ["linear_rows", "linear_ln", "linear_wide", "linear_gemm", "linear_any"]),
-    ("voxel hash + pair lists", ["plan_", "direct_", "vh_", "kmap", "pack_weight", "inner_"]),
+    ("serialization (codes, sort)", SERIALIZATION),
+    ("index: voxel hash, pair and tile lists, pooled tables, attention tables", INDEX),
+    ("sparse conv (sparse tile and tile forms, pair kernels, segment sum)", CONV),
+    ("weight copies (casts, packed orders)", ["cast_params", "pack_", "mlp_pack"]),
+    ("Linear kernels (rows, wide, tiles, few rows, with LayerNorm)", LINEAR),
     ("fused block head/tail, fused MLP", ["block_", "mlp_"]),
     ("LayerNorm / BatchNorm kernels", ["layer_norm", "bn_act"]),
+    ("pooling / unpooling", ["segment_reduce", "unpool"]),
+    ("padded input rows", ["pad_rows"]),
     ("torch elementwise / index / cat", ["at::native", "at::cuda"]),
-    ("copies (D2D residual copies, D2H counts)", ["copyBuffer", "fillBuffer"]),
-    ("serialization (encode, sort, pooled orders)",
-     ["scatter_kernel", "digit_totals", "zero_words", "order_", "encode", "grid_max"]),
-    ("pooling / unpooling", ["pool_", "segment_reduce", "unpool", "cluster_"]),
-    ("attention index tables", ["attn_slots", "pad_index", "pad_prefix"]),
-    ("offset2batch", ["offset2batch"]),
+    ("copies", ["copyBuffer", "fillBuffer"]),
 ])
 
 TRAIN_GROUPS = collections.OrderedDict([
-    ("attention backward (attn_bwd_q / attn_bwd_kv / fill)", ["attn_bwd"]),
+    ("attention backward", ["attn_bwd"]),
     ("attention forward (keeps log-sum-exp rows)", ["patch_attn"]),
-    ("weight gradients: conv (gather) and Linear (outer_rows, slab_sum)", ["outer_rows", "slab_sum", "conv_wgrad"]),
-    ("sparse conv forward and input gradient (sparse tile and tile forms, pair kernels, segment sum)",
-     ["pair_gemm", "pair_wstat", "pair_segment", "subm_conv", "conv_tile", "conv_sparse", "pack_weight"]),
-    ("LayerNorm + residual add, forward and backward", ["add_layer_norm", "layer_norm", "scaled_add"]),
-    ("parameter casts and transposes (cast_params)", ["cast_params"]),
-    ("Linear forward / input gradient on the row kernels (with the MLP's GELU)", ["linear_rows", "linear_wide", "linear_any"]),
-    ("library GEMMs", ["Cijk"]),
+    ("serialization (codes, sort)", SERIALIZATION),
+    ("index: voxel hash, pair and tile lists, pooled tables, attention tables", INDEX),
+    ("weight gradients: conv (gather) and Linear (outer_rows, slab_sum)", ["outer_rows", "slab_sum", "conv_wgrad", "cut_rows", "zero_ranges"]),
+    ("sparse conv forward and input gradient (sparse tile and tile forms, pair kernels, segment sum)", CONV),
+    ("weight copies (casts, transposes, packed orders)", ["cast_params", "pack_", "mlp_pack"]),
+    ("LayerNorm + residual add, forward and backward", ["add_layer_norm", "layer_norm", "scaled_add", "two_sums"]),
+    ("Linear forward / input gradient (with the MLP's GELU)", LINEAR),
     ("BatchNorm (+ GELU) training kernels", ["bn_stats", "bn_finalize", "bn_bwd", "bn_act", "batch_norm", "zero_kernel"]),
+    ("pooling / unpooling and their backward", ["segment_reduce", "unpool"]),
+    ("padded input rows", ["pad_rows"]),
+    ("library GEMMs (the 13-class head)", ["Cijk"]),
     ("torch elementwise, reductions, optimizer", ["at::native", "at::cuda"]),
-    ("voxel hash + pair lists + neighbour maps", ["plan_", "direct_", "vh_", "kmap", "inner_"]),
-    ("pooling / unpooling and their backward", ["pool_", "segment_reduce", "unpool", "cluster_"]),
     ("copies / fills", ["copyBuffer", "fillBuffer"]),
-    ("serialization (encode, sort, pooled orders)",
-     ["scatter_kernel", "digit_totals", "zero_words", "order_", "encode", "grid_max"]),
 ])
 
 
@@ -180,18 +182,19 @@ def forward_trace(d, out_dir):
         return "forward trace: needs bench.json, prof_bench.json and prof_csv/ (recipe lines 1-2)"
     bench, pbench = _last_json(need[0]), _last_json(need[1])
     steps = pbench["steps"]
-    # per-kernel statistics over the timed forwards only: a forward starts at its offset2batch kernel; what bench.py
-    # launches around the forwards (set-up, flop accounting) is left out
+    # per-kernel statistics over the timed forwards only: a forward starts at its facts_kernel (grid extent and scene ids, the
+    # first launch of its index); what bench.py launches around the forwards (set-up, flop accounting) is left out
     trace = list(csv.DictReader(open(trace_path)))
     trace.sort(key=lambda r: int(r["Start_Timestamp"]))
-    marks = [i for i, r in enumerate(trace) if "offset2batch" in r["Kernel_Name"]]
+    marks = [i for i, r in enumerate(trace) if "facts_kernel" in r["Kernel_Name"] and "publish" not in r["Kernel_Name"]]
     overlapped = pbench["config"].get("plain_schedule_ms_per_step") is not None
     # bench.py's loops, in order: warm-up, the `steps` timed forwards, then (when the timed ones overlapped their index
-    # prologues) 2 + steps forwards on the plain schedule, then 2 + steps with events around every launch. With a
-    # prologue running beside the forward before it, `steps` marks apart is still `steps` forwards' worth of kernels.
-    tail = steps + 2
-    plain = trace[marks[-2 * tail + 2]:marks[-tail]] if overlapped else None
-    t_first = -(2 * tail + steps) if overlapped else -(tail + steps)
+    # work) 2 + steps forwards on the plain schedule, then 2 + steps with events around the attention and steps with events
+    # around every launch (those two queued module by module). With a forward's index running beside the forward before
+    # it, `steps` marks apart is still `steps` forwards' worth of kernels.
+    before_events = -(2 * steps + 2)
+    plain = trace[marks[before_events - steps]:marks[before_events]] if overlapped else None
+    t_first = before_events - (2 * steps + 2 if overlapped else steps)
     window = trace[marks[t_first]:marks[t_first + steps]]
     agg = collections.OrderedDict()
     for r in window:
@@ -211,11 +214,11 @@ def forward_trace(d, out_dir):
         "command (run from the repository root on the GPU box):",
         "  rocprofv3 --kernel-trace --stats --output-format csv -d DIR/prof_csv -o fwd -- python3 bench.py --no-cpu --no-other-configs --steps %d --warmup %d"
         % (steps, pbench["warmup"]),
-        "source: the kernel trace of that run, the %d timed forwards (a forward = from one offset2batch kernel to the next%s); times in microseconds\n"
-        % (steps, "; the index prologue of a forward runs on its own stream beside the forward before, so the window is cut "
-                  "at the prologues and holds every kernel of a forward once" if overlapped else ""),
+        "source: the kernel trace of that run, the %d timed forwards (a forward = from one facts_kernel to the next%s), queued natively; times in microseconds\n"
+        % (steps, "; the index of a forward runs on its own stream beside the forward before, so the window is cut "
+                  "where an index begins and holds every kernel of a forward once" if overlapped else ""),
         "bench.py line of the same run: ms_per_step=%.2f  points/s=%.0f" % (pbench["ms_per_step"], pbench["value"]),
-        "  roofline (HIP events inside bench.py): kernel=%s launches=%d avg_launch_us=%.1f flops_per_launch=%.3e achieved=%.1f TFLOP/s frac=%.4f"
+        "  roofline (HIP events inside bench.py, forwards queued module by module): kernel=%s launches=%d avg_launch_us=%.1f flops_per_launch=%.3e achieved=%.1f TFLOP/s frac=%.4f"
         % (rf["kernel"], rf["launches"], rf["avg_launch_us"], rf["flops_per_launch"], rf["achieved"], rf["frac"]),
         "bench.py line without the profiler (`python3 bench.py`, same box, same build): ms_per_step=%.2f  points/s=%.0f  attention avg_launch_us=%.1f achieved=%.1f TFLOP/s frac=%.4f\n"
         % (bench["ms_per_step"], bench["value"], brf["avg_launch_us"], brf["achieved"], brf["frac"]),
@@ -230,7 +233,7 @@ def forward_trace(d, out_dir):
     out += _grouped([(n, v[1], v[0]) for n, v in rows], FORWARD_GROUPS, steps)
     if overlapped:
         ptot = sum(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]) for r in plain)
-        pspan = (int(trace[marks[-tail - 1]]["Start_Timestamp"]) - int(plain[0]["Start_Timestamp"])) / (steps - 1) / 1e3
+        pspan = (int(trace[marks[before_events - 1]]["Start_Timestamp"]) - int(plain[0]["Start_Timestamp"])) / (steps - 1) / 1e3
         out.append("\nthe plain schedule (every forward's index work in front of its own feature kernels), the %d forwards bench.py "
                    "times after the timed region: %.1f us of kernels per forward, %.1f us from forward to forward under the profiler; "
                    "bench.py's own clock: %.2f ms per forward with the profiler, %.2f ms without"
@@ -364,7 +367,7 @@ def index_kernel_counters(d, out_dir):
     tp, fp, wp = _find(base, "t_kernel_trace.csv"), _find(base, "f_counter_collection.csv"), _find(base, "w_counter_collection.csv")
     if tp is None or fp is None or wp is None:
         return "index kernel counters: needs kern_pmc/ (recipe lines 9-11)"
-    want = ("encode_kernel", "decode_kernel", "digit_totals_kernel", "scatter_kernel", "zero_words_kernel", "vh_insert_kernel",
+    want = ("encode_kernel", "decode_kernel", "digit_totals_kernel", "inverse_kernel", "vx_", "gather_rows", "scatter_kernel", "zero_words_kernel", "vh_insert_kernel",
             "vh_fill_kernel", "direct_count_kernel", "direct_fill_kernel", "plan_scan_kernel", "kmap_kernel", "kmap_build",
             "order_count_kernel", "order_assign_kernel", "pool_gather_kernel", "segment_reduce_kernel", "pool_", "voxel", "scene_min",
             "pad_index", "attn_slots", "plan_", "cluster_", "unpool")
