@@ -226,3 +226,40 @@ def test_dense_volumes_follow_the_module_class_setting(monkeypatch):
     monkeypatch.setattr(SubMConv3d, "PAIR_MODE_MAX_DENSITY", 1.0)
     got, want = _both(model, data, monkeypatch)
     assert torch.equal(got.feat, want.feat) and not torch.equal(got.feat, first)
+
+
+def test_one_model_in_several_threads_and_streams():
+    """Threads with a stream of their own each run one model on different inputs: the results of one after the other."""
+    import threading
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(shuffle_orders=False, **KW).eval().to(DEV)
+    _each(model, "SerializedPooling", "shuffle_orders", False)
+    datas = [_inputs(s, sizes, torch.float32) for s, sizes in ((4, (5000,)), (11, (3000, 700)), (23, (9000,)), (31, (2500, 2500)))]
+    torch.cuda.synchronize()
+
+    def run(data):
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):     # weight copies made by every forward
+            return model(dict(data)).feat
+
+    want = [run(d) for d in datas]
+    torch.cuda.synchronize()
+    got, failed = [[] for _ in datas], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(6):
+                    got[i].append(run(datas[i]))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(datas))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failed and not any(t.is_alive() for t in threads)
+    for w, rows in zip(want, got):
+        assert len(rows) == 6 and all(torch.equal(w, r) for r in rows)
