@@ -674,8 +674,8 @@ int ptv3_block_tail_few(const void *attn, const void *shortcut, const void *w_pr
  *   pool   pooled tables, padding and slot tables, pair counts of the pooled levels. Data: pair counts.
  *   lists  pair lists and tile lists (want[l]: PTV3_LISTS_*).
  * The caller allocates: `state` (PTV3_INDEX_STATE_BYTES host bytes, kept until after `lists`), and the device buffers
- * whose sizes the *_bytes calls return; begin's and pool's scratch must stay until `lists` has run on the stream,
- * the rest as long as the tables are used. ptv3_index_levels describes the result. Nothing is allocated or kept
+ * whose sizes the *_bytes calls return: begin's and pool's scratch must stay until `lists` has run on the stream (later
+ * work on that stream may have it), the tables and the lists as long as they are used. ptv3_index_levels describes the result. Nothing is allocated or kept
  * inside. At most PTV3_MAX_LEVELS levels and PTV3_MAX_ORDERS orders; n < 2^24 where tile lists are wanted. */
 #define PTV3_MAX_LEVELS 8
 #define PTV3_MAX_ORDERS 8
@@ -747,7 +747,8 @@ const ptv3_level *ptv3_index_levels(const void *state);
  * precision stem_w has its input channels padded to a multiple of 16 (ptv3_pad_rows over the weight's rows), and the
  * packed copies are those of ptv3_subm_conv_pack_weight (conv_packed, 32 / 64 / 128 channels), ptv3_mlp_pack_weights_batch
  * (mlp_packed from 128 channels on, proj_packed at 128 and 256, head_packed = xCPE Linear + qkv at 128).
- * Level l needs the lists ptv3_conv_form names for its blocks' channels (float: pairs), level 0 also the 5x5x5 lists.
+ * Level l needs the lists ptv3_conv_form names for its blocks' channels (float: pairs), level 0 also the 5x5x5 lists;
+ * neighbour maps are made in the workspace where ptv3_conv_pair_form asks for them.
  * stage_out: NULL, or per stage a buffer for the encoder stage's rows (or NULL in it); out: the decoder's (n, channels)
  * rows. Queues only; allocates and keeps nothing. */
 typedef struct ptv3_linear_w { const void *w, *b; int32_t in, out; } ptv3_linear_w;
@@ -803,8 +804,8 @@ int ptv3_net_refresh(const ptv3_refresh *jobs, void *stream);
  * float, BatchNorm's also in dtype. The residual stream is float, rows between layers are in dtype. Gradients are
  * written, not accumulated, to `grads` + the g* offsets (floats; a BatchNorm's bias gradient follows its weight's);
  * `zero` lists the ranges that are summed with atomics (the LayerNorms').
- * Levels need: tile lists or pair lists as ptv3_conv_form says, below 128 channels pair lists with PAIR_OUT, from 128 on
- * the neighbour map, level 0 PAIRS5 with PAIR_OUT5. masks: per block, encoder stages then decoder stages from the
+ * Levels need: pair lists with PAIR_OUT (weight gradients; product rows), tile lists too where ptv3_conv_form says so,
+ * level 0 PAIRS5 with PAIR_OUT5. A neighbour map is made inside where ptv3_conv_pair_form asks for one. masks: per block, encoder stages then decoder stages from the
  * bottom, the row factors (n,) in dtype of the attention's and the MLP's stochastic depth, or NULL.
  * Same forward as ptv3_train_fwd's buffers: acts is kept by the caller until after the backward, which only reads it. */
 typedef struct ptv3_train_linear { const void *w, *wt, *b; int32_t in, out; int64_t gw, gb; } ptv3_train_linear;

@@ -1,4 +1,5 @@
-// Submanifold sparse convolution forward over the neighbour map, in two forms.
+// Submanifold sparse convolution forward, dense over the neighbour map or over its pairs (tile forms: convtile.hip,
+// convsparse.hip; which of them a layer takes: ptv3_conv_form in features.hip, ptv3_conv_pair_form here).
 //
 // Replaces spconv.SubMConv3d.forward at the reference call sites model.py:546-552 (xCPE,
 // 3x3x3, bias) and :767-774 (stem, 5x5x5, no bias).
@@ -11,6 +12,8 @@
 // grouped by tap, so every MFMA column is real work whatever the sparsity (a 2 cm surface scan
 // has 2-5 of 27 taps per voxel); one product row per pair goes to a scratch matrix and a segment
 // sum per voxel finishes. Costs a round trip of that matrix; best for sparse maps, thin channels.
+// Its rows are half, or float (ptv3_subm_conv_pairs_wide_fwd) where the other forms of the shape
+// keep a voxel's sum on chip in float.
 //
 // Both take the product transposed (rows = output channels, columns = voxels / pairs) with
 // v_mfma_f32_32x32x16: a lane's operand is then 8 consecutive input channels of one row, and its
@@ -18,7 +21,8 @@
 // segments (several lanes x 16 B per row) and a small wave-private LDS buffer converts between
 // that shape and the one-row-per-lane operand layout: touching 8-16 lines per memory instruction
 // instead of 32 is what keeps the address path from bounding the kernels.
-// fp32: one thread per output element, plain FMA (parity path, not tuned).
+// fp32: the pair form runs on the fp32 matrix cores (gemmf32.hip); the dense form is one thread per output element
+// with plain FMA, for dense volumes whose product rows would not fit (ptv3_conv_pair_form).
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 

@@ -1,10 +1,13 @@
 """A training step's forward and backward from native code (ptv3_train_fwd / ptv3_train_bwd): under half-precision
-autocast the whole feature side of a PointTransformerV3 is one autograd node whose parameter gradients come as views of
-one flat buffer: they all come at the end of the backward (a reducer that wants to overlap them with it has nothing to
-start on before; a hook on any submodule, which sends the step through the modules, gives them one by one), and a p.grad that
-is kept or saved keeps the buffer, 185 MB for the default model (p.grad.clone() lets go of it). Module by module the same step is some 250 Python autograd functions each way and about 20 ms of host
-time whatever the batch. Takes the default architecture in training mode (see native.Parts, TrainEngine); anything else
-goes through the modules (model.py), which stay the definition of the result."""
+autocast the whole feature side of a PointTransformerV3 is one autograd node. Module by module the same step is some 250
+Python autograd functions each way and about 20 ms of host time whatever the batch. Takes the default architecture in
+training mode (see native.Parts, TrainEngine); anything else goes through the modules (model.py), which stay the
+definition of the result.
+
+The parameter gradients are views of one flat buffer and all come at the end of the backward: a reducer that wants to
+overlap them with it has nothing to start on before (a hook on any submodule, which sends the step through the modules,
+gives them one by one), and a p.grad that is kept or saved keeps the buffer, 185 MB for the default model (its clone does
+not)."""
 import ctypes
 import weakref
 
