@@ -289,7 +289,7 @@ class _Step(torch.autograd.Function):
         _lib.check(lib.ptv3_train_fwd(ctypes.byref(engine.net), index.levels, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype],
                                       _addresses(masks), acts.data_ptr(), scratch.data_ptr(), sizes[1], out.data_ptr(), ops._stream()), "ptv3_train_fwd")
         ctx.engine, ctx.index, ctx.scratch_bytes = engine, index, sizes[2]
-        ctx.masked = [m is not None for m in masks]
+        ctx.acts_bytes, ctx.masked = sizes[0], [0 if m is None else m.numel() for m in masks]
         # freed by autograd after the backward, as the activations of separate nodes would be; the versions go with them, so
         # that activations which a checkpoint computes again are held against the weights they were computed with
         ctx.save_for_backward(acts, torch.tensor(engine.versions()), *[m for m in masks if m is not None])
@@ -307,6 +307,11 @@ class _Step(torch.autograd.Function):
         if versions.tolist() != engine.versions():
             raise RuntimeError("one of the variables needed for gradient computation has been modified by an inplace operation: "
                                "a parameter of PointTransformerV3 was written between a training step's forward and its backward")
+        want = [(torch.uint8, ctx.acts_bytes)] + [(engine.dtype, n) for n in ctx.masked if n]
+        for t, (dtype, numel) in zip((acts, *kept), want):
+            if t.device != dout.device or t.dtype != dtype or t.numel() != numel:
+                raise _lib.Ptv3Error("a saved-tensor hook handed back another tensor than it was given: "
+                                     f"{t.numel()} x {t.dtype} on {t.device}, not {numel} x {dtype} on {dout.device}")
         acts, *kept = [t if t.is_contiguous() and t.data_ptr() % 256 == 0 else t.clone(memory_format=torch.contiguous_format)
                        for t in (acts, *kept)]
         kept = iter(kept)

@@ -76,7 +76,7 @@ def train_step(monkeypatch):
     monkeypatch.setattr(native_train._lib, "load", lambda: lib)
     monkeypatch.setattr(native_train.ops, "_stream", lambda: None)
     weight = torch.nn.Parameter(torch.ones(1))
-    engine = types.SimpleNamespace(net=native_train._Net(), out_channels=4,
+    engine = types.SimpleNamespace(net=native_train._Net(), out_channels=4, dtype=torch.float32,
                                    total=1, params=[weight], read_back=[weight])
     engine.versions = types.MethodType(native_train.TrainEngine.versions, engine)
     index = types.SimpleNamespace(levels=None)
@@ -108,6 +108,17 @@ def test_backward_of_a_step_reads_the_masks_that_autograd_kept(hooks, train_step
     out.sum().backward()
     assert train_step.lib.read == [want, want]
     assert float(train_step.weight.grad) == 0.0
+
+
+@pytest.mark.parametrize("change", [lambda t: t[:-1], lambda t: t.double(), lambda t: t.to("meta")], ids=["shorter", "dtype", "device"])
+@pytest.mark.parametrize("which", [torch.uint8, torch.float32], ids=["activations", "masks"])
+def test_backward_of_a_step_refuses_tensors_that_hooks_changed(change, which, train_step):
+    """What the kernels would read past the end of, or where they cannot reach, is an error."""
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: change(t) if t.dtype == which else t):
+        out = train_step.step([torch.ones(6, 1)])
+    with pytest.raises(RuntimeError, match="saved-tensor hook"):
+        out.sum().backward()
+    assert len(train_step.lib.read) == 1      # the forward only
 
 
 def test_backward_of_a_step_refuses_weights_written_since_its_forward(train_step):
