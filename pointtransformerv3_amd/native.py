@@ -98,6 +98,11 @@ def _names(m):
     return names
 
 
+def _n_orders(attributes):
+    orders = attributes.get("order")
+    return len(orders) if isinstance(orders, (list, tuple)) else 0
+
+
 def _values(dicts):
     return itertools.chain.from_iterable(map(dict.values, dicts))
 
@@ -127,7 +132,10 @@ class Structure:
         self.hooks = [d for m in (model, *self.modules) for d in (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
                                                                   m._backward_pre_hooks)]
         self.density = SubMConv3d.PAIR_MODE_MAX_DENSITY
-        self._attributes, self._n_orders = model.__dict__, len(model.order)
+        self._attributes = model.__dict__
+        self._n_orders = _n_orders(model.__dict__)
+        if not self._n_orders:
+            self.why = "orders that are no list"
         self._forwards = [(t, t.forward) for t in set(map(type, self.modules))]
         self._roots = [(model._modules, name, root) for name, root in zip(self.PARTS, roots) if root is not None]
         self._holders = [m._modules for m in self.modules if m._modules]
@@ -175,7 +183,7 @@ class Structure:
         """Whether everything this was made from still is what it was."""
         try:
             return (list(map(len, self._dicts)) == self._sizes and all(t.forward is f for t, f in self._forwards)
-                    and len(self._attributes["order"]) == self._n_orders and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
+                    and _n_orders(self._attributes) == self._n_orders and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
                     and all(d.get(name) is root for d, name, root in self._roots)
                     and list(_values(self._holders)) == self._children and [f(d) for f, d in self._reads] == self._values
                     and _same_objects(list(_values(self._tables)), self._held) and self._places_now() == self._places)
@@ -239,7 +247,7 @@ class Parts:
 
     def __init__(self, model):
         S = model.num_stages
-        self.n_orders = len(model.order)
+        self.n_orders = _n_orders(model.__dict__)
         _need(2 <= S <= levels.MAX_LEVELS and 1 <= self.n_orders <= levels.MAX_ORDERS and len(model.stride) == S - 1, "stages")
         embedding, enc = _child(model, "embedding", Embedding, "stem"), _child(model, "enc", PointSequential, "encoder")
         self.stem_conv, self.stem_bn, act = _sequence(embedding, "stem", (SubMConv3d, nn.BatchNorm1d, nn.GELU), "stem")

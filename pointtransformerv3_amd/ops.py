@@ -751,7 +751,7 @@ class PrologueOverlap:
         may read on the current stream at any later time are marked for that stream (the allocator then holds their
         memory back until those reads are over); everything else of the index belongs to the forward."""
         main = torch.cuda.current_stream(self.device)
-        while point is not None:   # an encoder-only result hands out the levels above as well
+        while isinstance(point, dict):   # an encoder-only result hands out the levels above as well
             for key in self.PUBLIC_KEYS:
                 t = point.get(key)
                 if isinstance(t, torch.Tensor) and t.is_cuda:

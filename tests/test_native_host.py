@@ -322,7 +322,8 @@ FOREIGN = dict(
     reduce=_set("enc.enc1.down.reduce", "median"), strides=_set("stride", (2,)),
     pruned=lambda m: setattr(m.enc.enc1.block0.mlp[0].fc1.weight, "data", m.enc.enc1.block0.mlp[0].fc1.weight.data[:64]),
     pruned_norm=lambda m: setattr(m.enc.enc1.block0.norm1[0].weight, "data", torch.ones(32)),
-    heads=_set("enc.enc1.block0.attn.num_heads", 0),
+    heads=_set("enc.enc1.block0.attn.num_heads", 0), order_set=_set("order", {"z"}), order_gone=_without("order"),
+    order_iterator=lambda m: setattr(m, "order", iter(["z", "hilbert"])),
 )
 
 
