@@ -3,7 +3,7 @@ kernel traces and counter collections) into the short text summaries kept under 
 
 Every summary names the commands its figures come from. A section whose raw files are missing from DIR is skipped and
 says which command writes them; `python bench.py --summarise DIR --recipe` prints the whole batch, in order, as shell
-lines (run them from the repository root on the GPU box, `cd /tmp && export TMPDIR=/tmp` first; each rocprofv3 --pmc
+lines (run them from the repository root on an MI355X, `cd /tmp && export TMPDIR=/tmp` first; each rocprofv3 --pmc
 line is a run of its own and holds at most 8 SQ and 4 TCC counters).
 """
 import collections
@@ -211,7 +211,7 @@ def forward_trace(d, out_dir):
     rf, brf = pbench["roofline"], bench["roofline"]
     out = [
         "rocprofv3 kernel-trace summary: full PTv3 forward, 4 room scenes (%d points), fp16, MI355X\n" % POINTS,
-        "command (run from the repository root on the GPU box):",
+        "command (run from the repository root on an MI355X):",
         "  rocprofv3 --kernel-trace --stats --output-format csv -d DIR/prof_csv -o fwd -- python3 bench.py --no-cpu --no-other-configs --steps %d --warmup %d"
         % (steps, pbench["warmup"]),
         "source: the kernel trace of that run, the %d timed forwards (a forward = from one facts_kernel to the next%s), queued natively; times in microseconds\n"
@@ -260,7 +260,7 @@ def attention_traffic(d, out_dir):
     txt = [
         "rocprofv3 --pmc summary: HBM traffic of the patch attention kernel inside the full PTv3 forward",
         "(4 room scenes, %d points, fp16, MI355X)\n" % POINTS,
-        "commands (run from the repository root on the GPU box, one counter per run):",
+        "commands (run from the repository root on an MI355X, one counter per run):",
         "  rocprofv3 --pmc FETCH_SIZE --output-format csv -d DIR/pmc_fetch -o f -- python3 bench.py --no-cpu --no-other-configs --steps 2 --warmup 1 --copy-calibration",
         "  rocprofv3 --pmc WRITE_SIZE --output-format csv -d DIR/pmc_write -o w -- python3 bench.py --no-cpu --no-other-configs --steps 2 --warmup 1 --copy-calibration\n",
         "calibration (--copy-calibration: one 1 GiB device-to-device copy, kernel __amd_rocclr_copyBuffer):",
@@ -310,7 +310,7 @@ def attention_counters(d, out_dir):
     t = [
         "rocprofv3 --pmc summary: instruction mix and issue utilisation of the patch attention kernel at baseline",
         "config 2 (one room scene, %d points, Hilbert order, patch 1024, C=512, 32 heads, fp16), MI355X\n" % cfg2["points"],
-        "commands (run from the repository root on the GPU box):",
+        "commands (run from the repository root on an MI355X):",
         "  python3 bench.py --attention-config2 20",
         "  rocprofv3 --pmc %s --output-format csv -d DIR/pmc_attn -o a -- python3 bench.py --attention-config2 3" % SQ_A,
         "  rocprofv3 --pmc %s --output-format csv -d DIR/pmc_attn -o b -- python3 bench.py --attention-config2 3\n" % SQ_B,
@@ -345,7 +345,7 @@ def kernel_rooflines(d, out_dir):
     rows = json.load(open(path))
     k = [
         "per-kernel measurements at the sizes of the baseline configurations (and at 16x the points for the index kernels), MI355X\n",
-        "command (run from the repository root on the GPU box):",
+        "command (run from the repository root on an MI355X):",
         "  python3 bench.py --no-cpu --no-other-configs --steps 5 --warmup 2 --kernels DIR/kernel_rooflines.json",
         "each kernel is called alone 20 times back to back through the Python wrapper and timed with HIP events, so",
         "the figure includes output allocation, launch overhead and, where the wrapper reads a count back, that",
@@ -388,7 +388,7 @@ def index_kernel_counters(d, out_dir):
         "rocprofv3 summary: HBM traffic and L2 requests of the serialization, radix sort, voxel-hash / pair-list, pooling and",
         "voxelisation kernels at the sizes bench.py --kernels runs them (4 room scenes of %d points; the same 16 times over;" % POINTS,
         "baseline config 3's 200,000 voxels; the levels of the benchmark batch), MI355X\n",
-        "commands (run from the repository root on the GPU box; each counter set in a run of its own):",
+        "commands (run from the repository root on an MI355X; each counter set in a run of its own):",
         "  rocprofv3 --kernel-trace --output-format csv -d DIR/kern_pmc -o t -- python3 bench.py --no-cpu --no-other-configs --steps 2 --warmup 1 --kernels DIR/kr_t.json",
         "  rocprofv3 --pmc FETCH_SIZE TCC_HIT_sum --output-format csv -d DIR/kern_pmc -o f -- (the same bench.py line)",
         "  rocprofv3 --pmc WRITE_SIZE TCC_REQ_sum TCC_MISS_sum --output-format csv -d DIR/kern_pmc -o w -- (the same bench.py line)\n",
@@ -426,7 +426,7 @@ def training_trace(d, out_dir):
     o = [
         "rocprofv3 kernel-trace summary: PTv3 training step (forward + backward + AdamW), default model in training mode,",
         "4 room scenes (%d points), bf16 autocast, MI355X\n" % POINTS,
-        "command (run from the repository root on the GPU box):",
+        "command (run from the repository root on an MI355X):",
         "  rocprofv3 --kernel-trace --stats --output-format csv -d DIR/train_prof -o tr -- python3 bench.py --train bfloat16 --steps %d --warmup %d" % (tp["steps"], tp["warmup"]),
         "source: the kernel statistics of that run; all %d steps of the process (%d warm-up + %d timed), figures divided by %d; times in microseconds\n"
         % (nstep, tp["warmup"], tp["steps"], nstep),
@@ -468,7 +468,7 @@ def conv_counters(d, out_dir):
             f"rocprofv3 summary: the 3x3x3 submanifold convolution of one level alone -- {line['workload']}, fp16, MI355X",
             f"{line['voxels']} voxels, {line['channels']} channels, {line['pairs']} active pairs ({line['pairs_per_voxel']:.2f} per voxel), form: {line['form']}",
             "",
-            "commands (run from the repository root on the GPU box; each counter set in a run of its own):",
+            "commands (run from the repository root on an MI355X; each counter set in a run of its own):",
             f"  python3 bench.py --conv {wl} --reps 20",
             f"  rocprofv3 --kernel-trace --stats --output-format csv -d DIR/conv_{wl} -o t -- python3 bench.py --conv {wl} --reps 5",
             f"  rocprofv3 --pmc {CONV_A} --output-format csv -d DIR/conv_{wl} -o a -- python3 bench.py --conv {wl} --reps 3",
@@ -518,7 +518,7 @@ def dense_counters(d, out_dir):
         "rocprofv3 --pmc summary: the fused dense kernels of a transformer block, each alone at the rows and width of a level of the",
         "benchmark batch (4 room scenes, fp16), MI355X",
         "",
-        "commands (run from the repository root on the GPU box; CASE = " + ", ".join(DENSE_CASES) + "; each counter set in a run of its own):",
+        "commands (run from the repository root on an MI355X; CASE = " + ", ".join(DENSE_CASES) + "; each counter set in a run of its own):",
         "  python3 bench.py --dense CASE --reps 20",
         f"  rocprofv3 --pmc {DENSE_A} --output-format csv -d DIR/dense_CASE -o a -- python3 bench.py --dense CASE --reps 3",
         f"  rocprofv3 --pmc {DENSE_B} --output-format csv -d DIR/dense_CASE -o b -- python3 bench.py --dense CASE --reps 3",
@@ -565,7 +565,7 @@ def micro_reports(d, out_dir):
             continue
         body = [l for l in open(path).read().splitlines() if "amdgpu.ids" not in l]
         head = [f"microbenchmark of the part (libptv3_micro.so, pointtransformerv3_amd/csrc/micro.hip), MI355X",
-                f"command (run from the repository root on the GPU box): python3 bench.py --micro {which}", ""]
+                f"command (run from the repository root on an MI355X): python3 bench.py --micro {which}", ""]
         open(os.path.join(out_dir, f"micro_{which}.txt"), "w").write("\n".join(head + body) + "\n")
         done.append(which)
     return "micro reports: " + (", ".join(done) if done else "needs micro_issue.txt / micro_loads.txt (recipe: the --micro lines)")

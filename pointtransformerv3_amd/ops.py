@@ -617,9 +617,6 @@ class ConvPlan:
     def n_pairs(self, value):
         self._n_pairs = value
 
-    def density(self):
-        return self.n_pairs / max(1, self.n * self.taps)
-
     def slot_pair(self):
         """Output-major pair words (tap << 24 | input row) for subm_conv_tiles, made on first use."""
         if getattr(self, "_slot_pair", None) is None:
