@@ -90,6 +90,16 @@ _PLAIN = (bool, int, float, str, tuple)
 _shape = operator.attrgetter("shape")
 
 
+# the classes a covered model is made of, with what they do
+_FORWARDS = [(t, t.forward) for t in (
+    nn.Linear, nn.GELU, nn.Dropout, nn.BatchNorm1d, nn.Identity, LayerNorm, SubMConv3d, MLP, Block, DropPath, Embedding, PointSequential,
+    SerializedAttention, SerializedPooling, SerializedUnpooling)]
+
+
+def _as_imported():
+    return all(t.forward is f for t, f in _FORWARDS)
+
+
 def _names(m):
     """What _READ names of a module."""
     names = _READ.get(type(m), ())
@@ -112,8 +122,8 @@ def _same_objects(a, b):
 
 
 class Structure:
-    """What of a model's modules the native paths rely on, and whether it still holds: which modules there are, their types'
-    forward, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
+    """What of a model's modules the native paths rely on, and whether it still holds: which modules there are, their
+    classes' forward, the attributes that were read, each parameter and statistic with its place and geometry. A change in any of them
     makes the model be looked at anew. same() runs in front of every forward (a few hundred modules, 0.08 - 0.13 ms), so it
     is lists compared by mapped C functions.
 
@@ -136,7 +146,8 @@ class Structure:
         self._n_orders = _n_orders(model.__dict__)
         if not self._n_orders:
             self.why = "orders that are no list"
-        self._forwards = [(t, t.forward) for t in set(map(type, self.modules))]
+        if not _as_imported():
+            self.why = "a class's forward was replaced"
         self._roots = [(model._modules, name, root) for name, root in zip(self.PARTS, roots) if root is not None]
         self._holders = [m._modules for m in self.modules if m._modules]
         self._children = list(_values(self._holders))
@@ -182,7 +193,7 @@ class Structure:
     def same(self):
         """Whether everything this was made from still is what it was."""
         try:
-            return (list(map(len, self._dicts)) == self._sizes and all(t.forward is f for t, f in self._forwards)
+            return (list(map(len, self._dicts)) == self._sizes and _as_imported()
                     and _n_orders(self._attributes) == self._n_orders and SubMConv3d.PAIR_MODE_MAX_DENSITY == self.density
                     and all(d.get(name) is root for d, name, root in self._roots)
                     and list(_values(self._holders)) == self._children and [f(d) for f, d in self._reads] == self._values

@@ -381,3 +381,18 @@ def test_rule_of_convolutions_that_no_tile_form_takes():
     assert form(f32, 10_000_000, 27 * 10_000_000, 27, 32, 32, 0.6) == ops.CONV_DENSE
     assert form(f32, 100_000_000, 27 * 10_000_000, 27, 512, 512, 0.6) == ops.CONV_PAIRS
     assert form(f16, 0, 0, 27, 32, 32, 0.6) == ops.CONV_PAIRS
+
+
+@pytest.mark.parametrize("when", ["before", "after"])
+@pytest.mark.parametrize("kind", [native.SerializedAttention, native.Block, torch.nn.Linear])
+def test_a_class_whose_forward_was_replaced_is_left_to_the_modules(kind, when, monkeypatch):
+    from pointtransformerv3_amd import PointTransformerV3
+    model = PointTransformerV3(**SMALL)
+    structure = native.Structure(model)
+    monkeypatch.setattr(kind, "forward", lambda self, x: x)
+    if when == "after":
+        assert not structure.same()
+    else:
+        assert native.Structure(model).why is not None
+    monkeypatch.undo()
+    assert structure.same() and native.Structure(model).why is None
