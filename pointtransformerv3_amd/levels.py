@@ -123,6 +123,9 @@ def build(layout, grid_coord, offset, batch, orders, shuffle, want, between=None
     check(lib.ptv3_index_wait(slot.ptr, 0, seq, stream), "ptv3_index_wait")
     out.grid_max = words[_SLOT_DATA:_SLOT_DATA + 3]
     out.offset_host = words[_SLOT_ENDS:_SLOT_ENDS + nb]
+    if out.offset_host[-1] != n or any(b < a for a, b in zip(out.offset_host, out.offset_host[1:])):
+        hostslot.give(slot)
+        raise _lib.Ptv3Error(f"offset {out.offset_host[-4:]} does not end the scenes of {n} points in ascending order")
     depth = max(out.grid_max).bit_length()            # model.py:98-101
     assert depth * 3 + nb.bit_length() <= 63          # model.py:103
     assert depth <= 16                                # model.py:108

@@ -630,9 +630,15 @@ def plain_inputs(data):
         return False
     if any(k in data for k in _OWN_KEYS) or any(k.startswith("_") for k in data) or not ("offset" in data or "batch" in data):
         return False
-    where = data.get("grid_coord", data.get("coord"))
-    ends = data.get("offset", data.get("batch"))
-    return isinstance(where, torch.Tensor) and where.is_cuda and where.shape[0] == feat.shape[0] and ends.is_cuda and ends.numel() > 0
+    n, where, offset, batch = feat.shape[0], data.get("grid_coord", data.get("coord")), data.get("offset"), data.get("batch")
+    # the kernels take addresses: what is not of these shapes on this GPU is the modules' to convert or to refuse
+    return (_placed(where, feat, 2) and where.shape == (n, 3) and ("grid_coord" in data or "grid_size" in data)
+            and ("offset" not in data or (_placed(offset, feat, 1) and offset.shape[0] > 0))
+            and ("batch" not in data or (_placed(batch, feat, 1) and batch.shape[0] == n)))
+
+
+def _placed(t, feat, dim):
+    return isinstance(t, torch.Tensor) and t.device == feat.device and t.dim() == dim
 
 
 def _stem_weight(model):
@@ -649,7 +655,7 @@ def engine_for(model, data):
         return None
     feat = data["feat"]
     weight = _stem_weight(model)
-    dtype = None if weight is None else _compute_dtype(feat, weight)
+    dtype = None if weight is None or weight.device != feat.device else _compute_dtype(feat, weight)
     if dtype not in ops.DTYPE_CODES or feat.shape[1] != weight.shape[-1]:
         return None
     held = _ENGINES.setdefault(model, {})

@@ -347,6 +347,8 @@ def engine_for(model, data):
         held[dtype] = engine
     if isinstance(engine, native.Refused) or data["feat"].shape[1] != engine.net.stem.cin or data["feat"].shape[0] < 2:
         return None
+    if data["feat"].device != engine.device:
+        return None
     if engine.structure.hooked() or not all(m.training for m in engine.structure.flagged):
         return None
     return engine if engine.averaging() and any(p.requires_grad for p in engine.params) else None

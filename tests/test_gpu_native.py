@@ -263,3 +263,36 @@ def test_one_model_in_several_threads_and_streams():
     assert not failed and not any(t.is_alive() for t in threads)
     for w, rows in zip(want, got):
         assert len(rows) == 6 and all(torch.equal(w, r) for r in rows)
+
+
+def test_inputs_that_kernels_cannot_address_are_not_taken():
+    """Other shapes and places than the kernels assume go to the modules; scene ends that are none are refused before any
+    table is made from them."""
+    from pointtransformerv3_amd import PointTransformerV3, native
+    from pointtransformerv3_amd._lib import Ptv3Error
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().half().to(DEV)
+    data = _inputs(7, (1500, 900), torch.float16)
+    n = data["feat"].shape[0]
+    batch = torch.zeros(n, dtype=torch.int64, device=DEV)
+    batch[int(data["offset"][0]):] = 1
+    with torch.inference_mode():
+        want = model(dict(data)).feat
+        assert native.engine_for(model, dict(data, batch=batch)) is not None
+        for change in (dict(grid_coord=data["grid_coord"].cpu()), dict(offset=data["offset"].cpu()), dict(batch=batch.cpu()),
+                       dict(batch=batch[:-1]), dict(batch=batch[:, None]), dict(offset=data["offset"][:, None]),
+                       dict(grid_coord=torch.cat([data["grid_coord"]] * 2, 1)), dict(grid_coord=data["grid_coord"][:-1]),
+                       dict(offset=data["offset"].tolist()), dict(offset=data["offset"][:0])):
+            assert native.engine_for(model, dict(data, **change)) is None, list(change)
+        without = {k: v for k, v in data.items() if k != "grid_coord"}
+        assert native.engine_for(model, without) is None                     # coordinates, but no grid size
+        assert native.engine_for(model, dict(without, grid_size=0.04)) is not None
+        for ends in ([n - 1], [n + 1], [n + 5, n], [n, 5, n]):
+            with pytest.raises(Ptv3Error):
+                model(dict(data, offset=torch.tensor(ends, device=DEV)))
+        assert torch.equal(model(dict(data, offset=torch.tensor([0, int(data["offset"][0]), n], device=DEV))).offset,
+                           torch.tensor([0, int(data["offset"][0]), n], device=DEV))   # an empty scene is one
+        torch.manual_seed(9)
+        a = model(dict(data, batch=batch)).feat
+        torch.manual_seed(9)
+        assert torch.equal(a, model(dict(data)).feat) and want.shape == a.shape
