@@ -160,14 +160,13 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void patch_attn_half_kernel(
     float* knorm_lds = (float*)(vt_lds + (size_t)HD * vt_stride);
     unsigned char* const_lds = (unsigned char*)knorm_lds + ((lds_keys / 64 * 4 + 15) & ~15);
 
-    // The first `full_items` work-groups take one (sequence, head) each. The items left over
-    // after the last full round of resident work-groups are cut into `split` query ranges, one
-    // work-group each, so that the partial round at the end of the launch is short.
+    // The first `full_items` work-groups take one (sequence, head) each; the items left over are cut into
+    // `split` query ranges, one work-group each (tail_split).
     int wg, part = 0, parts = 1;
     if ((int)blockIdx.x < full_items) {
         wg = xcd_chunked_id(blockIdx.x, full_items);
     } else {
-        // Work-group ids go round the XCDs (full_items is a multiple of the resident work-groups). Every XCD takes a
+        // Work-group ids go round the XCDs (full_items is a multiple of the CUs). Every XCD takes a
         // contiguous eighth of the tail's items, range after range of one item, then the next item: the ranges of
         // an item meet in one L2 (the keys and values the later ranges stage are there), and so do the heads of a
         // sequence, which read neighbouring pieces of the same cache lines.
@@ -508,6 +507,26 @@ bool half_kernel_takes(int dtype, int channels, int heads, int64_t max_seqlen) {
     return dtype != PTV3_F32 && channels / heads == HD && half_lds_bytes(max_seqlen) <= 160 * 1024;
 }
 
+// How a launch is cut. Two work-groups are resident per CU (LDS), but one alone keeps the VALU of its CU nearly as busy as
+// two do: an item of 1024 slots takes 36 us by itself on a CU and 33.5 per item with company. So a launch lasts as long as
+// the CU with the most items, not the most rounds of two: items up to the last multiple of the CU count go out whole, the
+// rest are cut into `split` ranges of query tiles, as many as make the fullest CU's share of tiles least; the staging
+// that every range repeats counts as four tiles. Where there are no whole items, a range alone on its CU also waits for
+// its own staging (eight). Measured (fp16, 1024 slots; us, rounds of two with up to four ranges before / this): 312 items
+// 57 -> 48, 788: 114 -> 105, 592: 83.4 -> 80.4, 192: 43.8 -> 39.1, 96 of 800 slots: 20.7 -> 19.0, 40 of 704: 13.1 -> 11.1,
+// 4 items: 15.2 -> 12.9. Ranges of less than four tiles gain nothing (4 items in 16 ranges: 13.0).
+int64_t tail_split(int64_t total, int64_t cus, int64_t tiles, int64_t* full) {
+    const int64_t rem = total % cus;
+    int64_t split = 1, best = tiles + (total < cus ? 8 : 4);
+    for (int64_t sp = 2; sp <= 8 && tiles >= 4 * sp; ++sp) {
+        const int64_t per_cu = ptv3_ceil_div(rem * sp, cus);
+        const int64_t cost = per_cu * (ptv3_ceil_div(tiles, sp) + (per_cu == 1 && total < cus ? 8 : 4));
+        if (cost < best) { best = cost; split = sp; }
+    }
+    *full = split == 1 ? total : total - rem;
+    return split;
+}
+
 template <typename T, bool LSE, bool DROP>
 int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_src,
                 const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
@@ -520,28 +539,17 @@ int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_sr
     static LdsGrant grant_lds_allowed;   // per instantiation and device; raised monotonically
     if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_lds_allowed)) return rc_;
     const float scale_log2e = scale * 1.4426950408889634f;
-    // resident work-groups: two per CU (LDS-bound)
-    static int slots = 0;
-    if (slots == 0) {
-        int dev = 0, cus = 0;
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-        slots = 2 * cus;
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        cus = n;
     }
-    // Items beyond the last full round of resident work-groups are cut into `split` query ranges
-    // (each re-stages K/V, about a tenth of an item): pick the split that makes the tail shortest.
     const int64_t total = n_seq * heads;
-    const int64_t rem = total % slots;
-    int64_t full = total - rem, split = 1;
-    if (rem != 0) {
-        double best = 1.0;
-        for (int64_t sp = 2; sp <= 4; ++sp) {
-            const double cost = (double)((rem * sp + slots - 1) / slots) / (double)sp + 0.1;
-            if (cost < best - 1e-9) { best = cost; split = sp; }
-        }
-    }
-    if (split == 1) full = total;
+    int64_t full = 0;
+    const int64_t split = tail_split(total, cus, ptv3_ceil_div(max_seqlen, 32), &full);
     const int64_t tail = (total - full + 7) / 8 * 8;   // the tail's items in groups of 8, one per XCD
     hipLaunchKernelGGL(kern, dim3((unsigned)(full + tail * split)), dim3(ATT_THREADS), lds, stream,
                        (const T*)qkv, channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys,

@@ -81,6 +81,18 @@ def test_attention_patch_1024_launch_shapes(dtype, counts, heads):
     assert rel_err(got, want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("counts,patch,heads", [([1024] * 65, 1024, 4),        # 256 items whole, 4 in eight ranges
+                                                ([20_000, 20_500], 1024, 8),  # 328: 256 whole, the rest in ranges
+                                                ([3500, 20], 704, 8),         # 48 items, ranges of unequal length
+                                                ([86_016], 1024, 2),          # 168 items in three ranges
+                                                ([6000], 288, 1),             # nine tiles: two ranges at most
+                                                ([40_000], 96, 3)])           # three tiles: never cut
+def test_attention_ranges_of_cut_items(counts, patch, heads):
+    """The items left over after every CU has the same number are cut into 2 ... 8 ranges of query tiles."""
+    got, want = _case(counts, patch, heads, torch.float16, seed=sum(counts) + heads)
+    assert rel_err(got, want) < TOL[torch.float16]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_is_deterministic(dtype):
     """Two launches over the same input give the same bits."""
