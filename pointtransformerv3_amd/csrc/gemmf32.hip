@@ -1,24 +1,31 @@
-// fp32 products on the matrix cores (v_mfma_f32_32x32x2f32: full fp32 operands and accumulation): Linear layers of the
-// float model and the pair form of the float submanifold convolution.
+// fp32 products on the matrix cores: Linear layers of the float model and the pair form of the float submanifold
+// convolution.
 //
-// A work-group of four waves owns TM rows x TN outputs. 16 inputs of its rows and of its weight rows at a time go
-// global -> registers -> LDS (two buffers, one barrier per step); a lane reads four consecutive inputs of its row or
-// weight row as one 16-byte LDS word and feeds them to four MFMAs (the inputs of a step are taken in the order
-// {j, 4 + j}, the same on both sides). The matrix pipe bounds it: a 32 x 32 x 2 product holds the pipe for 64 cycles and
-// needs one register per operand, so LDS and L2 are nearly idle and a plain two-buffer pipeline is enough; the fp32
-// rate of the pipe (157 TFLOP/s) is twice what unpacked VALU FMAs could reach.
+// A float is taken as the sum of two halves, h = half(v 2^S) and l = half((v 2^S - h) 2^11): 22 bits and both signs, and a
+// product is h h' + 2^-11 (h l' + l h') with float sums, three v_mfma_f32_32x32x16_f16 in 96 cycles where eight
+// v_mfma_f32_32x32x2_f32 take 512. What the pieces leave out (l l' and the half of the last bit) is below what the longer
+// chain of roundings of the float instruction adds: error against 64 bits (2-norm, unit normal operands), float
+// instruction -> pieces: K = 32 1.03e-7 -> 0.91e-7, 64 1.44e-7 -> 0.98e-7, 256 2.87e-7 -> 1.31e-7, 2048 8.1e-7 -> 3.0e-7. Below
+// 32 inputs it is not (K = 6: 0.47e-7 -> 0.88e-7), and those layers, and every tile where the pieces do not carry the
+// values, are taken on whole floats: `again` below.
 //
-// Measured (MI355X, float model on one room of 100k voxels): the 23 convolutions of a forward take 3.7 ms with their
-// segment sums, where one thread per (voxel, output) walking the stored neighbour map took 506 ms; its dense layers
-// 5.2 ms, where 64 x 64 tiles of VALU FMAs took 10 ms. Forward 530 -> 11.6 ms. A large product runs at 60 % of the
-// 153 TFLOP/s a library reaches on this part.
+// A work-group of four waves owns TM rows x TN outputs. KC inputs of its rows and of its weight rows at a time go
+// global -> registers -> pieces in LDS, two buffers and one barrier per step; the loads of two steps are on the way, none of
+// them under a condition (a condition made the compiler wait for all of them), and the splitting of the next step is
+// scheduled between the products of this one. Bound by the splitting (VALU) and by the latency of a step where a launch has
+// few tiles, by memory at 32 and 64 inputs.
+// Measured (MI355X; us, float instruction -> pieces): 100k x 64 -> 192 40 -> 29, 36k x 128 -> 384 55 -> 31,
+// 11.6k x 256 -> 1024 74 -> 34, 4.8k x 2048 -> 512 125 -> 63, 300 x 2048 -> 512 41 -> 30; a float forward of one room of 100k
+// voxels 10.9 -> 7.8 ms.
 #include "rowtile.h"
 
 namespace {
 
-constexpr int F32_KC = 16;              // inputs per step
-constexpr int F32_STRIDE = F32_KC + 4;  // floats per LDS row: 5 16-byte words, rows start in distinct bank groups
 constexpr int F32_THREADS = 256;
+// Scales of the pieces: rows up to 16376 (2^16 / 4) and weights up to 255 are carried, rows whose largest value is below
+// 2^-16 and weight rows below 2^-22 would lose bits of the second piece. Rows that are halves already are their first piece.
+constexpr int F32_SX = 2, F32_SW = 8;
+constexpr int F32_MIN_K = 32;   // fewer inputs: whole floats
 
 struct F32Args {
     const void* x;          // (rows, k) float or half
@@ -34,44 +41,70 @@ struct F32Args {
     int taps;
 };
 
+// Four values of a row of k from place `at` on; places past the row's end read its last ones again, and are made zero
+// before they are parked (cut).
 template <typename XT, bool VEC> struct Load4;
 template <> struct Load4<float, true> {
-    static __device__ __forceinline__ f32x4 at(const float* p, int left) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (left >= 4) v = *(const f32x4*)p;
-        return v;
-    }
+    typedef f32x4 raw;
+    static __device__ __forceinline__ raw at(const float* p, int at, int k) { return *(const f32x4*)(p + min(at, k - 4)); }
+    static __device__ __forceinline__ f32x4 value(raw v) { return v; }
+    static __device__ __forceinline__ raw cut(raw v, int left) { return left > 0 ? v : (f32x4){0.f, 0.f, 0.f, 0.f}; }
 };
 template <> struct Load4<float, false> {
-    static __device__ __forceinline__ f32x4 at(const float* p, int left) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    typedef f32x4 raw;
+    static __device__ __forceinline__ raw at(const float* p, int at, int k) {
+        f32x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j < left) v[j] = p[j];
+        for (int j = 0; j < 4; ++j) v[j] = p[min(at + j, k - 1)];
+        return v;
+    }
+    static __device__ __forceinline__ f32x4 value(raw v) { return v; }
+    static __device__ __forceinline__ raw cut(raw v, int left) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = j < left ? v[j] : 0.f;
         return v;
     }
 };
 template <> struct Load4<_Float16, true> {
-    static __device__ __forceinline__ f32x4 at(const _Float16* p, int left) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (left >= 4) {
-            const u32x2 r = *(const u32x2*)p;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                v[2 * j] = H16<_Float16>::lo(r[j]);
-                v[2 * j + 1] = H16<_Float16>::hi(r[j]);
-            }
-        }
-        return v;
+    typedef u32x2 raw;
+    static __device__ __forceinline__ raw at(const _Float16* p, int at, int k) { return *(const u32x2*)(p + min(at, k - 4)); }
+    static __device__ __forceinline__ f32x4 value(raw v) {
+        return (f32x4){H16<_Float16>::lo(v[0]), H16<_Float16>::hi(v[0]), H16<_Float16>::lo(v[1]), H16<_Float16>::hi(v[1])};
     }
+    static __device__ __forceinline__ raw cut(raw v, int left) { return left > 0 ? v : (u32x2){0u, 0u}; }
 };
 
-template <int TM, int TN, int WM, int WN, typename XT, typename OT, bool VEC, bool PAIRS>
+// four consecutive values of a row as pieces, the second ones KC halves behind the first
+template <int S, int KC> __device__ __forceinline__ void park_pieces(unsigned char* at, f32x4 v) {
+    u32x2 h, l;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const f16x2 t = __builtin_convertvector((f32x2){v[2 * j] * (float)(1 << S), v[2 * j + 1] * (float)(1 << S)}, f16x2);
+        h[j] = __builtin_bit_cast(uint32_t, t);
+        l[j] = H16<_Float16>::pack2(fmaf((float)t[0], -2048.f, v[2 * j] * (float)(2048 << S)),
+                                    fmaf((float)t[1], -2048.f, v[2 * j + 1] * (float)(2048 << S)));
+    }
+    *(u32x2*)at = h;
+    *(u32x2*)(at + KC * 2) = l;
+}
+// max(m, |v|): two instructions; fmaxf would quiet every operand first
+__device__ __forceinline__ float largest(float m, f32x4 v) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v[0]), "v"(v[1]));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v[2]), "v"(v[3]));
+    return m;
+}
+
+template <int TM, int TN, int WM, int WN, int KC, typename XT, typename OT, bool VEC, bool PAIRS>
 __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
     static_assert(WM * WN == 4 && TM % (32 * WM) == 0 && TN % (32 * WN) == 0, "four waves share the tile");
     constexpr int MT = TM / (32 * WM), NT = TN / (32 * WN);
-    constexpr int XP = (TM * 4 + F32_THREADS - 1) / F32_THREADS, WP = (TN * 4 + F32_THREADS - 1) / F32_THREADS;
-    __shared__ float lds[2][(TM + TN) * F32_STRIDE];
+    constexpr int RL = KC / 4;                  // lanes that hold a row's values of a step, four each
+    constexpr int XP = (TM * RL + F32_THREADS - 1) / F32_THREADS, WP = (TN * RL + F32_THREADS - 1) / F32_THREADS;
+    constexpr int ROW = 2 * KC * 2 + 16;        // bytes of an LDS row of pieces: rows start in distinct bank groups
+    constexpr int STRIDE = KC + 4;              // floats of an LDS row of whole values
+    constexpr bool XHALF = sizeof(XT) == 2;   // a half is its own first piece
+    constexpr int SX = XHALF ? 0 : F32_SX;
+    __shared__ __align__(16) unsigned char lds[2][(TM + TN) * ROW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hf = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
@@ -118,95 +151,215 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
     // staging: piece e of a tile is 16 bytes of row e / 4; rows and outputs past the end repeat the last one
     const XT* xrow[XP];
     const float* wrow[WP];
-    const int pc = (tid & 3) * 4;
+    const int pc = (tid % RL) * 4;
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
-        int r = (tid + i * F32_THREADS) >> 2;
+        int r = (tid + i * F32_THREADS) / RL;
         r = min(r, count - 1);
         const int64_t src = PAIRS ? (int64_t)g.pair_in[start + r] : start + r;
-        xrow[i] = (const XT*)g.x + src * g.k + pc;
+        xrow[i] = (const XT*)g.x + src * g.k;
     }
 #pragma unroll
     for (int i = 0; i < WP; ++i) {
-        const int c = min(col0 + ((tid + i * F32_THREADS) >> 2), g.nout - 1);
-        wrow[i] = g.w + (int64_t)c * g.w_row + (int64_t)tap * g.w_tap + pc;
+        const int c = min(col0 + ((tid + i * F32_THREADS) / RL), g.nout - 1);
+        wrow[i] = g.w + (int64_t)c * g.w_row + (int64_t)tap * g.w_tap;
     }
-    f32x4 xr[XP], wr[WP];
-    auto fetch = [&](int k0) {
-        const int left = g.k - k0 - pc;
+    float xm[XP], wm_[WP];   // the largest value of a row among this thread's pieces
 #pragma unroll
-        for (int i = 0; i < XP; ++i) xr[i] = Load4<XT, VEC>::at(xrow[i] + k0, left);
+    for (int i = 0; i < XP; ++i) xm[i] = 0.f;
 #pragma unroll
-        for (int i = 0; i < WP; ++i) wr[i] = Load4<float, VEC>::at(wrow[i] + k0, left);
+    for (int i = 0; i < WP; ++i) wm_[i] = 0.f;
+    struct Stage {   // two steps are on the way
+        typename Load4<XT, VEC>::raw x[XP];
+        f32x4 w[WP];
+    } st0, st1;
+    auto fetch = [&](Stage& t, int k0) {
+#pragma unroll
+        for (int i = 0; i < XP; ++i) t.x[i] = Load4<XT, VEC>::at(xrow[i], k0 + pc, g.k);
+#pragma unroll
+        for (int i = 0; i < WP; ++i) t.w[i] = Load4<float, VEC>::at(wrow[i], k0 + pc, g.k);
     };
-    auto park = [&](int buf) {
+    auto trim = [&](Stage& t, int s) {   // the last step of a row that is no whole number of steps
+        const int left = g.k - s * KC - pc;
+        if (left >= KC - pc) return;
+#pragma unroll
+        for (int i = 0; i < XP; ++i) t.x[i] = Load4<XT, VEC>::cut(t.x[i], left);
+#pragma unroll
+        for (int i = 0; i < WP; ++i) t.w[i] = Load4<float, VEC>::cut(t.w[i], left);
+    };
+    auto park = [&](const Stage& t, int s) {
+        unsigned char* to = lds[s & 1] + pc * 2;
 #pragma unroll
         for (int i = 0; i < XP; ++i) {
             const int e = tid + i * F32_THREADS;
-            if (TM * 4 % F32_THREADS == 0 || e < TM * 4) *(f32x4*)(&lds[buf][(e >> 2) * F32_STRIDE + pc]) = xr[i];
+            const f32x4 v = Load4<XT, VEC>::value(t.x[i]);
+            if (!XHALF) xm[i] = largest(xm[i], v);
+            if (TM * RL % F32_THREADS == 0 || e < TM * RL) park_pieces<SX, KC>(to + (e / RL) * ROW, v);
         }
 #pragma unroll
         for (int i = 0; i < WP; ++i) {
             const int e = tid + i * F32_THREADS;
-            if (TN * 4 % F32_THREADS == 0 || e < TN * 4) *(f32x4*)(&lds[buf][(TM + (e >> 2)) * F32_STRIDE + pc]) = wr[i];
+            wm_[i] = largest(wm_[i], t.w[i]);
+            if (TN * RL % F32_THREADS == 0 || e < TN * RL) park_pieces<F32_SW, KC>(to + (TM + (e / RL)) * ROW, t.w[i]);
         }
     };
 
-    f32x16 acc[MT][NT];
+    f32x16 acc[MT][NT], low[MT][NT];   // sums of h h', and of (h l' + l h') 2^11
+    const int steps = (g.k + KC - 1) / KC;
+    auto clear = [&](f32x16 (&t)[MT][NT]) {
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int b = 0; b < NT; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) t[a][b][v] = 0.f;
+    };
+
+    // step s from buffer s & 1; `t` holds step s + 1 and takes step s + 3
+    auto step = [&](int s, Stage& t) {
+        trim(t, s + 1);
+        const unsigned char* xs = lds[s & 1] + (wm * MT * 32 + col) * ROW + hf * 16;
+        const unsigned char* ws = lds[s & 1] + (TM + wn * NT * 32 + col) * ROW + hf * 16;
+#pragma unroll
+        for (int c = 0; c < KC / 16; ++c) {
+            f16x8 xa[MT][2], wb[NT][2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int off = c * 32 + q * KC * 2;
+#pragma unroll
+                for (int a = 0; a < MT; ++a)
+                    if (q == 0 || !XHALF) xa[a][q] = __builtin_bit_cast(f16x8, *(const u32x4*)(xs + a * 32 * ROW + off));
+#pragma unroll
+                for (int b = 0; b < NT; ++b) wb[b][q] = __builtin_bit_cast(f16x8, *(const u32x4*)(ws + b * 32 * ROW + off));
+            }
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < NT; ++b) {
+                    acc[a][b] = H16<_Float16>::mfma(xa[a][0], wb[b][0], acc[a][b]);
+                    low[a][b] = H16<_Float16>::mfma(xa[a][0], wb[b][1], low[a][b]);
+                    if (!XHALF) low[a][b] = H16<_Float16>::mfma(xa[a][1], wb[b][0], low[a][b]);
+                }
+        }
+        park(t, s + 1);
+        fetch(t, (s + 3) * KC);
+#pragma unroll
+        for (int i = 0; i < KC / 16 * MT * NT * (XHALF ? 2 : 3); ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one product, then the splitting of the next step's values
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+        }
+        __syncthreads();
+    };
+    const bool pieces = g.k >= F32_MIN_K;
+    clear(acc);
+    clear(low);
+    if (pieces) {
+        fetch(st0, 0);
+        fetch(st1, KC);
+        trim(st0, 0);
+        park(st0, 0);
+        fetch(st0, 2 * KC);
+        __syncthreads();
+        for (int s = 0; s < steps; s += 2) {
+            step(s, st1);
+            if (s + 1 < steps) step(s + 1, st0);
+        }
+    }
+
+    // Where the pieces do not carry a float - a sum that is not finite (infinities, NaN, values beyond a piece's range), a
+    // row whose values are all so small that the second piece runs out of bits - the work-group takes its tile again on
+    // whole floats.
+    float odd = 0.f;
 #pragma unroll
     for (int a = 0; a < MT; ++a)
 #pragma unroll
         for (int b = 0; b < NT; ++b)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-
-    const int steps = (g.k + F32_KC - 1) / F32_KC;
-    fetch(0);
-    park(0);
-    __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-        if (s + 1 < steps) fetch((s + 1) * F32_KC);
-        const float* xs = &lds[s & 1][(wm * MT * 32 + col) * F32_STRIDE + hf * 4];
-        const float* ws = &lds[s & 1][(TM + wn * NT * 32 + col) * F32_STRIDE + hf * 4];
+            for (int v = 0; v < 16; ++v) {
+                acc[a][b][v] = fmaf(low[a][b][v], 1.f / 2048.f, acc[a][b][v]) * (1.f / (float)(1 << (SX + F32_SW)));
+                odd = fmaf(acc[a][b][v], 0.f, odd);
+            }
+    bool again = odd != 0.f || !pieces;
+    auto small = [&](float m, float least) {   // RL neighbouring lanes hold a row
 #pragma unroll
-        for (int c = 0; c < F32_KC / 8; ++c) {
-            f32x4 xa[MT], wb[NT];
+        for (int off = 1; off < RL; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, PTV3_WAVE));
+        again |= m > 0.f && m < least;
+    };
 #pragma unroll
-            for (int a = 0; a < MT; ++a) xa[a] = *(const f32x4*)(xs + a * 32 * F32_STRIDE + c * 8);
+    for (int i = 0; i < XP; ++i)
+        if (!XHALF) small(xm[i], 1.f / (float)(1 << (14 + F32_SX)));
 #pragma unroll
-            for (int b = 0; b < NT; ++b) wb[b] = *(const f32x4*)(ws + b * 32 * F32_STRIDE + c * 8);
+    for (int i = 0; i < WP; ++i) small(wm_[i], 1.f / (float)(1 << (14 + F32_SW)));
+    if (__syncthreads_or(again)) {
+        float* whole = (float*)lds;
+        clear(acc);
+        for (int s = 0; s < steps; ++s) {
+            fetch(st0, s * KC);
+            trim(st0, s);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int i = 0; i < XP; ++i) {
+                const int e = tid + i * F32_THREADS;
+                if (TM * RL % F32_THREADS == 0 || e < TM * RL)
+                    *(f32x4*)(whole + (e / RL) * STRIDE + pc) = Load4<XT, VEC>::value(st0.x[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < WP; ++i) {
+                const int e = tid + i * F32_THREADS;
+                if (TN * RL % F32_THREADS == 0 || e < TN * RL) *(f32x4*)(whole + (TM + (e / RL)) * STRIDE + pc) = st0.w[i];
+            }
+            __syncthreads();
+            const float* xs = whole + (wm * MT * 32 + col) * STRIDE + hf;
+            const float* ws = whole + (TM + wn * NT * 32 + col) * STRIDE + hf;
+#pragma unroll 2
+            for (int c = 0; c < KC; c += 2)
 #pragma unroll
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
                     for (int b = 0; b < NT; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[a][j], wb[b][j], acc[a][b], 0, 0, 0);
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[a * 32 * STRIDE + c],
+                                                                         ws[b * 32 * STRIDE + c], acc[a][b], 0, 0, 0);
+            __syncthreads();
         }
-        if (s + 1 < steps) park((s + 1) & 1);
-        __syncthreads();
     }
 
     // acc[a][b][v]: row 8*(v/4) + 4*hf + v%4 of its 32, output `col`: a store instruction writes two 128-byte runs
 #pragma unroll
-    for (int b = 0; b < NT; ++b) {
-        const int c = col0 + (wn * NT + b) * 32 + col;
-        if (c >= g.nout) continue;
-        const float bias = g.bias ? g.bias[c] : 0.f;
+    for (int a = 0; a < MT; ++a) {
+        const int r0 = (wm * MT + a) * 32 + 4 * hf;
+        int64_t at[16];
 #pragma unroll
-        for (int a = 0; a < MT; ++a)
+        for (int v = 0; v < 16; ++v) {
+            const int r = min(r0 + 8 * (v / 4) + (v & 3), count - 1);
+            at[v] = (PAIRS ? (int64_t)g.pair_slot[start + r] : start + r) * g.nout;
+        }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int r = (wm * MT + a) * 32 + 8 * (v / 4) + 4 * hf + (v & 3);
-                if (r >= count) continue;
-                const int64_t at = (PAIRS ? (int64_t)g.pair_slot[start + r] : start + r) * g.nout + c;
-                float y = acc[a][b][v] + bias;
-                if (!PAIRS) {
-                    if (g.gelu) y = 0.5f * y * (1.f + erff(y * 0.70710678118654752f));
-                    if (g.resid) y += g.resid[at];
-                }
-                ((OT*)g.out)[at] = (OT)y;
+        for (int b = 0; b < NT; ++b) {
+            const int c = col0 + (wn * NT + b) * 32 + col;
+            if (c >= g.nout) continue;
+            const float bias = g.bias ? g.bias[c] : 0.f;
+            f32x16 y = acc[a][b];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) y[v] += bias;
+            if (!PAIRS && g.gelu) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = 0.5f * y[v] * (1.f + erff(y[v] * 0.70710678118654752f));
             }
+            if (!PAIRS && g.resid) {
+                f32x16 r;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) r[v] = g.resid[at[v] + c];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] += r[v];
+            }
+            if (count == TM) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) ((OT*)g.out)[at[v] + c] = (OT)y[v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (r0 + 8 * (v / 4) + (v & 3) < count) ((OT*)g.out)[at[v] + c] = (OT)y[v];
+            }
+        }
     }
 }
 
@@ -219,21 +372,24 @@ int launch_f32(F32Args& g, int64_t rows, hipStream_t stream) {
         const int64_t tiles = (rows / tm + (PAIRS ? extra : (rows % tm != 0))) * ptv3_ceil_div(g.nout, tn);
         return (double)ptv3_ceil_div(tiles, 256) * tm * tn * weight;
     };
-#define PTV3_TILE(TM, TN, WM, WN)                                                                              \
+#define PTV3_TILE(TM, TN, WM, WN, KC)                                                                          \
     do {                                                                                                      \
         const int64_t rt = rows / TM + (PAIRS ? extra : (rows % TM != 0));                                    \
         g.col_tiles = (int)ptv3_ceil_div(g.nout, TN);                                                         \
         if (rt * g.col_tiles >= (1ll << 31)) return PTV3_EINVAL;                                              \
         g.row_tiles = (int)rt;                                                                                \
-        hipLaunchKernelGGL((gemm_f32_kernel<TM, TN, WM, WN, XT, OT, VEC, PAIRS>),                             \
+        hipLaunchKernelGGL((gemm_f32_kernel<TM, TN, WM, WN, KC, XT, OT, VEC, PAIRS>),                             \
                            dim3((unsigned)(rt * g.col_tiles)), dim3(F32_THREADS), 0, stream, g);              \
         PTV3_RETURN_LAUNCH();                                                                                 \
     } while (0)
-    if (g.nout <= 32) PTV3_TILE(128, 32, 4, 1);
+    if (g.nout <= 32) PTV3_TILE(128, 32, 4, 1, 16);
     const double c11 = cost(128, 128, 1.0), c10 = cost(128, 64, 1.05), c00 = cost(64, 64, 1.12);
-    if (g.nout > 64 && c11 <= c10 && c11 <= c00) PTV3_TILE(128, 128, 2, 2);
-    if (c10 <= c00) PTV3_TILE(128, 64, 2, 2);
-    PTV3_TILE(64, 64, 2, 2);
+    if (g.nout > 64 && c11 <= c10 && c11 <= c00) PTV3_TILE(128, 128, 2, 2, 16);
+    if (c10 <= c00) PTV3_TILE(128, 64, 2, 2, 16);
+    // steps of 32 inputs halve the barriers of a long row (300 x 2048 -> 512 39 -> 30 us, 11.6k x 1024 -> 256 43 -> 37); a short
+    // one is sooner through its first step with 16 (100k x 64 -> 256 37 against 45)
+    if (g.k >= 256) PTV3_TILE(64, 64, 2, 2, 32);
+    PTV3_TILE(64, 64, 2, 2, 16);
 #undef PTV3_TILE
 }
 

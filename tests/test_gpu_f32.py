@@ -39,6 +39,37 @@ def test_linear_f32_halves_on_one_side(n, k, nout):
     assert torch.equal(o.linear_f32(x.half(), w, b), o.linear_f32(x.half().float(), w, b))
 
 
+@pytest.mark.parametrize("k", [20, 31, 32, 33, 64, 255, 256, 260])
+@pytest.mark.parametrize("x_scale,w_scale", [(1.0, 1.0), (3e3, 30.0), (1e-4, 1e-6), (1e-7, 1.0), (1.0, 1e-9), (1e30, 1.0), (1.0, 400.0)])
+def test_linear_f32_ranges(k, x_scale, w_scale):
+    """Scales that two halves carry, and scales where a tile is taken on whole floats: every row as exact as float sums
+    are. A sum of k products rounded k times is off by at most k 2^-24 of the sum of their sizes; half of it, and an
+    eighth of it for the longer rows, holds for either way (roundings do not all point the same way)."""
+    g = torch.Generator().manual_seed(k)
+    x, w = torch.randn(300, k, generator=g) * x_scale, torch.randn(70, k, generator=g) * w_scale
+    x[7] *= 1e-9     # one row far below the others, one of zeros
+    x[8] = 0.0
+    w[5] *= 1e-9
+    want = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()
+    got = ops().linear_f32(x.to(DEV), w.to(DEV)).cpu().double()
+    bound = size * (k * 2.0 ** -24 / (8 if k >= 64 else 2)) + 1e-42
+    assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("k", [16, 64, 256])
+def test_linear_f32_infinities_and_nan(k):
+    g = torch.Generator().manual_seed(k)
+    x, w = torch.randn(200, k, generator=g), torch.randn(70, k, generator=g)
+    x[3, 5], x[10, 2], x[40, 0], w[7, 7] = float("inf"), float("nan"), 3.0e38, -float("inf")
+    w[:, 0] = w[:, 0].abs() + 2.0     # 3e38 times more than two leaves the range whatever else is added
+    x[40, 7] = -1.0                   # and meets no infinity of the other sign
+    want = (x.double() @ w.double().t()).float()
+    got = ops().linear_f32(x.to(DEV), w.to(DEV)).cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got.sign()[want.isinf()], want.sign()[want.isinf()])
+
+
 @pytest.mark.parametrize("ks,cin,cout,n,extent", [(3, 32, 32, 400, 12), (3, 64, 64, 3000, 18), (3, 128, 128, 60, 5),
                                                   (3, 20, 36, 700, 10), (5, 6, 32, 900, 14), (5, 3, 5, 40, 6),
                                                   (3, 256, 256, 1500, 14)])
