@@ -61,33 +61,65 @@ __device__ __forceinline__ void ln_lane_pair(float (&val)[OT][16], float eps, co
         }
 }
 
-// copy an (rows x C) weight matrix into LDS rows of stride `stride`; PERM stores the input axis of
-// every 32-block in MFMA result-register order
-template <typename T, bool PERM>
-__device__ __forceinline__ void stage_weight(T* __restrict__ dst, const T* __restrict__ src, int rows, int c,
-                                             int stride, int tid) {
-    if (PERM) {
-        for (int e = tid; e < rows * c; e += BLK_THREADS) {
-            const int r = e / c, k = e % c;
-            dst[r * stride + (k & ~31) + perm32(k & 31)] = src[(int64_t)r * c + k];
+// Weights and vectors of a work-group on their way from memory to LDS: everything is asked for before anything is waited
+// for. A launch of few tiles is as long as its trips to memory, one after the other: with the weights whose input axis is
+// stored in MFMA result-register order copied two bytes at a time and every vector behind a loop of its own, 1500 rows of 64
+// channels took 9.0 us (head) and 15.5 (tail), with this 7.7 and 13.1; 100k rows 18.1 -> 16.2 and 29.5 -> 26.5; 403k, where the
+// memory of the rows bounds both, 1 - 3 % less.
+template <int PIECES> struct Staged { u32x4 v[PIECES]; };
+
+// an (ROWS x C) matrix, 16 bytes at a time
+template <typename T, int ROWS, int C>
+__device__ __forceinline__ Staged<(ROWS * C / 8 + BLK_THREADS - 1) / BLK_THREADS> fetch_weight(const T* __restrict__ src, int tid) {
+    constexpr int N = ROWS * C / 8, PIECES = (N + BLK_THREADS - 1) / BLK_THREADS;
+    Staged<PIECES> s;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) s.v[i] = *(const u32x4*)(src + (int64_t)min(tid + i * BLK_THREADS, N - 1) * 8);
+    return s;
+}
+// into LDS rows of STRIDE; PERM stores the input axis of every 32-block in MFMA result-register order, which keeps fours
+// together (perm32)
+template <typename T, bool PERM, int ROWS, int C, int STRIDE, int PIECES>
+__device__ __forceinline__ void park_weight(T* __restrict__ dst, const Staged<PIECES>& s, int tid) {
+    constexpr int N = ROWS * C / 8;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int e = tid + i * BLK_THREADS;
+        if (N % BLK_THREADS != 0 && e >= N) break;
+        const int r = e / (C / 8), k = e % (C / 8) * 8;
+        if (PERM) {
+            T* to = dst + r * STRIDE + (k & ~31) + perm32(k & 31);
+            *(u32x2*)to = (u32x2){s.v[i][0], s.v[i][1]};
+            *(u32x2*)(to + 16) = (u32x2){s.v[i][2], s.v[i][3]};
+        } else {
+            *(u32x4*)(dst + r * STRIDE + k) = s.v[i];
         }
-    } else {
-        const int ppr = c / 8;
-        for (int e = tid; e < rows * ppr; e += BLK_THREADS) {
-            const int r = e / ppr, pc = e % ppr;
-            *(u32x4*)(dst + r * stride + pc * 8) = *(const u32x4*)(src + (int64_t)r * c + pc * 8);
+    }
+}
+// entry `at` of a vector, or what stands for it where the pointer is null
+template <typename T>
+__device__ __forceinline__ float vec_entry(const T* __restrict__ src, int at, float fill) { return src ? (float)src[at] : fill; }
+
+// 32 rows of C channels of two matrices, 16-byte pieces in lane order; rows past the end are zero
+template <typename T, int C, int IT>
+__device__ __forceinline__ void fetch_rows(const T* __restrict__ a, const T* __restrict__ b, int64_t row0, int64_t n, int lane,
+                                           u32x4 (&xr)[IT], u32x4 (&rr)[IT]) {
+    constexpr int PPR = C / 8;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int pidx = it * PTV3_WAVE + lane;
+        const int64_t r = row0 + pidx / PPR;
+        xr[it] = (u32x4){0, 0, 0, 0};
+        rr[it] = (u32x4){0, 0, 0, 0};
+        if (r < n) {
+            xr[it] = *(const u32x4*)(a + r * C + (pidx % PPR) * 8);
+            rr[it] = *(const u32x4*)(b + r * C + (pidx % PPR) * 8);
         }
     }
 }
 
-template <typename T>
-__device__ __forceinline__ void stage_vec(float* __restrict__ dst, const T* __restrict__ src, int len, int tid,
-                                          float fill) {
-    for (int e = tid; e < len; e += BLK_THREADS) dst[e] = src ? (float)src[e] : fill;
-}
-
 template <typename T, int C>
-__global__ __launch_bounds__(BLK_THREADS, 2) void block_head_kernel(
+__global__ __launch_bounds__(BLK_THREADS, 4) void block_head_kernel(
     const T* __restrict__ conv, const T* __restrict__ shortcut, const T* __restrict__ wc,
     const T* __restrict__ bc, const T* __restrict__ gc, const T* __restrict__ bec, float eps_c,
     const T* __restrict__ g1, const T* __restrict__ be1, float eps_1, const T* __restrict__ wq,
@@ -111,33 +143,30 @@ __global__ __launch_bounds__(BLK_THREADS, 2) void block_head_kernel(
     const int col = lane & 31, hf = lane >> 5;
     T* xs = xs_all + wave * (32 * XSS);
 
-    stage_weight<T, false>(wc_lds, wc, C, C, WS, tid);
-    stage_weight<T, true>(wq_lds, wq, 3 * C, C, WS, tid);
-    stage_vec<T>(bc_lds, bc, C, tid, 0.f);
-    stage_vec<T>(gc_lds, gc, C, tid, 1.f);
-    stage_vec<T>(bec_lds, bec, C, tid, 0.f);
-    stage_vec<T>(g1_lds, g1, C, tid, 1.f);
-    stage_vec<T>(be1_lds, be1, C, tid, 0.f);
-    stage_vec<T>(bq_lds, bq, 3 * C, tid, 0.f);
-    __syncthreads();
-
     constexpr int PPR = C / 8;                       // 16-byte pieces per row
     constexpr int IT = 32 * PPR / PTV3_WAVE;         // pieces per lane: 2 (C=32) or 4 (C=64)
     const int64_t n_tiles = (n + 31) / 32;
+    {
+        const auto swc = fetch_weight<T, C, C>(wc, tid);
+        const auto swq = fetch_weight<T, 3 * C, C>(wq, tid);
+        // the vectors' 8 C entries lie one behind the other in LDS, a thread takes one
+        static_assert(8 * C <= BLK_THREADS, "an entry per thread");
+        const int which = tid / C, at = tid % C;
+        float entry = 0.f;
+        if (which < 8) {
+            const T* src = which == 0 ? bc : which == 1 ? gc : which == 2 ? bec : which == 3 ? g1 : which == 4 ? be1 : bq;
+            entry = vec_entry(src, which >= 5 ? tid - 5 * C : at, which == 1 || which == 3 ? 1.f : 0.f);
+        }
+        park_weight<T, false, C, C, WS>(wc_lds, swc, tid);
+        park_weight<T, true, 3 * C, C, WS>(wq_lds, swq, tid);
+        if (which < 8) bc_lds[tid] = entry;
+    }
+    __syncthreads();
+
     for (int64_t tile = (int64_t)blockIdx.x * BLK_WAVES + wave; tile < n_tiles; tile += (int64_t)gridDim.x * BLK_WAVES) {
         const int64_t row0 = tile * 32;
         u32x4 xr[IT], rr[IT];
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int pidx = it * PTV3_WAVE + lane;
-            const int64_t r = row0 + pidx / PPR;
-            xr[it] = (u32x4){0, 0, 0, 0};
-            rr[it] = (u32x4){0, 0, 0, 0};
-            if (r < n) {
-                xr[it] = *(const u32x4*)(conv + r * C + (pidx % PPR) * 8);
-                rr[it] = *(const u32x4*)(shortcut + r * C + (pidx % PPR) * 8);
-            }
-        }
+        fetch_rows<T, C>(conv, shortcut, row0, n, lane, xr, rr);
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int pidx = it * PTV3_WAVE + lane;
@@ -277,33 +306,31 @@ __global__ __launch_bounds__(BLK_THREADS, 2) void block_tail_kernel(
     const int col = lane & 31, hf = lane >> 5;
     T* xs = xs_all + wave * (32 * XSS);
 
-    stage_weight<T, false>(wp_lds, wp, C, C, WS, tid);
-    stage_weight<T, true>(w1_lds, w1, H, C, WS, tid);
-    stage_weight<T, true>(w2_lds, w2, C, H, W2S, tid);
-    stage_vec<T>(bp_lds, bp, C, tid, 0.f);
-    stage_vec<T>(g2_lds, g2, C, tid, 1.f);
-    stage_vec<T>(be2_lds, be2, C, tid, 0.f);
-    stage_vec<T>(b2_lds, b2, C, tid, 0.f);
-    stage_vec<T>(b1_lds, b1, H, tid, 0.f);
-    __syncthreads();
-
     constexpr int PPR = C / 8;
     constexpr int IT = 32 * PPR / PTV3_WAVE;
     const int64_t n_tiles = (n + 31) / 32;
+    {
+        const auto swp = fetch_weight<T, C, C>(wp, tid);
+        const auto sw1 = fetch_weight<T, H, C>(w1, tid);
+        const auto sw2 = fetch_weight<T, C, H>(w2, tid);
+        static_assert(8 * C <= BLK_THREADS, "an entry of the vectors per thread");
+        const int which = tid / C, at = tid % C;
+        float entry = 0.f;
+        if (which < 8) {
+            const T* src = which == 0 ? bp : which == 1 ? g2 : which == 2 ? be2 : which == 3 ? b2 : b1;
+            entry = vec_entry(src, which >= 4 ? tid - 4 * C : at, which == 1 ? 1.f : 0.f);
+        }
+        park_weight<T, false, C, C, WS>(wp_lds, swp, tid);
+        park_weight<T, true, H, C, WS>(w1_lds, sw1, tid);
+        park_weight<T, true, C, H, W2S>(w2_lds, sw2, tid);
+        if (which < 8) bp_lds[tid] = entry;
+    }
+    __syncthreads();
+
     for (int64_t tile = (int64_t)blockIdx.x * BLK_WAVES + wave; tile < n_tiles; tile += (int64_t)gridDim.x * BLK_WAVES) {
         const int64_t row0 = tile * 32;
         u32x4 xr[IT], rr[IT];
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int pidx = it * PTV3_WAVE + lane;
-            const int64_t r = row0 + pidx / PPR;
-            xr[it] = (u32x4){0, 0, 0, 0};
-            rr[it] = (u32x4){0, 0, 0, 0};
-            if (r < n) {
-                xr[it] = *(const u32x4*)(attn + r * C + (pidx % PPR) * 8);
-                rr[it] = *(const u32x4*)(shortcut + r * C + (pidx % PPR) * 8);
-            }
-        }
+        fetch_rows<T, C>(attn, shortcut, row0, n, lane, xr, rr);
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int pidx = it * PTV3_WAVE + lane;
