@@ -955,12 +955,10 @@ template <typename T>
 __global__ __launch_bounds__(256) void attn_bwd_fill_kernel(const T* __restrict__ fill, int channels,
                                                             const int32_t* __restrict__ slot_src,
                                                             const int32_t* __restrict__ slot_dst, int64_t n_pad,
-                                                            T* __restrict__ dqkv) {
-    const int per = 2 * channels / 8;   // 8-channel pieces per slot
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_pad * per) return;
-    const int64_t slot = i / per;
-    const int piece = (int)(i % per);
+                                                            PieceDiv per, T* __restrict__ dqkv) {   // per: pieces of 8 channels a slot
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = ptv3_row_of(i, per);
+    if (slot >= n_pad) return;
+    const int piece = (int)(i - slot * per.count);
     if (slot_dst[slot] >= 0) return;
     const T* src = fill + slot * 2 * channels + piece * 8;
     T* dst = dqkv + (int64_t)slot_src[slot] * 3 * channels + channels + piece * 8;
@@ -1056,7 +1054,7 @@ int launch_half_bwd(const void* qkv, const void* out, const void* dout, int chan
     }
     const int64_t items = n_pad * (2 * channels / 8);
     hipLaunchKernelGGL(attn_bwd_fill_kernel<T>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
-                       (const T*)ws.fill, channels, slot_src, slot_dst, n_pad, (T*)dqkv);
+                       (const T*)ws.fill, channels, slot_src, slot_dst, n_pad, ptv3_piece_div(2 * channels / 8), (T*)dqkv);
     PTV3_RETURN_LAUNCH();
 }
 
@@ -1115,6 +1113,6 @@ extern "C" int ptv3_patch_attn_rpe_bwd(const void* qkv, const void* out, const v
                        ws.d, (float*)dqkv, (float*)ws.fill, rpe, drop);
     const int64_t items = n_pad * (2 * channels / 8);
     hipLaunchKernelGGL(attn_bwd_fill_kernel<float>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
-                       (const float*)ws.fill, channels, slot_src, slot_dst, n_pad, (float*)dqkv);
+                       (const float*)ws.fill, channels, slot_src, slot_dst, n_pad, ptv3_piece_div(2 * channels / 8), (float*)dqkv);
     PTV3_RETURN_LAUNCH();
 }

@@ -337,12 +337,11 @@ namespace {
 // (n, c) rows in any dtype -> (n, padded) rows in dtype TO, zeros behind the c channels; a thread writes eight channels
 template <typename TI, typename TO>
 __global__ __launch_bounds__(256) void pad_rows_kernel(const TI* __restrict__ x, int64_t n, int c, int padded,
-                                                       TO* __restrict__ out) {
-    const int pieces = padded / 8;
+                                                       PieceDiv pieces, TO* __restrict__ out) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= n * pieces) return;
-    const int64_t i = e / pieces;
-    const int ch = (int)(e - i * pieces) * 8;
+    const int64_t i = ptv3_row_of(e, pieces);
+    if (i >= n) return;
+    const int ch = (int)(e - i * pieces.count) * 8;
     typedef TO vec __attribute__((ext_vector_type(8)));
     vec v;
 #pragma unroll
@@ -396,7 +395,7 @@ extern "C" int ptv3_pad_rows(const void* x, int x_dtype, int64_t n, int c, int p
     if (!x || !out) return PTV3_EINVAL;
     const dim3 grid((unsigned)ptv3_ceil_div(n * (padded / 8), 256)), block(256);
     hipStream_t stream = (hipStream_t)stream_;
-#define PTV3_PAD(TI, TO) hipLaunchKernelGGL((pad_rows_kernel<TI, TO>), grid, block, 0, stream, (const TI*)x, n, c, padded, (TO*)out)
+#define PTV3_PAD(TI, TO) hipLaunchKernelGGL((pad_rows_kernel<TI, TO>), grid, block, 0, stream, (const TI*)x, n, c, padded, ptv3_piece_div(padded / 8), (TO*)out)
     if (out_dtype == PTV3_F16) {
         if (x_dtype == PTV3_F32) PTV3_PAD(float, _Float16);
         else if (x_dtype == PTV3_F16) PTV3_PAD(_Float16, _Float16);

@@ -397,14 +397,13 @@ int launch_f32(F32Args& g, int64_t rows, hipStream_t stream) {
 template <int V>
 __global__ __launch_bounds__(256) void pair_segment_sum_f32_kernel(const float* __restrict__ y,
                                                                    const int32_t* __restrict__ row_ptr, int64_t n,
-                                                                   int cout, const float* __restrict__ bias,
+                                                                   int cout, PieceDiv groups, const float* __restrict__ bias,
                                                                    float* __restrict__ out) {
     typedef float vec __attribute__((ext_vector_type(V)));
-    const int groups = cout / V;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * groups) return;
-    const int64_t i = e / groups;
-    const int c = (int)(e - i * groups) * V;
+    const int64_t i = ptv3_row_of(e, groups);
+    if (i >= n) return;
+    const int c = (int)(e - i * groups.count) * V;
     vec acc;
 #pragma unroll
     for (int k = 0; k < V; ++k) acc[k] = bias ? bias[c + k] : 0.f;
@@ -442,10 +441,10 @@ int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, in
     }
     if (cout % 4 == 0)
         hipLaunchKernelGGL(pair_segment_sum_f32_kernel<4>, dim3((unsigned)ptv3_ceil_div(n * (cout / 4), 256)), dim3(256),
-                           0, stream, y, row_ptr, n, cout, bias, out);
+                           0, stream, y, row_ptr, n, cout, ptv3_piece_div(cout / 4), bias, out);
     else
         hipLaunchKernelGGL(pair_segment_sum_f32_kernel<1>, dim3((unsigned)ptv3_ceil_div(n * cout, 256)), dim3(256), 0,
-                           stream, y, row_ptr, n, cout, bias, out);
+                           stream, y, row_ptr, n, cout, ptv3_piece_div(cout), bias, out);
     PTV3_RETURN_LAUNCH();
 }
 

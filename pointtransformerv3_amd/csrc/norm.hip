@@ -175,11 +175,10 @@ template <typename T, typename S>
 __global__ __launch_bounds__(256) void bn_act_kernel(const T* __restrict__ x, const S* __restrict__ mean,
                                                      const S* __restrict__ var, const T* __restrict__ gamma,
                                                      const T* __restrict__ beta, float eps, int act, int64_t n,
-                                                     int c, T* __restrict__ out) {
-    const int groups = c / 8;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * groups) return;
-    const int ch = (int)(e % groups) * 8;
+                                                     PieceDiv groups, T* __restrict__ out) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, row = ptv3_row_of(e, groups);
+    if (row >= n) return;
+    const int ch = (int)(e - row * groups.count) * 8;
     float v[8], g[8], b[8], mu[8], va[8];
     load8(x + e * 8, v);
     load8(mean + ch, mu);
@@ -267,8 +266,8 @@ template <typename T, typename S>
 void launch_bn_act(const void* x, const void* mean, const void* var, const void* gamma, const void* beta, float eps,
                    int act, int64_t n, int c, void* out, hipStream_t stream) {
     hipLaunchKernelGGL((bn_act_kernel<T, S>), dim3((unsigned)ptv3_ceil_div(n * (c / 8), 256)), dim3(256), 0, stream,
-                       (const T*)x, (const S*)mean, (const S*)var, (const T*)gamma, (const T*)beta, eps, act, n, c,
-                       (T*)out);
+                       (const T*)x, (const S*)mean, (const S*)var, (const T*)gamma, (const T*)beta, eps, act, n,
+                       ptv3_piece_div(c / 8), (T*)out);
 }
 
 extern "C" int ptv3_bn_act(const void* x, const void* running_mean, const void* running_var, int stats_f32,

@@ -213,13 +213,12 @@ template <typename T, int V> struct Pack { T v[V]; };
 
 template <typename T, int V>
 __global__ __launch_bounds__(256) void segment_reduce_kernel(
-    const T* __restrict__ src, int c, const int64_t* __restrict__ indices,
+    const T* __restrict__ src, int c, PieceDiv groups, const int64_t* __restrict__ indices,
     const int64_t* __restrict__ idx_ptr, int64_t m, int op, T* __restrict__ out) {
-    const int groups = c / V;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= m * groups) return;
-    const int64_t s = e / groups;
-    const int ch = (int)(e - s * groups) * V;
+    const int64_t s = ptv3_row_of(e, groups);
+    if (s >= m) return;
+    const int ch = (int)(e - s * groups.count) * V;
     const int64_t b = idx_ptr[s], t = idx_ptr[s + 1];
     float acc[V];
 #pragma unroll
@@ -310,13 +309,12 @@ __global__ __launch_bounds__(1024) void segment_reduce_long_kernel(
 template <typename T, int V>
 __global__ __launch_bounds__(256) void unpool_add_kernel(const T* __restrict__ parent,
                                                          const T* __restrict__ child, int64_t n,
-                                                         int c, const int64_t* __restrict__ cluster,
+                                                         int c, PieceDiv groups, const int64_t* __restrict__ cluster,
                                                          T* __restrict__ out) {
-    const int groups = c / V;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * groups) return;
-    const int64_t i = e / groups;
-    const int ch = (int)(e - i * groups) * V;
+    const int64_t i = ptv3_row_of(e, groups);
+    if (i >= n) return;
+    const int ch = (int)(e - i * groups.count) * V;
     const Pack<T, V> a = *(const Pack<T, V>*)(parent + i * c + ch);
     const Pack<T, V> b = *(const Pack<T, V>*)(child + cluster[i] * c + ch);
     Pack<T, V> r;
@@ -335,10 +333,10 @@ void launch_segment_reduce(const void* src, int64_t n, int c, const int64_t* ind
                            stream, (const T*)src, c, indices, idx_ptr, op, (T*)out);
     } else if (c % V == 0) {
         hipLaunchKernelGGL((segment_reduce_kernel<T, V>), dim3((unsigned)ptv3_ceil_div(m * (c / V), 256)), dim3(256), 0,
-                           stream, (const T*)src, c, indices, idx_ptr, m, op, (T*)out);
+                           stream, (const T*)src, c, ptv3_piece_div(c / V), indices, idx_ptr, m, op, (T*)out);
     } else {
         hipLaunchKernelGGL((segment_reduce_kernel<T, 1>), dim3((unsigned)ptv3_ceil_div(m * c, 256)), dim3(256), 0,
-                           stream, (const T*)src, c, indices, idx_ptr, m, op, (T*)out);
+                           stream, (const T*)src, c, ptv3_piece_div(c), indices, idx_ptr, m, op, (T*)out);
     }
 }
 
@@ -348,10 +346,10 @@ void launch_unpool_add(const void* parent, const void* child, int64_t n, int c, 
     constexpr int V = 16 / sizeof(T);
     if (c % V == 0) {
         hipLaunchKernelGGL((unpool_add_kernel<T, V>), dim3((unsigned)ptv3_ceil_div(n * (c / V), 256)), dim3(256), 0,
-                           stream, (const T*)parent, (const T*)child, n, c, cluster, (T*)out);
+                           stream, (const T*)parent, (const T*)child, n, c, ptv3_piece_div(c / V), cluster, (T*)out);
     } else {
         hipLaunchKernelGGL((unpool_add_kernel<T, 1>), dim3((unsigned)ptv3_ceil_div(n * c, 256)), dim3(256), 0, stream,
-                           (const T*)parent, (const T*)child, n, c, cluster, (T*)out);
+                           (const T*)parent, (const T*)child, n, c, ptv3_piece_div(c), cluster, (T*)out);
     }
 }
 
