@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include "common.h"
+#include "lintile.h"
 
 namespace {
 
@@ -170,10 +171,20 @@ int block_half(Run& r, const ptv3_block_w& b, int s, const void* xs, const void*
                                        b.ln_cpe.eps, feat, normed, r.stream));
             } else {
                 TRY(linear(r, conv, b.cpe, n, attn));
-                TRY(ptv3_layer_norm(attn, x, b.ln_cpe.g, b.ln_cpe.b, b.ln1.g, b.ln1.b, nullptr, r.dt, n, c, b.ln_cpe.eps, 3, feat,
-                                    normed, r.stream));
+                if (lin_front_pays(n, c, 3 * c)) {
+                    LinArgs a = {};
+                    LinFront f = {};
+                    a.x = attn, a.w = b.qkv.w, a.bias = b.qkv.b, a.n = n, a.k = c, a.nout = 3 * c, a.out = qkv;
+                    f.mode = LinFront::NORM_SUM_NORM, f.g = b.ln_cpe.g, f.b = b.ln_cpe.b, f.res = x, f.g2 = b.ln1.g, f.b2 = b.ln1.b;
+                    f.eps = b.ln_cpe.eps, f.sum = feat;
+                    TRY(lin_front(a, f, r.dt, (hipStream_t)r.stream));
+                    normed = nullptr;
+                } else {
+                    TRY(ptv3_layer_norm(attn, x, b.ln_cpe.g, b.ln_cpe.b, b.ln1.g, b.ln1.b, nullptr, r.dt, n, c, b.ln_cpe.eps, 3,
+                                        feat, normed, r.stream));
+                }
             }
-            TRY(linear(r, normed, b.qkv, n, qkv));
+            if (normed) TRY(linear(r, normed, b.qkv, n, qkv));
         }
         TRY(attention(r, b, v, patch, qkv, r.dt, attn));
         if (few) {

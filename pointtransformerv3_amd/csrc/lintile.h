@@ -21,3 +21,15 @@ struct LinArgs {
 bool lin_tiled_pays(int64_t n, int k, int nout, int act);
 bool lin_tiled_takes(int k, int nout);
 int lin_tiled(LinArgs& a, int dtype, hipStream_t stream);
+
+// The LayerNorm in front of a layer of few rows, formed by the layer itself instead of by a launch of its own.
+struct LinFront {
+    enum { NORM = 1, NORM_SUM_NORM = 2 };
+    int mode;
+    const void *g, *b;            // NORM: LayerNorm(x) is what is multiplied. NORM_SUM_NORM: the sum res + LayerNorm(x) goes
+    const void *res, *g2, *b2;    // to `sum`, and its LayerNorm (g2, b2) is what is multiplied
+    float eps;
+    void* sum;
+};
+bool lin_front_pays(int64_t n, int k, int nout);
+int lin_front(LinArgs& a, const LinFront& f, int dtype, hipStream_t stream);

@@ -13,6 +13,7 @@
 // Measured, 1500 rows: 256 -> 1024 12.0 -> 5.2 us, 1024 -> 256 13.2 -> 6.7, 512 -> 512 12.5 -> 4.8, 2048 -> 512 22.4 -> 10.9,
 // 256 -> 1024 with the GELU's input kept 21.2 -> 6.0.
 #include "lintile.h"
+#include "rownorm.h"
 #include "rowtile.h"
 
 namespace {
@@ -51,26 +52,35 @@ unsigned tile_grid(LinArgs& a, int rows, int cols) {
 
 // What follows the sum of the products, on eight neighbouring channels c .. c + 7 of rows that `rows` walks; roundings where
 // separate layers would have stored. One copy per kind: a launch of a few microseconds pays for every instruction it fetches.
-template <typename T, int ACT, typename F>
-__device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, F&& rows) {
+// PRE: the bias and, of a layer that reads one, the second matrix's piece of the one row were asked for by the caller.
+template <typename T> struct LinPre { typename H16<T>::v8 bias, other; };
+template <typename T, int ACT, bool PRE, typename F>
+__device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, const LinPre<T>& pre, F&& rows) {
     typedef typename H16<T>::v8 v8;
     v8 bias, gamma, beta;
     float mu[8], sc[8];
-    if (a.bias) bias = *(const v8*)((const T*)a.bias + c);
+    if (PRE) bias = pre.bias;
+    else if (a.bias) bias = *(const v8*)((const T*)a.bias + c);
     if (ACT >= ACT_BN) {
         if (a.gamma) gamma = *(const v8*)((const T*)a.gamma + c);
         if (a.beta) beta = *(const v8*)((const T*)a.beta + c);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            mu[u] = a.stats_f32 ? ((const float*)a.mean)[c + u] : (float)((const T*)a.mean)[c + u];
-            const float va = a.stats_f32 ? ((const float*)a.var)[c + u] : (float)((const T*)a.var)[c + u];
-            sc[u] = rsqrtf(va + a.bn_eps) * (a.gamma ? (float)gamma[u] : 1.f);
+        // one test for all of them: behind a test each, every value was a trip to memory of its own
+        float va[8];
+        if (a.stats_f32) {
+            load8((const float*)a.mean + c, mu);
+            load8((const float*)a.var + c, va);
+        } else {
+            load8((const T*)a.mean + c, mu);
+            load8((const T*)a.var + c, va);
         }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sc[u] = rsqrtf(va[u] + a.bn_eps) * (a.gamma ? (float)gamma[u] : 1.f);
     }
     rows([&](float (&y)[8], int64_t at) {
         v8 keep, other;
-        if (ACT == ACT_GELU_GRAD) other = *(const v8*)((const T*)a.aux + at);
-        if (ACT == ACT_NONE && a.resid) other = *(const v8*)((const T*)a.resid + at);
+        if (PRE) other = pre.other;
+        else if (ACT == ACT_GELU_GRAD) other = *(const v8*)((const T*)a.aux + at);
+        else if (ACT == ACT_NONE && a.resid) other = *(const v8*)((const T*)a.resid + at);
         if (a.bias)
 #pragma unroll
             for (int u = 0; u < 8; ++u) y[u] += (float)bias[u];
@@ -91,36 +101,93 @@ __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, F&& rows) 
         if (ACT == ACT_GELU_KEEP) *(v8*)((T*)a.aux + at) = keep;
     });
 }
-template <typename T, typename F>
-__device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, F&& rows) {
+template <typename T, bool PRE, typename F>
+__device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, const LinPre<T>& pre, F&& rows) {
     switch (a.act) {
-        case ACT_NONE: return lin_epilogue<T, ACT_NONE>(a, c, rows);
-        case ACT_GELU: return lin_epilogue<T, ACT_GELU>(a, c, rows);
-        case ACT_GELU_KEEP: return lin_epilogue<T, ACT_GELU_KEEP>(a, c, rows);
-        case ACT_GELU_GRAD: return lin_epilogue<T, ACT_GELU_GRAD>(a, c, rows);
-        case ACT_BN: return lin_epilogue<T, ACT_BN>(a, c, rows);
-        default: return lin_epilogue<T, ACT_BN_GELU>(a, c, rows);
+        case ACT_NONE: return lin_epilogue<T, ACT_NONE, PRE>(a, c, pre, rows);
+        case ACT_GELU: return lin_epilogue<T, ACT_GELU, PRE>(a, c, pre, rows);
+        case ACT_GELU_KEEP: return lin_epilogue<T, ACT_GELU_KEEP, PRE>(a, c, pre, rows);
+        case ACT_GELU_GRAD: return lin_epilogue<T, ACT_GELU_GRAD, PRE>(a, c, pre, rows);
+        case ACT_BN: return lin_epilogue<T, ACT_BN, PRE>(a, c, pre, rows);
+        default: return lin_epilogue<T, ACT_BN_GELU, PRE>(a, c, pre, rows);
     }
 }
 
 constexpr int FEW_THREADS = 256, FEW_WAVES = 4;
+constexpr int64_t FEW_TILES = 208;
 
-template <typename T, int MB, int NB, int D>
-__global__ __launch_bounds__(FEW_THREADS) void few_kernel(LinArgs a) {
+// The 32 normalised rows of a work-group, rounded where a launch of its own would have stored them (the same operations as
+// layer_norm_kernel's, in the same order), into LDS rows of K + 8. Every column tile makes its rows again: a few KB out of
+// L2 against a dependent launch.
+template <typename T, int MODE, int K>
+__device__ __forceinline__ void front_rows(const LinArgs& a, const LinFront& f, int64_t r0, bool first, T* xs) {
+    constexpr int LPR = K / 8, RPP = FEW_THREADS / LPR;   // lanes per row, rows per pass
+    const int sub = threadIdx.x % LPR;
+    float g[8], b[8], g2[8], b2[8];
+    load8((const T*)f.g + sub * 8, g);
+    load8((const T*)f.b + sub * 8, b);
+    if (MODE == LinFront::NORM_SUM_NORM) {
+        load8((const T*)f.g2 + sub * 8, g2);
+        load8((const T*)f.b2 + sub * 8, b2);
+    }
+    constexpr int P = 32 / RPP;
+    u32x4 xq[P], oq[P];   // every pass's rows are on the way before the first is waited for
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int64_t r = r0 + p * RPP + threadIdx.x / LPR, at = r < a.n ? r : a.n - 1;   // rows past the end are not stored
+        xq[p] = *(const u32x4*)((const T*)a.x + at * K + sub * 8);
+        if (MODE == LinFront::NORM_SUM_NORM) oq[p] = *(const u32x4*)((const T*)f.res + at * K + sub * 8);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int r = p * RPP + threadIdx.x / LPR;
+        float v[8], mean, rstd;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = H16<T>::lo(xq[p][i]);
+            v[2 * i + 1] = H16<T>::hi(xq[p][i]);
+        }
+        row_stats<LPR>(v, f.eps, mean, rstd);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (v[i] - mean) * rstd * g[i] + b[i];
+        if (MODE == LinFront::NORM_SUM_NORM) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[2 * i] = H16<T>::round(H16<T>::round(v[2 * i]) + H16<T>::lo(oq[p][i]));
+                v[2 * i + 1] = H16<T>::round(H16<T>::round(v[2 * i + 1]) + H16<T>::hi(oq[p][i]));
+            }
+            if (first && r0 + r < a.n) store8((T*)f.sum + (r0 + r) * K + sub * 8, v);
+            row_stats<LPR>(v, f.eps, mean, rstd);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = (v[i] - mean) * rstd * g2[i] + b2[i];
+        }
+        u32x4 o4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o4[q] = H16<T>::pack2(v[2 * q], v[2 * q + 1]);
+        *(u32x4*)(xs + r * (K + 8) + sub * 8) = o4;
+    }
+}
+
+// MODE: 0, rows from memory, K of the layer in LinArgs; otherwise what LinFront says, K = KF.
+template <typename T, int MB, int NB, int D, int MODE, int KF>
+__global__ __launch_bounds__(FEW_THREADS) void few_kernel(LinArgs a, LinFront f) {
     typedef typename H16<T>::v8 v8;
     constexpr int ROWS = MB * 16, COLS = NB * 16, CS = COLS + 4;
     __shared__ float red[FEW_WAVES][ROWS * CS];
+    __shared__ __align__(16) T xs[MODE ? ROWS * (KF + 8) : 1];
     int rt, ct;
     if (!tile_of(a, rt, ct)) return;
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE, lr = lane & 15, lg = lane >> 4;
     const int64_t r0 = (int64_t)rt * ROWS;
-    const int c0 = ct * COLS, K = a.k, steps = K / 32;
+    const int c0 = ct * COLS, K = MODE ? KF : a.k, steps = K / 32;
     const T* xr[MB];
     const T* wr[NB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         const int64_t r = r0 + mb * 16 + lr;
-        xr[mb] = (const T*)a.x + (r < a.n ? r : a.n - 1) * K + lg * 8;   // rows past the end are multiplied and not stored
+        xr[mb] = MODE ? xs + (mb * 16 + lr) * (KF + 8) + lg * 8
+                      : (const T*)a.x + (r < a.n ? r : a.n - 1) * K + lg * 8;   // rows past the end are multiplied and not stored
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) wr[nb] = (const T*)a.w + (int64_t)(c0 + nb * 16 + lr) * K + lg * 8;
@@ -131,12 +198,14 @@ __global__ __launch_bounds__(FEW_THREADS) void few_kernel(LinArgs a) {
         for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     v8 xf[2][D][MB], wf[2][D][NB];   // two sets of D steps: one is multiplied, one on its way
-    auto load = [&](v8 (&xv)[D][MB], v8 (&wv)[D][NB], int base) {   // the wave's steps base, base + 4, ...; the last one again past the end
+    auto load = [&](v8 (&xv)[D][MB], v8 (&wv)[D][NB], int base, bool rows, bool weights) {   // the wave's steps base, base + 4, ...; the last one again past the end
 #pragma unroll
         for (int i = 0; i < D; ++i) {
             const int st = base + i * FEW_WAVES, at = (st < steps ? st : steps - 1) * 32;
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) xv[i][mb] = *(const v8*)(xr[mb] + at);
+            for (int mb = 0; mb < MB; ++mb)
+                if (rows) xv[i][mb] = *(const v8*)(xr[mb] + at);
+            if (!weights) continue;
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) wv[i][nb] = *(const v8*)(wr[nb] + at);
         }
@@ -156,15 +225,30 @@ __global__ __launch_bounds__(FEW_THREADS) void few_kernel(LinArgs a) {
                 for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = few_mfma<T>(wv[i][nb], xv[i][mb], acc[nb][mb]);
         }
     };
-    load(xf[0], wf[0], wave);
+    load(xf[0], wf[0], wave, MODE == 0, true);
+    // what the epilogue reads is on its way as well: behind the sums it was one more trip to memory
+    constexpr int PIECES = COLS / 8;
+    static_assert(ROWS * PIECES <= FEW_THREADS, "a thread stores one piece");
+    LinPre<T> pre = {};
+    const int er = tid / PIECES, ec = c0 + tid % PIECES * 8;
+    const bool stores = er < ROWS && r0 + er < a.n;
+    const int64_t eat = (r0 + er) * a.nout + ec;
+    if (a.bias) pre.bias = *(const v8*)((const T*)a.bias + ec);
+    const void* second = a.act == ACT_GELU_GRAD ? a.aux : a.act == ACT_NONE ? a.resid : nullptr;
+    if (second && stores) pre.other = *(const v8*)((const T*)second + eat);
+    if (MODE) {   // the weights are on their way meanwhile
+        front_rows<T, MODE ? MODE : 1, MODE ? KF : 64>(a, f, r0, ct == 0, xs);
+        __syncthreads();
+        load(xf[0], wf[0], wave, true, false);
+    }
     constexpr int ROUND = D * FEW_WAVES;
     for (int base = wave;; base += 2 * ROUND) {
         const bool more = base - wave + ROUND < steps;
-        if (more) load(xf[1], wf[1], base + ROUND);
+        if (more) load(xf[1], wf[1], base + ROUND, true, true);
         multiply(xf[0], wf[0], base);
         if (!more) break;
         const bool again = base - wave + 2 * ROUND < steps;
-        if (again) load(xf[0], wf[0], base + 2 * ROUND);
+        if (again) load(xf[0], wf[0], base + 2 * ROUND, true, true);
         multiply(xf[1], wf[1], base + ROUND);
         if (!again) break;
     }
@@ -174,23 +258,18 @@ __global__ __launch_bounds__(FEW_THREADS) void few_kernel(LinArgs a) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) *(f32x4*)&red[wave][(mb * 16 + lr) * CS + nb * 16 + 4 * lg] = acc[nb][mb];
     __syncthreads();
-    constexpr int PIECES = COLS / 8;
-    lin_epilogue<T>(a, c0 + tid % PIECES * 8, [&](auto&& store) {
+    lin_epilogue<T, true>(a, ec, pre, [&](auto&& store) {
+        if (!stores) return;
+        float y[8];
 #pragma unroll
-        for (int it = 0; it < (ROWS * PIECES + FEW_THREADS - 1) / FEW_THREADS; ++it) {
-            const int e = it * FEW_THREADS + tid, r = e / PIECES, pc = e % PIECES;
-            if (r >= ROWS || r0 + r >= a.n) break;
-            float y[8];
+        for (int h = 0; h < 2; ++h) {
+            f32x4 s = *(const f32x4*)&red[0][er * CS + (ec - c0) + h * 4];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                f32x4 s = *(const f32x4*)&red[0][r * CS + pc * 8 + h * 4];
+            for (int w = 1; w < FEW_WAVES; ++w) s += *(const f32x4*)&red[w][er * CS + (ec - c0) + h * 4];
 #pragma unroll
-                for (int w = 1; w < FEW_WAVES; ++w) s += *(const f32x4*)&red[w][r * CS + pc * 8 + h * 4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) y[h * 4 + u] = s[u];
-            }
-            store(y, (r0 + r) * a.nout + c0 + pc * 8);
+            for (int u = 0; u < 4; ++u) y[h * 4 + u] = s[u];
         }
+        store(y, eat);
     });
 }
 
@@ -284,7 +363,7 @@ __global__ __launch_bounds__(TL_THREADS, 2) void linear_tile_kernel(LinArgs a) {
     float* stage = (float*)lds + wave * (32 * OS);
     constexpr int PIECES = NT * 4, RPI = PTV3_WAVE / PIECES;   // 16-byte pieces per row, rows per pass of the wave
     const int orow = lane / PIECES, opc = lane % PIECES;
-    lin_epilogue<T>(a, n0 + wc + opc * 8, [&](auto&& store) {
+    lin_epilogue<T, false>(a, n0 + wc + opc * 8, LinPre<T>{}, [&](auto&& store) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
 #pragma unroll
@@ -326,7 +405,16 @@ int tile_launch(LinArgs& a, hipStream_t stream) {
 template <typename T, int D>
 int few_launch(LinArgs& a, hipStream_t stream) {
     const unsigned grid = tile_grid(a, 32, 32);
-    hipLaunchKernelGGL((few_kernel<T, 2, 2, D>), dim3(grid), dim3(FEW_THREADS), 0, stream, a);
+    hipLaunchKernelGGL((few_kernel<T, 2, 2, D, 0, 0>), dim3(grid), dim3(FEW_THREADS), 0, stream, a, LinFront{});
+    PTV3_RETURN_LAUNCH();
+}
+
+template <typename T, int MODE>
+int front_launch(LinArgs& a, const LinFront& f, hipStream_t stream) {
+    const unsigned grid = tile_grid(a, 32, 32);
+    if (a.k == 64) hipLaunchKernelGGL((few_kernel<T, 2, 2, 1, MODE, 64>), dim3(grid), dim3(FEW_THREADS), 0, stream, a, f);
+    else if (a.k == 256) hipLaunchKernelGGL((few_kernel<T, 2, 2, 2, MODE, 256>), dim3(grid), dim3(FEW_THREADS), 0, stream, a, f);
+    else return PTV3_ESHAPE;
     PTV3_RETURN_LAUNCH();
 }
 
@@ -337,7 +425,7 @@ int few_launch(LinArgs& a, hipStream_t stream) {
 template <typename T>
 int lin_tiled_t(LinArgs& a, hipStream_t stream) {
     const int64_t t32 = ptv3_ceil_div(a.n, 32) * (a.nout / 32), t128 = ptv3_ceil_div(a.n, 128) * (a.nout / 128);
-    if (a.k % 64 != 0 || a.nout % 64 != 0 || t32 <= 208) {
+    if (a.k % 64 != 0 || a.nout % 64 != 0 || t32 <= FEW_TILES) {
         if (a.k <= 128) return few_launch<T, 1>(a, stream);
         if (a.k <= 256) return few_launch<T, 2>(a, stream);
         return few_launch<T, 4>(a, stream);
@@ -374,6 +462,28 @@ int lin_tiled(LinArgs& a, int dtype, hipStream_t stream) {
     return PTV3_ESHAPE;
 }
 
+// Whether the norm goes into the layer behind it. The launch it replaces costs 3 us and every column tile's own norm 2: with
+// 256 inputs while a CU has one tile (block tail of 250 rows 17.0 -> 15.7 us, of 350 no change; then the layer alone takes
+// few_kernel as well, and the sums are the same bits), with 64 up to a thousand tiles (1500 rows 13.8 -> 12.1, 4000 14.2 ->
+// 14.0). With 512 the norm of 32 rows takes as long as the launch (300 rows 23.2 -> 26.1).
+bool lin_front_pays(int64_t n, int k, int nout) {
+    const int64_t tiles = ptv3_ceil_div(n, 32) * (nout / 32);
+    return k == 64 ? tiles <= 1024 : k == 256 && tiles <= FEW_TILES;
+}
+
+int lin_front(LinArgs& a, const LinFront& f, int dtype, hipStream_t stream) {
+    if (dtype != PTV3_F16 && dtype != PTV3_BF16) return PTV3_ESHAPE;
+    if (a.nout % 32 != 0 || a.n >= (1ll << 31)) return PTV3_ESHAPE;
+#define PTV3_FRONT(T)                                                               \
+    do {                                                                            \
+        if (f.mode == LinFront::NORM) return front_launch<T, LinFront::NORM>(a, f, stream); \
+        return front_launch<T, LinFront::NORM_SUM_NORM>(a, f, stream);              \
+    } while (0)
+    if (dtype == PTV3_F16) PTV3_FRONT(_Float16);
+    PTV3_FRONT(__bf16);
+#undef PTV3_FRONT
+}
+
 // The second half of a block layer by layer: sum = shortcut + attn Wproj^T + b, then sum + fc2(GELU(fc1(LN(sum)))).
 // Against the fused kernels, which give a work-group whole rows: at 512 channels one streams 4 MB of weights through a CU
 // (53 us whatever the rows, against 21 - 49 us here up to 3000; 62 against 71 at 6000), at 256 (18 us against 15 - 18 up to
@@ -402,6 +512,15 @@ extern "C" int ptv3_block_tail_few(const void* attn, const void* shortcut, const
         return lin_tiled(a, dtype, s);
     };
     int rc = layer(attn, w_proj, b_proj, channels, channels, ACT_NONE, shortcut, sum);
+    if (rc == PTV3_OK && ln2_gamma && ln2_beta && lin_front_pays(n, channels, 4 * channels)) {
+        LinArgs a = {};
+        LinFront f = {};
+        a.x = sum, a.w = w1, a.bias = b1, a.n = n, a.k = channels, a.nout = 4 * channels, a.act = ACT_GELU, a.out = hidden;
+        f.mode = LinFront::NORM, f.g = ln2_gamma, f.b = ln2_beta, f.eps = ln2_eps;
+        rc = lin_front(a, f, dtype, s);
+        if (rc == PTV3_OK) rc = layer(hidden, w2, b2, 4 * channels, channels, ACT_NONE, sum, out);
+        return rc;
+    }
     if (rc == PTV3_OK)
         rc = ptv3_layer_norm(sum, nullptr, ln2_gamma, ln2_beta, nullptr, nullptr, nullptr, dtype, n, channels, ln2_eps, 0, normed,
                              nullptr, stream);

@@ -75,3 +75,10 @@ def test_block_tail_few(c, n, dtype):
         m.to(DEV)
     got = o.block_tail_few(attn.to(DEV), short.to(DEV), proj, ln, fc1, fc2)
     assert rel_err(got, want) < 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("c,n", [(64, 33), (64, 2000), (256, 1), (256, 31), (256, 200), (256, 208)])
+def test_block_tail_few_with_its_norm_in_front(c, n):
+    """Sizes whose LayerNorm is formed by the layer behind it: one row, a last tile of one row, as many tiles as CUs."""
+    test_block_tail_few(c, n, torch.float16)
+    test_block_tail_few(c, n, torch.bfloat16)
