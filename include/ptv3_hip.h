@@ -325,8 +325,9 @@ int ptv3_subm_conv_tiles_fwd(const void *feat, int dtype, int64_t n, int channel
                              const void *packed_weight, const void *bias, const int32_t *tile_tap,
                              const int32_t *tile_pair, const int32_t *vox_taps, void *out, void *stream);
 /* The same with tiles of tile_voxels outputs: 128 (what the three functions above use), or 96 at 128 channels
- * (same call site, model.py:546-552). The lists must have been made with the same tile_voxels. A launch runs in
- * rounds of the work-groups the part holds at a time; the caller picks the size whose last round is fuller. */
+ * (same call site, model.py:546-552). The lists must have been made with the same tile_voxels, ptv3_conv_tile_voxels
+ * names the size that pays: a launch takes what its fullest CU takes. */
+int ptv3_conv_tile_voxels(int64_t n, int channels);
 int64_t ptv3_conv_plan_tile_count_sized(int64_t n, int tile_voxels);
 int ptv3_conv_plan_tiles_sized(const int32_t *row_ptr, const int32_t *slot_pair, int64_t n, int taps, int tile_voxels,
                                int32_t *tile_tap, int32_t *tile_pair, int32_t *vox_taps, void *stream);

@@ -2,23 +2,28 @@
 //
 // Replaces spconv.SubMConv3d.forward at the xCPE call sites of the reference (model.py:546-552:
 // in_channels == out_channels, 3x3x3, bias) where the pair form's round trip of one product row
-// per (input, output) pair through HBM is what bounds it (up to 256 channels).
+// per (input, output) pair through HBM is what bounds it.
 //
-// A work-group owns TV consecutive output voxels and keeps their sums as fp32 in LDS. It reads
-// the voxels' pairs from the output-major list (slot_pair: tap << 24 | input row, voxel i's pairs
-// at [row_ptr[i], row_ptr[i+1])), sorts them by tap in LDS (counting sort), and walks the taps in
-// order: the input rows of up to 64 pairs of one tap are gathered into LDS in whole row segments,
-// every wave multiplies them with its own 32 output channels of that tap's weights
-// (v_mfma_f32_32x32x16, product transposed: a column is a pair), and adds its 32x32 block into the
-// LDS sums of the pairs' output voxels. MFMA columns are real pairs whatever the sparsity, an
-// output is written once, nothing is atomic, and the order of the additions (tap order, fp32) is
-// fixed. Waves own disjoint channel slices, or disjoint pairs of the same tap, and a barrier per
-// chunk orders the taps, so the read-modify-write of the sums needs no atomics.
+// A work-group owns 32 to 128 consecutive output voxels and keeps their sums as fp32 in MFMA accumulators: a wave holds 32
+// output channels of all of them (64 channels: of half of them). From the tile's pair list (plan_tiles_kernel) it makes a
+// table of the row that every output reads at every tap, and walks the taps that occur in the tile: the rows of a tap go
+// from memory to LDS without passing through registers (buffer_load ... lds, 16 bytes a lane, 16-byte pieces swizzled by
+// the row), a row per output, while the tap before is multiplied. An output without the tap has an offset past the
+// end of the buffer, for which the load's own range check writes zeros: nothing is read for it, nothing is branched on.
+// Groups of 32 outputs without the tap are not multiplied. Sums are fp32 in tap order whatever the tile: the same bits on
+// every run and for every tile size, closer to the exact sums than the pair form (which rounds every product row).
 //
 // The weights come in fragment order (ptv3_subm_conv_pack_weight): the 16 bytes lane l needs for
 // (tap, 32-channel slice, 16-channel step) are stored at consecutive addresses over the lanes, so a
-// wave fetches a fragment as one contiguous KB straight into registers, one tap ahead; the input
-// rows of the next chunk are in flight while this one is multiplied.
+// wave fetches a fragment as one contiguous KB straight into registers, one tap ahead.
+//
+// What bounds it: large levels the matrix cores - 70 % of the (tap, 32 outputs) of a level occur where 36 % of the pairs
+// do, and what is multiplied runs at 750 TFLOP/s of the 1090 a large product reaches; small ones a tile's chain of taps,
+// 20 us for 32 outputs to 38 for 128. Measured (fp16, MI355X), against gathering through registers into the row of the output
+// with two chunks in flight: 128 channels, 149k voxels of 9.8 pairs 167 -> 117 us, 371k 339 -> 257, 36k 54 -> 39; 64 channels,
+// 20k voxels of 5.3 pairs 18.9 (sparse tiles) -> 14.6. Tried: 64-channel slices with three in flight (125 us at 149k), waves of
+// 64 x 64 (137), 256 channels (93k voxels 274 - 300 us against 344 in pair form, 37k 131 - 153 against 122: half of the products
+// are of absent neighbours, and those of the pair form are not).
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -35,9 +40,16 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));   // a caller's vector may start at any of its elements
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+
 template <typename T> struct TileOps;
 template <> struct TileOps<_Float16> {
     typedef f16x8 v8;
+    typedef f16x4 v4;
     static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
@@ -48,6 +60,7 @@ template <> struct TileOps<_Float16> {
 };
 template <> struct TileOps<__bf16> {
     typedef bf16x8 v8;
+    typedef bf16x4 v4;
     static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
@@ -121,7 +134,7 @@ __global__ __launch_bounds__(CT_THREADS) void plan_slots_kernel(const int32_t* _
     slot_pair[pair_slot[q]] = (int32_t)((uint32_t)lo << 24 | (uint32_t)pair_in[q]);
 }
 
-constexpr int CT_TV = 128;          // output voxels per tile (the 128-channel tile form also takes tiles of 96)
+constexpr int CT_TV = 128;          // output voxels per tile of the lists (at 128 channels tiles of 96 as well)
 constexpr int CT_TILE_WORDS = 32;   // int32 per tile in tile_tap: 28 tap starts (relative), the tile's first pair
 
 // Per tile of blockDim.x (96 or 128) consecutive voxels: its pairs sorted by tap, inside a tap by output voxel.
@@ -179,222 +192,204 @@ __global__ __launch_bounds__(CT_TV) void plan_tiles_kernel(const int32_t* __rest
     }
 }
 
-// TV_ output voxels per tile: 128, or 96 where the four waves split the output channels (128 channels): a launch
-// whose 128-voxel tiles fill 2.2 rounds of the resident work-groups costs three, with 96-voxel tiles 2.97 rounds of
-// tiles that are a quarter cheaper
-template <int C, int TV_ = CT_TV>
-struct TileShape {
-    static constexpr int TV = TV_;
-    static constexpr int THREADS = 256;
-    static constexpr int COUT_WG = C > 128 ? 128 : C;     // output channels of a work-group
-    static constexpr int CW = COUT_WG / 32;               // waves across channels
-    static constexpr int PW = 4 / CW;                     // waves across the 32-voxel groups of the tile
-    static constexpr int GPW = TV / 32 / PW;              // groups per wave
-    static constexpr int CH = C >= 128 ? TV : 64;         // pairs per chunk (128 channels: a tap of a tile is one chunk)
-    static constexpr int KS = C / 16;                     // MFMA steps along the input channels
-    static constexpr int LPR = C / 8;                     // lanes (16 B each) per input row
-    static constexpr int RPP = THREADS / LPR;             // rows per gather instruction of the work-group
-    static constexpr int NL = CH / RPP;                   // gather instructions per chunk
-    static constexpr int CAP = TV * CT_TAPS;              // pairs of a tile at most
-    static constexpr int MAX_CHUNKS = CT_TAPS + CAP / CH;
-    static constexpr int OCC = 2;                         // work-groups per CU the registers allow
-    static constexpr int DEPTH = 2;                       // chunks in flight
-    static constexpr size_t XBUF = (size_t)TV * C * 2;    // bytes of one buffer of input rows (swizzled, no padding)
-    static constexpr size_t LDS = 2 * XBUF + (size_t)CAP * 4 + (size_t)C * 2;   // + one row of zeros
-    static_assert(CH % RPP == 0 && NL >= 1 && MAX_CHUNKS <= 128 && LPR >= 8 && GPW * PW * 32 == TV, "tile shape");
-};
+constexpr int CG_THREADS = 256;
+constexpr uint32_t CG_ABSENT = 0xFFFFFF00u;   // offset of a row that is not there: past fewer than 2^24 rows of 256 bytes
 
-// Input rows sit in LDS at the row of their OUTPUT voxel, 16-byte pieces swizzled by the row so that the
-// 32 rows a fragment read touches spread over the banks without padding.
-template <int C>
-__device__ __forceinline__ int swz(int row, int piece) {
-    return row * C + ((piece ^ (row & 7)) * 8);   // in halfs
-}
-
-template <typename T, int C, int TV_>
-__global__ __launch_bounds__((TileShape<C, TV_>::THREADS), (TileShape<C, TV_>::OCC)) void conv_tile_kernel(
+// G groups of 32 outputs; `sub` work-groups share a tile of the lists; DMA = 0: feat does not start at a multiple of 16 bytes
+template <typename T, int C, int G, int DMA>
+__global__ __launch_bounds__(CG_THREADS, 2) void conv_gather_kernel(
     const T* __restrict__ feat, int64_t n, const T* __restrict__ packed_w, const T* __restrict__ bias,
-    const int32_t* __restrict__ tile_tap, const uint32_t* __restrict__ tile_pair, const uint32_t* __restrict__ vox_taps,
-    T* __restrict__ out) {
-    typedef TileShape<C, TV_> S;
+    const int32_t* __restrict__ tile_tap, const uint32_t* __restrict__ tile_pair, int sub, T* __restrict__ out) {
     typedef typename TileOps<T>::v8 v8;
-    constexpr int TV = S::TV, CW = S::CW, GPW = S::GPW, CH = S::CH, KS = S::KS;
-    constexpr int LPR = S::LPR, RPP = S::RPP, NL = S::NL, COUT_WG = S::COUT_WG, DEPTH = S::DEPTH;
-    constexpr int THREADS = S::THREADS;
-    extern __shared__ __align__(16) char smem[];
-    T* xs = (T*)smem;                                        // [2][TV][C] input rows by output voxel
-    uint32_t* plist = (uint32_t*)(smem + 2 * S::XBUF);       // [CAP] the tile's pairs by tap
-    T* zero_row = (T*)(plist + S::CAP);                      // [C] what an output without the tap multiplies
-    __shared__ int32_t ch_tap[128], ch_base[128], ch_cnt[128];
-    __shared__ int32_t n_chunks;
+    typedef typename TileOps<T>::v4 v4;
+    constexpr int WC = C / 32, WR = 4 / WC, NG = G / WR, KS = C / 16;   // waves across channels and outputs, groups of a wave
+    constexpr int R = 32 * G, LPR = C / 8, ROWS = PTV3_WAVE / LPR;      // lanes of a row, rows of a load
+    constexpr int PER = R / ROWS / 4;                                   // loads of a wave per tap
+    static_assert(WC * WR == 4 && NG * WR == G && PER * ROWS * 4 == R, "four waves share channels, outputs and loads");
+    // apart, so that the compiler sees that reading one does not wait for the loads into the other
+    __shared__ __align__(16) T rows_a[R * C];
+    __shared__ __align__(16) T rows_b[R * C];
+    __shared__ uint32_t src[CT_TAPS * R];         // byte offset of the row an output reads at a tap
+    __shared__ int32_t starts[CT_TAPS + 1];
+    __shared__ uint32_t groups[CT_TAPS];          // groups in which a tap occurs
+    __shared__ int32_t taps[CT_TAPS + 3];         // tap | groups << 8 of the taps that occur, then tap 0 with no group
+    __shared__ int32_t n_taps;
 
-    const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / PTV3_WAVE), lane = tid % PTV3_WAVE;
     const int col = lane & 31, hf = lane >> 5;
-    const int cw = wave % CW, pw = wave / CW;
-    const int cout0 = blockIdx.y * COUT_WG;             // first output channel of the work-group
+    const int wc = wave % WC, wr = wave / WC;
     // work-group ids go round the XCDs: every XCD works through one contiguous eighth of the tiles, so that tiles
-    // which gather the same neighbour rows meet in one L2 (no faster, but half the HBM reads)
-    const int tile = xcd_chunked_id(blockIdx.x, gridDim.x);
-    const int64_t v0 = (int64_t)tile * TV;
-    const int nv = (int)min((int64_t)TV, n - v0);
+    // which gather the same neighbour rows meet in one L2
+    const int id = xcd_chunked_id(blockIdx.x, gridDim.x);
+    const int tile = id / sub, first = id % sub * R;   // this work-group's outputs inside the tile of the lists
+    const int64_t v0 = (int64_t)tile * (sub * R) + first;
+    const int nv = (int)min((int64_t)R, n - v0);
+    if (nv <= 0) return;
 
-    // ---- the tile's pair list and chunk table
     const int32_t* tt = tile_tap + (int64_t)tile * CT_TILE_WORDS;
     const int total = tt[CT_TAPS];
     const uint32_t* tp = tile_pair + tt[28];
-    for (int e = tid; e < total; e += THREADS) plist[e] = tp[e];
-    if (tid < C / 2) ((uint32_t*)zero_row)[tid] = 0u;
-    if (wave == 0) {
-        const int first = lane < 32 ? tt[lane] : 0;
-        const int c = lane < CT_TAPS ? tt[lane + 1] - first : 0;
-        const int nc = (c + CH - 1) / CH;
-        int x = nc;
+    if (tid <= CT_TAPS) starts[tid] = tt[tid];
+    if (tid < CT_TAPS) groups[tid] = 0u;
+    for (int e = tid; e < CT_TAPS * R; e += CG_THREADS) src[e] = CG_ABSENT;
+    u32x2 b4[4] = {};
+    if (bias)
 #pragma unroll
-        for (int off = 1; off < 32; off <<= 1) {
-            const int y = __shfl_up(x, off, PTV3_WAVE);
-            if (lane >= off) x += y;
+        for (int q = 0; q < 4; ++q) b4[q] = *(const u32x2_a2*)(bias + wc * 32 + 8 * q + 4 * hf);
+    __syncthreads();
+    for (int e = tid; e < total; e += CG_THREADS) {
+        const uint32_t word = tp[e];
+        const int o = (int)(word >> 24) - first;
+        if (o < 0 || o >= R) continue;
+        int t = 0, hi = CT_TAPS;   // the tap of pair e: the largest t with starts[t] <= e
+        while (hi - t > 1) {
+            const int mid = (t + hi) >> 1;
+            if (starts[mid] <= e) t = mid; else hi = mid;
         }
-        for (int j = 0; j < nc; ++j) {
-            ch_tap[x - nc + j] = lane;
-            ch_base[x - nc + j] = first + j * CH;
-            ch_cnt[x - nc + j] = min(CH, c - j * CH);
-        }
-        if (lane == 31) n_chunks = x;
-    }
-    // the taps of the output voxels this lane holds as MFMA columns, and their sums (start: the bias)
-    uint32_t taps_of[GPW];
-    f32x16 acc[GPW];
-#pragma unroll
-    for (int gi = 0; gi < GPW; ++gi) {
-        const int o = (pw * GPW + gi) * 32 + col;
-        taps_of[gi] = o < nv ? vox_taps[v0 + o] : 0u;
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-            acc[gi][v] = bias ? (float)bias[cout0 + 32 * cw + 8 * (v / 4) + 4 * hf + v % 4] : 0.f;
+        src[t * R + o] = (word & CT_IN_MASK) * (uint32_t)(C * sizeof(T));
+        atomicOr(&groups[t], 1u << (o >> 5));
     }
     __syncthreads();
-    const int nch = n_chunks;   // >= 1: every voxel pairs with itself
+    if (wave == 0) {
+        const uint32_t here = lane < CT_TAPS ? groups[lane] : 0u;
+        const uint64_t any = __ballot(here != 0u);
+        const int count = __popcll(any);
+        if (here) taps[__popcll(any & ((1ull << lane) - 1ull))] = lane | (int)(here << 8);
+        if (lane >= count && lane < CT_TAPS + 3) taps[lane] = 0;
+        if (lane == 0) n_taps = count;
+    }
+    __syncthreads();
+    const int count = __builtin_amdgcn_readfirstlane(n_taps);
 
-    // ---- a ring of DEPTH chunks in flight: the weights of the chunk's tap (this wave's 32 output
-    // channels) and the chunk's input rows, both as registers. Every load is unconditional (chunks
-    // past the end repeat the last one, rows past a chunk's count repeat its first row), so the
-    // number of loads in flight is fixed and a wait for one chunk leaves the younger ones in flight.
-    struct Slot {
-        u32x4 w[KS];
-        u32x4 g[NL];
-        uint32_t word[NL];
-    };
-    Slot ring[DEPTH];
-    const T* wbase = packed_w + ((int64_t)(cout0 / 32 + cw) * KS * 64 + lane) * 8;
-    constexpr int64_t W_TAP = (int64_t)(C / 32) * KS * 64 * 8;   // halfs per tap
-    auto issue = [&](int k, Slot& s) {
-        k = min(k, nch - 1);
-        const int t = ch_tap[k], base = ch_base[k], count = ch_cnt[k];
+    f32x16 acc[NG];
 #pragma unroll
-        for (int i = 0; i < KS; ++i) s.w[i] = *(const u32x4*)(wbase + t * W_TAP + (int64_t)i * 64 * 8);
+    for (int g = 0; g < NG; ++g)
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int row = i * RPP + tid / LPR;
-            s.word[i] = plist[base + (row < count ? row : 0)];
-            s.g[i] = *(const u32x4*)(feat + (int64_t)(s.word[i] & CT_IN_MASK) * C + (tid % LPR) * 8);
+        for (int q = 0; q < 4; ++q) {
+            const v4 b = __builtin_bit_cast(v4, b4[q]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[g][4 * q + k] = (float)b[k];
         }
+
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)feat, 0, (int)(uint32_t)(n * (int64_t)(C * sizeof(T))), 0x00020000);
+    u32x4 w_a[KS], w_b[KS];
+    const T* wbase = packed_w + ((int64_t)wc * KS * PTV3_WAVE + lane) * 8;
+    auto weights = [&](int t, u32x4 (&w)[KS]) {
+        const T* p = wbase + (int64_t)t * (WC * KS * PTV3_WAVE * 8);
+#pragma unroll
+        for (int i = 0; i < KS; ++i) w[i] = *(const u32x4*)(p + i * PTV3_WAVE * 8);
     };
-    auto stage = [&](int k, const Slot& s) {
-        const int count = ch_cnt[min(k, nch - 1)];
-        T* xb = xs + (size_t)(k & 1) * TV * C;
+    const uint32_t* my_src = src + wave * (PER * ROWS) + lane / LPR;
+    auto gather = [&](int t, T* buf) {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int row = i * RPP + tid / LPR;
-            if (row < count) *(u32x4*)(xb + swz<C>((int)(s.word[i] >> 24), tid % LPR)) = s.g[i];
-        }
-    };
-    auto multiply = [&](int k, const Slot& s) {
-        if (k >= nch) return;
-        const int t = ch_tap[k], base = ch_base[k], count = ch_cnt[k];
-        const int lo = (int)(plist[base] >> 24), hi = (int)(plist[base + count - 1] >> 24);   // outputs ascend inside a tap
-        const T* xb = xs + (size_t)(k & 1) * TV * C;
-#pragma unroll
-        for (int gi = 0; gi < GPW; ++gi) {
-            const int g = pw * GPW + gi;
-            if (g * 32 + 31 >= lo && g * 32 <= hi) {   // uniform: the chunk has outputs in this group
-                const int o = g * 32 + col;
-                const bool present = ((taps_of[gi] >> t) & 1u) && o >= lo && o <= hi;
-                if (__ballot(present) == 0) continue;   // none of the group's outputs has this tap
-                // an absent neighbour reads the row of zeros: no branch, no registers to clear
-                const T* row = present ? xb + o * C : zero_row;
-                const int sw = present ? (o & 7) : 0;
-#pragma unroll
-                for (int i = 0; i < KS; ++i) {
-                    const u32x4 x = *(const u32x4*)(row + (((2 * i + hf) ^ sw) * 8));
-                    acc[gi] = TileOps<T>::mfma(__builtin_bit_cast(v8, s.w[i]), __builtin_bit_cast(v8, x), acc[gi]);
-                }
+        for (int j = 0; j < PER; ++j) {
+            const int at = (wave * PER + j) * ROWS;   // 1 KB of LDS, lane after lane: the swizzle is in what a lane reads
+            const uint32_t row = my_src[t * R + j * ROWS], off = row + (uint32_t)(((lane % LPR) ^ ((at + lane / LPR) & 7)) * 16);
+            if constexpr (DMA) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(buf + at * C), 16, (int)off,
+                                                         0, 0, 0);
+            } else {
+                u32x4 piece = {};
+                if (row != CG_ABSENT) piece = *(const u32x4_a2*)((const char*)feat + off);
+                *(u32x4*)(buf + at * C + lane * 8) = piece;
             }
         }
     };
-
+    auto multiply = [&](int here, const T* buf, const u32x4 (&w)[KS]) {
 #pragma unroll
-    for (int j = 0; j < DEPTH; ++j) issue(j, ring[j]);
-    stage(0, ring[0]);
-    __syncthreads();
-    for (int k0 = 0; k0 < nch; k0 += DEPTH) {
+        for (int g = 0; g < NG; ++g) {
+            if (!(here >> (wr * NG + g) & 1)) continue;
+            const T* row = buf + ((wr * NG + g) * 32 + col) * C;
+            u32x4 x[KS];
 #pragma unroll
-        for (int j = 0; j < DEPTH; ++j) {
-            // no branch around the loads: past the end nothing is multiplied and the last chunk is staged again
-            const int k = k0 + j;
-            multiply(k, ring[j]);
-            stage(k + 1, ring[(j + 1) % DEPTH]);
-            __syncthreads();
-            issue(k + DEPTH, ring[j]);
+            for (int i = 0; i < KS; ++i) x[i] = *(const u32x4*)(row + ((2 * i + hf) ^ (col & 7)) * 8);
+#pragma unroll
+            for (int i = 0; i < KS; ++i)
+                acc[g] = TileOps<T>::mfma(__builtin_bit_cast(v8, w[i]), __builtin_bit_cast(v8, x[i]), acc[g]);
         }
+    };
+    int now = __builtin_amdgcn_readfirstlane(taps[0]), next = __builtin_amdgcn_readfirstlane(taps[1]);
+    gather(now & 31, rows_a);
+    weights(now & 31, w_a);
+    // The barrier: everyone's rows of this tap are in LDS, and everyone is through with the buffer of the tap before, which
+    // takes the next one's. Past the last tap, tap 0 is gathered and not multiplied.
+    auto step = [&](int i, T* mine, T* ahead, const u32x4 (&w)[KS], u32x4 (&w_ahead)[KS]) {
+        const int after = taps[i + 2];
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        gather(next & 31, ahead);
+        weights(next & 31, w_ahead);
+        multiply(now >> 8, mine, w);
+        now = next;
+        next = __builtin_amdgcn_readfirstlane(after);
+    };
+    for (int i = 0; i < count; i += 2) {
+        step(i, rows_a, rows_b, w_a, w_b);
+        if (i + 1 < count) step(i + 1, rows_b, rows_a, w_b, w_a);
     }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     // ---- sums -> halfs in LDS by output row -> out, 16 bytes per lane
-    // acc[gi][v]: output channel 32 cw + 8 (v / 4) + 4 hf + v % 4 of output voxel (pw GPW + gi) 32 + col
-    T* ob = xs;   // [TV][COUT_WG + 8]
-    constexpr int OS = COUT_WG + 8;
-    static_assert((size_t)TV * OS * 2 <= 2 * S::XBUF, "output staging fits in the input buffers");
+    // acc[g][v]: output channel 32 wc + 8 (v / 4) + 4 hf + v % 4 of output (wr NG + g) 32 + col
 #pragma unroll
-    for (int gi = 0; gi < GPW; ++gi) {
-        const int o = (pw * GPW + gi) * 32 + col;
+    for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const uint32_t p0 = TileOps<T>::pack2(acc[gi][4 * q], acc[gi][4 * q + 1]);
-            const uint32_t p1 = TileOps<T>::pack2(acc[gi][4 * q + 2], acc[gi][4 * q + 3]);
-            uint32_t* dst = (uint32_t*)(ob + o * OS + 32 * cw + 8 * q + 4 * hf);
-            dst[0] = p0;
-            dst[1] = p1;
+            const int r = (wr * NG + g) * 32 + col;
+            *(u32x2*)(rows_a + r * C + ((wc * 4 + q) ^ (r & 7)) * 8 + 4 * hf) =
+                (u32x2){TileOps<T>::pack2(acc[g][4 * q], acc[g][4 * q + 1]), TileOps<T>::pack2(acc[g][4 * q + 2], acc[g][4 * q + 3])};
         }
-    }
     __syncthreads();
-    for (int e = tid; e < nv * (COUT_WG / 8); e += THREADS) {
-        const int r = e / (COUT_WG / 8), c8 = e % (COUT_WG / 8);
-        *(u32x4*)(out + (v0 + r) * C + cout0 + c8 * 8) = *(const u32x4*)(ob + r * OS + c8 * 8);
+    for (int e = tid; e < nv * LPR; e += CG_THREADS) {
+        const int r = e / LPR, pc = e % LPR;
+        *(u32x4*)(out + (v0 + r) * C + pc * 8) = *(const u32x4*)(rows_a + r * C + (pc ^ (r & 7)) * 8);
     }
 }
 
-template <typename T, int C, int TV_ = CT_TV>
-int launch_tiles(const void* feat, int64_t n, const void* packed_w, const void* bias, const int32_t* tile_tap,
-                 const uint32_t* tile_pair, const uint32_t* vox_taps, void* out, hipStream_t stream) {
-    typedef TileShape<C, TV_> S;
-    auto kern = conv_tile_kernel<T, C, TV_>;
-    static LdsGrant grant_attr_set;   // per instantiation and device
-    if (const int rc_ = ptv3_allow_lds((const void*)kern, S::LDS, grant_attr_set)) return rc_;
-    const dim3 grid((unsigned)ptv3_ceil_div(n, S::TV), (unsigned)(C / S::COUT_WG));
-    hipLaunchKernelGGL(kern, grid, dim3(S::THREADS), S::LDS, stream, (const T*)feat, n, (const T*)packed_w,
-                       (const T*)bias, tile_tap, tile_pair, vox_taps, (T*)out);
+// The time of a launch at 128 channels whose fullest CU gets k work-groups of `groups` x 32 outputs and holds `at_once` of them,
+// in tenths of a us: once + each k + round ceil(k / at_once). Fitted to 2.5k - 220k voxels of 8 - 10 pairs: 38 us for one
+// work-group of 128 outputs a CU, 51 for two, 77 for three (measured 38, 53, 77); 32 outputs 20 us, 64 26, 96 31.
+struct GatherCost { int groups, once, each, round, at_once; };
+constexpr GatherCost GATHER_COST[4] = {{1, 100, 80, 0, 1}, {2, -10, 70, 200, 3}, {3, 20, 90, 195, 2}, {4, 126, 129, 130, 2}};
+int64_t gather_cost(int64_t n, const GatherCost& c) {
+    const int64_t k = ptv3_ceil_div(ptv3_ceil_div(n, 32 * c.groups), 256);
+    return c.once + c.each * k + c.round * ptv3_ceil_div(k, (int64_t)c.at_once);
+}
+
+// groups per work-group on lists of tile_voxels outputs: the cheapest that divides the tile; 64 channels: two up to two work-groups
+// a CU (30k voxels: 15.7 us against 17.5 with four), four on larger levels (40k: 19.9 against 22.5, 150k: 47 against 53)
+int gather_groups(int64_t n, int c, int tile_voxels) {
+    if (c == 64) return n <= 2 * 256 * 64 ? 2 : 4;
+    const GatherCost* best = nullptr;
+    for (const GatherCost& g : GATHER_COST)
+        if (tile_voxels % (32 * g.groups) == 0 && (!best || gather_cost(n, g) < gather_cost(n, *best))) best = &g;
+    return best->groups;
+}
+
+template <typename T, int C, int G>
+int launch_gather(const void* feat, int64_t n, int tile_voxels, const void* packed_w, const void* bias, const int32_t* tile_tap,
+                  const uint32_t* tile_pair, void* out, hipStream_t stream) {
+    const int sub = tile_voxels / (32 * G);
+    const bool dma = (uintptr_t)feat % 16 == 0;
+    hipLaunchKernelGGL((dma ? conv_gather_kernel<T, C, G, 1> : conv_gather_kernel<T, C, G, 0>),
+                       dim3((unsigned)(ptv3_ceil_div(n, tile_voxels) * sub)), dim3(CG_THREADS), 0, stream, (const T*)feat, n,
+                       (const T*)packed_w, (const T*)bias, tile_tap, tile_pair, sub, (T*)out);
     PTV3_RETURN_LAUNCH();
 }
 
 template <typename T>
 int dispatch_tiles(const void* feat, int64_t n, int c, int tile_voxels, const void* packed_w, const void* bias,
-                   const int32_t* tile_tap, const uint32_t* tile_pair, const uint32_t* vox_taps, void* out,
-                   hipStream_t stream) {
-    if (c == 64 && tile_voxels == 128)
-        return launch_tiles<T, 64>(feat, n, packed_w, bias, tile_tap, tile_pair, vox_taps, out, stream);
-    if (c == 128 && tile_voxels == 128)
-        return launch_tiles<T, 128>(feat, n, packed_w, bias, tile_tap, tile_pair, vox_taps, out, stream);
-    if (c == 128 && tile_voxels == 96)
-        return launch_tiles<T, 128, 96>(feat, n, packed_w, bias, tile_tap, tile_pair, vox_taps, out, stream);
+                   const int32_t* tile_tap, const uint32_t* tile_pair, void* out, hipStream_t stream) {
+    const int g = gather_groups(n, c, tile_voxels);
+#define PTV3_GATHER(C, G) \
+    if (c == C && g == G) return launch_gather<T, C, G>(feat, n, tile_voxels, packed_w, bias, tile_tap, tile_pair, out, stream)
+    PTV3_GATHER(64, 2);
+    PTV3_GATHER(64, 4);
+    PTV3_GATHER(128, 1);
+    PTV3_GATHER(128, 2);
+    PTV3_GATHER(128, 3);
+    PTV3_GATHER(128, 4);
+#undef PTV3_GATHER
     return PTV3_ESHAPE;
 }
 
@@ -408,6 +403,16 @@ extern "C" int ptv3_conv_plan_slots(const int32_t* tap_ptr, int taps, const int3
     hipLaunchKernelGGL(plan_slots_kernel, dim3((unsigned)ptv3_ceil_div(n_pairs, CT_THREADS)), dim3(CT_THREADS), 0,
                        (hipStream_t)stream_, tap_ptr, taps, pair_in, pair_slot, n_pairs, slot_pair);
     PTV3_RETURN_LAUNCH();
+}
+
+// 128, or at 128 channels 96 where three groups of 32 a work-group are the cheapest: 146k voxels are six work-groups of 96 on the
+// fullest CU (114 us), nine of 64 (119) or five of 128 (118); 60k are two of 128 (53), four of 64 (67) or three of 96 (72)
+extern "C" int ptv3_conv_tile_voxels(int64_t n, int channels) {
+    if (channels != 128) return 128;
+    const int64_t three = gather_cost(n, GATHER_COST[2]);
+    for (const GatherCost& g : GATHER_COST)
+        if (g.groups != 3 && gather_cost(n, g) <= three) return 128;
+    return 96;
 }
 
 extern "C" int64_t ptv3_conv_plan_tile_count(int64_t n) { return n < 0 ? 0 : ptv3_ceil_div(n, CT_TV); }
@@ -479,8 +484,8 @@ extern "C" int ptv3_subm_conv_tiles_fwd_sized(const void* feat, int dtype, int64
     if (n == 0) return PTV3_OK;
     if (!feat || !packed_weight || !tile_tap || !tile_pair || !vox_taps || !out) return PTV3_EINVAL;
     hipStream_t stream = (hipStream_t)stream_;
-    const uint32_t *tp = (const uint32_t*)tile_pair, *vt = (const uint32_t*)vox_taps;
+    const uint32_t* tp = (const uint32_t*)tile_pair;
     if (dtype == PTV3_F16)
-        return dispatch_tiles<_Float16>(feat, n, channels, tile_voxels, packed_weight, bias, tile_tap, tp, vt, out, stream);
-    return dispatch_tiles<__bf16>(feat, n, channels, tile_voxels, packed_weight, bias, tile_tap, tp, vt, out, stream);
+        return dispatch_tiles<_Float16>(feat, n, channels, tile_voxels, packed_weight, bias, tile_tap, tp, out, stream);
+    return dispatch_tiles<__bf16>(feat, n, channels, tile_voxels, packed_weight, bias, tile_tap, tp, out, stream);
 }

@@ -390,13 +390,15 @@ extern "C" int ptv3_conv_few_pairs(int64_t n_pairs, int channels) {
 // The form the 3x3x3 convolution of a half-precision level takes: 0 pair lists, 1 sparse tiles, 2 tiles. Above the few pairs
 // of ptv3_conv_few_pairs the rule is on pairs per voxel: 32 and 64 channels take the sparse tile form up to 14 (work in
 // proportion to the pairs; faster than both other forms from 2.5 to 10), 64 and 128 the tile form from 4 on (sums kept on
-// chip, no pair matrix through memory).
+// chip, no pair matrix). At 64 channels the tile form is faster up to two of its work-groups a CU: 14.6 us against 18.9 at 20k
+// voxels of 5.3 pairs, 20.8 against 22.9 at 55k, but 28.4 against 25.7 at 76k.
 extern "C" int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels) {
     if (n < 1 || n >= (1ll << 24)) return 0;
     if (ptv3_conv_few_pairs(n_pairs, channels)) return 0;
+    const bool tiles = (channels == 64 || channels == 128) && n_pairs >= 4 * n;
+    if (tiles && channels == 64 && n <= 2 * 256 * 128) return 2;
     if ((channels == 32 || channels == 64) && n_pairs <= 14 * n) return 1;
-    if ((channels == 64 || channels == 128) && n_pairs >= 4 * n) return 2;
-    return 0;
+    return tiles ? 2 : 0;
 }
 
 extern "C" int ptv3_pad_rows(const void* x, int x_dtype, int64_t n, int c, int padded, void* out, int out_dtype, void* stream_) {

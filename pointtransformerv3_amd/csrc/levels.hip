@@ -777,15 +777,6 @@ void carve_list_scratch(Carver& c, Carver& kept, ListLevel& v, bool five) {
     }
 }
 
-// outputs per tile at a level whose only tile form is the 128-channel one (see ops.tile_voxels_for): rounds of 512 resident
-// work-groups, a tile's cost a quarter fixed
-int group_of(int64_t n, bool only128) {
-    if (!only128) return 128;
-    const int64_t c128 = ptv3_ceil_div(ptv3_ceil_div(n, 128), 512) * (32 + 128);
-    const int64_t c96 = ptv3_ceil_div(ptv3_ceil_div(n, 96), 512) * (32 + 96);
-    return c96 < c128 ? 96 : 128;
-}
-
 int launch_hash_count(State& s, int first, int levels, hipStream_t stream) {
     ListArgs& a = s.lists;
     hipLaunchKernelGGL(hash_clear_kernel, dim3((unsigned)list_blocks(a, first, levels, 0)), dim3(256), 0, stream, a);
@@ -838,7 +829,7 @@ Bytes carve_begin(State& s, void* tables, void* scratch) {
     s.keys = c.take<uint64_t>((size_t)g.n_orders * n);
     ListLevel& v = s.lists.lv[0];
     v.n = n;
-    v.group = group_of(n, g.only128[0]);
+    v.group = ptv3_conv_tile_voxels(n, g.only128[0] ? 128 : 64);
     carve_list_scratch(c, kept, v, g.stem5);
     v.idx = (const int4*)s.lv[0].indices;
     return {kept.off, c.off};
@@ -1041,7 +1032,7 @@ Bytes carve_pool(State& s, void* tables, void* scratch) {
         s.cells.cid[l] = free.take<int32_t>(g.n);
         ListLevel& v = s.lists.lv[l];
         v.n = s.lv[l].n;
-        v.group = group_of(v.n, g.only128[l]);
+        v.group = ptv3_conv_tile_voxels(v.n, g.only128[l] ? 128 : 64);
         carve_list_scratch(free, c, v, false);
     }
     return {c.off, free.off};

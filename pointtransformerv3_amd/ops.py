@@ -895,18 +895,9 @@ def conv_pack_weight(weight, taps, dtype):
     return packed
 
 
-TILE_CONV_RESIDENT = 512   # work-groups of the tile form the part holds at a time (two per CU)
-
-
 def tile_voxels_for(n, channels):
-    """Outputs per tile for the tile form: a launch runs in rounds of TILE_CONV_RESIDENT work-groups and costs whole
-    rounds; a tile's cost is about a quarter fixed (its 27 weight matrices) and the rest in proportion to its
-    outputs. 128 unless tiles of 96 (128 channels only) make the cheaper set of rounds: 146,195 voxels are 2.2
-    rounds of 128-voxel tiles (three rounds paid) or 2.97 rounds of 96-voxel ones."""
-    if channels != 128:
-        return 128
-    cost = {tv: -(-(-(-n // tv)) // TILE_CONV_RESIDENT) * (32 + tv) for tv in (128, 96)}
-    return 96 if cost[96] < cost[128] else 128
+    """Outputs per tile of the lists that the tile form of this level reads (the rule stands beside the kernel)."""
+    return _lib.load().ptv3_conv_tile_voxels(n, channels)
 
 
 def subm_conv_tiles(feat, plan, packed_weight, bias=None, tile_voxels=None):

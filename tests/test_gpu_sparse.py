@@ -769,6 +769,40 @@ def test_subm_conv_tiles_parity(dtype, c, n, extent):
             o.subm_conv_tiles(feat.to(DEV), plan, packed, b.to(DEV), tile_voxels=96)     # 96 is for 128 channels
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c,n,groups", [(128, 31, (1, 1)), (128, 8193, (1, 1)), (128, 30_000, (2, 2)), (128, 36_000, (2, 3)),
+                                        (128, 65_536, (4, 1)), (64, 32_768, (2,)), (64, 32_769, (4,)), (64, 65, (2,))])
+def test_subm_conv_tiles_every_share_of_a_tile(dtype, c, n, groups):
+    """Work-groups of 32, 64, 96 and 128 outputs (`groups` by 32, for lists of 128 and 96), whole and ragged, and rows and a
+    bias that start at an odd element, against 64 bits: a sum of 27 c exact products in fp32 is off by at most 27 c 2^-23
+    of the products' magnitudes, its rounding by half a unit of the result."""
+    rng = np.random.default_rng(n)
+    g = torch.Generator().manual_seed(n)
+    idx = np.unique(np.concatenate([np.zeros((2 * n, 1)), rng.integers(0, max(int(n ** 0.5) // 2, 6), (2 * n, 3))], 1), axis=0)
+    idx = rng.permutation(idx.astype(np.int32))[:n]
+    n = len(idx)
+    o = ops()
+    plan = o.conv_plan_direct(to_dev(idx), 3)
+    x = torch.randn(n, c, generator=g).to(dtype)
+    w = (torch.randn(c, 27, c, generator=g) * 0.05).to(dtype)
+    b = torch.randn(c, generator=g).to(dtype)
+    nbr = torch.from_numpy(OI.subm_kmap(idx, 3).astype(np.int64)).to(DEV)
+    xd, wd = torch.cat([x, torch.zeros(1, c, dtype=dtype)]).to(DEV).double(), w.to(DEV).double()
+    want, size = b.to(DEV).double().expand(n, c).clone(), b.to(DEV).double().abs().expand(n, c).clone()
+    for t in range(27):
+        rows = xd[nbr[:, t]]                      # -1: the row of zeros
+        want += rows @ wd[:, t].t().contiguous()
+        size += rows.abs() @ wd[:, t].abs().t().contiguous()
+    bound = 27 * c * 2.0 ** -23 * size + (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) * want.abs() + 2.0 ** -24
+    packed = o.conv_pack_weight(w.to(DEV), 27, dtype)
+    odd = [torch.cat([v.new_zeros(1), v.flatten()]).to(DEV)[1:].view(v.shape) for v in (x, b)]
+    assert all(v.data_ptr() % 16 == 2 for v in odd)
+    for tile in (128, 96)[:len(groups)]:
+        got = o.subm_conv_tiles(x.to(DEV), plan, packed, b.to(DEV), tile_voxels=tile)
+        assert ((got.double() - want).abs() <= bound).all(), tile
+        assert torch.equal(o.subm_conv_tiles(odd[0], plan, packed, odd[1], tile_voxels=tile), got), tile
+
+
 def test_tile_size_choice_follows_the_rounds():
     o = ops()
     assert o.tile_voxels_for(146_195, 128) == 96      # 2.2 rounds of 128-voxel tiles, 2.97 of 96-voxel ones
