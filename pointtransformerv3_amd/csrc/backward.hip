@@ -600,6 +600,8 @@ __global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ out, int6
     if (i < count) out[i] = 0.f;
 }
 
+constexpr int LNB_WAVES = 8;   // of a work-group of add_layer_norm_bwd_kernel
+
 template <typename T> struct Row8;
 template <> struct Row8<float> {
     static __device__ __forceinline__ void load(const float* p, float* v) {
@@ -693,6 +695,19 @@ __device__ __forceinline__ void raw8_floats(const Raw8& r, int dtype, float* v) 
     }
 }
 
+// the same for one value
+__device__ __forceinline__ uint32_t raw1_load(const void* p, int dtype, int64_t off) {
+    uint32_t r;
+    if (dtype == PTV3_F32) r = ((const uint32_t*)p)[off];
+    else r = ((const uint16_t*)p)[off];
+    return r;
+}
+__device__ __forceinline__ float raw1_float(uint32_t r, int dtype) {
+    if (dtype == PTV3_F32) return __builtin_bit_cast(float, r);
+    if (dtype == PTV3_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)r);
+    return __builtin_bit_cast(float, r << 16);
+}
+
 // Tensors of one call, each with its own dtype: autocast mixes a float residual stream with half-precision
 // branches, and the kernels read and write each in place instead of going through cast passes.
 struct AnyRows {
@@ -708,6 +723,8 @@ struct AnyRowsOut {
 // per LPR lanes; the statistics are taken from the sum as stored, so the backward kernel sees the same numbers.
 // PRE: the branch goes through a LayerNorm of its own first (pre_gamma, pre_beta, pre_eps): the xCPE's norm in front
 // of the first residual connection of a Block (model.py:546-554, :589-592).
+// Bound by its traffic: with a row's operands asked for while the row before is worked on and three work-groups a CU 45 us at
+// 306k x 64 (skip and sum float: 235 MB at 5.2 TB/s), 40 with PRE; 58 and 57 without, with two (every row a trip to memory).
 template <int LPR, bool PRE>
 __global__ __launch_bounds__(256) void add_layer_norm_fwd_kernel(AnyRows skip, AnyRows branch, AnyRows row_scale,
                                                                  AnyRows gamma, AnyRows beta, int64_t n, float eps,
@@ -723,24 +740,32 @@ __global__ __launch_bounds__(256) void add_layer_norm_fwd_kernel(AnyRows skip, A
         load8_any(pre_gamma.p, pre_gamma.dtype, sub * 8, pg);
         load8_any(pre_beta.p, pre_beta.dtype, sub * 8, pb);
     }
+    // operands of a row, asked for one turn ahead; what is not there is read from the branch and not used, past the end the last row
+    const AnyRows skip_at = skip.p ? skip : branch, scale_at = row_scale.p ? row_scale : branch;
+    struct Row { Raw8 b, s; uint32_t m; };
+    auto fetch = [&](int64_t row) {
+        row = min(row, n - 1);
+        const int64_t off = row * C + sub * 8;
+        return Row{raw8_load(branch.p, branch.dtype, off), raw8_load(skip_at.p, skip_at.dtype, off),
+                   raw1_load(scale_at.p, scale_at.dtype, row)};
+    };
     const int64_t stride = (int64_t)gridDim.x * 4 * RPW;
-    for (int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RPW; row0 < n; row0 += stride) {
+    int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RPW;
+    Row next = fetch(row0 + rsub);
+    for (; row0 < n; row0 += stride) {
         const int64_t row = row0 + rsub;
         const bool valid = row < n;
         const int64_t off = row * C + sub * 8;
+        const Row now = next;
+        next = fetch(row + stride);
         float xv[8], sv[8];
+        raw8_floats(now.b, branch.dtype, xv);
+        raw8_floats(now.s, skip_at.dtype, sv);
+        const float m = row_scale.p ? raw1_float(now.m, row_scale.dtype) : 1.f;
+        if (!skip.p)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { xv[i] = 0.f; sv[i] = 0.f; }
-        float m = 1.f;
-        if (valid) {
-            const Raw8 rb = raw8_load(branch.p, branch.dtype, off);
-            Raw8 rs = rb;
-            if (skip.p) rs = raw8_load(skip.p, skip.dtype, off);
-            if (row_scale.p) m = load1_any(row_scale.p, row_scale.dtype, row);
-            raw8_floats(rb, branch.dtype, xv);
-            if (skip.p) raw8_floats(rs, skip.dtype, sv);
-        }
-        if (PRE) {   // every lane takes part in the row sums, rows past the end with zeros
+            for (int i = 0; i < 8; ++i) sv[i] = 0.f;
+        if (PRE) {   // every lane takes part in the row sums
             float ps = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) ps += xv[i];
@@ -752,14 +777,12 @@ __global__ __launch_bounds__(256) void add_layer_norm_fwd_kernel(AnyRows skip, A
 #pragma unroll
             for (int i = 0; i < 8; ++i) xv[i] = fmaf(xv[i] * prstd, pg[i], pb[i]);
         }
-        if (valid) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) xv[i] = fmaf(xv[i], m, sv[i]);
-            if (sum.p) {
+        for (int i = 0; i < 8; ++i) xv[i] = fmaf(xv[i], m, sv[i]);
+        if (sum.p) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) xv[i] = round_any(xv[i], sum.dtype);
-                store8_any(sum.p, sum.dtype, off, xv);
-            }
+            for (int i = 0; i < 8; ++i) xv[i] = round_any(xv[i], sum.dtype);
+            if (valid) store8_any(sum.p, sum.dtype, off, xv);
         }
         float s = 0.f;
 #pragma unroll
@@ -781,8 +804,11 @@ __global__ __launch_bounds__(256) void add_layer_norm_fwd_kernel(AnyRows skip, A
 // own dtype; dgamma / dbeta accumulated in fp32. Mean and rstd are recomputed from sum.
 // PRE: the branch came out of a LayerNorm of its own (see the forward kernel): pre_x is that norm's input,
 // dbranch its gradient, dpre_gamma / dpre_beta the norm's parameter gradients.
+// Large levels: its traffic (306k x 64: 313 MB, 60 us, 62 with PRE; 69 and 78 with a row's operands asked for in its own turn).
+// Small ones: the atomics of the column sums, so eight waves share a work-group and its one atomic a channel: 9.3k x 512
+// 21 and 23 us, with twice the work-groups of four waves 27 and 30; half as many waves leave loads unasked for (93 at 306k x 64).
 template <int LPR, bool PRE>
-__global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, AnyRows dy, AnyRows dsum, AnyRows row_scale,
+__global__ __launch_bounds__(LNB_WAVES * PTV3_WAVE) void add_layer_norm_bwd_kernel(AnyRows sum, AnyRows dy, AnyRows dsum, AnyRows row_scale,
                                                                  AnyRows gamma, int64_t n, float eps, AnyRowsOut dskip,
                                                                  AnyRowsOut dbranch, float* __restrict__ dgamma,
                                                                  float* __restrict__ dbeta, AnyRows pre_x,
@@ -790,7 +816,7 @@ __global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, An
                                                                  float* __restrict__ dpre_gamma,
                                                                  float* __restrict__ dpre_beta) {
     constexpr int C = LPR * 8, RPW = PTV3_WAVE / LPR;
-    __shared__ float part[PRE ? 4 : 2][4][C];
+    __shared__ float part[PRE ? 4 : 2][LNB_WAVES][C];
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
     const int sub = lane % LPR, rsub = lane / LPR;
     float g[8], ag[8], ab[8], pg[8], pag[8], pab[8];
@@ -798,33 +824,38 @@ __global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, An
     if (PRE) load8_any(pre_gamma.p, pre_gamma.dtype, sub * 8, pg);
 #pragma unroll
     for (int i = 0; i < 8; ++i) { ag[i] = 0.f; ab[i] = 0.f; pag[i] = 0.f; pab[i] = 0.f; }
-    const int64_t stride = (int64_t)gridDim.x * 4 * RPW;
-    for (int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RPW; row0 < n; row0 += stride) {
+    // as in the forward kernel: one turn ahead, what is not there read from the sum and not used
+    const bool scaled = row_scale.p && dbranch.p;
+    const AnyRows dsum_at = dsum.p ? dsum : sum, scale_at = scaled ? row_scale : sum;
+    struct Row { Raw8 x, g, e, c; uint32_t m; };
+    auto fetch = [&](int64_t row) {
+        row = min(row, n - 1);
+        const int64_t off = row * C + sub * 8;
+        Row r = {raw8_load(sum.p, sum.dtype, off), raw8_load(dy.p, dy.dtype, off), raw8_load(dsum_at.p, dsum_at.dtype, off), {},
+                 raw1_load(scale_at.p, scale_at.dtype, row)};
+        if (PRE) r.c = raw8_load(pre_x.p, pre_x.dtype, off);
+        return r;
+    };
+    const int64_t stride = (int64_t)gridDim.x * LNB_WAVES * RPW;
+    int64_t row0 = ((int64_t)blockIdx.x * LNB_WAVES + wave) * RPW;
+    Row next = fetch(row0 + rsub);
+    for (; row0 < n; row0 += stride) {
         const int64_t row = row0 + rsub;
         const bool valid = row < n;
         const int64_t off = row * C + sub * 8;
-        float xv[8], gv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) { xv[i] = 0.f; gv[i] = 0.f; }
-        float extra[8], scale = 1.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) extra[i] = 0.f;
-        if (valid) {
-            const Raw8 rx = raw8_load(sum.p, sum.dtype, off);
-            const Raw8 rg = raw8_load(dy.p, dy.dtype, off);
-            Raw8 re = rx;
-            if (dsum.p) re = raw8_load(dsum.p, dsum.dtype, off);   // gradient arriving at the sum by another path
-            if (row_scale.p && dbranch.p) scale = load1_any(row_scale.p, row_scale.dtype, row);
-            raw8_floats(rx, sum.dtype, xv);
-            raw8_floats(rg, dy.dtype, gv);
-            if (dsum.p) raw8_floats(re, dsum.dtype, extra);
-        }
+        const Row now = next;
+        next = fetch(row + stride);
+        float xv[8], gv[8], extra[8];
+        raw8_floats(now.x, sum.dtype, xv);
+        raw8_floats(now.g, dy.dtype, gv);
+        raw8_floats(now.e, dsum_at.dtype, extra);   // gradient arriving at the sum by another path
+        const float scale = scaled ? raw1_float(now.m, row_scale.dtype) : 1.f;
         float cv[8];   // PRE: the input of the branch's own norm
+        if (PRE) raw8_floats(now.c, pre_x.dtype, cv);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) cv[i] = 0.f;
-        if (PRE && valid) {
-            const Raw8 rc = raw8_load(pre_x.p, pre_x.dtype, off);
-            raw8_floats(rc, pre_x.dtype, cv);
+        for (int i = 0; i < 8; ++i) {
+            if (!valid) gv[i] = 0.f;   // rows past the end add nothing to the column sums
+            if (!dsum.p) extra[i] = 0.f;
         }
         float s = 0.f;
 #pragma unroll
@@ -838,7 +869,7 @@ __global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, An
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             xv[i] *= rstd;                      // xhat
-            ag[i] = fmaf(gv[i], xv[i], ag[i]);  // rows beyond n carry zeros
+            ag[i] = fmaf(gv[i], xv[i], ag[i]);
             ab[i] += gv[i];
             gv[i] *= g[i];
             s1 += gv[i];
@@ -853,7 +884,7 @@ __global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, An
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] *= scale;   // the gradient of the branch as it was added
         if (PRE) {
-            // back through the branch's own norm: statistics again from its input, rows past the end carry zeros
+            // back through the branch's own norm: statistics again from its input
             float cs = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) cs += cv[i];
@@ -910,33 +941,35 @@ __global__ __launch_bounds__(256) void add_layer_norm_bwd_kernel(AnyRows sum, An
         }
     }
     __syncthreads();
-    for (int c = tid; c < (PRE ? 4 : 2) * C; c += 256) {
+    for (int c = tid; c < (PRE ? 4 : 2) * C; c += LNB_WAVES * PTV3_WAVE) {
         const int which = c / C, ch = c % C;
-        const float v = part[which][0][ch] + part[which][1][ch] + part[which][2][ch] + part[which][3][ch];
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < LNB_WAVES; ++w) v += part[which][w][ch];
         float* dst = which == 0 ? dgamma : which == 1 ? dbeta : which == 2 ? dpre_gamma : dpre_beta;
         atomicAdd(dst + ch, v);
     }
 }
 
-int64_t ln_grid(int64_t n, int c) {
-    const int64_t cap = 512;   // two work-groups per CU: more only add atomics on the column sums (measured)
-    const int64_t rows_per_wg = 4 * (PTV3_WAVE / (c / 8));
-    const int64_t grid = ptv3_ceil_div(n, rows_per_wg);
+int64_t rows_grid(int64_t n, int c, int waves, int64_t cap) {
+    const int64_t grid = ptv3_ceil_div(n, (int64_t)waves * (PTV3_WAVE / (c / 8)));
     return grid > cap ? cap : grid;
 }
+int64_t ln_grid(int64_t n, int c) { return rows_grid(n, c, 4, 512); }   // more only add atomics on the column sums
 
 int launch_add_ln_fwd(AnyRows skip, AnyRows branch, AnyRows row_scale, AnyRows gamma, AnyRows beta, int64_t n, int c,
                       float eps, AnyRowsOut sum, AnyRowsOut y, AnyRows pre_gamma, AnyRows pre_beta, float pre_eps,
                       hipStream_t stream) {
+    const dim3 grid((unsigned)rows_grid(n, c, 4, 768));
 #define PTV3_LNF(L)                                                                                                   \
     if (c == 8 * L) {                                                                                                 \
         if (pre_gamma.p)                                                                                              \
-            hipLaunchKernelGGL((add_layer_norm_fwd_kernel<L, true>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0,     \
-                               stream, skip, branch, row_scale, gamma, beta, n, eps, sum, y, pre_gamma, pre_beta,     \
+            hipLaunchKernelGGL((add_layer_norm_fwd_kernel<L, true>), grid, dim3(256), 0, stream,                      \
+                               skip, branch, row_scale, gamma, beta, n, eps, sum, y, pre_gamma, pre_beta,             \
                                pre_eps);                                                                              \
         else                                                                                                          \
-            hipLaunchKernelGGL((add_layer_norm_fwd_kernel<L, false>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0,    \
-                               stream, skip, branch, row_scale, gamma, beta, n, eps, sum, y, pre_gamma, pre_beta,     \
+            hipLaunchKernelGGL((add_layer_norm_fwd_kernel<L, false>), grid, dim3(256), 0, stream,                     \
+                               skip, branch, row_scale, gamma, beta, n, eps, sum, y, pre_gamma, pre_beta,             \
                                pre_eps);                                                                              \
         PTV3_RETURN_LAUNCH();                                                                                         \
     }
@@ -948,15 +981,16 @@ int launch_add_ln_fwd(AnyRows skip, AnyRows branch, AnyRows row_scale, AnyRows g
 int launch_add_ln_bwd(AnyRows sum, AnyRows dy, AnyRows dsum, AnyRows row_scale, AnyRows gamma, int64_t n, int c, float eps,
                       AnyRowsOut dskip, AnyRowsOut dbranch, float* dgamma, float* dbeta, AnyRows pre_x, AnyRows pre_gamma,
                       float pre_eps, float* dpre_gamma, float* dpre_beta, hipStream_t stream) {
+    const dim3 grid((unsigned)rows_grid(n, c, LNB_WAVES, 256)), block(LNB_WAVES * PTV3_WAVE);
 #define PTV3_LNB(L)                                                                                                   \
     if (c == 8 * L) {                                                                                                 \
         if (pre_x.p)                                                                                                  \
-            hipLaunchKernelGGL((add_layer_norm_bwd_kernel<L, true>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0,     \
-                               stream, sum, dy, dsum, row_scale, gamma, n, eps, dskip, dbranch, dgamma, dbeta, pre_x, \
+            hipLaunchKernelGGL((add_layer_norm_bwd_kernel<L, true>), grid, block, 0, stream,                          \
+                               sum, dy, dsum, row_scale, gamma, n, eps, dskip, dbranch, dgamma, dbeta, pre_x,         \
                                pre_gamma, pre_eps, dpre_gamma, dpre_beta);                                            \
         else                                                                                                          \
-            hipLaunchKernelGGL((add_layer_norm_bwd_kernel<L, false>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0,    \
-                               stream, sum, dy, dsum, row_scale, gamma, n, eps, dskip, dbranch, dgamma, dbeta, pre_x, \
+            hipLaunchKernelGGL((add_layer_norm_bwd_kernel<L, false>), grid, block, 0, stream,                         \
+                               sum, dy, dsum, row_scale, gamma, n, eps, dskip, dbranch, dgamma, dbeta, pre_x,         \
                                pre_gamma, pre_eps, dpre_gamma, dpre_beta);                                            \
         PTV3_RETURN_LAUNCH();                                                                                         \
     }
