@@ -354,6 +354,34 @@ def test_segment_reduce_backward_parity(dtype, reduce):
         assert ((got != 0) == (want != 0)).float().mean() > 0.999
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c,odd", [(8, False), (8, True), (6, False), (100, False), (136, False)])
+def test_segment_reduce_backward_of_every_width(dtype, c, odd):
+    """Vectors of channels and one at a time (channels that are no whole vector, rows that start at an odd element), clusters
+    of 0 to 9 members: exact, the first member that equals the maximum takes the gradient."""
+    o = ops()
+    rng = np.random.default_rng(c)
+    sizes = rng.integers(0, 10, 301)
+    idx_ptr = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    n = int(idx_ptr[-1])
+    indices = rng.permutation(n)
+    g = torch.Generator().manual_seed(c)
+    src = torch.randint(-3, 4, (n, c), generator=g).to(dtype)     # ties
+    dout = torch.randn(len(sizes), c, generator=g).to(dtype)
+    out, want = torch.zeros(len(sizes), c, dtype=dtype), {r: torch.zeros(n, c, dtype=dtype) for r in ("max", "mean")}
+    for k, (b, t) in enumerate(zip(idx_ptr[:-1], idx_ptr[1:])):
+        if t > b:
+            rows = torch.as_tensor(indices[b:t])
+            out[k] = src[rows].max(0).values
+            first = rows[(src[rows] == out[k]).int().argmax(0)]
+            want["max"][first, torch.arange(c)] = dout[k]
+            want["mean"][rows] = (dout[k].float() / (t - b)).to(dtype)
+    at = lambda t: torch.cat([t.new_zeros(1), t.flatten()]).to(DEV)[1:].view(t.shape) if odd else t.to(DEV)
+    for reduce in ("max", "mean"):
+        got = o.segment_reduce_bwd(at(src), at(out), at(dout), to_dev(indices), to_dev(idx_ptr), reduce)
+        assert torch.equal(got.cpu(), want[reduce]), reduce
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_unpool_add_backward_parity(dtype):
     from pointtransformerv3_amd.autograd import UnpoolAdd
