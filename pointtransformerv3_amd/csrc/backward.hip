@@ -38,6 +38,9 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));   // a caller's rows may start at any of their elements
 
 constexpr int WG_T = 64;     // weight block: WG_T output x WG_T input channels
 constexpr int WG_P = 32;     // voxels per staging step
@@ -178,7 +181,6 @@ template <> struct Mfma16<__bf16> {
 // writes pieces of four consecutive rows 4 q .. 4 q + 3 (8 channels of group g each) transposed: per channel the
 // four halves are one 8-byte word at tile[8 g + c][4 q], chunks of 8 rows swizzled by the channel group
 __device__ __forceinline__ void put_transposed4(uint16_t* tile, int g, int q, const u32x4* w) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     uint16_t* base = tile + (8 * g) * OR_S + (((q >> 1) ^ (g & 3)) << 3) + ((q & 1) << 2);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
     typedef typename Mfma16<T>::v8 v8;
     __shared__ float wave_cols[4][OR_C];
     __shared__ __align__(16) uint16_t tiles[4][2][OR_C * OR_S];
-    __shared__ int32_t list_a[GATHER ? OR_LIST : 1], list_b[GATHER ? OR_LIST : 1];
+    __shared__ __align__(16) int32_t list_a[GATHER ? OR_LIST : 4], list_b[GATHER ? OR_LIST : 4];
     __shared__ int list_n;
     int tap, split, m0, k0;
     if (!outer_item<OR_C>((int)blockIdx.x - batch.first[which], taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
@@ -268,24 +270,33 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
     // A wave's LDS tiles are its own and its LDS operations complete in order, so the loop needs no barrier:
     // the waves drift apart and hide each other's load latency. The pieces of the next step are requested as
     // soon as this step's have been written to LDS, and arrive while the MFMAs run.
-    u32x4 wa[4], wb[4];
-    auto fetch = [&](int base) {
-        const int mine = base + wave * 32;
+    // The loads ask no question, so that a step waits for its own pieces only: rows past the end are the range's last (first)
+    // and cleared in front of LDS. Gathered rows are asked for two steps ahead (32 channels, 392k voxels 113 -> 99 us), rows in
+    // order one (two: 164 us against 159 for a block of 306k x 64).
+    constexpr int AHEAD = GATHER ? 2 : 1;
+    u32x4 wa[AHEAD][4], wb[AHEAD][4];
+    const T* a_col = a + (a_in ? m0 + 8 * g : 0);
+    const T* b_col = b + (b_in ? k0 + 8 * g : 0);
+    auto fetch = [&](int base, u32x4 (&wa)[4], u32x4 (&wb)[4]) {
+        const int idx = base + wave * 32 + 4 * rq;
+        i32x4 ra = {}, rb = {};
+        if (GATHER) {
+            ra = *(const i32x4*)(list_a + min(idx, OR_LIST - 4));
+            rb = *(const i32x4*)(list_b + min(idx, OR_LIST - 4));
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int idx = mine + 4 * rq + j;
-            wa[j] = (u32x4){0, 0, 0, 0};
-            wb[j] = (u32x4){0, 0, 0, 0};
-            if (idx < count) {
-                const int64_t ra = r0 + (GATHER ? list_a[idx] : idx);
-                const int64_t rb = GATHER ? (int64_t)list_b[idx] : ra;
-                if (a_in) wa[j] = *(const u32x4*)(a + ra * m_total + m0 + 8 * g);
-                if (b_in) wb[j] = *(const u32x4*)(b + rb * k_total + k0 + 8 * g);
-            }
+            const bool there = idx + j < count;
+            const int64_t row = r0 + (GATHER ? (there ? ra[j] : 0) : min(idx + j, count - 1));
+            wa[j] = *(const u32x4*)(a_col + row * m_total);
+            wb[j] = *(const u32x4*)(b_col + (GATHER ? (int64_t)(there ? rb[j] : 0) : row) * k_total);
         }
     };
-    if (count > 0) fetch(0);
-    for (int base = 0; base < count; base += 4 * 32) {
+    auto step = [&](int base, u32x4 (&wa)[4], u32x4 (&wb)[4]) {
+        if (base + 4 * 32 > count)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (base + wave * 32 + 4 * rq + j >= count) wa[j] = wb[j] = (u32x4){0, 0, 0, 0};
         if (sum_cols) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -296,7 +307,7 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
         }
         put_transposed4(ta, g, rq, wa);
         put_transposed4(tb, g, rq, wb);
-        if (base + 4 * 32 < count) fetch(base + 4 * 32);
+        fetch(base + 4 * 32 * AHEAD, wa, wb);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             v8 fa[2], fb[2];
@@ -313,7 +324,16 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
                 for (int j = 0; j < 2; ++j)
                     if (i < tm && j < tk) acc[i][j] = Mfma16<T>::mfma(fa[i], fb[j], acc[i][j]);
         }
-    }
+    };
+    if (count > 0)
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) fetch(4 * 32 * s, wa[s], wb[s]);
+    for (int base = 0; base < count; base += 4 * 32 * AHEAD)
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
+            if (base + 4 * 32 * s >= count) break;
+            step(base + 4 * 32 * s, wa[s], wb[s]);
+        }
     __syncthreads();   // every wave is done with its tiles
     // the four waves hold sums over different rows: add them up in LDS (the operand tiles are free now), then
     // every thread stores 16 of the block's 64 x 64 values into this split's slab, without atomics.
@@ -356,31 +376,70 @@ __global__ __launch_bounds__(256) void outer_rows_kernel(OuterBatch batch) {
     }
 }
 
-// The same reduction for results of 128 channels or more a side: a work-group owns a 128 x 128 block, its
-// four waves a 64 x 64 quadrant each, and the 32 rows of a step are staged once for all of them (threads
-// 0..127 the pieces of a, 128..255 those of b) into one of two LDS buffers, a barrier per step. Per MFMA that
-// is half the operand traffic and half the staging work of the 64 x 64 form, which at 256 channels is bound by
-// the gathered 128-byte pieces coming out of L2.
+// The same reduction for results of 128 channels or more a side: a work-group owns a 128 x 128 block, its four waves a 64 x 64
+// quadrant each. The 32 rows of a step go from memory to LDS as they are (global_load_lds, three steps ahead; 16-byte
+// pieces swizzled by the row), and ds_read_b64_tr_b16 turns them into operands on the way out: four rows of 16 channels
+// become 16 lanes' four rows of a channel. Rows past the end are the range's last on the way in and cleared before they
+// are read. The column sums of a are products with ones. DMA = 0: an operand does not start at a multiple of 16 bytes.
+// Bound by memory: the weight gradients of a block of 37k x 256 move 340 MB (68 us) in 130 us, 5 results of 52 blocks whose
+// work-groups start together and wait for the same lines; 161 us when the rows went through registers (v_perm and
+// ds_write). Gathered rows, 1.45M pairs of 128: 188 -> 127 us.
 constexpr int OW_C = 128;
+constexpr int OW_ROWS = 32, OW_BUFS = 4;
+constexpr int OW_LIST = 1408;   // most rows per work-group with GATHER
 
-template <typename T, bool GATHER>
-__global__ __launch_bounds__(256) void outer_rows_wide_kernel(OuterBatch batch) {
+__device__ __forceinline__ uint32_t lds_address(const uint16_t* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)p;
+}
+// This lane's channels (LDS addresses a0, a1, b0, b1) of rows 0 - 3, 4 - 7, 16 - 19 and 20 - 23 from its first on, OW_C halves a
+// row. Written out, with its wait: behind the builtin the compiler waits for every global_load_lds on its way first.
+struct WideOperands {
+    u32x2 a0[4], a1[4], b0[4], b1[4];
+};
+__device__ __forceinline__ void read_operands(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, WideOperands& f) {
+    static_assert(OW_C == 128, "the offsets below");
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\t"
+        "ds_read_b64_tr_b16 %1, %16 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %8, %18\n\t"
+        "ds_read_b64_tr_b16 %9, %18 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %4, %17\n\t"
+        "ds_read_b64_tr_b16 %5, %17 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %12, %19\n\t"
+        "ds_read_b64_tr_b16 %13, %19 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %16 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %3, %16 offset:5120\n\t"
+        "ds_read_b64_tr_b16 %10, %18 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %11, %18 offset:5120\n\t"
+        "ds_read_b64_tr_b16 %6, %17 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %7, %17 offset:5120\n\t"
+        "ds_read_b64_tr_b16 %14, %19 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %15, %19 offset:5120\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f.a0[0]), "=&v"(f.a0[1]), "=&v"(f.a0[2]), "=&v"(f.a0[3]), "=&v"(f.a1[0]), "=&v"(f.a1[1]), "=&v"(f.a1[2]),
+          "=&v"(f.a1[3]), "=&v"(f.b0[0]), "=&v"(f.b0[1]), "=&v"(f.b0[2]), "=&v"(f.b0[3]), "=&v"(f.b1[0]), "=&v"(f.b1[1]),
+          "=&v"(f.b1[2]), "=&v"(f.b1[3])
+        : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
+        : "memory");
+}
+
+template <typename T, bool GATHER, bool DMA>
+__global__ __launch_bounds__(256, 2) void outer_rows_wide_kernel(OuterBatch batch) {
     const int which = outer_which(batch);
     const OuterJob& job = batch.job[which];
-    const T* __restrict__ a = (const T*)job.a;
-    const T* __restrict__ b = (const T*)job.b;
     const int64_t n = job.n, rows_per_split = job.rows_per_split, slab_stride = job.slab_stride;
     const int m_total = job.m_total, k_total = job.k_total, taps = job.taps, splits = job.splits;
     const int32_t *__restrict__ nbr = job.nbr, *__restrict__ tap_ptr = job.tap_ptr, *__restrict__ pair_in = job.pair_in;
     float *__restrict__ d = job.d, *__restrict__ colsum = job.colsum;
     typedef typename Mfma16<T>::v8 v8;
-    __shared__ __align__(16) uint16_t tiles[2][2][OW_C * OR_S];
-    __shared__ int32_t list_a[GATHER ? OR_LIST : 1], list_b[GATHER ? OR_LIST : 1];
+    // a's rows, then b's; apart, so that the compiler sees that reading one does not wait for the loads into the others
+    __shared__ __align__(16) uint16_t buf0[2 * OW_ROWS * OW_C], buf1[2 * OW_ROWS * OW_C], buf2[2 * OW_ROWS * OW_C],
+        buf3[2 * OW_ROWS * OW_C];
+    __shared__ int32_t list[GATHER ? 2 * OW_LIST : 1];   // rows of a, rows of b
     __shared__ int list_n;
-    __shared__ float wave_cols[2][OW_C];
     int tap, split, m0, k0;
     if (!outer_item<OW_C>((int)blockIdx.x - batch.first[which], taps, splits, m_total, k_total, &tap, &split, &m0, &k0)) return;
-    const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / PTV3_WAVE), lane = tid % PTV3_WAVE;
     int64_t r0 = (int64_t)split * rows_per_split;
     const int64_t r1 = min(n, r0 + rows_per_split);
     int count = (int)(r1 - r0);
@@ -393,8 +452,8 @@ __global__ __launch_bounds__(256) void outer_rows_wide_kernel(OuterBatch batch) 
         // past the end of a short tap's list: the sum over ranges skips this one (a single range is the result itself)
         if (count == 0 && splits > 1) return;
         for (int e = tid; e < count; e += 256) {
-            list_a[e] = nbr[p0 + e];
-            list_b[e] = pair_in[p0 + e];
+            list[e] = nbr[p0 + e];
+            list[OW_LIST + e] = pair_in[p0 + e];
         }
         r0 = 0;
         __syncthreads();
@@ -410,106 +469,114 @@ __global__ __launch_bounds__(256) void outer_rows_wide_kernel(OuterBatch batch) 
             base = __shfl(base, 0, PTV3_WAVE);
             if (src >= 0) {
                 const int pos = base + __popcll(mask & ((1ull << lane) - 1));
-                list_a[pos] = (int32_t)(e - r0);
-                list_b[pos] = src;
+                list[pos] = (int32_t)(e - r0);
+                list[OW_LIST + pos] = src;
             }
         }
         __syncthreads();
         count = list_n;
     }
-    // this wave's quadrant, 2 x 2 tiles
-    const int qm = (wave & 1) * 64, qk = (wave >> 1) * 64;
-    f32x16 acc[2][2];
+    f32x16 acc[2][2], acc_cols[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc_cols[i][v] = 0.f;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    // staging role: operand, channel group, row quad
-    const bool is_b = tid >= 128;
-    const int st = tid & 127, g = st & 15, rq = st >> 4;
-    const T* src_ptr = is_b ? b : a;
-    const int width = is_b ? k_total : m_total, c0 = (is_b ? k0 : m0) + 8 * g;
-    const bool in_range = c0 < width;
-    const bool sum_cols = colsum != nullptr && k0 == 0 && (!GATHER || tap == taps / 2);
-    float cs[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) cs[c] = 0.f;
-    u32x4 w[4];
-    auto fetch = [&](int base) {
+    }
+    // staging: waves 0 and 1 bring a's rows, 2 and 3 b's, 16 each, four (1 KB) a load; lane l row l / 16, piece l % 16
+    const bool is_b = wave >= 2;
+    const int width = is_b ? k_total : m_total, st_row = (wave & 1) * 16 + lane / 16;
+    const int c0 = (is_b ? k0 : m0) + (((lane & 15) ^ ((lane / 16) << 2)) * 8);
+    const T* src_col = (const T*)(is_b ? job.b : job.a) + (c0 < width ? c0 : 0);   // sums of columns that are not there are not stored
+    const int list_at = is_b ? OW_LIST : 0;
+    if (!GATHER || !is_b) src_col += r0 * width;
+    const int st_at = ((is_b ? OW_ROWS : 0) + (wave & 1) * 16) * OW_C;
+    auto stage = [&](int base, uint16_t* buf) {
+        int row[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int idx = base + 4 * rq + j;
-            w[j] = (u32x4){0, 0, 0, 0};
-            if (idx < count && in_range) {
-                const int64_t ra = r0 + (GATHER ? list_a[idx] : idx);
-                const int64_t row = is_b ? (GATHER ? (int64_t)list_b[idx] : ra) : ra;
-                w[j] = *(const u32x4*)(src_ptr + row * width + c0);
-            }
+            const int idx = min(base + st_row + 4 * j, count - 1);
+            row[j] = GATHER ? list[list_at + idx] : idx;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const T* from = src_col + (int64_t)row[j] * width;
+            uint16_t* to = buf + st_at + 4 * j * OW_C;
+            if constexpr (DMA)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                                 (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+            else
+                *(u32x4*)(to + lane * 8) = *(const u32x4_a2*)from;
         }
     };
-    const int col = lane & 31, hf = lane >> 5;
-    if (count > 0) fetch(0);
-    int buf = 0;
-    for (int base = 0; base < count; base += 32, buf ^= 1) {
-        if (sum_cols && !is_b) {
+    // this wave's quadrant, 2 x 2 tiles; reading: 16 lanes take four rows of 16 channels, 8 bytes each
+    const int qm = (wave & 1) * 64, qk = (wave >> 1) * 64;
+    const int col = lane & 31, hf = lane >> 5, l16 = lane & 15;
+    const int in_row = (8 * hf + l16 / 4) * OW_C + (l16 & 1) * 4, low = 2 * ((lane >> 4) & 1) + ((l16 & 3) >> 1);
+    auto at = [&](int channel) { return in_row + ((((channel / 8) ^ ((l16 / 4) << 2)) | low) * 8); };
+    const uint32_t a0 = 2 * at(qm), a1 = 2 * at(qm + 32), b0 = 2 * (OW_ROWS * OW_C + at(qk)), b1 = 2 * (OW_ROWS * OW_C + at(qk + 32));
+    // the column sums of a (the bias gradient) ride along in the blocks that read each of a's rows exactly once: the
+    // first block along k, and with GATHER the centre tap, whose pairs are (i, i) for every voxel
+    const bool sum_cols = colsum != nullptr && k0 == 0 && (!GATHER || tap == taps / 2);
+    const bool my_cols = sum_cols && qk == 0;
+    v8 ones;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const v8 h = __builtin_bit_cast(v8, w[j]);
-#pragma unroll
-                for (int c = 0; c < 8; ++c) cs[c] += (float)h[c];
-            }
+    for (int i = 0; i < 8; ++i) ones[i] = (T)1.f;
+    auto step = [&](int base, uint16_t* buf, uint16_t* ahead) {
+        // Everyone's rows of this step are in LDS (those of the two after it may still be on their way), and everyone is
+        // through with the buffer of the step before, which takes the rows three steps on.
+        asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        stage(base + (OW_BUFS - 1) * OW_ROWS, ahead);
+        if (base + OW_ROWS > count) {
+            for (int e = tid; e < 2 * OW_ROWS * OW_C / 8; e += 256)
+                if (base + e / (OW_C / 8) % OW_ROWS >= count) *(u32x4*)(buf + e * 8) = (u32x4){0, 0, 0, 0};
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
-        put_transposed4(tiles[buf][is_b], g, rq, w);
-        if (base + 32 < count) fetch(base + 32);
-        // One barrier per step: it also keeps a wave from overwriting this buffer two steps on while another
-        // still reads it, because nobody passes the next step's barrier before everyone has finished these reads.
-        __syncthreads();
-        const uint16_t* ta = tiles[buf][0];
-        const uint16_t* tb = tiles[buf][1];
+        const uint32_t from = lds_address(buf);
+        WideOperands f;
+        read_operands(from + a0, from + a1, from + b0, from + b1, f);
+        auto whole = [](const u32x2* p) { return __builtin_bit_cast(v8, (u32x4){p[0][0], p[0][1], p[1][0], p[1][1]}); };
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            v8 fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int cha = qm + 32 * i + col, chb = qk + 32 * i + col;
-                fa[i] = __builtin_bit_cast(v8, *(const u32x4*)(ta + cha * OR_S + 8 * ((2 * ks + hf) ^ ((cha >> 3) & 3))));
-                fb[i] = __builtin_bit_cast(v8, *(const u32x4*)(tb + chb * OR_S + 8 * ((2 * ks + hf) ^ ((chb >> 3) & 3))));
-            }
+            const v8 fa[2] = {whole(f.a0 + 2 * ks), whole(f.a1 + 2 * ks)}, fb[2] = {whole(f.b0 + 2 * ks), whole(f.b1 + 2 * ks)};
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) acc[i][j] = Mfma16<T>::mfma(fa[i], fb[j], acc[i][j]);
+            if (my_cols)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc_cols[i] = Mfma16<T>::mfma(fa[i], ones, acc_cols[i]);
         }
-    }
+    };
+    uint16_t* const bufs[OW_BUFS] = {buf0, buf1, buf2, buf3};
+    if (count > 0)
+#pragma unroll
+        for (int s = 0; s < OW_BUFS - 1; ++s) stage(s * OW_ROWS, bufs[s]);
+    for (int base = 0; base < count; base += OW_BUFS * OW_ROWS)
+#pragma unroll
+        for (int s = 0; s < OW_BUFS; ++s) {
+            if (base + s * OW_ROWS >= count) break;
+            step(base + s * OW_ROWS, bufs[s], bufs[(s + OW_BUFS - 1) % OW_BUFS]);
+        }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be on its way into this LDS when the work-group ends
     // acc[i][j][v]: m = m0 + qm + 32 i + 8 (v / 4) + 4 hf + v % 4, k = k0 + qk + 32 j + col; the quadrant is this wave's alone
     float* slab = d + (int64_t)split * slab_stride;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int k = k0 + qk + 32 * j + col;
+        for (int v = 0; v < 16; ++v) {
+            const int m = m0 + qm + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
+            if (m >= m_total) continue;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int m = m0 + qm + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
-                if (m < m_total && k < k_total) slab[((int64_t)m * taps + tap) * k_total + k] = acc[i][j][v];
+            for (int j = 0; j < 2; ++j) {
+                const int k = k0 + qk + 32 * j + col;
+                if (k < k_total) slab[((int64_t)m * taps + tap) * k_total + k] = acc[i][j][v];
             }
+            if (my_cols && col == 0) colsum[(int64_t)split * slab_stride + m] = acc_cols[i][v];
         }
-    if (sum_cols) {   // the same for the whole work-group; waves 0 and 1 staged a
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            cs[c] += __shfl_xor(cs[c], 16, PTV3_WAVE);
-            cs[c] += __shfl_xor(cs[c], 32, PTV3_WAVE);
-        }
-        if (!is_b && lane < 16) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) wave_cols[wave][8 * g + c] = cs[c];
-        }
-        __syncthreads();
-        if (tid < OW_C && m0 + tid < m_total)
-            colsum[(int64_t)split * slab_stride + m0 + tid] = wave_cols[0][tid] + wave_cols[1][tid];
-    }
 }
 
 // out[i] = sum over the splits' slabs (of `stride` floats, the first `total` of them summed): a work-group takes 32 neighbouring values, its 8 thread rows share
@@ -1329,13 +1396,14 @@ void outer_split(int64_t n, int64_t blocks, int taps, int64_t cap, int64_t* spli
 }
 
 // Rows per range of the gathering 128 x 128 form. Over all taps there are about ten pairs per voxel at the levels that have
-// these widths: about 1200 work-groups, between the slabs that shorter ranges write (384 rows: 246 against 168 us at 156k
-// x 128) and the uneven end of longer ones (4096: 284 against 200 us at 43k x 256). A result whose blocks and taps alone
-// fill the part is left without slabs while its rows are few (570 x 512: 22 us against 49 in two ranges).
+// these widths: about 300 work-groups, between the slabs that shorter ranges write (384 rows: 54 against 39 us at 36k x 128,
+// 225 against 134 at 149k x 128, 59 against 39 at 9.2k x 256) and too few work-groups (1280 rows: 27 against 20 us at 5k x 128).
+// While a work-group's rows are few beside its blocks and taps, one range and no slabs (600 x 256: 15 us against 19 in two,
+// 1100 x 512: 24 against 40 in three).
 int64_t outer_gather_rows(int64_t n, int64_t blocks, int taps) {
-    if (n <= 1024 && blocks * taps >= 256) return ptv3_ceil_div(n, 128) * 128;
-    const int64_t r = ptv3_ceil_div(n * blocks, 120 * 128) * 128;
-    return r < 384 ? 384 : r > 1408 ? 1408 : r;
+    if (n <= OW_LIST && n <= 6 * blocks * taps) return ptv3_ceil_div(n, 128) * 128;
+    const int64_t r = ptv3_ceil_div(n * blocks, 30 * 128) * 128;
+    return r < 384 ? 384 : r > 1280 ? 1280 : r;
 }
 
 // block side: 128 when both sides of the result have that many channels, else 64
@@ -1383,8 +1451,13 @@ int outer_prepare(const void* a, const void* b, int64_t n, int m_total, int k_to
 
 template <typename T, bool GATHER>
 void outer_launch(const OuterBatch& batch, int side, hipStream_t stream) {
+    uintptr_t at = 0;
+    for (int i = 0; i < batch.count; ++i) at |= (uintptr_t)batch.job[i].a | (uintptr_t)batch.job[i].b;
+    const bool dma = at % 16 == 0;
     const dim3 grid((unsigned)batch.first[batch.count]);
-    if (side == OW_C) hipLaunchKernelGGL((outer_rows_wide_kernel<T, GATHER>), grid, dim3(256), 0, stream, batch);
+    if (side == OW_C)
+        hipLaunchKernelGGL((dma ? outer_rows_wide_kernel<T, GATHER, true> : outer_rows_wide_kernel<T, GATHER, false>), grid,
+                           dim3(256), 0, stream, batch);
     else hipLaunchKernelGGL((outer_rows_kernel<T, GATHER>), grid, dim3(256), 0, stream, batch);
 }
 

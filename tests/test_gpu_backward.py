@@ -354,6 +354,27 @@ def test_segment_reduce_backward_parity(dtype, reduce):
         assert ((got != 0) == (want != 0)).float().mean() > 0.999
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,nout,odd", [(1, 128, 128, False), (31, 136, 128, False), (33, 128, 200, False), (129, 256, 136, True),
+                                          (4097, 264, 384, False), (20_011, 128, 128, True)])
+def test_linear_wgrad_of_wide_results(dtype, n, k, nout, odd):
+    """Weight and bias gradients of 128 channels or more a side at the edges of its 32-row steps and 128 x 128 blocks, rows that
+    start at an odd element, against 64 bits: an fp32 sum of n exact products is off by at most n 2^-23 of their magnitudes.
+    An infinity stays in its own row and column."""
+    g = torch.Generator().manual_seed(n + k)
+    at = lambda t: torch.cat([t.new_zeros(1), t.flatten()]).to(DEV)[1:].view(t.shape) if odd else t.to(DEV)
+    x, dout = torch.randn(n, k, generator=g).to(dtype), torch.randn(n, nout, generator=g).to(dtype)
+    dw, db = ops().linear_wgrad(at(x), at(dout), with_bias=True)
+    a, b = dout.to(DEV).double(), x.to(DEV).double()
+    assert ((dw.double() - a.t().contiguous() @ b).abs() <= n * 2.0 ** -23 * (a.abs().t().contiguous() @ b.abs())).all()
+    assert ((db.double() - a.sum(0)).abs() <= n * 2.0 ** -23 * a.abs().sum(0)).all()
+    x[n - 1, k - 1], dout[n - 1, 0] = float("inf"), float("inf")
+    dw, db = ops().linear_wgrad(at(x), at(dout), with_bias=True)
+    finite = torch.ones(nout, k, dtype=torch.bool)
+    finite[0], finite[:, k - 1] = False, False
+    assert torch.equal(torch.isfinite(dw).cpu(), finite) and torch.equal(torch.isfinite(db).cpu(), finite[:, 0])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("c,odd", [(8, False), (8, True), (6, False), (100, False), (136, False)])
 def test_segment_reduce_backward_of_every_width(dtype, c, odd):
