@@ -668,6 +668,10 @@ __global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ out, int6
 }
 
 constexpr int LNB_WAVES = 8;   // of a work-group of add_layer_norm_bwd_kernel
+// Waves of a BatchNorm work-group that sums columns: its one atomic a channel counts, and with an exact GELU to differentiate
+// the VALU work, for which two waves a SIMD are too few: the 13 layers of a step on four rooms 814 -> 598 us backward, 253 -> 167
+// for the statistics, against two work-groups of four waves a CU without the rows of the next turn asked for.
+constexpr int BN_WAVES = 16;
 
 template <typename T> struct Row8;
 template <> struct Row8<float> {
@@ -1022,7 +1026,7 @@ int64_t rows_grid(int64_t n, int c, int waves, int64_t cap) {
     const int64_t grid = ptv3_ceil_div(n, (int64_t)waves * (PTV3_WAVE / (c / 8)));
     return grid > cap ? cap : grid;
 }
-int64_t ln_grid(int64_t n, int c) { return rows_grid(n, c, 4, 512); }   // more only add atomics on the column sums
+int64_t bn_grid(int64_t n, int c) { return rows_grid(n, c, BN_WAVES, 256); }
 
 int launch_add_ln_fwd(AnyRows skip, AnyRows branch, AnyRows row_scale, AnyRows gamma, AnyRows beta, int64_t n, int c,
                       float eps, AnyRowsOut sum, AnyRowsOut y, AnyRows pre_gamma, AnyRows pre_beta, float pre_eps,
@@ -1132,8 +1136,8 @@ __device__ __forceinline__ float gelu_grad(float z) {
 
 // adds every lane's eight column values up over the rows a wave holds side by side, the waves and, with one
 // atomic per channel, the work-groups: out[ch] += ..., out2[ch] += ...
-template <int LPR>
-__device__ __forceinline__ void column_sums_out(float* a, float* b, float (*part)[4][LPR * 8], float* out, float* out2) {
+template <int LPR, int WAVES>
+__device__ __forceinline__ void column_sums_out(float* a, float* b, float (*part)[WAVES][LPR * 8], float* out, float* out2) {
     constexpr int C = LPR * 8;
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
     const int sub = lane % LPR, rsub = lane / LPR;
@@ -1153,30 +1157,37 @@ __device__ __forceinline__ void column_sums_out(float* a, float* b, float (*part
         }
     }
     __syncthreads();
-    for (int c = tid; c < 2 * C; c += 256) {
+    for (int c = tid; c < 2 * C; c += WAVES * PTV3_WAVE) {
         const int which = c / C, ch = c % C;
-        const float v = part[which][0][ch] + part[which][1][ch] + part[which][2][ch] + part[which][3][ch];
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v += part[which][w][ch];
         atomicAdd((which ? out2 : out) + ch, v);
     }
 }
 
 // sums[0][ch] += sum_rows (x - x[0][ch]), sums[1][ch] += sum_rows (x - x[0][ch])^2
 template <int LPR>
-__global__ __launch_bounds__(256) void bn_stats_kernel(AnyRows x, int64_t n, float* __restrict__ sums) {
+__global__ __launch_bounds__(BN_WAVES * PTV3_WAVE) void bn_stats_kernel(AnyRows x, int64_t n, float* __restrict__ sums) {
     constexpr int C = LPR * 8, RPW = PTV3_WAVE / LPR;
-    __shared__ float part[2][4][C];
+    __shared__ float part[2][BN_WAVES][C];
     const int wave = threadIdx.x / PTV3_WAVE, lane = threadIdx.x % PTV3_WAVE;
     const int sub = lane % LPR, rsub = lane / LPR;
     float pivot[8], s1[8], s2[8];
     load8_any(x.p, x.dtype, sub * 8, pivot);
 #pragma unroll
     for (int i = 0; i < 8; ++i) { s1[i] = 0.f; s2[i] = 0.f; }
-    const int64_t stride = (int64_t)gridDim.x * 4 * RPW;
-    for (int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RPW; row0 < n; row0 += stride) {
+    const int64_t stride = (int64_t)gridDim.x * BN_WAVES * RPW;
+    int64_t row0 = ((int64_t)blockIdx.x * BN_WAVES + wave) * RPW;
+    auto fetch = [&](int64_t row) { return raw8_load(x.p, x.dtype, min(row, n - 1) * C + sub * 8); };
+    Raw8 next = fetch(row0 + rsub);   // a turn ahead
+    for (; row0 < n; row0 += stride) {
         const int64_t row = row0 + rsub;
+        const Raw8 now = next;
+        next = fetch(row + stride);
         if (row < n) {
             float v[8];
-            raw8_floats(raw8_load(x.p, x.dtype, row * C + sub * 8), x.dtype, v);
+            raw8_floats(now, x.dtype, v);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float d = v[i] - pivot[i];
@@ -1185,7 +1196,7 @@ __global__ __launch_bounds__(256) void bn_stats_kernel(AnyRows x, int64_t n, flo
             }
         }
     }
-    column_sums_out<LPR>(s1, s2, part, sums, sums + C);
+    column_sums_out<LPR, BN_WAVES>(s1, s2, part, sums, sums + C);
 }
 
 // one work-group: stats[0] = mean, stats[1] = rstd from the sums above; running averages updated in place
@@ -1213,11 +1224,11 @@ __global__ __launch_bounds__(256) void bn_finalize_kernel(AnyRows x, const float
 // PASS 1: dx = gamma * rstd * (dz - sums[1] / n - xhat * sums[0] / n), or gamma * rstd * dz when the statistics
 // were not the batch's own (evaluation mode). dz = dy * gelu'(gamma * xhat + beta) with GELU, else dy.
 template <int LPR, int PASS>
-__global__ __launch_bounds__(256) void bn_bwd_kernel(AnyRows x, AnyRows dy, const float* __restrict__ stats,
+__global__ __launch_bounds__((PASS == 0 ? BN_WAVES : 4) * PTV3_WAVE) void bn_bwd_kernel(AnyRows x, AnyRows dy, const float* __restrict__ stats,
                                                      AnyRows gamma, AnyRows beta, int64_t n, int gelu, int batch_stats,
                                                      float* __restrict__ sums, AnyRowsOut dx) {
-    constexpr int C = LPR * 8, RPW = PTV3_WAVE / LPR;
-    __shared__ float part[2][4][C];
+    constexpr int C = LPR * 8, RPW = PTV3_WAVE / LPR, WAVES = PASS == 0 ? BN_WAVES : 4;
+    __shared__ float part[2][PASS == 0 ? WAVES : 1][C];
     const int wave = threadIdx.x / PTV3_WAVE, lane = threadIdx.x % PTV3_WAVE;
     const int sub = lane % LPR, rsub = lane / LPR;
     float mean[8], rstd[8], g[8], b[8], a1[8], a2[8];
@@ -1240,13 +1251,20 @@ __global__ __launch_bounds__(256) void bn_bwd_kernel(AnyRows x, AnyRows dy, cons
             a2[i] = sums[C + sub * 8 + i] * inv_n;   // mean of dz
         }
     }
-    const int64_t stride = (int64_t)gridDim.x * 4 * RPW;
-    for (int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RPW; row0 < n; row0 += stride) {
+    struct Row { Raw8 x, g; };
+    auto fetch = [&](int64_t row) {
+        const int64_t off = min(row, n - 1) * C + sub * 8;
+        return Row{raw8_load(x.p, x.dtype, off), raw8_load(dy.p, dy.dtype, off)};
+    };
+    const int64_t stride = (int64_t)gridDim.x * WAVES * RPW;
+    int64_t row0 = ((int64_t)blockIdx.x * WAVES + wave) * RPW;
+    Row next = fetch(row0 + rsub);   // a turn ahead
+    for (; row0 < n; row0 += stride) {
         const int64_t row = row0 + rsub;
+        const auto [rx, rg] = next;
+        next = fetch(row + stride);
         if (row < n) {
             const int64_t off = row * C + sub * 8;
-            const Raw8 rx = raw8_load(x.p, x.dtype, off);
-            const Raw8 rg = raw8_load(dy.p, dy.dtype, off);
             float xv[8], dz[8];
             raw8_floats(rx, x.dtype, xv);
             raw8_floats(rg, dy.dtype, dz);
@@ -1269,15 +1287,16 @@ __global__ __launch_bounds__(256) void bn_bwd_kernel(AnyRows x, AnyRows dy, cons
             }
         }
     }
-    if (PASS == 0) column_sums_out<LPR>(a1, a2, part, sums, sums + C);
+    if constexpr (PASS == 0) column_sums_out<LPR, WAVES>(a1, a2, part, sums, sums + C);
 }
 
 template <int PASS>
 int launch_bn_bwd(AnyRows x, AnyRows dy, const float* stats, AnyRows gamma, AnyRows beta, int64_t n, int c, int gelu,
                   int batch_stats, float* sums, AnyRowsOut dx, hipStream_t stream) {
+    const dim3 grid((unsigned)(PASS == 0 ? bn_grid(n, c) : rows_grid(n, c, 4, 2048))), block((PASS == 0 ? BN_WAVES : 4) * PTV3_WAVE);
 #define PTV3_BNB(L)                                                                                                   \
     if (c == 8 * L) {                                                                                                 \
-        hipLaunchKernelGGL((bn_bwd_kernel<L, PASS>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0, stream, x, dy,      \
+        hipLaunchKernelGGL((bn_bwd_kernel<L, PASS>), grid, block, 0, stream, x, dy,                                   \
                            stats, gamma, beta, n, gelu, batch_stats, sums, dx);                                       \
         PTV3_RETURN_LAUNCH();                                                                                         \
     }
@@ -1753,7 +1772,7 @@ extern "C" int ptv3_batch_norm_stats(const void* x, int dtype, int64_t n, int c,
     hipLaunchKernelGGL(zero_kernel, dim3((unsigned)ptv3_ceil_div(2 * c, 256)), dim3(256), 0, stream, workspace, (int64_t)2 * c);
 #define PTV3_BNS(L)                                                                                                   \
     if (c == 8 * L)                                                                                                   \
-        hipLaunchKernelGGL((bn_stats_kernel<L>), dim3((unsigned)ln_grid(n, c)), dim3(256), 0, stream, xr, n, workspace);
+        hipLaunchKernelGGL((bn_stats_kernel<L>), dim3((unsigned)bn_grid(n, c)), dim3(BN_WAVES * PTV3_WAVE), 0, stream, xr, n, workspace);
     PTV3_BNS(4) PTV3_BNS(8) PTV3_BNS(16) PTV3_BNS(32) PTV3_BNS(64)
 #undef PTV3_BNS
     hipLaunchKernelGGL(bn_finalize_kernel, dim3(1), dim3(256), 0, stream, xr, (const float*)workspace, n, c, eps, momentum,
