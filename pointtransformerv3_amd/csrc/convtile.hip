@@ -95,9 +95,7 @@ __global__ __launch_bounds__(CT_THREADS) void pack_weight_kernel(const T* __rest
 
 // the same for several weights in one launch: job j owns blocks first_block[j] .. first_block[j + 1]
 __global__ __launch_bounds__(CT_THREADS) void pack_weight_batch_kernel(const ptv3_pack_job* __restrict__ jobs, int n_jobs) {
-    int j = 0;
-    for (int i = 1; i < n_jobs; ++i)
-        if (jobs[i].first_block <= (int64_t)blockIdx.x) j = i;   // uniform: a handful of jobs, first_block ascending
+    const int j = ptv3_job_of_block(jobs, n_jobs);
     const ptv3_pack_job job = jobs[j];
     const int c = job.channels, taps = job.taps;
     if (c < 32 || c % 32 != 0 || taps < 1) return;   // a row no *_blocks() helper would have sized: touch nothing

@@ -52,9 +52,7 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(const T* __restrict__ w1,
 
 // the same for several MLPs in one launch: job j owns blocks first_block[j] .. first_block[j + 1]
 __global__ __launch_bounds__(256) void mlp_pack_batch_kernel(const ptv3_mlp_pack_job* __restrict__ jobs, int n_jobs) {
-    int j = 0;
-    for (int i = 1; i < n_jobs; ++i)
-        if (jobs[i].first_block <= (int64_t)blockIdx.x) j = i;   // uniform: a handful of jobs, first_block ascending
+    const int j = ptv3_job_of_block(jobs, n_jobs);
     const ptv3_mlp_pack_job job = jobs[j];
     const int c = job.channels;
     if (c != 128 && c != 256 && c != 512) return;   // a width the fused kernel does not take: touch nothing
