@@ -794,7 +794,7 @@ def main():
                      "attn_ms_per_step": attn_ms / args.steps,
                      "valu_exp_floor_ms_per_step": exp_floor_ms / args.steps,
                      "valu_exp_frac": exp_floor_ms / attn_ms if attn_ms > 0 else 0.0,
-                     "conv": {"kernels": "conv_sparse, conv_tile, pair_wstat / pair_gemm + pair_segment_sum",
+                     "conv": {"kernels": "conv_sparse, conv_gather, pair_wstat / pair_gemm + pair_segment_sum",
                               "measured": "events around every convolution launch, in a loop of the same forwards "
                                           "right after the timed region, queued module by module (so are the attention "
                                           "above, serialize and kmap below; the timed forwards queue the same kernels "

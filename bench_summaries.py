@@ -136,7 +136,7 @@ def _grouped(rows, groups, per):
 INDEX = ["hash_", "list_", "cell_", "slots_kernel", "facts_kernel", "publish_", "plan_", "direct_", "vh_", "kmap", "inner_",
          "pool_gather", "pool_offsets", "cluster_", "attn_slots", "pad_index", "pad_prefix", "offset2batch"]
 SERIALIZATION = ["scatter_kernel", "digit_totals", "zero_words", "order_", "encode", "grid_max", "small_sort", "inverse_kernel"]
-CONV = ["pair_gemm", "pair_wstat", "pair_segment", "subm_conv", "conv_tile", "conv_sparse"]
+CONV = ["pair_gemm", "pair_wstat", "pair_segment", "subm_conv", "conv_gather", "conv_sparse"]
 LINEAR = ["linear_rows", "linear_ln", "linear_wide", "linear_tile", "few_kernel", "linear_any", "gemm_f32"]
 
 FORWARD_GROUPS = collections.OrderedDict([
@@ -447,7 +447,7 @@ def training_trace(d, out_dir):
 
 def conv_counters(d, out_dir):
     """profiles/conv_<workload>_counters.txt, one per workload whose raw files are there."""
-    keep = ("conv_sparse", "conv_tile", "pair_wstat", "pair_gemm", "subm_conv_pairs", "pair_segment_sum")
+    keep = ("conv_sparse", "conv_gather", "pair_wstat", "pair_gemm", "subm_conv_pairs", "pair_segment_sum")
     done = []
     for wl in CONV_CASES:
         base, line_path = os.path.join(d, f"conv_{wl}"), os.path.join(d, f"conv_{wl}.json")
