@@ -11,7 +11,7 @@
 //   inverse          voxel of every input point.
 // Bound by memory (about 130 bytes move per point). One table of all voxels in device memory cost two atomics per point
 // on lines that eight L2 caches hand to each other (170 us for 1.56M points in 3 scenes); a part's table never leaves the
-// CU (part 30 us, split 22, split_count and split_scan 15). Every point is read four times instead, in order, from the
+// CU (part 30 us, split 22, split_count and split_scan 13). Every point is read four times instead, in order, from the
 // last-level cache. All kernels of that size: 409 -> 149 us, with the rows of three arrays gathered behind them (41 -> 26).
 #include "voxelhash.h"
 
@@ -206,34 +206,39 @@ __global__ __launch_bounds__(VX_THREADS) void vx_split_count_kernel(const float*
     for (int b = threadIdx.x; b < parts; b += VX_THREADS) w.tile_parts[(int64_t)blockIdx.x * parts + b] = cnt[b];
 }
 
-// Down the tiles: 64 parts per work-group, 16 waves that take a sixteenth of the tiles each.
-__global__ __launch_bounds__(1024) void vx_split_scan_kernel(VoxWs w) {
-    __shared__ uint32_t sum[16][PTV3_WAVE];
-    const int parts = 1 << w.part_bits, lane = threadIdx.x % PTV3_WAVE, seg = threadIdx.x / PTV3_WAVE;
-    const int64_t per = (w.tiles + 15) / 16, t0 = min(w.tiles, seg * per), t1 = min(w.tiles, t0 + per);
-    uint32_t* __restrict__ col = w.tile_parts + blockIdx.x * PTV3_WAVE + lane;
-    uint32_t v[8], total = 0;
-    for (int64_t t = t0; t < t1; t += 8) {
+// Down the tiles: 16 parts per work-group, 64 threads of a part that take a 64th of the tiles each, up to 512 tiles (2M points)
+// in one trip to memory of eight loads a thread. Bound by that trip and the barrier's chain: 1.56M points in 3 scenes 5.4 us,
+// 7.2 with 64 parts and 16 threads of each, which went to memory three times down and three times back.
+constexpr int VX_SCAN_PARTS = 16, VX_SCAN_SEGS = 64, VX_SCAN_AT_ONCE = 8;
+static_assert(VX_SCAN_PARTS <= 1 << VX_MIN_PART_BITS, "whole work-groups");
+__global__ __launch_bounds__(VX_SCAN_PARTS * VX_SCAN_SEGS) void vx_split_scan_kernel(VoxWs w) {
+    __shared__ uint32_t sum[VX_SCAN_SEGS][VX_SCAN_PARTS];
+    const int parts = 1 << w.part_bits, mine = threadIdx.x % VX_SCAN_PARTS, seg = threadIdx.x / VX_SCAN_PARTS;
+    const int64_t per = (w.tiles + VX_SCAN_SEGS - 1) / VX_SCAN_SEGS, t0 = min(w.tiles, seg * per), t1 = min(w.tiles, t0 + per);
+    uint32_t* __restrict__ col = w.tile_parts + blockIdx.x * VX_SCAN_PARTS + mine;
+    uint32_t v[VX_SCAN_AT_ONCE], total = 0;
+    for (int64_t t = t0; t < t1; t += VX_SCAN_AT_ONCE) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = t + k < t1 ? col[(t + k) * parts] : 0u;
+        for (int k = 0; k < VX_SCAN_AT_ONCE; ++k) v[k] = t + k < t1 ? col[(t + k) * parts] : 0u;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) total += v[k];
+        for (int k = 0; k < VX_SCAN_AT_ONCE; ++k) total += v[k];
     }
-    sum[seg][lane] = total;
+    sum[seg][mine] = total;
     __syncthreads();
     uint32_t run = 0, all = 0;
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const uint32_t c = sum[s][lane];
+    for (int s = 0; s < VX_SCAN_SEGS; ++s) {
+        const uint32_t c = sum[s][mine];
         if (s < seg) run += c;
         all += c;
     }
-    if (seg == 0) w.part_size[blockIdx.x * PTV3_WAVE + lane] = all;
-    for (int64_t t = t0; t < t1; t += 8) {
+    if (seg == 0) w.part_size[blockIdx.x * VX_SCAN_PARTS + mine] = all;
+    for (int64_t t = t0; t < t1; t += VX_SCAN_AT_ONCE) {
+        if (per > VX_SCAN_AT_ONCE)   // else the loads above still stand in v
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = t + k < t1 ? col[(t + k) * parts] : 0u;
+            for (int k = 0; k < VX_SCAN_AT_ONCE; ++k) v[k] = t + k < t1 ? col[(t + k) * parts] : 0u;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < VX_SCAN_AT_ONCE; ++k) {
             if (t + k < t1) col[(t + k) * parts] = run;
             run += v[k];
         }
@@ -577,7 +582,7 @@ extern "C" int ptv3_voxelize(const float* coord, int64_t n, const int64_t* offse
     hipLaunchKernelGGL(vx_init_kernel, dim3((unsigned)ptv3_ceil_div(3 * (int64_t)n_scenes, 256)), dim3(256), 0, stream, w, n_scenes, offset_out);
     hipLaunchKernelGGL(vx_scene_min_kernel, tiles, threads, 0, stream, coord, n, offset, n_scenes, w);
     hipLaunchKernelGGL(vx_split_count_kernel, tiles, threads, parts * 4, stream, coord, n, offset, n_scenes, grid_size, w);
-    hipLaunchKernelGGL(vx_split_scan_kernel, dim3((unsigned)(parts / PTV3_WAVE)), dim3(1024), 0, stream, w);
+    hipLaunchKernelGGL(vx_split_scan_kernel, dim3((unsigned)(parts / VX_SCAN_PARTS)), dim3(VX_SCAN_PARTS * VX_SCAN_SEGS), 0, stream, w);
     hipLaunchKernelGGL(vx_split_kernel, tiles, threads, split_lds, stream, coord, n, offset, n_scenes, grid_size, w);
     hipLaunchKernelGGL(vx_part_kernel, dim3((unsigned)parts), threads, 0, stream, w, pick_seed);
     hipLaunchKernelGGL(vx_count_kernel, tiles, threads, 0, stream, n, w);

@@ -28,6 +28,12 @@ def test_voxelize_edges(sizes, grid, extent):
         assert np.array_equal(got[name].cpu().numpy(), want), name
 
 
+@pytest.mark.parametrize("n", [64 * 4096, 64 * 4096 + 1, 512 * 4096, 512 * 4096 + 1])
+def test_voxelize_where_the_scan_down_the_tiles_takes_another_turn(n):
+    """A thread of the scan has one tile | two, eight in one trip | nine in two."""
+    test_voxelize_edges([n - 5000, 5000], 0.05, 2.0)
+
+
 @pytest.mark.parametrize("seed", [0, 9])
 def test_voxelize_more_voxels_than_the_parts_tables_hold(seed):
     """14M voxels over 4096 parts: tables in memory. Against a sort of the voxel keys."""
