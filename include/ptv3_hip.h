@@ -138,7 +138,12 @@ int ptv3_patch_attn_fwd(const void *qkv, int dtype, int64_t n_rows, int channels
                         const int32_t *cu_seqlens, int64_t n_seq, int64_t max_seqlen,
                         float scale, void *out, void *stream);
 
-/* The same with the relative position bias of model.py:297-316, :468-469 (fp32 only: the reference
+/* How the MFMA kernel cuts a launch of `items` (sequence, head) pairs into work-groups on a part of `cus` CUs: the first *full
+ * items whole, the others as the number returned (1 ... 8) of ranges of query tiles; 1: all whole, *full = items. slots: of the
+ * n_seq sequences together. Results do not depend on it. */
+int ptv3_patch_attn_cut(int64_t items, int64_t slots, int64_t n_seq, int64_t max_seqlen, int64_t cus, int64_t *full);
+
+/* ptv3_patch_attn_fwd with the relative position bias of model.py:297-316, :468-469 (fp32 only: the reference
  * applies it on its non-fused path, in float): score(query i, key j, head h) +=
  * sum over the axes a of rpe_table[a * R + clamp(g_i[a] - g_j[a], -pos_bnd, pos_bnd) + pos_bnd][h],
  * R = 2 * pos_bnd + 1; grid_coord (n_rows, 3) int32 in point order, rpe_table (3 * R, heads) fp32,

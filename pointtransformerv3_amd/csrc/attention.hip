@@ -161,7 +161,7 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void patch_attn_half_kernel(
     unsigned char* const_lds = (unsigned char*)knorm_lds + ((lds_keys / 64 * 4 + 15) & ~15);
 
     // The first `full_items` work-groups take one (sequence, head) each; the items left over are cut into
-    // `split` query ranges, one work-group each (tail_split).
+    // `split` query ranges, one work-group each (ptv3_patch_attn_cut).
     int wg, part = 0, parts = 1;
     if ((int)blockIdx.x < full_items) {
         wg = xcd_chunked_id(blockIdx.x, full_items);
@@ -496,6 +496,45 @@ __global__ __launch_bounds__(F32_QB) void patch_attn_rpe_f32_kernel(
     }
 }
 
+}  // namespace
+
+// How a launch is cut into work-groups: the first *full items whole, every other one as that many ranges of query tiles.
+// Two work-groups are resident per CU (LDS), but one alone keeps the VALU of its CU nearly as busy as two do, so a launch
+// lasts as long as the CU with the most work: items up to the last multiple of the CU count go out whole, the rest in as many
+// ranges as make that least. Costs are in query tiles (of 32, against one item's keys):
+//   * the kernel deals items to XCDs by eighths, so the fullest CU is found within an XCD: 42 items in six ranges are 36 work-
+//     groups on 32 CUs, not 252 on 256 (19.8 us; in five 13.1). 84: 25.6 -> 20.3, 340: 56.0 -> 47.5, 1108: 138 -> 133.
+//   * sequences are of any length up to max_seqlen; how long one is, the slots say. 192 items of 250 slots under a patch of
+//     1024 go out whole, 7.7 us, not in four ranges, 10.7. A launch of unequal items lasts at least as long as its longest
+//     one, taken as 5/4 of the mean: 256 items of 723 slots 34.2 us whole, 25.7 in two ranges, of 486 17.4 and 18.9.
+//   * a range stages all keys again: four tiles for 1024 slots, up to nine for few (staging shrinks less than the products).
+//     Alone on its CU it also waits for that (eight). Equal costs go to two ranges where CUs would be left over: 198 and 232
+//     items of 1024 slots in a forward 37.3 -> 35.8 us and 37.7 -> 36.6, but 256 items 37.5 whole, 39.5 in two.
+//   * where ranges share a CU, one of less than seven tiles leaves waves idle: 96 items of 746 slots 25.5 us in three ranges,
+//     19.9 in two.
+// Measured in fp16, plain probabilities; with shifted ones (large scores) the order is the same. Cut or not, the same bits.
+extern "C" int ptv3_patch_attn_cut(int64_t items, int64_t slots, int64_t n_seq, int64_t max_seqlen, int64_t cus, int64_t* full) {
+    const int64_t rem = items <= cus ? items : items % cus;
+    *full = items;
+    if (rem == 0 || n_seq < 1) return 1;
+    const int64_t mean = max(min(slots / n_seq, max_seqlen), (int64_t)1);
+    const int64_t tiles = ptv3_ceil_div(mean, 32), longest = ptv3_ceil_div(min(mean * 5 / 4, max_seqlen), 32);
+    const int64_t xcd_cus = max(cus / 8, (int64_t)1);
+    // in sixths of a tile
+    const int64_t staging = 6 * 4 + (32 - min(tiles, (int64_t)32)), alone = 6 * (rem == items ? 8 : 4);
+    int64_t split = 1, best = max(ptv3_ceil_div(rem, cus) * (6 * tiles + staging), 6 * longest + alone);
+    for (int64_t sp = 2; sp <= 8; ++sp) {
+        const int64_t per_cu = ptv3_ceil_div(ptv3_ceil_div(rem, 8) * sp, xcd_cus);
+        if (per_cu == 1 ? longest < sp : tiles < 7 * sp) continue;
+        const int64_t cost = max(per_cu * (6 * ptv3_ceil_div(tiles, sp) + staging), 6 * ptv3_ceil_div(longest, sp) + alone);
+        if (cost < best || (cost == best && sp == 2 && items < cus)) { best = cost; split = sp; }
+    }
+    if (split > 1) *full = items - rem;
+    return (int)split;
+}
+
+namespace {
+
 // LDS of the MFMA kernel for sequences of up to max_seqlen keys: K (+ one prefetch-only step), V^T, per-step key
 // norms (padded to 16 B), ones and zeros. Beyond 160 KB (2368 keys) the sequence does not fit.
 size_t half_lds_bytes(int64_t max_seqlen) {
@@ -507,30 +546,10 @@ bool half_kernel_takes(int dtype, int channels, int heads, int64_t max_seqlen) {
     return dtype != PTV3_F32 && channels / heads == HD && half_lds_bytes(max_seqlen) <= 160 * 1024;
 }
 
-// How a launch is cut. Two work-groups are resident per CU (LDS), but one alone keeps the VALU of its CU nearly as busy as
-// two do: an item of 1024 slots takes 36 us by itself on a CU and 33.5 per item with company. So a launch lasts as long as
-// the CU with the most items, not the most rounds of two: items up to the last multiple of the CU count go out whole, the
-// rest are cut into `split` ranges of query tiles, as many as make the fullest CU's share of tiles least; the staging
-// that every range repeats counts as four tiles. Where there are no whole items, a range alone on its CU also waits for
-// its own staging (eight). Measured (fp16, 1024 slots; us, rounds of two with up to four ranges before / this): 312 items
-// 57 -> 48, 788: 114 -> 105, 592: 83.4 -> 80.4, 192: 43.8 -> 39.1, 96 of 800 slots: 20.7 -> 19.0, 40 of 704: 13.1 -> 11.1,
-// 4 items: 15.2 -> 12.9. Ranges of less than four tiles gain nothing (4 items in 16 ranges: 13.0).
-int64_t tail_split(int64_t total, int64_t cus, int64_t tiles, int64_t* full) {
-    const int64_t rem = total % cus;
-    int64_t split = 1, best = tiles + (total < cus ? 8 : 4);
-    for (int64_t sp = 2; sp <= 8 && tiles >= 4 * sp; ++sp) {
-        const int64_t per_cu = ptv3_ceil_div(rem * sp, cus);
-        const int64_t cost = per_cu * (ptv3_ceil_div(tiles, sp) + (per_cu == 1 && total < cus ? 8 : 4));
-        if (cost < best) { best = cost; split = sp; }
-    }
-    *full = split == 1 ? total : total - rem;
-    return split;
-}
-
 template <typename T, bool LSE, bool DROP>
 int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_src,
                 const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
-                int64_t max_seqlen, float scale, void* out, float* lse, int64_t lse_stride, Dropout drop,
+                int64_t max_seqlen, int64_t slots, float scale, void* out, float* lse, int64_t lse_stride, Dropout drop,
                 hipStream_t stream) {
     const int lds_keys = (int)((max_seqlen + 63) & ~63ll);
     const size_t lds = half_lds_bytes(max_seqlen);
@@ -549,20 +568,19 @@ int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_sr
     }
     const int64_t total = n_seq * heads;
     int64_t full = 0;
-    const int64_t split = tail_split(total, cus, ptv3_ceil_div(max_seqlen, 32), &full);
+    const int split = ptv3_patch_attn_cut(total, slots, n_seq, max_seqlen, cus, &full);
     const int64_t tail = (total - full + 7) / 8 * 8;   // the tail's items in groups of 8, one per XCD
     hipLaunchKernelGGL(kern, dim3((unsigned)(full + tail * split)), dim3(ATT_THREADS), lds, stream,
                        (const T*)qkv, channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys,
-                       scale_log2e, (T*)out, (int)full, (int)split, (int)total, lse, lse_stride, drop);
+                       scale_log2e, (T*)out, (int)full, split, (int)total, lse, lse_stride, drop);
     PTV3_RETURN_LAUNCH();
 }
 
 }  // namespace
 
-extern "C" int ptv3_patch_attn_fwd(const void* qkv, int dtype, int64_t n_rows, int channels,
-                                   int heads, const int32_t* slot_src, const int32_t* slot_dst,
-                                   const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
-                                   float scale, void* out, void* stream_) {
+int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
+                              const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
+                              int64_t slots, float scale, void* out, void* stream_) {
     if (n_rows < 0 || n_seq < 0 || channels < 1 || heads < 1 || max_seqlen < 1) return PTV3_EINVAL;
     if (dtype < PTV3_F32 || dtype > PTV3_BF16) return PTV3_EINVAL;
     if (channels % heads != 0 || !any_head_dim(channels / heads)) return PTV3_ESHAPE;
@@ -573,13 +591,21 @@ extern "C" int ptv3_patch_attn_fwd(const void* qkv, int dtype, int64_t n_rows, i
     if (half_kernel_takes(dtype, channels, heads, max_seqlen)) {
         if (dtype == PTV3_F16)
             return launch_half<_Float16, false, false>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                                       max_seqlen, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
+                                                       max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
         return launch_half<__bf16, false, false>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                                 max_seqlen, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
+                                                 max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
     }
     // fp32, and in half precision other head dims (8, 32, 64) or sequences beyond the MFMA kernel's LDS
     return launch_any(qkv, dtype, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, scale, out,
                       Dropout{0u, 0u, 1.f}, stream);
+}
+
+// The slots are not among the arguments: at least one for every row (a scene's last patch is filled up).
+extern "C" int ptv3_patch_attn_fwd(const void* qkv, int dtype, int64_t n_rows, int channels, int heads,
+                                   const int32_t* slot_src, const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
+                                   int64_t max_seqlen, float scale, void* out, void* stream_) {
+    return ptv3_patch_attn_fwd_slots(qkv, dtype, n_rows, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen,
+                                     n_rows, scale, out, stream_);
 }
 
 extern "C" int ptv3_patch_attn_fwd_lse(const void* qkv, int dtype, int64_t n_rows, int channels, int heads,
@@ -598,8 +624,8 @@ extern "C" int ptv3_patch_attn_fwd_lse(const void* qkv, int dtype, int64_t n_row
         return launch_any(qkv, dtype, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, scale, out, drop,
                           stream);
 #define PTV3_ATT(T, D)                                                                                               \
-    return launch_half<T, true, D>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, scale, out, \
-                                   lse, n_pad, drop, stream)
+    return launch_half<T, true, D>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, n_pad, scale, \
+                                   out, lse, n_pad, drop, stream)
     if (dtype == PTV3_F16) {
         if (drop.threshold) PTV3_ATT(_Float16, true);
         PTV3_ATT(_Float16, false);

@@ -67,6 +67,11 @@ static inline int ptv3_allow_lds(const void* kern, size_t lds, LdsGrant& grant) 
     return 0;
 }
 
+// ptv3_patch_attn_fwd where the number of slots, cu_seqlens[n_seq], is known: what ptv3_patch_attn_cut goes by.
+int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
+                              const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
+                              int64_t slots, float scale, void* out, void* stream);
+
 // Work-groups are dealt to the 8 XCDs round-robin in launch order, and every XCD has an L2 of its own.
 // Launch index (or persistent-loop index, with a grid that is a multiple of 8) -> item such that each XCD
 // works through one contiguous eighth of the items: neighbours in item order, which read the same cache lines

@@ -142,8 +142,8 @@ int conv3(Run& r, const ptv3_block_w& b, int s, const void* x, void* out) {
 
 int attention(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, const void* qkv, int dt, void* out) {
     if (r.dry) return PTV3_OK;
-    return ptv3_patch_attn_fwd(qkv, dt, v.n, b.channels, b.heads, v.slot_src[b.row], v.slot_dst[b.row], v.cu, v.n_seq, patch,
-                               b.scale, out, r.stream);
+    return ptv3_patch_attn_fwd_slots(qkv, dt, v.n, b.channels, b.heads, v.slot_src[b.row], v.slot_dst[b.row], v.cu, v.n_seq, patch,
+                                     v.n_pad, b.scale, out, r.stream);
 }
 
 // A block (model.py:586-606): x its rows, xs what its convolution reads, out the new rows.

@@ -93,6 +93,15 @@ def test_attention_ranges_of_cut_items(counts, patch, heads):
     assert rel_err(got, want) < TOL[torch.float16]
 
 
+@pytest.mark.parametrize("counts,heads", [([700, 901, 640, 1024] * 4, 16),   # 256 items of unequal length in two ranges
+                                          ([150, 163], 4),                  # 8 items: more ranges than some have tiles
+                                          ([981] * 21, 2), ([250, 180] * 6, 16)])
+def test_attention_ranges_of_unequal_items(counts, heads):
+    """Sequences shorter than the patch: the number of ranges follows their mean length, empty ranges write nothing."""
+    got, want = _case(counts, 1024, heads, torch.float16, seed=sum(counts) + heads)
+    assert rel_err(got, want) < TOL[torch.float16]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_is_deterministic(dtype):
     """Two launches over the same input give the same bits."""

@@ -396,3 +396,31 @@ def test_a_class_whose_forward_was_replaced_is_left_to_the_modules(kind, when, m
         assert native.Structure(model).why is not None
     monkeypatch.undo()
     assert structure.same() and native.Structure(model).why is None
+
+
+def _attention_cut(items, slots, n_seq, max_seqlen=1024, cus=256):
+    from pointtransformerv3_amd import _lib
+    full = ctypes.c_int64(-1)
+    split = _lib.load().ptv3_patch_attn_cut(items, slots, n_seq, max_seqlen, cus, ctypes.byref(full))
+    return full.value, split
+
+
+@pytest.mark.parametrize("cus", [256, 80, 6])
+@pytest.mark.parametrize("mean", [1, 131, 600, 1024])
+def test_attention_cut_fills_every_xcd_alike(mean, cus):
+    """Ranges that are meant to have a CU each do: counted where the kernel puts them, an eighth of the items on an XCD."""
+    for items in [*range(1, 1400), 4000, 100_000]:
+        full, split = _attention_cut(items, mean * items, items, cus=cus)
+        assert 1 <= split <= 8 and (full == items if split == 1 else full == (0 if items <= cus else items // cus * cus))
+        if split > 1:
+            fullest = -(-(-(-(items - full) // 8) * split) // max(cus // 8, 1))
+            assert fullest <= split     # never more on a CU than an item
+            assert fullest == 1 or -(-mean // 32) >= 7 * split
+
+
+@pytest.mark.parametrize("items,mean,want", [(42, 981, (0, 5)), (84, 976, (0, 2)), (340, 1024, (256, 2)), (554, 1024, (512, 5)),
+                                             (1108, 1024, (1024, 2)), (192, 250, (192, 1)), (416, 238, (416, 1)), (256, 723, (0, 2)),
+                                             (256, 804, (0, 2)), (256, 486, (256, 1)), (256, 1024, (256, 1)), (198, 1024, (0, 2)),
+                                             (232, 1024, (0, 2)), (312, 1024, (256, 4)), (4, 1024, (0, 8)), (512, 723, (512, 1))])
+def test_attention_cut_measured(items, mean, want):
+    assert _attention_cut(items, mean * items, items) == want
