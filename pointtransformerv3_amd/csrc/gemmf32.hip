@@ -1,31 +1,32 @@
 // fp32 products on the matrix cores: Linear layers of the float model and the pair form of the float submanifold
 // convolution.
 //
-// A float is taken as the sum of two halves, h = half(v 2^S) and l = half((v 2^S - h) 2^11): 22 bits and both signs, and a
-// product is h h' + 2^-11 (h l' + l h') with float sums, three v_mfma_f32_32x32x16_f16 in 96 cycles where eight
-// v_mfma_f32_32x32x2_f32 take 512. What the pieces leave out (l l' and the half of the last bit) is below what the longer
-// chain of roundings of the float instruction adds: error against 64 bits (2-norm, unit normal operands), float
-// instruction -> pieces: K = 32 1.03e-7 -> 0.91e-7, 64 1.44e-7 -> 0.98e-7, 256 2.87e-7 -> 1.31e-7, 2048 8.1e-7 -> 3.0e-7. Below
-// 32 inputs it is not (K = 6: 0.47e-7 -> 0.88e-7), and those layers, and every tile where the pieces do not carry the
-// values, are taken on whole floats: `again` below.
+// A float is taken as the sum of three bf16, each the rest of the one before rounded: 8 + 8 + 8 bits, all that a float has,
+// with a float's range (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019). Of the nine products of two such floats the six largest are taken, six
+// v_mfma_f32_32x32x16_bf16 in 192 cycles where eight v_mfma_f32_32x32x2_f32 take 512; what is left out is 2^-24 of a
+// product at most, 2^-27 of it on average. The first pieces' products have a sum of their own, the smaller ones another, put
+// together at the end: sixteen products a rounding instead of two, so sums are closer to 64 bits than the float
+// instruction's, whatever the operands.
+// Error (2-norm, unit normal operands), float instruction -> pieces: K = 6 4.7e-8 -> 2.8e-8, 32 1.03e-7 -> 0.39e-7,
+// 64 1.44e-7 -> 0.50e-7, 256 2.87e-7 -> 0.89e-7, 2048 8.1e-7 -> 2.7e-7; rows of one value of order 1 under a weight of 1e-8
+// and the rest the other way round, K = 256, 2.87e-7 -> 0.89e-7. (Two halves a float, 22 bits under a fixed scale, three
+// products, take 0.75 of the time but lose such rows: 2.3e-4.)
 //
 // A work-group of four waves owns TM rows x TN outputs. KC inputs of its rows and of its weight rows at a time go
 // global -> registers -> pieces in LDS, two buffers and one barrier per step; the loads of two steps are on the way, none of
 // them under a condition (a condition made the compiler wait for all of them), and the splitting of the next step is
-// scheduled between the products of this one. Bound by the splitting (VALU) and by the latency of a step where a launch has
-// few tiles, by memory at 32 and 64 inputs.
-// Measured (MI355X; us, float instruction -> pieces): 100k x 64 -> 192 40 -> 29, 36k x 128 -> 384 55 -> 31,
-// 11.6k x 256 -> 1024 74 -> 34, 4.8k x 2048 -> 512 125 -> 63, 300 x 2048 -> 512 41 -> 30; a float forward of one room of 100k
-// voxels 10.9 -> 7.8 ms.
+// scheduled between the products of this one. Bound by the matrix cores and the splitting (VALU), by the latency of a step
+// where a launch has few tiles, by memory at 32 and 64 inputs.
+// Measured (MI355X; us, float instruction -> pieces): 100k x 64 -> 192 40 -> 35, 36k x 128 -> 384 51 -> 35, 11.6k x 256 -> 1024
+// 70 -> 42, 2.1k x 2048 -> 512 93 -> 73, 300 x 512 -> 512 18 -> 13; rows of 1e-6, 100k x 64 -> 64 17.5 -> 16.1; a float forward
+// of one room of 100k voxels 10.9 -> 8.5 ms.
 #include "rowtile.h"
 
 namespace {
 
 constexpr int F32_THREADS = 256;
-// Scales of the pieces: rows up to 16376 (2^16 / 4) and weights up to 255 are carried, rows whose largest value is below
-// 2^-16 and weight rows below 2^-22 would lose bits of the second piece. Rows that are halves already are their first piece.
-constexpr int F32_SX = 2, F32_SW = 8;
-constexpr int F32_MIN_K = 32;   // fewer inputs: whole floats
+constexpr uint32_t F32_TINY = (127u - 102u) * (1u << 24) - 1u;   // 2^-102 as `least` sees it
 
 struct F32Args {
     const void* x;          // (rows, k) float or half
@@ -74,23 +75,25 @@ template <> struct Load4<_Float16, true> {
     static __device__ __forceinline__ raw cut(raw v, int left) { return left > 0 ? v : (u32x2){0u, 0u}; }
 };
 
-// four consecutive values of a row as pieces, the second ones KC halves behind the first
-template <int S, int KC> __device__ __forceinline__ void park_pieces(unsigned char* at, f32x4 v) {
-    u32x2 h, l;
+// four consecutive values of a row as PIECES pieces, each KC of them behind the one before
+template <int PIECES, int KC> __device__ __forceinline__ void park_pieces(unsigned char* at, f32x4 v) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const f16x2 t = __builtin_convertvector((f32x2){v[2 * j] * (float)(1 << S), v[2 * j + 1] * (float)(1 << S)}, f16x2);
-        h[j] = __builtin_bit_cast(uint32_t, t);
-        l[j] = H16<_Float16>::pack2(fmaf((float)t[0], -2048.f, v[2 * j] * (float)(2048 << S)),
-                                    fmaf((float)t[1], -2048.f, v[2 * j + 1] * (float)(2048 << S)));
+    for (int q = 0; q < PIECES; ++q) {
+        u32x2 p;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            p[j] = H16<__bf16>::pack2(v[2 * j], v[2 * j + 1]);
+            v[2 * j] -= __builtin_bit_cast(float, p[j] << 16);
+            v[2 * j + 1] -= __builtin_bit_cast(float, p[j] & 0xffff0000u);
+        }
+        *(u32x2*)(at + q * KC * 2) = p;
     }
-    *(u32x2*)at = h;
-    *(u32x2*)(at + KC * 2) = l;
 }
-// max(m, |v|): two instructions; fmaxf would quiet every operand first
-__device__ __forceinline__ float largest(float m, f32x4 v) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v[0]), "v"(v[1]));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(v[2]), "v"(v[3]));
+// the least of m and the sizes of v, in the order of their bits; zero is none
+__device__ __forceinline__ uint32_t least(uint32_t m, f32x4 v) {
+#pragma unroll
+    for (int j = 0; j < 4; j += 2)
+        m = min(m, min(__builtin_bit_cast(uint32_t, v[j]) * 2u - 1u, __builtin_bit_cast(uint32_t, v[j + 1]) * 2u - 1u));
     return m;
 }
 
@@ -100,10 +103,9 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
     constexpr int MT = TM / (32 * WM), NT = TN / (32 * WN);
     constexpr int RL = KC / 4;                  // lanes that hold a row's values of a step, four each
     constexpr int XP = (TM * RL + F32_THREADS - 1) / F32_THREADS, WP = (TN * RL + F32_THREADS - 1) / F32_THREADS;
-    constexpr int ROW = 2 * KC * 2 + 16;        // bytes of an LDS row of pieces: rows start in distinct bank groups
+    constexpr int ROW = 3 * KC * 2 + 16;        // bytes of an LDS row of pieces: rows start in distinct bank groups
     constexpr int STRIDE = KC + 4;              // floats of an LDS row of whole values
-    constexpr bool XHALF = sizeof(XT) == 2;   // a half is its own first piece
-    constexpr int SX = XHALF ? 0 : F32_SX;
+    constexpr int XQ = sizeof(XT) == 2 ? 2 : 3;   // pieces of a row's value: 11 bits of a half are in two
     __shared__ __align__(16) unsigned char lds[2][(TM + TN) * ROW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hf = lane >> 5;
@@ -164,11 +166,7 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
         const int c = min(col0 + ((tid + i * F32_THREADS) / RL), g.nout - 1);
         wrow[i] = g.w + (int64_t)c * g.w_row + (int64_t)tap * g.w_tap;
     }
-    float xm[XP], wm_[WP];   // the largest value of a row among this thread's pieces
-#pragma unroll
-    for (int i = 0; i < XP; ++i) xm[i] = 0.f;
-#pragma unroll
-    for (int i = 0; i < WP; ++i) wm_[i] = 0.f;
+    uint32_t tiny = ~0u;   // the least value that is not zero among this thread's pieces
     struct Stage {   // two steps are on the way
         typename Load4<XT, VEC>::raw x[XP];
         f32x4 w[WP];
@@ -193,18 +191,18 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
         for (int i = 0; i < XP; ++i) {
             const int e = tid + i * F32_THREADS;
             const f32x4 v = Load4<XT, VEC>::value(t.x[i]);
-            if (!XHALF) xm[i] = largest(xm[i], v);
-            if (TM * RL % F32_THREADS == 0 || e < TM * RL) park_pieces<SX, KC>(to + (e / RL) * ROW, v);
+            if (XQ == 3) tiny = least(tiny, v);
+            if (TM * RL % F32_THREADS == 0 || e < TM * RL) park_pieces<XQ, KC>(to + (e / RL) * ROW, v);
         }
 #pragma unroll
         for (int i = 0; i < WP; ++i) {
             const int e = tid + i * F32_THREADS;
-            wm_[i] = largest(wm_[i], t.w[i]);
-            if (TN * RL % F32_THREADS == 0 || e < TN * RL) park_pieces<F32_SW, KC>(to + (TM + (e / RL)) * ROW, t.w[i]);
+            tiny = least(tiny, t.w[i]);
+            if (TN * RL % F32_THREADS == 0 || e < TN * RL) park_pieces<3, KC>(to + (TM + (e / RL)) * ROW, t.w[i]);
         }
     };
 
-    f32x16 acc[MT][NT], low[MT][NT];   // sums of h h', and of (h l' + l h') 2^11
+    f32x16 acc[MT][NT], low[MT][NT];   // sums of the first pieces' products, and of the five smaller ones
     const int steps = (g.k + KC - 1) / KC;
     auto clear = [&](f32x16 (&t)[MT][NT]) {
 #pragma unroll
@@ -222,53 +220,52 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
         const unsigned char* ws = lds[s & 1] + (TM + wn * NT * 32 + col) * ROW + hf * 16;
 #pragma unroll
         for (int c = 0; c < KC / 16; ++c) {
-            f16x8 xa[MT][2], wb[NT][2];
+            bf16x8 xa[MT][3], wb[NT][3];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+            for (int q = 0; q < 3; ++q) {
                 const int off = c * 32 + q * KC * 2;
 #pragma unroll
                 for (int a = 0; a < MT; ++a)
-                    if (q == 0 || !XHALF) xa[a][q] = __builtin_bit_cast(f16x8, *(const u32x4*)(xs + a * 32 * ROW + off));
+                    if (q < XQ) xa[a][q] = __builtin_bit_cast(bf16x8, *(const u32x4*)(xs + a * 32 * ROW + off));
 #pragma unroll
-                for (int b = 0; b < NT; ++b) wb[b][q] = __builtin_bit_cast(f16x8, *(const u32x4*)(ws + b * 32 * ROW + off));
+                for (int b = 0; b < NT; ++b) wb[b][q] = __builtin_bit_cast(bf16x8, *(const u32x4*)(ws + b * 32 * ROW + off));
             }
 #pragma unroll
-            for (int a = 0; a < MT; ++a)
+            for (int i = 0; i < 6; ++i)   // the third piece of a row comes last: a half has none, and the same sums
 #pragma unroll
-                for (int b = 0; b < NT; ++b) {
-                    acc[a][b] = H16<_Float16>::mfma(xa[a][0], wb[b][0], acc[a][b]);
-                    low[a][b] = H16<_Float16>::mfma(xa[a][0], wb[b][1], low[a][b]);
-                    if (!XHALF) low[a][b] = H16<_Float16>::mfma(xa[a][1], wb[b][0], low[a][b]);
-                }
+                for (int a = 0; a < MT; ++a)
+#pragma unroll
+                    for (int b = 0; b < NT; ++b) {
+                        constexpr int QX[6] = {0, 0, 1, 1, 0, 2}, QW[6] = {0, 1, 0, 1, 2, 0};
+                        if (QX[i] >= XQ) continue;
+                        f32x16& sum = i == 0 ? acc[a][b] : low[a][b];
+                        sum = H16<__bf16>::mfma(xa[a][QX[i]], wb[b][QW[i]], sum);
+                    }
         }
         park(t, s + 1);
         fetch(t, (s + 3) * KC);
 #pragma unroll
-        for (int i = 0; i < KC / 16 * MT * NT * (XHALF ? 2 : 3); ++i) {
+        for (int i = 0; i < KC / 16 * MT * NT * (XQ == 2 ? 5 : 6); ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one product, then the splitting of the next step's values
-            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
         }
         __syncthreads();
     };
-    const bool pieces = g.k >= F32_MIN_K;
     clear(acc);
     clear(low);
-    if (pieces) {
-        fetch(st0, 0);
-        fetch(st1, KC);
-        trim(st0, 0);
-        park(st0, 0);
-        fetch(st0, 2 * KC);
-        __syncthreads();
-        for (int s = 0; s < steps; s += 2) {
-            step(s, st1);
-            if (s + 1 < steps) step(s + 1, st0);
-        }
+    fetch(st0, 0);
+    fetch(st1, KC);
+    trim(st0, 0);
+    park(st0, 0);
+    fetch(st0, 2 * KC);
+    __syncthreads();
+    for (int s = 0; s < steps; s += 2) {
+        step(s, st1);
+        if (s + 1 < steps) step(s + 1, st0);
     }
 
-    // Where the pieces do not carry a float - a sum that is not finite (infinities, NaN, values beyond a piece's range), a
-    // row whose values are all so small that the second piece runs out of bits - the work-group takes its tile again on
-    // whole floats.
+    // Where the pieces do not hold every bit - a sum that is not finite (infinities, NaN, values that round past the largest
+    // bf16), a value below 2^-102 whose last piece would be subnormal - the work-group takes its tile again on whole floats.
     float odd = 0.f;
 #pragma unroll
     for (int a = 0; a < MT; ++a)
@@ -276,21 +273,10 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
         for (int b = 0; b < NT; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                acc[a][b][v] = fmaf(low[a][b][v], 1.f / 2048.f, acc[a][b][v]) * (1.f / (float)(1 << (SX + F32_SW)));
+                acc[a][b][v] += low[a][b][v];
                 odd = fmaf(acc[a][b][v], 0.f, odd);
             }
-    bool again = odd != 0.f || !pieces;
-    auto small = [&](float m, float least) {   // RL neighbouring lanes hold a row
-#pragma unroll
-        for (int off = 1; off < RL; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, PTV3_WAVE));
-        again |= m > 0.f && m < least;
-    };
-#pragma unroll
-    for (int i = 0; i < XP; ++i)
-        if (!XHALF) small(xm[i], 1.f / (float)(1 << (14 + F32_SX)));
-#pragma unroll
-    for (int i = 0; i < WP; ++i) small(wm_[i], 1.f / (float)(1 << (14 + F32_SW)));
-    if (__syncthreads_or(again)) {
+    if (__syncthreads_or(odd != 0.f || tiny < F32_TINY)) {
         float* whole = (float*)lds;
         clear(acc);
         for (int s = 0; s < steps; ++s) {
@@ -386,8 +372,8 @@ int launch_f32(F32Args& g, int64_t rows, hipStream_t stream) {
     const double c11 = cost(128, 128, 1.0), c10 = cost(128, 64, 1.05), c00 = cost(64, 64, 1.12);
     if (g.nout > 64 && c11 <= c10 && c11 <= c00) PTV3_TILE(128, 128, 2, 2, 16);
     if (c10 <= c00) PTV3_TILE(128, 64, 2, 2, 16);
-    // steps of 32 inputs halve the barriers of a long row (300 x 2048 -> 512 39 -> 30 us, 11.6k x 1024 -> 256 43 -> 37); a short
-    // one is sooner through its first step with 16 (100k x 64 -> 256 37 against 45)
+    // steps of 32 inputs halve the barriers of a long row (300 x 512 -> 512 15.3 -> 12.6 us, 11.6k x 1024 -> 256 54 -> 48); a short
+    // one is sooner through its first step with 16 (100k x 64 -> 64 15.4 against 16.9)
     if (g.k >= 256) PTV3_TILE(64, 64, 2, 2, 32);
     PTV3_TILE(64, 64, 2, 2, 16);
 #undef PTV3_TILE

@@ -42,8 +42,7 @@ def test_linear_f32_halves_on_one_side(n, k, nout):
 @pytest.mark.parametrize("k", [20, 31, 32, 33, 64, 255, 256, 260])
 @pytest.mark.parametrize("x_scale,w_scale", [(1.0, 1.0), (3e3, 30.0), (1e-4, 1e-6), (1e-7, 1.0), (1.0, 1e-9), (1e30, 1.0), (1.0, 400.0)])
 def test_linear_f32_ranges(k, x_scale, w_scale):
-    """Scales that two halves carry, and scales where a tile is taken on whole floats: every row as exact as float sums
-    are. A sum of k products rounded k times is off by at most k 2^-24 of the sum of their sizes; half of it, and an
+    """Scales from 1e-16 to 1e30 of whole rows, next to rows far below them: every row as exact as float sums are. A sum of k products rounded k times is off by at most k 2^-24 of the sum of their sizes; half of it, and an
     eighth of it for the longer rows, holds for either way (roundings do not all point the same way)."""
     g = torch.Generator().manual_seed(k)
     x, w = torch.randn(300, k, generator=g) * x_scale, torch.randn(70, k, generator=g) * w_scale
@@ -54,6 +53,24 @@ def test_linear_f32_ranges(k, x_scale, w_scale):
     size = x.double().abs() @ w.double().abs().t()
     got = ops().linear_f32(x.to(DEV), w.to(DEV)).cpu().double()
     bound = size * (k * 2.0 ** -24 / (8 if k >= 64 else 2)) + 1e-42
+    assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("k,half", [(6, False), (31, False), (64, False), (256, False), (8, True), (64, True), (256, True)])
+@pytest.mark.parametrize("small", [1e-5, 1e-6, 1e-8, 1e-20, 1e-29, 1e-31, 1e-36])
+def test_linear_f32_rows_of_mixed_magnitude(k, half, small):
+    """Rows with one value of order 1 whose weights are small and the rest small, and the other way round: every value is
+    held in full, so each sum is off by at most k 2^-24 of the sum of its products' sizes, k roundings, whatever else the
+    row holds. A half holds 2^-24 and up: its smallest values are of 1e-5."""
+    g = torch.Generator().manual_seed(k)
+    x, w = torch.randn(300, k, generator=g) * (max(small, 1e-5) if half else small), torch.randn(70, k, generator=g)
+    x[:, 0], w[:, 0] = 1.0 + torch.rand(300, generator=g), w[:, 0] * small
+    x[100:, 1], w[35:, 2:] = torch.randn(200, generator=g), w[35:, 2:] * small
+    x = x.half() if half else x
+    want = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()
+    got = ops().linear_f32(x.to(DEV), w.to(DEV)).cpu().double()
+    bound = size * (k * 2.0 ** -24) + 1e-42
     assert ((got - want).abs() <= bound).all()
 
 
