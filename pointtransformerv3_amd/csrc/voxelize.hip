@@ -206,16 +206,19 @@ __global__ __launch_bounds__(VX_THREADS) void vx_split_count_kernel(const float*
     for (int b = threadIdx.x; b < parts; b += VX_THREADS) w.tile_parts[(int64_t)blockIdx.x * parts + b] = cnt[b];
 }
 
-// Down the tiles: 16 parts per work-group, 64 threads of a part that take a 64th of the tiles each, up to 512 tiles (2M points)
-// in one trip to memory of eight loads a thread. Bound by that trip and the barrier's chain: 1.56M points in 3 scenes 5.4 us,
-// 7.2 with 64 parts and 16 threads of each, which went to memory three times down and three times back.
-constexpr int VX_SCAN_PARTS = 16, VX_SCAN_SEGS = 64, VX_SCAN_AT_ONCE = 8;
-static_assert(VX_SCAN_PARTS <= 1 << VX_MIN_PART_BITS, "whole work-groups");
-__global__ __launch_bounds__(VX_SCAN_PARTS * VX_SCAN_SEGS) void vx_split_scan_kernel(VoxWs w) {
-    __shared__ uint32_t sum[VX_SCAN_SEGS][VX_SCAN_PARTS];
-    const int parts = 1 << w.part_bits, mine = threadIdx.x % VX_SCAN_PARTS, seg = threadIdx.x / VX_SCAN_PARTS;
-    const int64_t per = (w.tiles + VX_SCAN_SEGS - 1) / VX_SCAN_SEGS, t0 = min(w.tiles, seg * per), t1 = min(w.tiles, t0 + per);
-    uint32_t* __restrict__ col = w.tile_parts + blockIdx.x * VX_SCAN_PARTS + mine;
+// Down the tiles: SEGS threads of a part that take a share of the tiles each, eight tiles in one trip to memory. Bound by that
+// trip and by the chain of adding up the shares. Up to 128 tiles (524k points) 16 shares of 64 parts a work-group do it in one
+// trip: more shares make the chain longer and the runs that a wave reads shorter. Beyond, 64 shares of 16 parts do. 16 | 64
+// shares, us: 10k points 2.1 | 3.3, 50k 3.2 | 3.4, 150k 3.4 | 4.7, 400k 3.7 | 5.2, 530k 5.1 | 4.8, 1.5M 6.5 | 5.4, 3M 11.0 | 9.8.
+constexpr int VX_SCAN_THREADS = 1024, VX_SCAN_AT_ONCE = 8;
+template <int SEGS>
+__global__ __launch_bounds__(VX_SCAN_THREADS) void vx_split_scan_kernel(VoxWs w) {
+    constexpr int PARTS = VX_SCAN_THREADS / SEGS;
+    static_assert(PARTS <= 1 << VX_MIN_PART_BITS, "whole work-groups");
+    __shared__ uint32_t sum[SEGS][PARTS];
+    const int parts = 1 << w.part_bits, mine = threadIdx.x % PARTS, seg = threadIdx.x / PARTS;
+    const int64_t per = (w.tiles + SEGS - 1) / SEGS, t0 = min(w.tiles, seg * per), t1 = min(w.tiles, t0 + per);
+    uint32_t* __restrict__ col = w.tile_parts + blockIdx.x * PARTS + mine;
     uint32_t v[VX_SCAN_AT_ONCE], total = 0;
     for (int64_t t = t0; t < t1; t += VX_SCAN_AT_ONCE) {
 #pragma unroll
@@ -227,12 +230,12 @@ __global__ __launch_bounds__(VX_SCAN_PARTS * VX_SCAN_SEGS) void vx_split_scan_ke
     __syncthreads();
     uint32_t run = 0, all = 0;
 #pragma unroll
-    for (int s = 0; s < VX_SCAN_SEGS; ++s) {
+    for (int s = 0; s < SEGS; ++s) {
         const uint32_t c = sum[s][mine];
         if (s < seg) run += c;
         all += c;
     }
-    if (seg == 0) w.part_size[blockIdx.x * VX_SCAN_PARTS + mine] = all;
+    if (seg == 0) w.part_size[blockIdx.x * PARTS + mine] = all;
     for (int64_t t = t0; t < t1; t += VX_SCAN_AT_ONCE) {
         if (per > VX_SCAN_AT_ONCE)   // else the loads above still stand in v
 #pragma unroll
@@ -582,7 +585,10 @@ extern "C" int ptv3_voxelize(const float* coord, int64_t n, const int64_t* offse
     hipLaunchKernelGGL(vx_init_kernel, dim3((unsigned)ptv3_ceil_div(3 * (int64_t)n_scenes, 256)), dim3(256), 0, stream, w, n_scenes, offset_out);
     hipLaunchKernelGGL(vx_scene_min_kernel, tiles, threads, 0, stream, coord, n, offset, n_scenes, w);
     hipLaunchKernelGGL(vx_split_count_kernel, tiles, threads, parts * 4, stream, coord, n, offset, n_scenes, grid_size, w);
-    hipLaunchKernelGGL(vx_split_scan_kernel, dim3((unsigned)(parts / VX_SCAN_PARTS)), dim3(VX_SCAN_PARTS * VX_SCAN_SEGS), 0, stream, w);
+    if (w.tiles <= 16 * VX_SCAN_AT_ONCE)
+        hipLaunchKernelGGL(vx_split_scan_kernel<16>, dim3((unsigned)(parts * 16 / VX_SCAN_THREADS)), dim3(VX_SCAN_THREADS), 0, stream, w);
+    else
+        hipLaunchKernelGGL(vx_split_scan_kernel<64>, dim3((unsigned)(parts * 64 / VX_SCAN_THREADS)), dim3(VX_SCAN_THREADS), 0, stream, w);
     hipLaunchKernelGGL(vx_split_kernel, tiles, threads, split_lds, stream, coord, n, offset, n_scenes, grid_size, w);
     hipLaunchKernelGGL(vx_part_kernel, dim3((unsigned)parts), threads, 0, stream, w, pick_seed);
     hipLaunchKernelGGL(vx_count_kernel, tiles, threads, 0, stream, n, w);

@@ -28,9 +28,9 @@ def test_voxelize_edges(sizes, grid, extent):
         assert np.array_equal(got[name].cpu().numpy(), want), name
 
 
-@pytest.mark.parametrize("n", [64 * 4096, 64 * 4096 + 1, 512 * 4096, 512 * 4096 + 1])
+@pytest.mark.parametrize("n", [16 * 4096, 16 * 4096 + 1, 64 * 4096, 64 * 4096 + 1, 128 * 4096, 128 * 4096 + 1, 512 * 4096, 512 * 4096 + 1])
 def test_voxelize_where_the_scan_down_the_tiles_takes_another_turn(n):
-    """A thread of the scan has one tile | two, eight in one trip | nine in two."""
+    """A thread of the scan has one tile | two of 16 shares; eight of 16 | three of 64 shares; eight of 64 in one trip | nine in two."""
     test_voxelize_edges([n - 5000, 5000], 0.05, 2.0)
 
 
