@@ -558,17 +558,9 @@ int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_sr
     static LdsGrant grant_lds_allowed;   // per instantiation and device; raised monotonically
     if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_lds_allowed)) return rc_;
     const float scale_log2e = scale * 1.4426950408889634f;
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        cus = n;
-    }
     const int64_t total = n_seq * heads;
     int64_t full = 0;
-    const int split = ptv3_patch_attn_cut(total, slots, n_seq, max_seqlen, cus, &full);
+    const int split = ptv3_patch_attn_cut(total, slots, n_seq, max_seqlen, ptv3_cus(), &full);
     const int64_t tail = (total - full + 7) / 8 * 8;   // the tail's items in groups of 8, one per XCD
     hipLaunchKernelGGL(kern, dim3((unsigned)(full + tail * split)), dim3(ATT_THREADS), lds, stream,
                        (const T*)qkv, channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys,

@@ -1008,14 +1008,7 @@ int launch_half_bwd(const void* qkv, const void* out, const void* dout, int chan
     if (const int rc_ = ptv3_allow_lds((const void*)kkv, lds_kv, grant_kv[dropping])) return rc_;
     // one work-group per CU is resident (LDS): the items beyond the last full round are cut into ranges of
     // tiles when that shortens the round (each range stages the sequence again, about 0.15 of an item)
-    static int slots = 0;
-    if (slots == 0) {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-        slots = cus;
-    }
+    const int slots = ptv3_cus();
     const int64_t total = n_seq * heads;
     const int64_t rem = total % slots;
     int64_t full = total - rem, split = 1;

@@ -1373,18 +1373,6 @@ __global__ __launch_bounds__(256) void segment_reduce_bwd_kernel(const T* __rest
     }
 }
 
-int outer_cu_count() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v < 1)
-            v = 256;
-        cus = v;
-    }
-    return cus;
-}
-
 // Rows of the reduction per work-group. Two work-groups fit a CU, and they all start together: the launch takes
 // as long as the CU with the most of them, so a count just above a multiple of 2 x CUs costs a whole round more
 // (measured: 516 work-groups 55 us, 444 of the same layer 45 us). The number of ranges minimises
@@ -1393,7 +1381,7 @@ int outer_cu_count() {
 // (tap, range) pairs (see outer_item). The gathering form keeps its pair list in LDS (cap rows per range) and
 // runs several rounds anyway: about 1024 work-groups of at least 1024 rows.
 void outer_split(int64_t n, int64_t blocks, int taps, int64_t cap, int64_t* splits, int64_t* rows) {
-    const int64_t slots_per_xcd = 2 * outer_cu_count() / XCDS, fixed = 384;
+    const int64_t slots_per_xcd = 2 * ptv3_cus() / XCDS, fixed = 384;
     int64_t best = ptv3_ceil_div(1024, blocks * taps);
     if (best > ptv3_ceil_div(n, 1024)) best = ptv3_ceil_div(n, 1024);
     if (best < 1) best = 1;
@@ -1415,13 +1403,13 @@ void outer_split(int64_t n, int64_t blocks, int taps, int64_t cap, int64_t* spli
 }
 
 // Rows per range of the gathering 128 x 128 form. Over all taps there are about ten pairs per voxel at the levels that have
-// these widths: about 300 work-groups, between the slabs that shorter ranges write (384 rows: 54 against 39 us at 36k x 128,
+// these widths: about 300 work-groups on 256 CUs, between the slabs that shorter ranges write (384 rows: 54 against 39 us at 36k x 128,
 // 225 against 134 at 149k x 128, 59 against 39 at 9.2k x 256) and too few work-groups (1280 rows: 27 against 20 us at 5k x 128).
 // While a work-group's rows are few beside its blocks and taps, one range and no slabs (600 x 256: 15 us against 19 in two,
 // 1100 x 512: 24 against 40 in three).
 int64_t outer_gather_rows(int64_t n, int64_t blocks, int taps) {
     if (n <= OW_LIST && n <= 6 * blocks * taps) return ptv3_ceil_div(n, 128) * 128;
-    const int64_t r = ptv3_ceil_div(n * blocks, 30 * 128) * 128;
+    const int64_t r = ptv3_ceil_div(n * blocks, max(30 * ptv3_cus() / 256, 1) * 128) * 128;
     return r < 384 ? 384 : r > 1280 ? 1280 : r;
 }
 

@@ -67,6 +67,18 @@ static inline int ptv3_allow_lds(const void* kern, size_t lds, LdsGrant& grant) 
     return 0;
 }
 
+// CUs of the current device: what rules that fill the part go by. 256, the whole MI355X, where there is none to ask (a size
+// asked for before a device is there, on the host alone).
+static inline int ptv3_cus() {
+    static std::atomic<int> known[PTV3_MAX_DEVICES];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+    if (dev < PTV3_MAX_DEVICES && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 256;
+    if (dev < PTV3_MAX_DEVICES) known[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
 // ptv3_patch_attn_fwd where the number of slots, cu_seqlens[n_seq], is known: what ptv3_patch_attn_cut goes by.
 int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
                               const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,

@@ -346,18 +346,21 @@ __global__ __launch_bounds__(CG_THREADS, 2) void conv_gather_kernel(
 
 // The time of a launch at 128 channels whose fullest CU gets k work-groups of `groups` x 32 outputs and holds `at_once` of them,
 // in tenths of a us: once + each k + round ceil(k / at_once). Fitted to 2.5k - 220k voxels of 8 - 10 pairs: 38 us for one
-// work-group of 128 outputs a CU, 51 for two, 77 for three (measured 38, 53, 77); 32 outputs 20 us, 64 26, 96 31.
+// work-group of 128 outputs a CU, 51 for two, 77 for three (measured 38, 53, 77); 32 outputs 20 us, 64 26, 96 31. A level of
+// more or fewer pairs is slower or faster whatever the groups: at 5, 16 and 24 pairs a voxel from 3k to 400k voxels the row
+// that comes out cheapest was the fastest of the four each time, at 9 pairs but once (3 %). A constant below zero is the
+// fit's: the least a row comes to is 180. Larger levels take 128 outputs, the least per output.
 struct GatherCost { int groups, once, each, round, at_once; };
 constexpr GatherCost GATHER_COST[4] = {{1, 100, 80, 0, 1}, {2, -10, 70, 200, 3}, {3, 20, 90, 195, 2}, {4, 126, 129, 130, 2}};
 int64_t gather_cost(int64_t n, const GatherCost& c) {
-    const int64_t k = ptv3_ceil_div(ptv3_ceil_div(n, 32 * c.groups), 256);
+    const int64_t k = ptv3_ceil_div(ptv3_ceil_div(n, 32 * c.groups), (int64_t)ptv3_cus());
     return c.once + c.each * k + c.round * ptv3_ceil_div(k, (int64_t)c.at_once);
 }
 
 // groups per work-group on lists of tile_voxels outputs: the cheapest that divides the tile; 64 channels: two up to two work-groups
 // a CU (30k voxels: 15.7 us against 17.5 with four), four on larger levels (40k: 19.9 against 22.5, 150k: 47 against 53)
 int gather_groups(int64_t n, int c, int tile_voxels) {
-    if (c == 64) return n <= 2 * 256 * 64 ? 2 : 4;
+    if (c == 64) return n <= 2 * ptv3_cus() * 64 ? 2 : 4;
     const GatherCost* best = nullptr;
     for (const GatherCost& g : GATHER_COST)
         if (tile_voxels % (32 * g.groups) == 0 && (!best || gather_cost(n, g) < gather_cost(n, *best))) best = &g;

@@ -397,7 +397,7 @@ extern "C" int ptv3_conv_form(int64_t n, int64_t n_pairs, int channels) {
     if (n < 1 || n >= (1ll << 24)) return 0;
     if (ptv3_conv_few_pairs(n_pairs, channels)) return 0;
     const bool tiles = (channels == 64 || channels == 128) && n_pairs >= 4 * n;
-    if (tiles && channels == 64 && n <= 2 * 256 * 128) return 2;
+    if (tiles && channels == 64 && n <= 2 * ptv3_cus() * 128) return 2;
     if ((channels == 32 || channels == 64) && n_pairs <= 14 * n) return 1;
     return tiles ? 2 : 0;
 }

@@ -349,14 +349,15 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
     }
 }
 
-// Tile of a launch: rounds of work-groups over the 256 CUs times the products of a tile, smaller tiles a little dearer
+// Tile of a launch: rounds of work-groups over the CUs times the products of a tile, smaller tiles a little dearer
 // for the operands they re-read.
 template <typename XT, typename OT, bool VEC, bool PAIRS>
 int launch_f32(F32Args& g, int64_t rows, hipStream_t stream) {
     const int extra = PAIRS ? g.taps : 0;   // every tap may end with a partial tile
+    const int64_t cus = ptv3_cus();
     auto cost = [&](int tm, int tn, double weight) {
         const int64_t tiles = (rows / tm + (PAIRS ? extra : (rows % tm != 0))) * ptv3_ceil_div(g.nout, tn);
-        return (double)ptv3_ceil_div(tiles, 256) * tm * tn * weight;
+        return (double)ptv3_ceil_div(tiles, cus) * tm * tn * weight;
     };
 #define PTV3_TILE(TM, TN, WM, WN, KC)                                                                          \
     do {                                                                                                      \

@@ -454,10 +454,10 @@ int launch_linear_wide(const void* x, const void* w, const void* bias, int64_t n
     auto kern = linear_wide_kernel<T, GELU, LN>;
     static LdsGrant grant_allowed;   // per instantiation and device
     if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_allowed)) return rc_;
-    // one work-group per CU (its registers hold the weights): the 256 CUs are shared out over the tiles of
+    // one work-group per CU (its registers hold the weights): the CUs are shared out over the tiles of
     // output channels, and every work-group walks an equal span of rows in whole 64-row tiles
     const int col_tiles = nout / LW_N;
-    int64_t spans = 256 / col_tiles;
+    int64_t spans = ptv3_cus() / col_tiles;
     if (spans < 1) spans = 1;
     int64_t span_rows = ptv3_ceil_div(ptv3_ceil_div(n, spans), LW_ROWS) * LW_ROWS;
     spans = ptv3_ceil_div(n, span_rows);

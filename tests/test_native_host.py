@@ -424,3 +424,32 @@ def test_attention_cut_fills_every_xcd_alike(mean, cus):
                                              (232, 1024, (0, 2)), (312, 1024, (256, 4)), (4, 1024, (0, 8)), (512, 723, (512, 1))])
 def test_attention_cut_measured(items, mean, want):
     assert _attention_cut(items, mean * items, items) == want
+
+
+def test_rules_that_fill_the_part_ask_the_device_for_its_cus(tmp_path):
+    """On a quarter of the part (64 CUs, as one that is divided shows them) a rule decides as on the whole one for four times
+    the voxels. The device is a library that answers in the runtime's place; on the host the library's own answer is 256."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    from pointtransformerv3_amd import _lib
+    if shutil.which("gcc") is None:
+        pytest.skip("no C compiler")
+    src, so = tmp_path / "quarter.c", tmp_path / "quarter.so"
+    src.write_text("int hipGetDevice(int *d) { *d = 0; return 0; }\n"
+                   "int hipDeviceGetAttribute(int *v, int what, int dev) { *v = 64; return 0; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    voxels = list(range(384, 60_000, 384))
+    code = ("import ctypes, sys\n"
+            f"ctypes.CDLL({str(so)!r}, mode=ctypes.RTLD_GLOBAL)\n"
+            f"lib, i64 = ctypes.CDLL({_lib.LIB_PATH!r}), ctypes.c_int64\n"
+            f"v = {voxels}\n"
+            "print([lib.ptv3_conv_tile_voxels(i64(n), 128) for n in v], [lib.ptv3_conv_form(i64(n), i64(9 * n + 70_000), 64) for n in v])")
+    out = subprocess.run([sys.executable, "-c", code], check=True, capture_output=True, text=True, env=dict(os.environ)).stdout
+    lib = _lib.load()
+    tiles, form = [lib.ptv3_conv_tile_voxels(4 * n, 128) for n in voxels], [lib.ptv3_conv_form(4 * n, 4 * (9 * n + 70_000), 64) for n in voxels]
+    if not torch.cuda.is_available() or torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert {96, 128} == set(tiles) and {1, 2} == set(form)
+        assert out.split("\n")[0] == f"{tiles} {form}"
