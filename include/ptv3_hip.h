@@ -551,7 +551,7 @@ int ptv3_linear_gemm_fwd(const void *x, const void *w, const void *bias, const v
  * here: the MFMA kernels above take the shapes of the released models. */
 int ptv3_linear_any_fwd(const void *x, const void *w, const void *bias, const void *resid, int dtype, int64_t n,
                         int k, int nout, int gelu, void *out, void *stream);
-/* The fp32 layer, any k and nout, on the fp32 MFMA. x (n, k) is PTV3_F32, or PTV3_F16 rows that are converted on the
+/* The fp32 layer, any k and nout, on the matrix cores, every bit of the operands taken. x (n, k) is PTV3_F32, or PTV3_F16 rows that are converted on the
  * way in; out (n, nout) is PTV3_F32, or PTV3_F16 (one rounding): the projections on either side of an attention that
  * reads and writes halves in a float model. Half rows on either side: k a multiple of 4, x and w 16-byte aligned, not
  * both x and out (PTV3_ESHAPE). w, bias, resid are fp32. */

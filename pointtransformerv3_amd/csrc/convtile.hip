@@ -20,8 +20,8 @@
 // What bounds it: large levels the matrix cores - 70 % of the (tap, 32 outputs) of a level occur where 36 % of the pairs
 // do, and what is multiplied runs at 750 TFLOP/s of the 1090 a large product reaches; small ones a tile's chain of taps,
 // 20 us for 32 outputs to 38 for 128. Measured (fp16, MI355X), against gathering through registers into the row of the output
-// with two chunks in flight: 128 channels, 149k voxels of 9.8 pairs 167 -> 117 us, 371k 339 -> 257, 36k 54 -> 39; 64 channels,
-// 20k voxels of 5.3 pairs 18.9 (sparse tiles) -> 14.6. Tried: 64-channel slices with three in flight (125 us at 149k), waves of
+// with two chunks in flight, launches back to back: 128 channels, 149k voxels of 9.8 pairs 167 -> 117 us, 371k 339 -> 257, 36k
+// 54 -> 39; 64 channels, 20k voxels of 5.3 pairs 18.9 (sparse tiles) -> 14.6. In a traced forward 146k take 122 us. Tried: 64-channel slices with three in flight (125 us at 149k), waves of
 // 64 x 64 (137), 256 channels (93k voxels 274 - 300 us against 344 in pair form, 37k 131 - 153 against 122: half of the products
 // are of absent neighbours, and those of the pair form are not).
 #include <hip/hip_bf16.h>

@@ -382,8 +382,8 @@ bool net_ok(const ptv3_net* net, const ptv3_level* lv) {
 // sums what the tile forms keep on chip, rounded once: the error against 64 bits is theirs (2.08e-4 in fp16; half rows
 // 2.32e-4 at 1 - 4 us less). Measured in fp16, us, pair form with float rows / tile form / sparse tiles: 64 channels 11.7 /
 // 13.8 / 20.7 at 6k pairs, 13.6 / 14.3 / 24.3 at 18k, 19.6 / 14.0 / 23.8 at 67k; 128 channels 12.9 / 19.0 at 8k, 20.2 / 19.5 at
-// 36k, 25.2 / 20.4 at 92k, 40.5 / 26.6 at 167k. The lines are those of tiles that took 22 - 24 us (64) and 42 - 44 (128) and have
-// stayed where tests/test_gpu_small.py holds them; by these figures tiles would pay from 20k and 35k pairs on.
+// 36k, 25.2 / 20.4 at 92k, 40.5 / 26.6 at 167k. The lines are those of tiles that took 22 - 24 us (64) and 42 - 44 (128). By
+// these figures tiles would pay from 20k and 35k pairs on: not taken yet, tests/test_gpu_small.py holds the route up to the lines.
 extern "C" int ptv3_conv_few_pairs(int64_t n_pairs, int channels) {
     return (channels == 64 && n_pairs <= 70000) || (channels == 128 && n_pairs <= 185000);
 }

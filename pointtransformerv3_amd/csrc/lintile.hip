@@ -465,7 +465,8 @@ int lin_tiled(LinArgs& a, int dtype, hipStream_t stream) {
 // Whether the norm goes into the layer behind it. The launch it replaces costs 3 us and every column tile's own norm 2: with
 // 256 inputs while a CU has one tile (block tail of 250 rows 17.0 -> 15.7 us, of 350 no change; then the layer alone takes
 // few_kernel as well, and the sums are the same bits), with 64 up to a thousand tiles (1500 rows 13.8 -> 12.1, 4000 14.2 ->
-// 14.0). With 512 the norm of 32 rows takes as long as the launch (300 rows 23.2 -> 26.1).
+// 14.0; beyond FEW_TILES the layer alone takes linear_tile_kernel, which adds the inputs in one chain where few_kernel adds two
+// halves: the same float sums in another order, rounded at the same places). With 512 the norm of 32 rows takes as long as the launch (300 rows 23.2 -> 26.1).
 bool lin_front_pays(int64_t n, int k, int nout) {
     const int64_t tiles = ptv3_ceil_div(n, 32) * (nout / 32);
     return k == 64 ? tiles <= 1024 : k == 256 && tiles <= FEW_TILES;
