@@ -853,6 +853,7 @@ typedef struct ptv3_train_net {
     int32_t n_zero, reserved;
     int64_t zero_blocks;
     ptv3_train_stage stage[PTV3_MAX_LEVELS];
+    void *side;                               /* stream for the weight gradients of the backward (same device, any but its own); null: none */
 } ptv3_train_net;
 
 int ptv3_zero_ranges(float *base, const ptv3_zero_range *ranges, int count, int64_t blocks, void *stream);

@@ -56,6 +56,12 @@ struct StageActs {
     void *up_sum;               // unpooled rows: skip projection + child (half)
 };
 constexpr int MAX_BLOCKS = 256;
+// A group of weight gradients: what it holds before it is launched, and its lists. Every group is two events each way and
+// launches of its own, so small blocks share one: a step of 2 x 15k voxels has 12 groups at 64 MB and 31 at one a block, and
+// queueing its backward takes the host 1.3 ms and 2.3 ms. On the GPU the step takes 8.06 and 8.13 ms (8.38 without a second
+// stream), one of 4 x 100k 38.6 and 38.5 ms (39.6), whose blocks are all larger; 160 MB: 8.11, 38.6.
+constexpr size_t GROUP_BYTES = 64u << 20;
+constexpr int GROUP_LINEARS = 64, GROUP_CONVS = 16;
 
 struct Run {
     const ptv3_train_net& net;
@@ -305,68 +311,148 @@ struct Run {
 
     // ---- backward
     float* grads = nullptr;
-    SlabJob jobs[SLAB_JOBS];
-    int n_jobs = 0;
-    LinearGrad linears[8];
-    int n_linears = 0;
 
-    // the weight gradients of the Linear layers put off so far (of one number of rows), then all slab sums
-    int flush(Space& scratch) {
-        TRY(linear_wgrads(scratch));
-        const int n = n_jobs;
-        n_jobs = 0;
-        return n && !dry ? ptv3_slab_sums(jobs, n, hs) : PTV3_OK;
+    // Weight gradients are no part of the chain from dout to the first layer: nothing waits for them but the end of the
+    // call. They are put down while a block's chain is queued and launched together behind it (flush), on net.side if the
+    // caller gave one, beside the chain of the next blocks. What they read and their slabs lie in one of two arenas in
+    // turn; a group of blocks begins with a wait for the group before last, and ends when it holds GROUP_BYTES.
+    hipStream_t side = nullptr;
+    hipEvent_t ready = nullptr, done[2] = {};
+    bool busy[2] = {}, closed = true;
+    int turn = 0;
+    Space arenas[2] = {Space(nullptr), Space(nullptr)};
+    LinearGrad linears[GROUP_LINEARS];
+    int n_linears = 0;
+    struct ConvGrad {
+        const void *x, *dy;
+        const int32_t *pair_out, *tap_ptr, *pair_in;
+        int64_t n;
+        int cin, cout, taps;
+        float *dweight, *dbias;
+    } convs[GROUP_CONVS];
+    int n_convs = 0;
+
+    int open_side() {
+        if (!net.side || (hipStream_t)net.side == hs) return PTV3_OK;
+        hipError_t e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
+        for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
+        side = e == hipSuccess ? (hipStream_t)net.side : nullptr;
+        return (int)e;
     }
-    int linear_wgrads(Space& scratch) {
-        const int n = n_linears;
-        n_linears = 0;
-        if (!n) return PTV3_OK;
-        const size_t bytes = ptv3_linear_wgrads_bytes(linears, n);
-        void* ws = bytes ? scratch.take(bytes) : nullptr;
-        DO(ptv3_linear_wgrads_slabs(linears, n, dt, ws, bytes, jobs + n_jobs, hs));
-        n_jobs += n;
+    // `stream` goes on behind everything queued on the side
+    int join() {
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < 2; ++i) {
+            if (!busy[i]) continue;
+            busy[i] = false;
+            const hipError_t w = hipStreamWaitEvent(hs, done[i], 0);
+            e = e == hipSuccess ? w : e;
+        }
+        return (int)e;
+    }
+    int close_side() {   // also where a launch has failed: the caller's buffers are free again behind this call's work
+        const int rc = join();
+        for (int i = 0; i < 2; ++i)
+            if (done[i]) (void)hipEventDestroy(done[i]);
+        if (ready) (void)hipEventDestroy(ready);
+        return rc;
+    }
+    // the arena for what the weight gradients of the next block read
+    int enter(Space** arena) {
+        if (closed) {
+            closed = false;
+            turn ^= 1;
+            arenas[turn].at = 0;
+            if (busy[turn]) {
+                busy[turn] = false;
+                TRY((int)hipStreamWaitEvent(hs, done[turn], 0));
+            }
+        }
+        *arena = &arenas[turn];
         return PTV3_OK;
     }
-    // x and dy stay until flush, and so do a job's slabs in `scratch`
-    int wgrad(const ptv3_train_linear& l, int in, int out, const void* x, const void* dy, int64_t n, Space& scratch) {
-        if (n_linears && (n_linears == 8 || linears[0].n != n)) TRY(linear_wgrads(scratch));
-        if (n_jobs + n_linears >= SLAB_JOBS) TRY(flush(scratch));
+    int leave() {   // a block's chain has written what they read
+        const bool full = arenas[turn].at >= GROUP_BYTES || n_linears + 8 > GROUP_LINEARS || n_convs == GROUP_CONVS;
+        return full ? flush() : PTV3_OK;
+    }
+    // the weight gradients put down since the last flush
+    int flush() {
+        closed = true;
+        if (!n_linears && !n_convs) return PTV3_OK;
+        const bool beside = side && !dry;
+        if (beside) {
+            TRY((int)hipEventRecord(ready, hs));
+            TRY((int)hipStreamWaitEvent(side, ready, 0));
+        }
+        int rc = launch_wgrads(arenas[turn], beside ? side : hs);
+        n_linears = n_convs = 0;
+        if (beside) {
+            const int rec = (int)hipEventRecord(done[turn], side);
+            busy[turn] = rec == PTV3_OK;
+            rc = rc ? rc : rec;
+        }
+        return rc;
+    }
+    int launch_wgrads(Space& arena, hipStream_t on) {
+        SlabJob jobs[GROUP_LINEARS + GROUP_CONVS];
+        int n_jobs = 0;
+        for (int first = 0, last; first < n_linears; first = last) {   // up to eight in a row with as many rows share a launch
+            for (last = first + 1; last < n_linears && last < first + 8 && linears[last].n == linears[first].n;) ++last;
+            const size_t bytes = ptv3_linear_wgrads_bytes(linears + first, last - first);
+            void* ws = bytes ? arena.take(bytes) : nullptr;
+            DO(ptv3_linear_wgrads_slabs(linears + first, last - first, dt, ws, bytes, jobs + n_jobs, on));
+            n_jobs += last - first;
+        }
+        for (int i = 0; i < n_convs; ++i) {
+            const ConvGrad& g = convs[i];
+            const size_t bytes = ptv3_subm_conv_wgrad_workspace_bytes(dt, g.n, g.cin, g.cout, g.taps);
+            void* ws = bytes ? arena.take(bytes) : nullptr;
+            DO(ptv3_subm_conv_wgrad_slabs(g.x, g.dy, dt, g.n, g.cin, g.cout, g.pair_out, g.tap_ptr, g.pair_in, g.taps, g.dweight,
+                                           g.dbias, ws, bytes, &jobs[n_jobs], on));
+            ++n_jobs;
+        }
+        DO(ptv3_slab_sums(jobs, n_jobs, on));
+        return PTV3_OK;
+    }
+    // x and dy stay until the arena's next turn
+    int wgrad(const ptv3_train_linear& l, int in, int out, const void* x, const void* dy, int64_t n) {
+        if (n_linears == GROUP_LINEARS) return PTV3_EINVAL;
         linears[n_linears++] = LinearGrad{x, dy, n, in, out, grads + l.gw, grads + l.gb};
         return PTV3_OK;
     }
-    int conv_wgrad(const ptv3_train_block& b, const ptv3_level& v, const void* x, const void* dy, Space& scratch) {
-        const int c = b.channels;
-        const size_t bytes = ptv3_subm_conv_wgrad_workspace_bytes(dt, v.n, c, c, 27);
-        void* ws = bytes ? scratch.take(bytes) : nullptr;
-        DO(ptv3_subm_conv_wgrad_slabs(x, dy, dt, v.n, c, c, v.pair_out, v.tap_ptr, v.pair_in, 27, grads + b.g_conv_w,
-                                       grads + b.g_conv_b, ws, bytes, &jobs[n_jobs], hs));
-        return ++n_jobs + n_linears >= SLAB_JOBS ? flush(scratch) : PTV3_OK;
+    int conv_wgrad(const ptv3_train_block& b, const ptv3_level& v, const void* x, const void* dy) {
+        if (n_convs == GROUP_CONVS) return PTV3_EINVAL;
+        convs[n_convs++] = ConvGrad{x, dy, v.pair_out, v.tap_ptr, v.pair_in, v.n, b.channels, b.channels, 27, grads + b.g_conv_w,
+                                    grads + b.g_conv_b};
+        return PTV3_OK;
     }
     int bn_bwd(const ptv3_train_bn& b, const BnActs& a, int64_t n, int c, const void* dy, void* dx) {
         if (dry) return PTV3_OK;
         return ptv3_batch_norm_bwd(a.x, dt, dy, dt, a.stats, b.g, b.b, PTV3_F32, n, c, 1, 1, dx, dt, grads + b.gg, stream);
     }
 
-    // d32, d16: gradient of the block's output in float and, times mask2, in half. Leaves the gradients of its residual
-    // input in dskip (skip_out_dt) and of its convolution's rows in dxs (half); the weights' in `grads`.
+    // d32, d16: gradient of the block's output in float and, times mask2, in half (in the group's arena). Leaves the
+    // gradients of its residual input in dskip (skip_out_dt) and of its convolution's rows in dxs (half); the weights' in
+    // `grads`.
     int block_bwd(const ptv3_train_block& b, const BlockActs& a, const ptv3_level& v, int patch, const void* mask1, const void* d32,
-                  const void* d16, void* dskip, int skip_out_dt, void* dxs, Space& scratch) {
+                  const void* d16, void* dskip, int skip_out_dt, void* dxs, Space& scratch, Space& arena) {
         const int64_t n = v.n;
         const int c = b.channels;
         const size_t mark = scratch.at, half = (size_t)n * c * 2;
-        void *h4 = scratch.take(4 * half), *h3 = scratch.take(3 * half), *h1 = scratch.take(half), *hb = scratch.take(half);
-        void* dsum2 = scratch.take(2 * half);
+        void *h4 = arena.take(4 * half), *h3 = arena.take(3 * half), *hb = arena.take(half), *dcpe = arena.take(half);
+        void* dconv = arena.take(half);
+        void *h1 = scratch.take(half), *dsum2 = scratch.take(2 * half);
         // MLP
         DO(ptv3_linear_gelu_bwd(d16, b.fc2.wt, a.pre, dt, n, c, 4 * c, h4, stream));
-        TRY(wgrad(b.fc2, 4 * c, c, a.act, d16, n, scratch));
-        TRY(wgrad(b.fc1, c, 4 * c, a.y2, h4, n, scratch));
+        TRY(wgrad(b.fc2, 4 * c, c, a.act, d16, n));
+        TRY(wgrad(b.fc1, c, 4 * c, a.y2, h4, n));
         TRY(linear(h4, b.fc1.wt, nullptr, 4 * c, c, n, h1));
         // second LayerNorm and residual
         DO(ptv3_add_layer_norm_bwd(a.sum2, PTV3_F32, h1, dt, d32, PTV3_F32, mask1, dt, b.ln2.g, PTV3_F32, n, c, b.ln2.eps, dsum2,
                                     PTV3_F32, hb, dt, grads + b.ln2.gg, grads + b.ln2.gb, nullptr, 0, nullptr, 0.f, nullptr, nullptr,
                                     stream));
         // projection and attention
-        TRY(wgrad(b.proj, c, c, a.attn, hb, n, scratch));
+        TRY(wgrad(b.proj, c, c, a.attn, hb, n));
         TRY(linear(hb, b.proj.wt, nullptr, c, c, n, h1));
         {
             const size_t m2 = scratch.at, bytes = ptv3_patch_attn_bwd_workspace_bytes(dt, v.n_pad, c, b.heads);
@@ -375,18 +461,17 @@ struct Run {
                                     v.n_pad, b.scale, a.lse, 0.f, 0, h3, ws, bytes, stream));
             scratch.at = m2;
         }
-        TRY(wgrad(b.qkv, c, 3 * c, a.y1, h3, n, scratch));
+        TRY(wgrad(b.qkv, c, 3 * c, a.y1, h3, n));
         TRY(linear(h3, b.qkv.wt, nullptr, 3 * c, c, n, h1));
         // first LayerNorm, residual and the xCPE's norm
-        void* dcpe = scratch.take(half);
         DO(ptv3_add_layer_norm_bwd(a.sum1, PTV3_F32, h1, dt, dsum2, PTV3_F32, nullptr, 0, b.ln1.g, PTV3_F32, n, c, b.ln1.eps, dskip,
                                     skip_out_dt, dcpe, dt, grads + b.ln1.gg, grads + b.ln1.gb, a.cpe, dt, b.ln_cpe.g, b.ln_cpe.eps,
                                     grads + b.ln_cpe.gg, grads + b.ln_cpe.gb, stream));
-        TRY(wgrad(b.cpe, c, c, a.conv, dcpe, n, scratch));
-        TRY(linear(dcpe, b.cpe.wt, nullptr, c, c, n, h1));
-        TRY(conv_wgrad(b, v, a.xs, h1, scratch));
-        TRY(conv(b, v, true, h1, scratch, dxs));
-        TRY(flush(scratch));
+        TRY(wgrad(b.cpe, c, c, a.conv, dcpe, n));
+        TRY(linear(dcpe, b.cpe.wt, nullptr, c, c, n, dconv));
+        TRY(conv_wgrad(b, v, a.xs, dconv));
+        TRY(leave());
+        TRY(conv(b, v, true, dconv, scratch, dxs));
         scratch.at = mark;
         return PTV3_OK;
     }
@@ -398,10 +483,14 @@ struct Run {
         const ptv3_level& v = lv[level];
         const int c = bs[0].channels;
         const size_t mark = scratch.at;
-        void *d32 = scratch.take((size_t)v.n * c * 4), *d16 = scratch.take((size_t)v.n * c * 2), *ds = scratch.take((size_t)v.n * c * 4);
+        void *d32 = scratch.take((size_t)v.n * c * 4), *ds = scratch.take((size_t)v.n * c * 4);
         for (int i = count - 1; i >= 0; --i) {
+            Space* arena;
+            TRY(enter(&arena));
+            void* d16 = arena->take((size_t)v.n * c * 2);
             DO(ptv3_two_sums(a, a_dt, b, b_dt, nullptr, masks[2 * i + 1], dt, v.n, c, d32, d16, dt, hs));
-            TRY(block_bwd(bs[i], as[i], v, net.patch[level], masks[2 * i], d32, d16, i ? ds : dskip, i ? PTV3_F32 : dt, dxs, scratch));
+            TRY(block_bwd(bs[i], as[i], v, net.patch[level], masks[2 * i], d32, d16, i ? ds : dskip, i ? PTV3_F32 : dt, dxs, scratch,
+                          *arena));
             a = ds;
             a_dt = PTV3_F32;
             b = dxs;
@@ -435,23 +524,26 @@ struct Run {
             const ptv3_level &v = lv[s], &below = lv[s + 1];
             const int c = g.dec_channels;
             const size_t mark = scratch.at, half = (size_t)v.n * c * 2;
-            void *dskip = scratch.take(half), *dxs = scratch.take(half), *dpar = scratch.take(half), *dlin = scratch.take(half);
-            void *dchild = scratch.take((size_t)below.n * c * 2), *dlin2 = scratch.take((size_t)below.n * c * 2);
+            void *dskip = scratch.take(half), *dxs = scratch.take(half), *dpar = scratch.take(half);
+            void* dchild = scratch.take((size_t)below.n * c * 2);
             TRY(stage_bwd(g.dec, st[s].dec, g.n_dec, s, dec_masks[s], nullptr, dt, d, d_dt, dskip, dxs, scratch));
+            Space* arena;
+            TRY(enter(&arena));
+            void *dlin = arena->take(half), *dlin2 = arena->take((size_t)below.n * c * 2);
             // unpooling: the sum's gradient goes to the skip projection (whose rows the first convolution reads too) and,
             // summed over a cell's members, to the child
             DO(ptv3_two_sums(dskip, dt, dxs, dt, nullptr, nullptr, dt, v.n, c, nullptr, dpar, dt, hs));
             DO(ptv3_segment_reduce(dskip, dt, v.n, c, v.order, below.idx_ptr, below.n, 2, dchild, stream));
             TRY(bn_bwd(g.up_skip_bn, st[s].skip_bn, v.n, c, dpar, dlin));
-            TRY(wgrad(g.up_skip, g.up_skip.in, c, st[s].enc[g.n_enc - 1].out16, dlin, v.n, scratch));
+            TRY(wgrad(g.up_skip, g.up_skip.in, c, st[s].enc[g.n_enc - 1].out16, dlin, v.n));
             TRY(linear(dlin, g.up_skip.wt, nullptr, c, g.up_skip.in, v.n, from_skip[s]));
             TRY(bn_bwd(g.up_bn, st[s].up_bn, below.n, c, dchild, dlin2));
             const void* child_rows = s + 1 < S - 1 ? st[s + 1].dec[net.stage[s + 1].n_dec - 1].out16
                                                    : st[S - 1].enc[net.stage[S - 1].n_enc - 1].out16;
-            TRY(wgrad(g.up, g.up.in, c, child_rows, dlin2, below.n, scratch));
+            TRY(wgrad(g.up, g.up.in, c, child_rows, dlin2, below.n));
             void* dnext = s + 1 < S - 1 ? from_up[s + 1] : from_skip[S - 1];
+            TRY(leave());
             TRY(linear(dlin2, g.up.wt, nullptr, c, g.up.in, below.n, dnext));
-            TRY(flush(scratch));
             scratch.at = mark;
             d = dnext;
             d_dt = dt;
@@ -462,28 +554,29 @@ struct Run {
             const ptv3_level& v = lv[s];
             const int c = g.channels;
             const size_t mark = scratch.at, half = (size_t)v.n * c * 2;
-            void *dskip = scratch.take(half), *dxs = scratch.take(half), *dx = scratch.take(half), *dseg = scratch.take(half);
+            void *dskip = scratch.take(half), *dxs = scratch.take(half), *dx = scratch.take(half);
             TRY(stage_bwd(g.enc, st[s].enc, g.n_enc, s, enc_masks[s], s < S - 1 ? from_pool[s] : nullptr, dt, from_skip[s], dt, dskip,
                           dxs, scratch));
             DO(ptv3_two_sums(dskip, dt, dxs, dt, nullptr, nullptr, dt, v.n, c, nullptr, dx, dt, hs));
+            Space* arena;
+            TRY(enter(&arena));
+            void* dseg = arena->take(half);
             if (s > 0) {
                 const ptv3_level& up = lv[s - 1];
-                void* dproj = scratch.take((size_t)up.n * c * 2);
+                void* dproj = arena->take((size_t)up.n * c * 2);
                 TRY(bn_bwd(g.pool_bn, st[s].pool_bn, v.n, c, dx, dseg));
                 DO(ptv3_segment_reduce_bwd(st[s].pool_in, st[s].pooled, dseg, dt, up.n, c, up.order, v.idx_ptr, v.n, g.pool_reduce,
                                             dproj, stream));
-                TRY(wgrad(g.pool, g.pool.in, c, st[s - 1].enc[net.stage[s - 1].n_enc - 1].out16, dproj, up.n, scratch));
+                TRY(wgrad(g.pool, g.pool.in, c, st[s - 1].enc[net.stage[s - 1].n_enc - 1].out16, dproj, up.n));
+                TRY(leave());
                 TRY(linear(dproj, g.pool.wt, nullptr, c, g.pool.in, up.n, from_pool[s - 1]));
-                TRY(flush(scratch));
             } else {
                 TRY(bn_bwd(net.stem.bn, stem_bn, v.n, c, dx, dseg));
                 const int cp = net.stem.cin_padded;
-                const size_t bytes = ptv3_subm_conv_wgrad_workspace_bytes(dt, v.n, cp, c, 125);
-                void* ws = bytes ? scratch.take(bytes) : nullptr;
-                float* dw = (float*)scratch.take((size_t)c * 125 * cp * 4);
-                DO(ptv3_subm_conv_wgrad_slabs(stem_in, dseg, dt, v.n, cp, c, v.pair_out5, v.tap_ptr5, v.pair_in5, 125, dw, nullptr,
-                                               ws, bytes, &jobs[n_jobs++], hs));
-                TRY(flush(scratch));
+                float* dw = (float*)arena->take((size_t)c * 125 * cp * 4);
+                convs[n_convs++] = ConvGrad{stem_in, dseg, v.pair_out5, v.tap_ptr5, v.pair_in5, v.n, cp, c, 125, dw, nullptr};
+                TRY(flush());
+                TRY(join());
                 DO(ptv3_cut_rows(dw, (int64_t)c * 125, cp, net.stem.cin, grads + net.stem.gw, stream));
             }
             scratch.at = mark;
@@ -526,8 +619,8 @@ bool net_ok(const ptv3_train_net* net, const ptv3_level* lv) {
     return blocks <= MAX_BLOCKS;
 }
 
-// scratch of a pass, from a run of its own code that queues nothing
-size_t scratch_bytes(const ptv3_train_net& net, const ptv3_level* lv, bool back) {
+// scratch of a pass, from a run of its own code that queues nothing; `parts` (backward): what the chain and each arena take
+size_t scratch_bytes(const ptv3_train_net& net, const ptv3_level* lv, bool back, size_t* parts = nullptr) {
     Run* r = new Run(net, lv, nullptr);
     Space acts(nullptr), m(nullptr);
     r->place(acts);
@@ -535,8 +628,10 @@ size_t scratch_bytes(const ptv3_train_net& net, const ptv3_level* lv, bool back)
     r->dry = true;
     static const void* none[2 * MAX_BLOCKS] = {};
     const int rc = back ? r->backward(nullptr, PTV3_F32, none, m) : r->forward(nullptr, PTV3_F32, none, m);
+    const size_t sizes[3] = {m.top, r->arenas[0].top, r->arenas[1].top};
     delete r;
-    return rc == PTV3_OK ? m.top + 256 : 0;
+    if (parts) memcpy(parts, sizes, sizeof(sizes));
+    return rc == PTV3_OK ? sizes[0] + sizes[1] + sizes[2] + 256 : 0;
 }
 
 }  // namespace
@@ -589,13 +684,18 @@ extern "C" int ptv3_train_bwd(const ptv3_train_net* net, const ptv3_level* level
                               const void* const* masks, const void* acts, void* scratch, size_t scratch_size, float* grads,
                               void* stream) {
     if (!net_ok(net, levels) || !dout || !masks || !acts || !scratch || !grads) return PTV3_EINVAL;
-    if (scratch_size < scratch_bytes(*net, levels, true)) return PTV3_EWORKSPACE;
+    size_t parts[3];
+    if (scratch_size < scratch_bytes(*net, levels, true, parts)) return PTV3_EWORKSPACE;
     Run* r = new Run(*net, levels, stream);
     Space a(const_cast<void*>(acts)), s(scratch);
     r->place(a);
     r->link();
     r->grads = grads;
-    const int rc = r->backward(dout, dout_dtype, masks, s);
+    r->arenas[0] = Space((char*)scratch + parts[0]);
+    r->arenas[1] = Space((char*)scratch + parts[0] + parts[1]);
+    int rc = r->open_side();
+    if (rc == PTV3_OK) rc = r->backward(dout, dout_dtype, masks, s);
+    const int joined = r->close_side();
     delete r;
-    return rc;
+    return rc ? rc : joined;
 }

@@ -257,3 +257,32 @@ def test_native_training_step_on_a_second_stream(monkeypatch):
     rel = lambda x, y: float((x.double() - y.double()).norm() / y.double().norm())
     # batch statistics are summed by atomics: single roundings to half differ
     assert rel(point.feat.detach(), first) < 2e-2 and rel(got, want) < 2e-2
+
+
+@pytest.mark.parametrize("sizes", [(300,), (2000, 900), (30_000, 12_000)])
+@pytest.mark.parametrize("caller", ["default stream", "another stream"])
+def test_weight_gradients_beside_the_backward_are_those_of_one_stream(sizes, caller, monkeypatch):
+    """From one group of weight gradients to several that take turns in the two arenas, twice over one forward's activations.
+    The chain's sums by atomics differ in single roundings to half from run to run: the tolerance is that of this path
+    against the modules; an operand overwritten too early would be wrong by its own size."""
+    from pointtransformerv3_amd import PointTransformerV3, native_train
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).to(DEV).train()
+    data = _inputs(4, sizes, torch.float32)
+    on = torch.cuda.Stream() if caller == "another stream" else torch.cuda.current_stream()
+    on.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(on):
+        _step(model, data, torch.float16, True, monkeypatch)
+        engine = native_train._ENGINES[model][torch.float16]
+        assert engine.net.side and engine.net.side != on.cuda_stream
+        with torch.autocast("cuda", dtype=torch.float16):
+            feat = model(dict(data)).feat
+        got = []
+        for side in (engine.side.cuda_stream, None, on.cuda_stream, engine.side.cuda_stream):
+            engine.net.side = side
+            model.zero_grad(set_to_none=True)
+            feat.backward(torch.full_like(feat, 0.01), retain_graph=True)
+            got.append(torch.cat([p.grad.reshape(-1) for p in model.parameters()]).double())
+    torch.cuda.synchronize()
+    for g in got:
+        assert torch.isfinite(g).all() and float((g - got[1]).norm() / got[1].norm()) < 2e-2
