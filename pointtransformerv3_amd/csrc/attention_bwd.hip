@@ -15,8 +15,11 @@
 //      enter through the MFMAs' C operands), dS and dQ^T += K^T dS^T. lse and D go to a workspace.
 //   2. keys: Q, dO (rows), Q^T, dO^T (transposed), -lse and -D in LDS; per 32-key tile
 //      dV^T += dO^T P and dK^T += Q^T dS over all queries.
-// Where the forward kept the log-sum-exps and the sequences are long, one kernel does both (attn_bwd_both_kernel).
+// Where the forward kept the log-sum-exps and sequences are no longer than 1024 slots, one kernel does both
+// (attn_bwd_both_kernel); with attention dropout, only where it is the faster one.
 // fp32: one thread per query / per key, operands staged through LDS in chunks.
+#include <algorithm>
+
 #include "attn_half.h"
 
 namespace {
@@ -25,8 +28,9 @@ constexpr int BWD_THREADS = 512;    // keys kernel: 8 waves, two key tiles each 
 constexpr int BWD_WAVES = BWD_THREADS / PTV3_WAVE;
 constexpr int BWQ_THREADS = 1024;   // queries kernel: 16 waves, four per SIMD
 constexpr int BWQ_WAVES = BWQ_THREADS / PTV3_WAVE;
-constexpr int BOTH_KEYS = 1024;     // both-sides kernel: the keys that its waves hold in registers
+constexpr int BOTH_KEYS = 1024;     // both-sides kernel: the longest sequence, its queries in LDS
 constexpr int BOTH_WAVES = 8;
+constexpr int BOTH_PARTS = 4;       // at most as many work-groups share an item
 constexpr float LN2 = 0.6931471805599453f;
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -458,6 +462,15 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
     }
 }
 
+// How the work-groups of the both-sides kernel share the items from `first` on: `parts` work-groups an item, each with its
+// range of the keys. With more than one a part leaves its share of dQ (float) in row slot - cu[first / heads] of its own
+// `stride` rows, and attn_bwd_finish_kernel adds them up.
+struct BothParts {
+    float* dq;
+    int64_t stride;
+    int first, parts;
+};
+
 // ---- both sides in one kernel: one work-group per (sequence, head), scores computed once
 //
 // A wave owns KG groups of 16 keys; their K and V, and the sums of their dK and dV, stay in its registers while the
@@ -475,29 +488,44 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
 // measured with two waves a SIMD; the two kernels above take 890 together, the exponentials twice. Eight waves of 128 keys
 // and not 16 of 64: the query side of a step and the dQ sums pass LDS half as often, and the registers for a group ahead
 // are there (16 waves spill). bf16, 1024 slots: 1400 items 630 -> 489 us, 788 items 374 -> 298 us, 384 items 188 -> 154 us.
-template <typename T, int WAVES, bool DROP>
-__global__ __launch_bounds__(WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
+// With few items several work-groups share one, each with a range of its keys (KG 4 or 2) and all of its queries; a step's
+// query side passes LDS as often (96 KB a step for the eight waves, 0.4 us), so half the keys take 0.7 of the time.
+template <typename T, int KG, int QUERIES, bool DROP>
+__global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     const T* __restrict__ qkv, const T* __restrict__ out, const T* __restrict__ dout, int channels, int heads,
     const int32_t* __restrict__ slot_src, const int32_t* __restrict__ slot_dst, const int32_t* __restrict__ cu_seqlens,
-    float scale, int64_t n_pad, const float* __restrict__ lse, T* __restrict__ dqkv, T* __restrict__ fill, Dropout drop) {
-    constexpr int KG = BOTH_KEYS / 16 / WAVES;     // 16-key groups per wave
-    constexpr int T_STRIDE = BOTH_KEYS * 2 + VT_PAD_BYTES;
+    float scale, int64_t n_pad, const float* __restrict__ lse, T* __restrict__ dqkv, T* __restrict__ fill, Dropout drop, BothParts by) {
+    constexpr int WAVES = BOTH_WAVES;
+    constexpr int KEYS = KG * 16 * WAVES;          // keys of a work-group
+    constexpr int T_STRIDE = QUERIES * 2 + VT_PAD_BYTES;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* q_lds = smem;                                  // Q * scale * log2(e), rows
-    unsigned char* do_lds = q_lds + BOTH_KEYS * 32;               // dO rows
-    unsigned char* qt_lds = do_lds + BOTH_KEYS * 32;              // the same two, transposed
+    unsigned char* do_lds = q_lds + QUERIES * 32;                 // dO rows
+    unsigned char* qt_lds = do_lds + QUERIES * 32;                // the same two, transposed
     unsigned char* dot_lds = qt_lds + HD * T_STRIDE;
     float* nlse_lds = (float*)(dot_lds + HD * T_STRIDE);          // -lse (log2 units), -D per query slot
-    float* nd_lds = nlse_lds + BOTH_KEYS;
-    int32_t* dst_lds = (int32_t*)(nd_lds + BOTH_KEYS);            // the row that a query slot writes
-    float* dq_lds = (float*)(dst_lds + BOTH_KEYS);                // WAVES blocks of two 16-query tiles in lane order
+    float* nd_lds = nlse_lds + QUERIES;
+    int32_t* dst_lds = (int32_t*)(nd_lds + QUERIES);              // the row that a query slot writes
+    float* dq_lds = (float*)(dst_lds + QUERIES);                  // WAVES blocks of two 16-query tiles in lane order
 
-    const int item = xcd_chunked_id(blockIdx.x, gridDim.x);
+    // the parts of an item, like the heads of a sequence, are neighbours in an XCD: they read the same rows
+    const int wg = xcd_chunked_id(blockIdx.x, gridDim.x);
+    const int item = by.first + wg / by.parts, part = wg % by.parts;
     const int seq = item / heads, head = item % heads;
     const int s0 = cu_seqlens[seq];
-    const int len = min(cu_seqlens[seq + 1] - s0, BOTH_KEYS);
+    const int len = min(cu_seqlens[seq + 1] - s0, QUERIES);
     if (len <= 0) return;
     const int tid = threadIdx.x, wave = tid / PTV3_WAVE, lane = tid % PTV3_WAVE;
+    // where parts share an item, this one's dQ of query i: [i * channels]
+    float* dq_part = nullptr;
+    if (by.parts > 1) {
+        dq_part = by.dq + ((int64_t)part * by.stride + s0 - cu_seqlens[by.first / heads]) * channels + head * HD;
+        if (part * KEYS >= len) {   // a short sequence: no keys are left for it
+            for (int e = tid; e < len * 4; e += WAVES * PTV3_WAVE)
+                *(f32x4*)(dq_part + (int64_t)(e >> 2) * channels + (e & 3) * 4) = (f32x4){0.f, 0.f, 0.f, 0.f};
+            return;
+        }
+    }
     const int col = lane & 15, grp = lane >> 4;
     const int64_t row_stride = 3 * (int64_t)channels;
     const float scale_log2e = scale * LOG2E;
@@ -514,9 +542,9 @@ __global__ __launch_bounds__(WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     // Everything that the work-group reads, in two rounds of loads. A thread stages eight channels of four queries; a
     // query that does not exist, or a filler slot, gets lse = +inf: its probabilities come out as zero. A wave's keys:
     // lane = key, four channels; a key that does not exist repeats the last one, so that its scores stay in range.
-    constexpr int THREADS = WAVES * PTV3_WAVE, QP = BOTH_KEYS * 2 / THREADS;
+    constexpr int THREADS = WAVES * PTV3_WAVE, QP = QUERIES * 2 / THREADS;
     const int half8 = tid & 1;
-    const int key0 = wave * KG * 16;
+    const int key0 = part * KEYS + wave * KG * 16;
     const bool mine = key0 < len;                        // the same for the whole wave
     u32x2 kf[KG], vf[KG];
     u32x4 kt[KG / 2];
@@ -673,7 +701,7 @@ __global__ __launch_bounds__(WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
                 }
             }
             if (s + 1 < WAVES) fetch(b0 + ((blk + 1) & (WAVES - 1)));
-            else fetch(min(b0 + WAVES + wave, BOTH_KEYS / 32 - 1));
+            else fetch(min(b0 + WAVES + wave, QUERIES / 32 - 1));
             __syncthreads();   // the sums that step s - 1 left are complete, and nobody touches them any more
             if (there) {
 #pragma unroll
@@ -682,6 +710,9 @@ __global__ __launch_bounds__(WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
                     if (s > 0) dq[t] += *sum;
                     if (s < WAVES - 1) {
                         *sum = dq[t];
+                    } else if (by.parts > 1) {
+                        const int q = (b0 + blk) * 32 + t * 16 + col;
+                        if (q < len) *(f32x4*)(dq_part + (int64_t)q * channels + 4 * grp) = dq[t];
                     } else {
                         const int dst = dst_lds[(b0 + blk) * 32 + t * 16 + col];
                         if (dst >= 0)
@@ -950,16 +981,36 @@ __global__ __launch_bounds__(F32_B) void attn_bwd_kv_f32_kernel(
 }
 
 // Filler slots: their dK and dV, parked per slot, are added to the row the slot repeats. A row is
-// repeated by at most one filler slot, so plain read-modify-write is race-free.
+// repeated by at most one filler slot, so plain read-modify-write is race-free. Real slots whose items were shared by
+// several work-groups (by.parts > 1): their dQ, the parts' shares added up in order.
 template <typename T>
-__global__ __launch_bounds__(256) void attn_bwd_fill_kernel(const T* __restrict__ fill, int channels,
-                                                            const int32_t* __restrict__ slot_src,
-                                                            const int32_t* __restrict__ slot_dst, int64_t n_pad,
-                                                            PieceDiv per, T* __restrict__ dqkv) {   // per: pieces of 8 channels a slot
+__global__ __launch_bounds__(256) void attn_bwd_finish_kernel(const T* __restrict__ fill, int channels, int heads,
+                                                              const int32_t* __restrict__ slot_src,
+                                                              const int32_t* __restrict__ slot_dst,
+                                                              const int32_t* __restrict__ cu_seqlens, int64_t n_pad, float scale,
+                                                              PieceDiv per, T* __restrict__ dqkv, BothParts by) {   // per: pieces of 8 channels a slot
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = ptv3_row_of(i, per);
     if (slot >= n_pad) return;
     const int piece = (int)(i - slot * per.count);
-    if (slot_dst[slot] >= 0) return;
+    const int to = slot_dst[slot];
+    if (to >= 0) {
+        if constexpr (sizeof(T) == 2) {
+            if (by.parts < 2 || piece >= channels / 8) return;
+            const int seq = by.first / heads, s0 = cu_seqlens[seq];   // of the first shared item
+            if (slot < s0 || (piece * 8 / HD < by.first % heads && slot < cu_seqlens[seq + 1])) return;
+            const float* src = by.dq + (slot - s0) * channels + piece * 8;
+            f32x4 a = *(const f32x4*)src, b = *(const f32x4*)(src + 4);
+            for (int p = 1; p < by.parts; ++p) {
+                src += by.stride * channels;
+                a += *(const f32x4*)src;
+                b += *(const f32x4*)(src + 4);
+            }
+            *(u32x4*)(dqkv + (int64_t)to * 3 * channels + piece * 8) =
+                (u32x4){Half<T>::pack2(a[0] * scale, a[1] * scale), Half<T>::pack2(a[2] * scale, a[3] * scale),
+                        Half<T>::pack2(b[0] * scale, b[1] * scale), Half<T>::pack2(b[2] * scale, b[3] * scale)};
+        }
+        return;
+    }
     const T* src = fill + slot * 2 * channels + piece * 8;
     T* dst = dqkv + (int64_t)slot_src[slot] * 3 * channels + channels + piece * 8;
 #pragma unroll
@@ -970,6 +1021,8 @@ struct BwdWs {
     float* lse;
     float* d;
     void* fill;
+    float* dq;       // shares of dQ, where work-groups share an item
+    size_t dq_bytes;
     size_t bytes;
 };
 
@@ -983,71 +1036,122 @@ BwdWs carve(void* base, int dtype, int64_t n_pad, int channels, int heads) {
     off += ptv3_align256((size_t)n_pad * heads * sizeof(float));
     w.fill = (char*)base + off;
     off += ptv3_align256((size_t)n_pad * 2 * channels * elt);
+    // a shared item's parts are at most one round of work-groups; the first one's sequence may have heads that are not shared
+    w.dq = (float*)((char*)base + off);
+    const size_t round = ((size_t)ptv3_cus() + (size_t)BOTH_PARTS * heads) * BOTH_KEYS * HD, all = (size_t)BOTH_PARTS * n_pad * channels;
+    w.dq_bytes = dtype == PTV3_F32 ? 0 : (round < all ? round : all) * sizeof(float);
+    off += ptv3_align256(w.dq_bytes);
     w.bytes = off;
     return w;
 }
 
+template <int QUERIES> constexpr size_t both_lds() {
+    return 2 * QUERIES * 32 + 2 * HD * (QUERIES * 2 + VT_PAD_BYTES) + 3 * QUERIES * sizeof(float) + BOTH_WAVES * 32 * HD * sizeof(float);
+}
+static_assert(both_lds<BOTH_KEYS>() <= 160 * 1024, "one work-group fills a CU's LDS");
+
+struct HalfBwd {
+    const void *qkv, *out, *dout;
+    int channels, heads;
+    const int32_t *slot_src, *slot_dst, *cu_seqlens;
+    int64_t n_seq, max_seqlen, n_pad;
+    float scale;
+    void* dqkv;
+    float* lse;
+    Dropout drop;
+    hipStream_t stream;
+};
+
+template <typename T, int KG, int QUERIES, bool DROP>
+int launch_both(const HalfBwd& g, const BwdWs& ws, int64_t items, const BothParts& by) {
+    auto kern = attn_bwd_both_kernel<T, KG, QUERIES, DROP>;
+    static LdsGrant grant;
+    if (const int rc_ = ptv3_allow_lds((const void*)kern, both_lds<QUERIES>(), grant)) return rc_;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(items * by.parts)), dim3(BOTH_WAVES * PTV3_WAVE), both_lds<QUERIES>(), g.stream,
+                       (const T*)g.qkv, (const T*)g.out, (const T*)g.dout, g.channels, g.heads, g.slot_src, g.slot_dst, g.cu_seqlens,
+                       g.scale, g.n_pad, g.lse, (T*)g.dqkv, (T*)ws.fill, g.drop, by);
+    PTV3_RETURN_LAUNCH();
+}
+
 template <typename T>
-int launch_half_bwd(const void* qkv, const void* out, const void* dout, int channels, int heads,
-                    const int32_t* slot_src, const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
-                    int64_t max_seqlen, int64_t n_pad, float scale, void* dqkv, const BwdWs& ws, float* lse, Dropout drop,
-                    hipStream_t stream) {
-    const int lds_keys = (int)((max_seqlen + 63) & ~63ll);
+int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
+    const int lds_keys = (int)((g.max_seqlen + 63) & ~63ll);
     const size_t t_bytes = (size_t)HD * (lds_keys * 2 + VT_PAD_BYTES);
     const size_t lds_q = 2 * (size_t)lds_keys * 32 + t_bytes + 96;
     const size_t lds_kv = 2 * (size_t)lds_keys * 32 + 2 * t_bytes + 2 * (size_t)lds_keys * sizeof(float) + 96;
     if (lds_q > 160 * 1024 || lds_kv > 160 * 1024) return PTV3_ESHAPE;
-    const bool dropping = drop.threshold != 0u;
-    auto kq = dropping ? (lse ? attn_bwd_q_kernel<T, true, true> : attn_bwd_q_kernel<T, false, true>)
-                       : (lse ? attn_bwd_q_kernel<T, true, false> : attn_bwd_q_kernel<T, false, false>);
-    float* lse_buf = lse ? lse : ws.lse;
-    auto kkv = dropping ? attn_bwd_kv_kernel<T, true> : attn_bwd_kv_kernel<T, false>;
-    static LdsGrant grant_q[4], grant_kv[2];   // per kernel variant and device
-    const int qi_ = (lse != nullptr) + 2 * dropping;
-    if (const int rc_ = ptv3_allow_lds((const void*)kq, lds_q, grant_q[qi_])) return rc_;
-    if (const int rc_ = ptv3_allow_lds((const void*)kkv, lds_kv, grant_kv[dropping])) return rc_;
-    // one work-group per CU is resident (LDS): the items beyond the last full round are cut into ranges of
-    // tiles when that shortens the round (each range stages the sequence again, about 0.15 of an item)
+    const bool dropping = g.drop.threshold != 0u;
+    // one work-group per CU is resident (LDS)
     const int slots = ptv3_cus();
-    const int64_t total = n_seq * heads;
-    const int64_t rem = total % slots;
-    int64_t full = total - rem, split = 1;
-    double best = 1.0;
-    if (rem != 0)
-        for (int64_t sp = 2; sp <= 4; ++sp) {
-            const double cost = (double)((rem * sp + slots - 1) / slots) * (1.0 / (double)sp + 0.15);
-            if (cost < best - 1e-9) { best = cost; split = sp; }
+    const int64_t total = g.n_seq * g.heads, rem = total % slots;
+    BothParts shared = {ws.dq, 0, (int)total, 1};
+    if (g.lse && !dropping && g.max_seqlen <= BOTH_KEYS) {
+        // The both-sides kernel forms the scores once and takes sequences of up to 256, 512 and 1024 slots with 32, 64 and
+        // 128 keys a wave. Items that do not fill a round of CUs are shared by two or four work-groups, as many as the round has
+        // room for: more would start a second round. us, two kernels -> shared: 60 items of 1024 slots 55.4 -> 46.6 (by four;
+        // by two 55.0, whole 75.3), 92 76.8 -> 56.7, 120 84.9 -> 59.0, 64 48.6 -> 44.9, 792 (three rounds and 24) 298 -> 295
+        // (whole 325); 128 of 500 35.6 -> 27.1; 400 of 200 44.9 -> 19.2; 64 of 320 17.4 -> 19.0, but with a launch less
+        const int most = g.max_seqlen <= BOTH_KEYS / 4 ? 1 : g.max_seqlen <= BOTH_KEYS / 2 ? 2 : BOTH_PARTS;
+        int parts = 1;
+        while (parts < most && rem * parts * 2 <= slots) parts *= 2;
+        const int64_t first = parts == 1 ? total : total - rem;
+        const BothParts whole = {nullptr, 0, 0, 1};
+        int rc = PTV3_OK;
+        if (first > 0)
+            rc = most == 1 ? launch_both<T, 2, BOTH_KEYS / 4, false>(g, ws, first, whole)
+                 : most == 2 ? launch_both<T, 4, BOTH_KEYS / 2, false>(g, ws, first, whole)
+                             : launch_both<T, 8, BOTH_KEYS, false>(g, ws, first, whole);
+        if (rc != PTV3_OK) return rc;
+        if (first < total) {
+            // slots of the sequences from the first shared item's on
+            shared = {ws.dq, std::min(g.n_pad, (g.n_seq - first / g.heads) * g.max_seqlen), (int)first, parts};
+            if ((size_t)shared.stride * parts * g.channels * sizeof(float) > ws.dq_bytes) return PTV3_EWORKSPACE;
+            rc = most == 2 ? launch_both<T, 2, BOTH_KEYS / 2, false>(g, ws, total - first, shared)
+                 : parts == 2 ? launch_both<T, 4, BOTH_KEYS, false>(g, ws, total - first, shared)
+                              : launch_both<T, 2, BOTH_KEYS, false>(g, ws, total - first, shared);
+            if (rc != PTV3_OK) return rc;
         }
-    // The both-sides kernel holds BOTH_KEYS keys and needs the forward's log-sum-exps. It does an item in 0.78 of the time
-    // of the two kernels (84 against 107 us for 240 items of 1024 slots), so a last round that their ranges bring below 0.7
-    // is left to them, as are sequences that would leave half of its waves without keys (1600 items of 200 slots: 109
-    // against 104 us; 800 of 700 slots: 199 against 214 us).
-    int64_t first = 0;
-    if (lse && max_seqlen <= BOTH_KEYS && max_seqlen > BOTH_KEYS / 2) first = rem == 0 || best > 0.7 ? total : full;
-    if (split == 1 || first == total) full = total;
-    if (first > 0) {
-        constexpr size_t lds_both = 2 * BOTH_KEYS * 32 + 2 * HD * (BOTH_KEYS * 2 + VT_PAD_BYTES) + 3 * BOTH_KEYS * sizeof(float) +
-                                    BOTH_WAVES * 32 * HD * sizeof(float);
-        static_assert(lds_both <= 160 * 1024, "one work-group fills a CU's LDS");
-        auto kb = dropping ? attn_bwd_both_kernel<T, BOTH_WAVES, true> : attn_bwd_both_kernel<T, BOTH_WAVES, false>;
-        static LdsGrant grant_both[2];
-        if (const int rc_ = ptv3_allow_lds((const void*)kb, lds_both, grant_both[dropping])) return rc_;
-        hipLaunchKernelGGL(kb, dim3((unsigned)first), dim3(BOTH_WAVES * PTV3_WAVE), lds_both, stream, (const T*)qkv, (const T*)out,
-                           (const T*)dout, channels, heads, slot_src, slot_dst, cu_seqlens, scale, n_pad, lse, (T*)dqkv,
-                           (T*)ws.fill, drop);
+    } else {
+        // the items beyond the last full round are cut into ranges of
+        // tiles when that shortens the round (each range stages the sequence again, about 0.15 of an item)
+        int64_t full = total - rem, split = 1;
+        double best = 1.0;
+        if (rem != 0)
+            for (int64_t sp = 2; sp <= 4; ++sp) {
+                const double cost = (double)((rem * sp + slots - 1) / slots) * (1.0 / (double)sp + 0.15);
+                if (cost < best - 1e-9) { best = cost; split = sp; }
+            }
+        // With dropout the both-sides kernel takes whole items: 0.78 of the time of the two kernels (84 against 107 us for 240
+        // items of 1024 slots), so a last round that their ranges bring below 0.7 is left to them, as are sequences that would
+        // leave half of its waves without keys (1600 items of 200 slots: 109 against 104 us; 800 of 700 slots: 199 against 214).
+        int64_t first = 0;
+        if (g.lse && g.max_seqlen <= BOTH_KEYS && g.max_seqlen > BOTH_KEYS / 2) first = rem == 0 || best > 0.7 ? total : full;
+        if (split == 1 || first == total) full = total;
+        if (first > 0) {
+            const int rc = launch_both<T, 8, BOTH_KEYS, true>(g, ws, first, BothParts{nullptr, 0, 0, 1});
+            if (rc != PTV3_OK) return rc;
+        }
+        auto kq = dropping ? (g.lse ? attn_bwd_q_kernel<T, true, true> : attn_bwd_q_kernel<T, false, true>)
+                           : (g.lse ? attn_bwd_q_kernel<T, true, false> : attn_bwd_q_kernel<T, false, false>);
+        float* lse_buf = g.lse ? g.lse : ws.lse;
+        auto kkv = dropping ? attn_bwd_kv_kernel<T, true> : attn_bwd_kv_kernel<T, false>;
+        static LdsGrant grant_q[4], grant_kv[2];   // per kernel variant and device
+        if (const int rc_ = ptv3_allow_lds((const void*)kq, lds_q, grant_q[(g.lse != nullptr) + 2 * dropping])) return rc_;
+        if (const int rc_ = ptv3_allow_lds((const void*)kkv, lds_kv, grant_kv[dropping])) return rc_;
+        if (first < total) {
+            const unsigned grid = (unsigned)(full - first + (total - full) * split);
+            hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, g.stream, (const T*)g.qkv, (const T*)g.out, (const T*)g.dout,
+                               g.channels, g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, (T*)g.dqkv,
+                               lse_buf, ws.d, (int)first, (int)full, (int)split, g.drop);
+            hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, g.stream, (const T*)g.qkv, (const T*)g.dout, g.channels,
+                               g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, lse_buf, ws.d, (T*)g.dqkv,
+                               (T*)ws.fill, (int)first, (int)full, (int)split, g.drop);
+        }
     }
-    if (first < total) {
-        const unsigned grid = (unsigned)(full - first + (total - full) * split);
-        hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, stream, (const T*)qkv, (const T*)out, (const T*)dout,
-                           channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, (T*)dqkv, lse_buf, ws.d,
-                           (int)first, (int)full, (int)split, drop);
-        hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, stream, (const T*)qkv, (const T*)dout, channels,
-                           heads, slot_src, slot_dst, cu_seqlens, lds_keys, scale, n_pad, lse_buf, ws.d, (T*)dqkv,
-                           (T*)ws.fill, (int)first, (int)full, (int)split, drop);
-    }
-    const int64_t items = n_pad * (2 * channels / 8);
-    hipLaunchKernelGGL(attn_bwd_fill_kernel<T>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
-                       (const T*)ws.fill, channels, slot_src, slot_dst, n_pad, ptv3_piece_div(2 * channels / 8), (T*)dqkv);
+    const int64_t items = g.n_pad * (2 * g.channels / 8);
+    hipLaunchKernelGGL(attn_bwd_finish_kernel<T>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, g.stream,
+                       (const T*)ws.fill, g.channels, g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, g.n_pad, g.scale,
+                       ptv3_piece_div(2 * g.channels / 8), (T*)g.dqkv, shared);
     PTV3_RETURN_LAUNCH();
 }
 
@@ -1089,12 +1193,11 @@ extern "C" int ptv3_patch_attn_rpe_bwd(const void* qkv, const void* out, const v
     const BwdWs ws = carve(workspace, dtype, n_pad, channels, heads);
     if (workspace_bytes < ws.bytes) return PTV3_EWORKSPACE;
     hipStream_t stream = (hipStream_t)stream_;
-    if (dtype == PTV3_F16)
-        return launch_half_bwd<_Float16>(qkv, out, dout, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                         max_seqlen, n_pad, scale, dqkv, ws, (float*)lse, drop, stream);
-    if (dtype == PTV3_BF16)
-        return launch_half_bwd<__bf16>(qkv, out, dout, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                       max_seqlen, n_pad, scale, dqkv, ws, (float*)lse, drop, stream);
+    if (dtype != PTV3_F32) {
+        const HalfBwd g = {qkv, out, dout, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, n_pad, scale,
+                           dqkv, (float*)lse, drop, stream};
+        return dtype == PTV3_F16 ? launch_half_bwd<_Float16>(g, ws) : launch_half_bwd<__bf16>(g, ws);
+    }
     const int blocks = (int)ptv3_ceil_div(max_seqlen, F32_B);
     if (n_seq * heads * blocks >= (1ll << 31)) return PTV3_EINVAL;
     const unsigned grid = (unsigned)(n_seq * heads * blocks);
@@ -1105,7 +1208,8 @@ extern "C" int ptv3_patch_attn_rpe_bwd(const void* qkv, const void* out, const v
                        (const float*)dout, channels, heads, slot_src, slot_dst, cu_seqlens, blocks, scale, n_pad, ws.lse,
                        ws.d, (float*)dqkv, (float*)ws.fill, rpe, drop);
     const int64_t items = n_pad * (2 * channels / 8);
-    hipLaunchKernelGGL(attn_bwd_fill_kernel<float>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
-                       (const float*)ws.fill, channels, slot_src, slot_dst, n_pad, ptv3_piece_div(2 * channels / 8), (float*)dqkv);
+    hipLaunchKernelGGL(attn_bwd_finish_kernel<float>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, stream,
+                       (const float*)ws.fill, channels, heads, slot_src, slot_dst, cu_seqlens, n_pad, scale,
+                       ptv3_piece_div(2 * channels / 8), (float*)dqkv, BothParts{nullptr, 0, 0, 1});
     PTV3_RETURN_LAUNCH();
 }

@@ -191,6 +191,19 @@ def test_attention_backward_both_sides(dtype, lens, heads, drop_p):
             assert rel_err(got.cpu()[rows], p.grad.permute(2, 0, 1, 3).reshape(-1, 3 * C)) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,heads", [
+    ([1024] * 20, 3), ([1024, 513, 3, 1000, 257, 256], 4),        # shared by four, some parts without keys
+    ([1024] * 43, 2), ([600, 512, 1024, 1] * 8, 4),               # by two
+    ([1024] * 52, 5), ([1024] * 88, 3),                           # a whole round, the rest shared by four, by one
+    ([512, 300, 2, 511, 64], 7), ([500] * 33, 8), ([257] * 43, 3),   # up to 512 slots: shared, a round and the rest, one each
+    ([256, 1, 17, 255, 32, 33], 3), ([200] * 90, 5)])             # up to 256
+def test_attention_backward_items_shared_by_work_groups(dtype, lens, heads):
+    """Launches whose last items are shared by two or four work-groups, each with a range of the keys, and short sequences
+    in the instantiations that fit them: the same checks."""
+    test_attention_backward_both_sides(dtype, lens, heads, 0.0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("cin,cout,ks,n", [(6, 32, 5, 1500), (32, 32, 3, 2000), (64, 64, 3, 3000), (128, 128, 3, 1200),
                                            (48, 80, 3, 700)])
