@@ -328,7 +328,7 @@ __global__ __launch_bounds__(F32_THREADS, 2) void gemm_f32_kernel(F32Args g) {
             for (int v = 0; v < 16; ++v) y[v] += bias;
             if (!PAIRS && g.gelu) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = 0.5f * y[v] * (1.f + erff(y[v] * 0.70710678118654752f));
+                for (int v = 0; v < 16; ++v) y[v] = gelu_f32(y[v]);
             }
             if (!PAIRS && g.resid) {
                 f32x16 r;

@@ -73,6 +73,27 @@ __device__ __forceinline__ float gelu_erf(float x) {
     return fmaf(-a, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
 }
 
+// The same for results that stay float: degree 10 on q(a) = log2(erfc(a / sqrt 2)), its error weighted by what it does to
+// x Phi(x) (minimax on [0, 6], 2.7e-10 of |x|), then falling; without a constant term, so that small a lose nothing to rounding,
+// and with the last step one FMA: x - x t above zero, x t below. 17 instructions where 0.5 x (1 + erff(x / sqrt 2)) takes some
+// 45 and cancels in the negative tail. Error against 64 bits, normal inputs of deviation 3 / 1 / 0.3 / 0.01: 2.2e-8 /
+// 2.7e-8 / 3.1e-8 / 3.1e-8 (3.0e-8 / 3.9e-8 / 4.1e-8 / 3.7e-8 with erff). 11.6k x 256 -> 1024 with GELU 62.9 -> 55.7 us, 79k x
+// 64 -> 256 54.0 -> 44.7, a float forward of one room of 100k voxels 8.32 -> 8.15 ms. The clamp makes t exactly zero far out, so +inf stays itself and -inf and NaN give NaN, as they did.
+__device__ __forceinline__ float gelu_f32(float x) {
+    const float a = fminf(fabsf(x), 13.5f);
+    float q = fmaf(-5.150326032e-08f, a, 1.320617457e-06f);
+    q = fmaf(q, a, -1.480000356e-05f);
+    q = fmaf(q, a, 9.325502469e-05f);
+    q = fmaf(q, a, -3.217084159e-04f);
+    q = fmaf(q, a, 6.065531124e-05f);
+    q = fmaf(q, a, 6.898442749e-03f);
+    q = fmaf(q, a, -5.242196470e-02f);
+    q = fmaf(q, a, -4.592238367e-01f);
+    q = fmaf(q, a, -1.151104093e+00f);
+    const float t = 0.5f * __builtin_amdgcn_exp2f(q * a);
+    return fmaf(x > 0.f ? -a : x, t, fmaxf(x, 0.f));
+}
+
 // GELU of two first-layer sums as the separate layers would have stored them: rounded to the storage type, passed
 // through gelu_erf, rounded again and packed. For fp16 the rounded pair stays packed: the polynomial's FMAs read
 // its halves directly (v_fma_mix_f32 converts on the way in), max(x, 0) is one packed instruction for the pair, and

@@ -104,3 +104,18 @@ def test_subm_conv_pairs_f32(ks, cin, cout, n, extent):
     plan = o.conv_plan_direct(to_dev(idx), ks)
     got = o.subm_conv_pairs(feat.to(DEV), plan, w.to(DEV), None if b is None else b.to(DEV))
     assert rel_err(got, want) < 5e-6
+
+
+@pytest.mark.parametrize("n,scale", [(200_001, 3.0), (200_001, 0.3), (4096, 1e-3), (4096, 1e3)])
+def test_gelu_of_a_float_layer(n, scale):
+    """x Phi(x) of a layer that hands its input through, against 64 bits: the exponential is within two ulp and takes an
+    argument rounded once, the last step rounds once, so the result is off by 2^-23 of |x| at most."""
+    o = ops()
+    x = torch.randn(n, 1, generator=torch.Generator().manual_seed(1)) * scale
+    x[:8, 0] = torch.tensor([0.0, 13.4, -13.4, 13.6, -13.6, 1e30, -1e30, -1e-30])
+    got = o.linear_any(x.to(DEV), torch.ones(1, 1, device=DEV), None, gelu=True).cpu().double()
+    want = x.double() * 0.5 * torch.erfc(-x.double() / 2 ** 0.5)
+    assert ((got - want).abs() <= 2.0 ** -23 * x.double().abs()).all()
+    odd = torch.tensor([[float("inf")], [-float("inf")], [float("nan")]], device=DEV)
+    out = o.linear_any(odd, torch.ones(1, 1, device=DEV), None, gelu=True)
+    assert float(out[0]) == float("inf") and torch.isnan(out[1:]).all()
