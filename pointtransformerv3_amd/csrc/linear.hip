@@ -289,6 +289,9 @@ int dispatch_linear(const void* x, const void* w, const void* bias, const LinBn*
         if (bn) a.mean = bn->mean, a.var = bn->var, a.gamma = bn->gamma, a.beta = bn->beta, a.bn_eps = bn->eps, a.stats_f32 = bn->stats_f32;
         return lin_tiled(a, dtype, stream);
     }
+    // the register-weight kernel stores rows past the end again, so it takes no layer that works in place
+    if ((kind == ACT_GELU_KEEP || kind == ACT_GELU_GRAD) && out != aux && lin_wide_gelu_pays(n, k, nout))
+        return lin_wide_gelu(x, w, bias, dtype, n, nout, kind, out, aux, stream);
     const LinBn none = {nullptr, nullptr, nullptr, nullptr, 0.f, 0};
 #define PTV3_LIN(T, K)                                                                                                \
     if (k == K) {                                                                                                     \

@@ -29,7 +29,8 @@ constexpr int LW_WSTRIDE = LW_K + 8;
 constexpr int LW_OSTRIDE = 64 + 8;      // halfs per row of a wave's result staging
 
 // What follows the Linear when it is the cpe.1 or proj layer of a 256-channel block (LN = 3, 2; model.py:587-597),
-// as in ptv3_linear_ln_fwd: the residual, the LayerNorm(s) and the second output.
+// as in ptv3_linear_ln_fwd: the residual, the LayerNorm(s) and the second output. ACT_GELU_KEEP: out1 takes the sums in front
+// of the GELU; ACT_GELU_GRAD: res holds them, and the products are multiplied by its derivative there.
 template <typename T> struct LwNorm {
     const T *res, *gamma, *beta, *gamma2, *beta2, *shift;
     float eps;
@@ -48,7 +49,7 @@ template <typename T> struct LwLane {
 
 // acc -> out (and ln.out1) for the 64-row tile that starts at row tile_row0; resv: the residual rows of the wave's
 // 32 x 64 block (LN != 0). Contains work-group barriers when LN != 0: every wave calls it the same number of times.
-template <typename T, bool GELU, int LN>
+template <typename T, int ACT, int LN>
 __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv, const LwLane<T>& L, const LwNorm<T>& ln,
                                             T* out, int64_t tile_row0) {
     constexpr int NT = 2;
@@ -63,7 +64,13 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
             const int orow = it * 8 + (lane >> 3), opc = lane & 7;
-            const u32x4 val = *(const u32x4*)(stage + orow * LW_OSTRIDE + opc * 8);
+            u32x4 val = *(const u32x4*)(stage + orow * LW_OSTRIDE + opc * 8);
+            if constexpr (LN == 0 && ACT == ACT_GELU_GRAD) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    val[q] = H16<T>::pack2(H16<T>::lo(val[q]) * gelu_erf_grad(H16<T>::lo(resv[it][q])),
+                                           H16<T>::hi(val[q]) * gelu_erf_grad(H16<T>::hi(resv[it][q])));
+            }
             int64_t r = tile_row0 + row0 + orow;
             r = r < n ? r : n - 1;
             *(u32x4*)(dst + r * nout + cout0 + c0 + opc * 8) = val;
@@ -71,21 +78,31 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
         asm volatile("" ::: "memory");
     };
     if constexpr (LN == 0) {
+        u32x2 act[ACT == ACT_GELU_KEEP ? NT : 1][4];   // the activated values while the plain ones go out
 #pragma unroll
         for (int b = 0; b < NT; ++b)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const f32x4 bb = *(const f32x4*)(b_lds + c0 + b * 32 + 8 * q + 4 * hf);
-                float r[4];
+                float r[4], a[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     r[i] = acc[b][4 * q + i] + bb[i];
-                    if (GELU) r[i] = gelu_erf(H16<T>::round(r[i]));
+                    if (ACT == ACT_GELU) r[i] = gelu_erf(H16<T>::round(r[i]));
+                    if (ACT == ACT_GELU_KEEP) a[i] = gelu_erf(H16<T>::round(r[i]));
                 }
                 *(u32x2*)(stage + col * LW_OSTRIDE + b * 32 + 8 * q + 4 * hf) =
                     (u32x2){H16<T>::pack2(r[0], r[1]), H16<T>::pack2(r[2], r[3])};
+                if (ACT == ACT_GELU_KEEP) act[b][q] = (u32x2){H16<T>::pack2(a[0], a[1]), H16<T>::pack2(a[2], a[3])};
             }
-        store_rows(out);
+        store_rows(ACT == ACT_GELU_KEEP ? ln.out1 : out);
+        if constexpr (ACT == ACT_GELU_KEEP) {
+#pragma unroll
+            for (int b = 0; b < NT; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) *(u32x2*)(stage + col * LW_OSTRIDE + b * 32 + 8 * q + 4 * hf) = act[b][q];
+            store_rows(out);
+        }
     } else {
         // ---- the residual block through the staging rows into accumulator order
 #pragma unroll
@@ -185,7 +202,7 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
 // rows): modes 2 / 3 of the Linear + LayerNorm kernel on the accumulators, every intermediate rounded where the
 // separate kernels store it. A row's 256 channels are spread over the four waves of its row half: the sums of a
 // LayerNorm go through LDS (mean first, then the squared deviations), one barrier each.
-template <typename T, bool GELU, int LN>
+template <typename T, int ACT, int LN>
 __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_kernel(
     const T* __restrict__ x, const T* __restrict__ weight, const T* __restrict__ bias, int64_t n, int nout,
     T* __restrict__ out, int span_rows, LwNorm<T> ln) {
@@ -279,13 +296,14 @@ __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_kernel(
 
     for (int tile = 0; tile < n_tiles; ++tile) {
         const T* ptr_3 = row_ptr(tile + 3);
-        u32x4 resv[LN != 0 ? 4 : 1];   // the residual rows of this wave's 32 x 64 block, whole row segments
-        if (LN != 0) {
+        constexpr bool RES = LN != 0 || ACT == ACT_GELU_GRAD;
+        u32x4 resv[RES ? 4 : 1];   // the residual rows of this wave's 32 x 64 block, whole row segments
+        if (RES) {
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 int64_t r = r0 + (int64_t)tile * LW_ROWS + row0 + it * 8 + (lane >> 3);
                 r = r < n ? r : n - 1;
-                resv[it] = *(const u32x4*)(ln.res + r * LW_N + c0 + (lane & 7) * 8);
+                resv[it] = *(const u32x4*)(ln.res + r * nout + cout0 + c0 + (lane & 7) * 8);
             }
         }
         f32x16 acc[NT];
@@ -315,7 +333,7 @@ __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
         const LwLane<T> me = {stage, b_lds, p_lds, ex_lds, c0, row0, col, hf, lane, wave, cout0, nout, n};
-        lw_epilogue<T, GELU, LN>(acc, resv, me, ln, out, r0 + (int64_t)tile * LW_ROWS);
+        lw_epilogue<T, ACT, LN>(acc, resv, me, ln, out, r0 + (int64_t)tile * LW_ROWS);
         ptr_cur = ptr_nxt;
         ptr_nxt = ptr_nn;
         ptr_nn = ptr_3;
@@ -436,7 +454,7 @@ __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_resident_kernel(
 #pragma unroll
             for (int b = 0; b < NT; ++b) acc[b] = H16<T>::mfma(__builtin_bit_cast(v8, wreg[b][k]), xf, acc[b]);
         }
-        lw_epilogue<T, false, LN>(acc, resv, me, ln, out, r0 + (int64_t)tile * LW_ROWS);
+        lw_epilogue<T, ACT_NONE, LN>(acc, resv, me, ln, out, r0 + (int64_t)tile * LW_ROWS);
         if (LN != 0) {
 #pragma unroll
             for (int it = 0; it < 4; ++it) resv[it] = resn[it];
@@ -444,14 +462,14 @@ __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_resident_kernel(
     }
 }
 
-template <typename T, bool GELU, int LN = 0>
+template <typename T, int ACT, int LN = 0>
 int launch_linear_wide(const void* x, const void* w, const void* bias, int64_t n, int nout, void* out,
                        hipStream_t stream, LwNorm<T> ln = LwNorm<T>{}) {
     const size_t lds = ((size_t)LW_N * LW_WSTRIDE + 2 * (size_t)LW_ROWS * LW_XSTRIDE) * sizeof(T) + LW_N * sizeof(float);
     static_assert(8 * 32 * LW_OSTRIDE <= LW_N * LW_WSTRIDE, "the waves' staging rows fit where the weights were");
     static_assert((8 * 32 * LW_OSTRIDE) * 2 + (5 * LW_N + 4 * LW_ROWS * 4) * 4 <= LW_N * LW_WSTRIDE * 2,
                   "staging rows, LayerNorm parameters and partial sums fit where the weights were");
-    auto kern = linear_wide_kernel<T, GELU, LN>;
+    auto kern = linear_wide_kernel<T, ACT, LN>;
     static LdsGrant grant_allowed;   // per instantiation and device
     if (const int rc_ = ptv3_allow_lds((const void*)kern, lds, grant_allowed)) return rc_;
     // one work-group per CU (its registers hold the weights): the CUs are shared out over the tiles of
@@ -461,7 +479,7 @@ int launch_linear_wide(const void* x, const void* w, const void* bias, int64_t n
     if (spans < 1) spans = 1;
     int64_t span_rows = ptv3_ceil_div(ptv3_ceil_div(n, spans), LW_ROWS) * LW_ROWS;
     spans = ptv3_ceil_div(n, span_rows);
-    if constexpr (!GELU) {
+    if constexpr (ACT == ACT_NONE) {
         if (col_tiles == 1 && span_rows <= RS_ROWS) {   // the whole span stays in LDS
             static_assert((8 * 32 * LW_OSTRIDE) * 2 + (5 * LW_N + 4 * LW_ROWS * 4) * 4 + RS_ROWS * RS_XSTRIDE * 2 <=
                               (LW_N * LW_WSTRIDE + 2 * LW_ROWS * LW_XSTRIDE) * 2,
@@ -488,7 +506,7 @@ int linear_wide_ln_dispatch(const void* x, const void* w, const void* bias, cons
                             const void* beta, const void* gamma2, const void* beta2, const void* shift, int dtype,
                             int64_t n, int mode, float eps, void* out0, void* out1, hipStream_t stream) {
 #define PTV3_LWLN(T, M)                                                                                         \
-    return launch_linear_wide<T, false, M>(x, w, bias, n, LW_N, out0, stream,                                   \
+    return launch_linear_wide<T, ACT_NONE, M>(x, w, bias, n, LW_N, out0, stream,                                   \
                                            LwNorm<T>{(const T*)res, (const T*)gamma, (const T*)beta, (const T*)gamma2, \
                                                      (const T*)beta2, (const T*)shift, eps, (T*)out1})
     if (dtype == PTV3_F16) {
@@ -514,8 +532,26 @@ extern "C" int ptv3_linear_wide_fwd(const void* x, const void* w, const void* bi
         return lin_tiled(a, dtype, stream);
     }
     if (dtype == PTV3_F16)
-        return gelu ? launch_linear_wide<_Float16, true>(x, w, bias, n, nout, out, stream)
-                    : launch_linear_wide<_Float16, false>(x, w, bias, n, nout, out, stream);
-    return gelu ? launch_linear_wide<__bf16, true>(x, w, bias, n, nout, out, stream)
-                : launch_linear_wide<__bf16, false>(x, w, bias, n, nout, out, stream);
+        return gelu ? launch_linear_wide<_Float16, ACT_GELU>(x, w, bias, n, nout, out, stream)
+                    : launch_linear_wide<_Float16, ACT_NONE>(x, w, bias, n, nout, out, stream);
+    return gelu ? launch_linear_wide<__bf16, ACT_GELU>(x, w, bias, n, nout, out, stream)
+                : launch_linear_wide<__bf16, ACT_NONE>(x, w, bias, n, nout, out, stream);
+}
+
+// The GELU's training forms (ptv3_linear_gelu_fwd / _bwd) of a 256-input layer; `aux` as in LinArgs. linear_rows_kernel read
+// a fragment of the weights from LDS for every product. us, 256 -> 1024 in bf16, forward and backward form: 20k rows 28.3 ->
+// 27.0 and 34.1 -> 30.8, 37.7k 53.4 -> 49.2 and 66.6 -> 57.8 (in a training step of 4 x 100k voxels 88 -> 60 and 79 -> 74), 94k
+// 172 -> 125 and 155 -> 126; below 16M outputs the tiles of lintile.hip come first. The same bits.
+bool lin_wide_gelu_pays(int64_t n, int k, int nout) { return k == LW_K && nout % LW_N == 0 && n >= 4096; }
+int lin_wide_gelu(const void* x, const void* w, const void* bias, int dtype, int64_t n, int nout, int act, void* out, void* aux,
+                  hipStream_t stream) {
+#define PTV3_LWG(T)                                                                                                     \
+    if (act == ACT_GELU_KEEP)                                                                                           \
+        return launch_linear_wide<T, ACT_GELU_KEEP>(x, w, bias, n, nout, out, stream,                                   \
+                                                    LwNorm<T>{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, (T*)aux}); \
+    return launch_linear_wide<T, ACT_GELU_GRAD>(x, w, bias, n, nout, out, stream,                                       \
+                                                LwNorm<T>{(const T*)aux, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, nullptr})
+    if (dtype == PTV3_F16) { PTV3_LWG(_Float16); }
+    PTV3_LWG(__bf16);
+#undef PTV3_LWG
 }

@@ -22,6 +22,11 @@ bool lin_tiled_pays(int64_t n, int k, int nout, int act);
 bool lin_tiled_takes(int k, int nout);
 int lin_tiled(LinArgs& a, int dtype, hipStream_t stream);
 
+// the GELU's training forms of a 256-input layer on the register-weight kernel (linearw.hip)
+bool lin_wide_gelu_pays(int64_t n, int k, int nout);
+int lin_wide_gelu(const void* x, const void* w, const void* bias, int dtype, int64_t n, int nout, int act, void* out, void* aux,
+                  hipStream_t stream);
+
 // The LayerNorm in front of a layer of few rows, formed by the layer itself instead of by a launch of its own.
 struct LinFront {
     enum { NORM = 1, NORM_SUM_NORM = 2 };

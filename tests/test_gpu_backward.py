@@ -668,6 +668,24 @@ def test_linear_gelu_kernels_against_their_parts(dtype):
         assert rel_err(d, z.grad.cpu()) < 4e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,nout", [(15_681, 1024), (20_033, 1280), (65_537, 256), (49_217, 512)])
+def test_linear_gelu_of_many_256_input_rows(dtype, n, nout):
+    """The register-weight kernel's training forms of the GELU, one tile of rows a work-group and several, whole and cut
+    ones: the rows in front of the GELU are the plain kernel's bits, the rest follows to one rounding."""
+    o = ops()
+    g = torch.Generator(device=DEV).manual_seed(nout)
+    x, w, b = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((n, 256), (nout, 256), (nout,)))
+    w = w / 16
+    pre, act = o.linear_gelu(x, w, b)
+    assert torch.equal(pre, o.linear_rows(x, w, b))
+    assert rel_err(act, torch.nn.functional.gelu(pre.float()).cpu()) < TOL[dtype]
+    got = o.linear_gelu_bwd(x, w, pre)
+    q = pre.float()
+    grad = 0.5 * torch.erfc(-q / 2 ** 0.5) + q * torch.exp(-q * q / 2) / (2 * np.pi) ** 0.5
+    assert rel_err(got, (o.linear_rows(x, w).float() * grad).cpu()) < TOL[dtype]
+
+
 @pytest.mark.parametrize("skip_dtype,branch_dtype", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
                                                      (torch.float32, torch.float32), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("n,c", [(1000, 32), (77, 512), (1, 8), (4099, 64)])
