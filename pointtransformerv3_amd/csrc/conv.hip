@@ -26,7 +26,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
-#include "common.h"
+#include "bnact.h"
 
 namespace {
 
@@ -933,13 +933,13 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_pairs_kernel(
 // y (n_pairs, cout) in output-major slot order -> out[i] = bias + sum of voxel i's slots. Bound by memory on large levels (1M
 // points: 5.9 TB/s), by its chain of trips to memory (row pointer, slots) and by what precedes it on small ones: with the bias
 // in one load and the row found by a shift the 11 launches of a room of 100k voxels went from 166 to 145 us, the 21 of a scan of 2k
-// from 131 to 106.
-template <typename T, typename Y>
+// from 131 to 106. BN: the stem's BatchNorm and GELU on the sums, a pass over the rows and a launch less (bnact.h).
+template <typename T, typename Y, bool BN>
 __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restrict__ y,
                                                                const int32_t* __restrict__ row_ptr,
                                                                int64_t n, int cout, PieceDiv groups,
                                                                const T* __restrict__ bias,
-                                                               T* __restrict__ out) {
+                                                               T* __restrict__ out, BnGelu bn) {
     typedef Y v8 __attribute__((ext_vector_type(8)));
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t i = ptv3_row_of(e, groups);
@@ -950,6 +950,8 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
     typedef T b8 __attribute__((ext_vector_type(8)));
     b8 b = {0, 0, 0, 0, 0, 0, 0, 0};
     if (bias) b = *(const b8*)(bias + c);
+    BnChannels<T, 8> norm;
+    if constexpr (BN) norm.load(bn, c);
     float acc[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[k] = HalfOps<T>::to_float(b[k]);
@@ -971,6 +973,9 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
         }
     }
     u32x4 r;
+    if constexpr (BN)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] = norm.apply(acc[k], k, bn.eps);
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = HalfOps<T>::pack2(acc[2 * k], acc[2 * k + 1]);
     *(u32x4*)(out + i * cout + c) = r;
@@ -1126,10 +1131,11 @@ int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, co
     return launch_pair_gemm<T, 1, 4, 4, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
 }
 
-template <typename T, typename Y>
-void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int cout, const void* bias, void* out, hipStream_t stream) {
-    hipLaunchKernelGGL((pair_segment_sum_kernel<T, Y>), dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream,
-                       (const Y*)y, row_ptr, n, cout, ptv3_piece_div(cout / 8), (const T*)bias, (T*)out);
+template <typename T, typename Y, bool BN = false>
+void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int cout, const void* bias, void* out, hipStream_t stream,
+                        const BnGelu& bn = BnGelu{}) {
+    hipLaunchKernelGGL((pair_segment_sum_kernel<T, Y, BN>), dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream,
+                       (const Y*)y, row_ptr, n, cout, ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn);
 }
 
 }  // namespace
@@ -1161,7 +1167,7 @@ extern "C" int ptv3_subm_conv_fwd(const void* feat, int dtype, int64_t n, int ci
 int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
                              const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot,
                              const float* weight, const float* bias, int cout, float* y, float* out,
-                             hipStream_t stream);   // gemmf32.hip
+                             hipStream_t stream, const BnGelu* bn = nullptr);   // gemmf32.hip
 
 extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, int cin, int taps,
                                         int64_t n_pairs, const int32_t* tap_ptr,
@@ -1191,6 +1197,23 @@ extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, 
         if (rc != PTV3_OK) return rc;
         launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, cout, bias, out, stream);
     }
+    PTV3_RETURN_LAUNCH();
+}
+
+int ptv3_conv_pairs_bn_gelu(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
+                            const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot, const void* weight, int cout,
+                            const BnGelu& bn, void* y, void* out, hipStream_t stream) {
+    if (n < 1 || cin < 1 || cout < 1 || taps < 1 || n_pairs < 1 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
+    if (dtype < PTV3_F32 || dtype > PTV3_BF16 || cout % 8 != 0 || (dtype != PTV3_F32 && cin % 16 != 0)) return PTV3_ESHAPE;
+    if (!feat || !tap_ptr || !row_ptr || !pair_in || !pair_slot || !weight || !y || !out || !bn.mean || !bn.var) return PTV3_EINVAL;
+    if (dtype == PTV3_F32)
+        return ptv3_subm_conv_pairs_f32((const float*)feat, n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot,
+                                        (const float*)weight, nullptr, cout, (float*)y, (float*)out, stream, &bn);
+    const int rc = dtype == PTV3_F16 ? dispatch_pairs<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream)
+                                     : dispatch_pairs<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
+    if (rc != PTV3_OK) return rc;
+    if (dtype == PTV3_F16) launch_segment_sum<_Float16, _Float16, true>(y, row_ptr, n, cout, nullptr, out, stream, bn);
+    else launch_segment_sum<__bf16, __bf16, true>(y, row_ptr, n, cout, nullptr, out, stream, bn);
     PTV3_RETURN_LAUNCH();
 }
 

@@ -4,7 +4,7 @@
 // modules would pick (modules.py, ops.py), so the results are the same bits.
 #include <string.h>
 
-#include "common.h"
+#include "bnact.h"
 #include "lintile.h"
 
 namespace {
@@ -59,6 +59,8 @@ int linear(Run& r, const void* x, const ptv3_linear_w& w, int64_t n, void* out) 
         return ptv3_linear_gemm_fwd(x, w.w, w.b, nullptr, r.dt, n, w.in, w.out, out, r.stream);
     return ptv3_linear_any_fwd(x, w.w, w.b, nullptr, r.dt, n, w.in, w.out, 0, out, r.stream);
 }
+
+BnGelu bn_gelu(const ptv3_bn_w& bn) { return BnGelu{bn.mean, bn.var, bn.g, bn.b, bn.eps, bn.stats_f32}; }
 
 // Linear -> BatchNorm1d (running statistics) -> GELU
 int linear_bn_gelu(Run& r, const void* x, const ptv3_linear_w& w, const ptv3_bn_w& bn, int64_t n, void* out) {
@@ -281,11 +283,19 @@ int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, vo
             if (!r.dry) TRY(ptv3_pad_rows(feat, feat_dtype, n0, net.stem_in, cin, p, r.dt, r.stream));
             in = p;
         }
-        void* z = r.rows(n0, c0);
-        TRY(conv_rows(r, 0, 125, in, cin, net.stem_w, nullptr, c0, z));
-        if (!r.dry)
-            TRY(ptv3_bn_act(z, net.stem_bn.mean, net.stem_bn.var, net.stem_bn.stats_f32, net.stem_bn.g, net.stem_bn.b, r.dt, n0, c0,
-                            net.stem_bn.eps, 1, x, r.stream));
+        if (pair_form(r, 0, 125, cin, c0) == PTV3_CONV_PAIRS) {
+            const ptv3_level& v = r.lv[0];
+            void* y = r.rows(v.n_pairs5, c0);
+            if (!r.dry)
+                TRY(ptv3_conv_pairs_bn_gelu(in, r.dt, n0, cin, 125, v.n_pairs5, v.tap_ptr5, v.row_ptr5, v.pair_in5, v.pair_slot5,
+                                            net.stem_w, c0, bn_gelu(net.stem_bn), y, x, (hipStream_t)r.stream));
+        } else {
+            void* z = r.rows(n0, c0);
+            TRY(conv_rows(r, 0, 125, in, cin, net.stem_w, nullptr, c0, z));
+            if (!r.dry)
+                TRY(ptv3_bn_act(z, net.stem_bn.mean, net.stem_bn.var, net.stem_bn.stats_f32, net.stem_bn.g, net.stem_bn.b, r.dt, n0,
+                                c0, net.stem_bn.eps, 1, x, r.stream));
+        }
         r.mem.at = m2;
     }
     // ---- encoder
@@ -300,9 +310,8 @@ int forward(Run& r, const void* feat, int feat_dtype, void* const* stage_out, vo
             void *p = r.rows(up.n, st.channels), *q = r.rows(v.n, st.channels);
             TRY(linear(r, level_rows[s - 1], st.pool, up.n, p));
             if (!r.dry) {
-                TRY(ptv3_segment_reduce(p, r.dt, up.n, st.channels, up.order, v.idx_ptr, v.n, st.pool_reduce, q, r.stream));
-                TRY(ptv3_bn_act(q, st.pool_bn.mean, st.pool_bn.var, st.pool_bn.stats_f32, st.pool_bn.g, st.pool_bn.b, r.dt, v.n,
-                                st.channels, st.pool_bn.eps, 1, x, r.stream));
+                TRY(ptv3_segment_reduce_bn_gelu(p, r.dt, up.n, st.channels, up.order, v.idx_ptr, v.n, st.pool_reduce,
+                                                bn_gelu(st.pool_bn), q, x, (hipStream_t)r.stream));
             }
             r.mem.at = m2;
         }

@@ -21,6 +21,7 @@
 // Measured (MI355X; us, float instruction -> pieces): 100k x 64 -> 192 40 -> 35, 36k x 128 -> 384 51 -> 35, 11.6k x 256 -> 1024
 // 70 -> 42, 2.1k x 2048 -> 512 93 -> 73, 300 x 512 -> 512 18 -> 13; rows of 1e-6, 100k x 64 -> 64 17.5 -> 16.1; a float forward
 // of one room of 100k voxels 10.9 -> 8.5 ms.
+#include "bnact.h"
 #include "rowtile.h"
 
 namespace {
@@ -381,11 +382,11 @@ int launch_f32(F32Args& g, int64_t rows, hipStream_t stream) {
 }
 
 // y (pairs, cout) in output-major slot order -> out[i] = bias + sum of voxel i's slots, V channels per thread
-template <int V>
+template <int V, bool BN>
 __global__ __launch_bounds__(256) void pair_segment_sum_f32_kernel(const float* __restrict__ y,
                                                                    const int32_t* __restrict__ row_ptr, int64_t n,
                                                                    int cout, PieceDiv groups, const float* __restrict__ bias,
-                                                                   float* __restrict__ out) {
+                                                                   float* __restrict__ out, BnGelu bn) {
     typedef float vec __attribute__((ext_vector_type(V)));
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t i = ptv3_row_of(e, groups);
@@ -394,6 +395,8 @@ __global__ __launch_bounds__(256) void pair_segment_sum_f32_kernel(const float* 
     vec acc;
 #pragma unroll
     for (int k = 0; k < V; ++k) acc[k] = bias ? bias[c + k] : 0.f;
+    BnChannels<float, V> norm;
+    if constexpr (BN) norm.load(bn, c);
     const int s0 = row_ptr[i], s1 = row_ptr[i + 1];
     const float* src = y + (int64_t)s0 * cout + c;
     for (int s = s0; s < s1; s += 4, src += 4 * (int64_t)cout) {
@@ -405,6 +408,9 @@ __global__ __launch_bounds__(256) void pair_segment_sum_f32_kernel(const float* 
         for (int j = 0; j < 4; ++j)
             if (s + j < s1) acc += r[j];
     }
+    if constexpr (BN)
+#pragma unroll
+        for (int k = 0; k < V; ++k) acc[k] = norm.apply(acc[k], k, bn.eps);
     *(vec*)(out + i * cout + c) = acc;
 }
 
@@ -415,8 +421,8 @@ bool aligned16(const void* a, const void* b) { return (((uintptr_t)a | (uintptr_
 int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
                              const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot,
                              const float* weight, const float* bias, int cout, float* y, float* out,
-                             hipStream_t stream) {
-    if (taps > 128) return PTV3_ESHAPE;
+                             hipStream_t stream, const BnGelu* bn) {
+    if (taps > 128 || (bn && cout % 4 != 0)) return PTV3_ESHAPE;
     if (n_pairs > 0) {
         F32Args g = {};
         g.x = feat; g.w = weight; g.w_row = (int64_t)taps * cin; g.w_tap = cin; g.out = y;
@@ -426,12 +432,14 @@ int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, in
                                     : launch_f32<float, float, false, true>(g, n_pairs, stream);
         if (rc != PTV3_OK) return rc;
     }
-    if (cout % 4 == 0)
-        hipLaunchKernelGGL(pair_segment_sum_f32_kernel<4>, dim3((unsigned)ptv3_ceil_div(n * (cout / 4), 256)), dim3(256),
-                           0, stream, y, row_ptr, n, cout, ptv3_piece_div(cout / 4), bias, out);
-    else
-        hipLaunchKernelGGL(pair_segment_sum_f32_kernel<1>, dim3((unsigned)ptv3_ceil_div(n * cout, 256)), dim3(256), 0,
-                           stream, y, row_ptr, n, cout, ptv3_piece_div(cout), bias, out);
+    if (cout % 4 == 0) {
+        auto kern = bn ? pair_segment_sum_f32_kernel<4, true> : pair_segment_sum_f32_kernel<4, false>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n * (cout / 4), 256)), dim3(256), 0, stream, y, row_ptr, n, cout,
+                           ptv3_piece_div(cout / 4), bias, out, bn ? *bn : BnGelu{});
+    } else {
+        hipLaunchKernelGGL((pair_segment_sum_f32_kernel<1, false>), dim3((unsigned)ptv3_ceil_div(n * cout, 256)), dim3(256), 0,
+                           stream, y, row_ptr, n, cout, ptv3_piece_div(cout), bias, out, BnGelu{});
+    }
     PTV3_RETURN_LAUNCH();
 }
 

@@ -17,6 +17,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include "bnact.h"
 #include "rownorm.h"
 
 namespace {
@@ -121,20 +122,6 @@ __global__ __launch_bounds__(256) void layer_norm_generic_kernel(
 // Inference-mode BatchNorm1d followed (optionally) by exact GELU: y = act((x - mean) * rstd * gamma
 // + beta), per channel, 8 channels per thread. The normalised value is rounded to the storage type
 // before the activation, as two separate layers would round it.
-__device__ __forceinline__ float gelu_exact(float x) {
-    // 0.5 x (1 + erf(x / sqrt 2)); erf by Abramowitz-Stegun 7.1.26, |error| < 1.5e-7
-    const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
-    float p = fmaf(1.061405429f, t, -1.453152027f);
-    p = fmaf(p, t, 1.421413741f);
-    p = fmaf(p, t, -0.284496736f);
-    p = fmaf(p, t, 0.254829592f);
-    const float e = __builtin_amdgcn_exp2f(-z * z * 1.4426950408889634f);
-    const float erf_abs = fmaf(-p * t, e, 1.0f);
-    const float half_x = 0.5f * x;
-    return fmaf(copysignf(erf_abs, x), half_x, half_x);
-}
-
 template <typename T, typename S>
 __global__ __launch_bounds__(256) void bn_act_kernel(const T* __restrict__ x, const S* __restrict__ mean,
                                                      const S* __restrict__ var, const T* __restrict__ gamma,

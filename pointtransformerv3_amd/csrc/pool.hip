@@ -9,7 +9,7 @@
 
 #include <mutex>
 
-#include "common.h"
+#include "bnact.h"
 
 namespace {
 
@@ -211,15 +211,17 @@ template <typename T> __device__ __forceinline__ void st(T* p, float v) { *p = (
 // V consecutive channels per thread (V * sizeof(T) = 16 bytes when the channel count allows)
 template <typename T, int V> struct Pack { T v[V]; };
 
-template <typename T, int V>
+template <typename T, int V, bool BN>
 __global__ __launch_bounds__(256) void segment_reduce_kernel(
     const T* __restrict__ src, int c, PieceDiv groups, const int64_t* __restrict__ indices,
-    const int64_t* __restrict__ idx_ptr, int64_t m, int op, T* __restrict__ out) {
+    const int64_t* __restrict__ idx_ptr, int64_t m, int op, T* __restrict__ out, BnGelu bn) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t s = ptv3_row_of(e, groups);
     if (s >= m) return;
     const int ch = (int)(e - s * groups.count) * V;
     const int64_t b = idx_ptr[s], t = idx_ptr[s + 1];
+    BnChannels<T, V> norm;
+    if constexpr (BN) norm.load(bn, ch);
     float acc[V];
 #pragma unroll
     for (int k = 0; k < V; ++k) acc[k] = (op == 0) ? -INFINITY : (op == 3 ? INFINITY : 0.f);
@@ -249,6 +251,7 @@ __global__ __launch_bounds__(256) void segment_reduce_kernel(
         float v = acc[k];
         if (op == 1 && t > b) v /= (float)(t - b);
         if (t == b) v = 0.f;
+        if constexpr (BN) v = norm.apply(v, k, bn.eps);
         r.v[k] = (T)v;
     }
     *(Pack<T, V>*)(out + s * c + ch) = r;
@@ -323,21 +326,31 @@ __global__ __launch_bounds__(256) void unpool_add_kernel(const T* __restrict__ p
     *(Pack<T, V>*)(out + i * c + ch) = r;
 }
 
+// a thread per (segment, pack) leaves most of the part idle, and each walks 32 members or more
+bool long_segments(int64_t n, int c, int V, int64_t m) { return c % V == 0 && m * (c / V) <= 16384 && n >= 32 * m && m <= 65535; }
+
 template <typename T>
 void launch_segment_reduce(const void* src, int64_t n, int c, const int64_t* indices, const int64_t* idx_ptr, int64_t m,
                            int op, void* out, hipStream_t stream) {
     constexpr int V = 16 / sizeof(T);
-    // a thread per (segment, pack) leaves most of the part idle, and each walks 32 members or more
-    if (c % V == 0 && m * (c / V) <= 16384 && n >= 32 * m && m <= 65535) {
+    if (long_segments(n, c, V, m)) {
         hipLaunchKernelGGL((segment_reduce_long_kernel<T, V>), dim3((unsigned)m, (unsigned)ptv3_ceil_div(c, 16 * V)), dim3(1024), 0,
                            stream, (const T*)src, c, indices, idx_ptr, op, (T*)out);
     } else if (c % V == 0) {
-        hipLaunchKernelGGL((segment_reduce_kernel<T, V>), dim3((unsigned)ptv3_ceil_div(m * (c / V), 256)), dim3(256), 0,
-                           stream, (const T*)src, c, ptv3_piece_div(c / V), indices, idx_ptr, m, op, (T*)out);
+        hipLaunchKernelGGL((segment_reduce_kernel<T, V, false>), dim3((unsigned)ptv3_ceil_div(m * (c / V), 256)), dim3(256), 0,
+                           stream, (const T*)src, c, ptv3_piece_div(c / V), indices, idx_ptr, m, op, (T*)out, BnGelu{});
     } else {
-        hipLaunchKernelGGL((segment_reduce_kernel<T, 1>), dim3((unsigned)ptv3_ceil_div(m * c, 256)), dim3(256), 0,
-                           stream, (const T*)src, c, ptv3_piece_div(c), indices, idx_ptr, m, op, (T*)out);
+        hipLaunchKernelGGL((segment_reduce_kernel<T, 1, false>), dim3((unsigned)ptv3_ceil_div(m * c, 256)), dim3(256), 0,
+                           stream, (const T*)src, c, ptv3_piece_div(c), indices, idx_ptr, m, op, (T*)out, BnGelu{});
     }
+}
+
+template <typename T>
+void launch_segment_reduce_bn(const void* src, int c, const int64_t* indices, const int64_t* idx_ptr, int64_t m, int op,
+                              const BnGelu& bn, void* out, hipStream_t stream) {
+    constexpr int V = 16 / sizeof(T);
+    hipLaunchKernelGGL((segment_reduce_kernel<T, V, true>), dim3((unsigned)ptv3_ceil_div(m * (c / V), 256)), dim3(256), 0, stream,
+                       (const T*)src, c, ptv3_piece_div(c / V), indices, idx_ptr, m, op, (T*)out, bn);
 }
 
 template <typename T>
@@ -505,5 +518,21 @@ extern "C" int ptv3_pool_orders(const int64_t* order, const int64_t* cluster, in
     hipLaunchKernelGGL(order_scan_kernel, dim3((unsigned)k), dim3(PB), 0, stream, block_cnt, blocks);
     hipLaunchKernelGGL(order_assign_kernel, grid, dim3(PB), 0, stream, order, cluster, n, m, perm,
                        (const uint32_t*)block_cnt, order_out, inverse_out);
+    PTV3_RETURN_LAUNCH();
+}
+
+int ptv3_segment_reduce_bn_gelu(const void* src, int dtype, int64_t n, int c, const int64_t* indices, const int64_t* idx_ptr,
+                                int64_t m, int op, const BnGelu& bn, void* rows, void* out, hipStream_t stream) {
+    if (n < 0 || m < 0 || c < 1 || op < 0 || op > 3 || dtype < PTV3_F32 || dtype > PTV3_BF16) return PTV3_EINVAL;
+    if (m == 0) return PTV3_OK;
+    if (!src || !indices || !idx_ptr || !bn.mean || !bn.var || !out) return PTV3_EINVAL;
+    const int v = dtype == PTV3_F32 ? 4 : 8;
+    if (c % 8 != 0 || long_segments(n, c, v, m)) {
+        const int rc = ptv3_segment_reduce(src, dtype, n, c, indices, idx_ptr, m, op, rows, stream);
+        return rc != PTV3_OK ? rc : ptv3_bn_act(rows, bn.mean, bn.var, bn.stats_f32, bn.gamma, bn.beta, dtype, m, c, bn.eps, 1, out, stream);
+    }
+    if (dtype == PTV3_F32) launch_segment_reduce_bn<float>(src, c, indices, idx_ptr, m, op, bn, out, stream);
+    else if (dtype == PTV3_F16) launch_segment_reduce_bn<_Float16>(src, c, indices, idx_ptr, m, op, bn, out, stream);
+    else launch_segment_reduce_bn<__bf16>(src, c, indices, idx_ptr, m, op, bn, out, stream);
     PTV3_RETURN_LAUNCH();
 }
