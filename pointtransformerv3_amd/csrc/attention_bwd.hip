@@ -462,6 +462,16 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_kv_kernel(
     }
 }
 
+// Two tiles of 16 rows of 16 halves, one after the other in LDS, read by column: lane l passes p + 8 l and gets, of either tile,
+// rows 4 (l / 16) .. + 3 of column l % 16.
+__device__ __forceinline__ u32x4 columns(const unsigned char* p) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 512)));
+    return (u32x4){a[0], a[1], b[0], b[1]};
+}
+
 // How the work-groups of the both-sides kernel share the items from `first` on: `parts` work-groups an item, each with its
 // range of the keys. With more than one a part leaves its share of dQ (float) in row slot - cu[first / heads] of its own
 // `stride` rows, and attn_bwd_finish_kernel adds them up.
@@ -476,37 +486,42 @@ struct BothParts {
 // A wave owns KG groups of 16 keys; their K and V, and the sums of their dK and dV, stay in its registers while the
 // work-group walks over the queries in LDS. In a step a wave takes one block of 32 queries:
 //   S and dP as 16 x 16 tiles with a lane per key (registers: queries), P = 2^(S - lse), dS = P (dP - D);
-//   dV^T += dO^T P and dK^T += Q^T dS straight from those registers (the transposed Q and dO lie in LDS with the queries
-//   in the order in which the tiles hold them);
+//   dV^T += dO^T P and dK^T += Q^T dS straight from those registers (the transposed Q and dO are read out of the rows by
+//   column, the queries in the order in which the tiles hold them);
 //   dS^T, which dQ^T += K^T dS^T needs with a lane per query, by a product with the identity: exact, and it costs the
-//   matrix pipe 16 cycles a tile where the vector pipe would repeat the exponentials.
-// dQ sums over the keys of all waves: in step s wave w takes block (w + s) mod WAVES, so a block's fp32 sums in LDS
-// belong to one wave at a time, in a fixed order, and a barrier a step is all that this needs.
+//   matrix pipe 16 cycles a tile where the vector pipe would repeat the exponentials. Turned through LDS instead, the wait for
+//   it lasts longer than those cycles (770 items 298 -> 302 us).
+// dQ sums over the keys of all waves: `ring` blocks of queries are under way together, and in step s wave w takes block
+// (w ring / WAVES + s) mod ring. So a block's fp32 sums in LDS belong to one wave at a time, in a fixed order, and a barrier
+// every ring / WAVES steps is all that this needs. A ring is as long as a sequence fills it: missing blocks are idle steps.
 //
 // Bound by the two pipes of a SIMD together: for 32 x 32 scores 56 vector instructions (16 of them exponentials, which take
-// two issue slots), 18 matrix instructions and 288 cycles of the matrix pipe, about 400 cycles if all overlapped, 585
-// measured with two waves a SIMD; the two kernels above take 890 together, the exponentials twice. Eight waves of 128 keys
-// and not 16 of 64: the query side of a step and the dQ sums pass LDS half as often, and the registers for a group ahead
-// are there (16 waves spill). bf16, 1024 slots: 1400 items 630 -> 489 us, 788 items 374 -> 298 us, 384 items 188 -> 154 us.
+// two issue slots), 18 matrix instructions and 288 cycles of the matrix pipe. A loop of just these takes 174 ns with two waves a
+// SIMD (143 the matrix, 136 the vector instructions alone), here they take 265, and an eighth of the time is the staging, which
+// the CUs do at the same time, at the rate of memory. The older wave of a SIMD goes first and then waits at the barrier for
+// the other, so what a step asks of LDS at its start is exposed: the next step's scores are asked for as soon as the
+// registers are free, and dQ starts from its sums. Eight waves of 128 keys and not 16 of 64: the query side of a step and
+// the dQ sums pass LDS half as often, and the registers for a group ahead are there (16 waves spill). bf16, 1024 slots:
+// 1400 items 630 us in two kernels, 489 whole in this one; the transposes read by column, the ring and the early reads took 788
+// items from 271 to 259 us, 60 from 45.3 to 42.5, 512 of 512 slots from 63.2 to 59.0, 128 of 500 from 26.7 to 25.4.
 // With few items several work-groups share one, each with a range of its keys (KG 4 or 2) and all of its queries; a step's
 // query side passes LDS as often (96 KB a step for the eight waves, 0.4 us), so half the keys take 0.7 of the time.
+// Steps unrolled as far as the registers leave two work-groups on a CU up to 256 slots, one up to 512.
 template <typename T, int KG, int QUERIES, bool DROP>
 __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     const T* __restrict__ qkv, const T* __restrict__ out, const T* __restrict__ dout, int channels, int heads,
     const int32_t* __restrict__ slot_src, const int32_t* __restrict__ slot_dst, const int32_t* __restrict__ cu_seqlens,
     float scale, int64_t n_pad, const float* __restrict__ lse, T* __restrict__ dqkv, T* __restrict__ fill, Dropout drop, BothParts by) {
     constexpr int WAVES = BOTH_WAVES;
+    static_assert(QUERIES == 256 || QUERIES == 512 || QUERIES == 1024, "rings below");
     constexpr int KEYS = KG * 16 * WAVES;          // keys of a work-group
-    constexpr int T_STRIDE = QUERIES * 2 + VT_PAD_BYTES;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* q_lds = smem;                                  // Q * scale * log2(e), rows
     unsigned char* do_lds = q_lds + QUERIES * 32;                 // dO rows
-    unsigned char* qt_lds = do_lds + QUERIES * 32;                // the same two, transposed
-    unsigned char* dot_lds = qt_lds + HD * T_STRIDE;
-    float* nlse_lds = (float*)(dot_lds + HD * T_STRIDE);          // -lse (log2 units), -D per query slot
+    float* nlse_lds = (float*)(do_lds + QUERIES * 32);            // -lse (log2 units), -D per query slot
     float* nd_lds = nlse_lds + QUERIES;
     int32_t* dst_lds = (int32_t*)(nd_lds + QUERIES);              // the row that a query slot writes
-    float* dq_lds = (float*)(dst_lds + QUERIES);                  // WAVES blocks of two 16-query tiles in lane order
+    float* dq_lds = (float*)(dst_lds + QUERIES);                  // the ring's blocks, two 16-query tiles each in lane order
 
     // the parts of an item, like the heads of a sequence, are neighbours in an XCD: they read the same rows
     const int wg = xcd_chunked_id(blockIdx.x, gridDim.x);
@@ -593,20 +608,10 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
             }
         }
     }
-    // The transposed rows, again by the identity: a wave has just written 32 whole queries per piece and turns those. The
-    // queries of a channel lie in the order in which the score tiles hold them: lane group grp's four of the first tile, then
-    // of the second
     auto turned = [&](u32x2 a, u32x2 b) {
         const f32x4 x = Half<T>::mfma16(a, unit, zero), y = Half<T>::mfma16(b, unit, zero);
         return (u32x4){Half<T>::pack2(x[0], x[1]), Half<T>::pack2(x[2], x[3]), Half<T>::pack2(y[0], y[1]), Half<T>::pack2(y[2], y[3])};
     };
-#pragma unroll
-    for (int j = 0; j < QP; ++j) {
-        const int at = (wave * PTV3_WAVE + j * THREADS) >> 1;
-        const int row = (at + col) * 32 + grp * 8, t = col * T_STRIDE + at * 2 + grp * 16;
-        *(u32x4*)(qt_lds + t) = turned(*(const u32x2*)(q_lds + row), *(const u32x2*)(q_lds + row + 16 * 32));
-        *(u32x4*)(dot_lds + t) = turned(*(const u32x2*)(do_lds + row), *(const u32x2*)(do_lds + row + 16 * 32));
-    }
 #pragma unroll
     for (int p = 0; p < KG / 2; ++p) {   // K^T, a lane per channel: here a key that does not exist is zero
         const u32x2 none = {0, 0};
@@ -618,7 +623,7 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     u32x2 qa[2], ga[2];
     f32x4 cl[2], cd[2];
     u32x4 qt, gt;
-    auto fetch = [&](int block) {   // the query side of a step
+    auto fetch_scores = [&](int block) {   // the query side of a step: what its scores take
         const int at = block * 32;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -627,15 +632,29 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
             cl[t] = *(const f32x4*)(nlse_lds + at + t * 16 + grp * 4);
             cd[t] = *(const f32x4*)(nd_lds + at + t * 16 + grp * 4);
         }
-        qt = *(const u32x4*)(qt_lds + col * T_STRIDE + at * 2 + grp * 16);
-        gt = *(const u32x4*)(dot_lds + col * T_STRIDE + at * 2 + grp * 16);
     };
-    fetch(wave);
-    for (int b0 = 0; b0 < blocks; b0 += WAVES) {
-        for (int s = 0; s < WAVES; ++s) {
-            const int blk = (wave + s) & (WAVES - 1);
+    auto fetch_sums = [&](int block) {     // and what the sums over its queries take
+        qt = columns(q_lds + block * 32 * 32 + lane * 8);
+        gt = columns(do_lds + block * 32 * 32 + lane * 8);
+    };
+    // blocks that are under way together, of those that are left; whole rings end within QUERIES
+    auto ring_of = [](int left) { return QUERIES < BOTH_KEYS ? WAVES : left > 24 ? 32 : left > 8 ? 16 : 8; };
+    int ring = ring_of(blocks);
+    fetch_scores(wave * (ring / WAVES));
+    fetch_sums(wave * (ring / WAVES));
+    for (int b0 = 0, next; b0 < blocks; b0 += ring, ring = next) {
+        const int lag = ring / WAVES;
+        next = ring_of(blocks - b0 - ring);
+#pragma unroll(QUERIES == 512 ? 8 : QUERIES == 256 ? 4 : 1)
+        for (int s = 0; s < ring; ++s) {
+            const int blk = (wave * lag + s) & (ring - 1);
             const bool there = b0 + blk < blocks;
+            const int then = s + 1 < ring ? b0 + ((blk + 1) & (ring - 1)) : min(b0 + ring + wave * (next / WAVES), QUERIES / 32 - 1);
+            float* sums = dq_lds + blk * 512 + lane * 4;
             f32x4 dq[2] = {zero, zero};
+            if (there && s >= lag)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) dq[t] = *(const f32x4*)(sums + t * 256);
             if (there && mine) {
                 const int at = (b0 + blk) * 32;
                 // group k + 1's scores are on the matrix pipe while group k's exponentials are taken, group k - 1's
@@ -663,6 +682,7 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
 #pragma unroll
                 for (int k = 0; k < KG; ++k) {
                     if (k + 1 < KG) scores(k + 1);
+                    if (!DROP && k + 2 == KG) fetch_scores(then);
                     u32x4 pp, dd;
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
@@ -700,16 +720,13 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
                     __builtin_amdgcn_sched_group_barrier(0x402, 3, 0);   // VALU, transcendental
                 }
             }
-            if (s + 1 < WAVES) fetch(b0 + ((blk + 1) & (WAVES - 1)));
-            else fetch(min(b0 + WAVES + wave, QUERIES / 32 - 1));
-            __syncthreads();   // the sums that step s - 1 left are complete, and nobody touches them any more
+            if (DROP || !(there && mine)) fetch_scores(then);
+            fetch_sums(then);
             if (there) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    f32x4* sum = (f32x4*)(dq_lds + (blk * 2 + t) * 256 + lane * 4);
-                    if (s > 0) dq[t] += *sum;
-                    if (s < WAVES - 1) {
-                        *sum = dq[t];
+                    if (s < ring - lag) {
+                        *(f32x4*)(sums + t * 256) = dq[t];
                     } else if (by.parts > 1) {
                         const int q = (b0 + blk) * 32 + t * 16 + col;
                         if (q < len) *(f32x4*)(dq_part + (int64_t)q * channels + 4 * grp) = dq[t];
@@ -722,6 +739,7 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
                     }
                 }
             }
+            if (((s + 1) & (lag - 1)) == 0) __syncthreads();   // before another wave takes the sums of this one's blocks
         }
     }
 
@@ -1046,7 +1064,7 @@ BwdWs carve(void* base, int dtype, int64_t n_pad, int channels, int heads) {
 }
 
 template <int QUERIES> constexpr size_t both_lds() {
-    return 2 * QUERIES * 32 + 2 * HD * (QUERIES * 2 + VT_PAD_BYTES) + 3 * QUERIES * sizeof(float) + BOTH_WAVES * 32 * HD * sizeof(float);
+    return 2 * QUERIES * 32 + 3 * QUERIES * sizeof(float) + (QUERIES < BOTH_KEYS ? BOTH_WAVES * 32 : QUERIES) * HD * sizeof(float);
 }
 static_assert(both_lds<BOTH_KEYS>() <= 160 * 1024, "one work-group fills a CU's LDS");
 

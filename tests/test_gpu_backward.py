@@ -204,6 +204,14 @@ def test_attention_backward_items_shared_by_work_groups(dtype, lens, heads):
     test_attention_backward_both_sides(dtype, lens, heads, 0.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("blocks", [(32, 31, 25), (24, 17, 16), (9, 8, 1), (32, 24, 16, 9, 8)])
+@pytest.mark.parametrize("times,heads", [(2, 3), (8, 4), (15, 3)])   # shared by four, by two, whole
+def test_attention_backward_rounds_of_query_blocks(dtype, blocks, times, heads):
+    """Sequences at the edges of the rounds in which the waves take 32 queries at a time: the same checks."""
+    test_attention_backward_both_sides(dtype, [32 * b - (i + j) % 3 for j in range(times) for i, b in enumerate(blocks)], heads, 0.0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("cin,cout,ks,n", [(6, 32, 5, 1500), (32, 32, 3, 2000), (64, 64, 3, 3000), (128, 128, 3, 1200),
                                            (48, 80, 3, 700)])
