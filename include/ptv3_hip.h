@@ -625,7 +625,8 @@ int64_t ptv3_linear_pack_weights_blocks(int channels);
  * a job whose w2 is NULL and whose `reserved` is the number of channels-row chunks (1 and 3; packed = the buffer, and
  * the buffer + channels^2 elements); such a job owns reserved * ptv3_linear_pack_weights_blocks(channels) blocks.
  * Intermediates are rounded to dtype where the separate layers would store them; the normalised rows never leave
- * the CU. PTV3_ESHAPE for other widths or dtypes. */
+ * the CU. PTV3_ESHAPE for other widths or dtypes. ptv3_block_head_wide_pays: where it is faster than the separate layers. */
+int ptv3_block_head_wide_pays(int64_t n, int channels);
 int ptv3_block_head_wide(const void *conv, const void *shortcut, const void *packed, const void *cpe_bias,
                          const void *ln_cpe_weight, const void *ln_cpe_bias, float ln_cpe_eps, const void *ln1_weight,
                          const void *ln1_bias, float ln1_eps, const void *qkv_bias, int dtype, int64_t n, int channels,
@@ -752,7 +753,7 @@ const ptv3_level *ptv3_index_levels(const void *state);
  * LayerNorms of one eps, biases everywhere, BatchNorm + exact GELU behind stem, poolings and unpoolings. In half
  * precision stem_w has its input channels padded to a multiple of 16 (ptv3_pad_rows over the weight's rows), and the
  * packed copies are those of ptv3_subm_conv_pack_weight (conv_packed, 32 / 64 / 128 channels), ptv3_mlp_pack_weights_batch
- * (mlp_packed from 128 channels on, proj_packed at 128 and 256, head_packed = xCPE Linear + qkv at 128).
+ * (mlp_packed from 128 channels on, proj_packed and head_packed = xCPE Linear + qkv at 128 and 256).
  * Level l needs the lists ptv3_conv_form names for its blocks' channels (float: pairs), level 0 also the 5x5x5 lists;
  * neighbour maps are made in the workspace where ptv3_conv_pair_form asks for them.
  * stage_out: NULL, or per stage a buffer for the encoder stage's rows (or NULL in it); out: the decoder's (n, channels)

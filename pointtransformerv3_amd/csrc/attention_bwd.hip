@@ -515,6 +515,7 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     constexpr int WAVES = BOTH_WAVES;
     static_assert(QUERIES == 256 || QUERIES == 512 || QUERIES == 1024, "rings below");
     constexpr int KEYS = KG * 16 * WAVES;          // keys of a work-group
+    constexpr int UNROLL = QUERIES == 512 ? 8 : QUERIES == 256 ? 4 : 1;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* q_lds = smem;                                  // Q * scale * log2(e), rows
     unsigned char* do_lds = q_lds + QUERIES * 32;                 // dO rows
@@ -645,7 +646,7 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
     for (int b0 = 0, next; b0 < blocks; b0 += ring, ring = next) {
         const int lag = ring / WAVES;
         next = ring_of(blocks - b0 - ring);
-#pragma unroll(QUERIES == 512 ? 8 : QUERIES == 256 ? 4 : 1)
+#pragma unroll UNROLL
         for (int s = 0; s < ring; ++s) {
             const int blk = (wave * lag + s) & (ring - 1);
             const bool there = b0 + blk < blocks;

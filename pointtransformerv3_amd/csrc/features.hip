@@ -164,7 +164,7 @@ int block_half(Run& r, const ptv3_block_w& b, int s, const void* xs, const void*
         if (c <= 64) {
             TRY(ptv3_block_head_fused(conv, x, b.cpe.w, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b, b.ln1.eps,
                                       b.qkv.w, b.qkv.b, r.dt, n, c, feat, qkv, r.stream));
-        } else if (c == 128) {
+        } else if (ptv3_block_head_wide_pays(n, c)) {
             TRY(ptv3_block_head_wide(conv, x, b.head_packed, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b,
                                      b.ln1.eps, b.qkv.b, r.dt, n, c, feat, qkv, r.stream));
         } else {

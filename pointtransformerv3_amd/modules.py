@@ -439,7 +439,7 @@ class Block(PointModule):
             return point
         same_eps = ln_cpe.eps == ln1.eps
         qkv = None
-        if (fused_mlp and self.channels in ops.BLOCK_HEAD_WIDE_PAYS and type(self.cpe[1]) is nn.Linear
+        if (fused_mlp and ops.block_head_wide_pays(conv.shape[0], self.channels) and type(self.cpe[1]) is nn.Linear
                 and self.cpe[1].bias is not None and type(self.attn.qkv) is nn.Linear and self.attn.qkv.bias is not None
                 and self.attn.enable_flash):
             # cpe Linear, its LayerNorm, the residual, the attention's pre-norm and qkv in one kernel

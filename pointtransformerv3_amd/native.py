@@ -463,7 +463,6 @@ class Engine(Copies):
             if c in (128, 256):
                 d.proj_packed = self._packed(c * c)
                 self._jobs_mlp.append((d.proj.w, 0, d.proj_packed, c, 1))
-            if c == 128:
                 d.head_packed = self._packed(4 * c * c)
                 self._jobs_mlp.append((d.cpe.w, 0, d.head_packed, c, 1))
                 self._jobs_mlp.append((d.qkv.w, 0, d.head_packed + c * c * 2, c, 3))

@@ -1641,9 +1641,11 @@ def _packed_stream(m, dtype):
 
 
 BLOCK_TAIL_WIDE_CHANNELS = (128, 256)
-# block_head_wide takes the same widths; where it measured faster than linear_ln + qkv Linear: 74 -> 59 us at
-# 146k x 128, 46.5 -> 46 us at 37.7k x 256 (a pass there is too short for what it costs to start and to leave)
-BLOCK_HEAD_WIDE_PAYS = (128,)
+
+
+def block_head_wide_pays(n, channels):
+    """Whether block_head_wide is faster than linear_ln + qkv Linear for n rows (ptv3_block_head_wide_pays)."""
+    return bool(_lib.load().ptv3_block_head_wide_pays(n, channels))
 
 
 def block_tail_wide(attn, shortcut, proj, ln2, mlp):
