@@ -148,7 +148,7 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void patch_attn_half_kernel(
     const T* __restrict__ qkv, int channels, int heads, const int32_t* __restrict__ slot_src,
     const int32_t* __restrict__ slot_dst, const int32_t* __restrict__ cu_seqlens, int lds_keys,
     float scale_log2e, T* __restrict__ out, int full_items, int split, int total_items, float* __restrict__ lse,
-    int64_t lse_stride, Dropout drop) {
+    int64_t lse_stride, Dropout drop, Ahead ahead) {
     typedef typename Half<T>::v8 v8;
     extern __shared__ __align__(16) unsigned char smem[];
     // K tile: lds_keys + 64 rows of 32 B (the last 64 are only ever prefetched). V^T tile: 16 rows
@@ -258,6 +258,8 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void patch_attn_half_kernel(
     }
     __syncthreads();
 
+    const uint32_t asked = ptv3_ask(ahead, tid, ATT_THREADS);
+
     // lane l keeps the largest key norm of step l (at most 37 steps fit the LDS); the largest of all
     float kn_reg = lane < n_pairs ? sqrtf(knorm_lds[lane]) * 1.0009765625f : 0.f;   // margin for rounding in the bound
     float kn_all = kn_reg;
@@ -306,6 +308,7 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void patch_attn_half_kernel(
             if (LSE && hf == 0) lse[(int64_t)head * lse_stride + s0 + qi] = acc[9] + __builtin_amdgcn_logf(acc[8]);
         }
     }
+    ptv3_asked(asked);
 }
 
 // ---- the general shape: thread per query, fp32 FMA arithmetic, chunks of K and V in LDS (as floats), any
@@ -571,7 +574,7 @@ template <typename T, bool LSE, bool DROP>
 int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_src,
                 const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
                 int64_t max_seqlen, int64_t slots, float scale, void* out, float* lse, int64_t lse_stride, Dropout drop,
-                hipStream_t stream) {
+                const Ahead& ahead, hipStream_t stream) {
     const int lds_keys = (int)((max_seqlen + 63) & ~63ll);
     const size_t lds = half_lds_bytes(max_seqlen);
     if (lds > 160 * 1024) return PTV3_ESHAPE;
@@ -585,7 +588,7 @@ int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_sr
     const int64_t tail = (total - full + 7) / 8 * 8;   // the tail's items in groups of 8, one per XCD
     hipLaunchKernelGGL(kern, dim3((unsigned)(full + tail * split)), dim3(ATT_THREADS), lds, stream,
                        (const T*)qkv, channels, heads, slot_src, slot_dst, cu_seqlens, lds_keys,
-                       scale_log2e, (T*)out, (int)full, split, (int)total, lse, lse_stride, drop);
+                       scale_log2e, (T*)out, (int)full, split, (int)total, lse, lse_stride, drop, ahead);
     PTV3_RETURN_LAUNCH();
 }
 
@@ -593,7 +596,7 @@ int launch_half(const void* qkv, int channels, int heads, const int32_t* slot_sr
 
 int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
                               const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
-                              int64_t slots, float scale, void* out, void* stream_) {
+                              int64_t slots, float scale, void* out, const Ahead& ahead, void* stream_) {
     if (n_rows < 0 || n_seq < 0 || channels < 1 || heads < 1 || max_seqlen < 1) return PTV3_EINVAL;
     if (dtype < PTV3_F32 || dtype > PTV3_BF16) return PTV3_EINVAL;
     if (channels % heads != 0 || !any_head_dim(channels / heads)) return PTV3_ESHAPE;
@@ -604,9 +607,9 @@ int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int ch
     if (half_kernel_takes(dtype, channels, heads, max_seqlen)) {
         if (dtype == PTV3_F16)
             return launch_half<_Float16, false, false>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                                       max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
+                                                       max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, ahead, stream);
         return launch_half<__bf16, false, false>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq,
-                                                 max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, stream);
+                                                 max_seqlen, slots, scale, out, nullptr, 0, Dropout{0u, 0u, 1.f}, ahead, stream);
     }
     // fp32, and in half precision other head dims (8, 32, 64) or sequences beyond the MFMA kernel's LDS
     return launch_any(qkv, dtype, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, scale, out,
@@ -618,7 +621,7 @@ extern "C" int ptv3_patch_attn_fwd(const void* qkv, int dtype, int64_t n_rows, i
                                    const int32_t* slot_src, const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq,
                                    int64_t max_seqlen, float scale, void* out, void* stream_) {
     return ptv3_patch_attn_fwd_slots(qkv, dtype, n_rows, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen,
-                                     n_rows, scale, out, stream_);
+                                     n_rows, scale, out, Ahead{}, stream_);
 }
 
 extern "C" int ptv3_patch_attn_fwd_lse(const void* qkv, int dtype, int64_t n_rows, int channels, int heads,
@@ -638,7 +641,7 @@ extern "C" int ptv3_patch_attn_fwd_lse(const void* qkv, int dtype, int64_t n_row
                           stream);
 #define PTV3_ATT(T, D)                                                                                               \
     return launch_half<T, true, D>(qkv, channels, heads, slot_src, slot_dst, cu_seqlens, n_seq, max_seqlen, n_pad, scale, \
-                                   out, lse, n_pad, drop, stream)
+                                   out, lse, n_pad, drop, Ahead{}, stream)
     if (dtype == PTV3_F16) {
         if (drop.threshold) PTV3_ATT(_Float16, true);
         PTV3_ATT(_Float16, false);

@@ -79,10 +79,38 @@ static inline int ptv3_cus() {
     return n;
 }
 
+// Weights that every XCD reads whole in the launch behind this one: a kernel that leaves memory idle asks for them, and they are
+// in its XCD's L2 by then. In a forward they come from HBM otherwise, and a kernel that streams them has few requests in flight.
+struct Ahead {
+    const uint8_t* at[2];
+    uint32_t lines[2];   // of 128 bytes, each begun
+};
+static inline Ahead ptv3_ahead(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    return Ahead{{(const uint8_t*)a, (const uint8_t*)b}, {(uint32_t)ptv3_ceil_div(a_bytes, 128), (uint32_t)ptv3_ceil_div(b_bytes, 128)}};
+}
+// This work-group's share: the lines are dealt to the last AHEAD_GROUPS work-groups of each XCD, whose own traffic will not have
+// replaced them, at most four a thread. What comes back is used in ptv3_asked alone, at the kernel's end, and so waited for there.
+constexpr uint32_t AHEAD_GROUPS = 64;
+__device__ __forceinline__ uint32_t ptv3_ask(const Ahead& a, int tid, int threads) {
+    const uint32_t total = a.lines[0] + a.lines[1], groups = gridDim.x >> 3, slot = blockIdx.x >> 3;
+    const uint32_t askers = min(groups, AHEAD_GROUPS);
+    uint32_t v = 0;
+    if (total == 0 || slot >= groups || slot + askers < groups) return v;
+    const uint32_t per = (total + askers - 1) / askers, first = (slot + askers - groups) * per;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const uint32_t i = (uint32_t)(tid + u * threads), line = first + i;
+        if (i < per && line < total)
+            v |= line < a.lines[0] ? a.at[0][(size_t)line * 128] : a.at[1][(size_t)(line - a.lines[0]) * 128];
+    }
+    return v;
+}
+__device__ __forceinline__ void ptv3_asked(uint32_t v) { asm volatile("" ::"v"(v)); }
+
 // ptv3_patch_attn_fwd where the number of slots, cu_seqlens[n_seq], is known: what ptv3_patch_attn_cut goes by.
 int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
                               const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
-                              int64_t slots, float scale, void* out, void* stream);
+                              int64_t slots, float scale, void* out, const Ahead& ahead, void* stream);
 
 // Work-groups are dealt to the 8 XCDs round-robin in launch order, and every XCD has an L2 of its own.
 // Launch index (or persistent-loop index, with a grid that is a multiple of 8) -> item such that each XCD

@@ -144,8 +144,15 @@ int conv3(Run& r, const ptv3_block_w& b, int s, const void* x, void* out) {
 
 int attention(Run& r, const ptv3_block_w& b, const ptv3_level& v, int patch, const void* qkv, int dt, void* out) {
     if (r.dry) return PTV3_OK;
+    // 256 channels: the second half streams 1.2 MB through every work-group, 38.6 us of a room's 11.6k rows where they come from
+    // HBM, 32.0 from the L2 (the attention 34.7 and 35.4). At 128 channels it is 0.3 MB and no faster; the layers of few rows
+    // share their weights out over the work-groups.
+    Ahead ahead = {};
+    const int64_t square = (int64_t)b.channels * b.channels * 2;
+    if (r.dt != PTV3_F32 && b.channels == 256 && !ptv3_block_tail_few_pays(v.n, 256))
+        ahead = ptv3_ahead(b.proj_packed, square, b.mlp_packed, 8 * square);
     return ptv3_patch_attn_fwd_slots(qkv, dt, v.n, b.channels, b.heads, v.slot_src[b.row], v.slot_dst[b.row], v.cu, v.n_seq, patch,
-                                     v.n_pad, b.scale, out, r.stream);
+                                     v.n_pad, b.scale, out, ahead, r.stream);
 }
 
 // A block (model.py:586-606): x its rows, xs what its convolution reads, out the new rows.
