@@ -111,6 +111,10 @@ __device__ __forceinline__ void ptv3_asked(uint32_t v) { asm volatile("" ::"v"(v
 int ptv3_patch_attn_fwd_slots(const void* qkv, int dtype, int64_t n_rows, int channels, int heads, const int32_t* slot_src,
                               const int32_t* slot_dst, const int32_t* cu_seqlens, int64_t n_seq, int64_t max_seqlen,
                               int64_t slots, float scale, void* out, const Ahead& ahead, void* stream);
+// ptv3_subm_conv_pairs_fwd
+int ptv3_conv_pairs_ahead(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
+                          const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot, const void* weight,
+                          const void* bias, int cout, void* y, void* out, const Ahead& ahead, void* stream);
 
 // Work-groups are dealt to the 8 XCDs round-robin in launch order, and every XCD has an L2 of its own.
 // Launch index (or persistent-loop index, with a grid that is a multiple of 8) -> item such that each XCD

@@ -600,8 +600,11 @@ __global__ __launch_bounds__(WS_THREADS, 2) void pair_wstat_kernel(
     T* w_lds = (T*)ws_smem;                       // [COUT_T][WSTRIDE], only while the fragments are taken
     T* x_lds = w_lds + COUT_T * WSTRIDE;          // [2][WS_ROWS][WS_XSTRIDE]
 
-    // which (tap, range) is mine: ranges of range_rows pairs, tap after tap
-    int g = blockIdx.x, tap = -1, p0 = 0, p1 = 0;
+    // Which (tap, range) is mine: ranges of range_rows pairs, tap after tap. Short ranges go to the XCDs by eighths, so that the
+    // work-groups of a tap meet in one L2 and its 128 KB come from memory once (121k pairs 31.8 -> 31.0 us in a forward); with
+    // long ones the weights are no part of the time, and with few work-groups the eighths leave XCDs idle (11.2 -> 11.6).
+    const bool by_xcd = range_rows <= 1024 && gridDim.x >= 192;
+    int g = by_xcd ? xcd_chunked_id(blockIdx.x, gridDim.x) : blockIdx.x, tap = -1, p0 = 0, p1 = 0;
     for (int t = 0; t < taps; ++t) {
         const int first = tap_ptr[t], cnt = tap_ptr[t + 1] - first;
         const int nr = (cnt + range_rows - 1) / range_rows;
@@ -939,8 +942,9 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
                                                                const int32_t* __restrict__ row_ptr,
                                                                int64_t n, int cout, PieceDiv groups,
                                                                const T* __restrict__ bias,
-                                                               T* __restrict__ out, BnGelu bn) {
+                                                               T* __restrict__ out, BnGelu bn, Ahead ahead) {
     typedef Y v8 __attribute__((ext_vector_type(8)));
+    const uint32_t asked = ptv3_ask(ahead, threadIdx.x, blockDim.x);
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t i = ptv3_row_of(e, groups);
     if (i >= n) return;
@@ -979,6 +983,7 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = HalfOps<T>::pack2(acc[2 * k], acc[2 * k + 1]);
     *(u32x4*)(out + i * cout + c) = r;
+    ptv3_asked(asked);
 }
 
 // fp32: one thread per (voxel, output channel); a wave shares the voxel when cout >= 64.
@@ -1133,9 +1138,9 @@ int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, co
 
 template <typename T, typename Y, bool BN = false>
 void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int cout, const void* bias, void* out, hipStream_t stream,
-                        const BnGelu& bn = BnGelu{}) {
+                        const BnGelu& bn = BnGelu{}, const Ahead& ahead = Ahead{}) {
     hipLaunchKernelGGL((pair_segment_sum_kernel<T, Y, BN>), dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream,
-                       (const Y*)y, row_ptr, n, cout, ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn);
+                       (const Y*)y, row_ptr, n, cout, ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn, ahead);
 }
 
 }  // namespace
@@ -1169,12 +1174,9 @@ int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, in
                              const float* weight, const float* bias, int cout, float* y, float* out,
                              hipStream_t stream, const BnGelu* bn = nullptr);   // gemmf32.hip
 
-extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, int cin, int taps,
-                                        int64_t n_pairs, const int32_t* tap_ptr,
-                                        const int32_t* row_ptr, const int32_t* pair_in,
-                                        const int32_t* pair_slot, const void* weight,
-                                        const void* bias, int cout, void* y, void* out,
-                                        void* stream_) {
+int ptv3_conv_pairs_ahead(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
+                          const int32_t* row_ptr, const int32_t* pair_in, const int32_t* pair_slot, const void* weight,
+                          const void* bias, int cout, void* y, void* out, const Ahead& ahead, void* stream_) {
     if (n < 0 || cin < 1 || cout < 1 || taps < 1 || n_pairs < 0 || n_pairs >= (1ll << 31)) return PTV3_EINVAL;
     if (dtype < PTV3_F32 || dtype > PTV3_BF16) return PTV3_ESHAPE;
     if (dtype != PTV3_F32 && (cin % 16 != 0 || cout % 8 != 0)) return PTV3_ESHAPE;
@@ -1190,14 +1192,22 @@ extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, 
         if (n_pairs > 0)
             rc = dispatch_pairs<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        launch_segment_sum<_Float16, _Float16>(y, row_ptr, n, cout, bias, out, stream);
+        launch_segment_sum<_Float16, _Float16>(y, row_ptr, n, cout, bias, out, stream, BnGelu{}, ahead);
     } else {
         if (n_pairs > 0)
             rc = dispatch_pairs<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, cout, bias, out, stream);
+        launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, cout, bias, out, stream, BnGelu{}, ahead);
     }
     PTV3_RETURN_LAUNCH();
+}
+
+extern "C" int ptv3_subm_conv_pairs_fwd(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs,
+                                        const int32_t* tap_ptr, const int32_t* row_ptr, const int32_t* pair_in,
+                                        const int32_t* pair_slot, const void* weight, const void* bias, int cout, void* y, void* out,
+                                        void* stream) {
+    return ptv3_conv_pairs_ahead(feat, dtype, n, cin, taps, n_pairs, tap_ptr, row_ptr, pair_in, pair_slot, weight, bias, cout, y, out,
+                                 Ahead{}, stream);
 }
 
 int ptv3_conv_pairs_bn_gelu(const void* feat, int dtype, int64_t n, int cin, int taps, int64_t n_pairs, const int32_t* tap_ptr,
