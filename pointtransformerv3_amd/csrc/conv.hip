@@ -936,8 +936,11 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void subm_conv_pairs_kernel(
 // y (n_pairs, cout) in output-major slot order -> out[i] = bias + sum of voxel i's slots. Bound by memory on large levels (1M
 // points: 5.9 TB/s), by its chain of trips to memory (row pointer, slots) and by what precedes it on small ones: with the bias
 // in one load and the row found by a shift the 11 launches of a room of 100k voxels went from 166 to 145 us, the 21 of a scan of 2k
-// from 131 to 106. BN: the stem's BatchNorm and GELU on the sums, a pass over the rows and a launch less (bnact.h).
-template <typename T, typename Y, bool BN>
+// from 131 to 106. BN: the stem's BatchNorm and GELU on the sums, a pass over the rows and a launch less (bnact.h). ONCE: the rows
+// are more than the L2s hold and do not stay there, in place of what the next kernels read (a room's blocks of 256 channels:
+// the next kernel 19.4 -> 18.4 us, the forward 3212 -> 3202); rows that are still there from the kernel before are read from
+// there (a scan of 2k: 5.4 us, 5.9 with ONCE).
+template <typename T, typename Y, bool BN, bool ONCE>
 __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restrict__ y,
                                                                const int32_t* __restrict__ row_ptr,
                                                                int64_t n, int cout, PieceDiv groups,
@@ -966,7 +969,8 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             raw[j] = (v8){0, 0, 0, 0, 0, 0, 0, 0};
-            if (s + j < s1) raw[j] = *(const v8*)(src + (int64_t)j * cout);
+            const v8* at = (const v8*)(src + (int64_t)j * cout);
+            if (s + j < s1) raw[j] = ONCE ? __builtin_nontemporal_load(at) : *at;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1136,11 +1140,15 @@ int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, co
     return launch_pair_gemm<T, 1, 4, 4, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
 }
 
+constexpr int64_t L2_BYTES = 32 << 20;   // of the eight XCDs
+
 template <typename T, typename Y, bool BN = false>
-void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int cout, const void* bias, void* out, hipStream_t stream,
-                        const BnGelu& bn = BnGelu{}, const Ahead& ahead = Ahead{}) {
-    hipLaunchKernelGGL((pair_segment_sum_kernel<T, Y, BN>), dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream,
-                       (const Y*)y, row_ptr, n, cout, ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn, ahead);
+void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int64_t n_pairs, int cout, const void* bias, void* out,
+                        hipStream_t stream, const BnGelu& bn = BnGelu{}, const Ahead& ahead = Ahead{}) {
+    auto kern = n_pairs * cout * (int64_t)sizeof(Y) > L2_BYTES ? pair_segment_sum_kernel<T, Y, BN, true>
+                                                               : pair_segment_sum_kernel<T, Y, BN, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream, (const Y*)y, row_ptr, n, cout,
+                       ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn, ahead);
 }
 
 }  // namespace
@@ -1192,12 +1200,12 @@ int ptv3_conv_pairs_ahead(const void* feat, int dtype, int64_t n, int cin, int t
         if (n_pairs > 0)
             rc = dispatch_pairs<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        launch_segment_sum<_Float16, _Float16>(y, row_ptr, n, cout, bias, out, stream, BnGelu{}, ahead);
+        launch_segment_sum<_Float16, _Float16>(y, row_ptr, n, n_pairs, cout, bias, out, stream, BnGelu{}, ahead);
     } else {
         if (n_pairs > 0)
             rc = dispatch_pairs<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
-        launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, cout, bias, out, stream, BnGelu{}, ahead);
+        launch_segment_sum<__bf16, __bf16>(y, row_ptr, n, n_pairs, cout, bias, out, stream, BnGelu{}, ahead);
     }
     PTV3_RETURN_LAUNCH();
 }
@@ -1222,8 +1230,8 @@ int ptv3_conv_pairs_bn_gelu(const void* feat, int dtype, int64_t n, int cin, int
     const int rc = dtype == PTV3_F16 ? dispatch_pairs<_Float16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream)
                                      : dispatch_pairs<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
     if (rc != PTV3_OK) return rc;
-    if (dtype == PTV3_F16) launch_segment_sum<_Float16, _Float16, true>(y, row_ptr, n, cout, nullptr, out, stream, bn);
-    else launch_segment_sum<__bf16, __bf16, true>(y, row_ptr, n, cout, nullptr, out, stream, bn);
+    if (dtype == PTV3_F16) launch_segment_sum<_Float16, _Float16, true>(y, row_ptr, n, n_pairs, cout, nullptr, out, stream, bn);
+    else launch_segment_sum<__bf16, __bf16, true>(y, row_ptr, n, n_pairs, cout, nullptr, out, stream, bn);
     PTV3_RETURN_LAUNCH();
 }
 
@@ -1243,8 +1251,8 @@ extern "C" int ptv3_subm_conv_pairs_wide_fwd(const void* feat, int dtype, int64_
                            : dispatch_pairs_wide<__bf16>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
         if (rc != PTV3_OK) return rc;
     }
-    if (dtype == PTV3_F16) launch_segment_sum<_Float16, float>(y, row_ptr, n, cout, bias, out, stream);
-    else launch_segment_sum<__bf16, float>(y, row_ptr, n, cout, bias, out, stream);
+    if (dtype == PTV3_F16) launch_segment_sum<_Float16, float>(y, row_ptr, n, n_pairs, cout, bias, out, stream);
+    else launch_segment_sum<__bf16, float>(y, row_ptr, n, n_pairs, cout, bias, out, stream);
     PTV3_RETURN_LAUNCH();
 }
 
