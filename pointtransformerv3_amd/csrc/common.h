@@ -43,6 +43,15 @@ __device__ __forceinline__ int ptv3_job_of_block(const J* __restrict__ jobs, int
     return max(started - 1, 0);
 }
 
+// Rows that are read for the last time, or written for much later, go past the caches (the nontemporal hint) where they are more
+// than those hold: what the next kernels read stays there. Of less than that the last kernel's rows are still in the L2. The
+// choice is a template argument: the compiler makes one ordinary access of two behind a condition.
+constexpr int64_t PTV3_L2_BYTES = 32 << 20;   // of the eight XCDs
+template <bool ONCE, typename V> __device__ __forceinline__ V ptv3_read(const V* p) {
+    if constexpr (ONCE) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
 static inline size_t ptv3_align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // More than 64 KB of dynamic LDS has to be allowed per kernel, and the runtime keeps that attribute per device.

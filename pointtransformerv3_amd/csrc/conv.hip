@@ -969,8 +969,7 @@ __global__ __launch_bounds__(256) void pair_segment_sum_kernel(const Y* __restri
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             raw[j] = (v8){0, 0, 0, 0, 0, 0, 0, 0};
-            const v8* at = (const v8*)(src + (int64_t)j * cout);
-            if (s + j < s1) raw[j] = ONCE ? __builtin_nontemporal_load(at) : *at;
+            if (s + j < s1) raw[j] = ptv3_read<ONCE>((const v8*)(src + (int64_t)j * cout));
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1140,12 +1139,10 @@ int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, co
     return launch_pair_gemm<T, 1, 4, 4, float>(feat, cin, taps, n_pairs, tap_ptr, pair_in, pair_slot, weight, cout, y, stream);
 }
 
-constexpr int64_t L2_BYTES = 32 << 20;   // of the eight XCDs
-
 template <typename T, typename Y, bool BN = false>
 void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int64_t n_pairs, int cout, const void* bias, void* out,
                         hipStream_t stream, const BnGelu& bn = BnGelu{}, const Ahead& ahead = Ahead{}) {
-    auto kern = n_pairs * cout * (int64_t)sizeof(Y) > L2_BYTES ? pair_segment_sum_kernel<T, Y, BN, true>
+    auto kern = n_pairs * cout * (int64_t)sizeof(Y) > PTV3_L2_BYTES ? pair_segment_sum_kernel<T, Y, BN, true>
                                                                : pair_segment_sum_kernel<T, Y, BN, false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream, (const Y*)y, row_ptr, n, cout,
                        ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn, ahead);
