@@ -100,7 +100,9 @@ __device__ __forceinline__ void park_weight(T* __restrict__ dst, const Staged<PI
 template <typename T>
 __device__ __forceinline__ float vec_entry(const T* __restrict__ src, int at, float fill) { return src ? (float)src[at] : fill; }
 
-// 32 rows of C channels of two matrices, 16-byte pieces in lane order; rows past the end are zero
+// 32 rows of C channels of two matrices, 16-byte pieces in lane order; rows past the end are zero. Both halves of a block read their
+// rows for the last time, so these go past the caches (4 rooms of 100k voxels 9558 -> 9449 us with mlp_wide_kernel's, one of 1M
+// 25.6 -> 25.4 ms; a scan of 2k, whose rows the L2s hold, the same either way).
 template <typename T, int C, int IT>
 __device__ __forceinline__ void fetch_rows(const T* __restrict__ a, const T* __restrict__ b, int64_t row0, int64_t n, int lane,
                                            u32x4 (&xr)[IT], u32x4 (&rr)[IT]) {
@@ -112,8 +114,8 @@ __device__ __forceinline__ void fetch_rows(const T* __restrict__ a, const T* __r
         xr[it] = (u32x4){0, 0, 0, 0};
         rr[it] = (u32x4){0, 0, 0, 0};
         if (r < n) {
-            xr[it] = *(const u32x4*)(a + r * C + (pidx % PPR) * 8);
-            rr[it] = *(const u32x4*)(b + r * C + (pidx % PPR) * 8);
+            xr[it] = ptv3_read<true>((const u32x4*)(a + r * C + (pidx % PPR) * 8));
+            rr[it] = ptv3_read<true>((const u32x4*)(b + r * C + (pidx % PPR) * 8));
         }
     }
 }

@@ -207,15 +207,15 @@ __global__ __launch_bounds__(THREADS, MINW) void mlp_wide_kernel(
                         for (int q = 0; q < 4; ++q) hacc[a][rt][4 * g + q] = bias[q];
                 }
         };
-        // ---- x tile -> LDS
+        // ---- x tile -> LDS. A block's half reads its rows for the last time: past the caches, see fetch_rows in block.hip
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
             const int p = tid + i * THREADS;
             const int rr = p / PPR, pc = p % PPR;
             u32x4 v = {0, 0, 0, 0}, sh = {0, 0, 0, 0};
             if (row0 + rr < row_end) {
-                v = *(const u32x4*)(x + (row0 + rr) * C + pc * 8);
-                if (TAIL) sh = *(const u32x4*)(resid + (row0 + rr) * C + pc * 8);   // waits in LDS for the projection
+                v = ptv3_read<MODE != MLP_MODE>((const u32x4*)(x + (row0 + rr) * C + pc * 8));
+                if (TAIL) sh = ptv3_read<true>((const u32x4*)(resid + (row0 + rr) * C + pc * 8));   // waits in LDS for the projection
             }
             *(u32x4*)(xt + rr * XS + pc * 8) = v;
             if (TAIL) *(u32x4*)(sum_lds + rr * XS + pc * 8) = sh;
