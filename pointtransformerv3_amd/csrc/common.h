@@ -51,6 +51,10 @@ template <bool ONCE, typename V> __device__ __forceinline__ V ptv3_read(const V*
     if constexpr (ONCE) return __builtin_nontemporal_load(p);
     else return *p;
 }
+template <bool ONCE, typename V> __device__ __forceinline__ void ptv3_write(V* p, V v) {
+    if constexpr (ONCE) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
 
 static inline size_t ptv3_align256(size_t v) { return (v + 255) & ~(size_t)255; }
 

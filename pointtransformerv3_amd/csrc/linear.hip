@@ -161,7 +161,7 @@ __global__ __launch_bounds__(NW * PTV3_WAVE, (NW == 8 ? 2 : 1)) void linear_rows
                     const int pidx = it * PTV3_WAVE + lane;
                     const int64_t r = row0 + pidx / ppr_g;
                     pre[it] = (u32x4){0, 0, 0, 0};
-                    if (r < n) pre[it] = *(const u32x4*)(aux + r * nout + c0 + o0 + (pidx % ppr_g) * 8);
+                    if (r < n) pre[it] = ptv3_read<true>((const u32x4*)(aux + r * nout + c0 + o0 + (pidx % ppr_g) * 8));
                 }
             }
             u32x2 act[ACT == ACT_GELU_KEEP ? SW / 32 : 1][4];   // the activated values while the plain ones go out
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(NW * PTV3_WAVE, (NW == 8 ? 2 : 1)) void linear_rows
                                               H16<T>::hi(dw) * gelu_erf_grad(H16<T>::hi(hw)));
                     }
                 }
-                if (r < n) *(u32x4*)((ACT == ACT_GELU_KEEP ? aux : out) + r * nout + c0 + o0 + pc * 8) = o4;
+                if (r < n) ptv3_write<ACT == ACT_GELU_KEEP>((u32x4*)((ACT == ACT_GELU_KEEP ? aux : out) + r * nout + c0 + o0 + pc * 8), o4);
             }
             asm volatile("" ::: "memory");
             if (ACT == ACT_GELU_KEEP) {

@@ -15,6 +15,8 @@
 // next four steps (a whole tile) are in flight in a ring of registers that runs on across tile boundaries.
 // Bias and the exact GELU are applied on the accumulators; results are rounded to the storage type once and leave
 // as whole row segments (8 rows x 128 B per store) through the wave's own LDS rows.
+#include <type_traits>
+
 #include "lintile.h"
 #include "rowtile.h"
 
@@ -59,7 +61,7 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
     const int c0 = L.c0, row0 = L.row0, col = L.col, hf = L.hf, lane = L.lane, wave = L.wave, cout0 = L.cout0, nout = L.nout;
     const int64_t n = L.n;
     // acc[b][v]: output channel cout0 + c0 + b*32 + 8*(v/4) + 4*hf + v%4 of row row0 + col of the tile
-    auto store_rows = [&](T* dst) {   // the wave's staged 32 x 64 block as whole row segments
+    auto store_rows = [&](T* dst, auto once) {   // the wave's staged 32 x 64 block as whole row segments
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
@@ -73,7 +75,7 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
             }
             int64_t r = tile_row0 + row0 + orow;
             r = r < n ? r : n - 1;
-            *(u32x4*)(dst + r * nout + cout0 + c0 + opc * 8) = val;
+            ptv3_write<decltype(once)::value>((u32x4*)(dst + r * nout + cout0 + c0 + opc * 8), val);
         }
         asm volatile("" ::: "memory");
     };
@@ -95,13 +97,13 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
                     (u32x2){H16<T>::pack2(r[0], r[1]), H16<T>::pack2(r[2], r[3])};
                 if (ACT == ACT_GELU_KEEP) act[b][q] = (u32x2){H16<T>::pack2(a[0], a[1]), H16<T>::pack2(a[2], a[3])};
             }
-        store_rows(ACT == ACT_GELU_KEEP ? ln.out1 : out);
+        store_rows(ACT == ACT_GELU_KEEP ? ln.out1 : out, std::bool_constant<ACT == ACT_GELU_KEEP>{});
         if constexpr (ACT == ACT_GELU_KEEP) {
 #pragma unroll
             for (int b = 0; b < NT; ++b)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) *(u32x2*)(stage + col * LW_OSTRIDE + b * 32 + 8 * q + 4 * hf) = act[b][q];
-            store_rows(out);
+            store_rows(out, std::false_type{});
         }
     } else {
         // ---- the residual block through the staging rows into accumulator order
@@ -178,7 +180,7 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
                     (u32x2){H16<T>::pack2(val[b][4 * q] + sh[0], val[b][4 * q + 1] + sh[1]),
                             H16<T>::pack2(val[b][4 * q + 2] + sh[2], val[b][4 * q + 3] + sh[3])};
             }
-        store_rows(out);
+        store_rows(out, std::false_type{});
         row_stats(2, mean, rstd);
         const float* ga_l = p_lds + (LN == 3 ? 2 * LW_N : 0);
         const float* be_l = p_lds + (LN == 3 ? 3 * LW_N : LW_N);
@@ -194,7 +196,7 @@ __device__ __forceinline__ void lw_epilogue(f32x16 (&acc)[2], const u32x4* resv,
                 *(u32x2*)(stage + col * LW_OSTRIDE + b * 32 + 8 * q + 4 * hf) =
                     (u32x2){H16<T>::pack2(o[0], o[1]), H16<T>::pack2(o[2], o[3])};
             }
-        store_rows(ln.out1);
+        store_rows(ln.out1, std::false_type{});
     }
 }
 
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(LW_THREADS, 2) void linear_wide_kernel(
             for (int it = 0; it < 4; ++it) {
                 int64_t r = r0 + (int64_t)tile * LW_ROWS + row0 + it * 8 + (lane >> 3);
                 r = r < n ? r : n - 1;
-                resv[it] = *(const u32x4*)(ln.res + r * nout + cout0 + c0 + (lane & 7) * 8);
+                resv[it] = ptv3_read<ACT == ACT_GELU_GRAD>((const u32x4*)(ln.res + r * nout + cout0 + c0 + (lane & 7) * 8));
             }
         }
         f32x16 acc[NT];

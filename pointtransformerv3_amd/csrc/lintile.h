@@ -10,7 +10,9 @@ struct LinArgs {
     int k, nout, act;
     int row_tiles, col_tiles, order;            // filled in by the launch
     const void* resid;                          // ACT_NONE: added in fp32; may be out
-    void* aux;                                  // ACT_GELU_KEEP: the value in front of the GELU, out; ACT_GELU_GRAD: in
+    // ACT_GELU_KEEP: the value in front of the GELU, out; ACT_GELU_GRAD: in. Between the two lies the rest of the step: past the
+    // caches both ways (4 rooms of 100k voxels 38.0 -> 37.8 ms)
+    void* aux;
     const void *mean, *var, *gamma, *beta;      // ACT_BN, ACT_BN_GELU
     float bn_eps;
     int stats_f32;

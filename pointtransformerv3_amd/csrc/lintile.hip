@@ -79,7 +79,7 @@ __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, const LinP
     rows([&](float (&y)[8], int64_t at) {
         v8 keep, other;
         if (PRE) other = pre.other;
-        else if (ACT == ACT_GELU_GRAD) other = *(const v8*)((const T*)a.aux + at);
+        else if (ACT == ACT_GELU_GRAD) other = ptv3_read<true>((const v8*)((const T*)a.aux + at));
         else if (ACT == ACT_NONE && a.resid) other = *(const v8*)((const T*)a.resid + at);
         if (a.bias)
 #pragma unroll
@@ -98,7 +98,7 @@ __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int c, const LinP
 #pragma unroll
         for (int q = 0; q < 4; ++q) o[q] = H16<T>::pack2(y[2 * q], y[2 * q + 1]);
         *(u32x4*)((T*)a.out + at) = o;
-        if (ACT == ACT_GELU_KEEP) *(v8*)((T*)a.aux + at) = keep;
+        if (ACT == ACT_GELU_KEEP) ptv3_write<true>((v8*)((T*)a.aux + at), keep);
     });
 }
 template <typename T, bool PRE, typename F>
