@@ -31,6 +31,7 @@
 #include <hip/hip_fp16.h>
 
 #include "common.h"
+#include "bnact.h"
 #include "outer.h"
 
 namespace {
@@ -1205,18 +1206,11 @@ __global__ __launch_bounds__(256) void bn_finalize_kernel(AnyRows x, const float
                                                           float eps, float momentum, float* __restrict__ running_mean,
                                                           float* __restrict__ running_var, float* __restrict__ stats) {
     for (int ch = threadIdx.x; ch < c; ch += 256) {
-        const float pivot = load1_any(x.p, x.dtype, ch);
-        const float m1 = sums[ch] / (float)n;
-        const float var = fmaxf(sums[c + ch] / (float)n - m1 * m1, 0.f);
-        const float mean = pivot + m1;
-        stats[ch] = mean;
-        stats[c + ch] = rsqrtf(var + eps);
-        stats[2 * c + ch] = var;
-        if (running_mean) {
-            running_mean[ch] = (1.f - momentum) * running_mean[ch] + momentum * mean;
-            const float unbiased = n > 1 ? var * ((float)n / (float)(n - 1)) : var;
-            running_var[ch] = (1.f - momentum) * running_var[ch] + momentum * unbiased;
-        }
+        const BnMoments m = bn_moments(load1_any(x.p, x.dtype, ch), sums[ch], sums[c + ch], n);
+        stats[ch] = m.mean;
+        stats[c + ch] = rsqrtf(m.var + eps);
+        stats[2 * c + ch] = m.var;
+        if (running_mean) bn_running(m, n, momentum, running_mean + ch, running_var + ch);
     }
 }
 
@@ -1748,6 +1742,18 @@ extern "C" int ptv3_add_layer_norm_bwd(const void* sum, int sum_dtype, const voi
                              (hipStream_t)stream_);
 }
 
+int ptv3_batch_norm_sums(const void* x, int dtype, int64_t n, int c, float* sums, hipStream_t stream) {
+    const AnyRows xr = {x, dtype};
+#define PTV3_BNS(L)                                                                                                   \
+    if (c == 8 * L) {                                                                                                 \
+        hipLaunchKernelGGL((bn_stats_kernel<L>), dim3((unsigned)bn_grid(n, c)), dim3(BN_WAVES * PTV3_WAVE), 0, stream, xr, n, sums); \
+        PTV3_RETURN_LAUNCH();                                                                                         \
+    }
+    PTV3_BNS(4) PTV3_BNS(8) PTV3_BNS(16) PTV3_BNS(32) PTV3_BNS(64)
+#undef PTV3_BNS
+    return PTV3_ESHAPE;
+}
+
 extern "C" int ptv3_batch_norm_stats(const void* x, int dtype, int64_t n, int c, float eps, float momentum,
                                      float* running_mean, float* running_var, float* stats, float* workspace,
                                      void* stream_) {
@@ -1758,11 +1764,8 @@ extern "C" int ptv3_batch_norm_stats(const void* x, int dtype, int64_t n, int c,
     hipStream_t stream = (hipStream_t)stream_;
     const AnyRows xr = {x, dtype};
     hipLaunchKernelGGL(zero_kernel, dim3((unsigned)ptv3_ceil_div(2 * c, 256)), dim3(256), 0, stream, workspace, (int64_t)2 * c);
-#define PTV3_BNS(L)                                                                                                   \
-    if (c == 8 * L)                                                                                                   \
-        hipLaunchKernelGGL((bn_stats_kernel<L>), dim3((unsigned)bn_grid(n, c)), dim3(BN_WAVES * PTV3_WAVE), 0, stream, xr, n, workspace);
-    PTV3_BNS(4) PTV3_BNS(8) PTV3_BNS(16) PTV3_BNS(32) PTV3_BNS(64)
-#undef PTV3_BNS
+    const int rc = ptv3_batch_norm_sums(x, dtype, n, c, workspace, stream);
+    if (rc != PTV3_OK) return rc;
     hipLaunchKernelGGL(bn_finalize_kernel, dim3(1), dim3(256), 0, stream, xr, (const float*)workspace, n, c, eps, momentum,
                        running_mean, running_var, stats);
     PTV3_RETURN_LAUNCH();
@@ -1780,6 +1783,13 @@ extern "C" int ptv3_batch_norm_bwd(const void* x, int x_dtype, const void* dout,
     hipLaunchKernelGGL(zero_kernel, dim3((unsigned)ptv3_ceil_div(2 * c, 256)), dim3(256), 0, stream, dgamma_dbeta, (int64_t)2 * c);
     if (n == 0) PTV3_RETURN_LAUNCH();
     if (!x || !dout || !stats || !dx) return PTV3_EINVAL;
+    return ptv3_batch_norm_bwd_onto(x, x_dtype, dout, dout_dtype, stats, gamma, beta, param_dtype, n, c, gelu, batch_stats, dx, dx_dtype,
+                                    dgamma_dbeta, stream);
+}
+
+int ptv3_batch_norm_bwd_onto(const void* x, int x_dtype, const void* dout, int dout_dtype, const float* stats, const void* gamma,
+                             const void* beta, int param_dtype, int64_t n, int c, int gelu, int batch_stats, void* dx, int dx_dtype,
+                             float* dgamma_dbeta, hipStream_t stream) {
     const AnyRows xr = {x, x_dtype}, gr = {dout, dout_dtype}, ga = {gamma, param_dtype}, be = {beta, param_dtype};
     const AnyRowsOut out = {dx, dx_dtype};
     int rc = launch_bn_bwd<0>(xr, gr, stats, ga, be, n, c, gelu, batch_stats, dgamma_dbeta, out, stream);

@@ -69,6 +69,21 @@ template <typename T, int V> struct BnChannels {
     }
 };
 
+// A channel's mean and biased variance from the sums of bn_stats_kernel, which are around the first row's value
+struct BnMoments {
+    float mean, var;
+};
+__device__ __forceinline__ BnMoments bn_moments(float pivot, float s1, float s2, int64_t n) {
+    const float m1 = s1 / (float)n;
+    return BnMoments{pivot + m1, fmaxf(s2 / (float)n - m1 * m1, 0.f)};
+}
+// running averages follow (unbiased variance, as torch does)
+__device__ __forceinline__ void bn_running(BnMoments m, int64_t n, float momentum, float* mean, float* var) {
+    *mean = (1.f - momentum) * *mean + momentum * m.mean;
+    const float unbiased = n > 1 ? m.var * ((float)n / (float)(n - 1)) : m.var;
+    *var = (1.f - momentum) * *var + momentum * unbiased;
+}
+
 }  // namespace
 
 // ptv3_segment_reduce, BatchNorm, GELU. rows: (m, c) scratch, for shapes whose reduction has no such epilogue.

@@ -18,6 +18,7 @@
 #include <hip/hip_fp16.h>
 
 #include "bnact.h"
+#include "outer.h"
 #include "rownorm.h"
 
 namespace {
@@ -147,6 +148,43 @@ __global__ __launch_bounds__(256) void bn_act_kernel(const T* __restrict__ x, co
     store8(out + e * 8, v);
 }
 
+// The same in training (c <= 512): a work-group forms its channels' statistics from the sums, so that no launch of one work-group
+// stands between the sums and the rows; the first one leaves them, and the running averages, for later.
+template <typename T>
+__global__ __launch_bounds__(256) void bn_train_act_kernel(const T* __restrict__ x, const float* __restrict__ sums,
+                                                           const T* __restrict__ gamma, const T* __restrict__ beta, float eps,
+                                                           float momentum, float* __restrict__ running_mean,
+                                                           float* __restrict__ running_var, float* __restrict__ stats, int c, int64_t n,
+                                                           PieceDiv groups, T* __restrict__ out) {
+    __shared__ float mean_lds[512], rstd_lds[512];
+    for (int ch = threadIdx.x; ch < c; ch += 256) {
+        const BnMoments m = bn_moments((float)x[ch], sums[ch], sums[c + ch], n);
+        const float rstd = rsqrtf(m.var + eps);
+        mean_lds[ch] = m.mean;
+        rstd_lds[ch] = rstd;
+        if (blockIdx.x == 0) {
+            stats[ch] = m.mean;
+            stats[c + ch] = rstd;
+            stats[2 * c + ch] = m.var;
+            if (running_mean) bn_running(m, n, momentum, running_mean + ch, running_var + ch);
+        }
+    }
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, row = ptv3_row_of(e, groups);
+    const bool live = row < n;
+    const int ch = (int)(e - row * groups.count) * 8;
+    float v[8], g[8], b[8];
+    if (live) {
+        load8(x + e * 8, v);
+        load8(gamma + ch, g);
+        load8(beta + ch, b);
+    }
+    __syncthreads();
+    if (!live) return;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = gelu_exact(round_to<T>((v[i] - mean_lds[ch + i]) * rstd_lds[ch + i] * g[i] + b[i]));
+    store8(out + e * 8, v);
+}
+
 template <typename T, int MODE>
 void launch(const void* x, const void* res, const void* gamma, const void* beta, const void* gamma2,
             const void* beta2, const void* shift, int64_t n, int c, float eps, void* out0, void* out1,
@@ -239,5 +277,20 @@ extern "C" int ptv3_bn_act(const void* x, const void* running_mean, const void* 
     else if (dtype == PTV3_F16) PTV3_BN(_Float16);
     else PTV3_BN(__bf16);
 #undef PTV3_BN
+    PTV3_RETURN_LAUNCH();
+}
+
+int ptv3_batch_norm_gelu_train(const void* x, int dtype, int64_t n, int c, const float* sums, const void* gamma, const void* beta,
+                               float eps, float momentum, float* running_mean, float* running_var, float* stats, void* out,
+                               hipStream_t stream) {
+    if (c > 512 || c % 8 != 0 || (dtype != PTV3_F16 && dtype != PTV3_BF16)) return PTV3_ESHAPE;
+    const dim3 grid((unsigned)ptv3_ceil_div(n * (c / 8), 256));
+    const PieceDiv groups = ptv3_piece_div(c / 8);
+#define PTV3_BN_TRAIN(T)                                                                                             \
+    hipLaunchKernelGGL(bn_train_act_kernel<T>, grid, dim3(256), 0, stream, (const T*)x, sums, (const T*)gamma, (const T*)beta, eps, \
+                       momentum, running_mean, running_var, stats, c, n, groups, (T*)out)
+    if (dtype == PTV3_F16) PTV3_BN_TRAIN(_Float16);
+    else PTV3_BN_TRAIN(__bf16);
+#undef PTV3_BN_TRAIN
     PTV3_RETURN_LAUNCH();
 }

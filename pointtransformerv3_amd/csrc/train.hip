@@ -63,6 +63,15 @@ constexpr int MAX_BLOCKS = 256;
 constexpr size_t GROUP_BYTES = 64u << 20;
 constexpr int GROUP_LINEARS = 64, GROUP_CONVS = 16;
 
+__global__ __launch_bounds__(256) void zero_floats_kernel(float* __restrict__ out, int64_t count) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < count) out[i] = 0.f;
+}
+int zero_floats(float* out, int64_t count, hipStream_t stream) {
+    hipLaunchKernelGGL(zero_floats_kernel, dim3((unsigned)ptv3_ceil_div(count, 256)), dim3(256), 0, stream, out, count);
+    PTV3_RETURN_LAUNCH();
+}
+
 struct Run {
     const ptv3_train_net& net;
     const ptv3_level* lv;
@@ -217,13 +226,14 @@ struct Run {
         return PTV3_OK;
     }
 
-    int bn_gelu(const ptv3_train_bn& b, BnActs& a, int64_t n, int c, Space& scratch) {
-        const size_t mark = scratch.at;
-        float* ws = (float*)scratch.take(2 * (size_t)c * 4);
-        DO(ptv3_batch_norm_stats(a.x, dt, n, c, b.eps, b.momentum, b.running_mean, b.running_var, a.stats, ws, stream));
-        scratch.at = mark;
+    float* bn_sums = nullptr;   // zeroed sums of the layers to come
+    int bn_gelu(const ptv3_train_bn& b, BnActs& a, int64_t n, int c) {
         if (dry) return PTV3_OK;
-        return ptv3_bn_act(a.x, a.stats, a.stats + 2 * c, 1, b.g16, b.b16, dt, n, c, b.eps, 1, a.y, stream);
+        float* sums = bn_sums;
+        bn_sums += 2 * c;
+        TRY(ptv3_batch_norm_sums(a.x, dt, n, c, sums, hs));
+        return ptv3_batch_norm_gelu_train(a.x, dt, n, c, sums, b.g16, b.b16, b.eps, b.momentum, b.running_mean, b.running_var, a.stats,
+                                          a.y, hs);
     }
 
     // out: the block's rows in float, or null where only the half copy (out16) is read
@@ -274,10 +284,14 @@ struct Run {
         const int S = net.n_stages;
         const ptv3_level& v0 = lv[0];
         const int c0 = net.stage[0].channels;
+        int64_t count = 2 * c0;
+        for (int s = 0; s < S; ++s) count += 2 * (s > 0 ? net.stage[s].channels : 0) + 4 * (s < S - 1 ? net.stage[s].dec_channels : 0);
+        bn_sums = (float*)scratch.take((size_t)count * 4);
+        DO(zero_floats(bn_sums, count, hs));
         DO(ptv3_pad_rows(feat, feat_dt, v0.n, net.stem.cin, net.stem.cin_padded, stem_in, dt, stream));
         TRY(make_maps(scratch));
         TRY(conv_rows(0, 125, stem_in, net.stem.cin_padded, net.stem.w, nullptr, c0, stem_bn.x, scratch));
-        TRY(bn_gelu(net.stem.bn, stem_bn, v0.n, c0, scratch));
+        TRY(bn_gelu(net.stem.bn, stem_bn, v0.n, c0));
         const void* x = stem_bn.y;
         for (int s = 0; s < S; ++s) {
             const ptv3_train_stage& g = net.stage[s];
@@ -287,7 +301,7 @@ struct Run {
                            st[s].pool_in));
                 DO(ptv3_segment_reduce(st[s].pool_in, dt, up.n, g.channels, up.order, v.idx_ptr, v.n, g.pool_reduce, st[s].pooled,
                                         stream));
-                TRY(bn_gelu(g.pool_bn, st[s].pool_bn, v.n, g.channels, scratch));
+                TRY(bn_gelu(g.pool_bn, st[s].pool_bn, v.n, g.channels));
                 x = st[s].pool_bn.y;
             }
             TRY(stage_fwd(g.enc, st[s].enc, g.n_enc, s, x, nullptr, masks, scratch));
@@ -298,9 +312,9 @@ struct Run {
             const ptv3_level &v = lv[s], &below = lv[s + 1];
             const int c = g.dec_channels;
             TRY(linear(child, g.up.w, g.up.b, g.up.in, c, below.n, st[s].up_bn.x));
-            TRY(bn_gelu(g.up_bn, st[s].up_bn, below.n, c, scratch));
+            TRY(bn_gelu(g.up_bn, st[s].up_bn, below.n, c));
             TRY(linear(st[s].enc[g.n_enc - 1].out16, g.up_skip.w, g.up_skip.b, g.up_skip.in, c, v.n, st[s].skip_bn.x));
-            TRY(bn_gelu(g.up_skip_bn, st[s].skip_bn, v.n, c, scratch));
+            TRY(bn_gelu(g.up_skip_bn, st[s].skip_bn, v.n, c));
             DO(ptv3_unpool_add(st[s].skip_bn.y, st[s].up_bn.y, dt, v.n, c, below.cluster, below.n, st[s].up_sum, stream));
             // the first block's convolution reads the skip projection alone (model.py:746)
             TRY(stage_fwd(g.dec, st[s].dec, g.n_dec, s, st[s].up_sum, s ? nullptr : final_out, masks, scratch));
@@ -428,7 +442,7 @@ struct Run {
     }
     int bn_bwd(const ptv3_train_bn& b, const BnActs& a, int64_t n, int c, const void* dy, void* dx) {
         if (dry) return PTV3_OK;
-        return ptv3_batch_norm_bwd(a.x, dt, dy, dt, a.stats, b.g, b.b, PTV3_F32, n, c, 1, 1, dx, dt, grads + b.gg, stream);
+        return ptv3_batch_norm_bwd_onto(a.x, dt, dy, dt, a.stats, b.g, b.b, PTV3_F32, n, c, 1, 1, dx, dt, grads + b.gg, hs);
     }
 
     // d32, d16: gradient of the block's output in float and, times mask2, in half (in the group's arena). Leaves the
