@@ -50,6 +50,17 @@ def test_native_forward_equals_the_modules(dtype, amp, sizes, monkeypatch):
     assert torch.equal(got.sparse_conv_feat.features, want.feat)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_native_forward_with_weights_asked_for_ahead(dtype, monkeypatch):
+    """A level of 256 channels beyond the layers of few rows: the attention and the convolution's sum ask for the next kernel's
+    weights, which the modules' launches do not."""
+    from pointtransformerv3_amd import PointTransformerV3
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().to(dtype).to(DEV)
+    got, want = _both(model, _inputs(4, (40_000,), dtype, grid=0.02), monkeypatch)
+    assert got.feat.shape[0] > 30_000 and torch.equal(got.feat, want.feat)
+
+
 @pytest.mark.parametrize("reduce,stride,sizes", [("max", (2, 2, 2, 2), (5003, 61)), ("mean", (8, 2, 2, 2), (9000,)), ("min", (2, 2, 2, 2), (40,)),
                                                 ("sum", (4, 2, 2, 2), (3000, 500))])
 @pytest.mark.parametrize("dtype,stats", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32),

@@ -930,3 +930,27 @@ def test_conv_plan_inner_equals_direct_3x3x3(n, extent, nb):
     assert torch.equal(got.tap_ptr, ref.tap_ptr) and torch.equal(got.row_ptr, ref.row_ptr)
     assert torch.equal(got.pair_in[:got.n_pairs], ref.pair_in[:ref.n_pairs])
     assert torch.equal(got.pair_slot[:got.n_pairs], ref.pair_slot[:ref.n_pairs])
+
+
+@pytest.mark.parametrize("dtype,c", [(torch.float16, 256), (torch.bfloat16, 256), (torch.float32, 128)])
+@pytest.mark.parametrize("n", [65_536, 65_537])
+def test_product_rows_on_both_sides_of_what_the_l2_holds(dtype, c, n):
+    """32 MB of product rows and one row more, which is read past the caches: one tap whose pairs are (i, i), so that a voxel's
+    sum is one product row, rounded as stored and rounded again with the bias."""
+    from pointtransformerv3_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(n)
+    x, w, b = (torch.randn(*shape, generator=g).to(dtype).to(DEV) for shape in ((n, c), (c, 1, c), (c,)))
+    ids = torch.arange(n + 1, dtype=torch.int32, device=DEV)
+    tap_ptr = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    y, out = torch.empty((n, c), dtype=dtype, device=DEV), torch.empty((n, c), dtype=dtype, device=DEV)
+    _lib.check(lib.ptv3_subm_conv_pairs_fwd(x.data_ptr(), {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype], n, c, 1, n,
+                                            tap_ptr.data_ptr(), ids.data_ptr(), ids.data_ptr(), ids.data_ptr(), w.data_ptr(),
+                                            b.data_ptr(), c, y.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream),
+               "ptv3_subm_conv_pairs_fwd")
+    eps = {torch.float32: 2.0 ** -18, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    product = x.double().cpu() @ w.double().cpu()[:, 0].T
+    want = product + b.double().cpu()
+    # a rounding of the product, one of the sum, and float sums of c products of that size
+    bound = eps * (product.abs() + want.abs()) * 1.01 + 2.0 ** -20 * (x.double().cpu().norm(dim=1, keepdim=True) * w.double().cpu()[:, 0].norm(dim=1))
+    assert bool(((out.double().cpu() - want).abs() <= bound).all())
