@@ -753,7 +753,8 @@ const ptv3_level *ptv3_index_levels(const void *state);
  * LayerNorms of one eps, biases everywhere, BatchNorm + exact GELU behind stem, poolings and unpoolings. In half
  * precision stem_w has its input channels padded to a multiple of 16 (ptv3_pad_rows over the weight's rows), and the
  * packed copies are those of ptv3_subm_conv_pack_weight (conv_packed, 32 / 64 / 128 channels), ptv3_mlp_pack_weights_batch
- * (mlp_packed from 128 channels on, proj_packed and head_packed = xCPE Linear + qkv at 128 and 256).
+ * (mlp_packed from 128 channels on, proj_packed at 128 and 256, head_packed = xCPE Linear + qkv at
+ * 128 and, or NULL for the separate layers, at 256).
  * Level l needs the lists ptv3_conv_form names for its blocks' channels (float: pairs), level 0 also the 5x5x5 lists;
  * neighbour maps are made in the workspace where ptv3_conv_pair_form asks for them.
  * stage_out: NULL, or per stage a buffer for the encoder stage's rows (or NULL in it); out: the decoder's (n, channels)

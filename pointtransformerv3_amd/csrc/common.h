@@ -99,7 +99,8 @@ struct Ahead {
     uint32_t lines[2];   // of 128 bytes, each begun
 };
 static inline Ahead ptv3_ahead(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
-    return Ahead{{(const uint8_t*)a, (const uint8_t*)b}, {(uint32_t)ptv3_ceil_div(a_bytes, 128), (uint32_t)ptv3_ceil_div(b_bytes, 128)}};
+    return Ahead{{(const uint8_t*)a, (const uint8_t*)b},
+                 {a ? (uint32_t)ptv3_ceil_div(a_bytes, 128) : 0, b ? (uint32_t)ptv3_ceil_div(b_bytes, 128) : 0}};
 }
 // This work-group's share: the lines are dealt to the last AHEAD_GROUPS work-groups of each XCD, whose own traffic will not have
 // replaced them, at most four a thread. What comes back is used in ptv3_asked alone, at the kernel's end, and so waited for there.

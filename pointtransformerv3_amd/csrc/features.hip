@@ -131,13 +131,18 @@ int make_maps(Run& r) {
     return PTV3_OK;
 }
 
+// at 256 channels a caller may leave the packed copy out: the separate layers
+bool head_wide(const ptv3_block_w& b, int64_t n) {
+    return (b.channels == 128 || b.head_packed) && ptv3_block_head_wide_pays(n, b.channels);
+}
+
 int conv3(Run& r, const ptv3_block_w& b, int s, const void* x, void* out) {
     const int c = b.channels;
     const ptv3_level& v = r.lv[s];
     const int form = r.dt == PTV3_F32 ? 0 : ptv3_conv_form(v.n, v.n_pairs, c);
     if (form == 0) {
         Ahead ahead = {};   // what the first half streams through every work-group: 22.4 -> 19.9 us for 11.6k rows (see attention)
-        if (r.dt != PTV3_F32 && c == 256 && ptv3_block_head_wide_pays(v.n, c)) ahead = ptv3_ahead(b.head_packed, 8ll * c * c, nullptr, 0);
+        if (r.dt != PTV3_F32 && c == 256 && head_wide(b, v.n)) ahead = ptv3_ahead(b.head_packed, 8ll * c * c, nullptr, 0);
         return conv_rows(r, s, 27, x, c, b.conv_w, b.conv_b, c, out, ahead);
     }
     if (r.dry) return PTV3_OK;
@@ -176,7 +181,7 @@ int block_half(Run& r, const ptv3_block_w& b, int s, const void* xs, const void*
         if (c <= 64) {
             TRY(ptv3_block_head_fused(conv, x, b.cpe.w, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b, b.ln1.eps,
                                       b.qkv.w, b.qkv.b, r.dt, n, c, feat, qkv, r.stream));
-        } else if (ptv3_block_head_wide_pays(n, c)) {
+        } else if (head_wide(b, n)) {
             TRY(ptv3_block_head_wide(conv, x, b.head_packed, b.cpe.b, b.ln_cpe.g, b.ln_cpe.b, b.ln_cpe.eps, b.ln1.g, b.ln1.b,
                                      b.ln1.eps, b.qkv.b, r.dt, n, c, feat, qkv, r.stream));
         } else {

@@ -1,4 +1,6 @@
 """The natively queued inference forward against the same model's modules."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -59,6 +61,26 @@ def test_native_forward_with_weights_asked_for_ahead(dtype, monkeypatch):
     model = PointTransformerV3(**KW).eval().to(dtype).to(DEV)
     got, want = _both(model, _inputs(4, (40_000,), dtype, grid=0.02), monkeypatch)
     assert got.feat.shape[0] > 30_000 and torch.equal(got.feat, want.feat)
+
+
+def test_native_forward_without_the_packed_first_half_at_256_channels():
+    """A description without that copy takes the separate layers, as descriptions did before there was one: the same roundings,
+    sums in another order."""
+    from pointtransformerv3_amd import PointTransformerV3, native
+    torch.manual_seed(3)
+    model = PointTransformerV3(**KW).eval().half().to(DEV)
+    data = _inputs(4, (40_000,), torch.float16, grid=0.02)
+    outs = []
+    with torch.inference_mode():
+        for drop in (False, True):
+            torch.manual_seed(9)
+            outs.append(model(dict(data)).feat.float())
+            engine = native.engine_for(model, data)
+            left_out = [b for a in engine._keep if isinstance(a, ctypes.Array) and a._type_ is native._Block for b in a if b.channels == 256]
+            assert left_out and all(bool(b.head_packed) != drop for b in left_out)
+            for b in left_out:
+                b.head_packed = None
+    assert rel_err(outs[1], outs[0].cpu()) < 2e-2
 
 
 @pytest.mark.parametrize("reduce,stride,sizes", [("max", (2, 2, 2, 2), (5003, 61)), ("mean", (8, 2, 2, 2), (9000,)), ("min", (2, 2, 2, 2), (40,)),
