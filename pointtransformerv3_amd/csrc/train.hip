@@ -67,6 +67,23 @@ __global__ __launch_bounds__(256) void zero_floats_kernel(float* __restrict__ ou
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < count) out[i] = 0.f;
 }
+// the BatchNorms' places in the gradients, which their backward adds onto: a work-group each
+struct BnPlaces {
+    static constexpr int MAX = 1 + 3 * PTV3_MAX_LEVELS;
+    int64_t at[MAX];
+    int floats[MAX], count;
+    void add(const ptv3_train_bn& b, int c) {
+        at[count] = b.gg;
+        floats[count++] = 2 * c;
+    }
+};
+__global__ __launch_bounds__(256) void zero_places_kernel(float* __restrict__ base, BnPlaces places) {
+    for (int i = threadIdx.x; i < places.floats[blockIdx.x]; i += 256) base[places.at[blockIdx.x] + i] = 0.f;
+}
+int zero_places(float* base, const BnPlaces& places, hipStream_t stream) {
+    hipLaunchKernelGGL(zero_places_kernel, dim3((unsigned)places.count), dim3(256), 0, stream, base, places);
+    PTV3_RETURN_LAUNCH();
+}
 int zero_floats(float* out, int64_t count, hipStream_t stream) {
     hipLaunchKernelGGL(zero_floats_kernel, dim3((unsigned)ptv3_ceil_div(count, 256)), dim3(256), 0, stream, out, count);
     PTV3_RETURN_LAUNCH();
@@ -517,6 +534,17 @@ struct Run {
     int backward(const void* dout, int dout_dt, const void* const* masks, Space& scratch) {
         const int S = net.n_stages;
         DO(ptv3_zero_ranges(grads, net.zero, net.n_zero, net.zero_blocks, stream));
+        BnPlaces places = {};
+        places.add(net.stem.bn, net.stage[0].channels);
+        for (int s = 0; s < S; ++s) {
+            const ptv3_train_stage& g = net.stage[s];
+            if (s > 0) places.add(g.pool_bn, g.channels);
+            if (s < S - 1) {
+                places.add(g.up_bn, g.dec_channels);
+                places.add(g.up_skip_bn, g.dec_channels);
+            }
+        }
+        DO(zero_places(grads, places, hs));
         // gradients of the encoder stages' rows from the skip projections and the poolings (half)
         void *from_skip[PTV3_MAX_LEVELS] = {}, *from_pool[PTV3_MAX_LEVELS] = {}, *from_up[PTV3_MAX_LEVELS] = {};
         for (int s = 0; s < S; ++s) {

@@ -129,7 +129,6 @@ class TrainEngine(native.Copies):
         native.check_batch_norm(m, c)
         gg, gb = self._at(m.weight), self._at(m.bias)   # the kernel writes both, one behind the other
         assert gb == gg + c
-        self._zero.append((gg, 2 * c))
         self.read_back += [m.weight, m.bias]
         return _Bn(m.weight.data_ptr(), m.bias.data_ptr(), self._copy(m.weight), self._copy(m.bias), m.running_mean.data_ptr(),
                    m.running_var.data_ptr(), m.eps, 0.0, gg)
