@@ -349,7 +349,7 @@ struct Run {
     // turn; a group of blocks begins with a wait for the group before last, and ends when it holds GROUP_BYTES.
     hipStream_t side = nullptr;
     hipEvent_t ready = nullptr, done[2] = {};
-    bool busy[2] = {}, closed = true;
+    bool busy[2] = {}, unmarked = false, closed = true;   // unmarked: work on the side that no event stands behind
     int turn = 0;
     Space arenas[2] = {Space(nullptr), Space(nullptr)};
     LinearGrad linears[GROUP_LINEARS];
@@ -370,19 +370,26 @@ struct Run {
         side = e == hipSuccess ? (hipStream_t)net.side : nullptr;
         return (int)e;
     }
-    // `stream` goes on behind everything queued on the side
-    int join() {
-        hipError_t e = hipSuccess;
-        for (int i = 0; i < 2; ++i) {
-            if (!busy[i]) continue;
-            busy[i] = false;
-            const hipError_t w = hipStreamWaitEvent(hs, done[i], 0);
-            e = e == hipSuccess ? w : e;
-        }
+    // `stream` goes on behind the last group of arena i, which counts as busy until that is so
+    int wait_for(int i) {
+        if (!busy[i]) return PTV3_OK;
+        const hipError_t e = hipStreamWaitEvent(hs, done[i], 0);
+        busy[i] = e != hipSuccess;
         return (int)e;
     }
-    int close_side() {   // also where a launch has failed: the caller's buffers are free again behind this call's work
-        const int rc = join();
+    // `stream` goes on behind everything queued on the side
+    int join() {
+        const int first = wait_for(0), second = wait_for(1);
+        return first ? first : second;
+    }
+    // Also where a call has failed: the caller's buffers are free again behind this call's work. Where no event says when the
+    // side is through with them, the host waits for it.
+    int close_side() {
+        int rc = join();
+        if (unmarked || busy[0] || busy[1]) {
+            const int waited = (int)hipStreamSynchronize(side);
+            rc = rc ? rc : waited;
+        }
         for (int i = 0; i < 2; ++i)
             if (done[i]) (void)hipEventDestroy(done[i]);
         if (ready) (void)hipEventDestroy(ready);
@@ -394,10 +401,7 @@ struct Run {
             closed = false;
             turn ^= 1;
             arenas[turn].at = 0;
-            if (busy[turn]) {
-                busy[turn] = false;
-                TRY((int)hipStreamWaitEvent(hs, done[turn], 0));
-            }
+            TRY(wait_for(turn));
         }
         *arena = &arenas[turn];
         return PTV3_OK;
@@ -415,11 +419,13 @@ struct Run {
             TRY((int)hipEventRecord(ready, hs));
             TRY((int)hipStreamWaitEvent(side, ready, 0));
         }
+        unmarked = beside;
         int rc = launch_wgrads(arenas[turn], beside ? side : hs);
         n_linears = n_convs = 0;
         if (beside) {
             const int rec = (int)hipEventRecord(done[turn], side);
-            busy[turn] = rec == PTV3_OK;
+            unmarked = rec != PTV3_OK;
+            busy[turn] = !unmarked;
             rc = rc ? rc : rec;
         }
         return rc;
