@@ -852,7 +852,7 @@ typedef struct ptv3_train_net {
     float max_pair_density, reserved2;        /* ptv3_conv_pair_form */
     ptv3_train_stem stem;
     const ptv3_zero_range *zero;              /* device array */
-    int32_t n_zero, reserved;
+    int32_t n_zero, has_side;                 /* has_side 0: the description ends in front of `side`, which is not read */
     int64_t zero_blocks;
     ptv3_train_stage stage[PTV3_MAX_LEVELS];
     void *side;                               /* stream for the weight gradients of the backward (same device, any but its own); null: none */

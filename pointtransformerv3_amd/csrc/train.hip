@@ -364,7 +364,8 @@ struct Run {
     int n_convs = 0;
 
     int open_side() {
-        if (!net.side || (hipStream_t)net.side == hs) return PTV3_OK;
+        // descriptions of callers that do not know the field end in front of it, with a zero where the flag is
+        if (!net.has_side || !net.side || (hipStream_t)net.side == hs) return PTV3_OK;
         hipError_t e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
         for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
         side = e == hipSuccess ? (hipStream_t)net.side : nullptr;

@@ -56,7 +56,7 @@ class _Stem(ctypes.Structure):
 class _Net(ctypes.Structure):
     _fields_ = [("dtype", _i32), ("n_stages", _i32), ("patch", _i32 * levels.MAX_LEVELS),
                 ("max_pair_density", _f32), ("reserved2", _f32), ("stem", _Stem), ("zero", _ptr),
-                ("n_zero", _i32), ("reserved", _i32), ("zero_blocks", _i64), ("stage", _Stage * levels.MAX_LEVELS), ("side", _ptr)]
+                ("n_zero", _i32), ("has_side", _i32), ("zero_blocks", _i64), ("stage", _Stage * levels.MAX_LEVELS), ("side", _ptr)]
 
 
 class TrainEngine(native.Copies):
@@ -84,7 +84,7 @@ class TrainEngine(native.Copies):
         self._finish()
         # the weight gradients' stream; whatever is queued on it the backward's own stream waits for before the call returns
         self.side = torch.cuda.Stream(self.device)
-        self.net.side = self.side.cuda_stream
+        self.net.has_side, self.net.side = 1, self.side.cuda_stream
         self.batches = [m.num_batches_tracked for m in self.structure.modules
                         if isinstance(m, nn.BatchNorm1d) and m.num_batches_tracked is not None]
 

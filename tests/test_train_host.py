@@ -40,3 +40,33 @@ for op in ("create", "record", "wait"):
         assert joined(), (op, nth, [c for c in calls() if c[0] != "launch"])
         assert sum(c[0] == "create" and not c[3] for c in calls()) == sum(c[0] == "destroy" for c in calls())
 ''', tmp_path)
+
+
+def test_a_description_without_the_second_stream_is_not_read_past_its_end(tmp_path):
+    """A caller built before the field was there hands over a description that ends in front of it, here at the end of what
+    may be read."""
+    hip_stub.run(r'''
+import mmap
+from train_description import Step
+from pointtransformerv3_amd import native_train as t
+step = Step()
+step.net.has_side = 0
+size, known = step.sizes(lib)[2], t._Net.side.offset
+assert known == ctypes.sizeof(t._Net) - 8 and known % 8 == 0
+libc, page = ctypes.CDLL(None, use_errno=True), mmap.PAGESIZE
+pages = -(-known // page)
+area = mmap.mmap(-1, (pages + 1) * page)
+base = ctypes.addressof(ctypes.c_char.from_buffer(area))
+libc.mprotect.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+assert libc.mprotect(base + pages * page, page, 0) == 0
+at = base + pages * page - known
+ctypes.memmove(at, ctypes.addressof(step.net), known)
+clear()
+assert step.backward(lib, 0x100, size, net=at) == 0
+assert {a for op, a, b, failed in calls() if op == "launch"} == {0x100}
+assert not [c for c in calls() if c[0] in ("create", "record", "wait")]
+assert step.sizes(lib)[2] == size
+import os
+sys.stdout.flush()
+os._exit(0)   # the area is never unmapped: it is half protected
+''', tmp_path)

@@ -22,7 +22,7 @@ class Step:
 
     def __init__(self, points=(60_000, 40_000, 12_000), widths=(32, 64, 128)):
         bn = t._Bn(AT, AT, AT, AT, AT, AT, 1e-3, 0.1, 0)
-        self.net = net = t._Net(dtype=1, n_stages=len(points), max_pair_density=16.0, zero=AT, n_zero=1, zero_blocks=1,
+        self.net = net = t._Net(dtype=1, n_stages=len(points), max_pair_density=16.0, zero=AT, n_zero=1, zero_blocks=1, has_side=1,
                                 stem=t._Stem(AT, 6, 16, 0, bn))
         self.levels = (levels.Level * len(points))()
         self.keep, self.blocks = [], 0
