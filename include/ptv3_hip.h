@@ -173,7 +173,7 @@ int ptv3_patch_attn_fwd_lse(const void *qkv, int dtype, int64_t n_rows, int chan
  * every element written. Filler slots take no gradient as queries; as keys their share is added to
  * the row they repeat. n_pad = cu_seqlens[n_seq], the number of slots. lse: what ptv3_patch_attn_fwd_lse
  * wrote for the same inputs (fp16 / bf16 only), or NULL to have it recomputed. dropout_p, dropout_seed: as
- * given to the forward call. */
+ * given to the forward call. The workspace's size follows from the arguments alone, whatever the current device. */
 size_t ptv3_patch_attn_bwd_workspace_bytes(int dtype, int64_t n_pad, int channels, int heads);
 int ptv3_patch_attn_bwd(const void *qkv, const void *out, const void *dout, int dtype, int64_t n_rows,
                         int channels, int heads, const int32_t *slot_src, const int32_t *slot_dst,

@@ -31,6 +31,7 @@ constexpr int BWQ_WAVES = BWQ_THREADS / PTV3_WAVE;
 constexpr int BOTH_KEYS = 1024;     // both-sides kernel: the longest sequence, its queries in LDS
 constexpr int BOTH_WAVES = 8;
 constexpr int BOTH_PARTS = 4;       // at most as many work-groups share an item
+constexpr int BOTH_ROUND = 256;     // work-groups whose shares of dQ a workspace holds: a round of the whole MI355X
 constexpr float LN2 = 0.6931471805599453f;
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -1055,9 +1056,10 @@ BwdWs carve(void* base, int dtype, int64_t n_pad, int channels, int heads) {
     off += ptv3_align256((size_t)n_pad * heads * sizeof(float));
     w.fill = (char*)base + off;
     off += ptv3_align256((size_t)n_pad * 2 * channels * elt);
-    // a shared item's parts are at most one round of work-groups; the first one's sequence may have heads that are not shared
+    // A shared item's parts are at most one round of work-groups; the first one's sequence may have heads that are not shared.
+    // The size goes by the arguments alone, as the caller may ask for it on another device than the one it launches on
     w.dq = (float*)((char*)base + off);
-    const size_t round = ((size_t)ptv3_cus() + (size_t)BOTH_PARTS * heads) * BOTH_KEYS * HD, all = (size_t)BOTH_PARTS * n_pad * channels;
+    const size_t round = ((size_t)BOTH_ROUND + (size_t)BOTH_PARTS * heads) * BOTH_KEYS * HD, all = (size_t)BOTH_PARTS * n_pad * channels;
     w.dq_bytes = dtype == PTV3_F32 ? 0 : (round < all ? round : all) * sizeof(float);
     off += ptv3_align256(w.dq_bytes);
     w.bytes = off;
@@ -1111,8 +1113,11 @@ int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
         // by two 55.0, whole 75.3), 92 76.8 -> 56.7, 120 84.9 -> 59.0, 64 48.6 -> 44.9, 792 (three rounds and 24) 298 -> 295
         // (whole 325); 128 of 500 35.6 -> 27.1; 400 of 200 44.9 -> 19.2; 64 of 320 17.4 -> 19.0, but with a launch less
         const int most = g.max_seqlen <= BOTH_KEYS / 4 ? 1 : g.max_seqlen <= BOTH_KEYS / 2 ? 2 : BOTH_PARTS;
+        // slots of the sequences from the first shared item's on
+        const int64_t stride = std::min(g.n_pad, (g.n_seq - (total - rem) / g.heads) * g.max_seqlen);
+        auto held = [&](int parts) { return (size_t)stride * parts * g.channels * sizeof(float) <= ws.dq_bytes; };
         int parts = 1;
-        while (parts < most && rem * parts * 2 <= slots) parts *= 2;
+        while (parts < most && rem * parts * 2 <= slots && held(parts * 2)) parts *= 2;
         const int64_t first = parts == 1 ? total : total - rem;
         const BothParts whole = {nullptr, 0, 0, 1};
         int rc = PTV3_OK;
@@ -1122,9 +1127,7 @@ int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
                              : launch_both<T, 8, BOTH_KEYS, false>(g, ws, first, whole);
         if (rc != PTV3_OK) return rc;
         if (first < total) {
-            // slots of the sequences from the first shared item's on
-            shared = {ws.dq, std::min(g.n_pad, (g.n_seq - first / g.heads) * g.max_seqlen), (int)first, parts};
-            if ((size_t)shared.stride * parts * g.channels * sizeof(float) > ws.dq_bytes) return PTV3_EWORKSPACE;
+            shared = {ws.dq, stride, (int)first, parts};
             rc = most == 2 ? launch_both<T, 2, BOTH_KEYS / 2, false>(g, ws, total - first, shared)
                  : parts == 2 ? launch_both<T, 4, BOTH_KEYS, false>(g, ws, total - first, shared)
                               : launch_both<T, 2, BOTH_KEYS, false>(g, ws, total - first, shared);

@@ -36,7 +36,7 @@ int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** stream) {
 }
 int hipGetLastError(void) { return 0; }
 int hipPeekAtLastError(void) { return 0; }
-int hipGetDevice(int* d) { *d = 0; return 0; }
+int hipGetDevice(int* d) { *d = hip_cus / 8 % 64; return 0; }   /* one device a number of CUs: the library asks each once */
 int hipDeviceGetAttribute(int* v, int attr, int d) { *v = hip_cus; return 0; }
 int hipFuncSetAttribute(const void* f, int attr, int v) { return 0; }
 int hipEventCreateWithFlags(void** e, unsigned flags) {
