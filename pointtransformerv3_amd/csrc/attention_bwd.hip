@@ -639,8 +639,12 @@ __global__ __launch_bounds__(BOTH_WAVES * PTV3_WAVE) void attn_bwd_both_kernel(
         qt = columns(q_lds + block * 32 * 32 + lane * 8);
         gt = columns(do_lds + block * 32 * 32 + lane * 8);
     };
-    // blocks that are under way together, of those that are left; whole rings end within QUERIES
-    auto ring_of = [](int left) { return QUERIES < BOTH_KEYS ? WAVES : left > 24 ? 32 : left > 8 ? 16 : 8; };
+    // Blocks that are under way together, of those that are left; whole rings end within QUERIES. A step in which a wave has no
+    // block costs as much as one in which the others wait for it; with 128 keys a wave several short rings with few such steps
+    // are the faster from there on: 200 items of 795, 859 and 891 slots 71.4 -> 68.4, 72.3 -> 69.9 and 73.6 -> 70.9 us, of 379
+    // 28.1 -> 27.5. With fewer keys a step is short and the barriers between rings are what counts (60 of 795: 37.9, 40.3 that way).
+    constexpr int RING32 = KG == 8 ? 28 : 24, RING16 = KG == 8 ? 12 : 8;
+    auto ring_of = [](int left) { return QUERIES < BOTH_KEYS ? WAVES : left > RING32 ? 32 : left > RING16 ? 16 : 8; };
     int ring = ring_of(blocks);
     fetch_scores(wave * (ring / WAVES));
     fetch_sums(wave * (ring / WAVES));

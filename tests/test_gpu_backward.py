@@ -205,7 +205,7 @@ def test_attention_backward_items_shared_by_work_groups(dtype, lens, heads):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("blocks", [(32, 31, 25), (24, 17, 16), (9, 8, 1), (32, 24, 16, 9, 8)])
+@pytest.mark.parametrize("blocks", [(32, 31, 25), (24, 17, 16), (9, 8, 1), (32, 24, 16, 9, 8), (29, 28, 25), (28, 13, 12)])
 @pytest.mark.parametrize("times,heads", [(2, 3), (8, 4), (15, 3)])   # shared by four, by two, whole
 def test_attention_backward_rounds_of_query_blocks(dtype, blocks, times, heads):
     """Sequences at the edges of the rounds in which the waves take 32 queries at a time: the same checks."""
