@@ -16,7 +16,7 @@
 //   2. keys: Q, dO (rows), Q^T, dO^T (transposed), -lse and -D in LDS; per 32-key tile
 //      dV^T += dO^T P and dK^T += Q^T dS over all queries.
 // Where the forward kept the log-sum-exps and sequences are no longer than 1024 slots, one kernel does both
-// (attn_bwd_both_kernel); with attention dropout, only where it is the faster one.
+// (attn_bwd_both_kernel), save for a few items of short sequences; with attention dropout, only where it is the faster one.
 // fp32: one thread per query / per key, operands staged through LDS in chunks.
 #include <algorithm>
 
@@ -1098,6 +1098,24 @@ int launch_both(const HalfBwd& g, const BwdWs& ws, int64_t items, const BothPart
     PTV3_RETURN_LAUNCH();
 }
 
+// Whether the items beyond the last full round (where sequences of up to 512 slots are the longest: all) are left to the two
+// kernels, which cut them into ranges, instead of the both-sides kernel, which shares them. `mean` slots a sequence: where that
+// is much shorter than the longest sequence allowed, work-groups that share an item are left without keys or with few, and their
+// steps are all latency. us, two kernels / shared, items x mean length. Up to 1024 slots: 64 x 320 16.8 / 22.4, 64 x 513 28.7 /
+// 30.4, 60 x 571 29.8 / 30.4, 60 x 603 32.0 / 30.4; 32 x 640 27.7 / 28.8, 16 x 700 27.7 / 28.4; 76 x 700 37.5 / 39.3, 84 x 768
+// 40.7 / 40.8; 120 x 160 14.1 / 14.6, x 200 16.7 / 15.7, x 257 21.2 / 22.7, x 384 26.6 / 26.5, x 450 32.1 / 28.6; a round and 64 x
+// 384 47.7 / 50.1, x 640 84.0 / 81.3. Up to 512: 64 x 320 16.8 / 18.2, 64 x 360 18.9 / 18.9, 96 x 320 21.5 / 19.2, a round and 8 x
+// 320 33.7 / 36.0, a round and 16 x 360 40 / 38.
+bool two_kernels_pay(int most, int64_t total, int64_t rem, int slots, int64_t mean) {
+    if (rem == 0) return false;
+    if (most == BOTH_PARTS) {
+        if (rem * 4 <= slots) return mean <= (rem * 8 <= slots ? 704 : 576);
+        if (rem * 3 <= slots) return mean <= 768;
+        return rem * 2 <= slots && (mean <= 160 || (mean > 256 && mean <= 384));
+    }
+    return most == 2 && rem * 4 <= slots && total <= slots + rem && mean > 256 && mean <= (total > slots ? 320 : 384);
+}
+
 template <typename T>
 int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
     const int lds_keys = (int)((g.max_seqlen + 63) & ~63ll);
@@ -1110,53 +1128,61 @@ int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
     const int slots = ptv3_cus();
     const int64_t total = g.n_seq * g.heads, rem = total % slots;
     BothParts shared = {ws.dq, 0, (int)total, 1};
+    // The two kernels cut the items beyond the last full round into ranges of tiles when that shortens the round (each range
+    // stages the sequence again, about 0.15 of an item)
+    int64_t full = total - rem, split = 1;
+    double best = 1.0;
+    if (rem != 0)
+        for (int64_t sp = 2; sp <= 4; ++sp) {
+            const double cost = (double)((rem * sp + slots - 1) / slots) * (1.0 / (double)sp + 0.15);
+            if (cost < best - 1e-9) { best = cost; split = sp; }
+        }
+    int64_t first = 0;   // items that are left to the two kernels begin here
     if (g.lse && !dropping && g.max_seqlen <= BOTH_KEYS) {
         // The both-sides kernel forms the scores once and takes sequences of up to 256, 512 and 1024 slots with 32, 64 and
         // 128 keys a wave. Items that do not fill a round of CUs are shared by two or four work-groups, as many as the round has
         // room for: more would start a second round. us, two kernels -> shared: 60 items of 1024 slots 55.4 -> 46.6 (by four;
         // by two 55.0, whole 75.3), 92 76.8 -> 56.7, 120 84.9 -> 59.0, 64 48.6 -> 44.9, 792 (three rounds and 24) 298 -> 295
-        // (whole 325); 128 of 500 35.6 -> 27.1; 400 of 200 44.9 -> 19.2; 64 of 320 17.4 -> 19.0, but with a launch less
+        // (whole 325); 128 of 500 35.6 -> 27.1; 400 of 200 44.9 -> 19.2
         const int most = g.max_seqlen <= BOTH_KEYS / 4 ? 1 : g.max_seqlen <= BOTH_KEYS / 2 ? 2 : BOTH_PARTS;
+        const int64_t mean = g.n_pad / g.n_seq;
+        const bool two = two_kernels_pay(most, total, rem, slots, mean);
         // slots of the sequences from the first shared item's on
         const int64_t stride = std::min(g.n_pad, (g.n_seq - (total - rem) / g.heads) * g.max_seqlen);
         auto held = [&](int parts) { return (size_t)stride * parts * g.channels * sizeof(float) <= ws.dq_bytes; };
+        // a work-group of up to 512 slots has 256 keys where it shares its item: none are left for the second of a short one
+        // (64 of 200 12.7 -> 11.8 us, 288 of 40 17.3 -> 15.2)
+        const int limit = two || (most == 2 && mean <= 256) ? 1 : most;
         int parts = 1;
-        while (parts < most && rem * parts * 2 <= slots && held(parts * 2)) parts *= 2;
-        const int64_t first = parts == 1 ? total : total - rem;
-        const BothParts whole = {nullptr, 0, 0, 1};
+        while (parts < limit && rem * parts * 2 <= slots && held(parts * 2)) parts *= 2;
+        const int64_t whole = two ? (most == 2 ? 0 : total - rem) : parts == 1 ? total : total - rem;
+        const BothParts alone = {nullptr, 0, 0, 1};
         int rc = PTV3_OK;
-        if (first > 0)
-            rc = most == 1 ? launch_both<T, 2, BOTH_KEYS / 4, false>(g, ws, first, whole)
-                 : most == 2 ? launch_both<T, 4, BOTH_KEYS / 2, false>(g, ws, first, whole)
-                             : launch_both<T, 8, BOTH_KEYS, false>(g, ws, first, whole);
+        if (whole > 0)
+            rc = most == 1 ? launch_both<T, 2, BOTH_KEYS / 4, false>(g, ws, whole, alone)
+                 : most == 2 ? launch_both<T, 4, BOTH_KEYS / 2, false>(g, ws, whole, alone)
+                             : launch_both<T, 8, BOTH_KEYS, false>(g, ws, whole, alone);
         if (rc != PTV3_OK) return rc;
-        if (first < total) {
-            shared = {ws.dq, stride, (int)first, parts};
-            rc = most == 2 ? launch_both<T, 2, BOTH_KEYS / 2, false>(g, ws, total - first, shared)
-                 : parts == 2 ? launch_both<T, 4, BOTH_KEYS, false>(g, ws, total - first, shared)
-                              : launch_both<T, 2, BOTH_KEYS, false>(g, ws, total - first, shared);
+        if (!two && whole < total) {
+            shared = {ws.dq, stride, (int)whole, parts};
+            rc = most == 2 ? launch_both<T, 2, BOTH_KEYS / 2, false>(g, ws, total - whole, shared)
+                 : parts == 2 ? launch_both<T, 4, BOTH_KEYS, false>(g, ws, total - whole, shared)
+                              : launch_both<T, 2, BOTH_KEYS, false>(g, ws, total - whole, shared);
             if (rc != PTV3_OK) return rc;
         }
-    } else {
-        // the items beyond the last full round are cut into ranges of
-        // tiles when that shortens the round (each range stages the sequence again, about 0.15 of an item)
-        int64_t full = total - rem, split = 1;
-        double best = 1.0;
-        if (rem != 0)
-            for (int64_t sp = 2; sp <= 4; ++sp) {
-                const double cost = (double)((rem * sp + slots - 1) / slots) * (1.0 / (double)sp + 0.15);
-                if (cost < best - 1e-9) { best = cost; split = sp; }
-            }
+        first = two ? whole : total;
+    } else if (g.lse && g.max_seqlen <= BOTH_KEYS && g.max_seqlen > BOTH_KEYS / 2) {
         // With dropout the both-sides kernel takes whole items: 0.78 of the time of the two kernels (84 against 107 us for 240
         // items of 1024 slots), so a last round that their ranges bring below 0.7 is left to them, as are sequences that would
         // leave half of its waves without keys (1600 items of 200 slots: 109 against 104 us; 800 of 700 slots: 199 against 214).
-        int64_t first = 0;
-        if (g.lse && g.max_seqlen <= BOTH_KEYS && g.max_seqlen > BOTH_KEYS / 2) first = rem == 0 || best > 0.7 ? total : full;
-        if (split == 1 || first == total) full = total;
+        first = rem == 0 || best > 0.7 ? total : full;
         if (first > 0) {
             const int rc = launch_both<T, 8, BOTH_KEYS, true>(g, ws, first, BothParts{nullptr, 0, 0, 1});
             if (rc != PTV3_OK) return rc;
         }
+    }
+    if (first < total) {
+        if (split == 1) full = total;
         auto kq = dropping ? (g.lse ? attn_bwd_q_kernel<T, true, true> : attn_bwd_q_kernel<T, false, true>)
                            : (g.lse ? attn_bwd_q_kernel<T, true, false> : attn_bwd_q_kernel<T, false, false>);
         float* lse_buf = g.lse ? g.lse : ws.lse;
@@ -1164,15 +1190,13 @@ int launch_half_bwd(const HalfBwd& g, const BwdWs& ws) {
         static LdsGrant grant_q[4], grant_kv[2];   // per kernel variant and device
         if (const int rc_ = ptv3_allow_lds((const void*)kq, lds_q, grant_q[(g.lse != nullptr) + 2 * dropping])) return rc_;
         if (const int rc_ = ptv3_allow_lds((const void*)kkv, lds_kv, grant_kv[dropping])) return rc_;
-        if (first < total) {
-            const unsigned grid = (unsigned)(full - first + (total - full) * split);
-            hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, g.stream, (const T*)g.qkv, (const T*)g.out, (const T*)g.dout,
-                               g.channels, g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, (T*)g.dqkv,
-                               lse_buf, ws.d, (int)first, (int)full, (int)split, g.drop);
-            hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, g.stream, (const T*)g.qkv, (const T*)g.dout, g.channels,
-                               g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, lse_buf, ws.d, (T*)g.dqkv,
-                               (T*)ws.fill, (int)first, (int)full, (int)split, g.drop);
-        }
+        const unsigned grid = (unsigned)(full - first + (total - full) * split);
+        hipLaunchKernelGGL(kq, dim3(grid), dim3(BWQ_THREADS), lds_q, g.stream, (const T*)g.qkv, (const T*)g.out, (const T*)g.dout,
+                           g.channels, g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, (T*)g.dqkv,
+                           lse_buf, ws.d, (int)first, (int)full, (int)split, g.drop);
+        hipLaunchKernelGGL(kkv, dim3(grid), dim3(BWD_THREADS), lds_kv, g.stream, (const T*)g.qkv, (const T*)g.dout, g.channels,
+                           g.heads, g.slot_src, g.slot_dst, g.cu_seqlens, lds_keys, g.scale, g.n_pad, lse_buf, ws.d, (T*)g.dqkv,
+                           (T*)ws.fill, (int)first, (int)full, (int)split, g.drop);
     }
     const int64_t items = g.n_pad * (2 * g.channels / 8);
     hipLaunchKernelGGL(attn_bwd_finish_kernel<T>, dim3((unsigned)ptv3_ceil_div(items, 256)), dim3(256), 0, g.stream,

@@ -205,6 +205,21 @@ def test_attention_backward_items_shared_by_work_groups(dtype, lens, heads):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,heads", [
+    ([1024] * 6 + [3, 257, 513], 3), ([1024, 130] * 8, 4), ([1024, 128] * 8, 4),                   # mean 768, 577: shared by four; 576
+    ([1024, 512] * 10, 4), ([1024, 516] * 10, 4),                                                  # 768, 770 (shared by two)
+    ([1024] + [124] * 24, 4), ([1024] + [126] * 24, 4), ([1024] + [225] * 24, 4), ([1024] + [226] * 24, 4),
+    ([1024] + [357] * 24, 4), ([1024] + [359] * 24, 4),                                            # 160, 161, 256, 257, 383, 385
+    ([1024, 100] * 34, 4), ([1024, 100] * 27, 5),                                                  # a round and 16 or 14, whose sequence is cut
+    ([512, 2] * 9, 7), ([512, 300, 2] * 3, 7), ([512, 300] * 4, 7), ([512] * 4 + [300, 2, 511], 7),   # 257, 271, 406, 408
+    ([512, 100] * 34, 4), ([512, 40, 20] * 23, 4)])                                                # a round and 16 of 306, 20 of 190
+def test_attention_backward_on_both_sides_of_its_routes(dtype, lens, heads):
+    """Short sequences among long ones, where the items beyond a round go to the two kernels or to shared work-groups, some of
+    them without keys: the same checks."""
+    test_attention_backward_both_sides(dtype, lens, heads, 0.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("blocks", [(32, 31, 25), (24, 17, 16), (9, 8, 1), (32, 24, 16, 9, 8), (29, 28, 25), (28, 13, 12)])
 @pytest.mark.parametrize("times,heads", [(2, 3), (8, 4), (15, 3)])   # shared by four, by two, whole
 def test_attention_backward_rounds_of_query_blocks(dtype, blocks, times, heads):

@@ -21,3 +21,28 @@ for n_seq, length, heads in ((15, 1024, 4), (23, 1024, 4), (32, 1024, 2), (38, 9
                                          0.0, 0, AT, AT, min(sizes), None)
             assert rc == 0 and calls(), (n_seq, length, heads, dtype, cus, rc)
 ''', tmp_path)
+
+
+def test_attention_backward_takes_the_two_kernels_where_sequences_are_short(tmp_path):
+    """Launches on both sides of every line of the rule: the both-sides kernel and the one behind it are two, with a part that is
+    shared three, the two kernels three, behind full rounds of the both-sides kernel four."""
+    hip_stub.run(r'''
+AT = 1 << 20
+def launches(items, mean, longest, cus=256):
+    clear(cus=cus)
+    n, c = items * mean, 16
+    size = lib.ptv3_patch_attn_bwd_workspace_bytes(1, n, c, 1)
+    assert lib.ptv3_patch_attn_bwd(AT, AT, AT, 1, n, c, 1, AT, AT, AT, items, longest, n, 0.25, AT, 0.0, 0, AT, AT, size, None) == 0
+    return [c[2] for c in calls()]
+for longest, items, mean, count in (
+        (1024, 32, 704, 3), (1024, 32, 705, 2), (1024, 33, 704, 2), (1024, 64, 576, 3), (1024, 64, 577, 2), (1024, 65, 577, 3), (1024, 85, 768, 3), (1024, 85, 769, 2), (1024, 86, 768, 2),
+        (1024, 128, 160, 3), (1024, 128, 161, 2), (1024, 128, 256, 2), (1024, 128, 257, 3), (1024, 128, 384, 3), (1024, 128, 385, 2),
+        (1024, 129, 100, 2), (1024, 256, 100, 2), (1024, 512, 320, 2), (1024, 288, 320, 4), (1024, 288, 1000, 3), (1024, 400, 320, 2),
+        (512, 64, 256, 2), (512, 64, 257, 3), (512, 64, 384, 3), (512, 64, 385, 2), (512, 65, 300, 2), (512, 256, 300, 2),
+        (512, 320, 320, 3), (512, 320, 400, 3), (512, 320, 200, 2), (512, 576, 300, 3), (256, 64, 200, 2), (256, 300, 20, 2)):
+    got = launches(items, mean, longest)
+    assert len(got) == count, (longest, items, mean, got)
+# one launch for 320 items of 512 slots whose mean is 320 is the query kernel, at 400 the both-sides kernel, and a shared part
+assert launches(320, 320, 512)[:2] == launches(64, 300, 512)[:2] and launches(320, 400, 512)[0] == launches(256, 400, 512)[0]
+assert len(launches(32, 300, 1024, cus=128)) == 3 and len(launches(43, 577, 1024, cus=128)) == 2   # a quarter and a third of 128
+''', tmp_path)
