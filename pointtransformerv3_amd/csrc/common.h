@@ -46,7 +46,6 @@ __device__ __forceinline__ int ptv3_job_of_block(const J* __restrict__ jobs, int
 // Rows that are read for the last time, or written for much later, go past the caches (the nontemporal hint) where they are more
 // than those hold: what the next kernels read stays there. Of less than that the last kernel's rows are still in the L2. The
 // choice is a template argument: the compiler makes one ordinary access of two behind a condition.
-constexpr int64_t PTV3_L2_BYTES = 32 << 20;   // of the eight XCDs
 template <bool ONCE, typename V> __device__ __forceinline__ V ptv3_read(const V* p) {
     if constexpr (ONCE) return __builtin_nontemporal_load(p);
     else return *p;
@@ -92,6 +91,9 @@ static inline int ptv3_cus() {
     return n;
 }
 
+// What the device's L2s hold: 4 MB an XCD of 32 CUs
+static inline int64_t ptv3_l2_bytes() { return (int64_t)(ptv3_cus() / 32 > 1 ? ptv3_cus() / 32 : 1) << 22; }
+
 // Weights that every XCD reads whole in the launch behind this one: a kernel that leaves memory idle asks for them, and they are
 // in its XCD's L2 by then. In a forward they come from HBM otherwise, and a kernel that streams them has few requests in flight.
 struct Ahead {
@@ -103,7 +105,7 @@ static inline Ahead ptv3_ahead(const void* a, int64_t a_bytes, const void* b, in
                  {a ? (uint32_t)ptv3_ceil_div(a_bytes, 128) : 0, b ? (uint32_t)ptv3_ceil_div(b_bytes, 128) : 0}};
 }
 // This work-group's share: the lines are dealt to the last AHEAD_GROUPS work-groups of each XCD, whose own traffic will not have
-// replaced them, at most four a thread. What comes back is used in ptv3_asked alone, at the kernel's end, and so waited for there.
+// replaced them (two a CU), at most four a thread. What comes back is used in ptv3_asked alone, at the kernel's end, and so waited for there.
 constexpr uint32_t AHEAD_GROUPS = 64;
 __device__ __forceinline__ uint32_t ptv3_ask(const Ahead& a, int tid, int threads) {
     const uint32_t total = a.lines[0] + a.lines[1], groups = gridDim.x >> 3, slot = blockIdx.x >> 3;

@@ -1141,7 +1141,7 @@ int dispatch_pairs_wide(const void* feat, int cin, int taps, int64_t n_pairs, co
 template <typename T, typename Y, bool BN = false>
 void launch_segment_sum(const void* y, const int32_t* row_ptr, int64_t n, int64_t n_pairs, int cout, const void* bias, void* out,
                         hipStream_t stream, const BnGelu& bn = BnGelu{}, const Ahead& ahead = Ahead{}) {
-    auto kern = n_pairs * cout * (int64_t)sizeof(Y) > PTV3_L2_BYTES ? pair_segment_sum_kernel<T, Y, BN, true>
+    auto kern = n_pairs * cout * (int64_t)sizeof(Y) > ptv3_l2_bytes() ? pair_segment_sum_kernel<T, Y, BN, true>
                                                                : pair_segment_sum_kernel<T, Y, BN, false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n * (cout / 8), 256)), dim3(256), 0, stream, (const Y*)y, row_ptr, n, cout,
                        ptv3_piece_div(cout / 8), (const T*)bias, (T*)out, bn, ahead);

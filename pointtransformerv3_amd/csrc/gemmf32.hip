@@ -434,7 +434,7 @@ int ptv3_subm_conv_pairs_f32(const float* feat, int64_t n, int cin, int taps, in
         if (rc != PTV3_OK) return rc;
     }
     if (cout % 4 == 0) {
-        const bool once = n_pairs * cout * 4 > PTV3_L2_BYTES;
+        const bool once = n_pairs * cout * 4 > ptv3_l2_bytes();
         auto kern = bn ? (once ? pair_segment_sum_f32_kernel<4, true, true> : pair_segment_sum_f32_kernel<4, true, false>)
                        : (once ? pair_segment_sum_f32_kernel<4, false, true> : pair_segment_sum_f32_kernel<4, false, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned)ptv3_ceil_div(n * (cout / 4), 256)), dim3(256), 0, stream, y, row_ptr, n, cout,

@@ -573,10 +573,11 @@ extern "C" int64_t ptv3_linear_pack_weights_blocks(int channels) {
 // The first half of a block in one kernel, against the Linear with its LayerNorms and the qkv Linear. At 128 channels always
 // (12.6 -> 7.6 us for 1k rows, 30.6 -> 19.5 for 38k). At 256 a pass streams 512 KB of weights, 9.4 us for any number of rows, and
 // every 8192 rows take 7 - 9 us more, where the register-weight kernels start at 13 - 17 us and take 6.5 us for 8192: 4k rows
-// 14.9 -> 10.8 us, 11.6k 24.9 -> 18.3, 24k 32.9 -> 28.3, 40k 47.6 -> 45.5, but 42k 49.1 and 51.2. Up to 256 rows the qkv layer
-// forms the norms itself (8.4 us for both launches).
+// 14.9 -> 10.8 us, 11.6k 24.9 -> 18.3, 24k 32.9 -> 28.3, 40k 47.6 -> 45.5, but 42k 49.1 and 51.2. So up to five rounds of 32 rows
+// a CU: of 3 x 100k voxels, in the fourth, the forward takes 7358 us with a line at three rounds and 7300 so. Up to 256 rows the
+// qkv layer forms the norms itself (8.4 us for both launches).
 extern "C" int ptv3_block_head_wide_pays(int64_t n, int channels) {
-    return channels == 128 || (channels == 256 && n <= 40960 && !lin_front_pays(n, 256, 768));
+    return channels == 128 || (channels == 256 && n <= 5ll * 32 * ptv3_cus() && !lin_front_pays(n, 256, 768));
 }
 
 extern "C" int ptv3_block_head_wide(const void* conv, const void* shortcut, const void* packed, const void* cpe_bias,

@@ -46,3 +46,23 @@ for longest, items, mean, count in (
 assert launches(320, 320, 512)[:2] == launches(64, 300, 512)[:2] and launches(320, 400, 512)[0] == launches(256, 400, 512)[0]
 assert len(launches(32, 300, 1024, cus=128)) == 3 and len(launches(43, 577, 1024, cus=128)) == 2   # a quarter and a third of 128
 ''', tmp_path)
+
+
+def test_rules_of_the_256_channel_layers_and_of_product_rows_go_by_the_device(tmp_path):
+    """The first half of a block in one kernel up to five rounds of 32 rows a CU; product rows that the L2s (4 MB for 32 CUs) do
+    not hold are read past them, by another instantiation of the kernel that sums them."""
+    hip_stub.run(r'''
+AT = 1 << 20
+for cus in (256, 128, 32, 304):
+    clear(cus=cus)
+    rounds = 5 * 32 * cus
+    assert [lib.ptv3_block_head_wide_pays(n, 256) for n in (256, 257, rounds, rounds + 1)] == [0, 1, 1, 0], cus
+    assert lib.ptv3_block_head_wide_pays(10 * rounds, 128) == 1 and lib.ptv3_block_head_wide_pays(300, 64) == 0
+    held = (cus // 32 << 22) // (256 * 2)   # pairs whose 256 half-precision products the L2s hold
+    sums = []
+    for pairs in (1000, held, held + 1, 10 * held):
+        clear(cus=cus)
+        assert lib.ptv3_subm_conv_pairs_fwd(AT, 1, 900, 256, 27, pairs, AT, AT, AT, AT, AT, AT, 256, AT, AT, None) == 0
+        sums.append(calls()[-1][2])
+    assert sums[0] == sums[1] != sums[2] == sums[3], cus
+''', tmp_path)
