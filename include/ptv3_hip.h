@@ -855,7 +855,8 @@ typedef struct ptv3_train_net {
     int32_t n_zero, has_side;                 /* has_side 0: the description ends in front of `side`, which is not read */
     int64_t zero_blocks;
     ptv3_train_stage stage[PTV3_MAX_LEVELS];
-    void *side;                               /* stream for the weight gradients of the backward (same device, any but its own); null: none */
+    void *side;                               /* stream for the weight gradients of the backward (same device, any but its own); */
+                                              /* null: none, and bwd_scratch is the smaller for it */
 } ptv3_train_net;
 
 int ptv3_zero_ranges(float *base, const ptv3_zero_range *ranges, int count, int64_t blocks, void *stream);

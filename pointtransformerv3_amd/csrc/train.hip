@@ -346,7 +346,8 @@ struct Run {
     // Weight gradients are no part of the chain from dout to the first layer: nothing waits for them but the end of the
     // call. They are put down while a block's chain is queued and launched together behind it (flush), on net.side if the
     // caller gave one, beside the chain of the next blocks. What they read and their slabs lie in one of two arenas in
-    // turn; a group of blocks begins with a wait for the group before last, and ends when it holds GROUP_BYTES.
+    // turn; a group of blocks begins with a wait for the group before last, and ends when it holds GROUP_BYTES. On one stream
+    // one arena serves every group: 1.5 GiB of scratch at 4 x 100k voxels where two arenas make it 2.1.
     hipStream_t side = nullptr;
     hipEvent_t ready = nullptr, done[2] = {};
     bool busy[2] = {}, unmarked = false, closed = true;   // unmarked: work on the side that no event stands behind
@@ -363,9 +364,10 @@ struct Run {
     } convs[GROUP_CONVS];
     int n_convs = 0;
 
+    // descriptions of callers that do not know the field end in front of it, with a zero where the flag is
+    bool two_streams() const { return net.has_side && net.side; }
     int open_side() {
-        // descriptions of callers that do not know the field end in front of it, with a zero where the flag is
-        if (!net.has_side || !net.side || (hipStream_t)net.side == hs) return PTV3_OK;
+        if (!two_streams() || (hipStream_t)net.side == hs) return PTV3_OK;
         hipError_t e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
         for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
         side = e == hipSuccess ? (hipStream_t)net.side : nullptr;
@@ -400,7 +402,7 @@ struct Run {
     int enter(Space** arena) {
         if (closed) {
             closed = false;
-            turn ^= 1;
+            if (two_streams()) turn ^= 1;
             arenas[turn].at = 0;
             TRY(wait_for(turn));
         }

@@ -279,14 +279,20 @@ def _addresses(tensors):
     return (_ptr * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
 
 
+def _train_bytes(net, index_levels):
+    """Bytes of the activations, the forward's scratch and the backward's."""
+    sizes = (ctypes.c_size_t * 3)()
+    at = ctypes.addressof(sizes)
+    _lib.check(_lib.load().ptv3_train_bytes(ctypes.byref(net), index_levels, at, at + 8, at + 16), "ptv3_train_bytes")
+    return list(sizes)
+
+
 class _Step(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, feat, index, masks, *params):
         lib = _lib.load()
         u8 = dict(dtype=torch.uint8, device=feat.device)
-        sizes = (ctypes.c_size_t * 3)()
-        at = ctypes.addressof(sizes)
-        _lib.check(lib.ptv3_train_bytes(ctypes.byref(engine.net), index.levels, at, at + 8, at + 16), "ptv3_train_bytes")
+        sizes = _train_bytes(engine.net, index.levels)
         acts, scratch = torch.empty(sizes[0], **u8), torch.empty(sizes[1], **u8)
         out = torch.empty((feat.shape[0], engine.out_channels), dtype=torch.float32, device=feat.device)
         _lib.check(lib.ptv3_train_fwd(ctypes.byref(engine.net), index.levels, feat.data_ptr(), ops.DTYPE_CODES[feat.dtype],
@@ -320,10 +326,19 @@ class _Step(torch.autograd.Function):
         kept = iter(kept)
         masks = [next(kept) if masked else None for masked in ctx.masked]
         dout = dout.contiguous()
-        scratch = torch.empty(ctx.scratch_bytes, dtype=torch.uint8, device=dout.device)
         grads = torch.empty(engine.total, dtype=torch.float32, device=dout.device)
-        _lib.check(_lib.load().ptv3_train_bwd(ctypes.byref(engine.net), index.levels, dout.data_ptr(), ops.DTYPE_CODES[dout.dtype],
-                                              _addresses(masks), acts.data_ptr(), scratch.data_ptr(), ctx.scratch_bytes,
+        net, nbytes = engine.net, ctx.scratch_bytes
+        try:
+            scratch = torch.empty(nbytes, dtype=torch.uint8, device=dout.device)
+        except torch.cuda.OutOfMemoryError:
+            # what the weight gradients read is held twice for the sake of the second stream: at 4 x 100k voxels 2.1 GiB of
+            # scratch, 1.5 without
+            net = type(net).from_buffer_copy(net)
+            net.side = None
+            nbytes = _train_bytes(net, index.levels)[2]
+            scratch = torch.empty(nbytes, dtype=torch.uint8, device=dout.device)
+        _lib.check(_lib.load().ptv3_train_bwd(ctypes.byref(net), index.levels, dout.data_ptr(), ops.DTYPE_CODES[dout.dtype],
+                                              _addresses(masks), acts.data_ptr(), scratch.data_ptr(), nbytes,
                                               grads.data_ptr(), ops._stream()), "ptv3_train_bwd")
         views = torch._utils._unflatten_dense_tensors(grads, engine.params)
         needed = ctx.needs_input_grad[4:]

@@ -1,5 +1,11 @@
 """Host code of the native training step: what it asks of the runtime, over a stand-in for it (tests/hip_stub.py)."""
+import ctypes
+import types
+
 import hip_stub
+import torch
+
+from pointtransformerv3_amd import native_train
 
 
 def test_the_second_stream_is_waited_for_where_a_call_of_the_runtime_fails(tmp_path):
@@ -70,3 +76,59 @@ import os
 sys.stdout.flush()
 os._exit(0)   # the area is never unmapped: it is half protected
 ''', tmp_path)
+
+
+def test_without_the_second_stream_the_backward_needs_less_scratch(tmp_path):
+    """What it then asks for is refused by one byte, and on one stream it takes groups of weight gradients in turn."""
+    hip_stub.run(r'''
+from train_description import Step
+for points in ((60_000, 40_000, 12_000), (300_000, 200_000, 100_000)):
+    step = Step(points)
+    step.net.side = 0x200
+    two = step.sizes(lib)
+    step.net.side = None
+    one = step.sizes(lib)
+    assert one[:2] == two[:2] and one[2] < 0.85 * two[2], (one, two)
+    clear()
+    assert step.backward(lib, 0x100, one[2] - 1) == -3 and not calls()
+    assert step.backward(lib, 0x100, one[2]) == 0 and {c[1] for c in calls()} == {0x100}
+''', tmp_path)
+
+
+def test_a_backward_that_finds_no_memory_for_two_streams_takes_one(monkeypatch):
+    """A step that fitted without the second stream still runs: the description that is handed over then names none, the
+    engine's own stays as it is for the steps to come."""
+    weight, seen = torch.nn.Parameter(torch.ones(1)), []
+
+    class Lib:
+        def ptv3_train_bytes(self, net, levels, acts, fwd, bwd):
+            for at, size in ((acts, 512), (fwd, 512), (bwd, 4096 if net._obj.side else 2048)):
+                ctypes.c_size_t.from_address(at).value = size
+            return 0
+
+        def ptv3_train_fwd(self, *args):
+            return 0
+
+        def ptv3_train_bwd(self, net, levels, dout, dt, masks, acts, scratch, nbytes, grads, stream):
+            seen.append((net._obj.side, nbytes))
+            ctypes.memset(grads, 0, 4)
+            return 0
+
+    lib = Lib()
+    monkeypatch.setattr(native_train._lib, "load", lambda: lib)
+    monkeypatch.setattr(native_train.ops, "_stream", lambda: None)
+    net = native_train._Net(has_side=1, side=0x200)
+    engine = types.SimpleNamespace(net=net, out_channels=4, dtype=torch.float32, total=1, params=[weight], read_back=[weight])
+    engine.versions = lambda: [p._version for p in engine.read_back]
+    empty, short = torch.empty, [True]
+
+    def limited(*size, **kw):
+        if short[0] and size == (4096,):
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    for short[0] in (True, False):
+        out = native_train._Step.apply(engine, torch.zeros(6, 6), types.SimpleNamespace(levels=None), [None], weight)
+        out.sum().backward()
+    assert seen == [(None, 2048), (0x200, 4096)] and net.side == 0x200
