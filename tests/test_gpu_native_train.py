@@ -263,8 +263,11 @@ def test_native_training_step_on_a_second_stream(monkeypatch):
 @pytest.mark.parametrize("caller", ["default stream", "another stream"])
 def test_weight_gradients_beside_the_backward_are_those_of_one_stream(sizes, caller, monkeypatch):
     """From one group of weight gradients to several that take turns in the two arenas, twice over one forward's activations.
-    The chain's sums by atomics differ in single roundings to half from run to run: the tolerance is that of this path
-    against the modules; an operand overwritten too early would be wrong by its own size."""
+    An operand overwritten too early makes a parameter's gradient wrong by its own size, so every parameter is held by itself.
+    The backward's sums by atomics enter its chain at the first BatchNorm: the matrices of the blocks before it have the same
+    bits. From there on single roundings to half differ from run to run, on one stream as on two: 2.4 % of a parameter's norm
+    were seen (the first block's norm of 300 voxels), 5 % are allowed. A bias in front of a BatchNorm has no gradient but
+    rounding, up to 3.3e-4 of that of its layer's weight were seen, where the other biases have 8e-3 and more: 1e-3."""
     from pointtransformerv3_amd import PointTransformerV3, native_train
     torch.manual_seed(3)
     model = PointTransformerV3(**KW).to(DEV).train()
@@ -277,12 +280,24 @@ def test_weight_gradients_beside_the_backward_are_those_of_one_stream(sizes, cal
         assert engine.net.side and engine.net.side != on.cuda_stream
         with torch.autocast("cuda", dtype=torch.float16):
             feat = model(dict(data)).feat
-        got = []
-        for side in (engine.side.cuda_stream, None, on.cuda_stream, engine.side.cuda_stream):
+        runs = {"one stream": [], "second stream": [], "the caller's stream": []}
+        beside = engine.side.cuda_stream
+        for name, side in (("second stream", beside), ("one stream", None), ("the caller's stream", on.cuda_stream), ("second stream", beside)):
             engine.net.side = side
             model.zero_grad(set_to_none=True)
             feat.backward(torch.full_like(feat, 0.01), retain_graph=True)
-            got.append(torch.cat([p.grad.reshape(-1) for p in model.parameters()]).double())
+            runs[name].append([p.grad.double() for p in model.parameters()])
     torch.cuda.synchronize()
-    for g in got:
-        assert torch.isfinite(g).all() and float((g - got[1]).norm() / got[1].norm()) < 2e-2
+    (alone,) = runs.pop("one stream")
+    names = [name for name, _ in model.named_parameters()]
+    for i, name in enumerate(names):
+        allowed = 5e-2 * float(alone[i].norm())
+        if name.endswith(".bias"):
+            allowed += 1e-3 * float(alone[names.index(name[:-4] + "weight")].norm())
+        same = name.startswith("dec.dec0.block") and any(part in name for part in ("cpe.0", "cpe.1", "attn", "mlp"))
+        for case, got in ((c, g[i]) for c, gs in runs.items() for g in gs):
+            assert torch.isfinite(got).all(), (name, case)
+            assert torch.equal(got, alone[i]) if same else float((got - alone[i]).norm()) <= allowed, (name, case)
+    for got in (g for gs in runs.values() for g in gs):
+        got, want = torch.cat([g.reshape(-1) for g in got]), torch.cat([g.reshape(-1) for g in alone])
+        assert float((got - want).norm() / want.norm()) < 2e-2
