@@ -23,7 +23,8 @@
 //   statistics over all rows (sums of x - pivot and of its square per lane, pivot = the first row, so that
 //   a large mean does not cancel the variance), a one-work-group kernel that turns them into mean / rstd and
 //   updates the running averages, the normalisation itself by the inference kernel with the batch
-//   statistics; backward in two passes over x and dy: the column sums of dz and dz * xhat (dz = dy *
+//   statistics (ptv3_batch_norm_stats; the natively queued step has bn_train_act_kernel in norm.hip form both from the
+//   sums); backward in two passes over x and dy: the column sums of dz and dz * xhat (dz = dy *
 //   gelu'(z), z recomputed), then dx = gamma * rstd * (dz - mean(dz) - xhat * mean(dz * xhat)).
 // * torch_scatter.segment_csr (model.py:684-689): max / min send the gradient of a cluster to the first
 //   member that attains the value, sum copies it to every member, mean divides it by the cluster size.

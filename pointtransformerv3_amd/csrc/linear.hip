@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256) void linear_any_kernel(const T* x, const T* w,
             const int c = col0 + tc + 16 * j;
             if (r >= n || c >= nout) continue;
             float v = acc[i][j] + (bias ? any_f(bias[c]) : 0.f);
-            if (gelu) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
+            if (gelu) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));   // rows of 16 bits: float ones are gemmf32.hip's
             if (resid) v += any_f(resid[r * nout + c]);
             out[r * nout + c] = (T)v;
         }
